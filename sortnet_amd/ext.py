@@ -14,6 +14,24 @@ MASK_TERM = 0
 MASK_FACTORED = 1
 
 
+_host = None
+
+
+def host():
+    """The native autograd front-end (csrc/host.cpp, built next to libsortdist.so), loaded on first use.  There is no
+    fallback."""
+    global _host
+    if _host is None:
+        _lib.load()
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise RuntimeError("sortnet_amd: the native front-end _host.so is missing or does not load - build it with "
+                               "make -C sortnet_amd/csrc (%s)" % e) from e
+        _host = module
+    return _host
+
+
 def _chk(t, name, dtype=torch.float32):
     if not t.is_cuda:
         raise RuntimeError("%s must be a CUDA tensor" % name)

@@ -140,9 +140,7 @@ def _shift(z, vec, sign):
     (the attack differentiates an evaluation-mode stack with respect to its input, attack.py:26-29)."""
     if torch.is_grad_enabled() and (z.requires_grad or vec.requires_grad):
         return z + sign * vec.view(1, -1, 1)
-    out = torch.empty_like(z)
-    ext.channel_shift(z.contiguous(), vec.contiguous(), sign, out)
-    return out
+    return ext.host().channel_shift(z, vec, sign)
 
 
 class NormDistBase(nn.Module):
