@@ -275,6 +275,15 @@ int sd_mean_shift_index_forward(const float* input, const int* index, int B, int
                                 float* mean, float* running_mean, float momentum, float* output,
                                 sd_stream_t stream);
 
+/* ---- patches of the convolutional distance layer (core/models/norm_dist.py:148-155 uses torch's unfold) ----
+ * output (B, C * KH * KW, OH * OW): the windows of input (B, C, H, W) as columns, zeros outside the image;
+ * OH = (H + 2 padding - dilation (KH - 1) - 1) / stride + 1.  sd_fold is its transpose: output (B, C, H, W) = the sum
+ * of the column entries that a pixel went to, added in window order (deterministic). */
+int sd_unfold(const float* input, int B, int C, int H, int W, int KH, int KW, int stride, int padding, int dilation,
+              float* output, sd_stream_t stream);
+int sd_fold(const float* columns, int B, int C, int H, int W, int KH, int KW, int stride, int padding, int dilation,
+            float* output, sd_stream_t stream);
+
 /* ---- device-side mask sampling for the index-list form (replaces sample_mask,
  * core/models/norm_dist.py:14-17, which draws on the host with a device synchronisation) ---- */
 

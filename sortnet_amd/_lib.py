@@ -40,6 +40,8 @@ SIGNATURES = {
     "sd_mean_shift_forward": [_F, _i, _i, _i, _F, _F, _f, _F, _S],
     "sd_mean_shift_index_forward": [_F, _I, _i, _i, _i, _i, _i, _F, _F, _f, _F, _S],
     "sd_channel_shift": [_F, _F, _i, _i, _i, _f, _F, _S],
+    "sd_unfold": [_F, _i, _i, _i, _i, _i, _i, _i, _i, _i, _F, _S],
+    "sd_fold": [_F, _i, _i, _i, _i, _i, _i, _i, _i, _i, _F, _S],
     "sd_sample_index_lists": [_u, _i, _i, _i, _i, _I, _S],
 }
 _OTHER = {

@@ -383,6 +383,46 @@ Tensor channel_shift(const Tensor& z_in, const Tensor& vec_in, double sign) {
     return out;
 }
 
+// ---- windows of a convolutional layer as columns; the gradient is the sum back into the image --------------------------
+struct UnfoldNode : Node {
+    int B, C, H, W, KH, KW, stride, pad, dil;
+
+    variable_list apply(variable_list&& grads) override {
+        at::AutoDispatchBelowADInplaceOrView below;
+        variable_list out(1);
+        if (!grads[0].defined() || !task_should_compute_output(0)) return out;
+        const Tensor g = grads[0].contiguous();
+        const c10::DeviceGuard guard(g.device());
+        out[0] = new_floats(g, {B, C, H, W});
+        require(sd_fold(floats(g, "grad_output"), B, C, H, W, KH, KW, stride, pad, dil, floats(out[0], "grad_input"), stream_of(g)),
+                "sd_fold");
+        return out;
+    }
+    std::string name() const override { return "UnfoldNode"; }
+};
+
+Tensor unfold(const Tensor& x_in, int kh, int kw, int dil, int pad, int stride) {
+    const bool grad = want_grad(x_in);
+    const int B = (int)x_in.size(0), C = (int)x_in.size(1), H = (int)x_in.size(2), W = (int)x_in.size(3);
+    Tensor y;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        const c10::DeviceGuard guard(x_in.device());
+        const Tensor x = x_in.contiguous();
+        const int64_t oh = (H + 2 * pad - dil * (kh - 1) - 1) / stride + 1, ow = (W + 2 * pad - dil * (kw - 1) - 1) / stride + 1;
+        y = new_floats(x, {B, (int64_t)C * kh * kw, oh > 0 && ow > 0 ? oh * ow : 1});   // a window that does not fit is refused below
+        require(sd_unfold(floats(x, "input"), B, C, H, W, kh, kw, stride, pad, dil, floats(y, "output"), stream_of(x)), "sd_unfold");
+    }
+    if (grad) {
+        auto node = new_node<UnfoldNode>();
+        node->set_next_edges(collect_next_edges(x_in));
+        node->B = B; node->C = C; node->H = H; node->W = W; node->KH = kh; node->KW = kw;
+        node->stride = stride; node->pad = pad; node->dil = dil;
+        set_history(y, node);
+    }
+    return y;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_host, m) {
@@ -397,4 +437,5 @@ PYBIND11_MODULE(_host, m) {
     m.def("mean_shift", &mean_shift, released());
     m.def("mean_shift_index", &mean_shift_index, released());
     m.def("channel_shift", &channel_shift, released());
+    m.def("unfold", &unfold, released());
 }

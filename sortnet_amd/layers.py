@@ -21,7 +21,6 @@ from collections.abc import Iterable
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as TF
 
 from . import ext
 from . import functional as F
@@ -249,11 +248,16 @@ class NormDistConv(NormDistBase):
     def forward(self, x=None, lower=None, upper=None):
         ref = x if x is not None else lower
         h, w = ref.size(2), ref.size(3)
-        unfold = lambda z: TF.unfold(z, self.kernel_size, self.dilation, self.padding, self.stride).contiguous()
-        paras = super().forward(*apply_if_not_none((x, lower, upper), unfold))
+        paras = super().forward(*apply_if_not_none((x, lower, upper), self._columns))
         h, w = [(s + 2 * self.padding - self.dilation * (k - 1) - 1) // self.stride + 1
                 for s, k in zip((h, w), self.kernel_size)]
         return tuple(apply_if_not_none(paras, lambda z: z.reshape(z.size(0), -1, h, w)))
+
+    def _columns(self, z):
+        """The windows of z as columns (B, C * kh * kw, positions)."""
+        if self.kernel_size == (1, 1) and self.stride == 1 and self.padding == 0:
+            return z.flatten(2).contiguous()       # every pixel is its own window: no copy of what is contiguous
+        return ext.host().unfold(z, *self.kernel_size, self.dilation, self.padding, self.stride)
 
 
 class BoundSequential(nn.Sequential):
