@@ -4,6 +4,7 @@
 #include "bound_cols.h"
 #include "sort_cols.h"
 #include "row_cands.h"
+#include "row_stream.h"
 #include <atomic>
 #include <mutex>
 #include <type_traits>
@@ -122,14 +123,14 @@ extern "C" int sd_set_linf_candidate_depth(int depth) {
 }
 
 // One work-item per (row, chunk): the 32 keep bits of the factored mask for inputs
-// chunk*32 .. chunk*32+31 of an x row (stream 1) or a w row (stream 2).
-static __global__ void __launch_bounds__(256) build_masks_kernel(uint32_t* __restrict__ out, long long rows, int nchunks,
-                                                          int CIg, uint32_t seed, uint32_t stream, uint32_t t16) {
+// chunk*32 .. chunk*32+31 of an x row (stream 1) or, behind the xrows x rows, of a w row (stream 2).
+static __global__ void __launch_bounds__(256) build_masks_kernel(uint32_t* __restrict__ out, long long xrows, long long rows, int nchunks,
+                                                          int CIg, uint32_t seed, uint32_t t16) {
     long long i = (long long)blockIdx.x * 256 + threadIdx.x;
     if (i >= rows * nchunks) return;
-    uint32_t row = (uint32_t)(i / nchunks);
-    int chunk = (int)(i - (long long)row * nchunks);
-    uint32_t key = rng_row_key(seed, stream, row);
+    const long long r = i / nchunks;
+    const int chunk = (int)(i - r * nchunks);
+    const uint32_t key = r < xrows ? rng_row_key(seed, 1u, (uint32_t)r) : rng_row_key(seed, 2u, (uint32_t)(r - xrows));
     uint32_t bits = 0;
     #pragma unroll 8
     for (int k = 0; k < KT; k++) {
@@ -192,6 +193,8 @@ extern "C" int sd_inf_dist_forward_nograd(const float* input, const float* weigh
     SD_REQUIRE(output, "inf_dist_forward_nograd: null output");
     a.y0 = output;
     hipStream_t st = static_cast<hipStream_t>(stream);
+    const bool streamed = g_linf_density.load(std::memory_order_relaxed) <= 0.f;   // not where tables are forced
+    if (streamed && row_stream_ok(a, kStreamMaxTerms)) return row_stream_linf(a, st);
     static const int kTb42[] = {4, 2};   // 8 rows per work-item measured slower (168 registers, three waves per SIMD)
     const int TB = pick_tb(a, kTb42, 2, 128);
     a.nsplit = pick_nsplit(a, 16 * TB, 128);
@@ -220,6 +223,7 @@ extern "C" int sd_inf_dist_forward(const float* input, const float* weight,
     SD_REQUIRE(output && pos, "inf_dist_forward: null output or pos");
     a.y0 = output; a.p0 = pos;
     hipStream_t st = static_cast<hipStream_t>(stream);
+    if (g_linf_density.load(std::memory_order_relaxed) <= 0.f && row_stream_ok(a, kStreamPosTerms)) return row_stream_linf(a, st);
     const int KE = max_cols_eligible(a, 1.f, B, CO, CI, G, HW);
     if (!KE) return run_chunk_pos<LinfChunk>(a, w_index_ci || w_index_co, st);
     const int K = max_cols_wanted(a, KE, kHintSiteLinf, B, CO, CI, st);
@@ -315,7 +319,8 @@ extern "C" int sd_masked_inf_dist_forward(const float* input, const float* weigh
     size_t packed_bytes = 0;
     int K = 0;          // depth of the candidate tables' bound (0: no tables)
     void* tables = nullptr;
-    if (a.fast_x && a.fast_w) {
+    const bool streamable = HW == 1 && g_linf_density.load(std::memory_order_relaxed) <= 0.f;
+    if ((a.fast_x && a.fast_w) || streamable) {
         const int nchunks = (a.CIg + KT - 1) / KT;
         const long long xrows = (long long)a.R * G, wrows = (long long)CO;
         packed_bytes = pos ? (((size_t)a.R * CO * 8 + 255) / 256) * 256 : 0;
@@ -328,12 +333,11 @@ extern "C" int sd_masked_inf_dist_forward(const float* input, const float* weigh
         tables = base + packed_bytes + mask_bytes;
         uint32_t* xm = reinterpret_cast<uint32_t*>(base + packed_bytes);
         uint32_t* wm = xm + xrows * nchunks;
-        hipLaunchKernelGGL(build_masks_kernel, dim3((unsigned)((xrows * nchunks + 255) / 256)), dim3(256), 0, st,
-                           xm, xrows, nchunks, a.CIg, seed, 1u, a.t16);
-        hipLaunchKernelGGL(build_masks_kernel, dim3((unsigned)((wrows * nchunks + 255) / 256)), dim3(256), 0, st,
-                           wm, wrows, nchunks, a.CIg, seed, 2u, a.t16);
+        hipLaunchKernelGGL(build_masks_kernel, dim3((unsigned)(((xrows + wrows) * nchunks + 255) / 256)), dim3(256), 0, st,
+                           xm, xrows, xrows + wrows, nchunks, a.CIg, seed, a.t16);
         if ((rc = check_launch("build_masks_kernel"))) return rc;
         a.xmask = xm; a.wmask = wm;
+        if (streamable && row_stream_ok(a, kStreamMaskTerms)) return row_stream_linf(a, st);
     }
     if (pos) {
         if (K && (rc = queue_max_cols(a, K, B, CO, CI, tables, st))) return rc;
@@ -363,6 +367,7 @@ extern "C" int sd_bound_inf_dist_forward_nograd(const float* inputL, const float
     SD_REQUIRE(outputL && outputU, "bound_inf_dist_forward_nograd: null output");
     a.y0 = outputL; a.y1 = outputU;
     hipStream_t st = static_cast<hipStream_t>(stream);
+    if (g_bound_density.load(std::memory_order_relaxed) <= 0.f && row_stream_ok(a, kStreamBoundTerms)) return row_stream_bound(a, st);
     static const int kTb42[] = {4, 2};
     const int TB = pick_tb(a, kTb42, 2, 128);
     a.nsplit = pick_nsplit(a, 16 * TB, 16 * 8);
@@ -446,6 +451,7 @@ extern "C" int sd_bound_inf_dist_forward(const float* inputL, const float* input
     SD_REQUIRE(outputL && outputU && posL && posU, "bound_inf_dist_forward: null output or pos");
     a.y0 = outputL; a.y1 = outputU; a.p0 = posL; a.p1 = posU;
     hipStream_t st = static_cast<hipStream_t>(stream);
+    if (g_bound_density.load(std::memory_order_relaxed) <= 0.f && row_stream_ok(a, kStreamBoundPosTerms)) return row_stream_bound(a, st);
     static const int kTb42[] = {4, 2};
     const int TB = pick_tb(a, kTb42, 2, 64);
     a.nsplit = pick_nsplit(a, 16 * TB, 64);

@@ -1,0 +1,384 @@
+// Few batch rows (one image up to a small batch in evaluation): the layer is a pass over its weights, so its floor is
+// the time to read them (5120 x 5120: 105 MB).  The tile kernels cut such a layer into workgroups of 32 batch rows, most
+// of them padding, and the candidate tables read the weights three times to save arithmetic that costs nothing here.
+//
+// A wavefront owns one weight row: every lane loads its share of the row once (NE inputs, all loads in flight together)
+// and keeps it in registers; the batch rows pass by in LDS, shared by the four wavefronts of the workgroup.
+//   l-inf: 1.5 vector instructions per term and a reduction over the lanes; with positions, the first group of inputs
+//   that holds the maximum is found by one comparison per group.
+//   sort neuron: the K largest of the row without sorting it.  The K-th largest of the 64 lane maxima is a lower bound T
+//   of the K-th largest term (each of the K lanes above it holds one), found bit by bit with ballots; the terms of at
+//   least T, about K + 1 of them on data without ties, hold the K largest.  The groups of four inputs that reach T (as
+//   many) go to LDS, one term per lane, are ranked against each other and added up in the order of the other kernels
+//   (largest first, every product rounded on its own), so the result has the same bits.
+// More than 16 such groups, or more than 64 such terms (many equal terms): slower exact paths of the same kernel.
+#include "fwd_tile.h"
+#include "row_stream.h"
+
+namespace sd {
+namespace {
+
+enum StreamOp { kStreamMax, kStreamPos, kStreamSort };
+// weight rows (wavefronts) per workgroup: eight share a staged batch row, four where the registers of the sort neuron
+// leave room for twelve wavefronts per compute unit
+constexpr int stream_waves(StreamOp op) { return op == kStreamSort ? 4 : 8; }
+
+// maximum over the wavefront, in every lane (row-wise shifts, then the two row broadcasts; v >= 0)
+__device__ __forceinline__ float wave_max(float v) {
+#define SD_DPP_MAX(ctrl, rows) \
+    v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), ctrl, rows, 0xf, false)))
+    SD_DPP_MAX(0x111, 0xf);      // row_shr:1
+    SD_DPP_MAX(0x112, 0xf);      // row_shr:2
+    SD_DPP_MAX(0x114, 0xf);      // row_shr:4
+    SD_DPP_MAX(0x118, 0xf);      // row_shr:8
+    SD_DPP_MAX(0x142, 0xa);      // row_bcast:15 into rows 1 and 3
+    SD_DPP_MAX(0x143, 0xc);      // row_bcast:31 into rows 2 and 3
+#undef SD_DPP_MAX
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+
+__device__ __forceinline__ int lanes_below(unsigned long long mask) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
+// LDS operations of one wavefront complete in order; this keeps the compiler from moving them across
+__device__ __forceinline__ void wave_fence() { __builtin_amdgcn_wave_barrier(); }
+
+// NE inputs per lane in groups of four.  VEC: a group is four neighbouring inputs (rows a multiple of four long and
+// aligned), otherwise inputs 64 apart, so that loads coalesce either way.  grid.y: slices of the batch rows.
+// NX = 1: terms |x - w|.  NX = 2: interval bounds, terms -min(w - l, u - w) for the lower (side 0) and
+// max(w - l, u - w) for the upper result (side 1), inverted intervals repaired as everywhere.
+template <int NE, bool VEC, int NX, StreamOp OP>
+__global__ void __launch_bounds__(64 * stream_waves(OP), NE <= 48 ? 4 : NE <= 80 ? (OP == kStreamSort ? 3 : 4) : (OP == kStreamSort ? 1 : 2))
+row_stream_kernel(FwdArgs a, int K) {
+    constexpr int NG = NE / 4, kWaves = stream_waves(OP);
+    constexpr bool MASKABLE = NX == 1 && OP != kStreamSort;
+    __shared__ __attribute__((aligned(16))) float xs[NX][NE * 64];
+    __shared__ __attribute__((aligned(16))) float cand[OP == kStreamSort ? kWaves : 1][64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tiles = (a.COg + kWaves - 1) / kWaves, g = blockIdx.x / tiles;
+    const int CI = a.CIg, m = (blockIdx.x - g * tiles) * kWaves + wave;
+    const bool mine = m < a.COg;
+    const int c = g * a.COg + (mine ? m : a.COg - 1);
+    const float* wrow = a.w + (size_t)c * CI;
+    // factored mask: inputs and weights that the mask drops are undefined, and undefined terms never win a maximum
+    const int nchunks = (CI + KT - 1) / KT;
+    const uint32_t* wkeep = MASKABLE && a.xmask ? a.wmask + (size_t)c * nchunks : nullptr;
+    auto masked = [](float v, const uint32_t* keep, int n) {
+        return keep == nullptr || ((keep[n >> 5] >> (n & 31)) & 1u) ? v : __builtin_nanf("");
+    };
+    // the row as a buffer of 4 CI bytes
+    const uint64_t wbits = reinterpret_cast<uint64_t>(wrow);
+    void* wuni = reinterpret_cast<void*>(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(wbits >> 32)) << 32) |
+                                         (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)wbits));
+    const auto wrsrc = __builtin_amdgcn_make_buffer_rsrc(wuni, 0, 4 * CI, 0x00020000);
+
+    // inputs of group e of this lane: VEC: 4 (64 e + lane) + j, else 256 e + 64 j + lane; beyond the row x = w = 0
+    float w[NG][4];
+    #pragma unroll
+    for (int e = 0; e < NG; e++) {
+        if (VEC) {
+            const int n = 4 * (64 * e + lane);
+            const bool in = n < CI;
+            const int nn = in ? n : 0;
+            float4 v = *reinterpret_cast<const float4*>(wrow + nn);
+            if (wkeep) v = make_float4(masked(v.x, wkeep, nn), masked(v.y, wkeep, nn + 1), masked(v.z, wkeep, nn + 2), masked(v.w, wkeep, nn + 3));
+            w[e][0] = in ? v.x : 0.f; w[e][1] = in ? v.y : 0.f; w[e][2] = in ? v.z : 0.f; w[e][3] = in ? v.w : 0.f;
+        } else {
+            #pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int n = 256 * e + 64 * j + lane;
+                // (a buffer load returns 0 beyond the row: a select per input would keep a lane mask alive for each)
+                w[e][j] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(wrsrc, 4 * n, 0, 0));
+                if (wkeep && n < CI) w[e][j] = masked(w[e][j], wkeep, n);
+            }
+        }
+    }
+    #pragma unroll
+    for (int k = 0; k < NX; k++)
+        for (int n = CI + tid; n < NE * 64; n += 64 * kWaves) xs[k][n] = 0.f;
+
+    // The staged rows stay in LDS between the passes: keeps the compiler from holding what one pass read in registers for
+    // the next, and (every few groups) from starting a whole pass's reads at once
+    auto pass_fence = []() { asm volatile("" ::: "memory"); };
+    auto group_fence = [](int e) { if (NX == 2 && e % 2 == 1) { asm volatile("" ::: "memory"); __builtin_amdgcn_sched_barrier(0); } };
+    auto load4 = [&](const float* row, int e, float (&x)[4]) {
+        if (VEC) {
+            const float4 t = *reinterpret_cast<const float4*>(&row[4 * (64 * e + lane)]);
+            x[0] = t.x; x[1] = t.y; x[2] = t.z; x[3] = t.w;
+        } else {
+            #pragma unroll
+            for (int j = 0; j < 4; j++) x[j] = row[256 * e + 64 * j + lane];
+        }
+    };
+    // terms of group e, and what bit 31 of a position says about each (only evaluated where it is used)
+    auto terms = [&](int side, int e, float (&v)[4], bool (&flag)[4]) {
+        float x[4], u[4];
+        load4(xs[0], e, x);
+        if (NX == 2) load4(xs[NX - 1], e, u);
+        #pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (NX == 1) { const float d = x[j] - w[e][j]; v[j] = fabsf(d); flag[j] = d < 0.f; }
+            else {
+                const float t1 = w[e][j] - x[j], t2 = u[j] - w[e][j];
+                v[j] = side ? fmaxf(t1, t2) : -fminf(t1, t2);
+                flag[j] = !(t1 <= t2);
+            }
+        }
+    };
+
+    const int r_lo = (int)((long long)blockIdx.y * a.R / gridDim.y), r_hi = (int)((long long)(blockIdx.y + 1) * a.R / gridDim.y);
+    for (int r = r_lo; r < r_hi; r++) {
+        const size_t xoff = (size_t)(r * a.G + g) * CI;
+        const uint32_t* xkeep = MASKABLE && a.xmask ? a.xmask + (size_t)(r * a.G + g) * nchunks : nullptr;
+        if (r > r_lo) __syncthreads();                 // every wavefront is done with the row before
+        for (int n = VEC ? 4 * tid : tid; n < CI; n += (VEC ? 4 : 1) * 64 * kWaves) {
+            constexpr int W = VEC ? 4 : 1;
+            float x[W], u[W];
+            if (VEC) {
+                const float4 t = *reinterpret_cast<const float4*>(a.x0 + xoff + n);
+                x[0] = t.x; x[W / 2] = t.z; x[W > 1 ? 1 : 0] = W > 1 ? t.y : t.x; x[W - 1] = W > 1 ? t.w : t.x;
+            } else x[0] = a.x0[xoff + n];
+            if (NX == 2) {
+                if (VEC) {
+                    const float4 t = *reinterpret_cast<const float4*>(a.x1 + xoff + n);
+                    u[0] = t.x; u[W / 2] = t.z; u[W > 1 ? 1 : 0] = W > 1 ? t.y : t.x; u[W - 1] = W > 1 ? t.w : t.x;
+                } else u[0] = a.x1[xoff + n];
+            }
+            #pragma unroll
+            for (int j = 0; j < W; j++) {
+                if (NX == 2) { if (x[j] > u[j]) x[j] = u[j] = (x[j] + u[j]) * 0.5f; }
+                if (xkeep) x[j] = masked(x[j], xkeep, n + j);
+                xs[0][n + j] = x[j];
+                if (NX == 2) xs[NX - 1][n + j] = u[j];
+            }
+        }
+        __syncthreads();
+
+        const size_t o = (size_t)(r * a.G + g) * a.COg + m;
+        if (OP == kStreamMax) {
+            float top[NX];
+            #pragma unroll
+            for (int k = 0; k < NX; k++) top[k] = 0.f;
+            #pragma unroll
+            for (int e = 0; e < NG; e++) {
+                #pragma unroll
+                for (int k = 0; k < NX; k++) {
+                    float v[4];
+                    bool flag[4];
+                    terms(k, e, v, flag);
+                    top[k] = fmaxf(fmaxf(fmaxf(fmaxf(top[k], v[0]), v[1]), v[2]), v[3]);
+                }
+                group_fence(e);
+            }
+            #pragma unroll
+            for (int k = 0; k < NX; k++) asm volatile("" : "+v"(top[k]));   // both maxima are formed in the one pass above
+            #pragma unroll
+            for (int k = 0; k < NX; k++) {
+                top[k] = wave_max(top[k]);
+                if (mine && lane == 0) (k ? a.y1 : a.y0)[o] = fmaxf(top[k], kEps);
+            }
+            continue;
+        }
+        #pragma unroll
+        for (int side = 0; side < NX; side++) {
+            float gm[NG], top = 0.f;                   // maxima per group and per lane (undefined terms never win)
+            #pragma unroll
+            for (int e = 0; e < NG; e++) {
+                float v[4];
+                bool flag[4];
+                terms(side, e, v, flag);
+                gm[e] = fmaxf(fmaxf(fmaxf(v[0], v[1]), v[2]), v[3]);
+                top = fmaxf(top, gm[e]);
+                group_fence(e);
+            }
+            pass_fence();
+            if (OP == kStreamPos) {
+                top = wave_max(top);
+                int pos = NX == 2 && side == 0 ? (int)kNanId : 0;
+                bool found = !(top > kEps);
+                // groups in ascending order of their inputs; inside a group VEC: the lane decides before the element,
+                // else the element before the lane
+                #pragma unroll
+                for (int e = 0; e < NG; e++) {
+                    if (found || __builtin_amdgcn_ballot_w64(gm[e] == top) == 0ull) continue;
+                    found = true;
+                    float v[4];
+                    bool flag[4];
+                    terms(side, e, v, flag);
+                    if (VEC) {
+                        int at = 0;
+                        bool has = false;
+                        #pragma unroll
+                        for (int j = 3; j >= 0; j--)
+                            if (v[j] == top) { at = (4 * (64 * e + lane) + j) | (flag[j] ? (int)kSign : 0); has = true; }
+                        pos = __builtin_amdgcn_readlane(at, (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(has)));
+                    } else {
+                        #pragma unroll
+                        for (int j = 3; j >= 0; j--) {
+                            const unsigned long long hit = __builtin_amdgcn_ballot_w64(v[j] == top);
+                            const unsigned long long second = __builtin_amdgcn_ballot_w64(flag[j]);
+                            if (hit == 0ull) continue;
+                            const int l = (int)__builtin_ctzll(hit);
+                            pos = (256 * e + 64 * j + l) | ((second >> l) & 1ull ? (int)kSign : 0);
+                        }
+                    }
+                }
+                if (mine && lane == 0) {
+                    (side ? a.y1 : a.y0)[o] = fmaxf(top, kEps);
+                    (side ? a.p1 : a.p0)[o] = pos;
+                }
+                continue;
+            }
+            // lower bound of the K-th largest term: the largest bit pattern that K lane maxima reach (their order as
+            // numbers is their order as integers), or a smaller one that exactly K reach
+            uint32_t bits = 0u;
+            for (int bit = 30; bit >= 0; bit--) {
+                const uint32_t t = bits | (1u << bit);
+                const int reach = __builtin_popcountll(__builtin_amdgcn_ballot_w64(__float_as_uint(top) >= t));
+                if (reach < K) continue;
+                bits = t;
+                if (reach == K) break;
+            }
+            const float T = __uint_as_float(bits > 0u ? bits : 1u);   // fewer than K positive lane maxima: every positive term
+            int groups = 0;
+            #pragma unroll
+            for (int e = 0; e < NG; e++) groups += __builtin_popcountll(__builtin_amdgcn_ballot_w64(gm[e] >= T));
+            int count = 0;
+            if (groups <= 16) {
+                int at = 0;
+                #pragma unroll
+                for (int e = 0; e < NG; e++) {
+                    const unsigned long long any = __builtin_amdgcn_ballot_w64(gm[e] >= T);
+                    if (any == 0ull) continue;
+                    if (gm[e] >= T) {
+                        float v[4];
+                        bool flag[4];
+                        terms(side, e, v, flag);
+                        *reinterpret_cast<float4*>(&cand[wave][4 * (at + lanes_below(any))]) = make_float4(v[0], v[1], v[2], v[3]);
+                    }
+                    at += __builtin_popcountll(any);
+                }
+                wave_fence();
+                // the terms that reach T move to the front
+                const float v = lane < 4 * groups ? cand[wave][lane] : 0.f;
+                const unsigned long long hit = __builtin_amdgcn_ballot_w64(v >= T);
+                count = __builtin_popcountll(hit);
+                wave_fence();
+                if (v >= T) cand[wave][lanes_below(hit)] = v;
+            } else {
+                #pragma unroll
+                for (int e = 0; e < NG; e++) {
+                    if (__builtin_amdgcn_ballot_w64(gm[e] >= T) == 0ull) continue;
+                    float v[4];
+                    bool flag[4];
+                    terms(side, e, v, flag);
+                    #pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const unsigned long long hit = __builtin_amdgcn_ballot_w64(v[j] >= T);
+                        const int at = count + lanes_below(hit);
+                        if (v[j] >= T && at < 64) cand[wave][at] = v[j];
+                        count += __builtin_popcountll(hit);
+                    }
+                }
+            }
+            wave_fence();
+            float sorted = 0.f;                        // lane k: the k-th largest term (0 when there are fewer)
+            if (count <= 64) {
+                const float own = lane < count ? cand[wave][lane] : 0.f;
+                int rank = 0;
+                for (int j = 0; j < count; j++) {
+                    const float other = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(own), j));
+                    rank += (other > own || (other == own && j < lane)) ? 1 : 0;
+                }
+                wave_fence();
+                if (lane < count) cand[wave][rank] = own;   // ranks are the numbers 0 .. count - 1
+                wave_fence();
+                sorted = lane < count ? cand[wave][lane] : 0.f;
+                wave_fence();
+            } else {
+                float below = __builtin_inff();
+                bool first = true;
+                for (int k = 0; k < K;) {
+                    float best = 0.f;
+                    #pragma unroll
+                    for (int e = 0; e < NG; e++) {
+                        float v[4];
+                        bool flag[4];
+                        terms(side, e, v, flag);
+                        #pragma unroll
+                        for (int j = 0; j < 4; j++) best = (v[j] < below || (first && v[j] == below)) && v[j] > best ? v[j] : best;
+                    }
+                    best = wave_max(best);
+                    if (best == 0.f) break;
+                    int same = 0;
+                    #pragma unroll
+                    for (int e = 0; e < NG; e++) {
+                        float v[4];
+                        bool flag[4];
+                        terms(side, e, v, flag);
+                        #pragma unroll
+                        for (int j = 0; j < 4; j++) same += __builtin_popcountll(__builtin_amdgcn_ballot_w64(v[j] == best));
+                    }
+                    if (lane >= k && lane < k + same) sorted = best;
+                    k += same;
+                    below = best;
+                    first = false;
+                }
+            }
+            float ans = kEps, coef = 1.f;
+            for (int k = 0; k < K; k++) {
+                ans += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sorted), k)) * coef * a.q;
+                coef *= 1.f - a.q;
+            }
+            if (mine && lane == 0) (side ? a.y1 : a.y0)[o] = ans / (1.f - coef);
+        }
+    }
+}
+
+template <int NE, int NX, StreamOp OP>
+int launch(const FwdArgs& a, int K, hipStream_t stream) {
+    // few weight rows: the batch rows are dealt to several workgroups, each of which loads the weight rows again
+    constexpr int kWaves = stream_waves(OP);
+    const int tiles = (a.COg + kWaves - 1) / kWaves * a.G, want = 16 / kWaves * num_cus();
+    const int slices = tiles >= want ? 1 : (want + tiles - 1) / tiles;
+    const dim3 grid(tiles, slices < a.R ? slices : a.R), block(64 * kWaves);
+    note_forward_kernel("row_stream_kernel", kWaves, NE);
+    forward_kernel_timer(stream, false);
+    if (a.fast_x && a.fast_w) hipLaunchKernelGGL((row_stream_kernel<NE, true, NX, OP>), grid, block, 0, stream, a, K);
+    else hipLaunchKernelGGL((row_stream_kernel<NE, false, NX, OP>), grid, block, 0, stream, a, K);
+    forward_kernel_timer(stream, true);
+    return check_launch("row_stream_kernel");
+}
+
+template <int NX, StreamOp OP>
+int dispatch(const FwdArgs& a, int K, hipStream_t stream) {
+    if (a.CIg <= 16 * 64) return launch<16, NX, OP>(a, K, stream);
+    if (a.CIg <= 48 * 64) return launch<48, NX, OP>(a, K, stream);
+    if (a.CIg <= 80 * 64) return launch<80, NX, OP>(a, K, stream);
+    return launch<160, NX, OP>(a, K, stream);
+}
+
+}  // namespace
+
+bool row_stream_ok(const FwdArgs& a, long long limit) {
+    return a.HW == 1 && !a.ci_idx && !a.co_idx && a.CIg <= 160 * 64 && (long long)a.R * a.G * a.COg * a.CIg <= limit &&
+           (a.mask_mode < 0 || (a.mask_mode == SD_MASK_FACTORED && a.xmask && a.wmask));
+}
+
+bool row_stream_sort_ok(const FwdArgs& a) {
+    const long long outputs = (long long)a.R * a.G * a.COg, most = a.x1 ? 3ll << 14 : 1ll << 16, per_input = a.x1 ? 56 : 80;
+    return outputs <= most && outputs <= per_input * a.CIg && row_stream_ok(a, 1ll << 62);
+}
+
+int row_stream_linf(const FwdArgs& a, hipStream_t stream) {
+    return a.p0 ? dispatch<1, kStreamPos>(a, 0, stream) : dispatch<1, kStreamMax>(a, 0, stream);
+}
+int row_stream_bound(const FwdArgs& a, hipStream_t stream) {
+    return a.p0 ? dispatch<2, kStreamPos>(a, 0, stream) : dispatch<2, kStreamMax>(a, 0, stream);
+}
+int row_stream_sort(const FwdArgs& a, int K, hipStream_t stream) {
+    return a.x1 ? dispatch<2, kStreamSort>(a, K, stream) : dispatch<1, kStreamSort>(a, K, stream);
+}
+
+}  // namespace sd

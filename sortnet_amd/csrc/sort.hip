@@ -4,6 +4,7 @@
 #include "fwd_args.h"
 #include "sort_cols.h"
 #include "row_cands.h"
+#include "row_stream.h"
 #include <atomic>
 
 using namespace sd;
@@ -229,6 +230,8 @@ extern "C" int sd_sort_neuron_forward_nograd(const float* input, const float* we
     SD_REQUIRE(output, "sort_neuron_forward_nograd: null output");
     a.y0 = output; a.q = q;
     hipStream_t st = static_cast<hipStream_t>(stream);
+    if (g_sort_density.load(std::memory_order_relaxed) <= 0.f && row_stream_sort_ok(a))
+        return row_stream_sort(a, K, st);
     const bool small = few_tiles(a, 32, 64);
     const bool two = K <= 12 && two_level_ok(a, K), elig = sort_cols_eligible(a, B, CO, CI, G, HW);
     const bool cols = elig && sort_cols_ok(a, kHintSiteSort, B, CO, CI, st);
@@ -303,6 +306,8 @@ extern "C" int sd_bound_sort_neuron_forward(const float* inputL, const float* in
     SD_REQUIRE(outputL && outputU, "bound_sort_neuron_forward: null output");
     a.y0 = outputL; a.y1 = outputU; a.q = q;
     hipStream_t st = static_cast<hipStream_t>(stream);
+    if (g_sort_density.load(std::memory_order_relaxed) <= 0.f && row_stream_sort_ok(a))
+        return row_stream_sort(a, K, st);
     const bool small = few_tiles(a, 32, 32);
     const bool elig = sort_cols_eligible(a, B, CO, CI, G, HW);
     const bool cols = elig && sort_cols_ok(a, kHintSiteBoundSort, B, CO, CI, st);

@@ -1,0 +1,87 @@
+"""The kernels that stream the weights past few batch rows (a wavefront per weight row), against the oracle: values,
+positions and bounds bit for bit, weighted sums at the bar of every sort-neuron test (same products and sums in fp32)."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# batch rows, inputs per group, outputs per group, groups: one input, less than a wavefront, one over and under the
+# register tiles (1024, 3072, 5120, 10240 inputs), rows that are no multiple of four, more wavefronts than weight rows,
+# several slices of the batch rows, groups
+SHAPES = [(1, 1, 1, 1), (2, 5, 3, 1), (3, 63, 9, 1), (4, 64, 4, 1), (5, 1024, 7, 1), (2, 1028, 5, 1), (3, 1025, 6, 1),
+          (2, 3072, 9, 1), (1, 3076, 8, 1), (2, 5120, 3, 1), (2, 5124, 5, 1), (1, 10240, 2, 1), (2, 10239, 3, 1),
+          (17, 200, 33, 1), (6, 130, 10, 3), (70, 96, 5, 2)]
+KINDS = ["normal", "ties", "undefined"]
+
+
+def _data(shape, kind):
+    B, n, m, G = shape
+    g = torch.Generator().manual_seed(B * 31 + n + m)
+    if kind == "ties":
+        x = torch.randint(0, 4, (B, n * G, 1), generator=g).float()
+        w = torch.randint(0, 4, (m * G, n), generator=g).float()
+    else:
+        x, w = torch.randn(B, n * G, 1, generator=g), torch.randn(m * G, n, generator=g)
+    if kind == "undefined":
+        x[torch.rand(x.shape, generator=g) < 0.02] = float("nan")
+        w[torch.rand(w.shape, generator=g) < 0.02] = float("nan")
+        w[torch.rand(w.shape, generator=g) < 0.01] = float("inf")
+    return x, w
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_streamed_layers_match_oracle(oracle, shape, kind):
+    from sortnet_amd import _lib, ext
+    B, n, m, G = shape
+    x, w = _data(shape, kind)
+    xd, wd = x.cuda(), w.cuda()
+    new = lambda: torch.empty(B, m * G, 1, device="cuda")                     # noqa: E731
+    newi = lambda: torch.empty(B, m * G, 1, device="cuda", dtype=torch.int32)  # noqa: E731
+    y, y2, p, p2 = new(), new(), newi(), newi()
+
+    def streamed():
+        assert _lib.last_forward_kernel().startswith("row_stream_kernel"), _lib.last_forward_kernel()
+
+    def same(got, ref):
+        assert np.array_equal(got.cpu().numpy(), np.asarray(ref).reshape(tuple(got.shape)), equal_nan=True)
+
+    ry, rp = oracle.inf_dist_forward(x.numpy(), w.numpy(), groups=G)
+    ext.inf_dist_forward_nograd(xd, wd, y, G)
+    streamed()
+    same(y, ry)
+    ext.inf_dist_forward(xd, wd, y, p, G)
+    streamed()
+    same(y, ry)
+    same(p, rp)
+    ry, rp = oracle.masked_inf_dist_forward(x.numpy(), w.numpy(), 0.4, 11, oracle.MASK_FACTORED, groups=G)
+    ext.masked_inf_dist_forward(xd, wd, y, p, G, 0.4, 11, ext.MASK_FACTORED)
+    streamed()
+    same(y, ry)
+    same(p, rp)
+    lo, up = x - 0.1, x + 0.2
+    up[:, ::7] = lo[:, ::7] - 0.05                                           # inverted intervals
+    rl, ru, rpl, rpu = oracle.bound_inf_dist_forward(lo.numpy(), up.numpy(), w.numpy(), groups=G)
+    ext.bound_inf_dist_forward_nograd(lo.cuda(), up.cuda(), wd, y, y2, G)
+    streamed()
+    same(y, rl)
+    same(y2, ru)
+    ext.bound_inf_dist_forward(lo.cuda(), up.cuda(), wd, y, y2, p, p2, G)
+    streamed()
+    same(y, rl)
+    same(y2, ru)
+    same(p, rpl)
+    same(p2, rpu)
+    for K in sorted({2, min(n, 10), min(n, 25)}):
+        if K < 2 or K > n:
+            continue
+        ref = oracle.sort_neuron_forward(x.numpy(), w.numpy(), 0.6, K, groups=G, need_pos=False)
+        ext.sort_neuron_forward_nograd(xd, wd, y, G, 0.6, K)
+        if B * m * G <= 80 * n:
+            streamed()
+        np.testing.assert_allclose(y.cpu().numpy(), ref.reshape(B, m * G, 1), rtol=1e-5, atol=1e-6)
+        rl, ru = oracle.bound_sort_neuron_forward(lo.numpy(), up.numpy(), w.numpy(), 0.6, K, groups=G)
+        ext.bound_sort_neuron_forward(lo.cuda(), up.cuda(), wd, y, y2, G, 0.6, K)
+        np.testing.assert_allclose(y.cpu().numpy(), rl.reshape(B, m * G, 1), rtol=1e-5, atol=1e-6)
+        np.testing.assert_allclose(y2.cpu().numpy(), ru.reshape(B, m * G, 1), rtol=1e-5, atol=1e-6)
