@@ -55,7 +55,33 @@ inline int pick_nsplit(const FwdArgs& a, int BB, int BM, int per_cu = 8) {
     if (max_ns > 16) max_ns = 16;
     int ns = 1;
     while (ns * 2 <= max_ns && tiles * ns < want) ns *= 2;
+    // Where that leaves compute units idle the slices go down to one chunk, until every unit has two workgroups (one
+    // for the gather kernels): a workgroup of so small a problem waits on its chunks, one after the other, and the
+    // merge of the slices is a few microseconds at most.  In us, four-chunk slices -> this, with narrow tiles below:
+    // l-p at p = 8 on 32 x 784 x 256 40 -> 15, on 90 x 1600 x 230 41 -> 18; l-inf with positions 26 -> 10, 26 -> 17;
+    // interval bounds on 256 x 10240 x 200 103 -> 68.  Four workgroups per unit were slower from 128 x 3072 x 1024 on
+    // (l-inf 27 -> 33), one per unit below (p = 8 on 90 x 1600 x 230 18 -> 27).
+    const long long fill = (per_cu > 1 ? 2ll : 1ll) * num_cus();
+    if (tiles * ns < fill && aligned16(a.y0) && aligned16(a.y1)) {   // (a merge by maximum starts from filled outputs)
+        long long more = (fill + tiles - 1) / tiles;
+        if (more > chunks) more = chunks;
+        if (more > 64) more = 64;
+        if (more > ns) ns = (int)more;
+    }
     return ns;
+}
+
+// Whether the forward runs on tiles of 32 x 32 outputs (2 x 2 per work-item) instead of 32 or 64 x 64 or 128: up to as
+// many chunks of 32 x 128 outputs as 32 per compute unit.  The narrow tile reads more LDS per term but pads less, fills
+// the device with fewer slices and keeps more wavefronts in flight.  In us, wide -> narrow: l-inf on 300 x 1001 x 777
+// (21 chunks per unit) 31 -> 20, on 250 x 3072 x 1021 (24) 45 -> 41 and with positions 67 -> 54, interval bounds with
+// positions 137 -> 107; p = 100 on 40 x 5000 x 2000 (20) 265 -> 199; the one loss seen is 7 % (interval bounds,
+// 256 x 10240 x 200).  Larger layers keep the wide tiles, whose LDS traffic per term decides there.  What the gather kernel
+// serves goes narrow up to twice that size: its wide tile holds fewer wavefronts than the vector kernels' (512 rows of four
+// positions, 2700 inputs, 1024 channels (42): forward, backward and unfolding 184 -> 159).
+inline bool narrow_tiles(const FwdArgs& a) {
+    const long long tiles = (long long)((a.R + 31) / 32) * ((a.COg + 127) / 128) * a.G;
+    return tiles * ((a.CIg + 31) / 32) < (a.fast_x && a.fast_w ? 32ll : 64ll) * num_cus();
 }
 
 // rows per work-item (batch tile = 16 * TB rows): the largest candidate whose tiles, after split-N,

@@ -1247,15 +1247,15 @@ __device__ __forceinline__ uint32_t chunk_keep_bits(const FwdArgs& a, long long 
 // LISTS: the layer has kept-input index lists.  Without them an input's column is its number, and no load stands
 // between the two operand loads of one output and those of the next, so that a wavefront has them all in flight.
 template <bool PACKED, bool LISTS>
-__global__ void __launch_bounds__(256) resolve_pos_kernel(FwdArgs a) {
+__global__ void __launch_bounds__(256) resolve_pos_kernel(FwdArgs a, int per) {
     if (gate_closed(a.gate, a.gate_limit, a.gate_above)) return;   // one of two queued for the result
     __shared__ __attribute__((aligned(16))) ResolveSlot slots[4][64];
     const long long total = (long long)a.R * a.G * a.COg;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const long long o_base = ((long long)blockIdx.x * 4 + wave) * 64;
+    const long long o_base = ((long long)blockIdx.x * 4 + wave) * per;
     if (o_base >= total) return;                       // whole wavefront; no workgroup barrier below
     const long long o = o_base + lane;
-    const bool mine = o < total;
+    const bool mine = lane < per && o < total;
     ResolveSlot me;
     me.cid = -1; me.best = kEps; me.xoff = me.woff = me.coff = 0; me.keep = 0u; me.pad0 = me.pad1 = 0;
     if (mine) {
@@ -1286,7 +1286,7 @@ __global__ void __launch_bounds__(256) resolve_pos_kernel(FwdArgs a) {
     constexpr int U = 8;
     const int half = lane >> 5, l = lane & 31;
     int pos = 0;
-    for (int it0 = 0; it0 < 32; it0 += U) {
+    for (int it0 = 0; it0 < per / 2; it0 += U) {
         float d[U];
         bool cand[U];
         float best[U];
@@ -1327,15 +1327,15 @@ __global__ void __launch_bounds__(256) resolve_pos_kernel(FwdArgs a) {
 struct ResolveBoundSlot { int cl, cu; float vl, vu; unsigned long long xoff, woff; };
 
 template <bool PACKED>
-__global__ void __launch_bounds__(256) resolve_bound_kernel(FwdArgs a) {
+__global__ void __launch_bounds__(256) resolve_bound_kernel(FwdArgs a, int per) {
     __shared__ __attribute__((aligned(16))) ResolveBoundSlot slots[4][64];
     if (a.resolved != nullptr && *a.resolved != 0ull) return;   // (uniform over the launch)
     const long long total = (long long)a.R * a.G * a.COg;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const long long o_base = ((long long)blockIdx.x * 4 + wave) * 64;
+    const long long o_base = ((long long)blockIdx.x * 4 + wave) * per;
     if (o_base >= total) return;                       // whole wavefront; no workgroup barrier below
     const long long o = o_base + lane;
-    const bool mine = o < total;
+    const bool mine = lane < per && o < total;
     ResolveBoundSlot me;
     me.cl = me.cu = -1; me.vl = me.vu = kEps; me.xoff = me.woff = 0ull;
     if (mine) {
@@ -1359,7 +1359,7 @@ __global__ void __launch_bounds__(256) resolve_bound_kernel(FwdArgs a) {
     const int half = lane >> 5, l = lane & 31;
     uint32_t posl = kNanId, posu = 0u;
     constexpr int U = 4;
-    for (int it0 = 0; it0 < 32; it0 += U) {
+    for (int it0 = 0; it0 < per / 2; it0 += U) {
         float t1[U][2], t2[U][2], target[U][2];
         bool cand[U][2];
         int nn[U][2];
@@ -1406,23 +1406,33 @@ __global__ void __launch_bounds__(256) resolve_bound_kernel(FwdArgs a) {
     }
 }
 
+// Outputs of a wavefront: 64, or so few that a small result still gives every SIMD a wavefront (a step of the walk is
+// two dependent trips to memory, and 64 outputs take four to eight of them)
+inline int resolve_per_wave(long long total, int fewest) {
+    int per = 64;
+    while (per > fewest && total < (long long)per * 4 * num_cus()) per /= 2;
+    return per;
+}
+
 inline int launch_resolve_bound(const FwdArgs& a, hipStream_t stream) {
     long long total = (long long)a.R * a.G * a.COg;
-    dim3 grid((unsigned)((total + 255) / 256));
-    if (a.nsplit > 1) hipLaunchKernelGGL((resolve_bound_kernel<true>), grid, dim3(256), 0, stream, a);
-    else hipLaunchKernelGGL((resolve_bound_kernel<false>), grid, dim3(256), 0, stream, a);
+    const int per = resolve_per_wave(total, 16);
+    dim3 grid((unsigned)((total + 4 * per - 1) / (4 * per)));
+    if (a.nsplit > 1) hipLaunchKernelGGL((resolve_bound_kernel<true>), grid, dim3(256), 0, stream, a, per);
+    else hipLaunchKernelGGL((resolve_bound_kernel<false>), grid, dim3(256), 0, stream, a, per);
     return check_launch("resolve_bound_kernel");
 }
 
 inline int launch_resolve(const FwdArgs& a, hipStream_t stream) {
     long long total = (long long)a.R * a.G * a.COg;
-    dim3 grid((unsigned)((total + 255) / 256));
+    const int per = resolve_per_wave(total, 16);
+    dim3 grid((unsigned)((total + 4 * per - 1) / (4 * per)));
     if (a.ci_idx) {
-        if (a.nsplit > 1) hipLaunchKernelGGL((resolve_pos_kernel<true, true>), grid, dim3(256), 0, stream, a);
-        else hipLaunchKernelGGL((resolve_pos_kernel<false, true>), grid, dim3(256), 0, stream, a);
+        if (a.nsplit > 1) hipLaunchKernelGGL((resolve_pos_kernel<true, true>), grid, dim3(256), 0, stream, a, per);
+        else hipLaunchKernelGGL((resolve_pos_kernel<false, true>), grid, dim3(256), 0, stream, a, per);
     } else {
-        if (a.nsplit > 1) hipLaunchKernelGGL((resolve_pos_kernel<true, false>), grid, dim3(256), 0, stream, a);
-        else hipLaunchKernelGGL((resolve_pos_kernel<false, false>), grid, dim3(256), 0, stream, a);
+        if (a.nsplit > 1) hipLaunchKernelGGL((resolve_pos_kernel<true, false>), grid, dim3(256), 0, stream, a, per);
+        else hipLaunchKernelGGL((resolve_pos_kernel<false, false>), grid, dim3(256), 0, stream, a, per);
     }
     return check_launch("resolve_pos_kernel");
 }

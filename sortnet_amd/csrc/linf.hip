@@ -148,9 +148,14 @@ template <class P>
 static int run_chunk_pos(FwdArgs& a, bool index_lists, hipStream_t st, void* merge_buf = nullptr, size_t merge_cap = 0) {
     // with index lists a batch tile must stay inside one 32-sample sub-batch
     static const int kTb42[] = {4, 2};
-    const int TB = index_lists ? 2 : pick_tb(a, kTb42, 2, 16 * P::WIDE_TM);
-    const bool gather = index_lists && !(a.fast_x && a.fast_w);      // served by the scalar-load kernel
-    a.nsplit = TB == 2 ? pick_nsplit(a, 32, gather ? 128 : 16 * P::WIDE_TM, gather ? 1 : 8) : pick_nsplit(a, 16 * P::WIDE_TB, 16 * P::WIDE_TM);
+    const bool narrow = narrow_tiles(a);
+    // served by the scalar-load kernel, which the layers with several positions and rows that are no multiple of 16
+    // bytes take as well as the index lists (512 rows of 4 positions x 5120 x 2560: 490 -> 393 us against fwd_kernel,
+    // which loads a chunk only when the one before it is done)
+    const bool gather = P::LISTS && (index_lists || a.mask_mode < 0) && !(a.fast_x && a.fast_w);
+    const int TB = index_lists || narrow || gather ? 2 : pick_tb(a, kTb42, 2, 16 * P::WIDE_TM);
+    if (narrow) a.nsplit = pick_nsplit(a, 32, 32);
+    else a.nsplit = TB == 2 ? pick_nsplit(a, 32, gather ? 128 : 16 * P::WIDE_TM, gather && index_lists ? 1 : 8) : pick_nsplit(a, 16 * P::WIDE_TB, 16 * P::WIDE_TM);
     // dense exact tiles of the l-inf policy: LDS-direct kernel with 4 x 8 outputs per work-item and the chunk numbers
     // packed four to a register (same (value, chunk) results, so the same resolve pass follows)
     bool packed_direct = false;
@@ -178,6 +183,7 @@ static int run_chunk_pos(FwdArgs& a, bool index_lists, hipStream_t st, void* mer
         rc = launch_fwd_direct<LinfChunkPacked, 4, 8>(a, st);
         forward_kernel_timer(st, true);
     }
+    else if (narrow) rc = launch_fwd<P, 2, 2>(a, st);
     else if (TB == 2) rc = gather ? launch_fwd<P, 2, 8>(a, st) : launch_fwd<P, 2, P::WIDE_TM>(a, st);
     else rc = launch_fwd<P, P::WIDE_TB, P::WIDE_TM>(a, st);
     if (rc) return rc;
@@ -196,8 +202,9 @@ extern "C" int sd_inf_dist_forward_nograd(const float* input, const float* weigh
     const bool streamed = g_linf_density.load(std::memory_order_relaxed) <= 0.f;   // not where tables are forced
     if (streamed && row_stream_ok(a, kStreamMaxTerms)) return row_stream_linf(a, st);
     static const int kTb42[] = {4, 2};   // 8 rows per work-item measured slower (168 registers, three waves per SIMD)
-    const int TB = pick_tb(a, kTb42, 2, 128);
-    a.nsplit = pick_nsplit(a, 16 * TB, 128);
+    const bool narrow = narrow_tiles(a);
+    const int TB = narrow ? 2 : pick_tb(a, kTb42, 2, 128);
+    a.nsplit = pick_nsplit(a, 16 * TB, narrow ? 32 : 128);
     if (a.nsplit > 1 && (rc = fill_zero(output, (size_t)B * CO * HW, st))) return rc;
     const int KE = max_cols_eligible(a, 1.f, B, CO, CI, G, HW);
     const int K = max_cols_wanted(a, KE, kHintSiteLinf, B, CO, CI, st);
@@ -206,7 +213,7 @@ extern "C" int sd_inf_dist_forward_nograd(const float* input, const float* weigh
         if (!ws) return SD_ERR_HIP;
         if (K && (rc = queue_max_cols(a, K, B, CO, CI, ws, st))) return rc;
     }
-    rc = TB == 2 ? launch_fwd<LinfNograd, 2, 8>(a, st) : launch_fwd<LinfNograd, 4, 8>(a, st);
+    rc = narrow ? launch_fwd<LinfNograd, 2, 2>(a, st) : TB == 2 ? launch_fwd<LinfNograd, 2, 8>(a, st) : launch_fwd<LinfNograd, 4, 8>(a, st);
     if (K && rc == SD_OK) max_cols_report(a, kHintSiteLinf, B, CO, CI, st);
     return rc;
 }
@@ -346,11 +353,12 @@ extern "C" int sd_masked_inf_dist_forward(const float* input, const float* weigh
         return rc;
     }
     static const int kTb42[] = {4, 2};   // 8 rows per work-item measured slower (168 registers, three waves per SIMD)
-    const int TB = pick_tb(a, kTb42, 2, 128);
-    a.nsplit = pick_nsplit(a, 16 * TB, 128);
+    const bool narrow = narrow_tiles(a);
+    const int TB = narrow ? 2 : pick_tb(a, kTb42, 2, 128);
+    a.nsplit = pick_nsplit(a, 16 * TB, narrow ? 32 : 128);
     if (a.nsplit > 1 && (rc = fill_zero(output, (size_t)B * CO * HW, st))) return rc;
     if (K && (rc = queue_max_cols(a, K, B, CO, CI, tables, st))) return rc;
-    rc = TB == 2 ? launch_fwd<LinfNograd, 2, 8>(a, st) : launch_fwd<LinfNograd, 4, 8>(a, st);
+    rc = narrow ? launch_fwd<LinfNograd, 2, 2>(a, st) : TB == 2 ? launch_fwd<LinfNograd, 2, 8>(a, st) : launch_fwd<LinfNograd, 4, 8>(a, st);
     if (K && rc == SD_OK) max_cols_report(a, kHintSiteMasked, B, CO, CI, st);
     return rc;
 }
@@ -369,8 +377,9 @@ extern "C" int sd_bound_inf_dist_forward_nograd(const float* inputL, const float
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (g_bound_density.load(std::memory_order_relaxed) <= 0.f && row_stream_ok(a, kStreamBoundTerms)) return row_stream_bound(a, st);
     static const int kTb42[] = {4, 2};
-    const int TB = pick_tb(a, kTb42, 2, 128);
-    a.nsplit = pick_nsplit(a, 16 * TB, 16 * 8);
+    const bool narrow = narrow_tiles(a);
+    const int TB = narrow ? 2 : pick_tb(a, kTb42, 2, 128);
+    a.nsplit = pick_nsplit(a, 16 * TB, narrow ? 32 : 128);
     // dense single-group layers: a kernel that works from per-weight-row candidate tables is queued in front of the
     // one that evaluates every term, and a count taken on the device decides which of the two runs
     const float bound_density = g_bound_density.load(std::memory_order_relaxed);
@@ -405,7 +414,7 @@ extern "C" int sd_bound_inf_dist_forward_nograd(const float* inputL, const float
                                     bound_density > 0.f ? bound_density : kBoundSparseCap, &a.gate, &a.gate_limit, st)))
             return rc;
         a.gate_above = 1;
-        return TB == 2 ? launch_fwd<BoundNogradGated, 2, 8>(a, st) : launch_fwd<BoundNogradGated, 4, 8>(a, st);
+        return narrow ? launch_fwd<BoundNogradGated, 2, 2>(a, st) : TB == 2 ? launch_fwd<BoundNogradGated, 2, 8>(a, st) : launch_fwd<BoundNogradGated, 4, 8>(a, st);
     }
     if (a.nsplit > 1 || cols) {
         if ((rc = fill_zero2(outputL, (size_t)B * CO * HW, outputU, (size_t)B * CO * HW, st))) return rc;
@@ -416,13 +425,14 @@ extern "C" int sd_bound_inf_dist_forward_nograd(const float* inputL, const float
                                      bound_density >= 0.f ? bound_density : kBoundRowsCap, &a.gate, &a.gate_limit, st)))
             return rc;
         a.gate_above = 1;
-        rc = TB == 2 ? launch_fwd<BoundNogradGated, 2, 8>(a, st) : launch_fwd<BoundNogradGated, 4, 8>(a, st);
+        rc = narrow ? launch_fwd<BoundNogradGated, 2, 2>(a, st) : TB == 2 ? launch_fwd<BoundNogradGated, 2, 8>(a, st) : launch_fwd<BoundNogradGated, 4, 8>(a, st);
         if (hinted && rc == SD_OK) {
             hint_record(kHintSiteBound, weight, B, CO, CI, a.gate, st);   // the gate is 1 when every term ran
             if (bound_form == 0) hint_record(kHintSiteBoundSparse, weight, B, CO, CI, a.gate + 1, st);   // 1: very few marks
         }
         return rc;
     }
+    if (narrow) return launch_fwd<BoundNograd, 2, 2>(a, st);
     if (TB == 2) return launch_fwd<BoundNograd, 2, 8>(a, st);
     return launch_fwd<BoundNograd, 4, 8>(a, st);
 }
@@ -453,8 +463,9 @@ extern "C" int sd_bound_inf_dist_forward(const float* inputL, const float* input
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (g_bound_density.load(std::memory_order_relaxed) <= 0.f && row_stream_ok(a, kStreamBoundPosTerms)) return row_stream_bound(a, st);
     static const int kTb42[] = {4, 2};
-    const int TB = pick_tb(a, kTb42, 2, 64);
-    a.nsplit = pick_nsplit(a, 16 * TB, 64);
+    const bool narrow = narrow_tiles(a);
+    const int TB = narrow ? 2 : pick_tb(a, kTb42, 2, 64);
+    a.nsplit = pick_nsplit(a, 16 * TB, narrow ? 32 : 64);
     // dense single-group layers: the table kernel, tracking the chunk of every result, is queued in front
     // of the every-term kernel as for the forward without positions; both leave (value, chunk) pairs for the resolve
     const float bound_density = g_bound_density.load(std::memory_order_relaxed);
@@ -484,7 +495,7 @@ extern "C" int sd_bound_inf_dist_forward(const float* inputL, const float* input
     // exact dense tiles: the LDS-direct kernel with the chunk numbers packed (same (value, chunk) pairs, same resolve)
     if (TB == 4 && a.nsplit > 1 && direct_ok<4, 4>(a) && (a.CIg / KT + a.nsplit - 1) / a.nsplit <= BoundChunkPacked::MAX_CHUNKS)
         rc = launch_fwd_direct<BoundChunkPacked, 4, 4>(a, st);
-    else rc = TB == 2 ? launch_fwd<BoundChunk, 2, 4>(a, st) : launch_fwd<BoundChunk, 4, 4>(a, st);
+    else rc = narrow ? launch_fwd<BoundChunk, 2, 2>(a, st) : TB == 2 ? launch_fwd<BoundChunk, 2, 4>(a, st) : launch_fwd<BoundChunk, 4, 4>(a, st);
     if (rc) return rc;
     if (hinted && cols) hint_record(kHintSiteBoundPos, weight, B, CO, CI, a.gate, st);   // the gate is 1 when every term ran
     return launch_resolve_bound(a, st);
