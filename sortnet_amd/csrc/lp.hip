@@ -36,6 +36,14 @@ static inline float rows_cap(float builtin, float thr) {
     return thr >= kRowsFromThr ? builtin : 0.f;
 }
 
+// Layers below 2^30 terms go without tables under the built-in limits: the passes that build them take about as long as
+// every term there (normal inputs, p = 24, tables -> none, in us: forward 32 x 192 x 192 35 -> 18, 64 x 1024 x 1024
+// 61 -> 34, 128 x 3072 x 1024 169 -> 110, 250 x 3072 x 1021 264 -> 213; backward of the last 511 -> 476).
+constexpr long long kRowsMinTerms = 1ll << 30;
+static inline bool rows_large(int R, int CO, int CI) {
+    return g_rows_density.load(std::memory_order_relaxed) >= 0.f || (long long)R * CO * CI >= kRowsMinTerms;
+}
+
 static inline int int_power(float p) {
     if (p == (float)(int)p && p >= 0.f && p <= 8.f) return (int)p;
     return -1;
@@ -122,10 +130,12 @@ static int lp_forward_max_first(FwdArgs& a, bool small, hipStream_t st) {
     // is queued in front of the two steps below, and a count taken on the device decides which of the two runs
     const float thr_rows = powf(1e-6f / (float)a.CIg, 1.f / a.p);
     const float cap = rows_cap(a.skip_thr > 0.f ? kRowsCapForwardSkip : kRowsCapForward, thr_rows);
-    const bool rows = cap > 0.f && a.G == 1 && a.HW == 1 && !a.ci_idx && !a.co_idx && a.W_CIg == a.CIg &&
+    const bool rows = cap > 0.f && rows_large(a.R, a.COg, a.CIg) && a.G == 1 && a.HW == 1 && !a.ci_idx &&
+                      !a.co_idx && a.W_CIg == a.CIg &&
                       a.CIg % kRowsChunk == 0 && a.R < (1 << 22) && thr_rows > 0.f && thr_rows < 1.f;
     FwdArgs m = a;
-    m.nsplit = pick_nsplit(m, small ? 32 : 64, 128);
+    const bool narrow = narrow_tiles(a);
+    m.nsplit = pick_nsplit(m, small || narrow ? 32 : 64, narrow ? 32 : 128);
     a.nsplit = m.nsplit;
     const int ns_rows = rows ? lp_rows_forward_nsplit(a.R, a.COg, a.CIg) : 1;
     // maxima, then the slice results of whichever sum kernel runs (the table kernel leaves two values per slice)
@@ -151,15 +161,17 @@ static int lp_forward_max_first(FwdArgs& a, bool small, hipStream_t st) {
     }
     m.y0 = base;
     if (m.nsplit > 1 && (rc = fill_zero(base, total, st))) return rc;
-    if (rows) rc = small ? launch_fwd<LinfNogradGated, 2, 8>(m, st) : launch_fwd<LinfNogradGated, 4, 8>(m, st);
-    else rc = small ? launch_fwd<LinfNograd, 2, 8>(m, st) : launch_fwd<LinfNograd, 4, 8>(m, st);
+    if (rows) rc = narrow ? launch_fwd<LinfNogradGated, 2, 2>(m, st) : small ? launch_fwd<LinfNogradGated, 2, 8>(m, st)
+                                                             : launch_fwd<LinfNogradGated, 4, 8>(m, st);
+    else rc = narrow ? launch_fwd<LinfNograd, 2, 2>(m, st) : small ? launch_fwd<LinfNograd, 2, 8>(m, st)
+                                                             : launch_fwd<LinfNograd, 4, 8>(m, st);
     if (rc) return rc;
     a.aux = base;
     a.part_stride = total;
     a.part0 = a.nsplit > 1 ? base + total : nullptr;
     a.part1 = nullptr;
-    if (a.skip_thr > 0.f) rc = small ? launch_fwd<LpWithMaxSkip, 2, 8>(a, st) : launch_fwd<LpWithMaxSkip, 4, 8>(a, st);
-    else rc = small ? launch_fwd<LpWithMax<-1>, 2, 8>(a, st) : launch_fwd<LpWithMax<-1>, 4, 8>(a, st);
+    if (a.skip_thr > 0.f) rc = narrow ? launch_fwd<LpWithMaxSkip, 2, 2>(a, st) : small ? launch_fwd<LpWithMaxSkip, 2, 8>(a, st) : launch_fwd<LpWithMaxSkip, 4, 8>(a, st);
+    else rc = narrow ? launch_fwd<LpWithMax<-1>, 2, 2>(a, st) : small ? launch_fwd<LpWithMax<-1>, 2, 8>(a, st) : launch_fwd<LpWithMax<-1>, 4, 8>(a, st);
     if (rc) return rc;
     return lp_split_finish(a, st);
 }
@@ -192,7 +204,7 @@ struct LpBwdArgs {
     unsigned long long gate_limit;
     int gate_above;
     const float* ry;                  // 1 / y when the caller already holds it, else null
-    bool gx_is_zero;                  // grad_input was zero-filled by the caller
+    bool gx_is_zero;                  // grad_input (and grad_weight) were zero-filled by the caller
     int zsplit;  // slices of the output-channel range (grad_input then merges with atomic adds)
 };
 
@@ -248,13 +260,19 @@ __device__ __forceinline__ void lp_bwd_channel(const LpBwdArgs& a, const float2 
             }
         }
     } else {
+        // the last batch tile by groups of eight rows and a select per row: straight-line code is what hides the LDS
+        // latency (250 x 3072 x 1021, 26 rows in the last tile, p = 8: 0.36 ms with a branch per row, 0.25 now)
         #pragma unroll
-        for (int i = 0; i < RB; i++) {
-            if (FULL || i < rows) {
-                float2 t = gr[i];
-                float pw = signed_pow<IP>(xr[i] - wk, t.y, a.pm1);
-                acc[i] = fmaf(t.x, pw, acc[i]);
-                wsum = fmaf(t.x, pw, wsum);
+        for (int i0 = 0; i0 < RB; i0 += 8) {
+            if (FULL || i0 < rows) {
+                #pragma unroll
+                for (int i = i0; i < i0 + 8; i++) {
+                    float2 t = gr[i];
+                    float pw = signed_pow<IP>(xr[i] - wk, t.y, a.pm1);
+                    if (!FULL) pw = i < rows ? pw : 0.f;
+                    acc[i] = fmaf(t.x, pw, acc[i]);
+                    wsum = fmaf(t.x, pw, wsum);
+                }
             }
         }
     }
@@ -284,7 +302,9 @@ __device__ __forceinline__ void lp_bwd_chunk(const LpBwdArgs& a, const float2 (&
     }
 }
 
-template <int IP, bool WGRAD, bool SKIP = false>
+// RAGGED: the rows are no multiple of RB.  A kernel of its own: with the code for a part of a tile beside it the code for
+// whole tiles lost 10 to 20 % to the registers (512 x 5120 x 2560, p = 8: 1.17 -> 1.43 ms).
+template <int IP, bool WGRAD, bool SKIP, bool RAGGED>
 __global__ void __launch_bounds__(256, (SKIP ? 4 : 1)) lp_bwd_kernel(LpBwdArgs a) {
     __shared__ float2 gr[2][MC][RB];   // (g, 1/y) of output channel m0+k, row r0+i; two chunks
     if (gate_closed(a.gate, a.gate_limit, a.gate_above)) return;
@@ -362,7 +382,7 @@ __global__ void __launch_bounds__(256, (SKIP ? 4 : 1)) lp_bwd_kernel(LpBwdArgs a
         const float2 pn = pair_of(m0 + MC);
 
         const int mcount = m_hi - m0 < MC ? m_hi - m0 : MC;
-        if (rows == RB) lp_bwd_chunk<IP, WGRAD, SKIP, true>(a, gr[buf], xr, acc, wv, rows, mcount, rowv, n_ok, gwcol);
+        if (!RAGGED || rows == RB) lp_bwd_chunk<IP, WGRAD, SKIP, true>(a, gr[buf], xr, acc, wv, rows, mcount, rowv, n_ok, gwcol);
         else lp_bwd_chunk<IP, WGRAD, SKIP, false>(a, gr[buf], xr, acc, wv, rows, mcount, rowv, n_ok, gwcol);
 
         gr[buf ^ 1][sk][si] = make_float2(pn.x, 1.f / pn.y);   // last read in the previous iteration, before its barrier
@@ -580,18 +600,36 @@ static int launch_lp_bwd(int ip, const LpBwdArgs& a_in, hipStream_t st) {
         const double rounds = (double)blocks * z / slots, eff = rounds / std::ceil(rounds);
         if (eff > best * 1.03) { best = eff; a.zsplit = z; }
     }
+    // small layers: slices down to one chunk of MC channels until every compute unit has two workgroups (p = 8, in us:
+    // 32 x 784 x 256 64 -> 21, 64 x 1024 x 1024 64 -> 37; with four per unit the last is 51)
+    const long long fill = 2ll * num_cus();
+    if (blocks * a.zsplit < fill && aligned16(a.gx)) {   // (slices add to a filled grad_input)
+        const long long more = (fill + blocks - 1) / blocks, most = (a.COg + MC - 1) / MC;
+        a.zsplit = (int)(more < most ? more : most);
+    }
     int rc;
-    if (a.zsplit > 1 && !a.gx_is_zero && (rc = fill_zero(a.gx, (size_t)a.R * a.G * a.CIg, st))) return rc;
+    const size_t nx = a.zsplit > 1 ? (size_t)a.R * a.G * a.CIg : 0, nw = WGRAD ? (size_t)a.G * a.W_COg * a.W_CIg : 0;
+    if (!a.gx_is_zero && nx && nw) rc = fill_zero2(a.gx, nx, a.gw, nw, st);
+    else if (!a.gx_is_zero && nx + nw) rc = nx ? fill_zero(a.gx, nx, st) : fill_zero(a.gw, nw, st);
+    else rc = SD_OK;
+    if (rc) return rc;
     dim3 grid((a.CIg + 255) / 256, (a.R + RB - 1) / RB, a.G * a.zsplit);
-#define SD_CASE(k) case k: hipLaunchKernelGGL((lp_bwd_kernel<k, WGRAD>), grid, dim3(256), 0, st, a); break;
+    const bool ragged = a.R % RB != 0;
+#define SD_LAUNCH(k, skip)                                                                                  \
+    do {                                                                                                    \
+        if (ragged) hipLaunchKernelGGL((lp_bwd_kernel<k, WGRAD, skip, true>), grid, dim3(256), 0, st, a);   \
+        else hipLaunchKernelGGL((lp_bwd_kernel<k, WGRAD, skip, false>), grid, dim3(256), 0, st, a);         \
+    } while (0)
+#define SD_CASE(k) case k: SD_LAUNCH(k, false); break;
     switch (ip) {
         SD_CASE(0) SD_CASE(1) SD_CASE(2) SD_CASE(3) SD_CASE(4) SD_CASE(5) SD_CASE(6) SD_CASE(7) SD_CASE(8)
         default:
-            if (a.skip_thr > 0.f) hipLaunchKernelGGL((lp_bwd_kernel<-1, WGRAD, true>), grid, dim3(256), 0, st, a);
-            else hipLaunchKernelGGL((lp_bwd_kernel<-1, WGRAD>), grid, dim3(256), 0, st, a);
+            if (a.skip_thr > 0.f) SD_LAUNCH(-1, true);
+            else SD_LAUNCH(-1, false);
             break;
     }
 #undef SD_CASE
+#undef SD_LAUNCH
     return check_launch("lp_bwd_kernel");
 }
 
@@ -625,12 +663,14 @@ static int lp_backward(const char* who, const float* grad_output, const float* i
     const float thr_rows = (ip < 0 && a.pm1 > 1.f) ? powf(1e-16f, 1.f / a.pm1) : 0.f;
     bool zero_gx = false;
     // which kernel evaluates every term, and whether it runs its own wave-level tests
-    const bool fused = dense && grad_weight && a.skip_thr >= kLpSkipFromFused;
+    // (and enough workgroups for it: 512 x 600 x 600 at p = 100, 75 of them, took 480 us against 95)
+    const long long fused_groups = (long long)(f.CIg / FN) * ((f.COg + FMR - 1) / FMR);
+    const bool fused = dense && grad_weight && a.skip_thr >= kLpSkipFromFused && fused_groups >= 2 * num_cus();
     const bool tests = fused || a.skip_thr >= kLpSkipFromGeneral;
     const float cap = rows_cap(grad_weight ? (tests ? kRowsCapBackwardSkip : kRowsCapBackward)
                                            : (tests ? kRowsCapBackwardInputSkip : kRowsCapBackwardInput), thr_rows);
-    if (cap > 0.f && dense && thr_rows > 0.f && thr_rows < 1.f && f.CIg % kRowsChunk == 0 && f.W_CIg == f.CIg &&
-        B < (1 << 22)) {
+    if (cap > 0.f && rows_large(f.R, f.COg, f.CIg) && dense && thr_rows > 0.f && thr_rows < 1.f && f.CIg % kRowsChunk == 0 &&
+        f.W_CIg == f.CIg && B < (1 << 22)) {
         void* ws = workspace(lp_rows_workspace(f.R, f.COg, f.CIg) + (size_t)f.R * f.COg * sizeof(float), st);
         if (!ws) return SD_ERR_HIP;
         // the general kernel adds to a zero-filled grad_weight, which the table kernel must not find cleared after it ran
@@ -640,14 +680,10 @@ static int lp_backward(const char* who, const float* grad_output, const float* i
         a.gate_above = 1;
         zero_gx = true;
     }
-    if (dense && grad_weight && a.skip_thr >= kLpSkipFromFused) return launch_lp_bwd_fused(ip, a, st);
+    if (fused) return launch_lp_bwd_fused(ip, a, st);
     if (a.skip_thr < kLpSkipFromGeneral) a.skip_thr = 0.f;
     a.gx_is_zero = zero_gx;
-    if (grad_weight) {
-        if (!zero_gx && (rc = fill_zero(grad_weight, (size_t)G * f.W_COg * f.W_CIg, st))) return rc;
-        return launch_lp_bwd<true>(ip, a, st);
-    }
-    return launch_lp_bwd<false>(ip, a, st);
+    return grad_weight ? launch_lp_bwd<true>(ip, a, st) : launch_lp_bwd<false>(ip, a, st);
 }
 
 }  // namespace sd
@@ -674,7 +710,9 @@ extern "C" int sd_norm_dist_forward(const float* input, const float* weight,
     a.y0 = output; a.p = p; a.inv_p = 1.f / p;
     hipStream_t st = static_cast<hipStream_t>(stream);
     static const int kTb42[] = {4, 2};
-    const bool small = w_index_ci || w_index_co || pick_tb(a, kTb42, 2, 128) == 2;
+    const bool narrow = narrow_tiles(a) && p <= 10.f;
+    const bool small = w_index_ci || w_index_co || narrow || pick_tb(a, kTb42, 2, 128) == 2 ||
+                       !(a.fast_x && a.fast_w);   // (these take the scalar-load kernel, built for 32 rows)
     const bool online = p > 10.f;   // core/cuda/norm_dist.cpp:4,51-55
     const bool lists = w_index_ci || w_index_co;
     // p > 10: the exact maximum per output first, then one pass of sums relative to it.  On the vector path, and with
@@ -683,10 +721,10 @@ extern "C" int sd_norm_dist_forward(const float* input, const float* weight,
     const bool max_first = online && ((a.fast_x && a.fast_w && !w_index_co) || (lists && a.HW == 1));
     a.skip_thr = lp_skip_threshold(1e-6f / (float)a.CIg, p, max_first ? kLpSkipFrom : kLpSkipFromOnline);
     if (max_first) return lp_forward_max_first(a, small, st);
-    if ((rc = lp_split_setup(a, small ? 32 : 64, 128, online, st))) return rc;
+    if ((rc = lp_split_setup(a, small ? 32 : 64, narrow ? 32 : 128, online, st))) return rc;
     if (!online) {
         int ip = int_power(p);
-        rc = small ? launch_lp<LpPlain, 2, 8>(ip, a, st) : launch_lp<LpPlain, 4, 8>(ip, a, st);
+        rc = narrow ? launch_lp<LpPlain, 2, 2>(ip, a, st) : small ? launch_lp<LpPlain, 2, 8>(ip, a, st) : launch_lp<LpPlain, 4, 8>(ip, a, st);
     } else {
         if (a.skip_thr > 0.f) rc = small ? launch_fwd<LpOnlineSkip, 2, 8>(a, st) : launch_fwd<LpOnlineSkip, 4, 8>(a, st);
         else rc = small ? launch_fwd<LpOnline<-1>, 2, 8>(a, st) : launch_fwd<LpOnline<-1>, 4, 8>(a, st);
