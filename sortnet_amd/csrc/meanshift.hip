@@ -122,6 +122,82 @@ __global__ void __launch_bounds__(256) index_shift_kernel(const float* __restric
     y[i] = x[i] - mean[g * Cg + index[(size_t)(s * G + g) * cnt + j]];
 }
 
+// The three kernels above and the fill of their sums in one launch, for one position per sample.  A workgroup owns 64 full
+// channels of a group; its wavefronts take a sub-batch each (up to 16 at a time).  A wavefront reads its list once and
+// notes in LDS where each of the 64 channels stands in it (lists in any order), a lane then sums its channel's rows in
+// sample order and the sub-batches are added in order: the same bits as above.  The rows are read a second time, from
+// cache, for the shift.  Four launches of 4 to 7 us each were bound by their launches: 32 x 192 of 256 channels
+// 24 -> 6 us, 128 x 3840 of 5120 24 -> 12 us, 512 x 3840 of 5120 23 both ways.
+constexpr int kFuseWaves = 16, kFuseSubs = 128;   // sub-batches at a time / at most (their positions are held in LDS)
+__global__ void __launch_bounds__(64 * kFuseWaves) index_mean_shift_kernel(
+    const float* __restrict__ x, const int* __restrict__ index, int B, int G, int cnt, int Cg, int S,
+    float* __restrict__ mean, float* __restrict__ running, float momentum, float* __restrict__ y) {
+    extern __shared__ int at[];                       // [S][64]: position of the channel in the sub-batch's list, or -1
+    __shared__ float sums[kFuseWaves][64];
+    __shared__ float shift[64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    const int g = blockIdx.y, c0 = blockIdx.x * 64, c = c0 + lane;
+    const size_t stride = (size_t)G * cnt;
+    // what a lane reads next may have been written by another lane of its wavefront
+    auto posted = []() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    float total = 0.f, seen = 1e-10f;                 // of wavefront 0
+    for (int s0 = 0; s0 < S; s0 += waves) {
+        const int s = s0 + wave;
+        float t = 0.f;
+        if (s < S) {
+            int* slot = at + s * 64;
+            slot[lane] = -1;
+            posted();
+            const int* list = index + (size_t)(s * G + g) * cnt;
+            #pragma unroll 8
+            for (int j = lane; j < cnt; j += 64) {
+                const int k = list[j] - c0;
+                if (k >= 0 && k < 64) slot[k] = j;
+            }
+            posted();
+            const int j = slot[lane];
+            if (j >= 0) {
+                const int b0 = s * kSubBatch, b1 = b0 + kSubBatch < B ? b0 + kSubBatch : B;
+                const float* src = x + (size_t)g * cnt + j;
+                #pragma unroll 8
+                for (int b = b0; b < b1; b++) t += src[b * stride];
+            }
+        }
+        sums[wave][lane] = t;
+        __syncthreads();
+        if (wave == 0) {
+            for (int k = 0; k < waves && s0 + k < S; k++) {
+                const int b0 = (s0 + k) * kSubBatch, b1 = b0 + kSubBatch < B ? b0 + kSubBatch : B;
+                total += sums[k][lane];
+                seen += at[(s0 + k) * 64 + lane] >= 0 ? (float)(b1 - b0) : 0.f;
+            }
+        }
+        __syncthreads();
+    }
+    if (wave == 0) {
+        const float m = total / seen;
+        shift[lane] = m;
+        if (c < Cg) {
+            mean[g * Cg + c] = m;
+            if (running) running[g * Cg + c] = (1.f - momentum) * running[g * Cg + c] + momentum * m;
+        }
+    }
+    __syncthreads();
+    const float m = shift[lane];
+    for (int s = wave; s < S; s += waves) {
+        const int j = at[s * 64 + lane];
+        if (j < 0) continue;
+        const int b0 = s * kSubBatch, b1 = b0 + kSubBatch < B ? b0 + kSubBatch : B;
+        const size_t o = (size_t)g * cnt + j;
+        #pragma unroll 8
+        for (int b = b0; b < b1; b++) y[o + b * stride] = x[o + b * stride] - m;
+    }
+}
+
 static int check_dims(const char* who, int B, int C, int HW) {
     SD_REQUIRE(B > 0 && C > 0 && HW > 0, "%s: sizes must be positive", who);
     SD_REQUIRE((long long)B * C * HW < (1ll << 31), "%s: tensor too large for 32-bit indexing", who);
@@ -175,6 +251,12 @@ extern "C" int sd_mean_shift_index_forward(const float* input, const int* index,
     SD_REQUIRE(input && index && mean && output, "mean_shift_index_forward: null pointer");
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int S = (B + kSubBatch - 1) / kSubBatch, C = G * Cg;
+    if (HW == 1 && S <= kFuseSubs && G < 65536) {
+        const int waves = S < kFuseWaves ? S : kFuseWaves;
+        hipLaunchKernelGGL(index_mean_shift_kernel, dim3((Cg + 63) / 64, G), dim3(64 * waves), (size_t)S * 64 * sizeof(int), st,
+                           input, index, B, G, cnt, Cg, S, mean, running_mean, momentum, output);
+        return check_launch("index_mean_shift_kernel");
+    }
     float* part = static_cast<float*>(workspace((size_t)2 * S * C * sizeof(float), st));
     if (!part) return SD_ERR_HIP;
     float* rows = part + (size_t)S * C;
