@@ -244,8 +244,10 @@ struct BoundNode : Node {
         const Tensor gu = grads[1].defined() ? grads[1].contiguous() : at::zeros(posu.sizes(), l.options());
         const c10::DeviceGuard guard(l.device());
         const int B = (int)gl.size(0), CO = (int)gl.size(1), HW = (int)gl.size(2), CI = (int)l.size(1);
-        if (!want_w && !(want_l && want_u)) {
-            // one input alone gets no gradient from this op (core/norm_dist.py:157-173: zeros)
+        // One bound alone, with a frozen weight, gets no gradient from this op (core/norm_dist.py:157-173: zeros).  What
+        // counts is which inputs require a gradient (should_compute_output: the graph's edges), not which of them this
+        // backward pass asks for (task_should_compute_output).
+        if (!should_compute_output(2) && !(should_compute_output(0) && should_compute_output(1))) {
             if (want_l) out[0] = at::zeros_like(l);
             if (want_u) out[1] = at::zeros_like(u);
             return out;

@@ -1,0 +1,86 @@
+"""Graph nodes of the native front-end: gradients with respect to any subset of the inputs."""
+import itertools
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _op(name):
+    """(inputs, function of them): the inputs are leaves that require gradients, the function returns the outputs that
+    gradients flow from."""
+    from sortnet_amd import ext
+    from sortnet_amd import functional as F
+    g = torch.Generator().manual_seed(5)
+    B, n, m = 70, 96, 40
+    x, w = torch.randn(B, n, 1, generator=g).cuda(), torch.randn(m, n, generator=g).cuda()
+    if name.startswith("norm_dist "):
+        p = float(name.split()[1])
+        return [x, w], lambda x, w: [F.norm_dist(x, w, p)]
+    if name.startswith("lists "):
+        p = float(name.split()[1])
+        keep = lambda c, k: torch.rand(3, 1, c, generator=g).argsort(-1)[..., :k].sort(-1)[0].to(torch.int32).cuda()   # noqa: E731
+        ci, co = keep(n, 64), keep(m, 30)
+        return [x[:, :64].contiguous(), w], lambda x, w: [F.norm_dist_dropout(x, w, ci, co, p)]
+    if name == "sort_neuron":
+        return [x, w], lambda x, w: [F.sort_neuron(x, w, q=0.6)]
+    if name == "masked_inf_dist":
+        return [x, w], lambda x, w: [F.masked_inf_dist(x, w, 0.5, 3)]
+    if name == "bound_inf_dist":
+        return [x - 0.1, x + 0.1, w], lambda l, u, w: list(F.bound_inf_dist(l, u, w))
+    if name == "mean_shift":
+        return [x], lambda x: [F.mean_shift(x)[0]]
+    if name == "mean_shift_index":
+        index = torch.rand(3, 1, 130, generator=g).argsort(-1)[..., :n].to(torch.int32).cuda()
+        return [x], lambda x: [F.mean_shift_index(x, index, 130)[0]]
+    assert name == "unfold"
+    return [torch.randn(5, 3, 9, 7, generator=g).cuda()], lambda x: [ext.host().unfold(x, 3, 2, 1, 1, 2)]
+
+
+OPS = ["norm_dist inf", "norm_dist 3", "norm_dist 24", "lists inf", "lists 8", "sort_neuron", "masked_inf_dist", "bound_inf_dist",
+       "mean_shift", "mean_shift_index", "unfold"]
+
+
+def _graph(name):
+    inputs, fn = _op(name)
+    inputs = [t.requires_grad_() for t in inputs]
+    outs = fn(*inputs)
+    g = torch.Generator().manual_seed(6)
+    return inputs, outs, [torch.randn(o.shape, generator=g).cuda() for o in outs]
+
+
+def _close(a, b):
+    # the same addends in another order (gradients merge by fp32 additions in memory)
+    assert a.shape == b.shape and (a - b).norm() <= 1e-5 * b.norm()
+
+
+@pytest.mark.parametrize("name", OPS)
+def test_gradients_of_any_subset_of_the_inputs(name):
+    inputs, outs, gys = _graph(name)
+    torch.autograd.backward(outs, gys, retain_graph=True)
+    full = [t.grad for t in inputs]
+    assert all(t is not None and t.norm() > 0 for t in full)
+    for k in range(1, len(inputs) + 1):
+        for subset in itertools.combinations(range(len(inputs)), k):
+            got = torch.autograd.grad(outs, [inputs[i] for i in subset], gys, retain_graph=True)
+            for i, t in zip(subset, got):
+                _close(t, full[i])
+
+
+@pytest.mark.parametrize("wanted", [w for w in itertools.product([False, True], repeat=3) if any(w)])
+def test_bound_gradients_by_what_requires_them(wanted):
+    """One bound alone, with a frozen weight, gets zeros (core/norm_dist.py:157-173); every other set gets its gradients, also
+    when only a part of it is asked for."""
+    from sortnet_amd import functional as F
+    inputs, outs, gys = _graph("bound_inf_dist")
+    full = torch.autograd.grad(outs, inputs, gys)
+    some = [t.detach().clone().requires_grad_(r) for t, r in zip(inputs, wanted)]
+    outs = F.bound_inf_dist(*some)
+    for i, t in enumerate(some):
+        if wanted[i]:
+            got, = torch.autograd.grad(outs, [t], gys, retain_graph=True)
+            if sum(wanted) == 1 and not wanted[2]:
+                assert got.shape == t.shape and not got.any()
+            else:
+                _close(got, full[i])
