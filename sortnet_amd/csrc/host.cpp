@@ -14,6 +14,7 @@
 #include <ATen/ATen.h>
 #include <ATen/core/grad_mode.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
@@ -64,6 +65,17 @@ struct Dims {
 Tensor new_floats(const Tensor& like, at::IntArrayRef size) { return at::empty(size, like.options().dtype(at::kFloat)); }
 Tensor new_ints(const Tensor& like, at::IntArrayRef size) { return at::empty(size, like.options().dtype(at::kInt)); }
 Tensor new_out(const Tensor& x, int64_t channels) { return new_floats(x, {x.size(0), channels, x.size(2)}); }
+
+// The nodes below hold backward formulas and nothing else.  An input with a forward-mode tangent would come out without
+// one, which a caller reads as a zero derivative, and the kernels know nothing of the wrapped tensors of torch.func: both
+// are refused, as an autograd function without `jvp` and `setup_context` refuses them.
+template <class... T>
+void reverse_mode_only(const char* who, const T&... t) {
+    if (c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode))   // inside a transform
+        throw std::runtime_error(std::string("sortnet_amd.") + who + " does not support the transforms of torch.func (vmap, grad, jvp, ...)");
+    TORCH_CHECK_NOT_IMPLEMENTED(!(... || (t.defined() && t._fw_grad(0).defined())),
+                                "sortnet_amd.", who, " does not support forward mode AD: an input carries a tangent");
+}
 
 template <class... T>
 bool want_grad(const T&... t) { return at::GradMode::is_enabled() && (t.requires_grad() || ...); }
@@ -139,6 +151,7 @@ std::shared_ptr<DistNode> attach(const Tensor& x, const Tensor& w, int64_t group
 
 Tensor norm_dist_lists(const Tensor& x, const Tensor& w, const OptTensor& ci, const OptTensor& co, int64_t groups, double p,
                        bool lists) {
+    reverse_mode_only("norm_dist", x, w);
     const bool grad = want_grad(x, w);
     const int64_t channels = co && co->defined() ? co->size(-1) * groups : w.size(0);
     Tensor y, pos;
@@ -182,6 +195,7 @@ Tensor norm_dist_dropout(const Tensor& x, const Tensor& w, const OptTensor& ci, 
 }
 
 Tensor masked_inf_dist(const Tensor& x, const Tensor& w, int64_t groups, double q, uint32_t seed, int mode) {
+    reverse_mode_only("masked_inf_dist", x, w);
     const bool grad = want_grad(x, w);
     Tensor y, pos;
     {
@@ -203,6 +217,7 @@ Tensor masked_inf_dist(const Tensor& x, const Tensor& w, int64_t groups, double 
 }
 
 Tensor sort_neuron(const Tensor& x, const Tensor& w, int64_t groups, double q, int truncate) {
+    reverse_mode_only("sort_neuron", x, w);
     const bool grad = want_grad(x, w);
     Tensor y, pos;
     {
@@ -275,6 +290,7 @@ struct BoundNode : Node {
 };
 
 std::pair<Tensor, Tensor> bound_inf_dist(const Tensor& xl, const Tensor& xu, const Tensor& w, int64_t groups) {
+    reverse_mode_only("bound_inf_dist", xl, xu, w);
     const bool grad = want_grad(xl, xu, w);
     Tensor lo, up, pl, pu;
     {
@@ -306,6 +322,7 @@ std::pair<Tensor, Tensor> bound_inf_dist(const Tensor& xl, const Tensor& xu, con
 
 std::pair<Tensor, Tensor> bound_sort_neuron(const Tensor& xl, const Tensor& xu, const Tensor& w, int64_t groups, double q,
                                             int truncate) {
+    reverse_mode_only("bound_sort_neuron", xl, xu, w);
     at::AutoDispatchBelowADInplaceOrView below;
     const c10::DeviceGuard guard(xl.device());
     Tensor lo = new_out(xl, w.size(0)), up = new_out(xl, w.size(0));
@@ -350,6 +367,7 @@ struct ShiftNode : Node {
 
 std::pair<Tensor, Tensor> mean_shift_index(const Tensor& x_in, const OptTensor& index, int64_t channels, const OptTensor& running,
                                            double momentum) {
+    reverse_mode_only("mean_shift", x_in);
     const bool grad = want_grad(x_in);
     Tensor y, mean, idx = index ? *index : Tensor();
     {
@@ -376,6 +394,7 @@ std::pair<Tensor, Tensor> mean_shift(const Tensor& x, const OptTensor& running, 
 
 // z + sign * vec[channel], outside any graph
 Tensor channel_shift(const Tensor& z_in, const Tensor& vec_in, double sign) {
+    reverse_mode_only("channel_shift", z_in, vec_in);
     at::AutoDispatchBelowADInplaceOrView below;
     const c10::DeviceGuard guard(z_in.device());
     const Tensor z = z_in.contiguous(), vec = vec_in.contiguous();
@@ -404,6 +423,7 @@ struct UnfoldNode : Node {
 };
 
 Tensor unfold(const Tensor& x_in, int kh, int kw, int dil, int pad, int stride) {
+    reverse_mode_only("unfold", x_in);
     const bool grad = want_grad(x_in);
     const int B = (int)x_in.size(0), C = (int)x_in.size(1), H = (int)x_in.size(2), W = (int)x_in.size(3);
     Tensor y;

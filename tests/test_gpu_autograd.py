@@ -1,4 +1,4 @@
-"""Graph nodes of the native front-end: gradients with respect to any subset of the inputs."""
+"""Graph nodes of the native front-end: gradients with respect to any subset of the inputs, and what the nodes refuse."""
 import itertools
 
 import pytest
@@ -84,3 +84,25 @@ def test_bound_gradients_by_what_requires_them(wanted):
                 assert got.shape == t.shape and not got.any()
             else:
                 _close(got, full[i])
+
+
+@pytest.mark.parametrize("grad", [True, False])
+@pytest.mark.parametrize("name", OPS)
+def test_forward_mode_is_refused(name, grad):
+    """There is no forward-mode formula: an output without a tangent would pass for a zero derivative."""
+    import torch.autograd.forward_ad as fw
+    inputs, fn = _op(name)
+    for i in range(len(inputs)):
+        with fw.dual_level(), torch.set_grad_enabled(grad):
+            dual = [fw.make_dual(t, torch.ones_like(t)) if j == i else t for j, t in enumerate(inputs)]
+            with pytest.raises(NotImplementedError, match="forward mode"):
+                fn(*dual)
+
+
+@pytest.mark.parametrize("name", OPS)
+def test_function_transforms_are_refused(name):
+    inputs, fn = _op(name)
+    with pytest.raises(RuntimeError, match="torch.func"):
+        torch.func.grad(lambda t: fn(t, *inputs[1:])[0].sum())(inputs[0])
+    with pytest.raises(RuntimeError, match="torch.func"):
+        torch.func.vmap(lambda s: fn(*inputs)[0].sum() * s)(torch.ones(2, device="cuda"))
