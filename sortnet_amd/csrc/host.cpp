@@ -8,6 +8,7 @@
 // interpreter.  Tensors stay torch's: outputs come from its caching allocator and work is queued on its current
 // stream.
 #include <cmath>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 
@@ -80,6 +81,10 @@ void reverse_mode_only(const char* who, const T&... t) {
 template <class... T>
 bool want_grad(const T&... t) { return at::GradMode::is_enabled() && (t.requires_grad() || ...); }
 
+// Every node takes its mutex_ while it reads or frees what it saved: two threads may run backward through a graph that they
+// share.  Saved tensors are unpacked before autograd is switched off, since the caller's unpack hooks run inside.
+using Locked = std::lock_guard<std::mutex>;
+
 template <class N>
 std::shared_ptr<N> new_node() { return std::shared_ptr<N>(new N(), torch::autograd::deleteNode); }
 
@@ -93,14 +98,15 @@ struct DistNode : Node {
     double p = 0, q = 0;
 
     variable_list apply(variable_list&& grads) override {
-        at::AutoDispatchBelowADInplaceOrView below;
+        const Locked lock(mutex_);
         variable_list out(2);
         if (!grads[0].defined()) return out;
         const bool want_w = task_should_compute_output(1), want_x = task_should_compute_output(0);
         if (!want_w && !want_x) return out;
-        const Tensor g = grads[0].contiguous(), xs = x.unpack(), ws = weight.unpack();
-        const Tensor st = state.unpack(shared_from_this());
+        const Tensor xs = x.unpack(), ws = weight.unpack(), st = state.unpack(shared_from_this());
         const Tensor cis = ci.unpack(), cos = co.unpack();
+        at::AutoDispatchBelowADInplaceOrView below;
+        const Tensor g = grads[0].contiguous();
         const c10::DeviceGuard guard(g.device());
         const int B = (int)g.size(0), CO = (int)g.size(1), HW = (int)g.size(2), CI = (int)xs.size(1), G = groups;
         const int W_CO = (int)ws.size(0), W_CI = (int)ws.size(1) * G;
@@ -133,6 +139,7 @@ struct DistNode : Node {
         return out;
     }
     void release_variables() override {
+        const Locked lock(mutex_);
         x.reset_data(); weight.reset_data(); state.reset_data(); ci.reset_data(); co.reset_data();
     }
     std::string name() const override { return "DistNode"; }
@@ -249,12 +256,13 @@ struct BoundNode : Node {
     int groups = 1;
 
     variable_list apply(variable_list&& grads) override {
-        at::AutoDispatchBelowADInplaceOrView below;
+        const Locked lock(mutex_);
         variable_list out(3);
         if (!grads[0].defined() && !grads[1].defined()) return out;
         const bool want_l = task_should_compute_output(0), want_u = task_should_compute_output(1), want_w = task_should_compute_output(2);
         if (!want_l && !want_u && !want_w) return out;
         const Tensor l = xl.unpack(), u = xu.unpack(), w = weight.unpack(), posl = pl.unpack(), posu = pu.unpack();
+        at::AutoDispatchBelowADInplaceOrView below;
         const Tensor gl = grads[0].defined() ? grads[0].contiguous() : at::zeros(posl.sizes(), l.options());
         const Tensor gu = grads[1].defined() ? grads[1].contiguous() : at::zeros(posu.sizes(), l.options());
         const c10::DeviceGuard guard(l.device());
@@ -284,6 +292,7 @@ struct BoundNode : Node {
         return out;
     }
     void release_variables() override {
+        const Locked lock(mutex_);
         xl.reset_data(); xu.reset_data(); weight.reset_data(); pl.reset_data(); pu.reset_data();
     }
     std::string name() const override { return "BoundNode"; }
@@ -352,16 +361,21 @@ struct ShiftNode : Node {
     int64_t channels = 0;
 
     variable_list apply(variable_list&& grads) override {
-        at::AutoDispatchBelowADInplaceOrView below;
+        const Locked lock(mutex_);
         variable_list out(1);
         if (!grads[0].defined() || !task_should_compute_output(0)) return out;
-        const Tensor g = grads[0].contiguous(), idx = index.unpack();
+        const Tensor idx = index.unpack();
+        at::AutoDispatchBelowADInplaceOrView below;
+        const Tensor g = grads[0].contiguous();
         const c10::DeviceGuard guard(g.device());
         out[0] = at::empty(g.sizes(), g.options());
         shift_kernels(g, idx, channels, new_floats(g, {channels}), {}, 0.0, out[0]);
         return out;
     }
-    void release_variables() override { index.reset_data(); }
+    void release_variables() override {
+        const Locked lock(mutex_);
+        index.reset_data();
+    }
     std::string name() const override { return "ShiftNode"; }
 };
 
@@ -405,7 +419,7 @@ Tensor channel_shift(const Tensor& z_in, const Tensor& vec_in, double sign) {
 }
 
 // ---- windows of a convolutional layer as columns; the gradient is the sum back into the image --------------------------
-struct UnfoldNode : Node {
+struct UnfoldNode : Node {   // saves sizes only, which nothing changes or frees
     int B, C, H, W, KH, KW, stride, pad, dil;
 
     variable_list apply(variable_list&& grads) override {

@@ -1,5 +1,6 @@
 """Graph nodes of the native front-end: gradients with respect to any subset of the inputs, and what the nodes refuse."""
 import itertools
+import threading
 
 import pytest
 import torch
@@ -106,3 +107,62 @@ def test_function_transforms_are_refused(name):
         torch.func.grad(lambda t: fn(t, *inputs[1:])[0].sum())(inputs[0])
     with pytest.raises(RuntimeError, match="torch.func"):
         torch.func.vmap(lambda s: fn(*inputs)[0].sum() * s)(torch.ones(2, device="cuda"))
+
+
+def _run(threads):
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+
+
+@pytest.mark.parametrize("name", OPS)
+def test_two_threads_run_backward_through_one_graph(name):
+    inputs, outs, gys = _graph(name)
+    full = torch.autograd.grad(outs, inputs, gys, retain_graph=True)
+    wrong = []
+
+    def retained():
+        for _ in range(20):
+            for a, b in zip(torch.autograd.grad(outs, inputs, gys, retain_graph=True), full):
+                if not (a - b).norm() <= 1e-5 * b.norm():
+                    wrong.append(name)
+
+    _run([threading.Thread(target=retained) for _ in range(2)])
+    assert not wrong
+
+    def released():                     # frees what the nodes saved: the other pass gets its gradients or is told so
+        try:
+            got = torch.autograd.grad(outs, inputs, gys)
+        except RuntimeError as e:
+            if "second time" not in str(e):
+                wrong.append(str(e))
+            return
+        for a, b in zip(got, full):
+            if not (a - b).norm() <= 1e-5 * b.norm():
+                wrong.append(name)
+
+    _run([threading.Thread(target=released) for _ in range(2)])
+    assert not wrong
+
+
+@pytest.mark.parametrize("name", OPS)
+def test_saved_tensor_hooks_and_second_pass(name):
+    inputs, outs, gys = _graph(name)
+    full = torch.autograd.grad(outs, inputs, gys)
+    if name not in ("mean_shift", "unfold"):        # these save nothing
+        with pytest.raises(RuntimeError, match="second time"):
+            torch.autograd.grad(outs, inputs, gys)
+    recorded = []
+
+    def unpack(packed):                 # runs with autograd as the caller left it
+        if packed.is_floating_point() and torch.is_grad_enabled():
+            leaf = packed.detach().requires_grad_()
+            recorded.append((leaf * 2).requires_grad)
+        return packed.cuda()
+
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), unpack):
+        inputs, outs, gys = _graph(name)
+    for a, b in zip(torch.autograd.grad(outs, inputs, gys, create_graph=True), full):
+        _close(a.detach(), b)
+    assert all(recorded)
