@@ -85,6 +85,12 @@ bool want_grad(const T&... t) { return at::GradMode::is_enabled() && (t.requires
 // share.  Saved tensors are unpacked before autograd is switched off, since the caller's unpack hooks run inside.
 using Locked = std::lock_guard<std::mutex>;
 
+// The gradient that flows into output `i` of a node, zeros where none does (an op behind it that has no gradient to give):
+// the inputs then get zeros and not nothing.
+Tensor incoming(const Node& node, const variable_list& grads, int i) {
+    return grads[i].defined() ? grads[i].contiguous() : node.input_metadata(i).zeros_like();
+}
+
 template <class N>
 std::shared_ptr<N> new_node() { return std::shared_ptr<N>(new N(), torch::autograd::deleteNode); }
 
@@ -100,13 +106,12 @@ struct DistNode : Node {
     variable_list apply(variable_list&& grads) override {
         const Locked lock(mutex_);
         variable_list out(2);
-        if (!grads[0].defined()) return out;
         const bool want_w = task_should_compute_output(1), want_x = task_should_compute_output(0);
         if (!want_w && !want_x) return out;
         const Tensor xs = x.unpack(), ws = weight.unpack(), st = state.unpack(shared_from_this());
         const Tensor cis = ci.unpack(), cos = co.unpack();
         at::AutoDispatchBelowADInplaceOrView below;
-        const Tensor g = grads[0].contiguous();
+        const Tensor g = incoming(*this, grads, 0);
         const c10::DeviceGuard guard(g.device());
         const int B = (int)g.size(0), CO = (int)g.size(1), HW = (int)g.size(2), CI = (int)xs.size(1), G = groups;
         const int W_CO = (int)ws.size(0), W_CI = (int)ws.size(1) * G;
@@ -258,13 +263,11 @@ struct BoundNode : Node {
     variable_list apply(variable_list&& grads) override {
         const Locked lock(mutex_);
         variable_list out(3);
-        if (!grads[0].defined() && !grads[1].defined()) return out;
         const bool want_l = task_should_compute_output(0), want_u = task_should_compute_output(1), want_w = task_should_compute_output(2);
         if (!want_l && !want_u && !want_w) return out;
         const Tensor l = xl.unpack(), u = xu.unpack(), w = weight.unpack(), posl = pl.unpack(), posu = pu.unpack();
         at::AutoDispatchBelowADInplaceOrView below;
-        const Tensor gl = grads[0].defined() ? grads[0].contiguous() : at::zeros(posl.sizes(), l.options());
-        const Tensor gu = grads[1].defined() ? grads[1].contiguous() : at::zeros(posu.sizes(), l.options());
+        const Tensor gl = incoming(*this, grads, 0), gu = incoming(*this, grads, 1);
         const c10::DeviceGuard guard(l.device());
         const int B = (int)gl.size(0), CO = (int)gl.size(1), HW = (int)gl.size(2), CI = (int)l.size(1);
         // One bound alone, with a frozen weight, gets no gradient from this op (core/norm_dist.py:157-173: zeros).  What
@@ -363,10 +366,10 @@ struct ShiftNode : Node {
     variable_list apply(variable_list&& grads) override {
         const Locked lock(mutex_);
         variable_list out(1);
-        if (!grads[0].defined() || !task_should_compute_output(0)) return out;
+        if (!task_should_compute_output(0)) return out;
         const Tensor idx = index.unpack();
         at::AutoDispatchBelowADInplaceOrView below;
-        const Tensor g = grads[0].contiguous();
+        const Tensor g = incoming(*this, grads, 0);
         const c10::DeviceGuard guard(g.device());
         out[0] = at::empty(g.sizes(), g.options());
         shift_kernels(g, idx, channels, new_floats(g, {channels}), {}, 0.0, out[0]);

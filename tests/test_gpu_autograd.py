@@ -166,3 +166,27 @@ def test_saved_tensor_hooks_and_second_pass(name):
     for a, b in zip(torch.autograd.grad(outs, inputs, gys, create_graph=True), full):
         _close(a.detach(), b)
     assert all(recorded)
+
+
+class _NoGradient(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, *ts):
+        return tuple(t.clone() for t in ts)
+
+    @staticmethod
+    def backward(ctx, *gs):
+        return (None,) * len(gs)
+
+
+@pytest.mark.parametrize("name", [n for n in OPS if n != "unfold"])    # as torch's own unfold, which passes nothing on
+def test_zeros_where_no_gradient_flows_in(name):
+    inputs, outs, gys = _graph(name)
+    for t, got in zip(inputs, torch.autograd.grad(_NoGradient.apply(*outs), inputs, gys, allow_unused=True)):
+        assert got is not None and got.shape == t.shape and not got.any()
+    if len(outs) == 1:
+        return
+    for i in range(len(outs)):          # one of the outputs: the others' gradients count as zeros
+        (ia, oa, _), (ib, ob, _) = _graph(name), _graph(name)
+        part = torch.autograd.grad(oa[i], ia, gys[i])
+        for a, b in zip(part, torch.autograd.grad(ob, ib, [g if j == i else g * 0 for j, g in enumerate(gys)])):
+            _close(a, b)
