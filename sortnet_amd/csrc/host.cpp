@@ -54,7 +54,11 @@ void require(int rc, const char* who) {
     throw std::runtime_error(std::string(who) + " failed (status " + std::to_string(rc) + "): " + (msg ? msg : "?"));
 }
 
-sd_stream_t stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+// torch's current stream on t's GPU (queried while the arguments of an entry point are formed, perhaps before t is checked)
+sd_stream_t stream_of(const Tensor& t) {
+    if (!t.is_cuda()) throw std::runtime_error("input must be a CUDA tensor");
+    return c10::hip::getCurrentHIPStream(t.device().index()).stream();
+}
 
 // sizes of a layer call on x (B, C, HW)
 struct Dims {
@@ -351,6 +355,7 @@ void shift_kernels(const Tensor& x, const Tensor& index, int64_t channels, const
     float* rp = running && running->defined() ? floats(*running, "running_mean") : nullptr;
     if (index.defined()) {
         const int G = (int)index.size(-2), cnt = (int)index.size(-1);
+        if (G == 0) throw std::runtime_error("index names no groups: its size must be (sub-batches, groups, channels)");
         require(sd_mean_shift_index_forward(floats(x, "input"), ints(index, "index"), (int)x.size(0), G, cnt, (int)(channels / G),
                                             (int)x.size(2), floats(mean, "mean"), rp, (float)momentum, floats(y, "output"),
                                             stream_of(x)), "sd_mean_shift_index_forward");
@@ -448,6 +453,7 @@ Tensor unfold(const Tensor& x_in, int kh, int kw, int dil, int pad, int stride) 
         at::AutoDispatchBelowADInplaceOrView below;
         const c10::DeviceGuard guard(x_in.device());
         const Tensor x = x_in.contiguous();
+        if (stride < 1) throw std::runtime_error("unfold: stride=" + std::to_string(stride) + " must be positive");
         const int64_t oh = (H + 2 * pad - dil * (kh - 1) - 1) / stride + 1, ow = (W + 2 * pad - dil * (kw - 1) - 1) / stride + 1;
         y = new_floats(x, {B, (int64_t)C * kh * kw, oh > 0 && ow > 0 ? oh * ow : 1});   // a window that does not fit is refused below
         require(sd_unfold(floats(x, "input"), B, C, H, W, kh, kw, stride, pad, dil, floats(y, "output"), stream_of(x)), "sd_unfold");

@@ -111,14 +111,18 @@ def _checked(x, weight, group):
     return _C.host()
 
 
+def _check_power(p):
+    if not (math.isinf(p) or p > 0):    # neither zero nor undefined
+        raise NotImplementedError
+
+
 class NormDistF:
     """l-p (finite p) or l-inf (p = inf) distance layer.  Mirrors core/norm_dist.py:6-51."""
 
     @staticmethod
     def apply(x, weight, group, p, need_grad=None, tag=None):
         host = _checked(x, weight, group)
-        if p <= 0:
-            raise NotImplementedError
+        _check_power(p)
         return host.norm_dist(x, weight, group, p)
 
 
@@ -129,8 +133,7 @@ class NormDistDropoutF:
     @staticmethod
     def apply(x, weight, w_index_ci, w_index_co, group, p, tag=None):
         assert weight.size(1) * group == x.size(1) or w_index_ci.size(-1) * group == x.size(1)
-        if p <= 0:
-            raise NotImplementedError
+        _check_power(p)
         return _C.host().norm_dist_dropout(x, weight, w_index_ci, w_index_co, group, p)
 
 
@@ -180,6 +183,8 @@ class MeanShiftIndexF:
 
     @staticmethod
     def apply(x, index, channels, running_mean, momentum):
+        if index is None:
+            raise TypeError("mean_shift_index needs an index list; mean_shift is the form without one")
         return _C.host().mean_shift_index(x, index, channels, running_mean, momentum)
 
 
