@@ -188,7 +188,8 @@ static int lp_forward_max_first(FwdArgs& a, bool small, hipStream_t st) {
 // next chunk (index lists: the row numbers of the chunk after it, one per lane, handed out with
 // v_readlane), its weights (MC independent loads into registers) and its (g, 1/y) pairs (into the other
 // half of the LDS buffer, one barrier per chunk).  The sum over the 32 rows of grad_w is formed in
-// registers and added to memory with one coalesced atomic per work-item and output channel.
+// registers and added to memory with one coalesced atomic per work-item and output channel, or stored to the
+// batch tile's own plane where the result has to be the same bits in every call (plan_lp_bwd).
 constexpr int RB = 32;   // batch rows per workgroup (= one index-list sub-batch)
 constexpr int MC = 8;    // output channels per chunk (the chunk body is unrolled: weights sit in named registers)
 static_assert(MC * RB == 256, "one (g, 1/y) pair per work-item and chunk");
@@ -205,8 +206,14 @@ struct LpBwdArgs {
     int gate_above;
     const float* ry;                  // 1 / y when the caller already holds it, else null
     bool gx_is_zero;                  // grad_input (and grad_weight) were zero-filled by the caller
-    int zsplit;  // slices of the output-channel range (grad_input then merges with atomic adds)
+    int zsplit;      // slices of the output-channel range
+    float* gx_part;  // a plane of grad_input per slice, gx_plane apart, that lp_merge_kernel adds up; null: slices add to gx
+    float* gw_part;  // a plane of grad_weight per batch tile, gw_plane apart; null: batch tiles add to gw
+    size_t gx_plane, gw_plane;
 };
+
+// what becomes of the sums over a batch tile that make up grad_weight
+enum LpGradWeight { kGwNone, kGwAdd, kGwStore };
 
 template <int IP>
 __device__ __forceinline__ float signed_pow(float d, float ry, float pm1) {
@@ -236,7 +243,7 @@ __device__ __forceinline__ float signed_pow_ratio(float sr, float pm1) {
 }
 
 // terms of output channel k of a chunk: FULL = all RB rows present
-template <int IP, bool WGRAD, bool SKIP, bool FULL>
+template <int IP, LpGradWeight GW, bool SKIP, bool FULL>
 __device__ __forceinline__ void lp_bwd_channel(const LpBwdArgs& a, const float2 (&gr)[RB], const float (&xr)[RB],
                                                float (&acc)[RB], float wk, int rows, int row, bool n_ok,
                                                float* __restrict__ gwcol) {
@@ -276,12 +283,13 @@ __device__ __forceinline__ void lp_bwd_channel(const LpBwdArgs& a, const float2 
             }
         }
     }
-    if (WGRAD && n_ok) unsafeAtomicAdd(gwcol + (size_t)row * a.W_CIg, -wsum);
+    if (GW == kGwAdd && n_ok) unsafeAtomicAdd(gwcol + (size_t)row * a.W_CIg, -wsum);
+    if (GW == kGwStore && n_ok) gwcol[(size_t)row * a.W_CIg] = -wsum;
 }
 
 // one chunk.  The multiply-chain and plain general-p forms unroll the channels (weights in named registers); the
 // significance-test form is branchy and large, so it loops and picks its weight with selects.
-template <int IP, bool WGRAD, bool SKIP, bool FULL>
+template <int IP, LpGradWeight GW, bool SKIP, bool FULL>
 __device__ __forceinline__ void lp_bwd_chunk(const LpBwdArgs& a, const float2 (&gr)[MC][RB], const float (&xr)[RB],
                                              float (&acc)[RB], const float (&wv)[MC], int rows, int mcount,
                                              int rowv, bool n_ok, float* __restrict__ gwcol) {
@@ -291,20 +299,20 @@ __device__ __forceinline__ void lp_bwd_chunk(const LpBwdArgs& a, const float2 (&
             float wk = wv[0];
             #pragma unroll
             for (int j = 1; j < MC; j++) wk = k == j ? wv[j] : wk;
-            lp_bwd_channel<IP, WGRAD, SKIP, FULL>(a, gr[k], xr, acc, wk, rows, __builtin_amdgcn_readlane(rowv, k), n_ok, gwcol);
+            lp_bwd_channel<IP, GW, SKIP, FULL>(a, gr[k], xr, acc, wk, rows, __builtin_amdgcn_readlane(rowv, k), n_ok, gwcol);
         }
     } else {
         #pragma unroll
         for (int k = 0; k < MC; k++) {
             if (k < mcount)
-                lp_bwd_channel<IP, WGRAD, SKIP, FULL>(a, gr[k], xr, acc, wv[k], rows, __builtin_amdgcn_readlane(rowv, k), n_ok, gwcol);
+                lp_bwd_channel<IP, GW, SKIP, FULL>(a, gr[k], xr, acc, wv[k], rows, __builtin_amdgcn_readlane(rowv, k), n_ok, gwcol);
         }
     }
 }
 
 // RAGGED: the rows are no multiple of RB.  A kernel of its own: with the code for a part of a tile beside it the code for
 // whole tiles lost 10 to 20 % to the registers (512 x 5120 x 2560, p = 8: 1.17 -> 1.43 ms).
-template <int IP, bool WGRAD, bool SKIP, bool RAGGED>
+template <int IP, LpGradWeight GW, bool SKIP, bool RAGGED>
 __global__ void __launch_bounds__(256, (SKIP ? 4 : 1)) lp_bwd_kernel(LpBwdArgs a) {
     __shared__ float2 gr[2][MC][RB];   // (g, 1/y) of output channel m0+k, row r0+i; two chunks
     if (gate_closed(a.gate, a.gate_limit, a.gate_above)) return;
@@ -314,7 +322,7 @@ __global__ void __launch_bounds__(256, (SKIP ? 4 : 1)) lp_bwd_kernel(LpBwdArgs a
     // output channels of this slice, whole chunks
     const int per = ((a.COg + a.zsplit - 1) / a.zsplit + MC - 1) / MC * MC;
     const int m_lo = slice * per, m_hi = m_lo + per < a.COg ? m_lo + per : a.COg;
-    if (m_lo >= m_hi) return;   // whole workgroup; grad_input of a sliced launch is zero-filled beforehand
+    if (m_lo >= m_hi) return;   // whole workgroup; no slice is empty where each has a plane of its own
     const int r0 = blockIdx.y * RB;
     const int n = blockIdx.x * 256 + tid;
     const bool n_ok = n < a.CIg;
@@ -325,7 +333,8 @@ __global__ void __launch_bounds__(256, (SKIP ? 4 : 1)) lp_bwd_kernel(LpBwdArgs a
     const int wcol = n_ok ? (a.ci_idx ? a.ci_idx[(s * a.G + g) * a.CIg + n] : n) : 0;
     const int* __restrict__ co = a.co_idx ? a.co_idx + (size_t)(s * a.G + g) * a.COg : nullptr;
     const float* __restrict__ wcolp = a.w + (size_t)g * a.W_COg * a.W_CIg + wcol;
-    float* __restrict__ gwcol = WGRAD ? a.gw + (size_t)g * a.W_COg * a.W_CIg + wcol : nullptr;
+    float* __restrict__ gwcol = GW == kGwNone ? nullptr
+        : (GW == kGwStore ? a.gw_part + blockIdx.y * a.gw_plane : a.gw) + (size_t)g * a.W_COg * a.W_CIg + wcol;
     // weight row of output channel m0 + (lane mod MC), clamped into the slice so that every load stays inside W
     const int kl = tid & (MC - 1);
     auto row_of = [&](int m0) {
@@ -382,8 +391,8 @@ __global__ void __launch_bounds__(256, (SKIP ? 4 : 1)) lp_bwd_kernel(LpBwdArgs a
         const float2 pn = pair_of(m0 + MC);
 
         const int mcount = m_hi - m0 < MC ? m_hi - m0 : MC;
-        if (!RAGGED || rows == RB) lp_bwd_chunk<IP, WGRAD, SKIP, true>(a, gr[buf], xr, acc, wv, rows, mcount, rowv, n_ok, gwcol);
-        else lp_bwd_chunk<IP, WGRAD, SKIP, false>(a, gr[buf], xr, acc, wv, rows, mcount, rowv, n_ok, gwcol);
+        if (!RAGGED || rows == RB) lp_bwd_chunk<IP, GW, SKIP, true>(a, gr[buf], xr, acc, wv, rows, mcount, rowv, n_ok, gwcol);
+        else lp_bwd_chunk<IP, GW, SKIP, false>(a, gr[buf], xr, acc, wv, rows, mcount, rowv, n_ok, gwcol);
 
         gr[buf ^ 1][sk][si] = make_float2(pn.x, 1.f / pn.y);   // last read in the previous iteration, before its barrier
         __syncthreads();
@@ -393,13 +402,15 @@ __global__ void __launch_bounds__(256, (SKIP ? 4 : 1)) lp_bwd_kernel(LpBwdArgs a
         rown = rownn;
     }
     if (n_ok) {
+        float* gx = a.gx_part ? a.gx_part + slice * a.gx_plane : a.gx;
+        const bool add = a.zsplit > 1 && !a.gx_part;
         #pragma unroll
         for (int i = 0; i < RB; i++) {
             if (i < rows) {
                 int r = r0 + i;
                 int b = r / a.HW, hw = r - b * a.HW;
-                float* dst = a.gx + ((size_t)(b * a.G + g) * a.CIg + n) * a.HW + hw;
-                if (a.zsplit > 1) unsafeAtomicAdd(dst, acc[i]);
+                float* dst = gx + ((size_t)(b * a.G + g) * a.CIg + n) * a.HW + hw;
+                if (add) unsafeAtomicAdd(dst, acc[i]);
                 else *dst = acc[i];
             }
         }
@@ -584,41 +595,101 @@ static int launch_lp_bwd_fused(int ip, const LpBwdArgs& a, hipStream_t st) {
     return check_launch("lp_bwd_fused_kernel");
 }
 
-template <bool WGRAD>
-static int launch_lp_bwd(int ip, const LpBwdArgs& a_in, hipStream_t st) {
+// grad[o] (+)= sum of `planes` partial sums, in plane order: the same bits in every call.  A work-item adds four neighbouring
+// elements over a quarter of the planes, the quarters meet in LDS (a few planes of a small layer: what counts is how many
+// loads are in flight: 32 slices of 32 x 784 take 3.9 us; 8 tiles of 1021 x 3072, 113 MB read and written, 21.7).  The blocks of grad_input first, then those of grad_weight, in one launch.
+struct LpMerge { const float* part; float* out; size_t total, plane; int planes; unsigned blocks; bool add; };
+__global__ void __launch_bounds__(256) lp_merge_kernel(LpMerge gx, LpMerge gw, const unsigned long long* gate,
+                                                       unsigned long long gate_limit, int gate_above) {
+    __shared__ float4 sums[4][64];
+    if (gate_closed(gate, gate_limit, gate_above)) return;
+    const LpMerge m = blockIdx.x < gx.blocks ? gx : gw;
+    const int lane = threadIdx.x & 63, quarter = threadIdx.x >> 6;
+    const size_t o = ((size_t)(blockIdx.x < gx.blocks ? blockIdx.x : blockIdx.x - gx.blocks) * 64 + lane) * 4;
+    const int per = (m.planes + 3) / 4, lo = quarter * per, hi = lo + per < m.planes ? lo + per : m.planes;
+    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (o < m.total) {      // (a plane is a whole number of 16-byte words)
+        #pragma unroll 8
+        for (int k = lo; k < hi; k++) {
+            const float4 v = *reinterpret_cast<const float4*>(m.part + k * m.plane + o);
+            s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
+        }
+    }
+    sums[quarter][lane] = s;
+    __syncthreads();
+    if (quarter != 0 || o >= m.total) return;
+    #pragma unroll
+    for (int k = 1; k < 4; k++) {
+        const float4 v = sums[k][lane];
+        s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
+    }
+    const float r[4] = {s.x, s.y, s.z, s.w};
+    if (o + 4 <= m.total && !m.add) *reinterpret_cast<float4*>(m.out + o) = s;
+    else {
+        for (int k = 0; k < 4 && o + k < m.total; k++) m.out[o + k] = m.add ? m.out[o + k] + r[k] : r[k];
+    }
+}
+
+// How the general kernel's sums are cut and merged.  Sums of up to two addends have one result; more of them are merged in
+// a fixed order, from planes in the workspace, or by atomic additions in any order.
+struct LpBwdPlan {
+    int zsplit;                  // slices of the output-channel range
+    int rows;                    // batch rows per launch
+    size_t gx_plane, gw_plane;   // floats per plane of partial sums, 0: no planes, the sums meet by atomic additions
+    size_t gx_words, gw_words;   // floats of all planes of a launch
+    size_t words() const { return gx_words + gw_words; }
+};
+
+// same_bits: the planes that make the gradients of a dense layer the same bits in every call
+static LpBwdPlan plan_lp_bwd(const LpBwdArgs& a, bool same_bits, bool planes) {
+    LpBwdPlan plan{1, a.R, 0, 0, 0, 0};
+    int tiles = (a.R + RB - 1) / RB;
+    if (planes && same_bits && a.gw && tiles > 2) {
+        // planes of at most 128 MB: a larger batch is taken in several launches
+        const size_t most = ((size_t)1 << 25) / ((size_t)a.COg * a.CIg);
+        if ((size_t)tiles > most) { tiles = most > 4 ? (int)most : 4; plan.rows = tiles * RB; }
+        plan.gw_plane = ((size_t)a.COg * a.CIg + 3) / 4 * 4;
+        plan.gw_words = plan.gw_plane * tiles;
+    }
     // a workgroup covers 256 input channels x 32 rows and walks the output channels; when that leaves the
     // device mostly idle (index lists: a few hundred kept inputs per sub-batch) the output-channel range is
-    // cut in slices that merge into grad_input with atomic adds
-    LpBwdArgs a = a_in;
-    const long long blocks = (long long)((a.CIg + 255) / 256) * ((a.R + RB - 1) / RB) * a.G;
+    // cut in slices
+    const long long blocks = (long long)((a.CIg + 255) / 256) * tiles * a.G;
     // workgroups run in rounds of (resident workgroups per CU) x CUs: take the slice count whose last round
     // is fullest, a smaller count unless a larger one gains 3 %, slices of at least 64 channels
     const double slots = (double)((a.skip_thr > 0.f ? 4 : 3) * num_cus());
     double best = 0.0;
-    a.zsplit = 1;
     for (int z = 1; z <= 16 && (z == 1 || a.COg / z >= 64); z++) {
         const double rounds = (double)blocks * z / slots, eff = rounds / std::ceil(rounds);
-        if (eff > best * 1.03) { best = eff; a.zsplit = z; }
+        if (eff > best * 1.03) { best = eff; plan.zsplit = z; }
     }
-    // small layers: slices down to one chunk of MC channels until every compute unit has two workgroups (p = 8, in us:
-    // 32 x 784 x 256 64 -> 21, 64 x 1024 x 1024 64 -> 37; with four per unit the last is 51)
+    if (!planes || !aligned16(a.gx)) return plan;
+    // small layers: slices down to one chunk of MC channels until every compute unit has two workgroups, merged in slice order
+    // (p = 8, both gradients, in us, slices of 64 channels -> this, in brackets with atomic additions in any order:
+    // 32 x 784 x 256 61 -> 20 (17), 90 x 1600 x 230 199 -> 37 (31), 64 x 1024 x 1024 64 -> 35 (36); with four per unit 51)
     const long long fill = 2ll * num_cus();
-    if (blocks * a.zsplit < fill && aligned16(a.gx)) {   // (slices add to a filled grad_input)
+    const bool fine = blocks * plan.zsplit < fill;
+    if (fine) {
         const long long more = (fill + blocks - 1) / blocks, most = (a.COg + MC - 1) / MC;
-        a.zsplit = (int)(more < most ? more : most);
+        plan.zsplit = (int)(more < most ? more : most);
+        const int per = ((a.COg + plan.zsplit - 1) / plan.zsplit + MC - 1) / MC * MC;   // as the kernel cuts
+        plan.zsplit = (a.COg + per - 1) / per;
     }
-    int rc;
-    const size_t nx = a.zsplit > 1 ? (size_t)a.R * a.G * a.CIg : 0, nw = WGRAD ? (size_t)a.G * a.W_COg * a.W_CIg : 0;
-    if (!a.gx_is_zero && nx && nw) rc = fill_zero2(a.gx, nx, a.gw, nw, st);
-    else if (!a.gx_is_zero && nx + nw) rc = nx ? fill_zero(a.gx, nx, st) : fill_zero(a.gw, nw, st);
-    else rc = SD_OK;
-    if (rc) return rc;
+    if (plan.zsplit > 2 && (fine || same_bits)) {
+        plan.gx_plane = ((size_t)(plan.rows < a.R ? plan.rows : a.R) * a.G * a.CIg + 3) / 4 * 4;
+        plan.gx_words = plan.gx_plane * plan.zsplit;
+    }
+    return plan;
+}
+
+template <LpGradWeight GW>
+static int launch_lp_bwd(int ip, const LpBwdArgs& a, hipStream_t st) {
     dim3 grid((a.CIg + 255) / 256, (a.R + RB - 1) / RB, a.G * a.zsplit);
     const bool ragged = a.R % RB != 0;
-#define SD_LAUNCH(k, skip)                                                                                  \
-    do {                                                                                                    \
-        if (ragged) hipLaunchKernelGGL((lp_bwd_kernel<k, WGRAD, skip, true>), grid, dim3(256), 0, st, a);   \
-        else hipLaunchKernelGGL((lp_bwd_kernel<k, WGRAD, skip, false>), grid, dim3(256), 0, st, a);         \
+#define SD_LAUNCH(k, skip)                                                                               \
+    do {                                                                                                 \
+        if (ragged) hipLaunchKernelGGL((lp_bwd_kernel<k, GW, skip, true>), grid, dim3(256), 0, st, a);   \
+        else hipLaunchKernelGGL((lp_bwd_kernel<k, GW, skip, false>), grid, dim3(256), 0, st, a);         \
     } while (0)
 #define SD_CASE(k) case k: SD_LAUNCH(k, false); break;
     switch (ip) {
@@ -631,6 +702,39 @@ static int launch_lp_bwd(int ip, const LpBwdArgs& a_in, hipStream_t st) {
 #undef SD_CASE
 #undef SD_LAUNCH
     return check_launch("lp_bwd_kernel");
+}
+
+// the general kernel as `plan` cuts it; `part`: room for the planes
+static int run_lp_bwd(int ip, LpBwdArgs& a, const LpBwdPlan& plan, float* part, hipStream_t st) {
+    a.zsplit = plan.zsplit;
+    a.gx_plane = plan.gx_plane; a.gw_plane = plan.gw_plane;
+    a.gx_part = plan.gx_words ? part : nullptr;
+    a.gw_part = plan.gw_words ? part + plan.gx_words : nullptr;
+    const size_t w_words = a.gw ? (size_t)a.G * a.W_COg * a.W_CIg : 0;
+    int rc = SD_OK;
+    if (!a.gx_is_zero) {   // what atomics add to
+        const size_t nx = a.zsplit > 1 && !a.gx_part ? (size_t)a.R * a.G * a.CIg : 0, nw = a.gw_part ? 0 : w_words;
+        if (nx && nw) rc = fill_zero2(a.gx, nx, a.gw, nw, st);
+        else if (nx + nw) rc = nx ? fill_zero(a.gx, nx, st) : fill_zero(a.gw, nw, st);
+        if (rc) return rc;
+    }
+    for (int left = a.R, first = 1; left > 0; left -= plan.rows, first = 0) {
+        a.R = left < plan.rows ? left : plan.rows;
+        rc = !a.gw ? launch_lp_bwd<kGwNone>(ip, a, st) : a.gw_part ? launch_lp_bwd<kGwStore>(ip, a, st) : launch_lp_bwd<kGwAdd>(ip, a, st);
+        if (rc) return rc;
+        const size_t x_words = (size_t)a.R * a.G * a.CIg;
+        if (plan.words()) {
+            LpMerge mx{}, mw{};
+            if (a.gx_part) mx = LpMerge{a.gx_part, a.gx, x_words, plan.gx_plane, a.zsplit, (unsigned)((x_words + 255) / 256), false};
+            if (a.gw_part) mw = LpMerge{a.gw_part, a.gw, w_words, plan.gw_plane, (a.R + RB - 1) / RB, (unsigned)((w_words + 255) / 256), !first};
+            hipLaunchKernelGGL(lp_merge_kernel, dim3(mx.blocks + mw.blocks), dim3(256), 0, st, mx, mw, a.gate, a.gate_limit, a.gate_above);
+            if ((rc = check_launch("lp_merge_kernel"))) return rc;
+        }
+        // (only dense single-group layers are taken in several launches)
+        a.x += x_words; a.gx += x_words;
+        a.gy += (size_t)a.R * a.COg; a.y += (size_t)a.R * a.COg;
+    }
+    return SD_OK;
 }
 
 static int lp_backward(const char* who, const float* grad_output, const float* input, const float* weight,
@@ -661,29 +765,42 @@ static int lp_backward(const char* who, const float* grad_output, const float* i
     // dense layers at general p: a kernel that works from per-row candidate tables is queued in front of the one
     // that evaluates every term, and a count taken on the device decides which of the two runs
     const float thr_rows = (ip < 0 && a.pm1 > 1.f) ? powf(1e-16f, 1.f / a.pm1) : 0.f;
-    bool zero_gx = false;
     // which kernel evaluates every term, and whether it runs its own wave-level tests
-    // (and enough workgroups for it: 512 x 600 x 600 at p = 100, 75 of them, took 480 us against 95)
+    // (and enough workgroups for it: 512 x 600 x 600 at p = 100, 75 of them, took 480 us against 101)
     const long long fused_groups = (long long)(f.CIg / FN) * ((f.COg + FMR - 1) / FMR);
-    const bool fused = dense && grad_weight && a.skip_thr >= kLpSkipFromFused && fused_groups >= 2 * num_cus();
+    const bool fused_p = dense && grad_weight && a.skip_thr >= kLpSkipFromFused, fused = fused_p && fused_groups >= 2 * num_cus();
     const bool tests = fused || a.skip_thr >= kLpSkipFromGeneral;
     const float cap = rows_cap(grad_weight ? (tests ? kRowsCapBackwardSkip : kRowsCapBackward)
                                            : (tests ? kRowsCapBackwardInputSkip : kRowsCapBackwardInput), thr_rows);
-    if (cap > 0.f && rows_large(f.R, f.COg, f.CIg) && dense && thr_rows > 0.f && thr_rows < 1.f && f.CIg % kRowsChunk == 0 &&
-        f.W_CIg == f.CIg && B < (1 << 22)) {
-        void* ws = workspace(lp_rows_workspace(f.R, f.COg, f.CIg) + (size_t)f.R * f.COg * sizeof(float), st);
-        if (!ws) return SD_ERR_HIP;
+    const bool rows_p = cap > 0.f && dense && thr_rows > 0.f && thr_rows < 1.f && f.CIg % kRowsChunk == 0 &&
+                        f.W_CIg == f.CIg && B < (1 << 22);
+    const bool rows = rows_p && rows_large(f.R, f.COg, f.CIg);
+    if (!fused && a.skip_thr < kLpSkipFromGeneral) a.skip_thr = 0.f;
+    // At such p the table kernel and the fused kernel form a grad_weight that is the same bits in every call, and grad_input
+    // too where few weight rows meet; so does the general kernel where it takes the place of one of them for want of size
+    // (both gradients, in us, by atomic additions -> from planes: 250 x 3072 x 1021 at p = 24 297 -> 312, 512 x 600 x 600
+    // at p = 100 94 -> 101, 2048 x 1024 x 1024 at p = 120 in eight launches 639 -> 717, the fused kernel 3215).
+    const bool same_bits = !fused && (fused_p || (rows_p && !rows));
+    // one request for every user of the workspace: the tables and 1 / y, then the planes of partial sums
+    const size_t table_bytes = rows ? (lp_rows_workspace(f.R, f.COg, f.CIg) + (size_t)f.R * f.COg * sizeof(float) + 255) / 256 * 256 : 0;
+    LpBwdPlan plan{};
+    char* ws = nullptr;
+    if (!fused) {
+        plan = plan_lp_bwd(a, same_bits, true);
+        if (plan.words() && !(ws = static_cast<char*>(workspace(table_bytes + plan.words() * sizeof(float), st))))
+            plan = plan_lp_bwd(a, same_bits, false);   // no room for planes (a stream under capture)
+    }
+    if (rows) {
+        if (!ws && !(ws = static_cast<char*>(workspace(table_bytes, st)))) return SD_ERR_HIP;
         // the general kernel adds to a zero-filled grad_weight, which the table kernel must not find cleared after it ran
-        if (grad_weight && !fused && (rc = fill_zero(grad_weight, (size_t)G * f.W_COg * f.W_CIg, st))) return rc;
+        if (grad_weight && !fused && !plan.gw_words && (rc = fill_zero(grad_weight, (size_t)G * f.W_COg * f.W_CIg, st))) return rc;
         if ((rc = lp_rows_backward(grad_output, input, weight, output, f.R, f.COg, f.CIg, a.pm1, thr_rows, grad_input,
                                    grad_weight, ws, cap, &a.ry, &a.gate, &a.gate_limit, st))) return rc;
         a.gate_above = 1;
-        zero_gx = true;
+        a.gx_is_zero = true;
     }
     if (fused) return launch_lp_bwd_fused(ip, a, st);
-    if (a.skip_thr < kLpSkipFromGeneral) a.skip_thr = 0.f;
-    a.gx_is_zero = zero_gx;
-    return grad_weight ? launch_lp_bwd<true>(ip, a, st) : launch_lp_bwd<false>(ip, a, st);
+    return run_lp_bwd(ip, a, plan, reinterpret_cast<float*>(ws + table_bytes), st);
 }
 
 }  // namespace sd
