@@ -134,7 +134,8 @@ __global__ void __launch_bounds__(256) index_shift_kernel(const float* __restric
 // channels of a group; its wavefronts take a sub-batch each (up to 16 at a time).  A wavefront reads its list once and
 // notes in LDS where each of the 64 channels stands in it (lists in any order), a lane then sums its channel's rows in
 // sample order and the sub-batches are added in order: the same bits as above.  The rows are read a second time, from
-// cache, for the shift.  Four launches of 4 to 7 us each were bound by their launches: 32 x 192 of 256 channels
+// cache, for the shift.  A list that names a channel more than once (no list of a sampler does) has one of its columns in the
+// mean, as above, and all of them shifted.  Four launches of 4 to 7 us each were bound by their launches: 32 x 192 of 256 channels
 // 24 -> 6 us, 128 x 3840 of 5120 24 -> 12 us, 512 x 3840 of 5120 23 both ways.
 constexpr int kFuseWaves = 16, kFuseSubs = 128;   // sub-batches at a time / at most (their positions are held in LDS)
 __global__ void __launch_bounds__(64 * kFuseWaves) index_mean_shift_kernel(
@@ -143,6 +144,7 @@ __global__ void __launch_bounds__(64 * kFuseWaves) index_mean_shift_kernel(
     extern __shared__ int at[];                       // [S][64]: position of the channel in the sub-batch's list, or -1
     __shared__ float sums[kFuseWaves][64];
     __shared__ float shift[64];
+    __shared__ int repeated;                          // a list names one of the channels more than once
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
     const int g = blockIdx.y, c0 = blockIdx.x * 64, c = c0 + lane;
     const size_t stride = (size_t)G * cnt;
@@ -152,6 +154,8 @@ __global__ void __launch_bounds__(64 * kFuseWaves) index_mean_shift_kernel(
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     };
+    if (threadIdx.x == 0) repeated = 0;
+    __syncthreads();
     float total = 0.f, seen = 1e-10f;                 // of wavefront 0
     for (int s0 = 0; s0 < S; s0 += waves) {
         const int s = s0 + wave;
@@ -164,7 +168,7 @@ __global__ void __launch_bounds__(64 * kFuseWaves) index_mean_shift_kernel(
             #pragma unroll 8
             for (int j = lane; j < cnt; j += 64) {
                 const int k = list[j] - c0;
-                if (k >= 0 && k < 64) slot[k] = j;
+                if (k >= 0 && k < 64 && atomicExch(&slot[k], j) >= 0) repeated = 1;
             }
             posted();
             const int j = slot[lane];
@@ -195,6 +199,19 @@ __global__ void __launch_bounds__(64 * kFuseWaves) index_mean_shift_kernel(
         }
     }
     __syncthreads();
+    if (repeated) {
+        for (int s = wave; s < S; s += waves) {
+            const int* list = index + (size_t)(s * G + g) * cnt;
+            const int b0 = s * kSubBatch, b1 = b0 + kSubBatch < B ? b0 + kSubBatch : B;
+            for (int j = lane; j < cnt; j += 64) {
+                const int k = list[j] - c0;
+                if (k < 0 || k >= 64) continue;
+                const size_t o = (size_t)g * cnt + j;
+                for (int b = b0; b < b1; b++) y[o + b * stride] = x[o + b * stride] - shift[k];
+            }
+        }
+        return;
+    }
     const float m = shift[lane];
     for (int s = wave; s < S; s += waves) {
         const int j = at[s * 64 + lane];

@@ -26,3 +26,18 @@ def test_mean_shift_of_compacted_layers(B, G, cnt, Cg, HW):
     assert (m.cpu().double() - mean).abs().max() <= bar
     assert (rd.cpu().double() - (0.9 * running.double() + 0.1 * mean)).abs().max() <= bar
     assert (y.cpu().double() - (x.double() - mean[chan][:, :, None])).abs().max() <= 2 * bar
+
+
+@pytest.mark.parametrize("B,G,cnt,Cg,HW", [(40, 1, 6, 8, 1), (33, 2, 70, 70, 1), (600, 1, 100, 130, 1), (40, 1, 6, 8, 2)])
+def test_lists_that_name_a_channel_more_than_once(B, G, cnt, Cg, HW):
+    """One of the columns makes the channel's mean; all of them are shifted."""
+    from sortnet_amd import ext
+    g = torch.Generator().manual_seed(B)
+    S = -(-B // 32)
+    index = torch.randint(0, Cg, (S, G, cnt), generator=g).to(torch.int32)
+    index[..., 1] = index[..., 0]
+    x = torch.randn(B, G * cnt, HW, generator=g).cuda()
+    chan = (index.long() + torch.arange(G)[None, :, None] * Cg).reshape(S, G * cnt).repeat_interleave(32, 0)[:B].cuda()
+    y, mean = torch.full_like(x, float("nan")), torch.empty(G * Cg, device="cuda")
+    ext.mean_shift_index_forward(x, index.cuda(), Cg, mean, None, 0.1, y)
+    assert torch.equal(y, x - mean[chan][:, :, None])
