@@ -255,8 +255,10 @@ class NormDistConv(NormDistBase):
 
     def _columns(self, z):
         """The windows of z as columns (B, C * kh * kw, positions)."""
-        if self.kernel_size == (1, 1) and self.stride == 1 and self.padding == 0:
-            return z.flatten(2).contiguous()       # every pixel is its own window: no copy of what is contiguous
+        if self.kernel_size == (1, 1) and self.stride == 1 and self.padding == 0 and not torch.is_grad_enabled():
+            # every pixel is its own window: no copy of what is contiguous, unless a backward pass may need what the caller
+            # could have changed in place by then
+            return z.flatten(2).contiguous()
         return ext.host().unfold(z, *self.kernel_size, self.dilation, self.padding, self.stride)
 
 

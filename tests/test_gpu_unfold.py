@@ -34,3 +34,20 @@ def test_unfold_refuses_a_window_that_does_not_fit():
     from sortnet_amd import ext
     with pytest.raises(RuntimeError, match="does not fit"):
         ext.host().unfold(torch.rand(1, 1, 4, 4, device="cuda"), 5, 5, 1, 0, 1)
+
+
+@pytest.mark.parametrize("window", [1, 3])
+def test_input_changed_in_place_between_the_passes(window):
+    """The columns are the layer's own: what happens to the image after the forward does not concern the backward."""
+    from sortnet_amd.layers import DropoutRegistry, NormDistConv
+    layer = NormDistConv(3, 5, window, padding=window // 2, p=3.0, bias=False, mean_shift=False, registry=DropoutRegistry(1)).cuda()
+    leaf = torch.rand(4, 3, 6, 6, generator=torch.Generator().manual_seed(2)).cuda().requires_grad_()
+    want = torch.autograd.grad(layer(leaf)[0].sum(), [leaf, layer.weight])
+    image = leaf * 1
+    y = layer(image)[0]
+    with torch.no_grad():
+        image.mul_(2)
+    for got, ref in zip(torch.autograd.grad(y.sum(), [leaf, layer.weight]), want):
+        assert (got - ref).norm() <= 1e-5 * ref.norm()
+    with torch.no_grad():
+        assert torch.equal(layer(leaf)[0], y)
