@@ -322,17 +322,20 @@ extern "C" int sd_masked_inf_dist_forward(const float* input, const float* weigh
     }
     // factored mask: dropped inputs / weights are replaced by NaN while staging the tiles and
     // NaN terms never win the maximum, so the plain l-inf policies apply unchanged.  On the
-    // vector-load path the keep bits are built once per call into the library workspace.
-    size_t packed_bytes = 0;
+    // vector-load path, and for the kernels that stream the weights, the keep bits are built once per call into the
+    // library workspace; elsewhere the kernels draw them term by term.
     int K = 0;          // depth of the candidate tables' bound (0: no tables)
     void* tables = nullptr;
-    const bool streamable = HW == 1 && g_linf_density.load(std::memory_order_relaxed) <= 0.f;
-    if ((a.fast_x && a.fast_w) || streamable) {
-        const int nchunks = (a.CIg + KT - 1) / KT;
-        const long long xrows = (long long)a.R * G, wrows = (long long)CO;
-        packed_bytes = pos ? (((size_t)a.R * CO * 8 + 255) / 256) * 256 : 0;
+    const int nchunks = (a.CIg + KT - 1) / KT;
+    const long long xrows = (long long)a.R * G, wrows = (long long)CO;
+    const size_t packed_bytes = pos ? (((size_t)a.R * CO * 8 + 255) / 256) * 256 : 0;
+    const size_t mask_bytes = ((size_t)(xrows + wrows) * nchunks * 4 + 255) / 256 * 256;
+    const bool vector = a.fast_x && a.fast_w;
+    // (rows that are not streamed for speed need no scratch without positions, so a stream under capture must not ask for it)
+    const bool streamed = g_linf_density.load(std::memory_order_relaxed) <= 0.f && row_stream_sizes_ok(a, kStreamMaskTerms) &&
+                          (vector || workspace_ready(packed_bytes + mask_bytes, st));
+    if (vector || streamed) {
         // one request for every user of the workspace: merge buffer, keep bits, candidate tables
-        const size_t mask_bytes = ((size_t)(xrows + wrows) * nchunks * 4 + 255) / 256 * 256;
         const int KE = max_cols_eligible(a, (float)a.t16 / 65536.f, B, CO, CI, G, HW);
         K = max_cols_wanted(a, KE, kHintSiteMasked, B, CO, CI, st);
         char* base = static_cast<char*>(workspace(packed_bytes + mask_bytes + (KE ? max_tables_bytes(B, CO, CI, KE) : 0), st));
@@ -344,7 +347,7 @@ extern "C" int sd_masked_inf_dist_forward(const float* input, const float* weigh
                            xm, xrows, xrows + wrows, nchunks, a.CIg, seed, a.t16);
         if ((rc = check_launch("build_masks_kernel"))) return rc;
         a.xmask = xm; a.wmask = wm;
-        if (streamable && row_stream_ok(a, kStreamMaskTerms)) return row_stream_linf(a, st);
+        if (streamed) return row_stream_linf(a, st);
     }
     if (pos) {
         if (K && (rc = queue_max_cols(a, K, B, CO, CI, tables, st))) return rc;

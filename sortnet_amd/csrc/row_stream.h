@@ -19,8 +19,9 @@ namespace sd {
 constexpr long long kStreamMaxTerms = 3ll << 25, kStreamPosTerms = 5ll << 24, kStreamMaskTerms = 3ll << 24;
 constexpr long long kStreamBoundTerms = 5ll << 24, kStreamBoundPosTerms = 7ll << 23;
 
-// whether the streaming kernels serve a call of at most `limit` terms: dense, no mask or a factored one with its keep
-// bits built, rows short enough for the registers
+// whether the streaming kernels serve a call of at most `limit` terms by its sizes: dense, rows short enough for the registers
+bool row_stream_sizes_ok(const FwdArgs& a, long long limit);
+// the same with what they read at hand: no mask, or a factored one with its keep bits built
 bool row_stream_ok(const FwdArgs& a, long long limit);
 // the same for the sort neuron (a.x1: its interval form)
 bool row_stream_sort_ok(const FwdArgs& a);

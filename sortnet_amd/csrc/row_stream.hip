@@ -361,8 +361,12 @@ int dispatch(const FwdArgs& a, int K, hipStream_t stream) {
 
 }  // namespace
 
+bool row_stream_sizes_ok(const FwdArgs& a, long long limit) {
+    return a.HW == 1 && !a.ci_idx && !a.co_idx && a.CIg <= 160 * 64 && (long long)a.R * a.G * a.COg * a.CIg <= limit;
+}
+
 bool row_stream_ok(const FwdArgs& a, long long limit) {
-    return a.HW == 1 && !a.ci_idx && !a.co_idx && a.CIg <= 160 * 64 && (long long)a.R * a.G * a.COg * a.CIg <= limit &&
+    return row_stream_sizes_ok(a, limit) &&
            (a.mask_mode < 0 || (a.mask_mode == SD_MASK_FACTORED && a.xmask && a.wmask));
 }
 

@@ -74,22 +74,39 @@ int num_cus() {
     return n;
 }
 
+namespace {
+struct Slot { int dev; hipStream_t stream; void* buf; size_t cap; };
+std::mutex g_slot_mu;
+std::vector<Slot> g_slots;
+
+bool capturing(hipStream_t stream) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &cap) != hipSuccess) { (void)hipGetLastError(); return false; }
+    return cap != hipStreamCaptureStatusNone;
+}
+}  // namespace
+
+bool workspace_ready(size_t bytes, hipStream_t stream) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0) { (void)hipGetLastError(); return false; }
+    {
+        std::lock_guard<std::mutex> lock(g_slot_mu);
+        for (const Slot& c : g_slots) if (c.dev == dev && c.stream == stream && c.cap >= bytes) return true;
+    }
+    return !capturing(stream);
+}
+
 void* workspace(size_t bytes, hipStream_t stream) {
-    struct Slot { int dev; hipStream_t stream; void* buf; size_t cap; };
-    static std::mutex mu;
-    static std::vector<Slot> slots;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0) { set_error("workspace: no current device"); return nullptr; }
-    std::lock_guard<std::mutex> lock(mu);
+    std::lock_guard<std::mutex> lock(g_slot_mu);
     Slot* slot = nullptr;
-    for (Slot& c : slots) if (c.dev == dev && c.stream == stream) { slot = &c; break; }
-    if (!slot) { slots.push_back(Slot{dev, stream, nullptr, 0}); slot = &slots.back(); }
+    for (Slot& c : g_slots) if (c.dev == dev && c.stream == stream) { slot = &c; break; }
+    if (!slot) { g_slots.push_back(Slot{dev, stream, nullptr, 0}); slot = &g_slots.back(); }
     if (slot->cap < bytes) {
         // nothing may be allocated or waited for while the stream records a graph: the caller runs the same
         // call once on this stream beforehand, which sizes the buffer
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(stream, &cap) != hipSuccess) (void)hipGetLastError();
-        if (cap != hipStreamCaptureStatusNone) {
+        if (capturing(stream)) {
             set_error("workspace: %zu bytes needed while the stream is capturing; run the call once on this stream before the capture", bytes);
             return nullptr;
         }
@@ -119,12 +136,6 @@ struct HintSlot {
 std::mutex g_hint_mu;
 std::vector<HintSlot> g_hints;
 unsigned long long g_hint_clock = 0;
-
-bool capturing(hipStream_t stream) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &cap) != hipSuccess) { (void)hipGetLastError(); return false; }
-    return cap != hipStreamCaptureStatusNone;
-}
 
 // A slot that is handed to another layer keeps its pinned memory and events (copies into them may still be on their
 // way); what is queued at that moment is counted as stale and thrown away when it arrives.

@@ -6,6 +6,8 @@ several times on new input contents, with eager work between the replays; every 
 results (bit for bit for the l-inf values and positions, to the gradient tolerance for the atomically
 accumulated sums).  The library zero-fills with a kernel, never a memset node.  The workspace is kept per
 (device, stream), so calls queued on two streams may overlap: the second test checks that."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -399,3 +401,40 @@ def test_two_host_threads_on_one_stream_leave_results_unchanged():
         for k, outs in enumerate(got[i]):
             for a, b in zip(outs, alone[i]):
                 assert torch.equal(a, b), "thread %d, call %d" % (i, k)
+
+
+def _captured_on_a_new_stream(call, outs):
+    """Captures the call on a stream that the library has not seen, so that no scratch is at hand; returns what a replay
+    leaves in `outs`, and what the eager call does."""
+    from sortnet_amd import _lib
+    handle = ctypes.c_void_p()
+    assert _lib.load().hipStreamCreate(ctypes.byref(handle)) == 0      # from the runtime that the library binds; kept
+    stream = torch.cuda.ExternalStream(handle.value)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        call()
+    results = []
+    for _ in range(3):
+        for o in outs:
+            o.fill_(5)
+        graph.replay()
+        torch.cuda.synchronize()
+        results.append([o.clone() for o in outs])
+    for o in outs:
+        o.fill_(6)
+    call()
+    torch.cuda.synchronize()
+    return results, [o.clone() for o in outs]
+
+
+# rows of 1001 inputs are not loaded by 16 bytes; the first is streamed where scratch for its keep bits is at hand
+@pytest.mark.parametrize("B,n,m", [(8, 1001, 50), (512, 1001, 200), (33, 37, 4001)])
+def test_masked_layer_without_positions_is_captured_unprepared(B, n, m):
+    from sortnet_amd import ext
+    dev = _dev()
+    g = torch.Generator().manual_seed(n + m)
+    x, w, y = torch.randn(B, n, 1, generator=g).to(dev), torch.randn(m, n, generator=g).to(dev), torch.empty(B, m, 1, device=dev)
+    replays, eager = _captured_on_a_new_stream(lambda: ext.masked_inf_dist_forward(x, w, y, None, 1, 0.4, 7, ext.MASK_FACTORED), [y])
+    for r in replays:
+        assert torch.equal(r[0], eager[0])
