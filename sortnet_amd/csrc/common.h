@@ -52,6 +52,7 @@ struct FwdArgs {
     int COg, CIg;         // per-group output / input channels (compact sizes with index lists)
     int W_COg, W_CIg;     // per-group rows / row length of the weight tensor
     int nsplit;           // number of slices the reduction range is cut in (grid.z = G * nsplit)
+    int coarse;           // slices of four chunks at least: the scratch that more of them merge in is not at hand
     int fast_x, fast_w;   // 128-bit loads allowed for the x / w tiles
     float p, inv_p, q;
     float skip_thr;       // l-p, large p: ratios to the running scale below this cannot change the fp32 result (0 = unused)

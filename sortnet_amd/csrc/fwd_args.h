@@ -62,7 +62,7 @@ inline int pick_nsplit(const FwdArgs& a, int BB, int BM, int per_cu = 8) {
     // interval bounds on 256 x 10240 x 200 103 -> 68.  Four workgroups per unit were slower from 128 x 3072 x 1024 on
     // (l-inf 27 -> 33), one per unit below (p = 8 on 90 x 1600 x 230 18 -> 27).
     const long long fill = (per_cu > 1 ? 2ll : 1ll) * num_cus();
-    if (tiles * ns < fill && aligned16(a.y0) && aligned16(a.y1)) {   // (a merge by maximum starts from filled outputs)
+    if (!a.coarse && tiles * ns < fill && aligned16(a.y0) && aligned16(a.y1)) {   // (a merge by maximum starts from filled outputs)
         long long more = (fill + tiles - 1) / tiles;
         if (more > chunks) more = chunks;
         if (more > 64) more = 64;

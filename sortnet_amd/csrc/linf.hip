@@ -154,8 +154,13 @@ static int run_chunk_pos(FwdArgs& a, bool index_lists, hipStream_t st, void* mer
     // which loads a chunk only when the one before it is done)
     const bool gather = P::LISTS && (index_lists || a.mask_mode < 0) && !(a.fast_x && a.fast_w);
     const int TB = index_lists || narrow || gather ? 2 : pick_tb(a, kTb42, 2, 16 * P::WIDE_TM);
-    if (narrow) a.nsplit = pick_nsplit(a, 32, 32);
-    else a.nsplit = TB == 2 ? pick_nsplit(a, 32, gather ? 128 : 16 * P::WIDE_TM, gather && index_lists ? 1 : 8) : pick_nsplit(a, 16 * P::WIDE_TB, 16 * P::WIDE_TM);
+    auto slices = [&] {
+        if (narrow) return pick_nsplit(a, 32, 32);
+        return TB == 2 ? pick_nsplit(a, 32, gather ? 128 : 16 * P::WIDE_TM, gather && index_lists ? 1 : 8) : pick_nsplit(a, 16 * P::WIDE_TB, 16 * P::WIDE_TM);
+    };
+    a.nsplit = slices();
+    // (what went in one slice needs no scratch, so a stream under capture must not ask for it)
+    if (a.nsplit > 1 && !merge_buf && !a.xmask && !workspace_ready((size_t)a.R * a.G * a.COg * 8, st)) { a.coarse = 1; a.nsplit = slices(); }
     // dense exact tiles of the l-inf policy: LDS-direct kernel with 4 x 8 outputs per work-item and the chunk numbers
     // packed four to a register (same (value, chunk) results, so the same resolve pass follows)
     bool packed_direct = false;
@@ -469,6 +474,7 @@ extern "C" int sd_bound_inf_dist_forward(const float* inputL, const float* input
     const bool narrow = narrow_tiles(a);
     const int TB = narrow ? 2 : pick_tb(a, kTb42, 2, 64);
     a.nsplit = pick_nsplit(a, 16 * TB, narrow ? 32 : 64);
+    if (a.nsplit > 1 && !workspace_ready((size_t)a.R * a.G * a.COg * 16, st)) { a.coarse = 1; a.nsplit = pick_nsplit(a, 16 * TB, narrow ? 32 : 64); }
     // dense single-group layers: the table kernel, tracking the chunk of every result, is queued in front
     // of the every-term kernel as for the forward without positions; both leave (value, chunk) pairs for the resolve
     const float bound_density = g_bound_density.load(std::memory_order_relaxed);

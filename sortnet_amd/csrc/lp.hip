@@ -104,9 +104,11 @@ __global__ void __launch_bounds__(256) lp_finalize_kernel(const float* __restric
 // library workspace and are merged by lp_finalize_kernel
 static int lp_split_setup(FwdArgs& a, int BB, int BM, bool online, hipStream_t st) {
     a.nsplit = pick_nsplit(a, BB, BM);
+    a.part_stride = (size_t)a.R * a.G * a.COg;
+    auto bytes = [&] { return a.part_stride * a.nsplit * (online ? 2 : 1) * sizeof(float); };
+    if (a.nsplit > 1 && !workspace_ready(bytes(), st)) { a.coarse = 1; a.nsplit = pick_nsplit(a, BB, BM); }
     if (a.nsplit > 1) {
-        a.part_stride = (size_t)a.R * a.G * a.COg;
-        a.part0 = static_cast<float*>(workspace(a.part_stride * a.nsplit * (online ? 2 : 1) * sizeof(float), st));
+        a.part0 = static_cast<float*>(workspace(bytes(), st));
         if (!a.part0) return SD_ERR_HIP;
         a.part1 = online ? a.part0 + a.part_stride * a.nsplit : nullptr;
     }
@@ -139,10 +141,18 @@ static int lp_forward_max_first(FwdArgs& a, bool small, hipStream_t st) {
     a.nsplit = m.nsplit;
     const int ns_rows = rows ? lp_rows_forward_nsplit(a.R, a.COg, a.CIg) : 1;
     // maxima, then the slice results of whichever sum kernel runs (the table kernel leaves two values per slice)
-    const int slots = a.nsplit > 1 ? a.nsplit : 0, slots_rows = ns_rows > 1 ? 2 * ns_rows : 0;
-    const size_t head = total * (size_t)(1 + (slots > slots_rows ? slots : slots_rows)) * sizeof(float);
-    const size_t head_al = (head + 255) / 256 * 256;
-    float* base = static_cast<float*>(workspace(head_al + (rows ? lp_rows_workspace(a.R, a.COg, a.CIg) : 0), st));
+    const size_t table_bytes = rows ? lp_rows_workspace(a.R, a.COg, a.CIg) : 0;
+    auto head_bytes = [&] {
+        const int slots = a.nsplit > 1 ? a.nsplit : 0, slots_rows = ns_rows > 1 ? 2 * ns_rows : 0;
+        const size_t head = total * (size_t)(1 + (slots > slots_rows ? slots : slots_rows)) * sizeof(float);
+        return (head + 255) / 256 * 256;
+    };
+    if (!workspace_ready(head_bytes() + table_bytes, st)) {
+        m.coarse = 1;
+        a.nsplit = m.nsplit = pick_nsplit(m, small || narrow ? 32 : 64, narrow ? 32 : 128);
+    }
+    const size_t head_al = head_bytes();
+    float* base = static_cast<float*>(workspace(head_al + table_bytes, st));
     if (!base) return SD_ERR_HIP;
     int rc;
     if (rows) {

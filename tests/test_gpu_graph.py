@@ -438,3 +438,32 @@ def test_masked_layer_without_positions_is_captured_unprepared(B, n, m):
     replays, eager = _captured_on_a_new_stream(lambda: ext.masked_inf_dist_forward(x, w, y, None, 1, 0.4, 7, ext.MASK_FACTORED), [y])
     for r in replays:
         assert torch.equal(r[0], eager[0])
+
+
+@pytest.mark.parametrize("op", ["positions", "masked positions", "bounds", "power", "power gradients"])
+def test_layers_of_one_slice_are_captured_unprepared(op):
+    """Few inputs: cut in slices where scratch to merge them in is at hand, and in one piece, without scratch, where not."""
+    from sortnet_amd import ext
+    dev = _dev()
+    g = torch.Generator().manual_seed(3)
+    B, n, m, hw = 20, 200, 310, 4 if op != "masked positions" else 1
+    x, w, gy = (t.to(dev) for t in (torch.randn(B, n, hw, generator=g), torch.randn(m, n, generator=g), torch.randn(B, m, hw, generator=g)))
+    y, y2, p, p2 = (torch.empty(B, m, hw, device=dev, dtype=t) for t in (torch.float32,) * 2 + (torch.int32,) * 2)
+    gx, gw = torch.empty_like(x), torch.empty_like(w)
+    if op == "positions":
+        replays, eager = _captured_on_a_new_stream(lambda: ext.inf_dist_forward(x, w, y, p, 1), [y, p])
+    elif op == "masked positions":
+        replays, eager = _captured_on_a_new_stream(lambda: ext.masked_inf_dist_forward(x, w, y, p, 1, 0.4, 7, ext.MASK_TERM), [y, p])
+    elif op == "bounds":
+        replays, eager = _captured_on_a_new_stream(lambda: ext.bound_inf_dist_forward(x, x + 0.1, w, y, y2, p, p2, 1), [y, y2, p, p2])
+    elif op == "power":
+        replays, eager = _captured_on_a_new_stream(lambda: ext.norm_dist_forward(x, w, y, 1, 3.0), [y])
+    else:
+        ext.norm_dist_forward(x, w, y, 1, 3.0)
+        replays, eager = _captured_on_a_new_stream(lambda: ext.norm_dist_backward_input_weight(gy, x, w, y, gx, gw, 1, 3.0), [gx, gw])
+    for r in replays:
+        for got, ref in zip(r, eager):
+            if "power" in op:      # the same addends in another order
+                _close(got, ref, op)
+            else:
+                assert torch.equal(got, ref)
