@@ -73,15 +73,24 @@ inline int pick_nsplit(const FwdArgs& a, int BB, int BM, int per_cu = 8) {
 
 // Whether the forward runs on tiles of 32 x 32 outputs (2 x 2 per work-item) instead of 32 or 64 x 64 or 128: up to as
 // many chunks of 32 x 128 outputs as 32 per compute unit.  The narrow tile reads more LDS per term but pads less, fills
-// the device with fewer slices and keeps more wavefronts in flight.  In us, wide -> narrow: l-inf on 300 x 1001 x 777
-// (21 chunks per unit) 31 -> 20, on 250 x 3072 x 1021 (24) 45 -> 41 and with positions 67 -> 54, interval bounds with
-// positions 137 -> 107; p = 100 on 40 x 5000 x 2000 (20) 265 -> 199; the one loss seen is 7 % (interval bounds,
-// 256 x 10240 x 200).  Larger layers keep the wide tiles, whose LDS traffic per term decides there.  What the gather kernel
-// serves goes narrow up to twice that size: its wide tile holds fewer wavefronts than the vector kernels' (512 rows of four
-// positions, 2700 inputs, 1024 channels (42): forward, backward and unfolding 184 -> 159).
+// the device with fewer slices and keeps more wavefronts in flight; larger layers keep the wide tiles, whose LDS traffic per
+// term decides there.  Time on narrow over time on wide tiles, vector loads:
+//   chunks per unit             4     24 (250 x 3072 x 1021)  24 (256 x 3072 x 1024)  32 (512 x 2048 x 1024)  48     72
+//   l-inf                       0.78  0.89                    1.03                    1.08                    1.19   1.30
+//   l-inf with positions        0.91  0.80                    0.84                    0.85                    1.02   1.05
+//   interval / with positions   0.81  0.97 / 0.77             1.07 / 0.96             1.08 / 0.98             1.14   1.16
+//   l-p, p = 8 / p = 24         0.85  0.98 / 0.96             0.99                    1.04 / 1.02             1.06   1.05
+//   masked / with positions     -     0.88 / 0.81             -                       1.03 / 0.84             1.13   1.17
+// The scalar-load kernels (index lists, several positions per sample, rows that are no multiple of 16 bytes) hold fewer wavefronts
+// with their wide tile and go narrow up to twice that size.  Between 32 and 64 chunks per unit: lists p = inf 0.71 to 0.81,
+// p = 8 0.95 to 0.99, p = 24 0.94 to 0.98; l-inf 0.50 to 0.87, with positions 0.80 to 0.86, p = 8 0.55 to 1.00; interval
+// with positions 0.78 to 0.94, without 0.44 to 0.99 and, on four of nine shapes, 1.04 to 1.11; mask per term 0.94 to 0.98.
+// (Above 64: lists at p = 8 1.04 to 1.07, l-p 1.06 to 1.11, interval 1.07 to 1.29.)  Under the factored mask, whose keep
+// bits are drawn as a tile is staged, and a narrow one is staged more often, they keep the first limit: there 0.93 to 1.20.
 inline bool narrow_tiles(const FwdArgs& a) {
     const long long tiles = (long long)((a.R + 31) / 32) * ((a.COg + 127) / 128) * a.G;
-    return tiles * ((a.CIg + 31) / 32) < (a.fast_x && a.fast_w ? 32ll : 64ll) * num_cus();
+    const bool vector = a.fast_x && a.fast_w;
+    return tiles * ((a.CIg + 31) / 32) < (vector || a.mask_mode == SD_MASK_FACTORED ? 32ll : 64ll) * num_cus();
 }
 
 // rows per work-item (batch tile = 16 * TB rows): the largest candidate whose tiles, after split-N,
