@@ -217,9 +217,9 @@ struct LpBwdArgs {
     const float* ry;                  // 1 / y when the caller already holds it, else null
     bool gx_is_zero;                  // grad_input (and grad_weight) were zero-filled by the caller
     int zsplit;      // slices of the output-channel range
-    float* gx_part;  // a plane of grad_input per slice, gx_plane apart, that lp_merge_kernel adds up; null: slices add to gx
-    float* gw_part;  // a plane of grad_weight per batch tile, gw_plane apart; null: batch tiles add to gw
-    size_t gx_plane, gw_plane;
+    // floats between the planes of grad_input (one per slice) and grad_weight (one per batch tile) that gx and gw then point
+    // to and lp_merge_kernel adds up; 0: slices and batch tiles add to gx and gw
+    unsigned gx_plane, gw_plane;
 };
 
 // what becomes of the sums over a batch tile that make up grad_weight
@@ -344,7 +344,7 @@ __global__ void __launch_bounds__(256, (SKIP ? 4 : 1)) lp_bwd_kernel(LpBwdArgs a
     const int* __restrict__ co = a.co_idx ? a.co_idx + (size_t)(s * a.G + g) * a.COg : nullptr;
     const float* __restrict__ wcolp = a.w + (size_t)g * a.W_COg * a.W_CIg + wcol;
     float* __restrict__ gwcol = GW == kGwNone ? nullptr
-        : (GW == kGwStore ? a.gw_part + blockIdx.y * a.gw_plane : a.gw) + (size_t)g * a.W_COg * a.W_CIg + wcol;
+        : a.gw + (GW == kGwStore ? (size_t)blockIdx.y * a.gw_plane : (size_t)0) + (size_t)g * a.W_COg * a.W_CIg + wcol;
     // weight row of output channel m0 + (lane mod MC), clamped into the slice so that every load stays inside W
     const int kl = tid & (MC - 1);
     auto row_of = [&](int m0) {
@@ -412,8 +412,8 @@ __global__ void __launch_bounds__(256, (SKIP ? 4 : 1)) lp_bwd_kernel(LpBwdArgs a
         rown = rownn;
     }
     if (n_ok) {
-        float* gx = a.gx_part ? a.gx_part + slice * a.gx_plane : a.gx;
-        const bool add = a.zsplit > 1 && !a.gx_part;
+        float* gx = a.gx + (size_t)slice * a.gx_plane;
+        const bool add = a.zsplit > 1 && a.gx_plane == 0;
         #pragma unroll
         for (int i = 0; i < RB; i++) {
             if (i < rows) {
@@ -717,31 +717,33 @@ static int launch_lp_bwd(int ip, const LpBwdArgs& a, hipStream_t st) {
 // the general kernel as `plan` cuts it; `part`: room for the planes
 static int run_lp_bwd(int ip, LpBwdArgs& a, const LpBwdPlan& plan, float* part, hipStream_t st) {
     a.zsplit = plan.zsplit;
-    a.gx_plane = plan.gx_plane; a.gw_plane = plan.gw_plane;
-    a.gx_part = plan.gx_words ? part : nullptr;
-    a.gw_part = plan.gw_words ? part + plan.gx_words : nullptr;
-    const size_t w_words = a.gw ? (size_t)a.G * a.W_COg * a.W_CIg : 0;
+    a.gx_plane = (unsigned)plan.gx_plane; a.gw_plane = (unsigned)plan.gw_plane;
+    float *gx = a.gx, *const gw = a.gw;
+    float *const gx_part = plan.gx_words ? part : nullptr, *const gw_part = plan.gw_words ? part + plan.gx_words : nullptr;
+    const size_t w_words = gw ? (size_t)a.G * a.W_COg * a.W_CIg : 0;
     int rc = SD_OK;
     if (!a.gx_is_zero) {   // what atomics add to
-        const size_t nx = a.zsplit > 1 && !a.gx_part ? (size_t)a.R * a.G * a.CIg : 0, nw = a.gw_part ? 0 : w_words;
-        if (nx && nw) rc = fill_zero2(a.gx, nx, a.gw, nw, st);
-        else if (nx + nw) rc = nx ? fill_zero(a.gx, nx, st) : fill_zero(a.gw, nw, st);
+        const size_t nx = a.zsplit > 1 && !gx_part ? (size_t)a.R * a.G * a.CIg : 0, nw = gw_part ? 0 : w_words;
+        if (nx && nw) rc = fill_zero2(gx, nx, gw, nw, st);
+        else if (nx + nw) rc = nx ? fill_zero(gx, nx, st) : fill_zero(gw, nw, st);
         if (rc) return rc;
     }
     for (int left = a.R, first = 1; left > 0; left -= plan.rows, first = 0) {
         a.R = left < plan.rows ? left : plan.rows;
-        rc = !a.gw ? launch_lp_bwd<kGwNone>(ip, a, st) : a.gw_part ? launch_lp_bwd<kGwStore>(ip, a, st) : launch_lp_bwd<kGwAdd>(ip, a, st);
+        a.gx = gx_part ? gx_part : gx;
+        a.gw = gw_part ? gw_part : gw;
+        rc = !gw ? launch_lp_bwd<kGwNone>(ip, a, st) : gw_part ? launch_lp_bwd<kGwStore>(ip, a, st) : launch_lp_bwd<kGwAdd>(ip, a, st);
         if (rc) return rc;
         const size_t x_words = (size_t)a.R * a.G * a.CIg;
         if (plan.words()) {
             LpMerge mx{}, mw{};
-            if (a.gx_part) mx = LpMerge{a.gx_part, a.gx, x_words, plan.gx_plane, a.zsplit, (unsigned)((x_words + 255) / 256), false};
-            if (a.gw_part) mw = LpMerge{a.gw_part, a.gw, w_words, plan.gw_plane, (a.R + RB - 1) / RB, (unsigned)((w_words + 255) / 256), !first};
+            if (gx_part) mx = LpMerge{gx_part, gx, x_words, plan.gx_plane, a.zsplit, (unsigned)((x_words + 255) / 256), false};
+            if (gw_part) mw = LpMerge{gw_part, gw, w_words, plan.gw_plane, (a.R + RB - 1) / RB, (unsigned)((w_words + 255) / 256), !first};
             hipLaunchKernelGGL(lp_merge_kernel, dim3(mx.blocks + mw.blocks), dim3(256), 0, st, mx, mw, a.gate, a.gate_limit, a.gate_above);
             if ((rc = check_launch("lp_merge_kernel"))) return rc;
         }
         // (only dense single-group layers are taken in several launches)
-        a.x += x_words; a.gx += x_words;
+        a.x += x_words; gx += x_words;
         a.gy += (size_t)a.R * a.COg; a.y += (size_t)a.R * a.COg;
     }
     return SD_OK;
