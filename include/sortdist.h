@@ -36,7 +36,8 @@
  * The sd_set_* limits are process-wide atomics that a call reads once when it starts; per-layer
  * table hints (which of two queued kernels has been running lately) are kept for the 256 most
  * recently used (entry point, weight pointer, shape) triples and never change a result.  A call that would have to grow the buffer while its stream is being captured
- * into a graph fails with SD_ERR_HIP: run it once on that stream before the capture.
+ * into a graph fails with SD_ERR_HIP: run it once on that stream before the capture.  Calls that use scratch only to be
+ * faster (finer slices, partial gradients merged in order) do without it there.
  * Outputs that are zero-filled or merged with 128-bit stores must be 16-byte aligned.
  */
 #ifndef SORTDIST_H

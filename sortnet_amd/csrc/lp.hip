@@ -12,7 +12,7 @@ namespace sd {
 // smallest thresholds from which the significance tests paid at B = 512, M = N = 5120 (p of about 32 for the
 // vector-load forward, about 77 for the two-pass forward of the index lists)
 constexpr float kLpSkipFrom = 0.5f, kLpSkipFromOnline = 0.75f;
-// backward: the dense both-gradient kernel (p of about 65) and the general kernel (p of about 80)
+// backward: the dense both-gradient kernel (p of about 97) and the general kernel (p of about 118)
 constexpr float kLpSkipFromFused = 0.68f, kLpSkipFromGeneral = 0.73f;
 
 // largest share of marked (tile, row, input) triples at which the candidate-table kernels run instead of the
