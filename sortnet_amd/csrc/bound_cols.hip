@@ -1,5 +1,6 @@
 // Interval-bound forward from per-weight-row candidate tables (see bound_cols.h).
 #include "bound_cols.h"
+#include "cand_walk.h"
 
 namespace sd {
 
@@ -696,29 +697,26 @@ __global__ void __launch_bounds__(1024) sum_tables_kernel(const uint32_t* __rest
 }
 
 // Main kernel of this orientation.  A wavefront takes one batch row against the tile's 128 weight rows (lane l holds the
-// rows l and l + 64): it reads the row's table words 64 chunks at a time, lists the marked inputs in LDS and walks the
-// list four marks at a time with the loads of the next four in flight: lane l fetches the number and the (l, u) of mark
-// l % 4 (read back lane by lane, so they are scalar operands of the terms), every lane its two weights from the
-// transposed copy (two coalesced 256-byte loads per mark).  No tile is staged and no barrier is met; the workgroups of a
-// tile (eight wavefronts = eight batch rows each) are dealt to one die, whose cache then holds the tile's transposed
-// weights.  Every load is issued unconditionally (groups past the end of the list repeat its last mark and are not
-// used).  One wavefront sees every input of its outputs, so the results are stored, not merged.
+// rows l and l + 64): it lists the row's marked inputs in LDS, cuts the list by what a few strong marks say (cand_walk.h) and
+// walks what is left: per mark the row's (l, u) (scalar operands) and the lane's two weights from the transposed copy (two
+// coalesced 256-byte loads).  No tile is staged and no barrier is met; the workgroups of a tile (eight wavefronts = eight
+// batch rows each) are dealt to one die, whose cache then holds the tile's transposed weights.  One wavefront sees every
+// input of its outputs, so the results are stored, not merged.
 // POS: the mark that last improved a bound strictly is the first input attaining it (the marks go by in input order,
 // and every input that attains a bound is marked), so values and positions are stored as they are
 // (core/cuda/bound_inf_dist_cuda.cu:176-212: position = input | bit 31 when w - l > u - w; a lower bound that never
 // left its floor keeps 0xffffffff) and the resolve pass is told to skip the call (count[4]).
 constexpr int kWalkWaves = 8;        // wavefronts of a workgroup
-constexpr int kWalkBatch = 64;       // chunks whose table words a wavefront reads at a time, one per lane
-constexpr int kWalkListCap = 2304;   // entries of a wavefront's list of marked inputs (16-bit input numbers)
 
 template <bool POS>
 __global__ void __launch_bounds__(64 * kWalkWaves)
 bound_rows_walk_kernel(const float* __restrict__ xl, const float* __restrict__ xu, const float* __restrict__ wt,
-                       const uint32_t* __restrict__ bits, const unsigned long long* __restrict__ count,
-                       unsigned long long limit_col, unsigned long long limit_row, int B, int Bp, int M, int N,
-                       float* __restrict__ yL, float* __restrict__ yU, int* __restrict__ posL, int* __restrict__ posU) {
+                       const float* __restrict__ wr, const uint32_t* __restrict__ bits,
+                       const unsigned long long* __restrict__ count, unsigned long long limit_col,
+                       unsigned long long limit_row, int B, int Bp, int M, int N, float* __restrict__ yL,
+                       float* __restrict__ yU, int* __restrict__ posL, int* __restrict__ posU) {
     if (count[0] <= limit_col || count[1] > limit_row) return;   // the other table's turn, or the every-term kernel's
-    __shared__ uint16_t list[kWalkWaves][kWalkListCap];
+    __shared__ uint16_t lists[kWalkWaves][kWalkListCap];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int NCH = N / kChunk, BG = (B + kWalkWaves - 1) / kWalkWaves;
@@ -728,92 +726,60 @@ bound_rows_walk_kernel(const float* __restrict__ xl, const float* __restrict__ x
     const int b = bg * kWalkWaves + wave;
     if (b >= B) return;   // wave-uniform
     const float* __restrict__ wcol = wt + (size_t)t * N * kTileW + lane;
-    uint16_t* mine = list[wave];
+    uint16_t* list = lists[wave];
     const uint32_t* __restrict__ rowbits = bits + ((size_t)t * Bp + b) * NCH;
     const float* __restrict__ xlrow = xl + (size_t)b * N;
     const float* __restrict__ xurow = xu + (size_t)b * N;
+    const float* __restrict__ wmin = wr + (size_t)(t * 2) * N;
+    const float* __restrict__ wmax = wmin + N;
+    const bool in0 = t * kTileW + lane < M, in1 = t * kTileW + lane + 64 < M;   // the lane's weight rows exist
     float lo[2] = {-kEps, -kEps}, hi[2] = {kEps, kEps};
     int pl[2] = {-1, -1}, pu[2] = {0, 0};   // POS: the input that last improved the bound, with its flag
-    int cnt = 0;   // marks in the list
-    float lreg[2], ureg[2];
-    int nreg[2];
     float wa[2][4], wb[2][4];
-    auto load = [&](int buf, int k0, int total) __attribute__((always_inline)) {
-        int k = k0 + (lane & 3);
-        k = k < total ? k : total - 1;
-        const int nn = (int)mine[k];
-        float l = xlrow[nn], u = xurow[nn];
-        repair(l, u);
-        lreg[buf] = l; ureg[buf] = u; nreg[buf] = nn;
-        #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int n = __builtin_amdgcn_readlane(nn, i);
-            wa[buf][i] = wcol[(size_t)n * kTileW];
-            wb[buf][i] = wcol[(size_t)n * kTileW + 64];
+    auto load = [&](int buf, int i, int n) __attribute__((always_inline)) {
+        wa[buf][i] = wcol[(size_t)n * kTileW];
+        wb[buf][i] = wcol[(size_t)n * kTileW + 64];
+    };
+    auto use = [&](int buf, int i, int k, int n, const Own& o) __attribute__((always_inline)) {
+        const float li = lane_value(o.a, k), ui = lane_value(o.b, k);
+        const float a1 = wa[buf][i] - li, a2 = ui - wa[buf][i], b1 = wb[buf][i] - li, b2 = ui - wb[buf][i];
+        if constexpr (POS) {
+            const int p0 = a1 <= a2 ? n : n | (int)0x80000000, p1 = b1 <= b2 ? n : n | (int)0x80000000;
+            const float v0 = fminf(a1, a2), V0 = fmaxf(a1, a2), v1 = fminf(b1, b2), V1 = fmaxf(b1, b2);
+            const bool w0 = v0 < lo[0], w1 = v1 < lo[1], w2 = V0 > hi[0], w3 = V1 > hi[1];
+            lo[0] = w0 ? v0 : lo[0]; lo[1] = w1 ? v1 : lo[1];
+            hi[0] = w2 ? V0 : hi[0]; hi[1] = w3 ? V1 : hi[1];
+            pl[0] = w0 ? p0 : pl[0]; pl[1] = w1 ? p1 : pl[1];
+            pu[0] = w2 ? p0 : pu[0]; pu[1] = w3 ? p1 : pu[1];
+        } else {
+            lo[0] = fminf(fminf(lo[0], a1), a2);
+            hi[0] = fmaxf(fmaxf(hi[0], a1), a2);
+            lo[1] = fminf(fminf(lo[1], b1), b2);
+            hi[1] = fmaxf(fmaxf(hi[1], b1), b2);
         }
     };
-    auto compute = [&](int buf, int k0, int total) __attribute__((always_inline)) {
-        #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            if (k0 + i < total) {   // wave-uniform
-                const float li = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lreg[buf]), i));
-                const float ui = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ureg[buf]), i));
-                const float a1 = wa[buf][i] - li, a2 = ui - wa[buf][i], b1 = wb[buf][i] - li, b2 = ui - wb[buf][i];
-                if constexpr (POS) {
-                    const int n = __builtin_amdgcn_readlane(nreg[buf], i);
-                    const int p0 = a1 <= a2 ? n : n | (int)0x80000000, p1 = b1 <= b2 ? n : n | (int)0x80000000;
-                    const float v0 = fminf(a1, a2), V0 = fmaxf(a1, a2), v1 = fminf(b1, b2), V1 = fmaxf(b1, b2);
-                    const bool w0 = v0 < lo[0], w1 = v1 < lo[1], w2 = V0 > hi[0], w3 = V1 > hi[1];
-                    lo[0] = w0 ? v0 : lo[0]; lo[1] = w1 ? v1 : lo[1];
-                    hi[0] = w2 ? V0 : hi[0]; hi[1] = w3 ? V1 : hi[1];
-                    pl[0] = w0 ? p0 : pl[0]; pl[1] = w1 ? p1 : pl[1];
-                    pu[0] = w2 ? p0 : pu[0]; pu[1] = w3 ? p1 : pu[1];
-                } else {
-                    lo[0] = fminf(fminf(lo[0], a1), a2);
-                    hi[0] = fmaxf(fmaxf(hi[0], a1), a2);
-                    lo[1] = fminf(fminf(lo[1], b1), b2);
-                    hi[1] = fmaxf(fmaxf(hi[1], b1), b2);
-                }
-            }
-        }
-    };
-    auto walk = [&](int total) __attribute__((always_inline)) {
-        if (total == 0) return;
-        load(0, 0, total);
-        for (int k0 = 0; k0 < total; k0 += 8) {
-            load(1, k0 + 4, total);
-            compute(0, k0, total);
-            load(0, k0 + 8, total);
-            compute(1, k0 + 4, total);
-        }
-    };
-    uint32_t next = lane < NCH ? rowbits[lane] : 0u;
-    for (int c0 = 0; c0 < NCH; c0 += kWalkBatch) {
-        uint32_t word = next;
-        if (c0 + kWalkBatch < NCH) next = c0 + kWalkBatch + lane < NCH ? rowbits[c0 + kWalkBatch + lane] : 0u;
-        // every lane appends the marks of its word behind those of the lanes before it
-        const int mine_n = __builtin_popcount(word);
-        int incl = mine_n;
-        #pragma unroll
-        for (int o = 1; o < kWalkBatch; o <<= 1) {
-            const int v = __shfl_up(incl, o);
-            if (lane >= o) incl += v;
-        }
-        int off = cnt + incl - mine_n;
-        cnt += __builtin_amdgcn_readlane(incl, kWalkBatch - 1);
-        while (word) {
-            const int i = __builtin_ctz(word);
-            word &= word - 1;
-            mine[off++] = (uint16_t)(((c0 + lane) << 5) | i);   // the input's number (rows of at most 65536 inputs)
-        }
-        // a row's marks are walked in one go unless the list could overflow with the next chunks
-        if (cnt > kWalkListCap - kWalkBatch * kChunk || c0 + kWalkBatch >= NCH) {
-            __builtin_amdgcn_wave_barrier();
-            walk(cnt);
-            cnt = 0;
-            __builtin_amdgcn_wave_barrier();   // the reads of the list come before the next marks
-        }
-    }
+    // smallest results of the lane's rows over the wavefront (weight rows past the last one do not count)
+    float thU = 0.f, thL = 0.f;
+    for_marks(list, NCH, lane, [&](int c) __attribute__((always_inline)) { return rowbits[c]; },
+              [&](int total, bool first) __attribute__((always_inline)) {
+        walk_marks<POS, true>(list, total, first, lane,
+            [&](int n) __attribute__((always_inline)) { Own o{xlrow[n], xurow[n]}; repair(o.a, o.b); return o; },
+            // (the two caps of an input differ by the same width nearly everywhere, so the upper one ranks for both)
+            [&](int n, const Own& o) __attribute__((always_inline)) { return fmaxf(wmax[n] - o.a, o.b - wmin[n]); },
+            load, use, use,
+            [&](bool) __attribute__((always_inline)) {
+                thU = wave_min_nonneg(fminf(in0 ? hi[0] : __builtin_inff(), in1 ? hi[1] : __builtin_inff()));
+                thL = wave_min_nonneg(fminf(in0 ? -lo[0] : __builtin_inff(), in1 ? -lo[1] : __builtin_inff()));
+            },
+            [&](int n, const Own& o) __attribute__((always_inline)) {
+                const float a = wmin[n], b = wmax[n];
+                return !(fmaxf(b - o.a, o.b - a) < thU) || !(fmaxf(o.a - a, b - o.b) < thL);
+            },
+            [&]() __attribute__((always_inline)) {
+                lo[0] = lo[1] = -kEps; hi[0] = hi[1] = kEps;
+                pl[0] = pl[1] = -1; pu[0] = pu[1] = 0;
+            });
+    });
     #pragma unroll
     for (int j = 0; j < 2; j++) {
         const int col = t * kTileW + lane + 64 * j;
@@ -902,13 +868,13 @@ int bound_cols_forward(const float* xl, const float* xu, const float* w, int B, 
                            c.order, c.count, limit_col, B, CO, Mp, CI, nsplit, nullptr, nullptr, packedL, packedU);
         if ((rc = check_launch("bound_table_kernel"))) return rc;
         hipLaunchKernelGGL(bound_rows_walk_kernel<true>, dim3((unsigned)(T * BG)), dim3(64 * kWalkWaves), 0, st, xl, xu, c.wt,
-                           c.bits, c.count, limit_col, limit_row, B, Bp, CO, CI, outL, outU, posL, posU);
+                           c.wr, c.bits, c.count, limit_col, limit_row, B, Bp, CO, CI, outL, outU, posL, posU);
         return check_launch("bound_rows_walk_kernel");
     }
     hipLaunchKernelGGL(bound_table_kernel<false>, dim3((unsigned)(wgs * nsplit)), dim3(1024), 0, st, w, c.xt, c.bits, c.order,
                        c.count, limit_col, B, CO, Mp, CI, nsplit, outL, outU, nullptr, nullptr);
     if ((rc = check_launch("bound_table_kernel"))) return rc;
-    hipLaunchKernelGGL(bound_rows_walk_kernel<false>, dim3((unsigned)(T * BG)), dim3(64 * kWalkWaves), 0, st, xl, xu, c.wt, c.bits,
+    hipLaunchKernelGGL(bound_rows_walk_kernel<false>, dim3((unsigned)(T * BG)), dim3(64 * kWalkWaves), 0, st, xl, xu, c.wt, c.wr, c.bits,
                        c.count, limit_col, limit_row, B, Bp, CO, CI, outL, outU, nullptr, nullptr);
     return check_launch("bound_rows_walk_kernel");
 }

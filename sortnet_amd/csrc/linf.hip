@@ -75,8 +75,8 @@ constexpr long long kMaxRowsMinTerms = 1ll << 33;
 
 // bytes of both tables' workspace for one call: per weight row first, per batch row behind it
 static size_t max_tables_bytes(int B, int CO, int CI, int K) {
-    const size_t cols = (max_cols_workspace(B, CO, CI, K) + 255) / 256 * 256;
-    return cols + (row_cands_supported(kRowsMax, K) ? (row_cands_workspace(kRowsMax, B, CO, CI, K) + 255) / 256 * 256 : 0);
+    const size_t cols = (sort_cols_workspace(B, CO, CI) + 255) / 256 * 256;
+    return cols + (row_cands_supported(kRowsMax, K) ? (row_cands_workspace(kRowsMax, B, CO, CI) + 255) / 256 * 256 : 0);
 }
 
 // `ws`: max_tables_bytes() bytes.  Afterwards a.gate[0] is non-zero when the every-term kernels are to run.
@@ -94,7 +94,7 @@ static int queue_max_cols(FwdArgs& a, int K, int B, int CO, int CI, void* ws, hi
         return rc;
     }
     const unsigned long long* col_count = a.gate;
-    char* rows_ws = static_cast<char*>(ws) + (max_cols_workspace(B, CO, CI, K) + 255) / 256 * 256;
+    char* rows_ws = static_cast<char*>(ws) + (sort_cols_workspace(B, CO, CI) + 255) / 256 * 256;
     const unsigned long long* every = nullptr;
     rc = row_cands_forward(kRowsMax, a.x0, nullptr, a.w, xkeep, wkeep, B, CO, CI, 0.f, K, nullptr, a.y0, a.p0, rows_ws,
                            density > 0.f ? density : kMaxRowsCap, density > 0.f, sort_cols_probe_sums(col_count), col_count, &every, st);
@@ -399,7 +399,7 @@ extern "C" int sd_bound_inf_dist_forward_nograd(const float* inputL, const float
     // which always builds the staged tables, never needs more than the eager call before it did.
     char* wsbase = nullptr;
     if (cols) {
-        const size_t staged = bound_cols_workspace(B, CO, CI), walk = CI <= 65536 ? sort_cols_workspace(B, CO, CI, 1) : 0;
+        const size_t staged = bound_cols_workspace(B, CO, CI), walk = CI <= 65536 ? sort_cols_workspace(B, CO, CI) : 0;
         wsbase = static_cast<char*>(workspace(staged > walk ? staged : walk, st));   // the only request of this call
         if (!wsbase) return SD_ERR_HIP;
     }

@@ -28,7 +28,7 @@ enum RowCandsForm {
 };
 
 // bytes of workspace row_cands_forward needs
-size_t row_cands_workspace(int form, int B, int CO, int CI, int K);
+size_t row_cands_workspace(int form, int B, int CO, int CI);
 
 // True when this build has a main kernel for (form, K): the sort-neuron forms for K = 2 .. 25, the l-inf form for the
 // depths of max_cols_depth.

@@ -1,5 +1,8 @@
 // Sort neuron, its interval bounds and the l-inf forward from candidate tables per batch row (see row_cands.h).
 #include "row_cands.h"
+#include <type_traits>
+#include "cand_tables.h"
+#include "cand_walk.h"
 #include "fwd_tile.h"
 
 namespace sd {
@@ -9,56 +12,52 @@ namespace {
 constexpr int kChunk = kRowCandsChunk;
 constexpr int kTileW = 128;          // weight rows of a tile: 64 lanes x 2
 constexpr int kBPad = 128;           // batch rows are padded to a multiple of this in the tables
-constexpr int kMaxPer = 32;          // most chunks a slice of the table kernels covers
 
 inline size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 inline int tiles_w(int M) { return (M + kTileW - 1) / kTileW; }
 inline int bpad_of(int B) { return (B + kBPad - 1) / kBPad * kBPad; }
-inline int slices_of(int NCH) {
-    int s = (NCH + kMaxPer - 1) / kMaxPer;
-    if (s < 16) s = 16;
-    return s < NCH ? s : NCH;
-}
+// Counters.  Zeroed by rc_range_kernel, which is queued in front of the tables.
+struct RowCount {
+    unsigned long long marks;      // all ones when the table was not built
+    unsigned long long every;      // 1: the every-term kernels run
+    unsigned long long run;        // 1: this table's kernel runs
+    unsigned long long col_marks;  // marks per weight row (copy)
+    unsigned long long fixes;      // outputs to recompute
+    unsigned long long sum;        // see add_marks
+};
 
 struct Carve {
-    float* wr;        // [T][2][N]  per tile of weight rows and input: min w, max w over the rows that keep the input
-    float* lists;     // [T][slices][nw][K][Bp]  K largest chunk maxima of the lower bounds of a batch row's terms within a slice
-    float* low;       // [T][nw][Bp]  K-th largest of them over all slices: upper list, lower list
-    uint32_t* bits;   // [T][Bp][NCH] bit i of a word = input 32 c + i may be among the K largest of that batch row in that tile
-    uint32_t* partial;            // marks per wavefront of the table kernel
-    unsigned long long* count;    // [0] marks, [1] every-term kernels run, [2] this table's kernel runs, [3] marks per weight row (copy), [4] outputs to recompute
+    RowCount* count;
+    float* wr;        // [T][N]  per tile of weight rows and input: (min, max) of the weights over the rows that keep the input
+    float* low;       // [T][Bp]  lower bounds of the K-th largest terms of a batch row
+    uint32_t* bits;   // [T][Bp][table_row_words] the marks
     uint32_t* fix;    // [B * M] outputs of the masked l-inf form whose bound did not hold (recomputed from every input)
     float* wt;        // [T][N][128] the weights of a tile, one 512-byte row per input (dropped weights undefined)
 };
 
-size_t carve_sizes(int form, int B, int M, int N, int K, size_t (&sz)[8]) {
-    const size_t T = tiles_w(M), Bp = bpad_of(B), NCH = N / kChunk, slices = slices_of((int)NCH);
-    const size_t nw = form == kRowsSortInterval ? 2 : 1;
-    sz[0] = align256(T * 2 * N * 4);
-    sz[1] = align256(T * slices * nw * K * Bp * 4);
-    sz[2] = align256(T * nw * Bp * 4);
-    sz[3] = align256(T * NCH * Bp * 4);
-    sz[4] = align256(Bp / 64 * slices * ((T + 3) / 4) * 4 * 4);
-    sz[5] = 256;
-    sz[6] = form == kRowsMax ? align256((size_t)B * M * 4) : 0;
-    sz[7] = align256(T * N * kTileW * 4);
+size_t carve_sizes(int form, int B, int M, int N, size_t (&sz)[6]) {
+    const size_t T = tiles_w(M), Bp = bpad_of(B);
+    sz[0] = 256;
+    sz[1] = align256(T * 2 * N * 4);
+    sz[2] = align256(T * Bp * 4);
+    sz[3] = align256(T * Bp * table_row_words(N) * 4);
+    sz[4] = form == kRowsMax ? align256((size_t)B * M * 4) : 0;
+    sz[5] = align256(T * N * kTileW * 4);
     size_t t = 0;
     for (size_t v : sz) t += v;
     return t;
 }
 
-Carve carve(void* ws, int form, int B, int M, int N, int K) {
-    size_t sz[8];
-    carve_sizes(form, B, M, N, K, sz);
+Carve carve(void* ws, int form, int B, int M, int N) {
+    size_t sz[6];
+    carve_sizes(form, B, M, N, sz);
     char* p = static_cast<char*>(ws);
     Carve c;
-    c.wr = reinterpret_cast<float*>(p); p += sz[0];
-    c.lists = reinterpret_cast<float*>(p); p += sz[1];
+    c.count = reinterpret_cast<RowCount*>(p); p += sz[0];
+    c.wr = reinterpret_cast<float*>(p); p += sz[1];
     c.low = reinterpret_cast<float*>(p); p += sz[2];
     c.bits = reinterpret_cast<uint32_t*>(p); p += sz[3];
-    c.partial = reinterpret_cast<uint32_t*>(p); p += sz[4];
-    c.count = reinterpret_cast<unsigned long long*>(p); p += sz[5];
-    c.fix = reinterpret_cast<uint32_t*>(p); p += sz[6];
+    c.fix = reinterpret_cast<uint32_t*>(p); p += sz[4];
     c.wt = reinterpret_cast<float*>(p);
     return c;
 }
@@ -79,35 +78,19 @@ __device__ __forceinline__ bool rows_decide(const float* stat, int S, float rati
     return stat[0] > ratio * (float)S * stat[1];
 }
 
-// Top-K lists hold their values ascending (res[K-1] largest) and start at 0: new[k] = max(res[k], min(res[k+1], v))
-// (core/cuda/sort_neuron.cu:76-77) = the median of the three.  An undefined v leaves the list unchanged (the
-// median instruction then returns the smallest defined operand), a negative one as well.
-template <int K>
-__device__ __forceinline__ void insert_value(float (&res)[K], float v) {
-    #pragma unroll
-    for (int k = 0; k < K - 1; k++) res[k] = __builtin_amdgcn_fmed3f(res[k], v, res[k + 1]);
-    res[K - 1] = __builtin_amdgcn_fmed3f(res[K - 1], v, __builtin_inff());
-}
-// The same with +infinity held in a register the compiler cannot see through: with the literal it rewrites the last
-// median as a maximum and adds an instruction that quiets res[K - 1] first (two instructions per list and mark).
-template <int K>
-__device__ __forceinline__ void insert_value(float (&res)[K], float v, float inf) {
-    #pragma unroll
-    for (int k = 0; k < K - 1; k++) res[k] = __builtin_amdgcn_fmed3f(res[k], v, res[k + 1]);
-    res[K - 1] = __builtin_amdgcn_fmed3f(res[K - 1], v, inf);
-}
-
 // ---- tables ----------------------------------------------------------------------------------
 // Column ranges of the weights over a tile of 128 weight rows (WMASK: over the rows that keep the input; a column
 // that no row keeps, or that holds an undefined or infinite weight, becomes (-inf, +inf): no lower bound, always a
-// candidate).  64 inputs x 4 groups of 32 rows per workgroup.
+// candidate), and the transposed copy of the tile.  64 inputs x 4 groups of 32 rows per workgroup; a wavefront's keep bits of
+// a row are one or two words, the same for all its lanes.
 template <bool WMASK>
 __global__ void __launch_bounds__(256) rc_range_kernel(const float* __restrict__ w, const uint32_t* __restrict__ wkeep,
                                                        int M, int N, int S, float* __restrict__ wr, float* __restrict__ wt,
-                                                       const float* __restrict__ stat, float ratio) {
+                                                       RowCount* __restrict__ count, const float* __restrict__ stat, float ratio) {
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) count->sum = count->fixes = 0ull;
     if (!rows_decide(stat, S, ratio)) return;
     __shared__ float part[4][3][64];
-    const int nl = threadIdx.x & 63, grp = threadIdx.x >> 6;
+    const int nl = threadIdx.x & 63, grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = blockIdx.x * 64 + nl, t = blockIdx.y;
     const int r0 = t * kTileW + grp * (kTileW / 4);
     float lo = __builtin_inff(), hi = -__builtin_inff(), odd = 0.f;
@@ -115,11 +98,14 @@ __global__ void __launch_bounds__(256) rc_range_kernel(const float* __restrict__
         float v[kTileW / 4];
         #pragma unroll
         for (int i = 0; i < kTileW / 4; i++) v[i] = r0 + i < M ? w[(size_t)(r0 + i) * N + n] : 0.f;
+        const int c0 = blockIdx.x * 2, c1 = c0 + 1 < N / kChunk ? c0 + 1 : c0;
         #pragma unroll
         for (int i = 0; i < kTileW / 4; i++) {
             bool kept = r0 + i < M;
             if constexpr (WMASK) {
-                if (kept) kept = (wkeep[(size_t)(r0 + i) * (N / kChunk) + (n >> 5)] >> (n & 31)) & 1u;
+                const uint32_t* words = wkeep + (size_t)(kept ? r0 + i : M - 1) * (N / kChunk);
+                const unsigned long long both = (unsigned long long)words[c0] | ((unsigned long long)words[c1] << 32);   // wave-uniform
+                kept = kept && ((both >> nl) & 1ull);
             }
             if (kept) { lo = fminf(lo, v[i]); hi = fmaxf(hi, v[i]); odd += v[i] - v[i]; }
             else if (WMASK) v[i] = __builtin_nanf("");
@@ -134,273 +120,46 @@ __global__ void __launch_bounds__(256) rc_range_kernel(const float* __restrict__
         #pragma unroll
         for (int g = 1; g < 4; g++) { lo = fminf(lo, part[g][0][nl]); hi = fmaxf(hi, part[g][1][nl]); odd += part[g][2][nl]; }
         if (!(odd == 0.f) || lo > hi) { lo = -__builtin_inff(); hi = __builtin_inff(); }
-        wr[(size_t)(t * 2) * N + n] = lo;
-        wr[(size_t)(t * 2 + 1) * N + n] = hi;
+        reinterpret_cast<float2*>(wr)[(size_t)t * N + n] = make_float2(lo, hi);
     }
 }
 
-// The two table kernels share their tiling: a workgroup takes 64 batch rows (one per lane; l and u through LDS,
-// repaired) and a slice of the inputs; wavefront v works on weight tile 4 blockIdx.z + v, whose column ranges are
-// LDS broadcasts.
-// Lower bounds.  The smallest a term can be over the weight rows of the tile bounds it from below for every one of
-// them (fp32 subtraction is monotone, so this holds for the rounded terms), and K chunks of inputs whose largest
-// such bound is at least t hold K terms that are at least t for every weight row: the kernel keeps the K largest
-// chunk maxima of the slice (one insertion per 32 inputs), whose K-th largest over all slices bounds the K-th
-// largest term.  Value form: l = u = x.
-// XMASK (l-inf form under the factored mask): xkeep holds one word per (batch row, 32 inputs); an input the batch row
-// does not keep has no term.
-template <int K, bool IV, bool XMASK>
-__global__ void __launch_bounds__(256) rc_low_kernel(const float* __restrict__ xl, const float* __restrict__ xu,
-                                                     const uint32_t* __restrict__ xkeep, const float* __restrict__ wr,
-                                                     int B, int N, int T, int Bp, int S, float* __restrict__ lists,
-                                                     const float* __restrict__ stat, float ratio) {
-    if (!rows_decide(stat, S, ratio)) return;
-    __shared__ __attribute__((aligned(16))) float lt[64][kChunk + 4];
-    __shared__ __attribute__((aligned(16))) float ut[IV ? 64 : 1][kChunk + 4];
-    __shared__ __attribute__((aligned(16))) float ws[4][2][kChunk];
-    const int tid = threadIdx.x, r = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int b0 = blockIdx.x * 64, NCH = N / kChunk;
-    const int slices = gridDim.y, slice = blockIdx.y;
-    const int per = (NCH + slices - 1) / slices;
-    const int c_lo = slice * per, c_hi = c_lo + per < NCH ? c_lo + per : NCH;
-    const int lrow = tid >> 2, q = tid & 3;
-    const int bload = b0 + lrow < B ? b0 + lrow : B - 1;
-    const int brow = b0 + r < B ? b0 + r : B - 1;
-    const int xt = tid >> 6, xk = (tid >> 5) & 1, xn = tid & 31;   // this work-item's value of ws
-    const int tb = blockIdx.z * 4, t = tb + wave;
-    const bool active = t < T;
-    constexpr int nw = IV ? 2 : 1;
-    float hi[K], lo[IV ? K : 1];
-    #pragma unroll
-    for (int k = 0; k < K; k++) { hi[k] = 0.f; if constexpr (IV) lo[k] = 0.f; }
-    float4 la, lb, ua, ub;
-    float px;
-    const float* wsrc = wr + ((size_t)(tb + xt < T ? tb + xt : T - 1) * 2 + xk) * N + xn;
-    auto fetch = [&](int c) {
-        const int cc = c < c_hi ? c : c_hi - 1;
-        const size_t off = (size_t)bload * N + cc * kChunk + 8 * q;
-        la = *reinterpret_cast<const float4*>(xl + off); lb = *reinterpret_cast<const float4*>(xl + off + 4);
-        if constexpr (IV) { ua = *reinterpret_cast<const float4*>(xu + off); ub = *reinterpret_cast<const float4*>(xu + off + 4); }
-        px = wsrc[cc * kChunk];
-    };
-    if (c_lo < c_hi) fetch(c_lo);
-    for (int c = c_lo; c < c_hi; c++) {
-        {
-            float4 a = la, b = lb;
-            if constexpr (IV) {
-                float4 d = ua, e = ub;
-                repair(a.x, d.x); repair(a.y, d.y); repair(a.z, d.z); repair(a.w, d.w);
-                repair(b.x, e.x); repair(b.y, e.y); repair(b.z, e.z); repair(b.w, e.w);
-                *reinterpret_cast<float4*>(&ut[lrow][8 * q]) = d; *reinterpret_cast<float4*>(&ut[lrow][8 * q + 4]) = e;
-            }
-            *reinterpret_cast<float4*>(&lt[lrow][8 * q]) = a; *reinterpret_cast<float4*>(&lt[lrow][8 * q + 4]) = b;
-            ws[xt][xk][xn] = px;
-        }
-        fetch(c + 1);
-        __syncthreads();
-        if (active) {
-            // largest lower bound of the chunk: fmaxf drops undefined differences, and the lists start at 0
-            float cu = 0.f, cl = 0.f;
-            uint32_t kx = ~0u;
-            if constexpr (XMASK) kx = xkeep[(size_t)brow * NCH + c];
-            #pragma unroll
-            for (int n4 = 0; n4 < kChunk; n4 += 4) {
-                const float4 l4 = *reinterpret_cast<const float4*>(&lt[r][n4]);
-                const float4 u4 = IV ? *reinterpret_cast<const float4*>(&ut[IV ? r : 0][n4]) : l4;
-                const float4 a4 = *reinterpret_cast<const float4*>(&ws[wave][0][n4]);   // min w
-                const float4 b4 = *reinterpret_cast<const float4*>(&ws[wave][1][n4]);   // max w
-                const float l[4] = {l4.x, l4.y, l4.z, l4.w}, u[4] = {u4.x, u4.y, u4.z, u4.w};
-                const float wmin[4] = {a4.x, a4.y, a4.z, a4.w}, wmax[4] = {b4.x, b4.y, b4.z, b4.w};
-                #pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    if constexpr (XMASK) {
-                        const float a = fmaxf(wmin[k] - l[k], u[k] - wmax[k]);
-                        cu = fmaxf(cu, ((kx >> (n4 + k)) & 1u) ? a : 0.f);
-                    } else cu = fmaxf(fmaxf(cu, wmin[k] - l[k]), u[k] - wmax[k]);
-                    if constexpr (IV) cl = fmaxf(fmaxf(cl, l[k] - wmax[k]), wmin[k] - u[k]);
-                }
-            }
-            insert_value<K>(hi, cu);
-            if constexpr (IV) insert_value<K>(lo, cl);
-        }
-        __syncthreads();
-    }
-    if (active) {
-        float* dst = lists + (((size_t)t * slices + slice) * nw) * K * Bp + b0 + r;
-        #pragma unroll
-        for (int k = 0; k < K; k++) {
-            dst[(size_t)k * Bp] = hi[k];
-            if constexpr (IV) dst[(size_t)(K + k) * Bp] = lo[k];
-        }
-    }
-}
-
-// K-th largest of the slices' lists (0 when fewer than K lower bounds are positive); grid.y = T * nw
-template <int K>
-__global__ void __launch_bounds__(256) rc_merge_kernel(const float* __restrict__ lists, int slices, int Bp, int nw, int S,
-                                                       float* __restrict__ low, const float* __restrict__ stat, float ratio) {
-    if (!rows_decide(stat, S, ratio)) return;
-    const int b = blockIdx.x * 256 + threadIdx.x;
-    if (b >= Bp) return;
-    const int t = blockIdx.y / nw, which = blockIdx.y % nw;
-    float res[K];
-    #pragma unroll
-    for (int k = 0; k < K; k++) res[k] = 0.f;
-    for (int slice = 0; slice < slices; slice++) {
-        const float* src = lists + ((((size_t)t * slices + slice) * nw + which) * K) * Bp + b;
-        #pragma unroll
-        for (int k = 0; k < K; k++) insert_value<K>(res, src[(size_t)k * Bp]);
-    }
-    low[((size_t)t * nw + which) * Bp + b] = res[0];
-}
-
-// One table word per (tile, chunk, batch row): bit n set when the largest the term of input n can be over the weight
-// rows of the tile reaches the bound of its list and is positive (the lists start at 0 and take larger values only;
-// an undefined bound or term compares false: an undefined term is left out of every list).  Marks counted per
-// wavefront.
-// The words of a (tile, batch row) lie side by side over the chunks, bits[(t Bp + b) NCH + c]: the main kernel reads a
-// row's words 64 at a time.
-template <bool IV, bool XMASK>
-__global__ void __launch_bounds__(256) rc_bits_kernel(const float* __restrict__ xl, const float* __restrict__ xu,
-                                                      const uint32_t* __restrict__ xkeep, const float* __restrict__ wr,
-                                                      const float* __restrict__ low, int B, int N, int T, int Bp, int S,
-                                                      uint32_t* __restrict__ bits, uint32_t* __restrict__ partial,
-                                                      const float* __restrict__ stat, float ratio) {
-    if (!rows_decide(stat, S, ratio)) return;
-    __shared__ __attribute__((aligned(16))) float lt[64][kChunk + 4];
-    __shared__ __attribute__((aligned(16))) float ut[IV ? 64 : 1][kChunk + 4];
-    __shared__ __attribute__((aligned(16))) float ws[4][2][kChunk];
-    const int tid = threadIdx.x, r = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int b0 = blockIdx.x * 64, NCH = N / kChunk;
-    const int slices = gridDim.y, slice = blockIdx.y;
-    const int per = (NCH + slices - 1) / slices;
-    const int c_lo = slice * per, c_hi = c_lo + per < NCH ? c_lo + per : NCH;
-    const int lrow = tid >> 2, q = tid & 3;
-    const int bload = b0 + lrow < B ? b0 + lrow : B - 1;
-    const int brow = b0 + r < B ? b0 + r : B - 1;
-    const bool valid = b0 + r < B;
-    const int xt = tid >> 6, xk = (tid >> 5) & 1, xn = tid & 31;
-    const int tb = blockIdx.z * 4, t = tb + wave;
-    const bool active = t < T;
-    constexpr int nw = IV ? 2 : 1;
-    int marks = 0;
-    float LU = 0.f, LL = 0.f;
-    if (active) {
-        LU = low[((size_t)t * nw) * Bp + b0 + r];
-        if constexpr (IV) LL = low[((size_t)t * nw + 1) * Bp + b0 + r];
-    }
-    float4 la, lb, ua, ub;
-    float px;
-    const float* wsrc = wr + ((size_t)(tb + xt < T ? tb + xt : T - 1) * 2 + xk) * N + xn;
-    auto fetch = [&](int c) {
-        const int cc = c < c_hi ? c : c_hi - 1;
-        const size_t off = (size_t)bload * N + cc * kChunk + 8 * q;
-        la = *reinterpret_cast<const float4*>(xl + off); lb = *reinterpret_cast<const float4*>(xl + off + 4);
-        if constexpr (IV) { ua = *reinterpret_cast<const float4*>(xu + off); ub = *reinterpret_cast<const float4*>(xu + off + 4); }
-        px = wsrc[cc * kChunk];
-    };
-    if (c_lo < c_hi) fetch(c_lo);
-    for (int c = c_lo; c < c_hi; c++) {
-        {
-            float4 a = la, b = lb;
-            if constexpr (IV) {
-                float4 d = ua, e = ub;
-                repair(a.x, d.x); repair(a.y, d.y); repair(a.z, d.z); repair(a.w, d.w);
-                repair(b.x, e.x); repair(b.y, e.y); repair(b.z, e.z); repair(b.w, e.w);
-                *reinterpret_cast<float4*>(&ut[lrow][8 * q]) = d; *reinterpret_cast<float4*>(&ut[lrow][8 * q + 4]) = e;
-            }
-            *reinterpret_cast<float4*>(&lt[lrow][8 * q]) = a; *reinterpret_cast<float4*>(&lt[lrow][8 * q + 4]) = b;
-            ws[xt][xk][xn] = px;
-        }
-        fetch(c + 1);
-        __syncthreads();
-        if (active) {
-            uint32_t word = 0;
-            #pragma unroll
-            for (int n4 = 0; n4 < kChunk; n4 += 4) {
-                const float4 l4 = *reinterpret_cast<const float4*>(&lt[r][n4]);
-                const float4 u4 = IV ? *reinterpret_cast<const float4*>(&ut[IV ? r : 0][n4]) : l4;
-                const float4 a4 = *reinterpret_cast<const float4*>(&ws[wave][0][n4]);
-                const float4 b4 = *reinterpret_cast<const float4*>(&ws[wave][1][n4]);
-                const float l[4] = {l4.x, l4.y, l4.z, l4.w}, u[4] = {u4.x, u4.y, u4.z, u4.w};
-                const float wmin[4] = {a4.x, a4.y, a4.z, a4.w}, wmax[4] = {b4.x, b4.y, b4.z, b4.w};
-                #pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const float capU = fmaxf(wmax[k] - l[k], u[k] - wmin[k]);
-                    bool mark = capU >= LU && capU > 0.f;
-                    if constexpr (IV) {
-                        const float capL = fmaxf(l[k] - wmin[k], wmax[k] - u[k]);
-                        mark = mark || (capL >= LL && capL > 0.f);
-                    }
-                    word |= (uint32_t)mark << (n4 + k);
-                }
-            }
-            if (!valid) word = 0u;
-            if constexpr (XMASK) word &= xkeep[(size_t)brow * NCH + c];
-            bits[((size_t)t * Bp + b0 + r) * NCH + c] = word;
-            marks += __builtin_popcount(word);
-        }
-        __syncthreads();
-    }
-    #pragma unroll
-    for (int o = 32; o; o >>= 1) marks += __shfl_xor(marks, o);
-    if (r == 0) partial[(((size_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * 4 + wave] = (uint32_t)marks;
-}
-
-// count[0] = marks (all ones when the table was not built), count[1] = 1 when the kernels that evaluate every term
-// are to run (neither table is below its limit), count[2] = 1 when this table's kernel runs, count[3] = marks per
-// weight row (copy), count[4] = 0 (the main kernel counts the outputs to recompute there)
-__global__ void __launch_bounds__(1024) rc_sum_kernel(const uint32_t* __restrict__ partial, size_t n,
-                                                      unsigned long long* __restrict__ count,
-                                                      const unsigned long long* __restrict__ col_count,
-                                                      const float* __restrict__ stat, int S, unsigned long long limit,
-                                                      float ratio) {
-    __shared__ unsigned long long acc[1024];
-    const bool rows = rows_decide(stat, S, ratio);
-    unsigned long long s0 = 0;
-    if (rows) for (size_t i = threadIdx.x; i < n; i += 1024) s0 += partial[i];
-    acc[threadIdx.x] = s0;
-    __syncthreads();
-    for (int o = 512; o; o >>= 1) {
-        if ((int)threadIdx.x < o) acc[threadIdx.x] += acc[threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        const bool run = rows && acc[0] <= limit;
-        count[0] = rows ? acc[0] : ~0ull;
-        count[1] = (col_count[1] != 0ull && !run) ? 1ull : 0ull;
-        count[2] = run ? 1ull : 0ull;
-        count[3] = col_count[0];
-        count[4] = 0ull;
-    }
+// Bounds and marks (cand_tables.h): four tiles of weight rows at a time
+template <bool PAIR, bool MASK>
+__global__ void __launch_bounds__(64 * kTableWaves)
+rc_tables_kernel(TableArgs a, RowCount* __restrict__ c, const unsigned long long* __restrict__ col_count,
+                 const float* __restrict__ stat, int S, unsigned long long limit, float ratio) {
+    __shared__ __attribute__((aligned(16))) float smem[4 * 2 * kTableSlice];
+    unsigned long long marks = ~0ull;
+    if (rows_decide(stat, S, ratio)) {
+        const int part = build_tables<1, 4, PAIR, false, MASK>(a, blockIdx.x, blockIdx.y, smem);
+        if (!add_marks(&c->sum, part, &marks)) return;
+    } else if (blockIdx.x != 0 || blockIdx.y != 0 || threadIdx.x != 0) return;
+    const bool run = marks <= limit;   // (the limit is a share of the (tile, row, input) triples: never all ones)
+    c->marks = marks;
+    c->every = (col_count[1] != 0ull && !run) ? 1ull : 0ull;
+    c->run = run ? 1ull : 0ull;
+    c->col_marks = col_count[0];
 }
 
 // ---- main kernel -------------------------------------------------------------------------------
-// A wavefront takes one batch row at a time against the tile's 128 weight rows (lane l holds the rows l and l + 64):
-// it reads the row's table words 64 chunks at a time, lists the marked inputs in LDS and walks the list four marks at
-// a time with the loads of the next four in flight: lane l fetches the number and the row's value(s) of mark l % 4
-// (read back lane by lane, so they are scalar operands of the terms), every lane its two weights from the transposed
-// copy (two coalesced 256-byte loads per mark).  No tile is staged and no barrier is met, so a wavefront with many
-// marks holds nobody up; a workgroup is eight wavefronts = eight batch rows, and the workgroups of a tile are dealt to
-// one die, so that the tile's transposed weights (2.6 MB at 5120 inputs) stay in that die's cache while its 64
-// resident workgroups walk them.  Every load is issued unconditionally (groups past the end of the list repeat its last
-// mark and are not used), so that the waits the compiler places cover exactly the group that is used next.
-// Forms: top-K lists of values (branch-free median insertion), of both interval bounds, of values with the input
-// numbers (the reference's ordered insertion: the marks go by in ascending input order), and the l-inf distance (the
-// difference of largest magnitude and, optionally, its input; under the factored mask the dropped weights of the
-// transposed copy are undefined, the table holds no input the batch row drops, and an output that ends below the bound
-// its marks were taken against is listed for rc_fix_kernel).
+// A wavefront takes one batch row against the tile's 128 weight rows (lane l holds the rows l and l + 64): it lists the
+// row's marked inputs in LDS, cuts the list by what a few strong marks say (cand_walk.h) and walks what is left: per mark
+// the row's value(s) (scalar operands) and the lane's two weights from the transposed copy (two coalesced 256-byte loads).
+// No tile is staged and no barrier is met, so a wavefront with many marks holds nobody up; a workgroup is eight wavefronts
+// = eight batch rows, and the workgroups of a tile are dealt to one die, so that the tile's transposed weights (2.6 MB at
+// 5120 inputs) stay in that die's cache while its 64 resident workgroups walk them.
+// Forms: top-K lists of values (branch-free median insertion, left out where it would change no lane's list), of both
+// interval bounds, of values with the input numbers (the reference's ordered insertion: the marks go by in ascending input
+// order), and the l-inf distance (the difference of largest magnitude and, optionally, its input; under the factored mask the
+// dropped weights of the transposed copy are undefined, the table holds no input the batch row drops, and an output that
+// ends below the bound its marks were taken against is listed for rc_fix_kernel).
 constexpr int kRtWaves = 8;          // wavefronts of a workgroup
-constexpr int kRtRows = 1;           // batch rows a wavefront takes, one after the other
-constexpr int kRtBatch = 64;         // chunks whose table words a wavefront reads at a time, one per lane
-constexpr int kRtListCap = 2304;     // entries of a wavefront's list of marked inputs (16-bit input numbers)
 
 struct RtArgs {
-    const float* xl; const float* xu; const float* wt;
+    const float* xl; const float* xu; const float* wt; const float* wr;
     const uint32_t* bits; const float* low;
-    unsigned long long* count;
+    RowCount* count;
     uint32_t* fix;
     int B, Bp, M, N;
     float q;
@@ -409,38 +168,39 @@ struct RtArgs {
 
 template <int FORM, int K, bool POS, bool MASKED>
 __global__ void __launch_bounds__(64 * kRtWaves) rt_main_kernel(RtArgs a) {
-    if (a.count[2] == 0ull) return;
+    if (a.count->run == 0ull) return;
     constexpr bool IV = FORM == kRowsSortInterval;
     constexpr bool LISTS = FORM != kRowsMax;
-    constexpr bool IDX = FORM == kRowsSortPos || (FORM == kRowsMax && POS);
-    __shared__ uint16_t list[kRtWaves][kRtListCap];
+    constexpr bool ORDERED = FORM == kRowsSortPos || (FORM == kRowsMax && POS);   // the input a term sits at is wanted
+    __shared__ uint16_t lists[kRtWaves][kWalkListCap];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int B = a.B, M = a.M, N = a.N, NCH = N / kChunk;
-    const int BG = (B + kRtWaves * kRtRows - 1) / (kRtWaves * kRtRows);
+    const int BG = (B + kRtWaves - 1) / kRtWaves;
     // consecutive (tile, batch rows) pairs are dealt out so that the workgroups of a tile share a die and its cache
     int item = blockIdx.x;
     if (gridDim.x % 8 == 0) item = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
     const int bg = item % BG, t = item / BG;
+    const int b = bg * kRtWaves + wave;
+    if (b >= B) return;   // wave-uniform
     const float* __restrict__ wcol = a.wt + (size_t)t * N * kTileW + lane;
-    uint16_t* mine = list[wave];
-    float inf = __builtin_inff();
-    asm volatile("" : "+v"(inf));                     // (see insert_value)
+    uint16_t* list = lists[wave];
     const size_t plane = (size_t)B * M;
+    const bool in0 = t * kTileW + lane < M, in1 = t * kTileW + lane + 64 < M;   // the lane's weight rows exist
 
-    for (int rr = 0; rr < kRtRows; rr++) {
-        const int b = (bg * kRtWaves + wave) * kRtRows + rr;
-        if (b >= B) break;   // wave-uniform; the rows of a wavefront ascend
-        // state of the row x the lane's two weight rows: top-K lists (ascending), or the difference of largest magnitude
-        float hi[2][LISTS ? K : 1], lo[IV ? 2 : 1][IV ? K : 1];
-        int idx[IDX ? 2 : 1][FORM == kRowsSortPos ? K : 1];
+    // state of the row x the lane's two weight rows: top-K lists (ascending; as bit patterns where only values are wanted), or
+    // the difference of largest magnitude
+    using Entry = typename std::conditional<FORM == kRowsSortValues || IV, int, float>::type;
+    Entry hi[2][LISTS ? K : 1], lo[IV ? 2 : 1][IV ? K : 1];
+    int idx[ORDERED ? 2 : 1][FORM == kRowsSortPos ? K : 1];
+    auto clear = [&]() __attribute__((always_inline)) {
         #pragma unroll
         for (int j = 0; j < 2; j++) {
             if constexpr (LISTS) {
                 #pragma unroll
                 for (int k = 0; k < K; k++) {
-                    hi[j][k] = 0.f;
-                    if constexpr (IV) lo[j][k] = 0.f;
+                    hi[j][k] = 0;
+                    if constexpr (IV) lo[j][k] = 0;
                     if constexpr (FORM == kRowsSortPos) idx[j][k] = 0;
                 }
             } else {
@@ -448,135 +208,114 @@ __global__ void __launch_bounds__(64 * kRtWaves) rt_main_kernel(RtArgs a) {
                 if constexpr (POS) idx[j][0] = 0;
             }
         }
-        const uint32_t* __restrict__ rowbits = a.bits + ((size_t)t * a.Bp + b) * NCH;
-        const float* __restrict__ xlrow = a.xl + (size_t)b * N;
-        const float* __restrict__ xurow = IV ? a.xu + (size_t)b * N : nullptr;
-        int cnt = 0;   // marks in the list
-        float xreg[2], ureg[IV ? 2 : 1];
-        int nreg[IDX ? 2 : 1];
-        float wa[2][4], wb[2][4];
-        auto load = [&](int buf, int k0, int total) __attribute__((always_inline)) {
-            int k = k0 + (lane & 3);
-            k = k < total ? k : total - 1;
-            const int nn = (int)mine[k];
-            float l = xlrow[nn];
-            if constexpr (IV) {
-                float u = xurow[nn];
-                repair(l, u);
-                ureg[buf] = u;
-            }
-            xreg[buf] = l;
-            if constexpr (IDX) nreg[buf] = nn;
-            #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int n = __builtin_amdgcn_readlane(nn, i);
-                wa[buf][i] = wcol[(size_t)n * kTileW];
-                wb[buf][i] = wcol[(size_t)n * kTileW + 64];
-            }
-        };
-        auto compute = [&](int buf, int k0, int total) __attribute__((always_inline)) {
-            #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                if (k0 + i < total) {   // wave-uniform
-                    const float xi = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, xreg[buf]), i));
-                    if constexpr (IV) {
-                        const float ui = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ureg[buf]), i));
-                        const float a1 = wa[buf][i] - xi, a2 = ui - wa[buf][i];
-                        const float b1 = wb[buf][i] - xi, b2 = ui - wb[buf][i];
-                        insert_value<K>(lo[0], -fminf(a1, a2), inf);
-                        insert_value<K>(hi[0], fmaxf(a1, a2), inf);
-                        insert_value<K>(lo[1], -fminf(b1, b2), inf);
-                        insert_value<K>(hi[1], fmaxf(b1, b2), inf);
-                    } else {
-                        const float d0 = xi - wa[buf][i], d1 = xi - wb[buf][i];
-                        [[maybe_unused]] int n = 0;
-                        if constexpr (IDX) n = __builtin_amdgcn_readlane(nreg[IDX ? buf : 0], i);
-                        if constexpr (FORM == kRowsSortValues) {
-                            insert_value<K>(hi[0], fabsf(d0), inf);
-                            insert_value<K>(hi[1], fabsf(d1), inf);
-                        } else if constexpr (FORM == kRowsSortPos) {
-                            // the marks of a row go by in ascending input order: the ordered insertion of the scan
-                            // over all inputs (core/cuda/sort_neuron.cu:108-113, 176-185), ties included
-                            if (fabsf(d0) > hi[0][0]) topk_insert<K>(hi[0], idx[0], fabsf(d0), n | (d0 >= 0.f ? 0 : (int)kSign));
-                            if (fabsf(d1) > hi[1][0]) topk_insert<K>(hi[1], idx[1], fabsf(d1), n | (d1 >= 0.f ? 0 : (int)kSign));
-                        } else {
-                            // running maximum; only a larger term replaces it, so the first of equal terms keeps the
-                            // position (core/cuda/inf_dist_cuda.cu:176-190); an undefined term (a weight the row of
-                            // the mask drops) never compares greater
-                            // (the difference itself is kept: its magnitude is the maximum, its sign the flag of
-                            // the position)
-                            const bool g0 = fabsf(d0) > fabsf(hi[0][0]), g1 = fabsf(d1) > fabsf(hi[1][0]);
-                            hi[0][0] = g0 ? d0 : hi[0][0];
-                            hi[1][0] = g1 ? d1 : hi[1][0];
-                            if constexpr (POS) {
-                                idx[0][0] = g0 ? n : idx[0][0];
-                                idx[1][0] = g1 ? n : idx[1][0];
-                            }
-                        }
-                    }
+    };
+    clear();
+    const uint32_t* __restrict__ rowbits = a.bits + ((size_t)t * a.Bp + b) * table_row_words(N);
+    const float* __restrict__ xlrow = a.xl + (size_t)b * N;
+    const float* __restrict__ xurow = IV ? a.xu + (size_t)b * N : xlrow;
+    const float2* __restrict__ ranges = reinterpret_cast<const float2*>(a.wr) + (size_t)t * N;
+    float wa[2][4], wb[2][4];
+    float least[2] = {0.f, 0.f};   // kRowsSortPos: lower bounds of the K-th largest terms
+    auto load = [&](int buf, int i, int n) __attribute__((always_inline)) {
+        wa[buf][i] = wcol[(size_t)n * kTileW];
+        wb[buf][i] = wcol[(size_t)n * kTileW + 64];
+    };
+    // VALUES: a strong mark of kRowsSortPos, whose value alone is wanted
+    auto term = [&](auto values, int buf, int i, int k, int n, const Own& o) __attribute__((always_inline)) {
+        const float xi = lane_value(o.a, k);
+        if constexpr (IV) {
+            const float ui = lane_value(o.b, k);
+            const float a1 = wa[buf][i] - xi, a2 = ui - wa[buf][i];
+            const float b1 = wb[buf][i] - xi, b2 = ui - wb[buf][i];
+            // (the maximum with -1 turns a term that is undefined altogether into a negative one, which the lists ignore)
+            insert_pair<K>(lo[0], fmaxf(fmaxf(-a1, -a2), -1.f), lo[1], fmaxf(fmaxf(-b1, -b2), -1.f));
+            insert_pair<K>(hi[0], fmaxf(fmaxf(a1, a2), -1.f), hi[1], fmaxf(fmaxf(b1, b2), -1.f));
+        } else {
+            const float d0 = xi - wa[buf][i], d1 = xi - wb[buf][i];
+            if constexpr (FORM == kRowsSortValues) {
+                insert_pair<K>(hi[0], fmaxf(fabsf(d0), -1.f), hi[1], fmaxf(fabsf(d1), -1.f));
+            } else if constexpr (decltype(values)::value) {
+                topk_insert_values<K>(hi[0], fabsf(d0));
+                topk_insert_values<K>(hi[1], fabsf(d1));
+            } else if constexpr (FORM == kRowsSortPos) {
+                // the marks of a row go by in ascending input order: the ordered insertion of the scan
+                // over all inputs (core/cuda/sort_neuron.cu:108-113, 176-185), ties included
+                if (fabsf(d0) > hi[0][0] && fabsf(d0) >= least[0]) topk_insert<K>(hi[0], idx[0], fabsf(d0), n | (d0 >= 0.f ? 0 : (int)kSign));
+                if (fabsf(d1) > hi[1][0] && fabsf(d1) >= least[1]) topk_insert<K>(hi[1], idx[1], fabsf(d1), n | (d1 >= 0.f ? 0 : (int)kSign));
+            } else {
+                // running maximum; only a larger term replaces it, so the first of equal terms keeps the
+                // position (core/cuda/inf_dist_cuda.cu:176-190); an undefined term (a weight the row of
+                // the mask drops) never compares greater
+                // (the difference itself is kept: its magnitude is the maximum, its sign the flag of
+                // the position)
+                const bool g0 = fabsf(d0) > fabsf(hi[0][0]), g1 = fabsf(d1) > fabsf(hi[1][0]);
+                hi[0][0] = g0 ? d0 : hi[0][0];
+                hi[1][0] = g1 ? d1 : hi[1][0];
+                if constexpr (POS) {
+                    idx[0][0] = g0 ? n : idx[0][0];
+                    idx[1][0] = g1 ? n : idx[1][0];
                 }
             }
-        };
-        // walks the list, the loads of a group in flight while the group before it is used
-        auto walk = [&](int total) __attribute__((always_inline)) {
-            if (total == 0) return;
-            load(0, 0, total);
-            for (int k0 = 0; k0 < total; k0 += 8) {
-                load(1, k0 + 4, total);
-                compute(0, k0, total);
-                load(0, k0 + 8, total);
-                compute(1, k0 + 4, total);
-            }
-        };
-        uint32_t next = lane < NCH ? rowbits[lane] : 0u;
-        for (int c0 = 0; c0 < NCH; c0 += kRtBatch) {
-            uint32_t word = next;
-            if (c0 + kRtBatch < NCH) next = c0 + kRtBatch + lane < NCH ? rowbits[c0 + kRtBatch + lane] : 0u;
-            // every lane appends the marks of its word behind those of the lanes before it
-            const int mine_n = __builtin_popcount(word);
-            int incl = mine_n;
-            #pragma unroll
-            for (int o = 1; o < kRtBatch; o <<= 1) {
-                const int v = __shfl_up(incl, o);
-                if (lane >= o) incl += v;
-            }
-            int off = cnt + incl - mine_n;
-            cnt += __builtin_amdgcn_readlane(incl, kRtBatch - 1);
-            while (word) {
-                const int i = __builtin_ctz(word);
-                word &= word - 1;
-                mine[off++] = (uint16_t)(((c0 + lane) << 5) | i);   // the input's number (rows of at most 65536 inputs)
-            }
-            // a row's marks are walked in one go unless the list could overflow with the next chunks
-            if (cnt > kRtListCap - kRtBatch * kChunk || c0 + kRtBatch >= NCH) {
-                __builtin_amdgcn_wave_barrier();
-                walk(cnt);
-                cnt = 0;
-                __builtin_amdgcn_wave_barrier();   // the reads of the list come before the next marks
-            }
         }
-        float bound = 0.f;
-        if constexpr (MASKED) bound = a.low[(size_t)t * a.Bp + b];   // wave-uniform
-        #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int col = t * kTileW + lane + 64 * j;
-            if (col < M) {
-                const size_t o = (size_t)b * M + col;
-                if constexpr (LISTS) {
-                    a.outU[o] = geo_sum<K>(hi[j], a.q);
-                    if constexpr (IV) a.outL[o] = geo_sum<K>(lo[j], a.q);
-                    if constexpr (FORM == kRowsSortPos) {
-                        #pragma unroll
-                        for (int k = 0; k < K; k++) a.pos[(size_t)(K - 1 - k) * plane + o] = idx[j][k];   // plane 0 = largest
-                    }
-                } else {
-                    a.outU[o] = fabsf(hi[j][0]);
-                    if constexpr (POS) a.pos[o] = idx[j][0] | (hi[j][0] >= 0.f ? 0 : (int)kSign);
-                    if constexpr (MASKED) {
-                        // The bound rests on K inputs that the batch row keeps; a weight row that keeps none of them
-                        // may have its maximum at an unmarked input: such an output is recomputed from every input.
-                        if (!(fabsf(hi[j][0]) >= bound)) a.fix[atomicAdd(a.count + 4, 1ull)] = (uint32_t)o;
-                    }
+    };
+    auto value = [&](int buf, int i, int k, int n, const Own& o) __attribute__((always_inline)) { term(std::bool_constant<FORM == kRowsSortPos>{}, buf, i, k, n, o); };
+    auto use = [&](int buf, int i, int k, int n, const Own& o) __attribute__((always_inline)) { term(std::false_type{}, buf, i, k, n, o); };
+    const float LU = a.low[(size_t)t * a.Bp + b];   // wave-uniform
+    // smallest results of the lane's rows over the wavefront (weight rows past the last one do not count)
+    float thU = 0.f, thL = 0.f;
+    auto smallest = [&](float v0, float v1) __attribute__((always_inline)) {
+        return wave_min_nonneg(fminf(in0 ? v0 : __builtin_inff(), in1 ? v1 : __builtin_inff()));
+    };
+    // In kRowsSortPos the strong marks give each row a lower bound of its K-th largest term.  A term below it is never among
+    // the K largest, and whether one at or above it enters depends only on entries at least that large, so the walk in input
+    // order may leave the others out.
+    for_marks(list, NCH, lane, [&](int c) __attribute__((always_inline)) { return table_word(rowbits, c); },
+              [&](int total, bool first) __attribute__((always_inline)) {
+        walk_marks<ORDERED, IV>(list, total, first, lane,
+            [&](int n) __attribute__((always_inline)) {
+                Own o{xlrow[n], 0.f};
+                if constexpr (IV) { o.b = xurow[n]; repair(o.a, o.b); }
+                return o;
+            },
+            [&](int n, const Own& o) __attribute__((always_inline)) {
+                const float2 r = ranges[n];
+                return fmaxf(r.y - o.a, (IV ? o.b : o.a) - r.x);
+            },
+            load, value, use,
+            [&](bool strong) __attribute__((always_inline)) {
+                if (FORM == kRowsSortPos && strong) { least[0] = hi[0][0]; least[1] = hi[1][0]; }
+                if constexpr (FORM == kRowsSortValues || IV) thU = smallest(__int_as_float(hi[0][0]), __int_as_float(hi[1][0]));
+                else thU = smallest(fmaxf(fabsf(hi[0][0]), least[0]), fmaxf(fabsf(hi[1][0]), least[1]));
+                if constexpr (IV) thL = smallest(__int_as_float(lo[0][0]), __int_as_float(lo[1][0]));
+            },
+            [&](int n, const Own& o) __attribute__((always_inline)) {
+                const float2 r = ranges[n];
+                bool keep = !(fmaxf(r.y - o.a, (IV ? o.b : o.a) - r.x) < thU);
+                if constexpr (IV) keep = keep || !(fmaxf(o.a - r.x, r.y - o.b) < thL);
+                return keep;
+            },
+            clear);
+    });
+    #pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const int col = t * kTileW + lane + 64 * j;
+        if (col < M) {
+            const size_t o = (size_t)b * M + col;
+            if constexpr (LISTS) {
+                if constexpr (FORM == kRowsSortPos) a.outU[o] = geo_sum<K>(hi[j], a.q);
+                else a.outU[o] = geo_sum_bits<K>(hi[j], a.q);
+                if constexpr (IV) a.outL[o] = geo_sum_bits<K>(lo[j], a.q);
+                if constexpr (FORM == kRowsSortPos) {
+                    #pragma unroll
+                    for (int k = 0; k < K; k++) a.pos[(size_t)(K - 1 - k) * plane + o] = idx[j][k];   // plane 0 = largest
+                }
+            } else {
+                a.outU[o] = fabsf(hi[j][0]);
+                if constexpr (POS) a.pos[o] = idx[j][0] | (hi[j][0] >= 0.f ? 0 : (int)kSign);
+                if constexpr (MASKED) {
+                    // The bound rests on K inputs that the batch row keeps; a weight row that keeps none of them
+                    // may have its maximum at an unmarked input: such an output is recomputed from every input.
+                    if (!(fabsf(hi[j][0]) >= LU)) a.fix[atomicAdd(&a.count->fixes, 1ull)] = (uint32_t)o;
                 }
             }
         }
@@ -586,7 +325,7 @@ __global__ void __launch_bounds__(64 * kRtWaves) rt_main_kernel(RtArgs a) {
 struct FixArgs {
     const float* xl; const float* w;
     const uint32_t* xkeep; const uint32_t* wkeep;
-    const unsigned long long* count;
+    const RowCount* count;
     const uint32_t* fix;
     int M, N;
     float* outU; int* pos;
@@ -596,8 +335,8 @@ struct FixArgs {
 // wavefront per output over every input that both rows keep, lowest input first among equal terms.
 template <bool POS>
 __global__ void __launch_bounds__(256) rc_fix_kernel(FixArgs a) {
-    if (a.count[2] == 0ull) return;
-    const unsigned long long total = a.count[4];
+    if (a.count->run == 0ull) return;
+    const unsigned long long total = a.count->fixes;
     const int lane = threadIdx.x & 63;
     const int N = a.N, NCH = N / kChunk;
     for (unsigned long long e = (unsigned long long)blockIdx.x * 4 + (threadIdx.x >> 6); e < total; e += (unsigned long long)gridDim.x * 4) {
@@ -630,51 +369,43 @@ __global__ void __launch_bounds__(256) rc_fix_kernel(FixArgs a) {
 
 template <int FORM, int K, bool POS, bool MASKED>
 int launch_rt(const RtArgs& a, hipStream_t st) {
-    const int T = tiles_w(a.M), BG = (a.B + kRtWaves * kRtRows - 1) / (kRtWaves * kRtRows);
+    const int T = tiles_w(a.M), BG = (a.B + kRtWaves - 1) / kRtWaves;
     hipLaunchKernelGGL((rt_main_kernel<FORM, K, POS, MASKED>), dim3((unsigned)(T * BG)), dim3(64 * kRtWaves), 0, st, a);
     return check_launch("rt_main_kernel");
+}
+
+// ranges, transposed weights, tables
+template <bool PAIR, bool MASK>
+int run_tables(const float* xl, const float* xu, const float* w, const uint32_t* xkeep, const uint32_t* wkeep, int B, int M,
+               int N, int K, const Carve& c, unsigned long long limit, const float* col_stat, const unsigned long long* col_count,
+               float ratio, hipStream_t st) {
+    const int T = tiles_w(M), S = (B + 127) / 128;
+    int rc;
+    hipLaunchKernelGGL((rc_range_kernel<MASK>), dim3((N + 63) / 64, T), dim3(256), 0, st, w, wkeep, M, N, S, c.wr, c.wt, c.count, col_stat, ratio);
+    if ((rc = check_launch("rc_range_kernel"))) return rc;
+    const TableArgs t{PAIR ? xu : xl, xl, xkeep, c.wr, B, bpad_of(B), N, T, K, c.low, c.bits};
+    hipLaunchKernelGGL((rc_tables_kernel<PAIR, MASK>), dim3((B + kTableWaves - 1) / kTableWaves, (T + 3) / 4), dim3(64 * kTableWaves), 0, st,
+                       t, c.count, col_count, col_stat, S, limit, ratio);
+    return check_launch("rc_tables_kernel");
 }
 
 template <int FORM, int K>
 int run(const float* xl, const float* xu, const float* w, int B, int M, int N, float q, float* outL, float* outU, int* pos,
         const Carve& c, unsigned long long limit, const float* col_stat, const unsigned long long* col_count, hipStream_t st) {
     constexpr bool IV = FORM == kRowsSortInterval;
-    const int T = tiles_w(M), Bp = bpad_of(B), NCH = N / kChunk, slices = slices_of(NCH), S = (B + 127) / 128;
-    int rc;
-    hipLaunchKernelGGL((rc_range_kernel<false>), dim3((N + 63) / 64, T), dim3(256), 0, st, w, nullptr, M, N, S, c.wr, c.wt, col_stat, kProbeRatio);
-    if ((rc = check_launch("rc_range_kernel"))) return rc;
-    const dim3 tgrid(Bp / 64, slices, (T + 3) / 4);
-    hipLaunchKernelGGL((rc_low_kernel<K, IV, false>), tgrid, dim3(256), 0, st, xl, xu, nullptr, c.wr, B, N, T, Bp, S, c.lists, col_stat, kProbeRatio);
-    if ((rc = check_launch("rc_low_kernel"))) return rc;
-    constexpr int nw = IV ? 2 : 1;
-    hipLaunchKernelGGL((rc_merge_kernel<K>), dim3((Bp + 255) / 256, T * nw), dim3(256), 0, st, c.lists, slices, Bp, nw, S, c.low, col_stat, kProbeRatio);
-    if ((rc = check_launch("rc_merge_kernel"))) return rc;
-    hipLaunchKernelGGL((rc_bits_kernel<IV, false>), tgrid, dim3(256), 0, st, xl, xu, nullptr, c.wr, c.low, B, N, T, Bp, S, c.bits, c.partial, col_stat, kProbeRatio);
-    if ((rc = check_launch("rc_bits_kernel"))) return rc;
-    hipLaunchKernelGGL(rc_sum_kernel, dim3(1), dim3(1024), 0, st, c.partial, (size_t)tgrid.x * tgrid.y * tgrid.z * 4, c.count, col_count, col_stat, S, limit, kProbeRatio);
-    if ((rc = check_launch("rc_sum_kernel"))) return rc;
-    RtArgs a{xl, xu, c.wt, c.bits, c.low, c.count, c.fix, B, Bp, M, N, q, outL, outU, pos};
+    const int rc = run_tables<IV, false>(xl, xu, w, nullptr, nullptr, B, M, N, K, c, limit, col_stat, col_count, kProbeRatio, st);
+    if (rc) return rc;
+    RtArgs a{xl, xu, c.wt, c.wr, c.bits, c.low, c.count, c.fix, B, bpad_of(B), M, N, q, outL, outU, pos};
     return launch_rt<FORM, K, false, false>(a, st);
 }
 
-template <int K, bool MASKED>
-int run_max(const float* x, const float* w, const uint32_t* xkeep, const uint32_t* wkeep, int B, int M, int N, float* y,
+template <bool MASKED>
+int run_max(const float* x, const float* w, const uint32_t* xkeep, const uint32_t* wkeep, int B, int M, int N, int K, float* y,
             int* pos, const Carve& c, unsigned long long limit, const float* col_stat, const unsigned long long* col_count,
             float ratio, hipStream_t st) {
-    const int T = tiles_w(M), Bp = bpad_of(B), NCH = N / kChunk, slices = slices_of(NCH), S = (B + 127) / 128;
-    int rc;
-    hipLaunchKernelGGL((rc_range_kernel<MASKED>), dim3((N + 63) / 64, T), dim3(256), 0, st, w, wkeep, M, N, S, c.wr, c.wt, col_stat, ratio);
-    if ((rc = check_launch("rc_range_kernel"))) return rc;
-    const dim3 tgrid(Bp / 64, slices, (T + 3) / 4);
-    hipLaunchKernelGGL((rc_low_kernel<K, false, MASKED>), tgrid, dim3(256), 0, st, x, nullptr, xkeep, c.wr, B, N, T, Bp, S, c.lists, col_stat, ratio);
-    if ((rc = check_launch("rc_low_kernel"))) return rc;
-    hipLaunchKernelGGL((rc_merge_kernel<K>), dim3((Bp + 255) / 256, T), dim3(256), 0, st, c.lists, slices, Bp, 1, S, c.low, col_stat, ratio);
-    if ((rc = check_launch("rc_merge_kernel"))) return rc;
-    hipLaunchKernelGGL((rc_bits_kernel<false, MASKED>), tgrid, dim3(256), 0, st, x, nullptr, xkeep, c.wr, c.low, B, N, T, Bp, S, c.bits, c.partial, col_stat, ratio);
-    if ((rc = check_launch("rc_bits_kernel"))) return rc;
-    hipLaunchKernelGGL(rc_sum_kernel, dim3(1), dim3(1024), 0, st, c.partial, (size_t)tgrid.x * tgrid.y * tgrid.z * 4, c.count, col_count, col_stat, S, limit, ratio);
-    if ((rc = check_launch("rc_sum_kernel"))) return rc;
-    RtArgs a{x, nullptr, c.wt, c.bits, c.low, c.count, c.fix, B, Bp, M, N, 0.f, nullptr, y, pos};
+    int rc = run_tables<false, MASKED>(x, nullptr, w, xkeep, wkeep, B, M, N, K, c, limit, col_stat, col_count, ratio, st);
+    if (rc) return rc;
+    RtArgs a{x, nullptr, c.wt, c.wr, c.bits, c.low, c.count, c.fix, B, bpad_of(B), M, N, 0.f, nullptr, y, pos};
     if (pos) rc = launch_rt<kRowsMax, 1, true, MASKED>(a, st);
     else rc = launch_rt<kRowsMax, 1, false, MASKED>(a, st);
     if (rc || !MASKED) return rc;
@@ -686,9 +417,9 @@ int run_max(const float* x, const float* w, const uint32_t* xkeep, const uint32_
 
 }  // namespace
 
-size_t row_cands_workspace(int form, int B, int CO, int CI, int K) {
-    size_t sz[8];
-    return carve_sizes(form, B, CO, CI, K, sz);
+size_t row_cands_workspace(int form, int B, int CO, int CI) {
+    size_t sz[6];
+    return carve_sizes(form, B, CO, CI, sz);
 }
 
 bool row_cands_supported(int form, int K) {
@@ -719,10 +450,10 @@ int row_cands_forward(int form, const float* xl, const float* xu, const float* w
         set_error("row_cands_forward: rows of more than 65536 inputs");
         return SD_ERR_ARG;
     }
-    const Carve c = carve(ws, form, B, CO, CI, K);
+    const Carve c = carve(ws, form, B, CO, CI);
     const float d = density < 0.f ? 0.f : density > 1.f ? 1.f : density;
     const unsigned long long limit = (unsigned long long)((double)tiles_w(CO) * B * CI * d);
-    *every = c.count + 1;
+    *every = &c.count->every;
     switch (form) {
         case kRowsSortValues:
             switch (K) {
@@ -746,13 +477,8 @@ int row_cands_forward(int form, const float* xl, const float* xu, const float* w
             }
             break;
         case kRowsMax:
-            if (!xkeep) return run_max<1, false>(xl, w, nullptr, nullptr, B, CO, CI, outU, pos, c, limit, col_stat, col_count, ratio_max, st);
-            switch (K) {
-#define X(k) case k: return run_max<k, true>(xl, w, xkeep, wkeep, B, CO, CI, outU, pos, c, limit, col_stat, col_count, ratio_max, st);
-                X(8) X(12) X(16) X(20) X(24)
-#undef X
-            }
-            break;
+            return xkeep ? run_max<true>(xl, w, xkeep, wkeep, B, CO, CI, K, outU, pos, c, limit, col_stat, col_count, ratio_max, st)
+                         : run_max<false>(xl, w, nullptr, nullptr, B, CO, CI, K, outU, pos, c, limit, col_stat, col_count, ratio_max, st);
     }
     set_error("row_cands_forward: K=%d not supported for form %d", K, form);
     return SD_ERR_ARG;

@@ -174,8 +174,8 @@ constexpr long long kSortRowsMinTerms = 1ll << 28;
 // bytes of both tables' workspace for one call: per weight row first (with the probe and the counter the per-batch-row
 // tables read), per batch row behind it
 static size_t sort_tables_bytes(int form, int B, int CO, int CI, int K) {
-    const size_t cols = (sort_cols_workspace(B, CO, CI, K) + 255) / 256 * 256;
-    return cols + (row_cands_supported(form, K) ? (row_cands_workspace(form, B, CO, CI, K) + 255) / 256 * 256 : 0);
+    const size_t cols = (sort_cols_workspace(B, CO, CI) + 255) / 256 * 256;
+    return cols + (row_cands_supported(form, K) ? (row_cands_workspace(form, B, CO, CI) + 255) / 256 * 256 : 0);
 }
 
 // `ws`: sort_tables_bytes() bytes.  The gate it leaves in `a` points into `ws`: the kernels queued behind it must
@@ -196,7 +196,7 @@ static int queue_sort_cols(FwdArgs& a, int form, const float* xl, const float* x
         return rc;
     }
     const unsigned long long* col_count = a.gate;
-    char* rows_ws = static_cast<char*>(ws) + (sort_cols_workspace(B, CO, CI, K) + 255) / 256 * 256;
+    char* rows_ws = static_cast<char*>(ws) + (sort_cols_workspace(B, CO, CI) + 255) / 256 * 256;
     const unsigned long long* every = nullptr;
     rc = row_cands_forward(form, xl, xu, w, nullptr, nullptr, B, CO, CI, q, K, outL, outU, pos, rows_ws,
                            density > 0.f ? density : kSortRowsCap, density > 0.f, sort_cols_probe_sums(col_count), col_count, &every, st);

@@ -17,7 +17,7 @@ namespace sd {
 constexpr int kSortColsChunk = 32;
 
 // bytes of workspace sort_cols_forward needs
-size_t sort_cols_workspace(int B, int CO, int CI, int K);
+size_t sort_cols_workspace(int B, int CO, int CI);
 
 // Builds the table, counts its marks on the device and queues the table kernel so that it runs only when at most
 // `density` of all (tile, weight row, input) triples are marked; the caller queues the kernels that evaluate every
@@ -40,7 +40,6 @@ inline const float* sort_cols_probe_sums(const unsigned long long* gate) { retur
 // neither).  K = max_cols_depth(probability that a row keeps an input): how many inputs the bound of a weight row
 // rests on (1 without a mask; 0 = the mask keeps too little for a table).  Same contract as sort_cols_forward.
 int max_cols_depth(float keep_x);
-size_t max_cols_workspace(int B, int CO, int CI, int K);
 int max_cols_forward(const float* x, const float* w, const uint32_t* xkeep, const uint32_t* wkeep, int B, int CO, int CI,
                      int K, float* y, int* pos, void* ws, float density, const unsigned long long** gate,
                      unsigned long long* gate_limit, hipStream_t st);
