@@ -80,6 +80,10 @@ __global__ void __launch_bounds__(256) bound_bwd_kernel(BwdArgs a) {
 // neither a zero-fill pass nor global atomics.  grad_weight is still scattered with atomics.
 constexpr int kMaxRowLds = 12288;   // floats of LDS one row histogram may take
 
+// grid.y: parts of the inputs.  The sort neuron sends K values per output into a row, and with fewer rows than compute units
+// those adds are the time (128 rows of 5120 outputs, K = 10: 67 us with a workgroup to a row, 37 with four): every
+// part's workgroup reads the positions of its row and adds what falls into its own inputs.
+constexpr int kSlotsAtOnce = 5;     // positions of an output in flight
 template <bool SORT, bool HAS_W>
 __global__ void __launch_bounds__(1024) scatter_bwd_rows_kernel(BwdArgs a) {
     extern __shared__ float hist[];
@@ -88,7 +92,8 @@ __global__ void __launch_bounds__(1024) scatter_bwd_rows_kernel(BwdArgs a) {
     const int bg = row / a.HW;
     const int g = bg % a.G, b = bg / a.G;
     const int s = b / kSubBatch;
-    for (int n = threadIdx.x; n < a.CIg; n += blockDim.x) hist[n] = 0.f;
+    const int n0 = (int)((long long)a.CIg * blockIdx.y / gridDim.y), len = (int)((long long)a.CIg * (blockIdx.y + 1) / gridDim.y) - n0;
+    for (int n = threadIdx.x; n < len; n += blockDim.x) hist[n] = 0.f;
     __syncthreads();
     const size_t obase = ((size_t)(b * a.G + g) * a.COg) * a.HW + hw;
     const int K = SORT ? a.K : 1;
@@ -101,21 +106,27 @@ __global__ void __launch_bounds__(1024) scatter_bwd_rows_kernel(BwdArgs a) {
             int mm = a.co_idx ? a.co_idx[(s * a.G + g) * a.COg + m] : m;
             wrow = (size_t)(g * a.W_COg + mm) * a.W_CIg;
         }
-        for (int k = 0; k < K; k++) {
-            int pr = a.p0[(size_t)k * a.total + o];
-            int n = pr & 0x7fffffff;
-            float v = pr >= 0 ? grad : -grad;
-            if (SORT) { v = v * coef * a.q; coef *= 1.f - a.q; }
-            atomicAdd(&hist[n], v);
-            if (HAS_W) {
-                int nn = a.ci_idx ? a.ci_idx[(s * a.G + g) * a.CIg + n] : n;
-                unsafeAtomicAdd(a.gw + wrow + nn, -v);
+        for (int k0 = 0; k0 < K; k0 += kSlotsAtOnce) {
+            int pr[kSlotsAtOnce];
+            #pragma unroll
+            for (int i = 0; i < (SORT ? kSlotsAtOnce : 1); i++) pr[i] = a.p0[(size_t)(k0 + i < K ? k0 + i : K - 1) * a.total + o];
+            #pragma unroll
+            for (int i = 0; i < (SORT ? kSlotsAtOnce : 1); i++) {
+                if (k0 + i >= K) break;
+                const int n = pr[i] & 0x7fffffff;
+                float v = pr[i] >= 0 ? grad : -grad;
+                if (SORT) { v = v * coef * a.q; coef *= 1.f - a.q; }
+                if ((unsigned)(n - n0) < (unsigned)len) atomicAdd(&hist[n - n0], v);
+                if (HAS_W) {
+                    int nn = a.ci_idx ? a.ci_idx[(s * a.G + g) * a.CIg + n] : n;
+                    unsafeAtomicAdd(a.gw + wrow + nn, -v);
+                }
             }
         }
     }
     __syncthreads();
-    const size_t xbase = ((size_t)(b * a.G + g) * a.CIg) * a.HW + hw;
-    for (int n = threadIdx.x; n < a.CIg; n += blockDim.x) a.gx0[xbase + (size_t)n * a.HW] = hist[n];
+    const size_t xbase = ((size_t)(b * a.G + g) * a.CIg + n0) * a.HW + hw;
+    for (int n = threadIdx.x; n < len; n += blockDim.x) a.gx0[xbase + (size_t)n * a.HW] = hist[n];
 }
 
 template <bool HAS_W>
@@ -314,9 +325,13 @@ static int run_scatter(BwdArgs& a, hipStream_t st) {
     x.gw = gw_atomic;
     if (a.CIg <= kMaxRowLds) {
         dim3 rows((unsigned)(a.B * a.G * a.HW));
-        size_t lds = (size_t)a.CIg * sizeof(float);
-        // few rows: more work-items per row, so that enough position / index loads are in flight
+        // few rows: more work-items per row, so that enough position / index loads are in flight, and, where a row is sent many
+        // values (and grad_weight is not scattered as well), parts of the inputs until every compute unit has two workgroups
         const dim3 block(rows.x < 4u * (unsigned)num_cus() ? 1024 : 256);
+        if (SORT && !x.gw) {
+            while (rows.y < 8u && rows.x * rows.y < 2u * (unsigned)num_cus() && a.CIg / (int)(2 * rows.y) >= 256) rows.y *= 2;
+        }
+        const size_t lds = (size_t)((a.CIg + (int)rows.y - 1) / (int)rows.y) * sizeof(float);
         if (x.gw) hipLaunchKernelGGL((scatter_bwd_rows_kernel<SORT, true>), rows, block, lds, st, x);
         else hipLaunchKernelGGL((scatter_bwd_rows_kernel<SORT, false>), rows, block, lds, st, x);
         return check_launch("scatter_bwd_rows_kernel");
