@@ -15,17 +15,18 @@ using namespace sd;
 // forward runs instead of the kernel that evaluates every term (sd_set_bound_candidate_density); negative: built-in
 static std::atomic<float> g_bound_density{-1.f};
 // measured at B = 512, M = N = 5120: the table kernel takes 0.09 + 2.6 x share ms (about 60 SIMD cycles per marked
-// (tile, weight row, input)) after 0.10 ms for the tables, against 1.03-1.09 ms for every term; the kernel of the
-// tables per batch row 0.14 + 3.3 x share ms.  The tables are paid for by the time the choice is made, so the limits
-// sit a little below where the table kernel alone meets the every-term kernel.
-constexpr float kBoundColsCap = 0.30f, kBoundRowsCap = 0.26f;
+// (tile, weight row, input)) after 0.10 ms for the tables, against 1.00 ms for every term.  The tables are paid for by the time
+// the choice is made, so the limit sits a little below where the two would meet.  Per batch row (us, every term / tables):
+// 993 / 360 (6.5 % marked), 998 / 376 (13 %), 982 / 451 (25 %), with positions 1235 / 399, 1238 / 490, 1271 / 683; 128 x 5120 x
+// 5120 281 / 227 and 351 / 300 (25 %).
+constexpr float kBoundColsCap = 0.30f, kBoundRowsCap = 0.40f;
 // With the built-in limits, layers below this many terms go without tables: building them and starting the table
 // kernel takes about 0.19 ms, which is what the every-term kernel needs for 2.4 G terms (512 x 10 x 5120: 0.06 ms
 // for every term against 0.10 ms from tables).
 constexpr long long kBoundColsMinTerms = 1ll << 31;
 // The forward that also returns positions: its table kernel spends about twice as long per mark (a compare and two
 // selects per output instead of a three-operand minimum or maximum) and the every-term kernel 1.5 times as long per
-// term, so the limit is lower.
+// term, so the limit is lower per weight row.
 constexpr float kBoundPosColsCap = 0.15f;
 constexpr int kHintSiteBound = 1, kHintSiteBoundSparse = 8, kHintSiteBoundPos = 9;
 constexpr float kBoundSparseCap = 0.03f;   // marked share up to which the kernel without LDS staging runs
@@ -61,16 +62,14 @@ static int max_cols_wanted(const FwdArgs& a, int K, int site, int B, int CO, int
 }
 
 // Largest share of marked (tile of 128 weight rows, batch row, input) triples at which the l-inf kernel of the tables
-// per batch row runs, and the smallest layer (in terms) given such tables under the built-in limit.  Measured on inputs
-// in [0, 1] against weights ~ N(0, 1/N) (6.5 to 8.4 % marked): 512 x 5120 x 5120 0.34 ms (0.36 with positions; 0.15 ms
-// of it tables and the transposed copy of the weights) against 0.49 (0.61) for every term, 256 x 12288 x 10240 0.86
-// (0.89) against 1.28 (1.30), 512 x 3072 x 5120 0.26 (0.27) against 0.27 (0.43), 256 x 4096 x 2048 0.13 (0.13)
-// against 0.09 (0.12): the main kernel's time grows with the marks, so the limit sits where the two would meet at the
-// large sizes.  With the 512 x 3072 x 5120 layer served from tables the benchmark step gained 0.1 ms on one stream and
-// lost 0.05 ms on three (presumably the table passes and the transposed copy, which stream the operands through
-// memory, meet the traffic of the optimizer and the backward on the other streams), so the size limit sits above
-// that layer.
-constexpr float kMaxRowsCap = 0.10f;
+// per batch row runs, and the smallest layer (in terms) given such tables under the built-in limit.  Every term / tables, us,
+// 512 x 5120 x 5120, inputs in [0, 1] against weights of growing scale: without positions 384 / 263 (6.5 % marked), 383 / 303
+// (13 %), 387 / 373 (25 %); with them 516 / 281, 504 / 326, 507 / 422; factored mask with positions 554 / 326 (4 %), 552 / 352
+// (7 %), 549 / 409 (14 %).  Smaller layers lose: 128 x 5120 x 5120 110 / 139, with positions 168 / 146.  With the
+// 512 x 3072 x 5120 layer served from tables the benchmark step gained 0.1 ms on one stream and lost 0.05 ms on three
+// (presumably the table passes and the transposed copy, which stream the operands through memory, meet the traffic of the
+// optimizer and the backward on the other streams), so the size limit sits above that layer.
+constexpr float kMaxRowsCap = 0.20f;
 constexpr long long kMaxRowsMinTerms = 1ll << 33;
 
 // bytes of both tables' workspace for one call: per weight row first, per batch row behind it
@@ -495,7 +494,7 @@ extern "C" int sd_bound_inf_dist_forward(const float* inputL, const float* input
         if (a.nsplit > 1 && (rc = fill_zero(a.packed0, n * 4, st))) return rc;
         if (cols) {
             if ((rc = bound_cols_forward(inputL, inputU, weight, B, CO, CI, outputL, outputU, a.packed0, a.packed1, posL, posU,
-                                         ws + pairs, cap, cap, &a.gate, &a.gate_limit, st)))
+                                         ws + pairs, cap, bound_density >= 0.f ? bound_density : kBoundRowsCap, &a.gate, &a.gate_limit, st)))
                 return rc;
             a.gate_above = 1;
             a.resolved = a.gate + 2;   // the tables per batch row store final values and positions themselves

@@ -71,9 +71,9 @@ __device__ __forceinline__ void repair(float& l, float& u) {
 // of a weight column do.  stat[0] = widths of the input columns over all batch tiles, stat[1] = widths of the same
 // columns over 16 weight rows.
 // `ratio` is kProbeRatio for the sort-neuron forms.  The l-inf form asks for more (kProbeRatioMax): its kernel only pays
-// below about 10 % of marks, and on inputs spread evenly over their range the marked share is about 1 / (that ratio), so
+// below about 25 % of marks, and on inputs spread evenly over their range the marked share is about 1 / (that ratio), so
 // its tables are not even built unless the probe promises that few.
-constexpr float kProbeRatio = 2.5f, kProbeRatioMax = 10.f;
+constexpr float kProbeRatio = 2.5f, kProbeRatioMax = 5.f;
 __device__ __forceinline__ bool rows_decide(const float* stat, int S, float ratio) {
     return stat[0] > ratio * (float)S * stat[1];
 }

@@ -134,10 +134,18 @@ static int run_two_level(FwdArgs& a, bool small, int* keys, hipStream_t st) {
 
 // Dense single-group layers: a kernel that works from per-weight-row candidate tables is queued in front of the
 // kernels that evaluate every term, and a count taken on the device decides which of the two runs (at most
-// kSortColsCap of the terms marked: the table kernel).  Negative g_sort_density: built-in limit, and only layers
+// sort_cols_cap of the terms marked: the table kernel).  Negative g_sort_density: built-in limit, and only layers
 // large enough for the tables to pay; 0 never; up to 1: that share, at any size.
 static std::atomic<float> g_sort_density{-1.f};
-constexpr float kSortColsCap = 0.10f;
+// Every term / tables, us, by the marked share (activations of growing spread against unit weights, K = 10).  The time
+// follows the marks that are left after a wavefront has cut its list, so the two meet late; positions, which walk their strong
+// marks twice, meet first where a batch tile is not full.
+//   values       512 x 5120 x 5120 1809 / 394 (12 %), 1813 / 766 (43 %), 1797 / 1212 (91 %); 256 x 2048 x 512 101 / 74 (21 %),
+//                100 / 114 (61 %); 512 x 768 x 640 109 / 70 (36 %)
+//   interval     512 x 5120 x 5120 3901 / 702 (14 %), 4120 / 1448 (47 %); 256 x 2048 x 512 241 / 106 (23 %), 252 / 169 (66 %)
+//   positions    512 x 5120 x 5120 2447 / 818 (12 %), 2471 / 1592 (43 %); 128 x 5120 x 5120 583 / 305 (12 %), 600 / 561 (43 %);
+//                256 x 2048 x 512 139 / 125 (21 %), 143 / 204 (61 %); 96 x 5120 x 300 216 / 150 (11 %), 220 / 256 (38 %)
+static float sort_cols_cap(int form) { return form == kRowsSortPos ? 0.22f : 0.40f; }
 constexpr long long kSortColsMinTerms = 1ll << 24;
 
 // `site`: which entry point asks (with the built-in limit, a layer whose tables have not paid lately is not given
@@ -161,11 +169,11 @@ static void sort_cols_report(const FwdArgs& a, int site, int B, int CO, int CI, 
 }
 
 // Largest share of marked (tile of 128 weight rows, batch row, input) triples at which the kernel of the tables per
-// batch row runs.  Measured per 512 x 5120 x 5120 layer at K = 10 on inputs in [0, 1] against weights ~ N(0, 1/N)
-// (7.2 % marked): values 0.58 ms against 1.9 ms for every term, interval bounds 0.95 against 3.3, values with positions
-// 0.83 against 2.4; 0.16 ms of that are tables and the transposed copy of the weights, the rest grows with the marks
-// (the two would meet at 25 to 30 %).
-constexpr float kSortRowsCap = 0.22f;
+// batch row runs.  Every term / tables, us, on inputs in [0, 1] against weights of growing scale, K = 10:
+//   values       512 x 5120 x 5120 1714 / 416 (7 %), 1763 / 905 (27 %); 128 x 3072 x 1024 132 / 90 (9 %), 131 / 151 (35 %)
+//   interval     512 x 5120 x 5120 3225 / 675 (9 %), 3811 / 1560 (29 %); 128 x 3072 x 1024 312 / 116 (11 %), 342 / 216 (37 %)
+//   positions    512 x 5120 x 5120 2332 / 778 (7 %), 2443 / 1748 (27 %); 128 x 3072 x 1024 182 / 132 (9 %), 179 / 176 (18 %)
+static float sort_rows_cap(int form) { return form == kRowsSortInterval ? 0.45f : form == kRowsSortValues ? 0.27f : 0.22f; }
 // Smallest layers (in terms) given tables per batch row under the built-in limit (128 x 3072 x 1024, 0.4 G terms:
 // values 0.12 ms from tables against 0.14 ms for every term, with positions 0.16 against 0.19, interval bounds 0.17
 // against 0.32)
@@ -184,7 +192,7 @@ static size_t sort_tables_bytes(int form, int B, int CO, int CI, int K) {
 static int queue_sort_cols(FwdArgs& a, int form, const float* xl, const float* xu, const float* w, int B, int CO, int CI,
                            float q, int K, float* outL, float* outU, int* pos, void* ws, hipStream_t st) {
     const float density = g_sort_density.load(std::memory_order_relaxed);
-    const float cap = density > 0.f ? density : kSortColsCap;
+    const float cap = density > 0.f ? density : sort_cols_cap(form);
     int rc = sort_cols_forward(xl, xu, w, B, CO, CI, q, K, outL, outU, pos, ws, cap, &a.gate, &a.gate_limit, st);
     a.gate_above = 1;
     const long long terms = (long long)B * CO * CI;
@@ -199,7 +207,7 @@ static int queue_sort_cols(FwdArgs& a, int form, const float* xl, const float* x
     char* rows_ws = static_cast<char*>(ws) + (sort_cols_workspace(B, CO, CI) + 255) / 256 * 256;
     const unsigned long long* every = nullptr;
     rc = row_cands_forward(form, xl, xu, w, nullptr, nullptr, B, CO, CI, q, K, outL, outU, pos, rows_ws,
-                           density > 0.f ? density : kSortRowsCap, density > 0.f, sort_cols_probe_sums(col_count), col_count, &every, st);
+                           density > 0.f ? density : sort_rows_cap(form), density > 0.f, sort_cols_probe_sums(col_count), col_count, &every, st);
     if (rc) return rc;
     a.gate = every;
     a.gate_limit = 0ull;
