@@ -13,7 +13,7 @@ namespace {
 constexpr int kChunk = kSortColsChunk;
 constexpr int kTileB = 128;          // batch rows of a tile: 64 lanes x 2
 constexpr int kRowPad = 128;         // weight rows are padded to a multiple of this in the tables
-constexpr int kMainWaves = 8;        // wavefronts of a workgroup of the main kernels
+constexpr int kMainWaves = 4;        // wavefronts of a workgroup of the main kernels
 constexpr int kMainTile = kMainWaves;   // weight rows of a workgroup, one per wavefront
 
 inline size_t align256(size_t b) { return (b + 255) / 256 * 256; }
