@@ -63,6 +63,10 @@ struct FwdArgs {
     const unsigned long long* gate;
     unsigned long long gate_limit;
     int gate_above;
+    // pinned words that the gated kernel leaves its outcome in, for the table hints (null: none): 1 in the first when it
+    // runs, 0 when it does not; in the second 1 when the word behind the gate is not zero
+    unsigned long long* told;
+    unsigned long long* told2;
     // interval forward with positions: non-null and non-zero on the device when a table kernel has already stored the
     // final values and positions, so that resolve_bound_kernel has nothing to do
     const unsigned long long* resolved;
@@ -70,6 +74,16 @@ struct FwdArgs {
 
 __device__ __forceinline__ bool gate_closed(const unsigned long long* gate, unsigned long long limit, int above) {
     return gate != nullptr && (*gate > limit) != (above != 0);
+}
+
+// the same for a forward tile kernel, whose first work-item reports the outcome
+__device__ __forceinline__ bool gate_closed(const FwdArgs& a) {
+    const bool closed = gate_closed(a.gate, a.gate_limit, a.gate_above);
+    if ((a.told || a.told2) && threadIdx.x == 0 && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) {
+        if (a.told) __hip_atomic_store(a.told, closed ? 0ull : 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (a.told2) __hip_atomic_store(a.told2, a.gate[1] != 0ull ? 1ull : 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    return closed;
 }
 
 // ---- error reporting ---------------------------------------------------------------------------
@@ -119,15 +133,16 @@ public:
 };
 
 // Whether a call site's candidate tables have paid lately.  Calls that queue a table kernel and an every-term kernel
-// for one result let the device choose, and report afterwards which ran (hint_record: an 8-byte copy of the device's
-// flag into pinned host memory, read by a later call once its event has completed; nothing waits).  When the every-term
-// kernel ran kHintStreak times in a row for a (site, weight matrix, shape) - a layer - the next kHintSkip calls do not build tables at all
-// (hint_build_tables returns false), then one call probes again.  A performance hint only: results do not depend on
-// it.  Neither function does anything while `stream` is being captured (tables are then always built).
+// for one result let the device choose, and report afterwards which ran: hint_expect returns a pinned word that the
+// every-term kernel stores its outcome in (FwdArgs::told; a copy and an event behind every call cost 10 us), read by a later
+// call once it is there; nothing waits.  When the every-term kernel ran kHintStreak times in a row for a (site, weight matrix,
+// shape) - a layer - the next kHintSkip calls do not build tables at all (hint_build_tables returns false), then one call
+// probes again.  A performance hint only: results do not depend on it.  Nothing is expected or remembered while `stream` is
+// being captured (tables are then always built).  hint_forget: the kernel was not launched after all.
 constexpr int kHintStreak = 3, kHintSkip = 31;
 bool hint_build_tables(int site, const void* weight, int B, int CO, int CI, hipStream_t stream);
-void hint_record(int site, const void* weight, int B, int CO, int CI, const unsigned long long* every_term_ran,
-                 hipStream_t stream);
+unsigned long long* hint_expect(int site, const void* weight, int B, int CO, int CI, hipStream_t stream);
+void hint_forget(unsigned long long* word);
 
 // zero-fill n floats on `stream` with a kernel (graph-capture friendly, no memset node)
 int fill_zero(void* ptr, size_t n_words, hipStream_t stream);

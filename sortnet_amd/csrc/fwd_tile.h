@@ -139,7 +139,7 @@ __device__ __forceinline__ void load_w_tile(float (*ws)[LDP], const FwdArgs& a,
 // -------------------------------------------------------------------------------------------
 template <class P, int TB, int TM>
 __global__ void __launch_bounds__(256, P::MIN_WAVES) fwd_kernel(FwdArgs a) {
-    if constexpr (P::GATED) { if (gate_closed(a.gate, a.gate_limit, a.gate_above)) return; }
+    if constexpr (P::GATED) { if (gate_closed(a)) return; }
     constexpr int BB = 16 * TB, BM = 16 * TM, NX = P::NX;
     __shared__ __attribute__((aligned(16))) float xs[NX][BB][LDP];
     __shared__ __attribute__((aligned(16))) float ws[BM][LDP];
@@ -229,7 +229,7 @@ constexpr int pipe_unroll() { return (TM <= 4 && P::UNROLL4_TM4) ? P::UNROLL4_TM
 
 template <class P, int TB, int TM>
 __global__ void __launch_bounds__(256, (pipe_waves<P, TB, TM>())) fwd_kernel_pipe(FwdArgs a) {
-    if constexpr (P::GATED) { if (gate_closed(a.gate, a.gate_limit, a.gate_above)) return; }
+    if constexpr (P::GATED) { if (gate_closed(a)) return; }
     constexpr int BB = 16 * TB, BM = 16 * TM, NX = P::NX;
     constexpr int NXV = (BB * 8 + 255) / 256, NWV = (BM * 8 + 255) / 256;
     __shared__ __attribute__((aligned(16))) float xs[NX][BB][LDP];
@@ -392,7 +392,7 @@ __global__ void __launch_bounds__(256, (pipe_waves<P, TB, TM>())) fwd_kernel_pip
 // -------------------------------------------------------------------------------------------
 template <class P, int TB, int TM>
 __global__ void __launch_bounds__(256, (pipe_waves<P, TB, TM>())) fwd_kernel_lists(FwdArgs a) {
-    if constexpr (P::GATED) { if (gate_closed(a.gate, a.gate_limit, a.gate_above)) return; }
+    if constexpr (P::GATED) { if (gate_closed(a)) return; }
     static_assert(P::NX == 1 && KT == 32, "one input tile, 32 columns per chunk");
     constexpr int BB = 16 * TB, BM = 16 * TM;
     constexpr int NXR = BB / 8, NWR = BM / 8;

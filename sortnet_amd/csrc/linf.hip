@@ -104,8 +104,9 @@ static int queue_max_cols(FwdArgs& a, int K, int B, int CO, int CI, void* ws, hi
     return SD_OK;
 }
 
-static void max_cols_report(const FwdArgs& a, int site, int B, int CO, int CI, hipStream_t st) {
-    if (g_linf_density.load(std::memory_order_relaxed) < 0.f && a.gate) hint_record(site, a.w, B, CO, CI, a.gate, st);
+// before the every-term kernel is queued behind the table kernels: where it reports
+static void max_cols_expect(FwdArgs& a, int site, int B, int CO, int CI, hipStream_t st) {
+    if (g_linf_density.load(std::memory_order_relaxed) < 0.f && a.gate) a.told = hint_expect(site, a.w, B, CO, CI, st);
 }
 
 extern "C" int sd_set_linf_candidate_density(float density) {
@@ -217,8 +218,9 @@ extern "C" int sd_inf_dist_forward_nograd(const float* input, const float* weigh
         if (!ws) return SD_ERR_HIP;
         if (K && (rc = queue_max_cols(a, K, B, CO, CI, ws, st))) return rc;
     }
+    if (K) max_cols_expect(a, kHintSiteLinf, B, CO, CI, st);
     rc = narrow ? launch_fwd<LinfNograd, 2, 2>(a, st) : TB == 2 ? launch_fwd<LinfNograd, 2, 8>(a, st) : launch_fwd<LinfNograd, 4, 8>(a, st);
-    if (K && rc == SD_OK) max_cols_report(a, kHintSiteLinf, B, CO, CI, st);
+    if (rc) hint_forget(a.told);
     return rc;
 }
 
@@ -244,8 +246,9 @@ extern "C" int sd_inf_dist_forward(const float* input, const float* weight,
     char* base = static_cast<char*>(workspace(merge + max_tables_bytes(B, CO, CI, KE), st));
     if (!base) return SD_ERR_HIP;
     if (K && (rc = queue_max_cols(a, K, B, CO, CI, base + merge, st))) return rc;
+    if (K) max_cols_expect(a, kHintSiteLinf, B, CO, CI, st);
     rc = run_chunk_pos<LinfChunk>(a, false, st, base, merge);
-    if (K && rc == SD_OK) max_cols_report(a, kHintSiteLinf, B, CO, CI, st);
+    if (rc) hint_forget(a.told);
     return rc;
 }
 
@@ -355,8 +358,9 @@ extern "C" int sd_masked_inf_dist_forward(const float* input, const float* weigh
     }
     if (pos) {
         if (K && (rc = queue_max_cols(a, K, B, CO, CI, tables, st))) return rc;
+        if (K) max_cols_expect(a, kHintSiteMasked, B, CO, CI, st);
         rc = run_chunk_pos<LinfChunk>(a, false, st);
-        if (K && rc == SD_OK) max_cols_report(a, kHintSiteMasked, B, CO, CI, st);
+        if (rc) hint_forget(a.told);
         return rc;
     }
     static const int kTb42[] = {4, 2};   // 8 rows per work-item measured slower (168 registers, three waves per SIMD)
@@ -365,8 +369,9 @@ extern "C" int sd_masked_inf_dist_forward(const float* input, const float* weigh
     a.nsplit = pick_nsplit(a, 16 * TB, narrow ? 32 : 128);
     if (a.nsplit > 1 && (rc = fill_zero(output, (size_t)B * CO * HW, st))) return rc;
     if (K && (rc = queue_max_cols(a, K, B, CO, CI, tables, st))) return rc;
+    if (K) max_cols_expect(a, kHintSiteMasked, B, CO, CI, st);
     rc = narrow ? launch_fwd<LinfNograd, 2, 2>(a, st) : TB == 2 ? launch_fwd<LinfNograd, 2, 8>(a, st) : launch_fwd<LinfNograd, 4, 8>(a, st);
-    if (K && rc == SD_OK) max_cols_report(a, kHintSiteMasked, B, CO, CI, st);
+    if (rc) hint_forget(a.told);
     return rc;
 }
 
@@ -432,11 +437,12 @@ extern "C" int sd_bound_inf_dist_forward_nograd(const float* inputL, const float
                                      bound_density >= 0.f ? bound_density : kBoundRowsCap, &a.gate, &a.gate_limit, st)))
             return rc;
         a.gate_above = 1;
-        rc = narrow ? launch_fwd<BoundNogradGated, 2, 2>(a, st) : TB == 2 ? launch_fwd<BoundNogradGated, 2, 8>(a, st) : launch_fwd<BoundNogradGated, 4, 8>(a, st);
-        if (hinted && rc == SD_OK) {
-            hint_record(kHintSiteBound, weight, B, CO, CI, a.gate, st);   // the gate is 1 when every term ran
-            if (bound_form == 0) hint_record(kHintSiteBoundSparse, weight, B, CO, CI, a.gate + 1, st);   // 1: very few marks
+        if (hinted) {
+            a.told = hint_expect(kHintSiteBound, weight, B, CO, CI, st);
+            if (bound_form == 0) a.told2 = hint_expect(kHintSiteBoundSparse, weight, B, CO, CI, st);   // 1: very few marks
         }
+        rc = narrow ? launch_fwd<BoundNogradGated, 2, 2>(a, st) : TB == 2 ? launch_fwd<BoundNogradGated, 2, 8>(a, st) : launch_fwd<BoundNogradGated, 4, 8>(a, st);
+        if (rc) { hint_forget(a.told); hint_forget(a.told2); }
         return rc;
     }
     if (narrow) return launch_fwd<BoundNograd, 2, 2>(a, st);
@@ -500,11 +506,11 @@ extern "C" int sd_bound_inf_dist_forward(const float* inputL, const float* input
             a.resolved = a.gate + 2;   // the tables per batch row store final values and positions themselves
         }
     }
+    if (hinted && cols) a.told = hint_expect(kHintSiteBoundPos, weight, B, CO, CI, st);
     // exact dense tiles: the LDS-direct kernel with the chunk numbers packed (same (value, chunk) pairs, same resolve)
     if (TB == 4 && a.nsplit > 1 && direct_ok<4, 4>(a) && (a.CIg / KT + a.nsplit - 1) / a.nsplit <= BoundChunkPacked::MAX_CHUNKS)
         rc = launch_fwd_direct<BoundChunkPacked, 4, 4>(a, st);
     else rc = narrow ? launch_fwd<BoundChunk, 2, 2>(a, st) : TB == 2 ? launch_fwd<BoundChunk, 2, 4>(a, st) : launch_fwd<BoundChunk, 4, 4>(a, st);
-    if (rc) return rc;
-    if (hinted && cols) hint_record(kHintSiteBoundPos, weight, B, CO, CI, a.gate, st);   // the gate is 1 when every term ran
+    if (rc) { hint_forget(a.told); return rc; }
     return launch_resolve_bound(a, st);
 }

@@ -122,12 +122,12 @@ void* workspace(size_t bytes, hipStream_t stream) {
 
 namespace {
 constexpr int kHintRing = 4;   // outcomes of a layer that may be on their way to the host at once
+constexpr unsigned long long kHintPending = ~0ull, kHintVoid = ~1ull;
 constexpr size_t kHintSlots = 256;   // layers (site, weight matrix) the hints remember at a time
 struct HintSlot {
     int dev, site, B, CO, CI;
     const void* weight;         // the layer: same shapes with other weights are other layers
-    unsigned long long* host;   // pinned: kHintRing flags
-    hipEvent_t ev[kHintRing];   // recorded behind the copy of flag i
+    unsigned long long* host;   // pinned: kHintRing outcomes, kHintPending until one has arrived
     int head, queued;           // oldest outcome not yet looked at, and how many are queued
     int stale;                  // of the queued outcomes, how many belong to the layer the slot stood for before
     int streak, skip_left;
@@ -137,8 +137,7 @@ std::mutex g_hint_mu;
 std::vector<HintSlot> g_hints;
 unsigned long long g_hint_clock = 0;
 
-// A slot that is handed to another layer keeps its pinned memory and events (copies into them may still be on their
-// way); what is queued at that moment is counted as stale and thrown away when it arrives.
+// A slot that is handed to another layer keeps its pinned memory (outcomes may still be on their way); what is queued at that moment is counted as stale and thrown away when it arrives.
 void hint_rekey(HintSlot& h, int dev, int site, const void* weight, int B, int CO, int CI) {
     h.dev = dev; h.site = site; h.weight = weight; h.B = B; h.CO = CO; h.CI = CI;
     h.stale = h.queued;
@@ -160,7 +159,7 @@ HintSlot* hint_slot(int site, const void* weight, int B, int CO, int CI, bool cr
     if (g_hints.size() >= kHintSlots) {
         HintSlot* oldest = nullptr;
         for (HintSlot& h : g_hints)
-            if (h.dev == dev && (!oldest || h.used < oldest->used)) oldest = &h;   // events belong to their device
+            if (h.dev == dev && (!oldest || h.used < oldest->used)) oldest = &h;
         if (!oldest) return nullptr;
         hint_rekey(*oldest, dev, site, weight, B, CO, CI);
         oldest->used = ++g_hint_clock;
@@ -171,15 +170,7 @@ HintSlot* hint_slot(int site, const void* weight, int B, int CO, int CI, bool cr
         (void)hipGetLastError();
         return nullptr;
     }
-    for (int i = 0; i < kHintRing; i++) {
-        h.host[i] = 0;
-        if (hipEventCreateWithFlags(&h.ev[i], hipEventDisableTiming) != hipSuccess) {
-            (void)hipGetLastError();
-            for (int k = 0; k < i; k++) (void)hipEventDestroy(h.ev[k]);   // nothing has been recorded on them yet
-            (void)hipHostFree(h.host);
-            return nullptr;
-        }
-    }
+    for (int i = 0; i < kHintRing; i++) h.host[i] = kHintPending;
     hint_rekey(h, dev, site, weight, B, CO, CI);
     h.used = ++g_hint_clock;
     g_hints.push_back(h);
@@ -194,10 +185,11 @@ bool hint_build_tables(int site, const void* weight, int B, int CO, int CI, hipS
     if (!h) return true;
     // outcomes that have arrived, oldest first (the host may run several calls ahead of the device)
     while (h->queued > 0) {
-        if (hipEventQuery(h->ev[h->head]) != hipSuccess) { (void)hipGetLastError(); break; }   // not ready: next call
+        const unsigned long long ran = __atomic_load_n(&h->host[h->head], __ATOMIC_ACQUIRE);
+        if (ran == kHintPending) break;   // not there yet: next call
         if (h->stale > 0) h->stale--;   // an outcome of the layer this slot stood for before
-        else {
-            h->streak = h->host[h->head] != 0ull ? h->streak + 1 : 0;
+        else if (ran != kHintVoid) {
+            h->streak = ran != 0ull ? h->streak + 1 : 0;
             // the streak is long enough (or the probe after a stretch without tables came out the same): no tables
             // for the next kHintSkip calls, then one call probes again
             h->skip_left = h->streak >= kHintStreak ? kHintSkip : 0;
@@ -209,19 +201,19 @@ bool hint_build_tables(int site, const void* weight, int B, int CO, int CI, hipS
     return true;
 }
 
-void hint_record(int site, const void* weight, int B, int CO, int CI, const unsigned long long* every_term_ran,
-                 hipStream_t stream) {
-    if (capturing(stream)) return;
+unsigned long long* hint_expect(int site, const void* weight, int B, int CO, int CI, hipStream_t stream) {
+    if (capturing(stream)) return nullptr;
     std::lock_guard<std::mutex> lock(g_hint_mu);
     HintSlot* h = hint_slot(site, weight, B, CO, CI, true);
-    if (!h || h->queued == kHintRing) return;
-    const int i = (h->head + h->queued) % kHintRing;
-    if (hipMemcpyAsync(h->host + i, every_term_ran, sizeof(unsigned long long), hipMemcpyDeviceToHost, stream) != hipSuccess ||
-        hipEventRecord(h->ev[i], stream) != hipSuccess) {
-        (void)hipGetLastError();
-        return;
-    }
+    if (!h || h->queued == kHintRing) return nullptr;
+    unsigned long long* word = h->host + (h->head + h->queued) % kHintRing;
+    __atomic_store_n(word, kHintPending, __ATOMIC_RELEASE);
     h->queued++;
+    return word;
+}
+
+void hint_forget(unsigned long long* word) {
+    if (word) __atomic_store_n(word, kHintVoid, __ATOMIC_RELEASE);
 }
 
 __global__ void __launch_bounds__(256) fill_zero_kernel(uint32_t* __restrict__ p, size_t n) {

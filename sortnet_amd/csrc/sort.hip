@@ -163,9 +163,9 @@ static bool sort_cols_eligible(const FwdArgs& a, int B, int CO, int CI, int G, i
 static bool sort_cols_ok(const FwdArgs& a, int site, int B, int CO, int CI, hipStream_t st) {
     return g_sort_density.load(std::memory_order_relaxed) > 0.f || hint_build_tables(site, a.w, B, CO, CI, st);
 }
-// after the every-term kernels have been queued behind the table kernel
-static void sort_cols_report(const FwdArgs& a, int site, int B, int CO, int CI, hipStream_t st) {
-    if (g_sort_density.load(std::memory_order_relaxed) < 0.f && a.gate) hint_record(site, a.w, B, CO, CI, a.gate, st);
+// before the every-term kernels are queued behind the table kernel: where they report
+static void sort_cols_expect(FwdArgs& a, int site, int B, int CO, int CI, hipStream_t st) {
+    if (g_sort_density.load(std::memory_order_relaxed) < 0.f && a.gate) a.told = hint_expect(site, a.w, B, CO, CI, st);
 }
 
 // Largest share of marked (tile of 128 weight rows, batch row, input) triples at which the kernel of the tables per
@@ -253,6 +253,7 @@ extern "C" int sd_sort_neuron_forward_nograd(const float* input, const float* we
     }
     int* keys = reinterpret_cast<int*>(base + tbytes);
     if (cols && (rc = queue_sort_cols(a, kRowsSortValues, input, nullptr, weight, B, CO, CI, q, K, nullptr, output, nullptr, base, st))) return rc;
+    if (cols) sort_cols_expect(a, kHintSiteSort, B, CO, CI, st);
     rc = SD_ERR_ARG;
     switch (K) {
 #define X(k) case k: if (k <= 12 && two) rc = run_two_level<(k <= 12 ? k : 2), true>(a, small, keys, st); \
@@ -261,7 +262,7 @@ extern "C" int sd_sort_neuron_forward_nograd(const float* input, const float* we
         SD_FOR_EACH_K(X)
 #undef X
     }
-    if (cols && rc == SD_OK) sort_cols_report(a, kHintSiteSort, B, CO, CI, st);
+    if (rc) hint_forget(a.told);
     return rc;
 }
 
@@ -290,6 +291,7 @@ extern "C" int sd_sort_neuron_forward(const float* input, const float* weight,
     }
     int* keys = reinterpret_cast<int*>(base + tbytes);
     if (cols && (rc = queue_sort_cols(a, kRowsSortPos, input, nullptr, weight, B, CO, CI, q, K, nullptr, output, pos, base, st))) return rc;
+    if (cols) sort_cols_expect(a, kHintSiteSortPos, B, CO, CI, st);
     rc = SD_ERR_ARG;
     switch (K) {
 #define X(k) case k: if (k <= 12 && two) rc = run_two_level<(k <= 12 ? k : 2), false>(a, few_tiles(a, 32, 64), keys, st); \
@@ -298,7 +300,7 @@ extern "C" int sd_sort_neuron_forward(const float* input, const float* weight,
         SD_FOR_EACH_K(X)
 #undef X
     }
-    if (cols && rc == SD_OK) sort_cols_report(a, kHintSiteSortPos, B, CO, CI, st);
+    if (rc) hint_forget(a.told);
     return rc;
 }
 
@@ -324,12 +326,13 @@ extern "C" int sd_bound_sort_neuron_forward(const float* inputL, const float* in
         if (!ws) return SD_ERR_HIP;
         if (cols && (rc = queue_sort_cols(a, kRowsSortInterval, inputL, inputU, weight, B, CO, CI, q, K, outputL, outputU, nullptr, ws, st))) return rc;
     }
+    if (cols) sort_cols_expect(a, kHintSiteBoundSort, B, CO, CI, st);
     rc = SD_ERR_ARG;
     switch (K) {
 #define X(k) case k: rc = small ? launch_fwd<BoundSort<k>, 1, 2>(a, st) : launch_fwd<BoundSort<k>, 2, 2>(a, st); break;
         SD_FOR_EACH_K(X)
 #undef X
     }
-    if (cols && rc == SD_OK) sort_cols_report(a, kHintSiteBoundSort, B, CO, CI, st);
+    if (rc) hint_forget(a.told);
     return rc;
 }
