@@ -414,6 +414,16 @@ std::pair<Tensor, Tensor> mean_shift(const Tensor& x, const OptTensor& running, 
     return mean_shift_index(x, {}, x.size(1), running, momentum);
 }
 
+// (sub_batches, groups, count) ascending kept channels, drawn on the current stream of `device`
+Tensor sample_index_lists(int64_t seed, int64_t sub_batches, int64_t groups, int64_t channels, int64_t count, at::Device device) {
+    const c10::DeviceGuard guard(device);
+    const Tensor out = at::empty({sub_batches, groups, count}, at::TensorOptions().dtype(at::kInt).device(device));
+    if (count > 0)
+        require(sd_sample_index_lists((uint32_t)seed, (int)sub_batches, (int)groups, (int)channels, (int)count, ints(out, "index"),
+                                      stream_of(out)), "sd_sample_index_lists");
+    return out;
+}
+
 // z + sign * vec[channel], outside any graph
 Tensor channel_shift(const Tensor& z_in, const Tensor& vec_in, double sign) {
     reverse_mode_only("channel_shift", z_in, vec_in);
@@ -482,5 +492,6 @@ PYBIND11_MODULE(_host, m) {
     m.def("mean_shift", &mean_shift, released());
     m.def("mean_shift_index", &mean_shift_index, released());
     m.def("channel_shift", &channel_shift, released());
+    m.def("sample_index_lists", &sample_index_lists, released());
     m.def("unfold", &unfold, released());
 }

@@ -26,6 +26,7 @@ from . import ext
 from . import functional as F
 
 SUB_BATCH = 32   # samples that share one index list (core/cuda/inf_dist_cuda.cu:8)
+SMALL_DRAW = 1 << 15   # channels over all lists of a draw below which the layer is paced by the host: 256 samples x 1024 channels are 8192
 
 
 def apply_if_not_none(paras, func):
@@ -52,13 +53,16 @@ class DropoutRegistry:
 
     def sample(self, sub_batches, groups, channels, q, device):
         """Ascending kept-channel lists (sub_batches, groups, count), count ~ Binomial(channels, q).
-        The lists depend on nothing but the seed, and the sampler keeps only a few compute units busy, so it
-        is queued on a second stream (default priority) and overlaps the kernels already queued on the
-        caller's stream; the caller's stream waits for it before going on."""
+        The lists depend on nothing but the seed, and the sampler keeps only a few compute units busy, so for a
+        large layer it is queued on a second stream (default priority) and overlaps the kernels already queued on
+        the caller's stream; the caller's stream waits for it before going on.  A small layer is paced by the host,
+        for which the second stream is 50 us of events, so its lists are drawn on the caller's stream (11 us)."""
         self.draws += 1
         seed = (self.seed * 1000003 + self.draws) & 0xFFFFFFFF
         count = ext.mask_count(seed, channels, q)
         device = torch.device(device)
+        if device.type == "cuda" and sub_batches * groups * channels < SMALL_DRAW:
+            return ext.host().sample_index_lists(seed, sub_batches, groups, channels, count, device)
         if device.type != "cuda" or not self.overlap_sampler:
             return ext.sample_index_lists(seed, sub_batches, groups, channels, count, device)
         main = torch.cuda.current_stream(device)
@@ -189,8 +193,11 @@ class NormDistBase(nn.Module):
         """Training path with kept-channel lists (core/models/norm_dist.py:55-85)."""
         reg, dev = self.registry, x.device
         sub_batches = (x.size(0) - 1) // SUB_BATCH + 1
-        rows = torch.div(torch.arange(x.size(0), device=dev), SUB_BATCH, rounding_mode="trunc")
         dim_out = self.weight.size(0) // self.groups
+
+        def rows():      # sub-batch of every sample
+            return torch.div(torch.arange(x.size(0), device=dev), SUB_BATCH, rounding_mode="trunc")
+
         index_in = None
         if self.tag in reg.entries and self.dropout != 1.0:
             dim_in, dim_out, q = reg.entries[self.tag]
@@ -199,7 +206,7 @@ class NormDistBase(nn.Module):
             else:
                 index_in = reg.sample(sub_batches, self.groups, dim_in, q, dev)
                 xg = x.view(x.size(0), self.groups, -1, x.size(-1))
-                gather = index_in[rows].unsqueeze(-1).long().expand(-1, -1, -1, x.size(-1))
+                gather = index_in[rows()].unsqueeze(-1).long().expand(-1, -1, -1, x.size(-1))
                 x = torch.gather(xg, 2, gather).reshape(x.size(0), -1, x.size(-1))
         index_out, bias = None, self.bias
         nxt = reg.entries.get(self.tag + 1)
@@ -208,7 +215,7 @@ class NormDistBase(nn.Module):
             reg.buffer = (self.tag + 1, index_out)
             if self.bias is not None:
                 per_row = self.bias.view(1, self.groups, -1).expand(x.size(0), -1, -1)
-                bias = torch.gather(per_row, -1, index_out[rows].long()).reshape(x.size(0), -1)
+                bias = torch.gather(per_row, -1, index_out[rows()].long()).reshape(x.size(0), -1)
         y = F.norm_dist_dropout(x.contiguous(), self.weight, index_in, index_out, self.p, self.groups, tag=self.tag)
         return y, index_out, bias
 
