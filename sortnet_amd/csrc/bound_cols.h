@@ -19,20 +19,18 @@ constexpr int kColsChunk = 32;
 size_t bound_cols_workspace(int B, int CO, int CI);
 
 // Builds the table, counts its marks on the device and queues the table kernel so that it runs only when at most
-// `density` of all (tile, weight row, input) triples are marked (`density_rows` of all (tile of weight rows, batch
-// row, input) triples where the table is built per batch row); the caller queues the kernel that evaluates every
-// term with the opposite condition on the same counter (*gate, *gate_limit).  outL / outU must be zero-filled:
-// the slices of the input range merge by atomic maximum.  (*gate)[1] (the word behind the gate) is 1 when the marks
-// per weight row are so few (below a sixteenth of the limit) that a kernel without LDS staging would serve better.
-// With packedL / packedU (B x CO words each, zero-filled) and posL / posU: the forward with positions.  The kernel of
-// the tables per weight row leaves (value bits << 32 | ~chunk of 32 inputs) per output in packedL / packedU, merged by
-// atomic maximum, as the every-term kernel with chunk tracking does (fwd_tile.h: store_chunk_winner), for
-// resolve_bound_kernel to take values and positions from; the kernel of the tables per batch row stores final values
-// and positions in outL / outU / posL / posU itself and sets (*gate)[2], which the resolve pass must be given as
-// FwdArgs::resolved.
+// `density` of all (tile, weight row, input) triples are marked.  outL / outU must be zero-filled: the slices of the input
+// range merge by atomic maximum.  *count: [0] the marks, [1] 1 when they are above the limit, or the table was not built
+// because the batch decides where a maximum sits, [2] 1 when they are so few (below a sixteenth of the limit) that a kernel
+// without LDS staging would serve better; *stat: the probe's two sums, for row_cands_forward.
+// With packedL / packedU (B x CO words each, zero-filled): the forward with positions.  The kernel leaves (value bits << 32 |
+// ~chunk of 32 inputs) per output in packedL / packedU, merged by atomic maximum, as the every-term kernel with chunk
+// tracking does (fwd_tile.h: store_chunk_winner), for resolve_bound_kernel to take values and positions from.
 int bound_cols_forward(const float* xl, const float* xu, const float* w, int B, int CO, int CI, float* outL,
-                       float* outU, unsigned long long* packedL, unsigned long long* packedU, int* posL, int* posU,
-                       void* ws, float density, float density_rows, const unsigned long long** gate,
-                       unsigned long long* gate_limit, hipStream_t st);
+                       float* outU, unsigned long long* packedL, unsigned long long* packedU, void* ws, float density,
+                       const unsigned long long** count, const float** stat, hipStream_t st);
+
+// *count + 2 of a call with this workspace
+const unsigned long long* bound_cols_few(int B, int CO, int CI, void* ws);
 
 }  // namespace sd

@@ -1,6 +1,5 @@
 // Interval-bound forward from per-weight-row candidate tables (see bound_cols.h).
 #include "bound_cols.h"
-#include "cand_walk.h"
 
 namespace sd {
 
@@ -18,51 +17,42 @@ inline int mpad_of(int M) { return (M + kTileW - 1) / kTileW * kTileW; }
 
 struct Carve {
     float* xr;        // [S][4][N]  per batch tile and input: min l, max l, min u, max u over the tile's rows (repaired)
-    float* wr;        // [T][2][N]  per weight tile and input: min w, max w over the tile's rows
-    float* low;       // [S][2][Mp] (or [T][2][Bp]) lower bounds of the upper / lower result of every output of the table's rows
+    float* low;       // [S][2][Mp] lower bounds of the upper / lower result of every output of a weight row
     float* stat;      // two sums of col_range_kernel's probe, directly behind `low` (one fill clears both)
-    unsigned long long* count;   // [0] marks of the per-weight-row table, [1] of the per-batch-row table, [2] every-term kernel's turn
-    uint32_t* bits;   // [S][NCH][Mp] (or [T][Bp][NCH]): bit i of a word = input 32 c + i may hold a maximum of that row in that tile
+    unsigned long long* count;   // see sum_tables_kernel
+    uint32_t* bits;   // [S][NCH][Mp]: bit i of a word = input 32 c + i may hold a maximum of that row in that tile
     uint32_t* partial;   // marks per wavefront of the table kernel
     uint32_t* order;  // [S][Mp] per batch tile and block of 128 weight rows: the row (0..127) at each place of the block
     float* xt;        // [S][N][64][4] per batch tile and input: (l, l', u, u') of the tile's rows i and i + 64, repaired
-    float* wt;        // [T][N][128] per weight tile and input: the weights of the tile's rows (the per-batch-row kernel walks these)
 };
 
-inline int bpad_of(int B) { return (B + kTileB - 1) / kTileB * kTileB; }
-inline size_t maxz(size_t a, size_t b) { return a > b ? a : b; }
-
-size_t carve_sizes(int B, int M, int N, size_t (&sz)[9]) {
-    const size_t S = tiles_b(B), Mp = mpad_of(M), Bp = bpad_of(B), T = Mp / kTileW, NCH = N / kChunk;
+size_t carve_sizes(int B, int M, int N, size_t (&sz)[7]) {
+    const size_t S = tiles_b(B), Mp = mpad_of(M), NCH = N / kChunk;
     sz[0] = align256(S * 4 * N * 4);                               // xr
-    sz[1] = align256(T * 2 * N * 4);                               // wr
-    sz[2] = align256(maxz(S * 2 * Mp, T * 2 * Bp) * 4 + 8);        // low + stat
-    sz[3] = 256;                                                   // count
-    sz[4] = align256(maxz(S * NCH * Mp, T * NCH * Bp) * 4);        // bits
-    sz[5] = align256(maxz(Mp / 64, Bp / 64 * ((T + 3) / 4)) * kLowSlices * 4 * 4);   // partial
-    sz[6] = align256(S * N * 1024);                                // xt
-    sz[7] = align256(S * Mp * 4);                                  // order
-    sz[8] = align256(Mp * N * 4);                                  // wt
-    return sz[0] + sz[1] + sz[2] + sz[3] + sz[4] + sz[5] + sz[6] + sz[7] + sz[8];
+    sz[1] = align256(S * 2 * Mp * 4 + 8);                          // low + stat
+    sz[2] = 256;                                                   // count
+    sz[3] = align256(S * NCH * Mp * 4);                            // bits
+    sz[4] = align256(Mp / 64 * kLowSlices * 4 * 4);                // partial
+    sz[5] = align256(S * N * 1024);                                // xt
+    sz[6] = align256(S * Mp * 4);                                  // order
+    return sz[0] + sz[1] + sz[2] + sz[3] + sz[4] + sz[5] + sz[6];
 }
 
 Carve carve(void* ws, int B, int M, int N) {
-    size_t sz[9];
+    size_t sz[7];
     carve_sizes(B, M, N, sz);
-    const size_t S = tiles_b(B), Mp = mpad_of(M), Bp = bpad_of(B), T = Mp / kTileW;
+    const size_t S = tiles_b(B), Mp = mpad_of(M);
     char* p = static_cast<char*>(ws);
     Carve c;
     c.xr = reinterpret_cast<float*>(p); p += sz[0];
-    c.wr = reinterpret_cast<float*>(p); p += sz[1];
     c.low = reinterpret_cast<float*>(p);
-    c.stat = c.low + maxz(S * 2 * Mp, T * 2 * Bp);
-    p += sz[2];
-    c.count = reinterpret_cast<unsigned long long*>(p); p += sz[3];
-    c.bits = reinterpret_cast<uint32_t*>(p); p += sz[4];
-    c.partial = reinterpret_cast<uint32_t*>(p); p += sz[5];
-    c.xt = reinterpret_cast<float*>(p); p += sz[6];
-    c.order = reinterpret_cast<uint32_t*>(p); p += sz[7];
-    c.wt = reinterpret_cast<float*>(p);
+    c.stat = c.low + S * 2 * Mp;
+    p += sz[1];
+    c.count = reinterpret_cast<unsigned long long*>(p); p += sz[2];
+    c.bits = reinterpret_cast<uint32_t*>(p); p += sz[3];
+    c.partial = reinterpret_cast<uint32_t*>(p); p += sz[4];
+    c.xt = reinterpret_cast<float*>(p); p += sz[5];
+    c.order = reinterpret_cast<uint32_t*>(p);
     return c;
 }
 
@@ -140,8 +130,8 @@ __global__ void __launch_bounds__(256) col_range_kernel(const float* __restrict_
 
 // The batch rows of a tile differ by more than kProbeRatio times what 16 entries of a weight column do (images
 // against small weights: ratio 15; the bounds of hidden layers: below 1): a table per weight row would mark every
-// input, because it is the batch row that decides where the maximum sits.  Then the table is built the other way
-// round, per batch row and tile of 128 weight rows (row_* kernels below); otherwise per weight row (col_*).
+// input, because it is the batch row that decides where the maximum sits.  Then it is not built, and the tables per batch
+// row and tile of 128 weight rows (row_cands.h) are.
 constexpr float kProbeRatio = 2.5f;
 __device__ __forceinline__ bool rows_decide(const float* stat, int S) {
     return stat[0] > kProbeRatio * (float)S * stat[1];
@@ -513,172 +503,24 @@ __device__ __forceinline__ void bound_cols_body(const float* __restrict__ xT, co
     }
 }
 
-// ---- the other orientation: tables per batch row and tile of 128 weight rows ----------------------
-// Over a tile of 128 weight rows the terms of (b, n) are bracketed by the column minimum and maximum of the weights.
-// Same three steps with the roles exchanged: ranges of W per (tile, input), lower bounds of the results per
-// (tile, batch row), marks per (tile, chunk, batch row).  All of them return at once unless rows_decide().
-__global__ void __launch_bounds__(256) row_range_kernel(const float* __restrict__ w, int M, int N, int S,
-                                                        float* __restrict__ wr, float* __restrict__ wt,
-                                                        const float* __restrict__ stat) {
-    if (!rows_decide(stat, S)) return;
-    __shared__ float part[4][3][64];
-    const int nl = threadIdx.x & 63, grp = threadIdx.x >> 6;
-    const int n = blockIdx.x * 64 + nl, t = blockIdx.y;
-    const int r0 = t * kTileW + grp * (kTileW / 4);
-    float lo = __builtin_inff(), hi = -__builtin_inff(), odd = 0.f;
-    if (n < N) {
-        // also the transposed copy the main kernel walks: wt[(t N + n) 128 + row of the tile] (rows past the last: 0)
-        float v[kTileW / 4];
-        #pragma unroll
-        for (int i = 0; i < kTileW / 4; i++) v[i] = r0 + i < M ? w[(size_t)(r0 + i) * N + n] : 0.f;
-        #pragma unroll
-        for (int i = 0; i < kTileW / 4; i++) {
-            if (r0 + i < M) { lo = fminf(lo, v[i]); hi = fmaxf(hi, v[i]); odd += v[i] - v[i]; }
-        }
-        float4* dst = reinterpret_cast<float4*>(wt + ((size_t)t * N + n) * kTileW + grp * (kTileW / 4));
-        #pragma unroll
-        for (int i = 0; i < kTileW / 16; i++) dst[i] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
-    }
-    part[grp][0][nl] = lo; part[grp][1][nl] = hi; part[grp][2][nl] = odd;
-    __syncthreads();
-    if (grp == 0 && n < N) {
-        #pragma unroll
-        for (int g = 1; g < 4; g++) { lo = fminf(lo, part[g][0][nl]); hi = fmaxf(hi, part[g][1][nl]); odd += part[g][2][nl]; }
-        // an undefined or infinite weight drops terms its neighbours keep: the column's range becomes everything
-        if (!(odd == 0.f)) { lo = -__builtin_inff(); hi = __builtin_inff(); }
-        wr[(size_t)(t * 2) * N + n] = lo;
-        wr[(size_t)(t * 2 + 1) * N + n] = hi;
-    }
-}
-
-// a workgroup takes 64 batch rows (one per lane; l and u through LDS, repaired) and a slice of the inputs; wavefront
-// v works on weight tile 4 blockIdx.z + v, whose column ranges are LDS broadcasts
 template <bool LOW>
-__device__ __forceinline__ void row_table_body(const float* __restrict__ xl, const float* __restrict__ xu,
-                                               const float* __restrict__ wr, int B, int N, int T, int Bp,
-                                               float* __restrict__ low, uint32_t* __restrict__ bits,
-                                               uint32_t* __restrict__ partial, int bx, int by, int bz, int gx, int gy) {
-    __shared__ __attribute__((aligned(16))) float lt[64][kChunk + 4];
-    __shared__ __attribute__((aligned(16))) float ut[64][kChunk + 4];
-    __shared__ __attribute__((aligned(16))) float ws[4][2][kChunk];   // min w, max w of the four weight tiles of this pass
-    const int tid = threadIdx.x, r = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int b0 = bx * 64, NCH = N / kChunk;
-    const int per = (NCH + gy - 1) / gy;
-    const int c_lo = by * per, c_hi = c_lo + per < NCH ? c_lo + per : NCH;
-    const int lrow = tid >> 2, q = tid & 3;
-    const int bload = b0 + lrow < B ? b0 + lrow : B - 1;
-    const bool valid = b0 + r < B;
-    const int xt = tid >> 6, xk = (tid >> 5) & 1, xn = tid & 31;   // this work-item's value of ws
-    int marks = 0;
-    {
-        const int tb = bz * 4;
-        const int t = tb + wave;
-        const bool active = t < T;
-        float LU = kEps, LL = kEps;
-        if (!LOW && active) {
-            LU = fmaxf(kEps, low[(size_t)(t * 2) * Bp + b0 + r]);
-            LL = fmaxf(kEps, low[(size_t)(t * 2 + 1) * Bp + b0 + r]);
-        }
-        float4 la, lb, ua, ub;
-        float px;
-        const float* wsrc = wr + ((size_t)(tb + xt < T ? tb + xt : T - 1) * 2 + xk) * N + xn;
-        auto fetch = [&](int c) {
-            const int cc = c < c_hi ? c : c_hi - 1;
-            const size_t off = (size_t)bload * N + cc * kChunk + 8 * q;
-            la = *reinterpret_cast<const float4*>(xl + off); lb = *reinterpret_cast<const float4*>(xl + off + 4);
-            ua = *reinterpret_cast<const float4*>(xu + off); ub = *reinterpret_cast<const float4*>(xu + off + 4);
-            px = wsrc[cc * kChunk];
-        };
-        if (c_lo < c_hi) fetch(c_lo);
-        for (int c = c_lo; c < c_hi; c++) {
-            {
-                float4 a = la, b = lb, d = ua, e = ub;
-                repair(a.x, d.x); repair(a.y, d.y); repair(a.z, d.z); repair(a.w, d.w);
-                repair(b.x, e.x); repair(b.y, e.y); repair(b.z, e.z); repair(b.w, e.w);
-                *reinterpret_cast<float4*>(&lt[lrow][8 * q]) = a; *reinterpret_cast<float4*>(&lt[lrow][8 * q + 4]) = b;
-                *reinterpret_cast<float4*>(&ut[lrow][8 * q]) = d; *reinterpret_cast<float4*>(&ut[lrow][8 * q + 4]) = e;
-                ws[xt][xk][xn] = px;
-            }
-            fetch(c + 1);
-            __syncthreads();
-            if (active) {
-                uint32_t word = 0;
-                #pragma unroll
-                for (int n4 = 0; n4 < kChunk; n4 += 4) {
-                    const float4 l4 = *reinterpret_cast<const float4*>(&lt[r][n4]);
-                    const float4 u4 = *reinterpret_cast<const float4*>(&ut[r][n4]);
-                    const float4 a4 = *reinterpret_cast<const float4*>(&ws[wave][0][n4]);   // min w
-                    const float4 b4 = *reinterpret_cast<const float4*>(&ws[wave][1][n4]);   // max w
-                    const float l[4] = {l4.x, l4.y, l4.z, l4.w}, u[4] = {u4.x, u4.y, u4.z, u4.w};
-                    const float wmin[4] = {a4.x, a4.y, a4.z, a4.w}, wmax[4] = {b4.x, b4.y, b4.z, b4.w};
-                    #pragma unroll
-                    for (int k = 0; k < 4; k++) {
-                        if (LOW) {
-                            LU = fmaxf(fmaxf(LU, wmin[k] - l[k]), u[k] - wmax[k]);
-                            LL = fmaxf(fmaxf(LL, l[k] - wmax[k]), wmin[k] - u[k]);
-                        } else {
-                            const float capU = fmaxf(wmax[k] - l[k], u[k] - wmin[k]);
-                            const float capL = fmaxf(l[k] - wmin[k], wmax[k] - u[k]);
-                            word |= (uint32_t)(!(capU < LU) || !(capL < LL)) << (n4 + k);   // undefined counts as a candidate
-                        }
-                    }
-                }
-                if (!LOW) {
-                    if (!valid) word = 0u;
-                    bits[((size_t)t * Bp + b0 + r) * NCH + c] = word;   // a row's words side by side
-                    marks += __builtin_popcount(word);
-                }
-            }
-            __syncthreads();
-        }
-        if (LOW && active && valid) {
-            atomicMax(reinterpret_cast<int*>(low + (size_t)(t * 2) * Bp + b0 + r), __float_as_int(LU));
-            atomicMax(reinterpret_cast<int*>(low + (size_t)(t * 2 + 1) * Bp + b0 + r), __float_as_int(LL));
-        }
-    }
-    if (!LOW) {
-        #pragma unroll
-        for (int o = 32; o; o >>= 1) marks += __shfl_xor(marks, o);
-        if (r == 0)
-            partial[(((size_t)bz * gy + by) * gx + bx) * 4 + wave] = (uint32_t)marks;
-    }
+__global__ void __launch_bounds__(256) table_kernel(const float* __restrict__ w, const float* __restrict__ xr, int M, int N, int S,
+                                                    int Mp, float* __restrict__ low, uint32_t* __restrict__ bits,
+                                                    uint32_t* __restrict__ partial, uint32_t* __restrict__ order,
+                                                    const float* __restrict__ stat) {
+    if (rows_decide(stat, S)) return;
+    col_table_body<LOW>(w, xr, M, N, S, Mp, low, bits, partial, order, blockIdx.x, blockIdx.y, gridDim.x, gridDim.y);
 }
 
-// Both table steps as one launch each: the probe picks the orientation, and workgroups beyond the grid of that
-// orientation return at once.
-template <bool LOW>
-__global__ void __launch_bounds__(256) table_kernel(const float* __restrict__ xl, const float* __restrict__ xu,
-                                                    const float* __restrict__ w, const float* __restrict__ xr,
-                                                    const float* __restrict__ wr, int B, int M, int N, int S, int T,
-                                                    int Mp, int Bp, int slices, float* __restrict__ low,
-                                                    uint32_t* __restrict__ bits, uint32_t* __restrict__ partial,
-                                                    uint32_t* __restrict__ order, const float* __restrict__ stat) {
-    const int id = blockIdx.x;
-    if (rows_decide(stat, S)) {
-        const int gx = Bp / 64, gy = slices, gz = (T + 3) / 4;
-        if (id >= gx * gy * gz) return;
-        row_table_body<LOW>(xl, xu, wr, B, N, T, Bp, low, bits, partial, id % gx, (id / gx) % gy, id / (gx * gy), gx, gy);
-    } else {
-        const int gx = Mp / 64, gy = slices;
-        if (id >= gx * gy) return;
-        col_table_body<LOW>(w, xr, M, N, S, Mp, low, bits, partial, order, id % gx, id / gx, gx, gy);
-    }
-}
-
-// count[0] = marks of the table per weight row, count[1] = of the table per batch row (the one that was not built
-// counts as full), count[2] = 1 when neither is below its limit, which is what the every-term kernel waits for,
-// count[3] = 1 when the per-weight-row marks are below a sixteenth of their limit (for the caller's choice of kernel),
-// count[4] = 1 when the kernel of the tables per batch row runs (with positions it stores the final results itself)
-__global__ void __launch_bounds__(1024) sum_tables_kernel(const uint32_t* __restrict__ partial, size_t n_col,
-                                                          size_t n_row, unsigned long long* __restrict__ count,
-                                                          const float* __restrict__ stat, int S,
-                                                          unsigned long long limit_col, unsigned long long limit_row) {
+// count[0] = marks (a table that was not built counts as full), count[1] = 1 when they are above the limit, count[2] = 1 when
+// they are below a sixteenth of it (for the caller's choice of kernel)
+__global__ void __launch_bounds__(1024) sum_tables_kernel(const uint32_t* __restrict__ partial, size_t n,
+                                                          unsigned long long* __restrict__ count,
+                                                          const float* __restrict__ stat, int S, unsigned long long limit) {
     __shared__ unsigned long long acc[1024];
     const bool rows = rows_decide(stat, S);
-    const size_t n = rows ? n_row : n_col;
     unsigned long long s0 = 0;
-    for (size_t i = threadIdx.x; i < n; i += 1024) s0 += partial[i];
+    if (!rows) for (size_t i = threadIdx.x; i < n; i += 1024) s0 += partial[i];
     acc[threadIdx.x] = s0;
     __syncthreads();
     for (int o = 512; o; o >>= 1) {
@@ -686,112 +528,14 @@ __global__ void __launch_bounds__(1024) sum_tables_kernel(const uint32_t* __rest
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        const unsigned long long c = rows ? ~0ull : acc[0], r = rows ? acc[0] : ~0ull;
+        const unsigned long long c = rows ? ~0ull : acc[0];
         count[0] = c;
-        count[1] = r;
-        count[2] = (c > limit_col && r > limit_row) ? 1ull : 0ull;
+        count[1] = c > limit ? 1ull : 0ull;
         // so few marks per weight row that staging tiles through LDS is most of the main kernel's time
-        count[3] = c <= limit_col / 16 ? 1ull : 0ull;
-        count[4] = (c > limit_col && r <= limit_row) ? 1ull : 0ull;
+        count[2] = c <= limit / 16 ? 1ull : 0ull;
     }
 }
 
-// Main kernel of this orientation.  A wavefront takes one batch row against the tile's 128 weight rows (lane l holds the
-// rows l and l + 64): it lists the row's marked inputs in LDS, cuts the list by what a few strong marks say (cand_walk.h) and
-// walks what is left: per mark the row's (l, u) (scalar operands) and the lane's two weights from the transposed copy (two
-// coalesced 256-byte loads).  No tile is staged and no barrier is met; the workgroups of a tile (eight wavefronts = eight
-// batch rows each) are dealt to one die, whose cache then holds the tile's transposed weights.  One wavefront sees every
-// input of its outputs, so the results are stored, not merged.
-// POS: the mark that last improved a bound strictly is the first input attaining it (the marks go by in input order,
-// and every input that attains a bound is marked), so values and positions are stored as they are
-// (core/cuda/bound_inf_dist_cuda.cu:176-212: position = input | bit 31 when w - l > u - w; a lower bound that never
-// left its floor keeps 0xffffffff) and the resolve pass is told to skip the call (count[4]).
-constexpr int kWalkWaves = 8;        // wavefronts of a workgroup
-
-template <bool POS>
-__global__ void __launch_bounds__(64 * kWalkWaves)
-bound_rows_walk_kernel(const float* __restrict__ xl, const float* __restrict__ xu, const float* __restrict__ wt,
-                       const float* __restrict__ wr, const uint32_t* __restrict__ bits,
-                       const unsigned long long* __restrict__ count, unsigned long long limit_col,
-                       unsigned long long limit_row, int B, int Bp, int M, int N, float* __restrict__ yL,
-                       float* __restrict__ yU, int* __restrict__ posL, int* __restrict__ posU) {
-    if (count[0] <= limit_col || count[1] > limit_row) return;   // the other table's turn, or the every-term kernel's
-    __shared__ uint16_t lists[kWalkWaves][kWalkListCap];
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int NCH = N / kChunk, BG = (B + kWalkWaves - 1) / kWalkWaves;
-    int item = blockIdx.x;
-    if (gridDim.x % 8 == 0) item = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-    const int bg = item % BG, t = item / BG;
-    const int b = bg * kWalkWaves + wave;
-    if (b >= B) return;   // wave-uniform
-    const float* __restrict__ wcol = wt + (size_t)t * N * kTileW + lane;
-    uint16_t* list = lists[wave];
-    const uint32_t* __restrict__ rowbits = bits + ((size_t)t * Bp + b) * NCH;
-    const float* __restrict__ xlrow = xl + (size_t)b * N;
-    const float* __restrict__ xurow = xu + (size_t)b * N;
-    const float* __restrict__ wmin = wr + (size_t)(t * 2) * N;
-    const float* __restrict__ wmax = wmin + N;
-    const bool in0 = t * kTileW + lane < M, in1 = t * kTileW + lane + 64 < M;   // the lane's weight rows exist
-    float lo[2] = {-kEps, -kEps}, hi[2] = {kEps, kEps};
-    int pl[2] = {-1, -1}, pu[2] = {0, 0};   // POS: the input that last improved the bound, with its flag
-    float wa[2][4], wb[2][4];
-    auto load = [&](int buf, int i, int n) __attribute__((always_inline)) {
-        wa[buf][i] = wcol[(size_t)n * kTileW];
-        wb[buf][i] = wcol[(size_t)n * kTileW + 64];
-    };
-    auto use = [&](int buf, int i, int k, int n, const Own& o) __attribute__((always_inline)) {
-        const float li = lane_value(o.a, k), ui = lane_value(o.b, k);
-        const float a1 = wa[buf][i] - li, a2 = ui - wa[buf][i], b1 = wb[buf][i] - li, b2 = ui - wb[buf][i];
-        if constexpr (POS) {
-            const int p0 = a1 <= a2 ? n : n | (int)0x80000000, p1 = b1 <= b2 ? n : n | (int)0x80000000;
-            const float v0 = fminf(a1, a2), V0 = fmaxf(a1, a2), v1 = fminf(b1, b2), V1 = fmaxf(b1, b2);
-            const bool w0 = v0 < lo[0], w1 = v1 < lo[1], w2 = V0 > hi[0], w3 = V1 > hi[1];
-            lo[0] = w0 ? v0 : lo[0]; lo[1] = w1 ? v1 : lo[1];
-            hi[0] = w2 ? V0 : hi[0]; hi[1] = w3 ? V1 : hi[1];
-            pl[0] = w0 ? p0 : pl[0]; pl[1] = w1 ? p1 : pl[1];
-            pu[0] = w2 ? p0 : pu[0]; pu[1] = w3 ? p1 : pu[1];
-        } else {
-            lo[0] = fminf(fminf(lo[0], a1), a2);
-            hi[0] = fmaxf(fmaxf(hi[0], a1), a2);
-            lo[1] = fminf(fminf(lo[1], b1), b2);
-            hi[1] = fmaxf(fmaxf(hi[1], b1), b2);
-        }
-    };
-    // smallest results of the lane's rows over the wavefront (weight rows past the last one do not count)
-    float thU = 0.f, thL = 0.f;
-    for_marks(list, NCH, lane, [&](int c) __attribute__((always_inline)) { return rowbits[c]; },
-              [&](int total, bool first) __attribute__((always_inline)) {
-        walk_marks<POS, true>(list, total, first, lane,
-            [&](int n) __attribute__((always_inline)) { Own o{xlrow[n], xurow[n]}; repair(o.a, o.b); return o; },
-            // (the two caps of an input differ by the same width nearly everywhere, so the upper one ranks for both)
-            [&](int n, const Own& o) __attribute__((always_inline)) { return fmaxf(wmax[n] - o.a, o.b - wmin[n]); },
-            load, use, use,
-            [&](bool) __attribute__((always_inline)) {
-                thU = wave_min_nonneg(fminf(in0 ? hi[0] : __builtin_inff(), in1 ? hi[1] : __builtin_inff()));
-                thL = wave_min_nonneg(fminf(in0 ? -lo[0] : __builtin_inff(), in1 ? -lo[1] : __builtin_inff()));
-            },
-            [&](int n, const Own& o) __attribute__((always_inline)) {
-                const float a = wmin[n], b = wmax[n];
-                return !(fmaxf(b - o.a, o.b - a) < thU) || !(fmaxf(o.a - a, b - o.b) < thL);
-            },
-            [&]() __attribute__((always_inline)) {
-                lo[0] = lo[1] = -kEps; hi[0] = hi[1] = kEps;
-                pl[0] = pl[1] = -1; pu[0] = pu[1] = 0;
-            });
-    });
-    #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int col = t * kTileW + lane + 64 * j;
-        if (col < M) {
-            const size_t o = (size_t)b * M + col;
-            yL[o] = -lo[j]; yU[o] = hi[j];
-            if constexpr (POS) { posL[o] = pl[j]; posU[o] = pu[j]; }
-        }
-    }
-}
-
-// The kernel of the tables per weight row (the tables per batch row have bound_rows_walk_kernel)
 template <bool POS>
 __global__ void __launch_bounds__(1024, 1)
 bound_table_kernel(const float* __restrict__ w, const float* __restrict__ xT, const uint32_t* __restrict__ bits,
@@ -806,49 +550,36 @@ bound_table_kernel(const float* __restrict__ w, const float* __restrict__ xT, co
 }  // namespace
 
 size_t bound_cols_workspace(int B, int CO, int CI) {
-    size_t sz[9];
+    size_t sz[7];
     return carve_sizes(B, CO, CI, sz);
 }
 
+const unsigned long long* bound_cols_few(int B, int CO, int CI, void* ws) { return carve(ws, B, CO, CI).count + 2; }
+
 int bound_cols_forward(const float* xl, const float* xu, const float* w, int B, int CO, int CI, float* outL,
-                       float* outU, unsigned long long* packedL, unsigned long long* packedU, int* posL, int* posU,
-                       void* ws, float density, float density_rows, const unsigned long long** gate,
-                       unsigned long long* gate_limit, hipStream_t st) {
-    const bool with_pos = packedL != nullptr;
+                       float* outU, unsigned long long* packedL, unsigned long long* packedU, void* ws, float density,
+                       const unsigned long long** count, const float** stat, hipStream_t st) {
     if (CI % kChunk != 0 || B < 1 || CO < 1) { set_error("bound_cols_forward: shape not supported"); return SD_ERR_ARG; }
     const Carve c = carve(ws, B, CO, CI);
-    const int S = tiles_b(B), Mp = mpad_of(CO), Bp = bpad_of(B), T = Mp / kTileW, NCH = CI / kChunk;
-    const size_t lown = maxz((size_t)S * 2 * Mp, (size_t)T * 2 * Bp);
+    const int S = tiles_b(B), Mp = mpad_of(CO), T = Mp / kTileW, NCH = CI / kChunk;
     int rc;
-    if ((rc = fill_zero(c.low, lown + 2, st))) return rc;   // the lower bounds and the two sums behind them
+    if ((rc = fill_zero(c.low, (size_t)S * 2 * Mp + 2, st))) return rc;   // the lower bounds and the two sums behind them
     hipLaunchKernelGGL(col_range_kernel, dim3((CI + 63) / 64, S), dim3(256), 0, st, xl, xu, w, B, CO, CI, c.xr, c.stat);
     if ((rc = check_launch("col_range_kernel"))) return rc;
     const int slices = NCH < kLowSlices ? NCH : kLowSlices;
     const float d = density < 0.f ? 0.f : density > 1.f ? 1.f : density;
-    const float dr = density_rows < 0.f ? 0.f : density_rows > 1.f ? 1.f : density_rows;
-    const unsigned long long limit_col = (unsigned long long)((double)S * CO * CI * d);
-    // (the kernel of the tables per batch row lists 16-bit input numbers)
-    const unsigned long long limit_row = CI <= 65536 ? (unsigned long long)((double)T * B * CI * dr) : 0ull;
-    // ranges of W per tile of weight rows and the transposed copy: only when the probe picks the tables per batch row
-    hipLaunchKernelGGL(row_range_kernel, dim3((CI + 63) / 64, T), dim3(256), 0, st, w, CO, CI, S, c.wr, c.wt, c.stat);
-    if ((rc = check_launch("row_range_kernel"))) return rc;
-    const int wg_col = (Mp / 64) * slices, wg_row = (Bp / 64) * slices * ((T + 3) / 4);
-    const int wg_tab = wg_col > wg_row ? wg_col : wg_row;
-    hipLaunchKernelGGL(table_kernel<true>, dim3(wg_tab), dim3(256), 0, st, xl, xu, w, c.xr, c.wr, B, CO, CI, S, T, Mp, Bp,
-                       slices, c.low, c.bits, c.partial, c.order, c.stat);
+    const unsigned long long limit = (unsigned long long)((double)S * CO * CI * d);
+    const dim3 grid(Mp / 64, slices);
+    hipLaunchKernelGGL(table_kernel<true>, grid, dim3(256), 0, st, w, c.xr, CO, CI, S, Mp, c.low, c.bits, c.partial, c.order, c.stat);
     if ((rc = check_launch("table_kernel<low>"))) return rc;
-    hipLaunchKernelGGL(table_kernel<false>, dim3(wg_tab), dim3(256), 0, st, xl, xu, w, c.xr, c.wr, B, CO, CI, S, T, Mp, Bp,
-                       slices, c.low, c.bits, c.partial, c.order, c.stat);
+    hipLaunchKernelGGL(table_kernel<false>, grid, dim3(256), 0, st, w, c.xr, CO, CI, S, Mp, c.low, c.bits, c.partial, c.order, c.stat);
     if ((rc = check_launch("table_kernel<bits>"))) return rc;
-    hipLaunchKernelGGL(sum_tables_kernel, dim3(1), dim3(1024), 0, st, c.partial, (size_t)wg_col * 4, (size_t)wg_row * 4,
-                       c.count, c.stat, S, limit_col, limit_row);
+    hipLaunchKernelGGL(sum_tables_kernel, dim3(1), dim3(1024), 0, st, c.partial, (size_t)grid.x * grid.y * 4, c.count, c.stat, S, limit);
     if ((rc = check_launch("sum_tables_kernel"))) return rc;
-    // the every-term kernel runs when count[2] > 0
-    *gate = c.count + 2;
-    *gate_limit = 0ull;
-    note_term_counts(c.count, 2, (double)S * CO * CI, (double)T * B * CI, limit_col);
+    *count = c.count;
+    *stat = c.stat;
     // a few workgroups per compute unit over the run: the work of a workgroup follows the marks of its rows
-    hipLaunchKernelGGL(xt_kernel, dim3(CI / 16, S), dim3(256), 0, st, xl, xu, B, CI, c.count, limit_col, c.xt);
+    hipLaunchKernelGGL(xt_kernel, dim3(CI / 16, S), dim3(256), 0, st, xl, xu, B, CI, c.count, limit, c.xt);
     if ((rc = check_launch("xt_kernel"))) return rc;
     // Slices of the input range.  A workgroup takes a whole compute unit and stays for its whole run, so the launch
     // proceeds in rounds of num_cus() workgroups and 2.5 rounds cost three: the count with the least time by that
@@ -860,23 +591,16 @@ int bound_cols_forward(const float* xl, const float* xu, const float* w, int B, 
         const double cost = (double)((wgs * n + cus - 1) / cus) / n * (1.0 + 0.04 * n);
         if (n == 1 || cost < best) { best = cost; nsplit = n; }
     }
-    const int BG = (B + kWalkWaves - 1) / kWalkWaves;
-    if (with_pos) {
+    if (packedL) {
         // chunk numbers within a slice take 8 bits (255 = none)
         while ((((NCH + 1) / 2 + nsplit - 1) / nsplit) * 2 > 254) nsplit++;
         hipLaunchKernelGGL(bound_table_kernel<true>, dim3((unsigned)(wgs * nsplit)), dim3(1024), 0, st, w, c.xt, c.bits,
-                           c.order, c.count, limit_col, B, CO, Mp, CI, nsplit, nullptr, nullptr, packedL, packedU);
-        if ((rc = check_launch("bound_table_kernel"))) return rc;
-        hipLaunchKernelGGL(bound_rows_walk_kernel<true>, dim3((unsigned)(T * BG)), dim3(64 * kWalkWaves), 0, st, xl, xu, c.wt,
-                           c.wr, c.bits, c.count, limit_col, limit_row, B, Bp, CO, CI, outL, outU, posL, posU);
-        return check_launch("bound_rows_walk_kernel");
+                           c.order, c.count, limit, B, CO, Mp, CI, nsplit, nullptr, nullptr, packedL, packedU);
+    } else {
+        hipLaunchKernelGGL(bound_table_kernel<false>, dim3((unsigned)(wgs * nsplit)), dim3(1024), 0, st, w, c.xt, c.bits, c.order,
+                           c.count, limit, B, CO, Mp, CI, nsplit, outL, outU, nullptr, nullptr);
     }
-    hipLaunchKernelGGL(bound_table_kernel<false>, dim3((unsigned)(wgs * nsplit)), dim3(1024), 0, st, w, c.xt, c.bits, c.order,
-                       c.count, limit_col, B, CO, Mp, CI, nsplit, outL, outU, nullptr, nullptr);
-    if ((rc = check_launch("bound_table_kernel"))) return rc;
-    hipLaunchKernelGGL(bound_rows_walk_kernel<false>, dim3((unsigned)(T * BG)), dim3(64 * kWalkWaves), 0, st, xl, xu, c.wt, c.wr, c.bits,
-                       c.count, limit_col, limit_row, B, Bp, CO, CI, outL, outU, nullptr, nullptr);
-    return check_launch("bound_rows_walk_kernel");
+    return check_launch("bound_table_kernel");
 }
 
 }  // namespace sd

@@ -44,7 +44,7 @@ struct TableArgs {
     const float* v1;                // rows (R, N); PAIR: the upper of two values
     const float* v2;                // PAIR: the lower
     const uint32_t* keep;           // MASK: one word per (row, 32 inputs)
-    const float* ranges;            // [tiles][N] of (min, max), TWO: of (min l, max l, min u, max u)
+    const float* ranges;            // [tiles][N] of (min, max), TWO without PAIR: of (min l, max l, min u, max u)
     int R, Rp, N, tiles, K;
     float* low;                     // [tiles][TWO ? 2 : 1][Rp]
     uint32_t* bits;                 // [tiles][Rp][table_row_words(N)]
@@ -66,13 +66,13 @@ __device__ __forceinline__ float wave_max_nonneg(float f) {
 }
 
 // Row values v1, v2 (equal unless PAIR) against ranges (lo, hi): lowest and largest a term max(v1 - x, x - v2) can be.
-// TWO: ranges (min l, max l, min u, max u) of an interval [l, u] against one value, and the same for the lower bound of the
-// term, max(l - v, v - u).
+// TWO: a bound for each result of the intervals: marks for max(v1 - x, x - v2) and for max(v2 - x, x - v1) (PAIR), or ranges
+// (min l, max l, min u, max u) of an interval [l, u] against one value v, marks for max(u - v, v - l) and for max(l - v, v - u).
 // Returns the marks of a wavefront's rows.
 template <int RW, int NT, bool PAIR, bool TWO, bool MASK>
 __device__ __forceinline__ int build_tables(const TableArgs& a, int bx, int by, float* smem) {
-    static_assert(!(PAIR && TWO) && RW * NT <= 4 && kTableSlice == 2 * kTableBlock, "");
-    constexpr int NP = TWO ? 4 : 2, NL = TWO ? 2 : 1, T = 64 * kTableWaves, PER = NP * kTableSlice / T;
+    static_assert(RW * NT <= 4 && kTableSlice == 2 * kTableBlock, "");
+    constexpr int NP = TWO && !PAIR ? 4 : 2, NL = TWO ? 2 : 1, T = 64 * kTableWaves, PER = NP * kTableSlice / T;
     typedef float Plane[NP][kTableSlice];
     Plane* rg = reinterpret_cast<Plane*>(smem);   // [NT]
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -173,12 +173,15 @@ __device__ __forceinline__ int build_tables(const TableArgs& a, int bx, int by, 
             for (int t = 0; t < NT; t++) {
                 float p0[4], p1[4], p2[4], p3[4];
                 range4(t, 0, b, p0); range4(t, 1, b, p1);
-                if constexpr (TWO) { range4(t, 2, b, p2); range4(t, 3, b, p3); }
+                if constexpr (TWO && !PAIR) { range4(t, 2, b, p2); range4(t, 3, b, p3); }
                 #pragma unroll
                 for (int r = 0; r < RW; r++) {
                     #pragma unroll
                     for (int e = 0; e < 4; e++) {   // (fmaxf drops undefined differences)
-                        if constexpr (TWO) {
+                        if constexpr (TWO && PAIR) {
+                            best[r][t][0] = fmaxf(fmaxf(best[r][t][0], vu[b][r][e] - p1[e]), p0[e] - vl[b][r][e]);
+                            best[r][t][1] = fmaxf(fmaxf(best[r][t][1], vl[b][r][e] - p1[e]), p0[e] - vu[b][r][e]);
+                        } else if constexpr (TWO) {
                             best[r][t][0] = fmaxf(fmaxf(best[r][t][0], vu[b][r][e] - p1[e]), p2[e] - vl[b][r][e]);
                             best[r][t][1] = fmaxf(fmaxf(best[r][t][1], p0[e] - vu[b][r][e]), vl[b][r][e] - p3[e]);
                         } else {
@@ -244,13 +247,16 @@ __device__ __forceinline__ int build_tables(const TableArgs& a, int bx, int by, 
             for (int t = 0; t < NT; t++) {
                 float p0[4], p1[4], p2[4], p3[4];
                 range4(t, 0, b, p0); range4(t, 1, b, p1);
-                if constexpr (TWO) { range4(t, 2, b, p2); range4(t, 3, b, p3); }
+                if constexpr (TWO && !PAIR) { range4(t, 2, b, p2); range4(t, 3, b, p3); }
                 #pragma unroll
                 for (int r = 0; r < RW; r++) {
                     #pragma unroll
                     for (int e = 0; e < 4; e++) {
                         bool mark;
-                        if constexpr (TWO) {
+                        if constexpr (TWO && PAIR) {
+                            mark = fmaxf(vu[b][r][e] - p0[e], p1[e] - vl[b][r][e]) >= best[r][t][0];
+                            mark = mark || fmaxf(vl[b][r][e] - p0[e], p1[e] - vu[b][r][e]) >= best[r][t][1];
+                        } else if constexpr (TWO) {
                             mark = fmaxf(vu[b][r][e] - p0[e], p3[e] - vl[b][r][e]) >= best[r][t][0];
                             mark = mark || fmaxf(p1[e] - vu[b][r][e], vl[b][r][e] - p2[e]) >= best[r][t][1];
                         } else mark = fmaxf(vu[b][r][e] - p0[e], p1[e] - vl[b][r][e]) >= best[r][t][0];

@@ -64,9 +64,10 @@ struct FwdArgs {
     unsigned long long gate_limit;
     int gate_above;
     // pinned words that the gated kernel leaves its outcome in, for the table hints (null: none): 1 in the first when it
-    // runs, 0 when it does not; in the second 1 when the word behind the gate is not zero
+    // runs, 0 when it does not; in the second whether *few is not zero
     unsigned long long* told;
     unsigned long long* told2;
+    const unsigned long long* few;
     // interval forward with positions: non-null and non-zero on the device when a table kernel has already stored the
     // final values and positions, so that resolve_bound_kernel has nothing to do
     const unsigned long long* resolved;
@@ -81,7 +82,7 @@ __device__ __forceinline__ bool gate_closed(const FwdArgs& a) {
     const bool closed = gate_closed(a.gate, a.gate_limit, a.gate_above);
     if ((a.told || a.told2) && threadIdx.x == 0 && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) {
         if (a.told) __hip_atomic_store(a.told, closed ? 0ull : 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        if (a.told2) __hip_atomic_store(a.told2, a.gate[1] != 0ull ? 1ull : 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (a.told2) __hip_atomic_store(a.told2, *a.few != 0ull ? 1ull : 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
     return closed;
 }
@@ -99,11 +100,9 @@ void forward_kernel_timer(hipStream_t stream, bool after);
 // call lie on the device and how to turn them into the share of the terms that the call formed.
 //   kind 0: no tables were queued (every term is formed)
 //   kind 1: counts[0] = marked (tile, weight row, input) triples of denom0, counts[1] != 0 when the every-term kernel ran
-//   kind 2: counts[0] / counts[1] = marks of the table per weight row (of denom0) / per batch row (of denom1),
-//           counts[2] != 0 when the every-term kernel ran, else the per-weight-row table served iff counts[0] <= limit0
 //   kind 3: counts[0] = marks of the table per batch row (of denom0), counts[1] != 0 when the every-term kernels ran,
 //           counts[2] != 0 when the per-batch-row table served, counts[3] = marks of the table per weight row (of denom1)
-void note_term_counts(const unsigned long long* counts, int kind, double denom0, double denom1, unsigned long long limit0);
+void note_term_counts(const unsigned long long* counts, int kind, double denom0, double denom1);
 
 #define SD_REQUIRE(cond, ...)                                   \
     do {                                                        \

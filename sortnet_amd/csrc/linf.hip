@@ -17,7 +17,7 @@ static std::atomic<float> g_bound_density{-1.f};
 // measured at B = 512, M = N = 5120: the table kernel takes 0.09 + 2.6 x share ms (about 60 SIMD cycles per marked
 // (tile, weight row, input)) after 0.10 ms for the tables, against 1.00 ms for every term.  The tables are paid for by the time
 // the choice is made, so the limit sits a little below where the two would meet.  Per batch row (us, every term / tables):
-// 993 / 360 (6.5 % marked), 998 / 376 (13 %), 982 / 451 (25 %), with positions 1235 / 399, 1238 / 490, 1271 / 683; 128 x 5120 x
+// 1004 / 379 (9.2 % marked), with positions 1246 / 466; 982 / 451 (25 %), with positions 1271 / 683; 128 x 5120 x
 // 5120 281 / 227 and 351 / 300 (25 %).
 constexpr float kBoundColsCap = 0.30f, kBoundRowsCap = 0.40f;
 // With the built-in limits, layers below this many terms go without tables: building them and starting the table
@@ -28,6 +28,15 @@ constexpr long long kBoundColsMinTerms = 1ll << 31;
 // selects per output instead of a three-operand minimum or maximum) and the every-term kernel 1.5 times as long per
 // term, so the limit is lower per weight row.
 constexpr float kBoundPosColsCap = 0.15f;
+// Layers between kBoundRowsMinTerms + kBoundRowsMinOutputs x inputs and kBoundColsMinTerms terms are given the tables per batch
+// row alone: a wavefront walks a row, so the time follows the length of the rows (about 14 us + 17 us per 1024 inputs) and not
+// the outputs, which is what the every-term kernel's time follows.  Every term / tables, us, images against weights of scale
+// 0.02 (9.4 % marked), without and with positions: 512 x 1024 x 1024 57 / 41, 95 / 56; 250 x 3072 x 1021 84 / 70, 110 / 87; 400 x
+// 5120 x 640 139 / 95, 218 / 114; below the line 128 x 1024 x 1024 21 / 34, 39 / 42 and 100 x 3072 x 1024 44 / 65, 62 / 80.  At 22.5 %
+// marked 256 x 2048 x 1200 takes 67 / 73, 99 / 109 (512 x 1024 x 1024 57 / 51), which is where their limit comes from.  Weights
+// that decide mark everything: about 25 us for the tables, until the hints say not to build them.
+constexpr long long kBoundRowsMinTerms = 1ll << 27, kBoundRowsMinOutputs = 3ll << 16;
+constexpr float kBoundSmallRowsCap = 0.18f;
 constexpr int kHintSiteBound = 1, kHintSiteBoundSparse = 8, kHintSiteBoundPos = 9;
 constexpr float kBoundSparseCap = 0.03f;   // marked share up to which the kernel without LDS staging runs
 static std::atomic<int> g_bound_form{0};            // 0: chosen per layer, 1: staged tiles, 2: transposed-row walk
@@ -100,7 +109,7 @@ static int queue_max_cols(FwdArgs& a, int K, int B, int CO, int CI, void* ws, hi
     if (rc) return rc;
     a.gate = every;
     a.gate_limit = 0ull;
-    note_term_counts(every - 1, 3, (double)((CO + 127) / 128) * B * CI, (double)((B + 127) / 128) * CO * CI, 0ull);
+    note_term_counts(every - 1, 3, (double)((CO + 127) / 128) * B * CI, (double)((B + 127) / 128) * CO * CI);
     return SD_OK;
 }
 
@@ -375,6 +384,53 @@ extern "C" int sd_masked_inf_dist_forward(const float* input, const float* weigh
     return rc;
 }
 
+// Interval forward from tables per batch row (row_cands.h): what they need behind the tables per weight row, 0 where they do
+// not serve
+static size_t bound_rows_bytes(int B, int CO, int CI) {
+    return CI <= 65536 && (long long)B * CO < (1ll << 32) ? row_cands_workspace(kRowsBound, B, CO, CI) : 0;
+}
+
+// Tables for the interval forward in front of the every-term kernel: per weight row (`cols`, bound_cols.h) and per batch row, or
+// the latter alone, which are then built whatever the operands.  Afterwards a.gate[0] is non-zero when the every-term kernel is to run, and
+// a.resolved (with positions) when the kernel of the tables per batch row has stored final values and positions.
+// `ws`: bound_tables_bytes() bytes.
+static size_t bound_tables_bytes(bool cols, int B, int CO, int CI) {
+    return (cols ? bound_cols_workspace(B, CO, CI) : 0) + bound_rows_bytes(B, CO, CI);
+}
+
+static int queue_bound_tables(FwdArgs& a, bool cols, int B, int CO, int CI, float cap, char* ws, hipStream_t st) {
+    const float density = g_bound_density.load(std::memory_order_relaxed);
+    const unsigned long long* count = nullptr;
+    const float* stat = nullptr;
+    char* rows_ws = ws + (cols ? bound_cols_workspace(B, CO, CI) : 0);
+    int rc = cols ? bound_cols_forward(a.x0, a.x1, a.w, B, CO, CI, a.y0, a.y1, a.packed0, a.packed1, ws, cap, &count, &stat, st) : SD_OK;
+    if (rc) return rc;
+    a.gate_above = 1;
+    a.gate_limit = 0ull;
+    if (cols) a.gate = count + 1;
+    if (bound_rows_bytes(B, CO, CI) == 0) {
+        note_term_counts(count, 1, (double)((B + 127) / 128) * CO * CI, 1.0);
+        return SD_OK;
+    }
+    const unsigned long long* every = nullptr;
+    rc = row_cands_forward(kRowsBound, a.x0, a.x1, a.w, nullptr, nullptr, B, CO, CI, 0.f, 1, a.y0, a.y1, a.p1, rows_ws,
+                           density >= 0.f ? density : cols ? kBoundRowsCap : kBoundSmallRowsCap, density >= 0.f, stat, count, &every, st, a.p0);
+    if (rc) return rc;
+    a.gate = every;
+    if (a.p0) a.resolved = every + 1;
+    note_term_counts(every - 1, 3, (double)((CO + 127) / 128) * B * CI, (double)((B + 127) / 128) * CO * CI);
+    return SD_OK;
+}
+
+// whether an interval forward gets tables, by shape and size alone: of both orientations (0: none; 1: per batch row; 2: both)
+static int bound_tables_eligible(const FwdArgs& a, float cap, int B, int CO, int CI, int G, int HW) {
+    const float density = g_bound_density.load(std::memory_order_relaxed);
+    if (!(cap > 0.f && G == 1 && HW == 1 && CI % kColsChunk == 0 && a.fast_x && a.fast_w)) return 0;
+    const long long terms = (long long)B * CO * CI;
+    if (density >= 0.f || terms >= kBoundColsMinTerms) return 2;
+    return terms >= kBoundRowsMinTerms + kBoundRowsMinOutputs * CI && bound_rows_bytes(B, CO, CI) > 0 ? 1 : 0;
+}
+
 extern "C" int sd_bound_inf_dist_forward_nograd(const float* inputL, const float* inputU, const float* weight,
                                                 int B, int CO, int CI, int G, int HW, float* outputL, float* outputU,
                                                 sd_stream_t stream) {
@@ -397,25 +453,25 @@ extern "C" int sd_bound_inf_dist_forward_nograd(const float* inputL, const float
     const float bound_density = g_bound_density.load(std::memory_order_relaxed);
     const int bound_form = g_bound_form.load(std::memory_order_relaxed);
     const float cap = bound_density >= 0.f ? bound_density : kBoundColsCap;
-    bool cols = cap > 0.f && G == 1 && HW == 1 && CI % kColsChunk == 0 && a.fast_x && a.fast_w &&
-                (bound_density >= 0.f || (long long)B * CO * CI >= kBoundColsMinTerms);
+    int tables = bound_tables_eligible(a, cap, B, CO, CI, G, HW);
     // The workspace is sized by shape alone (whatever the hints below decide), so that a call under graph capture,
-    // which always builds the staged tables, never needs more than the eager call before it did.
+    // which always builds the tables, never needs more than the eager call before it did.
     char* wsbase = nullptr;
-    if (cols) {
-        const size_t staged = bound_cols_workspace(B, CO, CI), walk = CI <= 65536 ? sort_cols_workspace(B, CO, CI) : 0;
-        wsbase = static_cast<char*>(workspace(staged > walk ? staged : walk, st));   // the only request of this call
-        if (!wsbase) return SD_ERR_HIP;
+    if (tables) {
+        const size_t both = bound_tables_bytes(tables == 2, B, CO, CI), walk = tables == 2 && CI <= 65536 ? sort_cols_workspace(B, CO, CI) : 0;
+        const size_t bytes = both > walk ? both : walk;
+        if (bound_density < 0.f && !workspace_ready(bytes, st)) tables = 0;   // a first call under capture forms every term
+        else if (!(wsbase = static_cast<char*>(workspace(bytes, st)))) return SD_ERR_HIP;   // the only request of this call
     }
     // with the built-in limit, a layer whose tables have not paid lately is not given any for a while
-    const bool hinted = cols && bound_density < 0.f;
-    if (hinted && !hint_build_tables(kHintSiteBound, weight, B, CO, CI, st)) cols = false;
+    const bool hinted = tables && bound_density < 0.f;
+    if (hinted && !hint_build_tables(kHintSiteBound, weight, B, CO, CI, st)) tables = 0;
     // Very few marks (weights of unit scale against rows that are alike: below 1 %): the staged kernel would spend its
     // time moving tiles through LDS, and the kernel that walks a weight row's marks over a transposed copy of the
     // inputs serves better.  Chosen by hand (sd_set_bound_candidate_form) or, with the built-in limit, for a layer
     // whose last three staged calls reported that few marks ("not building" the staged tables, in the hint's terms).
-    bool sparse = cols && bound_form == 2 && CI <= 65536;
-    if (cols && bound_form == 0 && hinted && CI <= 65536)
+    bool sparse = tables == 2 && bound_form == 2 && CI <= 65536;
+    if (tables == 2 && bound_form == 0 && hinted && CI <= 65536)
         sparse = !hint_build_tables(kHintSiteBoundSparse, weight, B, CO, CI, st);
     if (sparse) {
         void* ws = wsbase;
@@ -428,18 +484,17 @@ extern "C" int sd_bound_inf_dist_forward_nograd(const float* inputL, const float
         a.gate_above = 1;
         return narrow ? launch_fwd<BoundNogradGated, 2, 2>(a, st) : TB == 2 ? launch_fwd<BoundNogradGated, 2, 8>(a, st) : launch_fwd<BoundNogradGated, 4, 8>(a, st);
     }
-    if (a.nsplit > 1 || cols) {
+    if (a.nsplit > 1 || tables == 2) {
         if ((rc = fill_zero2(outputL, (size_t)B * CO * HW, outputU, (size_t)B * CO * HW, st))) return rc;
     }
-    if (cols) {
-        void* ws = wsbase;
-        if ((rc = bound_cols_forward(inputL, inputU, weight, B, CO, CI, outputL, outputU, nullptr, nullptr, nullptr, nullptr, ws, cap,
-                                     bound_density >= 0.f ? bound_density : kBoundRowsCap, &a.gate, &a.gate_limit, st)))
-            return rc;
-        a.gate_above = 1;
+    if (tables) {
+        if ((rc = queue_bound_tables(a, tables == 2, B, CO, CI, cap, wsbase, st))) return rc;
         if (hinted) {
             a.told = hint_expect(kHintSiteBound, weight, B, CO, CI, st);
-            if (bound_form == 0) a.told2 = hint_expect(kHintSiteBoundSparse, weight, B, CO, CI, st);   // 1: very few marks
+            if (tables == 2 && bound_form == 0) {   // 1: very few marks
+                a.told2 = hint_expect(kHintSiteBoundSparse, weight, B, CO, CI, st);
+                a.few = bound_cols_few(B, CO, CI, wsbase);
+            }
         }
         rc = narrow ? launch_fwd<BoundNogradGated, 2, 2>(a, st) : TB == 2 ? launch_fwd<BoundNogradGated, 2, 8>(a, st) : launch_fwd<BoundNogradGated, 4, 8>(a, st);
         if (rc) { hint_forget(a.told); hint_forget(a.told2); }
@@ -484,29 +539,23 @@ extern "C" int sd_bound_inf_dist_forward(const float* inputL, const float* input
     // of the every-term kernel as for the forward without positions; both leave (value, chunk) pairs for the resolve
     const float bound_density = g_bound_density.load(std::memory_order_relaxed);
     const float cap = bound_density >= 0.f ? bound_density : kBoundPosColsCap;
-    bool cols = cap > 0.f && G == 1 && HW == 1 && CI % kColsChunk == 0 && a.fast_x && a.fast_w &&
-                (bound_density >= 0.f || (long long)B * CO * CI >= kBoundColsMinTerms);
-    const bool elig = cols;   // by shape alone: what the workspace is sized by (a captured call always builds tables)
-    const bool hinted = cols && bound_density < 0.f;
-    if (hinted && !hint_build_tables(kHintSiteBoundPos, weight, B, CO, CI, st)) cols = false;
-    if (cols && a.nsplit < 2) a.nsplit = 2;   // both kernels merge into the packed pairs
+    int tables = bound_tables_eligible(a, cap, B, CO, CI, G, HW);
+    const size_t pairs = ((size_t)a.R * a.G * a.COg * 16 + 255) / 256 * 256;
+    if (tables && bound_density < 0.f && !workspace_ready(pairs + bound_tables_bytes(tables == 2, B, CO, CI), st)) tables = 0;   // a first call under capture
+    const int elig = tables;   // by shape alone: what the workspace is sized by (a captured call always builds tables)
+    const bool hinted = tables && bound_density < 0.f;
+    if (hinted && !hint_build_tables(kHintSiteBoundPos, weight, B, CO, CI, st)) tables = 0;
+    if (tables == 2 && a.nsplit < 2) a.nsplit = 2;   // both kernels merge into the packed pairs
     if (a.nsplit > 1 || elig) {
         size_t n = (size_t)a.R * a.G * a.COg;
-        const size_t pairs = (n * 16 + 255) / 256 * 256;
-        char* ws = static_cast<char*>(workspace(pairs + (elig ? bound_cols_workspace(B, CO, CI) : 0), st));   // the only request
+        char* ws = static_cast<char*>(workspace(pairs + (elig ? bound_tables_bytes(elig == 2, B, CO, CI) : 0), st));   // the only request
         if (!ws) return SD_ERR_HIP;
         a.packed0 = reinterpret_cast<unsigned long long*>(ws);
         a.packed1 = a.packed0 + n;
         if (a.nsplit > 1 && (rc = fill_zero(a.packed0, n * 4, st))) return rc;
-        if (cols) {
-            if ((rc = bound_cols_forward(inputL, inputU, weight, B, CO, CI, outputL, outputU, a.packed0, a.packed1, posL, posU,
-                                         ws + pairs, cap, bound_density >= 0.f ? bound_density : kBoundRowsCap, &a.gate, &a.gate_limit, st)))
-                return rc;
-            a.gate_above = 1;
-            a.resolved = a.gate + 2;   // the tables per batch row store final values and positions themselves
-        }
+        if (tables && (rc = queue_bound_tables(a, tables == 2, B, CO, CI, cap, ws + pairs, st))) return rc;
     }
-    if (hinted && cols) a.told = hint_expect(kHintSiteBoundPos, weight, B, CO, CI, st);
+    if (hinted && tables) a.told = hint_expect(kHintSiteBoundPos, weight, B, CO, CI, st);
     // exact dense tiles: the LDS-direct kernel with the chunk numbers packed (same (value, chunk) pairs, same resolve)
     if (TB == 4 && a.nsplit > 1 && direct_ok<4, 4>(a) && (a.CIg / KT + a.nsplit - 1) / a.nsplit <= BoundChunkPacked::MAX_CHUNKS)
         rc = launch_fwd_direct<BoundChunkPacked, 4, 4>(a, st);

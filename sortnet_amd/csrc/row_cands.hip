@@ -29,7 +29,7 @@ struct RowCount {
 struct Carve {
     RowCount* count;
     float* wr;        // [T][N]  per tile of weight rows and input: (min, max) of the weights over the rows that keep the input
-    float* low;       // [T][Bp]  lower bounds of the K-th largest terms of a batch row
+    float* low;       // [T][Bp]  lower bounds of the K-th largest terms of a batch row (kRowsBound: [T][2][Bp], of the two results)
     uint32_t* bits;   // [T][Bp][table_row_words] the marks
     uint32_t* fix;    // [B * M] outputs of the masked l-inf form whose bound did not hold (recomputed from every input)
     float* wt;        // [T][N][128] the weights of a tile, one 512-byte row per input (dropped weights undefined)
@@ -39,7 +39,7 @@ size_t carve_sizes(int form, int B, int M, int N, size_t (&sz)[6]) {
     const size_t T = tiles_w(M), Bp = bpad_of(B);
     sz[0] = 256;
     sz[1] = align256(T * 2 * N * 4);
-    sz[2] = align256(T * Bp * 4);
+    sz[2] = align256((form == kRowsBound ? 2 : 1) * T * Bp * 4);
     sz[3] = align256(T * Bp * table_row_words(N) * 4);
     sz[4] = form == kRowsMax ? align256((size_t)B * M * 4) : 0;
     sz[5] = align256(T * N * kTileW * 4);
@@ -72,10 +72,10 @@ __device__ __forceinline__ void repair(float& l, float& u) {
 // columns over 16 weight rows.
 // `ratio` is kProbeRatio for the sort-neuron forms.  The l-inf form asks for more (kProbeRatioMax): its kernel only pays
 // below about 25 % of marks, and on inputs spread evenly over their range the marked share is about 1 / (that ratio), so
-// its tables are not even built unless the probe promises that few.
+// its tables are not even built unless the probe promises that few.  Without a probe (null) they are built.
 constexpr float kProbeRatio = 2.5f, kProbeRatioMax = 5.f;
 __device__ __forceinline__ bool rows_decide(const float* stat, int S, float ratio) {
-    return stat[0] > ratio * (float)S * stat[1];
+    return stat == nullptr || stat[0] > ratio * (float)S * stat[1];
 }
 
 // ---- tables ----------------------------------------------------------------------------------
@@ -132,21 +132,21 @@ __global__ void __launch_bounds__(256) rc_range_kernel(const float* __restrict__
 }
 
 // Bounds and marks (cand_tables.h): four tiles of weight rows at a time
-template <bool PAIR, bool MASK>
+template <bool PAIR, bool TWO, bool MASK>
 __global__ void __launch_bounds__(64 * kTableWaves)
 rc_tables_kernel(TableArgs a, RowCount* __restrict__ c, const unsigned long long* __restrict__ col_count,
                  const float* __restrict__ stat, int S, unsigned long long limit, float ratio) {
     __shared__ __attribute__((aligned(16))) float smem[4 * 2 * kTableSlice];
     unsigned long long marks = ~0ull;
     if (rows_decide(stat, S, ratio)) {
-        const int part = build_tables<1, 4, PAIR, false, MASK>(a, blockIdx.x, blockIdx.y, smem);
+        const int part = build_tables<1, 4, PAIR, TWO, MASK>(a, blockIdx.x, blockIdx.y, smem);
         if (!add_marks(&c->sum, part, &marks)) return;
     } else if (blockIdx.x != 0 || blockIdx.y != 0 || threadIdx.x != 0) return;
     const bool run = marks <= limit;   // (the limit is a share of the (tile, row, input) triples: never all ones)
     c->marks = marks;
-    c->every = (col_count[1] != 0ull && !run) ? 1ull : 0ull;
+    c->every = ((col_count == nullptr || col_count[1] != 0ull) && !run) ? 1ull : 0ull;
     c->run = run ? 1ull : 0ull;
-    c->col_marks = col_count[0];
+    c->col_marks = col_count == nullptr ? ~0ull : col_count[0];
 }
 
 // ---- main kernel -------------------------------------------------------------------------------
@@ -158,7 +158,7 @@ rc_tables_kernel(TableArgs a, RowCount* __restrict__ c, const unsigned long long
 // 5120 inputs) stay in that die's cache while its 64 resident workgroups walk them.
 // Forms: top-K lists of values (branch-free median insertion, left out where it would change no lane's list), of both
 // interval bounds, of values with the input numbers (the reference's ordered insertion: the marks go by in ascending input
-// order), and the l-inf distance (the difference of largest magnitude and, optionally, its input; under the factored mask the
+// order), the interval bounds of the l-inf distance, and the l-inf distance (the difference of largest magnitude and, optionally, its input; under the factored mask the
 // dropped weights of the transposed copy are undefined, the table holds no input the batch row drops, and an output that
 // ends below the bound its marks were taken against is listed for rc_fix_kernel).
 constexpr int kRtWaves = 8;          // wavefronts of a workgroup
@@ -170,15 +170,15 @@ struct RtArgs {
     uint32_t* fix;
     int B, Bp, M, N;
     float q;
-    float* outL; float* outU; int* pos;
+    float* outL; float* outU; int* pos; int* posL;
 };
 
 template <int FORM, int K, bool POS, bool MASKED>
 __global__ void __launch_bounds__(64 * kRtWaves) rt_main_kernel(RtArgs a) {
     if (a.count->run == 0ull) return;
-    constexpr bool IV = FORM == kRowsSortInterval;
-    constexpr bool LISTS = FORM != kRowsMax;
-    constexpr bool ORDERED = FORM == kRowsSortPos || (FORM == kRowsMax && POS);   // the input a term sits at is wanted
+    constexpr bool IV = FORM == kRowsSortInterval || FORM == kRowsBound;
+    constexpr bool LISTS = FORM != kRowsMax && FORM != kRowsBound;
+    constexpr bool ORDERED = FORM == kRowsSortPos || (!LISTS && POS);   // the input a term sits at is wanted
     __shared__ uint16_t lists[kRtWaves][kWalkListCap];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -197,9 +197,9 @@ __global__ void __launch_bounds__(64 * kRtWaves) rt_main_kernel(RtArgs a) {
 
     // state of the row x the lane's two weight rows: top-K lists (ascending; as bit patterns where only values are wanted), or
     // the difference of largest magnitude
-    using Entry = typename std::conditional<FORM == kRowsSortValues || IV, int, float>::type;
+    using Entry = typename std::conditional<FORM == kRowsSortValues || FORM == kRowsSortInterval, int, float>::type;
     Entry hi[2][LISTS ? K : 1], lo[IV ? 2 : 1][IV ? K : 1];
-    int idx[ORDERED ? 2 : 1][FORM == kRowsSortPos ? K : 1];
+    int idx[ORDERED ? 2 : 1][FORM == kRowsSortPos ? K : 1], idxL[2];
     auto clear = [&]() __attribute__((always_inline)) {
         #pragma unroll
         for (int j = 0; j < 2; j++) {
@@ -213,6 +213,7 @@ __global__ void __launch_bounds__(64 * kRtWaves) rt_main_kernel(RtArgs a) {
             } else {
                 hi[j][0] = kEps;
                 if constexpr (POS) idx[j][0] = 0;
+                if constexpr (FORM == kRowsBound) { lo[j][0] = kEps; idxL[j] = (int)kNanId; }
             }
         }
     };
@@ -234,9 +235,27 @@ __global__ void __launch_bounds__(64 * kRtWaves) rt_main_kernel(RtArgs a) {
             const float ui = lane_value(o.b, k);
             const float a1 = wa[buf][i] - xi, a2 = ui - wa[buf][i];
             const float b1 = wb[buf][i] - xi, b2 = ui - wb[buf][i];
+            if constexpr (FORM == kRowsBound) {
+                // an undefined operand leaves the other's term; only a strictly better term replaces a bound, so with
+                // positions the first of equal terms keeps it
+                const float L0 = -fminf(a1, a2), U0 = fmaxf(a1, a2), L1 = -fminf(b1, b2), U1 = fmaxf(b1, b2);
+                if constexpr (POS) {
+                    const int p0 = a1 <= a2 ? n : n | (int)kSign, p1 = b1 <= b2 ? n : n | (int)kSign;
+                    const bool l0 = L0 > lo[0][0], l1 = L1 > lo[1][0], u0 = U0 > hi[0][0], u1 = U1 > hi[1][0];
+                    lo[0][0] = l0 ? L0 : lo[0][0]; idxL[0] = l0 ? p0 : idxL[0];
+                    lo[1][0] = l1 ? L1 : lo[1][0]; idxL[1] = l1 ? p1 : idxL[1];
+                    hi[0][0] = u0 ? U0 : hi[0][0]; idx[0][0] = u0 ? p0 : idx[0][0];
+                    hi[1][0] = u1 ? U1 : hi[1][0]; idx[1][0] = u1 ? p1 : idx[1][0];
+                } else {
+                    lo[0][0] = fmaxf(lo[0][0], L0); lo[1][0] = fmaxf(lo[1][0], L1);
+                    hi[0][0] = fmaxf(hi[0][0], U0); hi[1][0] = fmaxf(hi[1][0], U1);
+                }
+                return;
+            } else {
             // (the maximum with -1 turns a term that is undefined altogether into a negative one, which the lists ignore)
             insert_pair<K>(lo[0], fmaxf(fmaxf(-a1, -a2), -1.f), lo[1], fmaxf(fmaxf(-b1, -b2), -1.f));
             insert_pair<K>(hi[0], fmaxf(fmaxf(a1, a2), -1.f), hi[1], fmaxf(fmaxf(b1, b2), -1.f));
+            }
         } else {
             const float d0 = xi - wa[buf][i], d1 = xi - wb[buf][i];
             if constexpr (FORM == kRowsSortValues) {
@@ -267,7 +286,6 @@ __global__ void __launch_bounds__(64 * kRtWaves) rt_main_kernel(RtArgs a) {
     };
     auto value = [&](int buf, int i, int k, int n, const Own& o) __attribute__((always_inline)) { term(std::bool_constant<FORM == kRowsSortPos>{}, buf, i, k, n, o); };
     auto use = [&](int buf, int i, int k, int n, const Own& o) __attribute__((always_inline)) { term(std::false_type{}, buf, i, k, n, o); };
-    const float LU = a.low[(size_t)t * a.Bp + b];   // wave-uniform
     // smallest results of the lane's rows over the wavefront (weight rows past the last one do not count)
     float thU = 0.f, thL = 0.f;
     auto smallest = [&](float v0, float v1) __attribute__((always_inline)) {
@@ -291,9 +309,10 @@ __global__ void __launch_bounds__(64 * kRtWaves) rt_main_kernel(RtArgs a) {
             load, value, use,
             [&](bool strong) __attribute__((always_inline)) {
                 if (FORM == kRowsSortPos && strong) { least[0] = hi[0][0]; least[1] = hi[1][0]; }
-                if constexpr (FORM == kRowsSortValues || IV) thU = smallest(__int_as_float(hi[0][0]), __int_as_float(hi[1][0]));
+                if constexpr (FORM == kRowsSortValues || FORM == kRowsSortInterval) thU = smallest(__int_as_float(hi[0][0]), __int_as_float(hi[1][0]));
                 else thU = smallest(fmaxf(fabsf(hi[0][0]), least[0]), fmaxf(fabsf(hi[1][0]), least[1]));
-                if constexpr (IV) thL = smallest(__int_as_float(lo[0][0]), __int_as_float(lo[1][0]));
+                if constexpr (FORM == kRowsSortInterval) thL = smallest(__int_as_float(lo[0][0]), __int_as_float(lo[1][0]));
+                else if constexpr (IV) thL = smallest(lo[0][0], lo[1][0]);
             },
             [&](int n, const Own& o) __attribute__((always_inline)) {
                 const float2 r = ranges[n];
@@ -318,11 +337,14 @@ __global__ void __launch_bounds__(64 * kRtWaves) rt_main_kernel(RtArgs a) {
                 }
             } else {
                 a.outU[o] = fabsf(hi[j][0]);
-                if constexpr (POS) a.pos[o] = idx[j][0] | (hi[j][0] >= 0.f ? 0 : (int)kSign);
+                if constexpr (FORM == kRowsBound) {
+                    a.outL[o] = lo[j][0];
+                    if constexpr (POS) { a.pos[o] = idx[j][0]; a.posL[o] = idxL[j]; }
+                } else if constexpr (POS) a.pos[o] = idx[j][0] | (hi[j][0] >= 0.f ? 0 : (int)kSign);
                 if constexpr (MASKED) {
                     // The bound rests on K inputs that the batch row keeps; a weight row that keeps none of them
                     // may have its maximum at an unmarked input: such an output is recomputed from every input.
-                    if (!(fabsf(hi[j][0]) >= LU)) a.fix[atomicAdd(&a.count->fixes, 1ull)] = (uint32_t)o;
+                    if (!(fabsf(hi[j][0]) >= a.low[(size_t)t * a.Bp + b])) a.fix[atomicAdd(&a.count->fixes, 1ull)] = (uint32_t)o;
                 }
             }
         }
@@ -382,7 +404,7 @@ int launch_rt(const RtArgs& a, hipStream_t st) {
 }
 
 // ranges, transposed weights, tables
-template <bool PAIR, bool MASK>
+template <bool PAIR, bool TWO, bool MASK>
 int run_tables(const float* xl, const float* xu, const float* w, const uint32_t* xkeep, const uint32_t* wkeep, int B, int M,
                int N, int K, const Carve& c, unsigned long long limit, const float* col_stat, const unsigned long long* col_count,
                float ratio, hipStream_t st) {
@@ -391,7 +413,7 @@ int run_tables(const float* xl, const float* xu, const float* w, const uint32_t*
     hipLaunchKernelGGL((rc_range_kernel<MASK>), dim3((N + 63) / 64, T), dim3(256), 0, st, w, wkeep, M, N, S, c.wr, c.wt, c.count, col_stat, ratio);
     if ((rc = check_launch("rc_range_kernel"))) return rc;
     const TableArgs t{PAIR ? xu : xl, xl, xkeep, c.wr, B, bpad_of(B), N, T, K, c.low, c.bits};
-    hipLaunchKernelGGL((rc_tables_kernel<PAIR, MASK>), dim3((B + kTableWaves - 1) / kTableWaves, (T + 3) / 4), dim3(64 * kTableWaves), 0, st,
+    hipLaunchKernelGGL((rc_tables_kernel<PAIR, TWO, MASK>), dim3((B + kTableWaves - 1) / kTableWaves, (T + 3) / 4), dim3(64 * kTableWaves), 0, st,
                        t, c.count, col_count, col_stat, S, limit, ratio);
     return check_launch("rc_tables_kernel");
 }
@@ -400,9 +422,9 @@ template <int FORM, int K>
 int run(const float* xl, const float* xu, const float* w, int B, int M, int N, float q, float* outL, float* outU, int* pos,
         const Carve& c, unsigned long long limit, const float* col_stat, const unsigned long long* col_count, hipStream_t st) {
     constexpr bool IV = FORM == kRowsSortInterval;
-    const int rc = run_tables<IV, false>(xl, xu, w, nullptr, nullptr, B, M, N, K, c, limit, col_stat, col_count, kProbeRatio, st);
+    const int rc = run_tables<IV, false, false>(xl, xu, w, nullptr, nullptr, B, M, N, K, c, limit, col_stat, col_count, kProbeRatio, st);
     if (rc) return rc;
-    RtArgs a{xl, xu, c.wt, c.wr, c.bits, c.low, c.count, c.fix, B, bpad_of(B), M, N, q, outL, outU, pos};
+    RtArgs a{xl, xu, c.wt, c.wr, c.bits, c.low, c.count, c.fix, B, bpad_of(B), M, N, q, outL, outU, pos, nullptr};
     return launch_rt<FORM, K, false, false>(a, st);
 }
 
@@ -410,9 +432,9 @@ template <bool MASKED>
 int run_max(const float* x, const float* w, const uint32_t* xkeep, const uint32_t* wkeep, int B, int M, int N, int K, float* y,
             int* pos, const Carve& c, unsigned long long limit, const float* col_stat, const unsigned long long* col_count,
             float ratio, hipStream_t st) {
-    int rc = run_tables<false, MASKED>(x, nullptr, w, xkeep, wkeep, B, M, N, K, c, limit, col_stat, col_count, ratio, st);
+    int rc = run_tables<false, false, MASKED>(x, nullptr, w, xkeep, wkeep, B, M, N, K, c, limit, col_stat, col_count, ratio, st);
     if (rc) return rc;
-    RtArgs a{x, nullptr, c.wt, c.wr, c.bits, c.low, c.count, c.fix, B, bpad_of(B), M, N, 0.f, nullptr, y, pos};
+    RtArgs a{x, nullptr, c.wt, c.wr, c.bits, c.low, c.count, c.fix, B, bpad_of(B), M, N, 0.f, nullptr, y, pos, nullptr};
     if (pos) rc = launch_rt<kRowsMax, 1, true, MASKED>(a, st);
     else rc = launch_rt<kRowsMax, 1, false, MASKED>(a, st);
     if (rc || !MASKED) return rc;
@@ -420,6 +442,14 @@ int run_max(const float* x, const float* w, const uint32_t* xkeep, const uint32_
     if (pos) hipLaunchKernelGGL((rc_fix_kernel<true>), dim3(256), dim3(256), 0, st, f);
     else hipLaunchKernelGGL((rc_fix_kernel<false>), dim3(256), dim3(256), 0, st, f);
     return check_launch("rc_fix_kernel");
+}
+
+int run_bound(const float* xl, const float* xu, const float* w, int B, int M, int N, float* outL, float* outU, int* posL, int* posU,
+              const Carve& c, unsigned long long limit, const float* col_stat, const unsigned long long* col_count, hipStream_t st) {
+    const int rc = run_tables<true, true, false>(xl, xu, w, nullptr, nullptr, B, M, N, 1, c, limit, col_stat, col_count, kProbeRatio, st);
+    if (rc) return rc;
+    RtArgs a{xl, xu, c.wt, c.wr, c.bits, c.low, c.count, c.fix, B, bpad_of(B), M, N, 0.f, outL, outU, posU, posL};
+    return posU ? launch_rt<kRowsBound, 1, true, false>(a, st) : launch_rt<kRowsBound, 1, false, false>(a, st);
 }
 
 }  // namespace
@@ -434,6 +464,7 @@ bool row_cands_supported(int form, int K) {
         case kRowsSortValues: return K >= 2 && K <= 25;
         case kRowsSortInterval: return K >= 2 && K <= 25;
         case kRowsSortPos: return K >= 2 && K <= 25;
+        case kRowsBound: return K == 1;
         case kRowsMax: return K == 1 || K == 8 || K == 12 || K == 16 || K == 20 || K == 24;
     }
     return false;
@@ -446,7 +477,7 @@ bool row_cands_supported(int form, int K) {
 int row_cands_forward(int form, const float* xl, const float* xu, const float* w, const uint32_t* xkeep,
                       const uint32_t* wkeep, int B, int CO, int CI, float q, int K, float* outL, float* outU, int* pos,
                       void* ws, float density, bool forced, const float* col_stat, const unsigned long long* col_count,
-                      const unsigned long long** every, hipStream_t st) {
+                      const unsigned long long** every, hipStream_t st, int* pos_lower) {
     const float ratio_max = forced ? kProbeRatio : kProbeRatioMax;
     if (CI % kChunk != 0 || B < 1 || CO < 1 || !row_cands_supported(form, K) || (xkeep == nullptr) != (wkeep == nullptr) ||
         (long long)B * CO >= (1ll << 32)) {
@@ -483,6 +514,8 @@ int row_cands_forward(int form, const float* xl, const float* xu, const float* w
 #undef X
             }
             break;
+        case kRowsBound:
+            return run_bound(xl, xu, w, B, CO, CI, outL, outU, pos_lower, pos, c, limit, col_stat, col_count, st);
         case kRowsMax:
             return xkeep ? run_max<true>(xl, w, xkeep, wkeep, B, CO, CI, K, outU, pos, c, limit, col_stat, col_count, ratio_max, st)
                          : run_max<false>(xl, w, nullptr, nullptr, B, CO, CI, K, outU, pos, c, limit, col_stat, col_count, ratio_max, st);

@@ -31,11 +31,11 @@ void note_forward_kernel(const char* kind, int tb, int tm) {
     snprintf(g_fwd_kernel, sizeof(g_fwd_kernel), "%s<%d,%d>", kind, tb, tm);
 }
 
-struct TermNote { const unsigned long long* counts; int kind; double denom0, denom1; unsigned long long limit0; };
-static thread_local TermNote g_term_note = {nullptr, 0, 1.0, 1.0, 0ull};
+struct TermNote { const unsigned long long* counts; int kind; double denom0, denom1; };
+static thread_local TermNote g_term_note = {nullptr, 0, 1.0, 1.0};
 
-void note_term_counts(const unsigned long long* counts, int kind, double denom0, double denom1, unsigned long long limit0) {
-    g_term_note = TermNote{counts, kind, denom0, denom1, limit0};
+void note_term_counts(const unsigned long long* counts, int kind, double denom0, double denom1) {
+    g_term_note = TermNote{counts, kind, denom0, denom1};
 }
 
 // sd_time_forward_kernels / sd_last_forward_kernel_ms: two events per thread, created on first use
@@ -297,9 +297,7 @@ float sd_last_forward_term_share(sd_stream_t stream) {
         return -1.f;
     }
     if (n.kind == 1) return c[1] != 0ull ? 1.f : (float)((double)c[0] / n.denom0);
-    if (n.kind == 3) return c[1] != 0ull ? 1.f : c[2] != 0ull ? (float)((double)c[0] / n.denom0) : (float)((double)c[3] / n.denom1);
-    if (c[2] != 0ull) return 1.f;
-    return c[0] <= n.limit0 ? (float)((double)c[0] / n.denom0) : (float)((double)c[1] / n.denom1);
+    return c[1] != 0ull ? 1.f : c[2] != 0ull ? (float)((double)c[0] / n.denom0) : (float)((double)c[3] / n.denom1);
 }
 
 uint32_t sd_rng_word(uint32_t seed, uint32_t stream_id, uint32_t row, uint32_t col) {

@@ -211,7 +211,7 @@ static int queue_sort_cols(FwdArgs& a, int form, const float* xl, const float* x
     if (rc) return rc;
     a.gate = every;
     a.gate_limit = 0ull;
-    note_term_counts(every - 1, 3, (double)((CO + 127) / 128) * B * CI, (double)((B + 127) / 128) * CO * CI, 0ull);
+    note_term_counts(every - 1, 3, (double)((CO + 127) / 128) * B * CI, (double)((B + 127) / 128) * CO * CI);
     return SD_OK;
 }
 

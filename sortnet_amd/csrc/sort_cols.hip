@@ -587,7 +587,7 @@ int sort_cols_forward(const float* xl, const float* xu, const float* w, int B, i
     const unsigned long long limit = (unsigned long long)((double)tiles_b(B) * CO * CI * d);
     *gate = &c.count->marks;
     *gate_limit = limit;
-    note_term_counts(&c.count->marks, 1, (double)tiles_b(B) * CO * CI, 1.0, 0ull);
+    note_term_counts(&c.count->marks, 1, (double)tiles_b(B) * CO * CI, 1.0);
     if (K == 1 && xu) return run<1, true, true>(xl, xu, w, B, CO, CI, q, outL, outU, nullptr, c, limit, st);
     switch (K) {
 #define X(k) case k: return xu ? run<k, true>(xl, xu, w, B, CO, CI, q, outL, outU, nullptr, c, limit, st) \
@@ -621,7 +621,7 @@ int max_cols_forward(const float* x, const float* w, const uint32_t* xkeep, cons
     const unsigned long long limit = (unsigned long long)((double)tiles_b(B) * CO * CI * d);
     *gate = &c.count->marks;
     *gate_limit = limit;
-    note_term_counts(&c.count->marks, 1, (double)tiles_b(B) * CO * CI, 1.0, 0ull);
+    note_term_counts(&c.count->marks, 1, (double)tiles_b(B) * CO * CI, 1.0);
     if (K < 1 || K > 64 || (!xkeep && K != 1)) { set_error("max_cols_forward: depth %d not supported", K); return SD_ERR_ARG; }
     return xkeep ? run_max<true>(x, w, xkeep, wkeep, B, CO, CI, K, y, pos, c, limit, st)
                  : run_max<false>(x, w, nullptr, nullptr, B, CO, CI, K, y, pos, c, limit, st);
