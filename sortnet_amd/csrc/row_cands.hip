@@ -131,15 +131,17 @@ __global__ void __launch_bounds__(256) rc_range_kernel(const float* __restrict__
     }
 }
 
-// Bounds and marks (cand_tables.h): four tiles of weight rows at a time
-template <bool PAIR, bool TWO, bool MASK>
-__global__ void __launch_bounds__(64 * kTableWaves)
+// Bounds and marks (cand_tables.h); J = 0: rows of any length
+template <int J, int R, int NT, bool PAIR, bool TWO, bool MASK>
+__global__ void __launch_bounds__(64 * (J ? kStreamWaves : kTableWaves))
 rc_tables_kernel(TableArgs a, RowCount* __restrict__ c, const unsigned long long* __restrict__ col_count,
                  const float* __restrict__ stat, int S, unsigned long long limit, float ratio) {
-    __shared__ __attribute__((aligned(16))) float smem[4 * 2 * kTableSlice];
+    extern __shared__ __attribute__((aligned(16))) float smem[];
     unsigned long long marks = ~0ull;
     if (rows_decide(stat, S, ratio)) {
-        const int part = build_tables<1, 4, PAIR, TWO, MASK>(a, blockIdx.x, blockIdx.y, smem);
+        int part;
+        if constexpr (J == 0) part = build_tables<R, NT, PAIR, TWO, MASK>(a, blockIdx.x, blockIdx.y, smem);
+        else part = stream_tables<J, R, NT, PAIR, TWO, MASK>(a, blockIdx.x, gridDim.x, blockIdx.y, smem);
         if (!add_marks(&c->sum, part, &marks)) return;
     } else if (blockIdx.x != 0 || blockIdx.y != 0 || threadIdx.x != 0) return;
     const bool run = marks <= limit;   // (the limit is a share of the (tile, row, input) triples: never all ones)
@@ -294,7 +296,7 @@ __global__ void __launch_bounds__(64 * kRtWaves) rt_main_kernel(RtArgs a) {
     // In kRowsSortPos the strong marks give each row a lower bound of its K-th largest term.  A term below it is never among
     // the K largest, and whether one at or above it enters depends only on entries at least that large, so the walk in input
     // order may leave the others out.
-    for_marks(list, NCH, lane, [&](int c) __attribute__((always_inline)) { return table_word(rowbits, c); },
+    for_marks(list, NCH, lane, [&](int c) __attribute__((always_inline)) { return rowbits[c]; },
               [&](int total, bool first) __attribute__((always_inline)) {
         walk_marks<ORDERED, IV>(list, total, first, lane,
             [&](int n) __attribute__((always_inline)) {
@@ -413,9 +415,31 @@ int run_tables(const float* xl, const float* xu, const float* w, const uint32_t*
     hipLaunchKernelGGL((rc_range_kernel<MASK>), dim3((N + 63) / 64, T), dim3(256), 0, st, w, wkeep, M, N, S, c.wr, c.wt, c.count, col_stat, ratio);
     if ((rc = check_launch("rc_range_kernel"))) return rc;
     const TableArgs t{PAIR ? xu : xl, xl, xkeep, c.wr, B, bpad_of(B), N, T, K, c.low, c.bits};
-    hipLaunchKernelGGL((rc_tables_kernel<PAIR, TWO, MASK>), dim3((B + kTableWaves - 1) / kTableWaves, (T + 3) / 4), dim3(64 * kTableWaves), 0, st,
-                       t, c.count, col_count, col_stat, S, limit, ratio);
-    return check_launch("rc_tables_kernel");
+    auto tables = [&](auto j, auto rows, auto nt) {
+        constexpr int J = decltype(j)::value, R = decltype(rows)::value, NT = decltype(nt)::value;
+        const int groups = (T + NT - 1) / NT;
+        dim3 grid((B + R * kTableWaves - 1) / (R * kTableWaves), groups), block(64 * kTableWaves);
+        size_t lds = (size_t)NT * 2 * kTableSlice * 4;
+        if (J) {
+            const StreamShape s = stream_shape(N, R, B, groups);
+            grid.x = s.rows;
+            block.x = 64 * s.waves;
+            lds = stream_lds(s.waves, R * NT * (TWO ? 2 : 1));
+        }
+        hipLaunchKernelGGL((rc_tables_kernel<J, R, NT, PAIR, TWO, MASK>), grid, block, lds, st, t, c.count, col_count, col_stat, S, limit, ratio);
+        return check_launch("rc_tables_kernel");
+    };
+    using std::integral_constant;
+    constexpr integral_constant<int, 4> four{};
+    constexpr integral_constant<int, 2> two{};
+    constexpr integral_constant<int, 1> one{};
+    // four tiles of weight rows at a time, two where the registers hold no more ranges
+    switch (stream_blocks(N)) {
+        case 1: return tables(one, two, four);
+        case 2: return tables(two, integral_constant<int, PAIR ? 1 : 2>{}, integral_constant<int, MASK ? 3 : 4>{});
+        case 3: return tables(integral_constant<int, 3>{}, one, two);
+    }
+    return tables(integral_constant<int, 0>{}, one, four);
 }
 
 template <int FORM, int K>

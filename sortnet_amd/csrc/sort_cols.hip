@@ -162,35 +162,55 @@ __device__ __forceinline__ bool table_pointless(const float* stat, int S) {
     return stat[0] > kProbeRatio * (float)S * stat[1];
 }
 
-// Bounds and marks (cand_tables.h)
-template <int RW, int NT, bool TWO, bool MASK>
-__global__ void __launch_bounds__(64 * kTableWaves)
+// Bounds and marks (cand_tables.h); J = 0: rows of any length
+template <int J, int R, int NT, bool TWO, bool MASK>
+__global__ void __launch_bounds__(64 * (J ? kStreamWaves : kTableWaves))
 sc_tables_kernel(TableArgs a, TableCount* __restrict__ c, unsigned long long limit) {
-    __shared__ __attribute__((aligned(16))) float smem[NT * (TWO ? 4 : 2) * kTableSlice];
+    extern __shared__ __attribute__((aligned(16))) float smem[];
     if (table_pointless(c->stat, a.tiles)) {
         if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) { c->marks = ~0ull; c->above = 1ull; }
         return;
     }
-    const int marks = build_tables<RW, NT, false, TWO, MASK>(a, blockIdx.x, blockIdx.y, smem);
+    int marks;
+    if constexpr (J == 0) marks = build_tables<R, NT, false, TWO, MASK>(a, blockIdx.x, blockIdx.y, smem);
+    else marks = stream_tables<J, R, NT, false, TWO, MASK>(a, blockIdx.x, gridDim.x, blockIdx.y, smem);
     unsigned long long total;
     if (add_marks(&c->sum, marks, &total)) { c->marks = total; c->above = total > limit ? 1ull : 0ull; }
 }
 
-template <int RW, int NT, bool TWO, bool MASK>
+template <int J, int R, int NT, bool TWO, bool MASK>
 int launch_tables(const TableArgs& t, TableCount* c, unsigned long long limit, hipStream_t st) {
-    const int per = RW * kTableWaves;
-    hipLaunchKernelGGL((sc_tables_kernel<RW, NT, TWO, MASK>), dim3((t.R + per - 1) / per, (t.tiles + NT - 1) / NT), dim3(64 * kTableWaves), 0, st,
-                       t, c, limit);
+    const int groups = (t.tiles + NT - 1) / NT;
+    dim3 grid((t.R + R * kTableWaves - 1) / (R * kTableWaves), groups), block(64 * kTableWaves);
+    size_t lds = (size_t)NT * (TWO ? 4 : 2) * kTableSlice * 4;
+    if (J) {
+        const StreamShape s = stream_shape(t.N, R, t.R, groups);
+        grid.x = s.rows;
+        block.x = 64 * s.waves;
+        lds = stream_lds(s.waves, R * NT * (TWO ? 2 : 1));
+    }
+    hipLaunchKernelGGL((sc_tables_kernel<J, R, NT, TWO, MASK>), grid, block, lds, st, t, c, limit);
     return check_launch("sc_tables_kernel");
 }
-// as many batch tiles at a time as there are, up to four
+// As many batch tiles at a time as there are, up to four, and as the registers hold ranges of (64 per lane).
 template <bool TWO, bool MASK>
 int run_tables(const float* w, const uint32_t* wkeep, int S, int M, int Mp, int N, int K, const Carve& c,
                unsigned long long limit, hipStream_t st) {
     const TableArgs t{w, w, wkeep, c.xr, M, Mp, N, S, K, c.low, c.bits};
-    if (S == 1) return launch_tables<2, 1, TWO, MASK>(t, c.count, limit, st);
-    if (S == 2) return launch_tables<2, 2, TWO, MASK>(t, c.count, limit, st);
-    return launch_tables<1, 4, TWO, MASK>(t, c.count, limit, st);
+    switch (stream_blocks(N)) {
+        case 1:
+            if (S == 1) return launch_tables<1, 4, 1, TWO, MASK>(t, c.count, limit, st);
+            if (S == 2) return launch_tables<1, 2, 2, TWO, MASK>(t, c.count, limit, st);
+            return launch_tables<1, 2, 4, TWO, MASK>(t, c.count, limit, st);
+        case 2:
+            if (S == 1) return launch_tables<2, 2, 1, TWO, MASK>(t, c.count, limit, st);
+            if (TWO || S == 2) return launch_tables<2, TWO ? 1 : 2, 2, TWO, MASK>(t, c.count, limit, st);
+            return launch_tables<2, MASK ? 1 : 2, TWO ? 2 : 4, TWO, MASK>(t, c.count, limit, st);
+        case 3:
+            if (TWO || S == 1) return launch_tables<3, 2, 1, TWO, MASK>(t, c.count, limit, st);
+            return launch_tables<3, 1, TWO ? 1 : 2, TWO, MASK>(t, c.count, limit, st);
+    }
+    return launch_tables<0, 1, 4, TWO, MASK>(t, c.count, limit, st);
 }
 
 // ---- main kernels ------------------------------------------------------------------------------
@@ -291,7 +311,7 @@ sc_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const 
             const int none = 0x7f800000;
             return wave_min_nonneg(__builtin_bit_cast(float, min(in0 ? v0 : none, in1 ? v1 : none)));
         };
-        for_marks(list, NCH, lane, [&](int c) __attribute__((always_inline)) { return table_word(rowbits, c); },
+        for_marks(list, NCH, lane, [&](int c) __attribute__((always_inline)) { return rowbits[c]; },
                   [&](int total, bool first) __attribute__((always_inline)) {
             walk_marks<false, false>(list, total, first, lane,
                 [&](int n) __attribute__((always_inline)) { return Own{wrow[n], 0.f}; },
@@ -385,7 +405,7 @@ mc_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const 
         const uint32_t* __restrict__ rowbits = bits + ((size_t)s * Mp + m) * table_row_words(N);
         for (int pass = 0; pass < 2; pass++) {
             for_marks(list, NCH, lane, [&](int c) __attribute__((always_inline)) {
-                          return pass == 0 ? table_word(rowbits, c) : wkeep ? wkeep[(size_t)m * NCH + c] : ~0u;
+                          return pass == 0 ? rowbits[c] : wkeep ? wkeep[(size_t)m * NCH + c] : ~0u;
                       },
                       [&](int total, bool first) __attribute__((always_inline)) {
                 walk_marks<POS, false>(list, total, first, lane,
@@ -495,7 +515,7 @@ sp_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const 
         // The strong marks give each row a lower bound of its K-th largest term.  A term below it is never among the K
         // largest, and whether one at or above it enters depends only on entries at least that large, so the walk in input
         // order may leave the others out.
-        for_marks(list, NCH, lane, [&](int c) __attribute__((always_inline)) { return table_word(rowbits, c); },
+        for_marks(list, NCH, lane, [&](int c) __attribute__((always_inline)) { return rowbits[c]; },
                   [&](int total, bool first) __attribute__((always_inline)) {
             walk_marks<true, false>(list, total, first, lane,
                 [&](int n) __attribute__((always_inline)) { return Own{wrow[n], 0.f}; },

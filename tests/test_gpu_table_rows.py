@@ -1,0 +1,48 @@
+"""Candidate tables at the lengths of a row where their kernel changes: a wavefront alone, one to three blocks of 256 inputs per
+wavefront (up to 4096, 8192 and 12288 inputs), rows that end inside a block, and longer ones, which are read twice; one to three
+tiles of the other operand.  The table kernels, forced to run, against the kernels that evaluate every term: the same bits."""
+import numpy as np
+import pytest
+import torch
+
+from test_gpu_candidate_random import _data
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("kind", [0, 3])
+@pytest.mark.parametrize("CI", [32, 256, 288, 4064, 4096, 4128, 8192, 8224, 12288, 12320])
+@pytest.mark.parametrize("B,CO", [(5, 130), (129, 3), (257, 258)])
+def test_tables_of_rows_of_any_length(B, CI, CO, kind):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from sortnet_amd import ext, _lib
+    dev = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(B + CI)
+    x, w = _data(np.random.default_rng(CI), B, CI, CO, kind, g, dev)
+    r = torch.rand(B, CI, 1, generator=g).to(dev) * 0.05 - 0.005   # some intervals are inverted
+    xl, xu = (x - r).contiguous(), (x + r).contiguous()
+    K = min(10, CI // 4)
+    results = []
+    try:
+        for density, form in ((0.0, 0), (1.0, 1), (1.0, 2)):
+            _lib.set_sort_candidate_density(density)
+            _lib.set_linf_candidate_density(density)
+            _lib.set_bound_candidate_density(density)
+            _lib.set_bound_candidate_form(form)
+            o = [torch.full((B, CO, 1), float("nan"), device=dev) for _ in range(7)]
+            p = [torch.full((B, CO, 1), -7, device=dev, dtype=torch.int32) for _ in range(2)]
+            ext.sort_neuron_forward_nograd(x, w, o[0], 1, 0.75, K)
+            ext.bound_sort_neuron_forward(xl, xu, w, o[1], o[2], 1, 0.75, K)
+            ext.inf_dist_forward(x, w, o[3], p[0], 1)
+            ext.masked_inf_dist_forward(x, w, o[4], p[1], 1, 0.5, 7, ext.MASK_FACTORED)
+            ext.bound_inf_dist_forward_nograd(xl, xu, w, o[5], o[6], 1)
+            results.append(o + p)
+    finally:
+        _lib.set_sort_candidate_density(-1.0)
+        _lib.set_linf_candidate_density(-1.0)
+        _lib.set_bound_candidate_density(-1.0)
+        _lib.set_bound_candidate_form(0)
+    for tables in results[1:]:
+        for i, (a, b) in enumerate(zip(results[0], tables)):
+            assert torch.equal(a, b), i
