@@ -44,14 +44,15 @@ __device__ __forceinline__ int wave_prefix_sum(int v) {
 
 // Lists the marked inputs of a row in ascending order and hands them over, as many at a time as the list holds: at least
 // once, also when there are none.  word(c): table word of inputs 32 c .. 32 c + 31, for c < NCH.  use(count, first): walks
-// the list.
+// the list.  ready: the number of marks when they are all listed already (of a list that was handed over whole).
+// Returns the number of marks when they were handed over whole, otherwise -1.
 template <class Word, class Use>
-__device__ __forceinline__ void for_marks(uint16_t* list, int NCH, int lane, Word&& word, Use&& use) {
-    int c0 = 0;
-    uint32_t next = lane < NCH ? word(lane) : 0u;
+__device__ __forceinline__ int for_marks(uint16_t* list, int NCH, int lane, Word&& word, Use&& use, int ready = -1) {
+    int c0 = ready >= 0 ? NCH : 0;
+    uint32_t next = ready < 0 && lane < NCH ? word(lane) : 0u;
     bool first = true;
     while (true) {
-        int cnt = 0;
+        int cnt = ready >= 0 ? ready : 0;
         while (c0 < NCH) {
             uint32_t bits = next;
             const int mine = __builtin_popcount(bits), incl = wave_prefix_sum(mine);
@@ -71,8 +72,8 @@ __device__ __forceinline__ void for_marks(uint16_t* list, int NCH, int lane, Wor
         __builtin_amdgcn_wave_barrier();
         use(cnt, first);
         __builtin_amdgcn_wave_barrier();   // the reads of the list come before the next marks
+        if (c0 >= NCH) return first ? cnt : -1;
         first = false;
-        if (c0 >= NCH) return;
     }
 }
 

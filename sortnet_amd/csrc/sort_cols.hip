@@ -463,22 +463,29 @@ __device__ __forceinline__ void static_for(F&& f, std::integer_sequence<int, R..
     (f(std::integral_constant<int, R>{}), ...);
 }
 
-// Value form with positions (core/cuda/sort_neuron.cu:111-214): as sc_main_kernel, with the ordered insertion that
-// carries the input numbers.  The marks of a row are walked in ascending input order, and every term that is at
-// least the final K-th largest value of an output is marked, so these terms meet the list in the order and against
-// the entries they meet in the scan over all inputs: same values and same positions, ties included.  pos is
-// (K, B, M) with slot 0 = largest; the K planes leave through LDS one after the other.
+// Value form with positions (core/cuda/sort_neuron.cu:111-214), in two walks.  The first is that of sc_main_kernel and gives
+// each output its K-th largest term.  A smaller term is never among the K largest, and whether one at or above it enters depends
+// only on entries at least that large; so the second walk, in ascending input order, takes the terms that reach it, K and
+// their ties per output, and only these meet the ordered insertion that carries the input numbers: same values and positions
+// as the scan over all inputs, ties included.  They differ from lane to lane, so the second walk only notes their inputs in
+// LDS, and the lists are formed at the end, all lanes at work (an insertion at every mark that any of 128 outputs takes is four
+// times the instructions of the value alone).  Outputs with more than two ties too many: their row is walked with an
+// insertion at every mark.
+// pos is (K, B, M) with slot 0 = largest; the K planes leave through LDS one after the other.
+// 128 x 5120 x 5120, K = 10, 12 % marked: 168 us, 234 with the insertion at every mark.
 template <int K>
 __global__ void __launch_bounds__(64 * kMainWaves)
 sp_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const uint32_t* __restrict__ bits,
                const float* __restrict__ xr, const unsigned long long* __restrict__ count, unsigned long long limit, int B,
                int Bp, int M, int Mp, int N, float q, float* __restrict__ y, int* __restrict__ pos) {
     if (gate_closed(count, limit, 0)) return;
+    constexpr int kSlots = K + 2;
     union Shared {
         uint16_t list[kMainWaves][kWalkListCap];
         int stage[kTileB][kMainTile + 1];
     };
     __shared__ Shared sh;
+    __shared__ uint16_t noted[kMainWaves][kSlots][kTileB];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int MB = Mp / kMainTile, NCH = N / kChunk, item = main_item();
@@ -494,47 +501,79 @@ sp_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const 
         const Caps<false> caps{xr + (size_t)s * N * 2};
         const bool in0 = s * kTileB + lane < B, in1 = s * kTileB + lane + 64 < B;   // the lane's batch rows exist
         uint16_t* list = sh.list[wave];
-        float least[2] = {0.f, 0.f};   // lower bounds of the K-th largest terms of the lane's rows
         float xa[2][4], xb[2][4];
         auto load = [&](int buf, int i, int n) __attribute__((always_inline)) {
             xa[buf][i] = xcol[(size_t)n * Bp];
             xb[buf][i] = xcol[(size_t)n * Bp + 64];
         };
-        auto value = [&](int buf, int i, int k, int, const Own& o) __attribute__((always_inline)) {
+        auto word = [&](int c) __attribute__((always_inline)) { return rowbits[c]; };
+        auto own = [&](int n) __attribute__((always_inline)) { return Own{wrow[n], 0.f}; };
+        auto cap = [&](int n, const Own& o) __attribute__((always_inline)) { return caps(n, o.a).x; };
+        float th = 0.f;   // smallest K-th largest term over the tile's rows so far (rows past the last one do not count)
+        auto keep = [&](int n, const Own& o) __attribute__((always_inline)) { return !(caps(n, o.a).x < th); };
+        float least[2];
+        int listed;
+        {
+            int top[2][K];
+            #pragma unroll
+            for (int k = 0; k < K; k++) top[0][k] = top[1][k] = 0;
+            auto value = [&](int buf, int i, int k, int, const Own& o) __attribute__((always_inline)) {
+                const float wi = lane_value(o.a, k);   // (the maximum with -1: see sc_main_kernel)
+                insert_pair<K>(top[0], fmaxf(fabsf(xa[buf][i] - wi), -1.f), top[1], fmaxf(fabsf(xb[buf][i] - wi), -1.f));
+            };
+            auto smallest = [&]() __attribute__((always_inline)) {
+                const int none = 0x7f800000;
+                th = wave_min_nonneg(__builtin_bit_cast(float, min(in0 ? top[0][0] : none, in1 ? top[1][0] : none)));
+            };
+            listed = for_marks(list, NCH, lane, word, [&](int total, bool first) __attribute__((always_inline)) {
+                walk_marks<false, false>(list, total, first, lane, own, cap, load, value, value,
+                                         [&](bool) __attribute__((always_inline)) { smallest(); }, keep, [] {});
+            });
+            smallest();
+            // only a positive term counts
+            #pragma unroll
+            for (int j = 0; j < 2; j++) least[j] = __builtin_bit_cast(float, max(top[j][0], 1));
+        }
+        int cnt[2] = {0, 0};
+        auto note = [&](int buf, int i, int k, int n, const Own& o) __attribute__((always_inline)) {
             const float wi = lane_value(o.a, k);
-            topk_insert_values<K>(res[0], fabsf(xa[buf][i] - wi));
-            topk_insert_values<K>(res[1], fabsf(xb[buf][i] - wi));
+            if (fabsf(xa[buf][i] - wi) >= least[0]) { noted[wave][min(cnt[0], kSlots - 1)][lane] = (uint16_t)n; cnt[0]++; }
+            if (fabsf(xb[buf][i] - wi) >= least[1]) { noted[wave][min(cnt[1], kSlots - 1)][lane + 64] = (uint16_t)n; cnt[1]++; }
         };
-        auto ordered = [&](int buf, int i, int k, int n, const Own& o) __attribute__((always_inline)) {
-            const float wi = lane_value(o.a, k);
-            const float d0 = xa[buf][i] - wi, d1 = xb[buf][i] - wi;
-            if (fabsf(d0) > res[0][0] && fabsf(d0) >= least[0]) topk_insert<K>(res[0], idx[0], fabsf(d0), n | (d0 >= 0.f ? 0 : (int)kSign));
-            if (fabsf(d1) > res[1][0] && fabsf(d1) >= least[1]) topk_insert<K>(res[1], idx[1], fabsf(d1), n | (d1 >= 0.f ? 0 : (int)kSign));
+        for_marks(list, NCH, lane, word, [&](int total, bool) __attribute__((always_inline)) {
+            walk_marks<true, false>(list, total, false, lane, own, cap, load, note, note, [](bool) {}, keep, [] {});
+        }, listed);
+        auto enter = [&](int j, float d, int n) __attribute__((always_inline)) {
+            if (fabsf(d) > res[j][0] && fabsf(d) >= least[j]) topk_insert<K>(res[j], idx[j], fabsf(d), n | (d >= 0.f ? 0 : (int)kSign));
         };
-        float th = 0.f;   // smallest of them, or of the K-th largest so far, over the tile's rows
-        // The strong marks give each row a lower bound of its K-th largest term.  A term below it is never among the K
-        // largest, and whether one at or above it enters depends only on entries at least that large, so the walk in input
-        // order may leave the others out.
-        for_marks(list, NCH, lane, [&](int c) __attribute__((always_inline)) { return rowbits[c]; },
-                  [&](int total, bool first) __attribute__((always_inline)) {
-            walk_marks<true, false>(list, total, first, lane,
-                [&](int n) __attribute__((always_inline)) { return Own{wrow[n], 0.f}; },
-                [&](int n, const Own& o) __attribute__((always_inline)) { return caps(n, o.a).x; },
-                load, value, ordered,
-                [&](bool strong) __attribute__((always_inline)) {
-                    if (strong) { least[0] = res[0][0]; least[1] = res[1][0]; }
-                    th = wave_min_nonneg(fminf(in0 ? fmaxf(least[0], res[0][0]) : __builtin_inff(),
-                                               in1 ? fmaxf(least[1], res[1][0]) : __builtin_inff()));
-                },
-                [&](int n, const Own& o) __attribute__((always_inline)) { return !(caps(n, o.a).x < th); },
-                [&]() __attribute__((always_inline)) {
-                    #pragma unroll
-                    for (int j = 0; j < 2; j++) {
-                        #pragma unroll
-                        for (int k = 0; k < K; k++) res[j][k] = 0.f;
-                    }
-                });
-        });
+        __builtin_amdgcn_wave_barrier();
+        if (__builtin_amdgcn_ballot_w64(max(cnt[0], cnt[1]) > kSlots) == 0ull) {
+            float d[2][2];
+            int n[2][2];
+            auto fetch = [&](int e) __attribute__((always_inline)) {
+                #pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    n[e & 1][j] = e < cnt[j] ? (int)noted[wave][e][lane + 64 * j] : 0;
+                    d[e & 1][j] = xcol[(size_t)n[e & 1][j] * Bp + 64 * j] - wrow[n[e & 1][j]];
+                }
+            };
+            fetch(0);
+            #pragma unroll
+            for (int e = 0; e < kSlots; e++) {
+                if (e + 1 < kSlots) fetch(e + 1);
+                #pragma unroll
+                for (int j = 0; j < 2; j++) if (e < cnt[j]) enter(j, d[e & 1][j], n[e & 1][j]);
+            }
+        } else {
+            auto ordered = [&](int buf, int i, int k, int n, const Own& o) __attribute__((always_inline)) {
+                const float wi = lane_value(o.a, k);
+                enter(0, xa[buf][i] - wi, n);
+                enter(1, xb[buf][i] - wi, n);
+            };
+            for_marks(list, NCH, lane, word, [&](int total, bool) __attribute__((always_inline)) {
+                walk_marks<true, false>(list, total, false, lane, own, cap, load, ordered, ordered, [](bool) {}, keep, [] {});
+            }, listed);
+        }
     }
     __syncthreads();
     const size_t plane = (size_t)B * M;

@@ -46,3 +46,32 @@ def test_tables_of_rows_of_any_length(B, CI, CO, kind):
     for tables in results[1:]:
         for i, (a, b) in enumerate(zip(results[0], tables)):
             assert torch.equal(a, b), i
+
+
+@pytest.mark.parametrize("equal", [0, 2, 3, 40])   # ties of the K-th largest term: none, as many as are noted, one more, many
+@pytest.mark.parametrize("B,CI,CO,K", [(130, 320, 9, 10), (128, 2144, 5, 2), (5, 4128, 3, 25)])
+def test_positions_with_ties_of_the_smallest_entry(B, CI, CO, K, equal):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from sortnet_amd import ext, _lib
+    dev = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(CI + equal)
+    w = torch.randn(CO, CI, generator=g)
+    x = torch.zeros(B, CI, 1)
+    # row 0 holds K - 1 distinct large terms and 1 + equal terms of one value against every weight row
+    for m in range(CO):
+        at = torch.randperm(CI, generator=g)[:K + equal]
+        w[m, at[:K - 1]] = 8 + torch.arange(K - 1) * 0.25
+        w[m, at[K - 1:]] = -6.0
+    x, w = x.to(dev), w.to(dev)
+    results = []
+    try:
+        for density in (0.0, 1.0):
+            _lib.set_sort_candidate_density(density)
+            y = torch.full((B, CO, 1), float("nan"), device=dev)
+            pos = torch.full((K, B, CO, 1), -7, device=dev, dtype=torch.int32)
+            ext.sort_neuron_forward(x, w, y, pos, 1, 0.75, K)
+            results.append((y, pos))
+    finally:
+        _lib.set_sort_candidate_density(-1.0)
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
