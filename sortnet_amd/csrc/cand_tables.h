@@ -499,7 +499,7 @@ __device__ __forceinline__ bool add_marks(unsigned long long* sum, int marks, un
     return all >> 40 == (unsigned long long)gridDim.x * gridDim.y * gridDim.z;
 }
 
-// What a table per weight row leaves for the choice of kernel.  All zero before the ranges are taken.
+// What a table per weight row leaves for the choice of kernel.
 struct TableCount {
     unsigned long long marks;       // all ones when the table was not built
     unsigned long long above;       // 1 when the marks are above the limit

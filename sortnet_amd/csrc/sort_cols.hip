@@ -25,22 +25,24 @@ struct Carve {
     float* xT;        // [N][Bp] the inputs transposed ((l, u) pairs in the interval form), intervals repaired
     float* low;       // [S][2][Mp] lower bounds of the K-th largest terms of a weight row (K = 1 in the interval form: for either bound)
     uint32_t* bits;   // [S][Mp][table_row_words] the marks
+    float2* widths;   // [S][N / 32] what the probe adds up, see sc_range_kernel
 };
 
-size_t carve_sizes(int B, int M, int N, size_t (&sz)[5]) {
+size_t carve_sizes(int B, int M, int N, size_t (&sz)[6]) {
     const size_t S = tiles_b(B), Bp = S * kTileB, Mp = mpad_of(M);
     sz[0] = 256;
     sz[1] = align256(S * N * 16);
     sz[2] = align256((size_t)N * Bp * 8);
     sz[3] = align256(S * 2 * Mp * 4);
     sz[4] = align256(S * Mp * table_row_words(N) * 4);
+    sz[5] = align256(S * (N / kChunk) * 8);
     size_t t = 0;
     for (size_t v : sz) t += v;
     return t;
 }
 
 Carve carve(void* ws, int B, int M, int N) {
-    size_t sz[5];
+    size_t sz[6];
     carve_sizes(B, M, N, sz);
     char* p = static_cast<char*>(ws);
     Carve c;
@@ -48,7 +50,8 @@ Carve carve(void* ws, int B, int M, int N) {
     c.xr = reinterpret_cast<float*>(p); p += sz[1];
     c.xT = reinterpret_cast<float*>(p); p += sz[2];
     c.low = reinterpret_cast<float*>(p); p += sz[3];
-    c.bits = reinterpret_cast<uint32_t*>(p);
+    c.bits = reinterpret_cast<uint32_t*>(p); p += sz[4];
+    c.widths = reinterpret_cast<float2*>(p);
     return c;
 }
 
@@ -62,9 +65,9 @@ __device__ __forceinline__ void repair(float& l, float& u) {
 // values per input).  Value form: l = u = x.  A workgroup takes 32 inputs, a work-item 16 of the rows at one of them, all
 // its loads in flight.
 // Also answers whether the table is worth building: it can only prune when the rows of a batch tile are alike
-// compared with the entries of a weight row.  stat[0] collects the widths of the column ranges over all tiles and
-// columns, stat[1] the ranges of the same columns over the first 16 weight rows (added once, by the workgroups of
-// tile 0); see table_pointless().
+// compared with the entries of a weight row.  A workgroup leaves the widths of its columns' ranges and, in tile 0, the
+// ranges of the same columns over the first 16 weight rows; sc_tables_kernel adds them up (the launch that cleared a sum for
+// atomics took 4.7 us, adding up 640 pairs 1).
 // MASKED (value form only): xkeep holds one word per (batch row, 32 inputs); an input a row does not keep takes no
 // part in the ranges and is undefined in the transposed copy, so that its term never wins a comparison.  A column no
 // row of the tile keeps has neither a lower bound nor a candidate.
@@ -73,7 +76,9 @@ template <bool IV, bool TWO, bool MASKED>
 __global__ void __launch_bounds__(256) sc_range_kernel(const float* __restrict__ xl, const float* __restrict__ xu,
                                                        const float* __restrict__ w, const uint32_t* __restrict__ xkeep,
                                                        int B, int M, int N, int Bp, float* __restrict__ xr,
-                                                       float* __restrict__ xT, float* __restrict__ stat) {
+                                                       float* __restrict__ xT, float2* __restrict__ widths,
+                                                       TableCount* __restrict__ count) {
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) count->sum = 0ull;
     static_assert(!(IV && MASKED) && (IV || !TWO), "the factored mask belongs to the value form, two ranges to the interval form");
     constexpr int kCols = kChunk, kGroups = 256 / kCols, kRows = kTileB / kGroups;
     __shared__ float part[kGroups][5][kCols];
@@ -142,10 +147,7 @@ __global__ void __launch_bounds__(256) sc_range_kernel(const float* __restrict__
         if (!(bw < 3.0e38f)) bw = 3.0e38f;   // infinite or undefined widths count as very wide
         #pragma unroll
         for (int o = kCols / 2; o; o >>= 1) { bw += __shfl_xor(bw, o); ww += __shfl_xor(ww, o); }
-        if (nl == 0) {
-            unsafeAtomicAdd(stat, bw);
-            if (s == 0) unsafeAtomicAdd(stat + 1, ww);
-        }
+        if (nl == 0) widths[(size_t)s * gridDim.x + blockIdx.x] = make_float2(bw, ww);
     }
     for (int e = tid; e < kCols * kTileB; e += 256) {
         const int nn = e >> 7, col = e & (kTileB - 1);
@@ -157,17 +159,30 @@ __global__ void __launch_bounds__(256) sc_range_kernel(const float* __restrict__
 
 // The batch rows of a tile differ by more than kProbeRatio times what 16 entries of a weight column do (images
 // against small weights): the table would mark nearly every input, so it is not built and reported as full.
+// stat[0]: widths of the column ranges over all tiles and columns, stat[1]: those of the weights.  Every workgroup adds them
+// up for itself, in the same order; the first leaves them for the tables per batch row.
 constexpr float kProbeRatio = 2.5f;
-__device__ __forceinline__ bool table_pointless(const float* stat, int S) {
-    return stat[0] > kProbeRatio * (float)S * stat[1];
+__device__ __forceinline__ bool table_pointless(const float2* __restrict__ widths, int n, int S, float* __restrict__ stat) {
+    __shared__ float2 part[kStreamWaves];
+    float bw = 0.f, ww = 0.f;
+    for (int i = threadIdx.x; i < n; i += (int)blockDim.x) { const float2 v = widths[i]; bw += v.x; ww += v.y; }
+    #pragma unroll
+    for (int o = 32; o; o >>= 1) { bw += __shfl_xor(bw, o); ww += __shfl_xor(ww, o); }
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = make_float2(bw, ww);
+    __syncthreads();
+    bw = ww = 0.f;
+    for (int i = 0; i < (int)(blockDim.x >> 6); i++) { bw += part[i].x; ww += part[i].y; }
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) { stat[0] = bw; stat[1] = ww; }
+    // (wave-uniform: a scalar comparison, so that no lane mask is held)
+    return __builtin_amdgcn_readfirstlane(bw > kProbeRatio * (float)S * ww ? 1 : 0) != 0;
 }
 
 // Bounds and marks (cand_tables.h); J = 0: rows of any length
 template <int J, int R, int NT, bool TWO, bool MASK>
 __global__ void __launch_bounds__(64 * (J ? kStreamWaves : kTableWaves))
-sc_tables_kernel(TableArgs a, TableCount* __restrict__ c, unsigned long long limit) {
+sc_tables_kernel(TableArgs a, const float2* __restrict__ widths, TableCount* __restrict__ c, unsigned long long limit) {
     extern __shared__ __attribute__((aligned(16))) float smem[];
-    if (table_pointless(c->stat, a.tiles)) {
+    if (table_pointless(widths, a.tiles * (a.N / kChunk), a.tiles, c->stat)) {
         if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) { c->marks = ~0ull; c->above = 1ull; }
         return;
     }
@@ -179,7 +194,7 @@ sc_tables_kernel(TableArgs a, TableCount* __restrict__ c, unsigned long long lim
 }
 
 template <int J, int R, int NT, bool TWO, bool MASK>
-int launch_tables(const TableArgs& t, TableCount* c, unsigned long long limit, hipStream_t st) {
+int launch_tables(const TableArgs& t, const Carve& c, unsigned long long limit, hipStream_t st) {
     const int groups = (t.tiles + NT - 1) / NT;
     dim3 grid((t.R + R * kTableWaves - 1) / (R * kTableWaves), groups), block(64 * kTableWaves);
     size_t lds = (size_t)NT * (TWO ? 4 : 2) * kTableSlice * 4;
@@ -189,7 +204,7 @@ int launch_tables(const TableArgs& t, TableCount* c, unsigned long long limit, h
         block.x = 64 * s.waves;
         lds = stream_lds(s.waves, R * NT * (TWO ? 2 : 1));
     }
-    hipLaunchKernelGGL((sc_tables_kernel<J, R, NT, TWO, MASK>), grid, block, lds, st, t, c, limit);
+    hipLaunchKernelGGL((sc_tables_kernel<J, R, NT, TWO, MASK>), grid, block, lds, st, t, c.widths, c.count, limit);
     return check_launch("sc_tables_kernel");
 }
 // As many batch tiles at a time as there are, up to four, and as the registers hold ranges of (64 per lane).
@@ -199,18 +214,18 @@ int run_tables(const float* w, const uint32_t* wkeep, int S, int M, int Mp, int 
     const TableArgs t{w, w, wkeep, c.xr, M, Mp, N, S, K, c.low, c.bits};
     switch (stream_blocks(N)) {
         case 1:
-            if (S == 1) return launch_tables<1, 4, 1, TWO, MASK>(t, c.count, limit, st);
-            if (S == 2) return launch_tables<1, 2, 2, TWO, MASK>(t, c.count, limit, st);
-            return launch_tables<1, 2, 4, TWO, MASK>(t, c.count, limit, st);
+            if (S == 1) return launch_tables<1, 4, 1, TWO, MASK>(t, c, limit, st);
+            if (S == 2) return launch_tables<1, 2, 2, TWO, MASK>(t, c, limit, st);
+            return launch_tables<1, 2, 4, TWO, MASK>(t, c, limit, st);
         case 2:
-            if (S == 1) return launch_tables<2, 2, 1, TWO, MASK>(t, c.count, limit, st);
-            if (TWO || S == 2) return launch_tables<2, TWO ? 1 : 2, 2, TWO, MASK>(t, c.count, limit, st);
-            return launch_tables<2, MASK ? 1 : 2, TWO ? 2 : 4, TWO, MASK>(t, c.count, limit, st);
+            if (S == 1) return launch_tables<2, 2, 1, TWO, MASK>(t, c, limit, st);
+            if (TWO || S == 2) return launch_tables<2, TWO ? 1 : 2, 2, TWO, MASK>(t, c, limit, st);
+            return launch_tables<2, MASK ? 1 : 2, TWO ? 2 : 4, TWO, MASK>(t, c, limit, st);
         case 3:
-            if (TWO || S == 1) return launch_tables<3, 2, 1, TWO, MASK>(t, c.count, limit, st);
-            return launch_tables<3, 1, TWO ? 1 : 2, TWO, MASK>(t, c.count, limit, st);
+            if (TWO || S == 1) return launch_tables<3, 2, 1, TWO, MASK>(t, c, limit, st);
+            return launch_tables<3, 1, TWO ? 1 : 2, TWO, MASK>(t, c, limit, st);
     }
-    return launch_tables<0, 1, 4, TWO, MASK>(t, c.count, limit, st);
+    return launch_tables<0, 1, 4, TWO, MASK>(t, c, limit, st);
 }
 
 // ---- main kernels ------------------------------------------------------------------------------
@@ -448,8 +463,7 @@ int run_max(const float* x, const float* w, const uint32_t* xkeep, const uint32_
             int* pos, const Carve& c, unsigned long long limit, hipStream_t st) {
     const int S = tiles_b(B), Bp = S * kTileB, Mp = mpad_of(M);
     int rc;
-    if ((rc = fill_zero(c.count, sizeof(TableCount) / 4, st))) return rc;
-    hipLaunchKernelGGL((sc_range_kernel<false, false, MASK>), dim3(N / kChunk, S), dim3(256), 0, st, x, nullptr, w, xkeep, B, M, N, Bp, c.xr, c.xT, c.count->stat);
+    hipLaunchKernelGGL((sc_range_kernel<false, false, MASK>), dim3(N / kChunk, S), dim3(256), 0, st, x, nullptr, w, xkeep, B, M, N, Bp, c.xr, c.xT, c.widths, c.count);
     if ((rc = check_launch("sc_range_kernel"))) return rc;
     if ((rc = run_tables<false, MASK>(w, wkeep, S, M, Mp, N, K, c, limit, st))) return rc;
     const dim3 grid((unsigned)(S * (Mp / kMainTile)));
@@ -607,8 +621,7 @@ int run(const float* xl, const float* xu, const float* w, int B, int M, int N, f
         int* pos, const Carve& c, unsigned long long limit, hipStream_t st) {
     const int S = tiles_b(B), Bp = S * kTileB, Mp = mpad_of(M);
     int rc;
-    if ((rc = fill_zero(c.count, sizeof(TableCount) / 4, st))) return rc;
-    hipLaunchKernelGGL((sc_range_kernel<IV, MAXFORM, false>), dim3(N / kChunk, S), dim3(256), 0, st, xl, xu, w, nullptr, B, M, N, Bp, c.xr, c.xT, c.count->stat);
+    hipLaunchKernelGGL((sc_range_kernel<IV, MAXFORM, false>), dim3(N / kChunk, S), dim3(256), 0, st, xl, xu, w, nullptr, B, M, N, Bp, c.xr, c.xT, c.widths, c.count);
     if ((rc = check_launch("sc_range_kernel"))) return rc;
     if ((rc = run_tables<MAXFORM, false>(w, nullptr, S, M, Mp, N, K, c, limit, st))) return rc;
     if constexpr (!IV) {
@@ -626,7 +639,7 @@ int run(const float* xl, const float* xu, const float* w, int B, int M, int N, f
 }  // namespace
 
 size_t sort_cols_workspace(int B, int CO, int CI) {
-    size_t sz[5];
+    size_t sz[6];
     return carve_sizes(B, CO, CI, sz);
 }
 
