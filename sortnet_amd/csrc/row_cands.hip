@@ -83,9 +83,10 @@ __device__ __forceinline__ bool rows_decide(const float* stat, int S, float rati
 // that no row keeps, or that holds an undefined or infinite weight, becomes (-inf, +inf): no lower bound, always a
 // candidate), and the transposed copy of the tile.  64 inputs x 4 groups of 32 rows per workgroup.
 // Under the mask a lane fetches the keep bits of one of the wavefront's rows, 64 inputs wide, and hands them to the others:
-// 67 us at 5120 x 5120, 92 with a word fetched per row and lane.
+// 59 us at 5120 x 5120 (92 with a word fetched per row and lane), held to 64 registers: with the 104 it takes otherwise half the
+// wavefronts are in flight, 66 us.
 template <bool WMASK>
-__global__ void __launch_bounds__(256) rc_range_kernel(const float* __restrict__ w, const uint32_t* __restrict__ wkeep,
+__global__ void __launch_bounds__(256, WMASK ? 8 : 1) rc_range_kernel(const float* __restrict__ w, const uint32_t* __restrict__ wkeep,
                                                        int M, int N, int S, float* __restrict__ wr, float* __restrict__ wt,
                                                        RowCount* __restrict__ count, const float* __restrict__ stat, float ratio) {
     if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) count->sum = count->fixes = 0ull;
