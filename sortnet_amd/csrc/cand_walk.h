@@ -108,15 +108,18 @@ __device__ __forceinline__ void walk_block(int n, const Own& o, int cnt, Load&& 
     }
 }
 
-// Walks the listed marks of a row (`total` of them).  Of a long list the first 128 form 32 groups (positions equal modulo
-// 32), whose strongest (`excess`, the larger the stronger) are walked first.  Then the list goes by 64 marks at a time, and
+// Walks the listed marks of a row (`total` of them).  Of a long list the first SAMPLE form 32 groups (positions equal modulo
+// 32), whose strongest (`excess`, the larger the stronger) are walked first.  Against tiles of batch rows 640 (two gathers per 64
+// marks that cost little: positions at 128 x 5120 x 5120, 605 marks, 168 us with 128, 160 with 256, 149; interval bounds of 256 x
+// 10240 x 10240 243 -> 235), against tiles of weight rows 128 (their rows come from beyond the die's cache: 256 x 12288 x
+// 10240 438 us, 481 with 256, 590).  Then the list goes by 64 marks at a time, and
 // of these only those are walked that keep() says can matter now.
 //   own(input) -> Own: a gather;  load / use: see walk_block;
 //   threshold(strong): brings what keep() compares with up to date, after the strong marks and after every 64;
 //   ORDERED: forms for which the order of the inputs counts.  The strong marks are then walked for their values alone, by
 //   value(): restart() clears the state behind them, and they go by again with the others, in order.  Only at the first
 //   call for a row (`first`): later parts of a long list are cut by what the row has reached.
-template <bool ORDERED, bool PAIR, class OwnOf, class Excess, class Load, class Value, class Use, class Threshold, class Keep, class Restart>
+template <bool ORDERED, bool PAIR, int SAMPLE, class OwnOf, class Excess, class Load, class Value, class Use, class Threshold, class Keep, class Restart>
 __device__ __forceinline__ void walk_marks(const uint16_t* list, int total, bool first, int lane, OwnOf&& own, Excess&& excess,
                                            Load&& load, Value&& value, Use&& use, Threshold&& threshold, Keep&& keep,
                                            Restart&& restart) {
@@ -132,6 +135,12 @@ __device__ __forceinline__ void walk_marks(const uint16_t* list, int total, bool
         const float x1 = excess(n1, o1);
         won = lane;
         if (x1 > x && 64 + lane < total) { x = x1; n = n1; o = o1; won = e1; }
+        for (int e0 = 128; e0 < (total < SAMPLE ? total : SAMPLE); e0 += 64) {
+            const int e2 = e0 + lane < total ? e0 + lane : total - 1, n2 = (int)list[e2];
+            const Own o2 = own(n2);
+            const float x2 = excess(n2, o2);
+            if (x2 > x && e0 + lane < total) { x = x2; n = n2; o = o2; won = e2; }
+        }
         // the two lanes of a group agree on the stronger of their marks
         const float ox = __shfl_xor(x, 32);
         const int on = __shfl_xor(n, 32), ow = __shfl_xor(won, 32);

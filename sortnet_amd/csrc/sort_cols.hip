@@ -15,6 +15,7 @@ constexpr int kTileB = 128;          // batch rows of a tile: 64 lanes x 2
 constexpr int kRowPad = 128;         // weight rows are padded to a multiple of this in the tables
 constexpr int kMainWaves = 4;        // wavefronts of a workgroup of the main kernels
 constexpr int kMainTile = kMainWaves;   // weight rows of a workgroup, one per wavefront
+constexpr int kSample = 640;         // see walk_marks
 
 inline size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 inline int tiles_b(int B) { return (B + kTileB - 1) / kTileB; }
@@ -328,7 +329,7 @@ sc_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const 
         };
         for_marks(list, NCH, lane, [&](int c) __attribute__((always_inline)) { return rowbits[c]; },
                   [&](int total, bool first) __attribute__((always_inline)) {
-            walk_marks<false, false>(list, total, first, lane,
+            walk_marks<false, false, kSample>(list, total, first, lane,
                 [&](int n) __attribute__((always_inline)) { return Own{wrow[n], 0.f}; },
                 [&](int n, const Own& o) __attribute__((always_inline)) { const float2 v = caps(n, o.a); return fmaxf(v.x - LU, v.y - LL); },
                 load, use, use,
@@ -423,7 +424,7 @@ mc_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const 
                           return pass == 0 ? rowbits[c] : wkeep ? wkeep[(size_t)m * NCH + c] : ~0u;
                       },
                       [&](int total, bool first) __attribute__((always_inline)) {
-                walk_marks<POS, false>(list, total, first, lane,
+                walk_marks<POS, false, kSample>(list, total, first, lane,
                     [&](int n) __attribute__((always_inline)) { return Own{wrow[n], 0.f}; },
                     [&](int n, const Own& o) __attribute__((always_inline)) { return caps(n, o.a).x; },
                     load, use, use,
@@ -486,7 +487,7 @@ __device__ __forceinline__ void static_for(F&& f, std::integer_sequence<int, R..
 // times the instructions of the value alone).  Outputs with more than two ties too many: their row is walked with an
 // insertion at every mark.
 // pos is (K, B, M) with slot 0 = largest; the K planes leave through LDS one after the other.
-// 128 x 5120 x 5120, K = 10, 12 % marked: 168 us, 234 with the insertion at every mark.
+// 128 x 5120 x 5120, K = 10, 12 % marked: 149 us, 234 with the insertion at every mark.
 template <int K>
 __global__ void __launch_bounds__(64 * kMainWaves)
 sp_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const uint32_t* __restrict__ bits,
@@ -540,7 +541,7 @@ sp_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const 
                 th = wave_min_nonneg(__builtin_bit_cast(float, min(in0 ? top[0][0] : none, in1 ? top[1][0] : none)));
             };
             listed = for_marks(list, NCH, lane, word, [&](int total, bool first) __attribute__((always_inline)) {
-                walk_marks<false, false>(list, total, first, lane, own, cap, load, value, value,
+                walk_marks<false, false, kSample>(list, total, first, lane, own, cap, load, value, value,
                                          [&](bool) __attribute__((always_inline)) { smallest(); }, keep, [] {});
             });
             smallest();
@@ -555,7 +556,7 @@ sp_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const 
             if (fabsf(xb[buf][i] - wi) >= least[1]) { noted[wave][min(cnt[1], kSlots - 1)][lane + 64] = (uint16_t)n; cnt[1]++; }
         };
         for_marks(list, NCH, lane, word, [&](int total, bool) __attribute__((always_inline)) {
-            walk_marks<true, false>(list, total, false, lane, own, cap, load, note, note, [](bool) {}, keep, [] {});
+            walk_marks<true, false, kSample>(list, total, false, lane, own, cap, load, note, note, [](bool) {}, keep, [] {});
         }, listed);
         auto enter = [&](int j, float d, int n) __attribute__((always_inline)) {
             if (fabsf(d) > res[j][0] && fabsf(d) >= least[j]) topk_insert<K>(res[j], idx[j], fabsf(d), n | (d >= 0.f ? 0 : (int)kSign));
@@ -585,7 +586,7 @@ sp_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const 
                 enter(1, xb[buf][i] - wi, n);
             };
             for_marks(list, NCH, lane, word, [&](int total, bool) __attribute__((always_inline)) {
-                walk_marks<true, false>(list, total, false, lane, own, cap, load, ordered, ordered, [](bool) {}, keep, [] {});
+                walk_marks<true, false, kSample>(list, total, false, lane, own, cap, load, ordered, ordered, [](bool) {}, keep, [] {});
             }, listed);
         }
     }
