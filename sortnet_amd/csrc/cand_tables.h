@@ -57,6 +57,15 @@ __device__ __forceinline__ uint32_t exchange_marks(uint32_t x, int lane) {
 // what marks are compared with: a term only counts when it is positive, and the difference from the bound is to be defined
 __device__ __forceinline__ float mark_bound(float kth) { return fminf(kth > 0.f ? kth : 1.401298464e-45f, 3.402823466e38f); }
 
+// An inverted interval becomes its midpoint.  One bound for both results (TWO = false) rests on the term of the upper one being at
+// least that of the lower one, which does not hold where an end is undefined (each result then takes the term of the other end):
+// such an input is given no bound and is always marked.
+template <bool TWO>
+__device__ __forceinline__ void repair_row(float& l, float& u) {
+    if (l > u) l = u = (l + u) * 0.5f;
+    if constexpr (!TWO) { if (!(l <= u)) { l = -__builtin_inff(); u = __builtin_inff(); } }
+}
+
 // largest value over the wavefront of floats that are not negative
 __device__ __forceinline__ float wave_max_nonneg(float f) {
     int v = __builtin_bit_cast(int, f);
@@ -144,7 +153,7 @@ __device__ __forceinline__ int build_tables(const TableArgs& a, int bx, int by, 
         }
         #pragma unroll
         for (int e = 0; e < 4; e++) {
-            if constexpr (PAIR) { if (vl[e] > vu[e]) vl[e] = vu[e] = (vl[e] + vu[e]) * 0.5f; }   // inverted interval: midpoint
+            if constexpr (PAIR) repair_row<TWO>(vl[e], vu[e]);
             if constexpr (MASK) {   // undefined where the row does not keep the input
                 const bool k = (kw[r][b] >> e) & 1u;
                 vu[e] = k ? vu[e] : __builtin_nanf("");
@@ -364,9 +373,7 @@ __device__ __forceinline__ int stream_tables(const TableArgs& a, int bx, int nbx
                 }
                 #pragma unroll
                 for (int e = 0; e < 4; e++) {
-                    if constexpr (PAIR) {   // inverted interval: midpoint
-                        if (vl[r][j][e] > vu[r][j][e]) vl[r][j][e] = vu[r][j][e] = (vl[r][j][e] + vu[r][j][e]) * 0.5f;
-                    }
+                    if constexpr (PAIR) repair_row<TWO>(vl[r][j][e], vu[r][j][e]);
                     if constexpr (MASK) {   // undefined where the row does not keep the input
                         const bool k = (kw[r][j] >> ((at[j] & 31) + e)) & 1u;
                         vu[r][j][e] = k ? vu[r][j][e] : __builtin_nanf("");
