@@ -26,7 +26,13 @@ from . import ext
 from . import functional as F
 
 SUB_BATCH = 32   # samples that share one index list (core/cuda/inf_dist_cuda.cu:8)
-SMALL_DRAW = 1 << 15   # channels over all lists of a draw below which the layer is paced by the host: 256 samples x 1024 channels are 8192
+# Terms (rows x kept channels squared, a hidden layer) below which the host paces a training pass, for the l-inf distance, whole
+# powers up to 8 and other powers: there a draw on a second stream is about 50 us of the host's time, above it hides 2 to 6 us of
+# the device's.  Training passes of the zoo (batch x width), us, lists drawn on the second stream / on the caller's:
+#   p = inf  256 x 2048 (6.0e8) 691 / 547, 512 x 2048 (1.2e9) 972 / 980, 128 x 5120 (1.9e9) 735 / 686, 256 x 5120 (3.8e9) 1059 / 1059
+#   p = 8    256 x 1024 (1.5e8) 907 / 751, 96 x 2048 (2.3e8) 783 / 701, 128 x 2048 (3.0e8) 773 / 793, 256 x 2048 (6.0e8) 1196 / 1216
+#   p = 24   64 x 1024 (3.8e7) 785 / 548, 128 x 1024 (7.6e7) 793 / 710, 192 x 1024 (1.1e8) 854 / 865, 128 x 2048 (3.0e8) 1249 / 1263
+HOST_PACED_TERMS = (1 << 31, 1 << 28, 3 << 25)
 
 
 def apply_if_not_none(paras, func):
@@ -51,17 +57,17 @@ class DropoutRegistry:
         self.next_tag += 1
         return self.next_tag
 
-    def sample(self, sub_batches, groups, channels, q, device):
+    def sample(self, sub_batches, groups, channels, q, device, host_paced=False):
         """Ascending kept-channel lists (sub_batches, groups, count), count ~ Binomial(channels, q).
-        The lists depend on nothing but the seed, and the sampler keeps only a few compute units busy, so for a
-        large layer it is queued on a second stream (default priority) and overlaps the kernels already queued on
-        the caller's stream; the caller's stream waits for it before going on.  A small layer is paced by the host,
-        for which the second stream is 50 us of events, so its lists are drawn on the caller's stream (11 us)."""
+        The lists depend on nothing but the seed, and the sampler keeps only a few compute units busy, so it
+        is queued on a second stream (default priority) and overlaps the kernels already queued on the
+        caller's stream; the caller's stream waits for it before going on.  With host_paced (the device would be idle
+        meanwhile) the lists are drawn on the caller's stream, which spares the host the second one's events."""
         self.draws += 1
         seed = (self.seed * 1000003 + self.draws) & 0xFFFFFFFF
         count = ext.mask_count(seed, channels, q)
         device = torch.device(device)
-        if device.type == "cuda" and sub_batches * groups * channels < SMALL_DRAW:
+        if device.type == "cuda" and host_paced:
             return ext.host().sample_index_lists(seed, sub_batches, groups, channels, count, device)
         if device.type != "cuda" or not self.overlap_sampler:
             return ext.sample_index_lists(seed, sub_batches, groups, channels, count, device)
@@ -195,6 +201,10 @@ class NormDistBase(nn.Module):
         sub_batches = (x.size(0) - 1) // SUB_BATCH + 1
         dim_out = self.weight.size(0) // self.groups
 
+        def host_paced(kept):
+            terms = x.size(0) * x.size(-1) * self.groups * kept * kept
+            return terms < HOST_PACED_TERMS[0 if math.isinf(self.p) else 1 if self.p <= 8 and self.p == int(self.p) else 2]
+
         def rows():      # sub-batch of every sample
             return torch.div(torch.arange(x.size(0), device=dev), SUB_BATCH, rounding_mode="trunc")
 
@@ -204,14 +214,14 @@ class NormDistBase(nn.Module):
             if reg.buffer is not None and reg.buffer[0] == self.tag:
                 index_in = reg.buffer[1]          # the predecessor already produced compacted outputs
             else:
-                index_in = reg.sample(sub_batches, self.groups, dim_in, q, dev)
+                index_in = reg.sample(sub_batches, self.groups, dim_in, q, dev, host_paced(dim_in * q))
                 xg = x.view(x.size(0), self.groups, -1, x.size(-1))
                 gather = index_in[rows()].unsqueeze(-1).long().expand(-1, -1, -1, x.size(-1))
                 x = torch.gather(xg, 2, gather).reshape(x.size(0), -1, x.size(-1))
         index_out, bias = None, self.bias
         nxt = reg.entries.get(self.tag + 1)
         if nxt is not None and nxt[0] == dim_out and nxt[2] != 1.0:
-            index_out = reg.sample(sub_batches, self.groups, dim_out, nxt[2], dev)
+            index_out = reg.sample(sub_batches, self.groups, dim_out, nxt[2], dev, host_paced(dim_out * nxt[2]))
             reg.buffer = (self.tag + 1, index_out)
             if self.bias is not None:
                 per_row = self.bias.view(1, self.groups, -1).expand(x.size(0), -1, -1)
