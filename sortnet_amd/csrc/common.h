@@ -137,9 +137,11 @@ public:
 // call once it is there; nothing waits.  When the every-term kernel ran kHintStreak times in a row for a (site, weight matrix,
 // shape) - a layer - the next kHintSkip calls do not build tables at all (hint_build_tables returns false), then one call
 // probes again.  A performance hint only: results do not depend on it.  Nothing is expected or remembered while `stream` is
-// being captured (tables are then always built).  hint_forget: the kernel was not launched after all.
+// being captured: tables are then always built, except those that no probe of the operands goes before (`unprobed`), which a
+// graph would pay for in every replay where they do not serve; they are captured where they served the layer's last call that
+// is known of.  hint_forget: the kernel was not launched after all.
 constexpr int kHintStreak = 3, kHintSkip = 31;
-bool hint_build_tables(int site, const void* weight, int B, int CO, int CI, hipStream_t stream);
+bool hint_build_tables(int site, const void* weight, int B, int CO, int CI, hipStream_t stream, bool unprobed = false);
 unsigned long long* hint_expect(int site, const void* weight, int B, int CO, int CI, hipStream_t stream);
 void hint_forget(unsigned long long* word);
 

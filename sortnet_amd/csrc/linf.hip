@@ -34,7 +34,8 @@ constexpr float kBoundPosColsCap = 0.15f;
 // 0.02 (9.4 % marked), without and with positions: 512 x 1024 x 1024 57 / 41, 95 / 56; 250 x 3072 x 1021 84 / 70, 110 / 87; 400 x
 // 5120 x 640 139 / 95, 218 / 114; below the line 128 x 1024 x 1024 21 / 34, 39 / 42 and 100 x 3072 x 1024 44 / 65, 62 / 80.  At 22.5 %
 // marked 256 x 2048 x 1200 takes 67 / 73, 99 / 109 (512 x 1024 x 1024 57 / 51), which is where their limit comes from.  Weights
-// that decide mark everything: about 25 us for the tables, until the hints say not to build them.
+// that decide mark everything: about 25 us for the tables, until the hints say not to build them; a graph, whose replays the
+// hints do not reach, holds them only where they served the layer's last calls.
 constexpr long long kBoundRowsMinTerms = 1ll << 27, kBoundRowsMinOutputs = 3ll << 16;
 constexpr float kBoundSmallRowsCap = 0.18f;
 constexpr int kHintSiteBound = 1, kHintSiteBoundSparse = 8, kHintSiteBoundPos = 9;
@@ -454,8 +455,8 @@ extern "C" int sd_bound_inf_dist_forward_nograd(const float* inputL, const float
     const int bound_form = g_bound_form.load(std::memory_order_relaxed);
     const float cap = bound_density >= 0.f ? bound_density : kBoundColsCap;
     int tables = bound_tables_eligible(a, cap, B, CO, CI, G, HW);
-    // The workspace is sized by shape alone (whatever the hints below decide), so that a call under graph capture,
-    // which always builds the tables, never needs more than the eager call before it did.
+    // The workspace is sized by shape alone (whatever the hints below decide), so that a call under graph capture, for
+    // which they may decide otherwise, never needs more than the eager call before it did.
     char* wsbase = nullptr;
     if (tables) {
         const size_t both = bound_tables_bytes(tables == 2, B, CO, CI), walk = tables == 2 && CI <= 65536 ? sort_cols_workspace(B, CO, CI) : 0;
@@ -465,7 +466,7 @@ extern "C" int sd_bound_inf_dist_forward_nograd(const float* inputL, const float
     }
     // with the built-in limit, a layer whose tables have not paid lately is not given any for a while
     const bool hinted = tables && bound_density < 0.f;
-    if (hinted && !hint_build_tables(kHintSiteBound, weight, B, CO, CI, st)) tables = 0;
+    if (hinted && !hint_build_tables(kHintSiteBound, weight, B, CO, CI, st, tables == 1)) tables = 0;
     // Very few marks (weights of unit scale against rows that are alike: below 1 %): the staged kernel would spend its
     // time moving tiles through LDS, and the kernel that walks a weight row's marks over a transposed copy of the
     // inputs serves better.  Chosen by hand (sd_set_bound_candidate_form) or, with the built-in limit, for a layer
@@ -542,9 +543,9 @@ extern "C" int sd_bound_inf_dist_forward(const float* inputL, const float* input
     int tables = bound_tables_eligible(a, cap, B, CO, CI, G, HW);
     const size_t pairs = ((size_t)a.R * a.G * a.COg * 16 + 255) / 256 * 256;
     if (tables && bound_density < 0.f && !workspace_ready(pairs + bound_tables_bytes(tables == 2, B, CO, CI), st)) tables = 0;   // a first call under capture
-    const int elig = tables;   // by shape alone: what the workspace is sized by (a captured call always builds tables)
+    const int elig = tables;   // by shape alone: what the workspace is sized by (a captured call may build tables that an eager one does not)
     const bool hinted = tables && bound_density < 0.f;
-    if (hinted && !hint_build_tables(kHintSiteBoundPos, weight, B, CO, CI, st)) tables = 0;
+    if (hinted && !hint_build_tables(kHintSiteBoundPos, weight, B, CO, CI, st, tables == 1)) tables = 0;
     if (tables == 2 && a.nsplit < 2) a.nsplit = 2;   // both kernels merge into the packed pairs
     if (a.nsplit > 1 || elig) {
         size_t n = (size_t)a.R * a.G * a.COg;

@@ -131,6 +131,7 @@ struct HintSlot {
     int head, queued;           // oldest outcome not yet looked at, and how many are queued
     int stale;                  // of the queued outcomes, how many belong to the layer the slot stood for before
     int streak, skip_left;
+    bool known;                 // an outcome of this layer has arrived
     unsigned long long used;    // g_hint_clock at the slot's last use: the least recently used slot is given away
 };
 std::mutex g_hint_mu;
@@ -142,6 +143,7 @@ void hint_rekey(HintSlot& h, int dev, int site, const void* weight, int B, int C
     h.dev = dev; h.site = site; h.weight = weight; h.B = B; h.CO = CO; h.CI = CI;
     h.stale = h.queued;
     h.streak = h.skip_left = 0;
+    h.known = false;
 }
 
 HintSlot* hint_slot(int site, const void* weight, int B, int CO, int CI, bool create) {
@@ -176,27 +178,34 @@ HintSlot* hint_slot(int site, const void* weight, int B, int CO, int CI, bool cr
     g_hints.push_back(h);
     return &g_hints.back();
 }
-}  // namespace
 
-bool hint_build_tables(int site, const void* weight, int B, int CO, int CI, hipStream_t stream) {
-    if (capturing(stream)) return true;
-    std::lock_guard<std::mutex> lock(g_hint_mu);
-    HintSlot* h = hint_slot(site, weight, B, CO, CI, false);
-    if (!h) return true;
-    // outcomes that have arrived, oldest first (the host may run several calls ahead of the device)
-    while (h->queued > 0) {
-        const unsigned long long ran = __atomic_load_n(&h->host[h->head], __ATOMIC_ACQUIRE);
+// takes the outcomes that have arrived, oldest first (the host may run several calls ahead of the device)
+void hint_drain(HintSlot& h) {
+    while (h.queued > 0) {
+        const unsigned long long ran = __atomic_load_n(&h.host[h.head], __ATOMIC_ACQUIRE);
         if (ran == kHintPending) break;   // not there yet: next call
-        if (h->stale > 0) h->stale--;   // an outcome of the layer this slot stood for before
+        if (h.stale > 0) h.stale--;   // an outcome of the layer this slot stood for before
         else if (ran != kHintVoid) {
-            h->streak = ran != 0ull ? h->streak + 1 : 0;
+            h.known = true;
+            h.streak = ran != 0ull ? h.streak + 1 : 0;
             // the streak is long enough (or the probe after a stretch without tables came out the same): no tables
             // for the next kHintSkip calls, then one call probes again
-            h->skip_left = h->streak >= kHintStreak ? kHintSkip : 0;
+            h.skip_left = h.streak >= kHintStreak ? kHintSkip : 0;
         }
-        h->head = (h->head + 1) % kHintRing;
-        h->queued--;
+        h.head = (h.head + 1) % kHintRing;
+        h.queued--;
     }
+}
+}  // namespace
+
+bool hint_build_tables(int site, const void* weight, int B, int CO, int CI, hipStream_t stream, bool unprobed) {
+    const bool graph = capturing(stream);
+    if (graph && !unprobed) return true;
+    std::lock_guard<std::mutex> lock(g_hint_mu);
+    HintSlot* h = hint_slot(site, weight, B, CO, CI, false);
+    if (h) hint_drain(*h);
+    if (graph) return h && h->known && h->streak == 0;
+    if (!h) return true;
     if (h->skip_left > 0) { h->skip_left--; return false; }
     return true;
 }

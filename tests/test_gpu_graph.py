@@ -467,3 +467,52 @@ def test_layers_of_one_slice_are_captured_unprepared(op):
                 _close(got, ref, op)
             else:
                 assert torch.equal(got, ref)
+
+
+def _nodes(call):
+    """Number of nodes of the call's graph, which is not run."""
+    from sortnet_amd import _lib
+    lib = _lib.load()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph, stream=torch.cuda.current_stream()):
+        call()
+    count = ctypes.c_size_t()
+    assert lib.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(count)) == 0
+    return count.value
+
+
+@pytest.mark.parametrize("positions", [False, True])
+def test_captured_interval_bounds_leave_out_tables_that_did_not_serve(positions):
+    """Layers given tables per batch row alone have no probe in front of them: a graph holds the tables where they served the
+    layer's last calls, and not where the weights decide or nothing is known of the layer yet."""
+    from sortnet_amd import ext, _lib
+    dev = _dev()
+    g = torch.Generator().manual_seed(11)
+    B, n, m = 251, 3072, 1021
+    xl = torch.rand(B, n, 1, generator=g).to(dev)
+    xu = xl + 0.03
+    yl, yu = torch.empty(B, m, 1, device=dev), torch.empty(B, m, 1, device=dev)
+    pl, pu = (torch.empty(B, m, 1, device=dev, dtype=torch.int32) for _ in range(2))
+    weights = {s: (torch.randn(m, n, generator=g) * s).to(dev) for s in (0.02, 1.0)}
+
+    def call(w):
+        if positions:
+            ext.bound_inf_dist_forward(xl, xu, w, yl, yu, pl, pu, 1)
+        else:
+            ext.bound_inf_dist_forward_nograd(xl, xu, w, yl, yu, 1)
+
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        call(weights[0.02])                      # the stream's scratch
+        _lib.set_bound_candidate_density(0.0)
+        call(weights[1.0])
+        torch.cuda.synchronize()
+        plain = _nodes(lambda: call(weights[1.0]))
+        _lib.set_bound_candidate_density(-1.0)
+        assert _nodes(lambda: call(weights[1.0])) == plain          # nothing is known of it
+        for scale, tables in ((1.0, False), (0.02, True)):
+            for _ in range(3):
+                call(weights[scale])
+            torch.cuda.synchronize()
+            assert (_nodes(lambda: call(weights[scale])) > plain) == tables, scale
+    torch.cuda.synchronize()
