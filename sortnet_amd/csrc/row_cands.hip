@@ -291,8 +291,9 @@ __global__ void __launch_bounds__(64 * kRtWaves) rt_main_kernel(RtArgs a) {
     auto use = [&](int buf, int i, int k, int n, const Own& o) __attribute__((always_inline)) { term(std::false_type{}, buf, i, k, n, o); };
     // smallest results of the lane's rows over the wavefront (weight rows past the last one do not count)
     float thU = 0.f, thL = 0.f;
-    auto smallest = [&](float v0, float v1) __attribute__((always_inline)) {
-        return wave_min_nonneg(fminf(in0 ? v0 : __builtin_inff(), in1 ? v1 : __builtin_inff()));
+    // (never below what it was: an ordered walk forgets the strong marks' results, but they are terms of these rows)
+    auto smallest = [&](float was, float v0, float v1) __attribute__((always_inline)) {
+        return fmaxf(was, wave_min_nonneg(fminf(in0 ? v0 : __builtin_inff(), in1 ? v1 : __builtin_inff())));
     };
     // In kRowsSortPos the strong marks give each row a lower bound of its K-th largest term.  A term below it is never among
     // the K largest, and whether one at or above it enters depends only on entries at least that large, so the walk in input
@@ -312,10 +313,10 @@ __global__ void __launch_bounds__(64 * kRtWaves) rt_main_kernel(RtArgs a) {
             load, value, use,
             [&](bool strong) __attribute__((always_inline)) {
                 if (FORM == kRowsSortPos && strong) { least[0] = hi[0][0]; least[1] = hi[1][0]; }
-                if constexpr (FORM == kRowsSortValues || FORM == kRowsSortInterval) thU = smallest(__int_as_float(hi[0][0]), __int_as_float(hi[1][0]));
-                else thU = smallest(fmaxf(fabsf(hi[0][0]), least[0]), fmaxf(fabsf(hi[1][0]), least[1]));
-                if constexpr (FORM == kRowsSortInterval) thL = smallest(__int_as_float(lo[0][0]), __int_as_float(lo[1][0]));
-                else if constexpr (IV) thL = smallest(lo[0][0], lo[1][0]);
+                if constexpr (FORM == kRowsSortValues || FORM == kRowsSortInterval) thU = smallest(thU, __int_as_float(hi[0][0]), __int_as_float(hi[1][0]));
+                else thU = smallest(thU, fmaxf(fabsf(hi[0][0]), least[0]), fmaxf(fabsf(hi[1][0]), least[1]));
+                if constexpr (FORM == kRowsSortInterval) thL = smallest(thL, __int_as_float(lo[0][0]), __int_as_float(lo[1][0]));
+                else if constexpr (IV) thL = smallest(thL, lo[0][0], lo[1][0]);
             },
             [&](int n, const Own& o) __attribute__((always_inline)) {
                 const float2 r = ranges[n];

@@ -428,8 +428,8 @@ mc_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const 
                     [&](int n) __attribute__((always_inline)) { return Own{wrow[n], 0.f}; },
                     [&](int n, const Own& o) __attribute__((always_inline)) { return caps(n, o.a).x; },
                     load, use, use,
-                    [&](bool) __attribute__((always_inline)) {
-                        th = wave_min_nonneg(fminf(in0 ? fabsf(best[0]) : __builtin_inff(), in1 ? fabsf(best[1]) : __builtin_inff()));
+                    [&](bool) __attribute__((always_inline)) {   // (never below what the strong marks showed, which an ordered walk forgets)
+                        th = fmaxf(th, wave_min_nonneg(fminf(in0 ? fabsf(best[0]) : __builtin_inff(), in1 ? fabsf(best[1]) : __builtin_inff())));
                     },
                     [&](int n, const Own& o) __attribute__((always_inline)) { return !(caps(n, o.a).x < th); },
                     [&]() __attribute__((always_inline)) { best[0] = best[1] = kEps; where[0] = where[1] = 0; });
