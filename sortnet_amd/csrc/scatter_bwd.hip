@@ -92,7 +92,14 @@ __global__ void __launch_bounds__(1024) scatter_bwd_rows_kernel(BwdArgs a) {
     const int bg = row / a.HW;
     const int g = bg % a.G, b = bg / a.G;
     const int s = b / kSubBatch;
-    const int n0 = (int)((long long)a.CIg * blockIdx.y / gridDim.y), len = (int)((long long)a.CIg * (blockIdx.y + 1) / gridDim.y) - n0;
+    // (a power of two of parts; without parts nothing of it is left: with 64-bit divisions here a layer of 128 x 3072 x 1024, one
+    // position per output, took 4.6 us instead of 3.9, 512 x 512 x 10 3.7 instead of 3.2)
+    int n0 = 0, len = a.CIg;
+    if constexpr (SORT) {
+        const int parts = __builtin_ctz(gridDim.y);
+        n0 = a.CIg * (int)blockIdx.y >> parts;
+        len = (a.CIg * (int)(blockIdx.y + 1) >> parts) - n0;
+    }
     for (int n = threadIdx.x; n < len; n += blockDim.x) hist[n] = 0.f;
     __syncthreads();
     const size_t obase = ((size_t)(b * a.G + g) * a.COg) * a.HW + hw;
@@ -116,7 +123,7 @@ __global__ void __launch_bounds__(1024) scatter_bwd_rows_kernel(BwdArgs a) {
                 const int n = pr[i] & 0x7fffffff;
                 float v = pr[i] >= 0 ? grad : -grad;
                 if (SORT) { v = v * coef * a.q; coef *= 1.f - a.q; }
-                if ((unsigned)(n - n0) < (unsigned)len) atomicAdd(&hist[n - n0], v);
+                if (!SORT || (unsigned)(n - n0) < (unsigned)len) atomicAdd(&hist[n - n0], v);
                 if (HAS_W) {
                     int nn = a.ci_idx ? a.ci_idx[(s * a.G + g) * a.CIg + n] : n;
                     unsafeAtomicAdd(a.gw + wrow + nn, -v);
