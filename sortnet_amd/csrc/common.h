@@ -77,8 +77,9 @@ __device__ __forceinline__ bool gate_closed(const unsigned long long* gate, unsi
     return gate != nullptr && (*gate > limit) != (above != 0);
 }
 
-// the same for a forward tile kernel, whose first work-item reports the outcome
+// the same for a forward tile kernel, whose first work-item reports the outcome (nothing is reported without a gate)
 __device__ __forceinline__ bool gate_closed(const FwdArgs& a) {
+    if (a.gate == nullptr) return false;
     const bool closed = gate_closed(a.gate, a.gate_limit, a.gate_above);
     if ((a.told || a.told2) && threadIdx.x == 0 && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) {
         if (a.told) __hip_atomic_store(a.told, closed ? 0ull : 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
