@@ -145,7 +145,12 @@ static std::atomic<float> g_sort_density{-1.f};
 //   interval     512 x 5120 x 5120 3901 / 702 (14 %), 4120 / 1448 (47 %); 256 x 2048 x 512 241 / 106 (23 %), 252 / 169 (66 %)
 //   positions    512 x 5120 x 5120 2447 / 818 (12 %), 2471 / 1592 (43 %); 128 x 5120 x 5120 583 / 305 (12 %), 600 / 561 (43 %);
 //                256 x 2048 x 512 139 / 125 (21 %), 143 / 204 (61 %); 96 x 5120 x 300 216 / 150 (11 %), 220 / 256 (38 %)
-static float sort_cols_cap(int form) { return form == kRowsSortPos ? 0.22f : 0.40f; }
+// Smallest layers that have no kernel of their own (row_stream_sort_ok), values: 100 x 480 x 450 48 / 30 (15 %), 49 / 36 (39 %); 72 x
+// 1024 x 1024 94 / 40 (23 %), 95 / 54 (49 %); 16 x 4096 x 4128 183 / 130 (29 %); 300 x 320 x 256 34 / 32 (20 %), 35 / 37 (47 %).  Rows of
+// 256 inputs are formed before the tables are done: 512 x 256 x 256 30 / 35 (26 %), 256 x 256 x 300 29 / 31 (25 %).
+static float sort_cols_cap(int form, int CI) {
+    return form == kRowsSortPos ? 0.22f : form == kRowsSortValues && CI < 320 ? 0.10f : 0.40f;
+}
 constexpr long long kSortColsMinTerms = 1ll << 24;
 
 // `site`: which entry point asks (with the built-in limit, a layer whose tables have not paid lately is not given
@@ -192,7 +197,7 @@ static size_t sort_tables_bytes(int form, int B, int CO, int CI, int K) {
 static int queue_sort_cols(FwdArgs& a, int form, const float* xl, const float* xu, const float* w, int B, int CO, int CI,
                            float q, int K, float* outL, float* outU, int* pos, void* ws, hipStream_t st) {
     const float density = g_sort_density.load(std::memory_order_relaxed);
-    const float cap = density > 0.f ? density : sort_cols_cap(form);
+    const float cap = density > 0.f ? density : sort_cols_cap(form, CI);
     int rc = sort_cols_forward(xl, xu, w, B, CO, CI, q, K, outL, outU, pos, ws, cap, &a.gate, &a.gate_limit, st);
     a.gate_above = 1;
     const long long terms = (long long)B * CO * CI;
