@@ -23,8 +23,10 @@ enum StreamOp { kStreamMax, kStreamPos, kStreamSort };
 // leave room for twelve wavefronts per compute unit
 constexpr int stream_waves(StreamOp op) { return op == kStreamSort ? 4 : 8; }
 
-// wavefronts per SIMD that the registers leave room for
+// wavefronts per SIMD that the registers are to leave room for, and how many to count on (rows of up to 1024 inputs leave room for
+// twice as many)
 constexpr int stream_occupancy(int NE, StreamOp op) { return NE <= 48 ? 4 : NE <= 80 ? (op == kStreamSort ? 3 : 4) : (op == kStreamSort ? 1 : 2); }
+constexpr int stream_resident(int NE, int NX, StreamOp op) { return NE <= 16 ? (NX == 2 && op == kStreamPos ? 7 : 8) : stream_occupancy(NE, op); }
 
 // maximum over the wavefront, in every lane (row-wise shifts, then the two row broadcasts; v >= 0)
 __device__ __forceinline__ float wave_max(float v) {
@@ -342,11 +344,14 @@ row_stream_kernel(FwdArgs a, int K) {
 template <int NE, int NX, StreamOp OP>
 int launch(const FwdArgs& a, int K, hipStream_t stream) {
     // few weight rows: the batch rows are dealt to several workgroups, each of which loads the weight rows again; as many as
-    // the device holds at once, so that none waits for another's end (512 x 5120 x 10, K = 10: 21 us; in 1.3 times as many 26
-    // and, interval bounds, 46 and 54)
-    constexpr int kWaves = stream_waves(OP), kPerCu = 4 * stream_occupancy(NE, OP) / kWaves;
+    // the device holds at once, so that none waits for another's end (512 x 5120 x 10, K = 10: 19 us; in 1.3 times as many 26
+    // and, interval bounds, 42 and 55).  Rows of up to 1024 inputs, with twice as many workgroups as for longer ones: 54 x 730 x 730
+    // 40 us instead of 50, intervals 75 and 99, l-inf with positions 11 and 14; 32 x 1024 x 1536 52 and 63.  (Three for two against rows
+    // of 1025 to 3072 inputs, values of the l-inf distance: 54 x 1500 x 730 12.5 and 13.9, but 7 x 3072 x 2000 15.1 and 13.2.)
+    constexpr int kWaves = stream_waves(OP), kPerCu = 4 * stream_resident(NE, NX, OP) / kWaves;
     const int tiles = (a.COg + kWaves - 1) / kWaves * a.G, most = (kPerCu > 1 ? kPerCu : 1) * num_cus();
-    const int slices = tiles >= most ? 1 : most / tiles, rows = slices < a.R ? (a.R + slices - 1) / slices : 1;
+    auto dealt = [&](int slices) { return slices < a.R ? (a.R + slices - 1) / slices : 1; };
+    const int rows = dealt(tiles >= most ? 1 : most / tiles);
     const dim3 grid(tiles, (a.R + rows - 1) / rows), block(64 * kWaves);
     note_forward_kernel("row_stream_kernel", kWaves, NE);
     forward_kernel_timer(stream, false);

@@ -87,3 +87,25 @@ def test_streamed_layers_match_oracle(oracle, shape, kind):
             streamed()
         np.testing.assert_allclose(y.cpu().numpy(), rl.reshape(B, m * G, 1), rtol=1e-5, atol=1e-6)
         np.testing.assert_allclose(y2.cpu().numpy(), ru.reshape(B, m * G, 1), rtol=1e-5, atol=1e-6)
+
+
+# batch rows dealt to the workgroups that the device holds at once, one to several rows each, the last one fewer
+@pytest.mark.parametrize("B,n,m", [(300, 1024, 70), (33, 700, 1537), (90, 2050, 24), (513, 3100, 10)])
+def test_batch_rows_dealt_to_workgroups(oracle, B, n, m):
+    from sortnet_amd import _lib, ext
+    x, w = _data((B, n, m, 1), "normal")
+    xd, wd = x.cuda(), w.cuda()
+    y, y2 = (torch.full((B, m, 1), float("nan"), device="cuda") for _ in range(2))
+    p = torch.full((B, m, 1), -7, device="cuda", dtype=torch.int32)
+    ry, rp = oracle.inf_dist_forward(x.numpy(), w.numpy())
+    ext.inf_dist_forward(xd, wd, y, p, 1)
+    assert _lib.last_forward_kernel().startswith("row_stream_kernel")
+    assert np.array_equal(y.cpu().numpy(), ry) and np.array_equal(p.cpu().numpy(), rp)
+    ext.sort_neuron_forward_nograd(xd, wd, y, 1, 0.6, 10)
+    assert _lib.last_forward_kernel().startswith("row_stream_kernel")
+    ref = oracle.sort_neuron_forward(x.numpy(), w.numpy(), 0.6, 10, need_pos=False)
+    np.testing.assert_allclose(y.cpu().numpy(), ref.reshape(B, m, 1), rtol=1e-5, atol=1e-6)   # the same ten products, summed in fp32
+    rl, ru = oracle.bound_sort_neuron_forward((x - 0.1).numpy(), (x + 0.1).numpy(), w.numpy(), 0.6, 10)
+    ext.bound_sort_neuron_forward((x - 0.1).cuda(), (x + 0.1).cuda(), wd, y, y2, 1, 0.6, 10)
+    np.testing.assert_allclose(y.cpu().numpy(), rl.reshape(B, m, 1), rtol=1e-5, atol=1e-6)
+    np.testing.assert_allclose(y2.cpu().numpy(), ru.reshape(B, m, 1), rtol=1e-5, atol=1e-6)
