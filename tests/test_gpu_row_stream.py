@@ -89,8 +89,10 @@ def test_streamed_layers_match_oracle(oracle, shape, kind):
         np.testing.assert_allclose(y2.cpu().numpy(), ru.reshape(B, m * G, 1), rtol=1e-5, atol=1e-6)
 
 
-# batch rows dealt to the workgroups that the device holds at once, one to several rows each, the last one fewer
-@pytest.mark.parametrize("B,n,m", [(300, 1024, 70), (33, 700, 1537), (90, 2050, 24), (513, 3100, 10)])
+# batch rows dealt to the workgroups that the device holds at once, one to several rows each, the last one fewer; as many rows as
+# workgroups and one more, where two to four rounds of them take over
+@pytest.mark.parametrize("B,n,m", [(300, 1024, 70), (33, 700, 1537), (32, 1023, 1536), (255, 5124, 12), (256, 5124, 12), (257, 5121, 12),
+                                   (90, 2050, 24), (513, 3100, 10)])
 def test_batch_rows_dealt_to_workgroups(oracle, B, n, m):
     from sortnet_amd import _lib, ext
     x, w = _data((B, n, m, 1), "normal")
