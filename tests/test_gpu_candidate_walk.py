@@ -1,7 +1,7 @@
 """Lists of marks at the sizes where they are handled differently: of at most 64 marks (walked as they are), of 65 to 128
 (groups of one or two), of more than 2048 (handed over in parts), and rows that end inside a block of 256 or a slice of 512
 inputs.  The table kernels, forced to run however many marks there are, against the kernels that evaluate every term: the
-same bits, ties and positions included."""
+same bits, ties and positions included.  (Rows that are alike: tables per weight row; images against small weights: per batch row.)"""
 import pytest
 import torch
 
@@ -23,7 +23,7 @@ def test_table_kernels_at_the_edges_of_their_lists(B, CI, CO, K, kind):
     x, w = _data(np.random.default_rng(CI), B, CI, CO, kind, g, dev)
     r = torch.rand(B, CI, 1, generator=g).to(dev) * 0.05
     xl, xu = (x - r).contiguous(), (x + r).contiguous()
-    results = []
+    results, shares = [], []
     try:
         for density, form in ((0.0, 0), (1.0, 1), (1.0, 2)):
             _lib.set_sort_candidate_density(density)
@@ -33,13 +33,16 @@ def test_table_kernels_at_the_edges_of_their_lists(B, CI, CO, K, kind):
             o = [torch.full((B, CO, 1), float("nan"), device=dev) for _ in range(10)]
             p = [torch.full((B, CO, 1), -7, device=dev, dtype=torch.int32) for _ in range(4)]
             pk = torch.full((K, B, CO, 1), -7, device=dev, dtype=torch.int32)
-            ext.sort_neuron_forward_nograd(x, w, o[0], 1, 0.75, K)
-            ext.sort_neuron_forward(x, w, o[1], pk, 1, 0.75, K)
-            ext.bound_sort_neuron_forward(xl, xu, w, o[2], o[3], 1, 0.75, K)
-            ext.inf_dist_forward(x, w, o[4], p[0], 1)
-            ext.masked_inf_dist_forward(x, w, o[5], p[1], 1, 0.5, 7, ext.MASK_FACTORED)
-            ext.bound_inf_dist_forward_nograd(xl, xu, w, o[6], o[7], 1)
-            ext.bound_inf_dist_forward(xl, xu, w, o[8], o[9], p[2], p[3], 1)
+            for call in (lambda: ext.sort_neuron_forward_nograd(x, w, o[0], 1, 0.75, K),
+                         lambda: ext.sort_neuron_forward(x, w, o[1], pk, 1, 0.75, K),
+                         lambda: ext.bound_sort_neuron_forward(xl, xu, w, o[2], o[3], 1, 0.75, K),
+                         lambda: ext.inf_dist_forward(x, w, o[4], p[0], 1),
+                         lambda: ext.masked_inf_dist_forward(x, w, o[5], p[1], 1, 0.5, 7, ext.MASK_FACTORED),
+                         lambda: ext.bound_inf_dist_forward_nograd(xl, xu, w, o[6], o[7], 1),
+                         lambda: ext.bound_inf_dist_forward(xl, xu, w, o[8], o[9], p[2], p[3], 1)):
+                call()
+                if density == 1.0 and (form == 1 or kind == 0):   # (the other form has no table per batch row)
+                    shares.append(_lib.last_forward_term_share())
             results.append(o + p + [pk])
     finally:
         _lib.set_sort_candidate_density(-1.0)
@@ -49,3 +52,5 @@ def test_table_kernels_at_the_edges_of_their_lists(B, CI, CO, K, kind):
     for tables in results[1:]:
         for i, (a, b) in enumerate(zip(results[0], tables)):
             assert torch.equal(a, b), i
+    if kind < 2 and CI >= 2048 and K <= 10:
+        assert max(shares) < 1.0   # a table served every call

@@ -1,6 +1,7 @@
 """Candidate tables at the lengths of a row where their kernel changes: a wavefront alone, one to three blocks of 256 inputs per
 wavefront (up to 4096, 8192 and 12288 inputs), rows that end inside a block, and longer ones, which are read twice; one to three
-tiles of the other operand.  The table kernels, forced to run, against the kernels that evaluate every term: the same bits."""
+tiles of the other operand.  The table kernels, forced to run, against the kernels that evaluate every term: the same bits.  Rows
+that are alike are served by the tables per weight row, images against small weights by those per batch row."""
 import numpy as np
 import pytest
 import torch
@@ -10,7 +11,7 @@ from test_gpu_candidate_random import _data
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("kind", [0, 3])
+@pytest.mark.parametrize("kind", [0, 1, 3])
 @pytest.mark.parametrize("CI", [32, 256, 288, 4064, 4096, 4128, 8192, 8224, 12288, 12320])
 @pytest.mark.parametrize("B,CO", [(5, 130), (129, 3), (257, 258)])
 def test_tables_of_rows_of_any_length(B, CI, CO, kind):
@@ -23,21 +24,27 @@ def test_tables_of_rows_of_any_length(B, CI, CO, kind):
     r = torch.rand(B, CI, 1, generator=g).to(dev) * 0.05 - 0.005   # some intervals are inverted
     xl, xu = (x - r).contiguous(), (x + r).contiguous()
     K = min(10, CI // 4)
-    results = []
+    results, shares = [], []
     try:
         for density, form in ((0.0, 0), (1.0, 1), (1.0, 2)):
             _lib.set_sort_candidate_density(density)
             _lib.set_linf_candidate_density(density)
             _lib.set_bound_candidate_density(density)
             _lib.set_bound_candidate_form(form)
-            o = [torch.full((B, CO, 1), float("nan"), device=dev) for _ in range(7)]
-            p = [torch.full((B, CO, 1), -7, device=dev, dtype=torch.int32) for _ in range(2)]
-            ext.sort_neuron_forward_nograd(x, w, o[0], 1, 0.75, K)
-            ext.bound_sort_neuron_forward(xl, xu, w, o[1], o[2], 1, 0.75, K)
-            ext.inf_dist_forward(x, w, o[3], p[0], 1)
-            ext.masked_inf_dist_forward(x, w, o[4], p[1], 1, 0.5, 7, ext.MASK_FACTORED)
-            ext.bound_inf_dist_forward_nograd(xl, xu, w, o[5], o[6], 1)
-            results.append(o + p)
+            o = [torch.full((B, CO, 1), float("nan"), device=dev) for _ in range(10)]
+            p = [torch.full((B, CO, 1), -7, device=dev, dtype=torch.int32) for _ in range(4)]
+            pk = torch.full((K, B, CO, 1), -7, device=dev, dtype=torch.int32)
+            for call in (lambda: ext.sort_neuron_forward_nograd(x, w, o[0], 1, 0.75, K),
+                         lambda: ext.bound_sort_neuron_forward(xl, xu, w, o[1], o[2], 1, 0.75, K),
+                         lambda: ext.sort_neuron_forward(x, w, o[7], pk, 1, 0.75, K),
+                         lambda: ext.inf_dist_forward(x, w, o[3], p[0], 1),
+                         lambda: ext.masked_inf_dist_forward(x, w, o[4], p[1], 1, 0.5, 7, ext.MASK_FACTORED),
+                         lambda: ext.bound_inf_dist_forward_nograd(xl, xu, w, o[5], o[6], 1),
+                         lambda: ext.bound_inf_dist_forward(xl, xu, w, o[8], o[9], p[2], p[3], 1)):
+                call()
+                if density == 1.0 and (form == 1 or kind == 0):   # (the other form has no table per batch row)
+                    shares.append(_lib.last_forward_term_share())
+            results.append(o + p + [pk])
     finally:
         _lib.set_sort_candidate_density(-1.0)
         _lib.set_linf_candidate_density(-1.0)
@@ -46,6 +53,8 @@ def test_tables_of_rows_of_any_length(B, CI, CO, kind):
     for tables in results[1:]:
         for i, (a, b) in enumerate(zip(results[0], tables)):
             assert torch.equal(a, b), i
+    if kind != 3 and CI >= 4064:
+        assert max(shares) < 1.0   # a table served every call
 
 
 @pytest.mark.parametrize("equal", [0, 2, 3, 40])   # ties of the K-th largest term: none, as many as are noted, one more, many
