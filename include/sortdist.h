@@ -87,11 +87,10 @@ float sd_last_forward_term_share(sd_stream_t stream);
 int sd_set_lp_candidate_density(float density);
 /* The same for sd_bound_inf_dist_forward_nograd and sd_bound_inf_dist_forward on dense single-group layers (CI a multiple of 32): a kernel that works
  * from a table of the inputs that can hold the maximum of a weight row over a tile of 128 batch rows, and the kernel
- * that evaluates every term; both give the same bits.  Built-in limits: 0.30 (0.40 where the table is built per batch
- * row and tile of 128 weight rows instead, which the call decides from its operands), layers of at least 2^31 terms (the
- * latter alone, at 0.18, from 2^27 terms and 3 * 2^16 outputs);
- * a `density` of 0 or more applies at any size.  The form with positions has a built-in limit of 0.15; values and
- * positions are the every-term kernel's.  No reference counterpart
+ * that evaluates every term; both give the same bits.  Built-in limits, layers of at least 2^31 terms: 0.30, with positions
+ * 0.15; 0.40 where the table is built per batch row and tile of 128 weight rows instead, which the call decides from its
+ * operands.  Smaller layers, of at least 2^27 + 3 * 2^16 * CI terms, get tables per batch row alone, at 0.18.  A `density` of 0 or
+ * more applies at any size.  Values and positions are the every-term kernel's.  No reference counterpart
  * (core/cuda/bound_inf_dist_cuda.cu evaluates every term). */
 int sd_set_bound_candidate_density(float density);
 /* Which table kernel serves sd_bound_inf_dist_forward_nograd: 1 = the one that stages tiles of inputs and weights
@@ -103,13 +102,15 @@ int sd_set_bound_candidate_form(int form);
 /* The same for sd_sort_neuron_forward[_nograd] and sd_bound_sort_neuron_forward on dense single-group layers (CI a
  * multiple of 32): a kernel that works from a table of the inputs that can be among the K largest terms of a weight
  * row over a tile of 128 batch rows, and the kernels that evaluate every term; both give the same bits (positions
- * included).  Built-in limits 0.40 and, with positions, 0.22 (per batch row 0.27, interval bounds 0.45, positions 0.22), and the table is only built for layers of at least 2^24 terms; a positive `density` applies at any
- * size.  No reference counterpart (core/cuda/sort_neuron.cu evaluates every term). */
+ * included).  Built-in limits 0.40 (values of rows of fewer than 320 inputs 0.10) and, with positions, 0.22, layers of
+ * at least 2^24 terms; per batch row and tile of 128 weight rows 0.27, interval bounds 0.45, positions 0.22, from 2^28 terms.  A positive
+ * `density` applies at any size.  No reference counterpart (core/cuda/sort_neuron.cu evaluates every term). */
 int sd_set_sort_candidate_density(float density);
 /* The same for sd_inf_dist_forward[_nograd] (no index lists) and sd_masked_inf_dist_forward (factored mask) on dense
  * single-group layers (CI a multiple of 32, at most 65536): a kernel that works from a table of the inputs that can hold
  * the maximum of a weight row over a tile of 128 batch rows, and the kernels that evaluate every term; same values and
- * positions either way.  Built-in limit 0.10, layers of at least 2^31 terms.  Under the mask the table's bound rests on
+ * positions either way.  Built-in limit 0.10, layers of at least 2^31 terms; where the table is built per batch row and tile of
+ * 128 weight rows instead 0.20, from 2^33 terms.  Under the mask the table's bound rests on
  * `depth` inputs per weight row, chosen so that a batch row keeps none of them less than once in 10^4 outputs (such an
  * output is recomputed from every input); sd_set_linf_candidate_depth overrides the choice (0 = automatic; 8, 12, 16,
  * 20 or 24).  No reference counterpart (core/cuda/inf_dist_cuda.cu evaluates every term). */

@@ -17,8 +17,8 @@ static std::atomic<float> g_bound_density{-1.f};
 // measured at B = 512, M = N = 5120: the table kernel takes 0.09 + 2.6 x share ms (about 60 SIMD cycles per marked
 // (tile, weight row, input)) after 0.10 ms for the tables, against 1.00 ms for every term.  The tables are paid for by the time
 // the choice is made, so the limit sits a little below where the two would meet.  Per batch row (us, every term / tables):
-// 1004 / 379 (9.2 % marked), with positions 1246 / 466; 982 / 451 (25 %), with positions 1271 / 683; 128 x 5120 x
-// 5120 281 / 227 and 351 / 300 (25 %).
+// 1004 / 379 (9.2 % marked), with positions 1246 / 466; 981 / 538 (37 %), with positions 1268 / 888; 128 x 5120 x
+// 5120 293 / 178 and 350 / 256 (19 %), 289 / 234 and 355 / 352 (37 %).
 constexpr float kBoundColsCap = 0.30f, kBoundRowsCap = 0.40f;
 // With the built-in limits, layers below this many terms go without tables: building them and starting the table
 // kernel takes about 0.19 ms, which is what the every-term kernel needs for 2.4 G terms (512 x 10 x 5120: 0.06 ms

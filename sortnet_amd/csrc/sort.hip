@@ -175,8 +175,9 @@ static void sort_cols_expect(FwdArgs& a, int site, int B, int CO, int CI, hipStr
 
 // Largest share of marked (tile of 128 weight rows, batch row, input) triples at which the kernel of the tables per
 // batch row runs.  Every term / tables, us, on inputs in [0, 1] against weights of growing scale, K = 10:
-//   values       512 x 5120 x 5120 1714 / 416 (7 %), 1763 / 905 (27 %); 128 x 3072 x 1024 132 / 90 (9 %), 131 / 151 (35 %)
-//   interval     512 x 5120 x 5120 3225 / 675 (9 %), 3811 / 1560 (29 %); 128 x 3072 x 1024 312 / 116 (11 %), 342 / 216 (37 %)
+//   values       512 x 5120 x 5120 1714 / 416 (7 %), 1763 / 905 (27 %); 128 x 3072 x 1024 132 / 90 (9 %), 130 / 117 (27 %), 131 / 151 (35 %)
+//   interval     512 x 5120 x 5120 3225 / 675 (9 %), 3993 / 2025 (42 %); 128 x 3072 x 1024 312 / 116 (11 %), 335 / 217 (41 %); 64 x 2048 x 2048
+//                231 / 152 (35 %), 237 / 188 (51 %)
 //   positions    512 x 5120 x 5120 2332 / 778 (7 %), 2443 / 1748 (27 %); 128 x 3072 x 1024 182 / 132 (9 %), 179 / 176 (18 %)
 static float sort_rows_cap(int form) { return form == kRowsSortInterval ? 0.45f : form == kRowsSortValues ? 0.27f : 0.22f; }
 // Smallest layers (in terms) given tables per batch row under the built-in limit (128 x 3072 x 1024, 0.4 G terms:

@@ -230,10 +230,10 @@ int run_tables(const float* w, const uint32_t* wkeep, int S, int M, int Mp, int 
 }
 
 // ---- main kernels ------------------------------------------------------------------------------
-// A workgroup takes eight weight rows and one batch tile; each of its wavefronts one of the rows, with lane l holding the
+// A workgroup takes four weight rows (kMainTile) and one batch tile; each of its wavefronts one of the rows, with lane l holding the
 // batch rows l and l + 64 of the tile.  For its row the wavefront lists the marked inputs in LDS, cuts the list by what a
 // few strong marks say (cand_walk.h) and walks what is left: per mark one weight (a scalar operand), one transposed row of
-// inputs (two coalesced loads) and the terms.  The results of the workgroup leave through LDS, 32 bytes wide.
+// inputs (two coalesced loads) and the terms.  The results of the workgroup leave through LDS, 16 bytes wide.
 // Workgroups go to the chip's eight dies in turn, each with a cache of its own: consecutive (tile, rows) pairs are dealt out
 // so that a die sees few batch tiles, whose transposed inputs it re-reads.
 __device__ __forceinline__ int main_item() {
