@@ -3,6 +3,7 @@
 #include <cstdlib>
 #include "fwd_tile.h"
 #include "fwd_args.h"
+#include "lp_grad.h"
 #include "lp_rows.h"
 
 namespace sd {
@@ -86,12 +87,15 @@ __global__ void __launch_bounds__(256) lp_finalize_kernel(const float* __restric
     if (o >= total || gate_closed(gate, gate_limit, gate_above)) return;
     if (part1 == nullptr) {
         float s = 0.f;
+        #pragma unroll 16   // (loads in flight: 64 slices of 32 x 256 outputs 9.4 us one after the other)
         for (int k = 0; k < nsplit; k++) s += part0[(size_t)k * total + o];
         y[o] = scale ? powf(s, inv_p) * scale[o] : powf(fmaxf(s, FLT_MIN), inv_p);
     } else {
         float M = kEps;
+        #pragma unroll 8
         for (int k = 0; k < nsplit; k++) M = fmaxf(M, part1[(size_t)k * total + o]);
         float s = 0.f;
+        #pragma unroll 8
         for (int k = 0; k < nsplit; k++) {
             float Mk = part1[(size_t)k * total + o];
             s += part0[(size_t)k * total + o] * __builtin_amdgcn_exp2f(p * __builtin_amdgcn_logf(Mk / M));
@@ -640,6 +644,12 @@ __global__ void __launch_bounds__(256) lp_merge_kernel(LpMerge gx, LpMerge gw, c
     }
 }
 
+int lp_merge_planes(const float* part, float* out, size_t total, size_t plane, int planes, hipStream_t st) {
+    const LpMerge m{part, out, total, plane, planes, (unsigned)((total + 255) / 256), false};
+    hipLaunchKernelGGL(lp_merge_kernel, dim3(m.blocks), dim3(256), 0, st, m, LpMerge{}, nullptr, 0ull, 0);
+    return check_launch("lp_merge_kernel");
+}
+
 // How the general kernel's sums are cut and merged.  Sums of up to two addends have one result; more of them are merged in
 // a fixed order, from planes in the workspace, or by atomic additions in any order.
 struct LpBwdPlan {
@@ -769,6 +779,17 @@ static int lp_backward(const char* who, const float* grad_output, const float* i
     a.skip_thr = int_power(p - 1.f) < 0 ? lp_skip_threshold(1e-16f, p - 1.f, kLpSkipFrom) : 0.f;
     hipStream_t st = static_cast<hipStream_t>(stream);
     int ip = int_power(p - 1.f);
+    // whole p up to 9: from scalar registers; the general kernel below takes them only where the stream is under capture and
+    // its scratch too small for that, and gradients that are not aligned to 16 bytes
+    if (ip >= 0 && aligned16(grad_input) && aligned16(grad_weight)) {
+        const LpGradArgs b{grad_output, input, weight, output, grad_input, grad_weight, ci_idx, co_idx,
+                           f.R, HW, G, f.COg, f.CIg, f.W_COg, f.W_CIg};
+        const size_t bytes = lp_grad_workspace(b);
+        if (workspace_ready(bytes, st)) {
+            void* ws = workspace(bytes, st);
+            return ws ? lp_grad(ip, b, ws, st) : SD_ERR_HIP;
+        }
+    }
     // large p with both gradients in the dense single-group case: the kernel that forms every term once for both
     // sums and owns its grad_weight block tests significance more cheaply than the general kernel, whose
     // test only pays from a higher threshold; everything else goes through the general kernel

@@ -1,0 +1,487 @@
+// Gradients of the l-p distance (core/cuda/norm_dist_cuda.cu:261-504)
+//   u(b,m,n) = g[b,m] sgn(d) (|d| / y[b,m])^(p-1), d = x[b,n] - w[m,n];  grad_x[b,n] = sum_m u,  grad_w[m,n] = - sum_b u
+// from scalar registers: a wavefront owns 64 inputs (one per lane) and 32 rows of the batch, whose inputs and grad_x sums
+// stay in vector registers, and walks a slice of the output channels.  All that a term needs of the pair (row, channel)
+// is the same for the 64 lanes; it is laid out by tile, channel and row beforehand and read with scalar loads, 16 rows at a
+// time and one block ahead, straight into an operand of the vector instructions.
+//
+// Vector issue bounds it: 7 instructions per term at p = 8 and no LDS read, at 59 T lane instructions/s (a loop of the same
+// instructions on registers alone: 60; with the pairs (g, 1/y) read from LDS, 8 instructions and 3 wavefronts per SIMD it was 43).
+// Both gradients in us, that kernel -> this, p = 8: 512 x 5120 x 5120 2300 -> 1630, 250 x 3072 x 1021 251 -> 145, 90 x 1600 x 230
+// 36 -> 26, 32 x 192 x 192 19.4 -> 15.8; convolutions of 80 x 27 x 576 on 32 x 32 positions 1700 -> 590, of 64 x 288 x 256 on
+// 16 x 16 1000 -> 225; index lists, 512 x 3840 x 3840 of 5120 the same 1400 (16 additions per weight go to memory, 0.4 ms).
+#include <cmath>
+#include <type_traits>
+#include "fwd_args.h"
+#include "lp_grad.h"
+
+namespace sd {
+
+namespace {
+
+constexpr int RB = 32;   // batch rows of a tile (= one index-list sub-batch)
+constexpr int MC = 4;    // output channels of a chunk: their weights are loaded a chunk ahead
+constexpr int kTiles = 4;   // batch tiles of a workgroup of four wavefronts
+
+typedef float f16v __attribute__((ext_vector_type(16)));
+// memory that no kernel writes while this one runs, read at wave-uniform addresses: scalar loads
+template <class T> using Const = const __attribute__((address_space(4))) T*;
+template <class T> __device__ __forceinline__ Const<T> as_const(const void* p) { return (Const<T>)(uintptr_t)p; }
+
+// Scales of y between which d^(p-1) g y^(1-p) is formed as the product of d^(p-1) and g y^(1-p), one multiplication less per
+// term than the power of the ratio: for p - 1 <= 8 neither overflows, and a d^(p-1) that is no normal number has
+// (|d| / y)^(p-1) below 2^-56.  Chunks with an output outside form the ratio.
+constexpr float kYLow = 1.f / 256.f, kYHigh = 256.f, kGLow = 0x1p-96f, kGHigh = 0x1p+96f;
+
+struct Batch {          // the batch side as the kernel reads it
+    float* scale;       // [tile][group][channel][row]: g y^(1-p), or g in a chunk that forms ratios; 0 for rows past the batch
+    float* recip;       // the same layout: 1 / y in chunks that form ratios
+    uint32_t* ratio;    // [tile][group][chunk]: the chunk forms ratios
+};
+
+struct Args {
+    LpGradArgs a;
+    Batch s;
+    int COp;        // channels of a group, whole chunks
+    int tile0;         // first batch tile of the launch (the tables begin with it)
+    int zsplit, per;   // slices of the output channels, channels of a slice
+    size_t gx_plane;   // floats between the planes of grad_x that the slices write, 0: they add to grad_x
+    unsigned nblocks, pairs, groups;   // blocks of 64 inputs; (block, group, slice) triples; groups of WAVES batch tiles
+    int span;          // the largest power of two up to 32 and the positions per image: rows that lie side by side
+    bool by_die;       // the triples fill the eight dies evenly
+    bool gw_store;     // a workgroup holds the whole batch: its sums are grad_weight
+};
+
+// u = (first of the pair times the second) from the difference and g y^(1-p)
+template <int IP>
+__device__ __forceinline__ float2 power_pair(float d, float s) {
+    const float t2 = d * d;
+    switch (IP) {
+        case 0: return make_float2(d >= 0.f ? s : -s, 1.f);
+        case 1: return make_float2(s, d);
+        case 2: return make_float2(fabsf(d) * s, d);
+        case 3: return make_float2(d * s, t2);
+        case 4: return make_float2(fabsf(d) * s, t2 * d);
+        case 5: return make_float2(d * s, t2 * t2);
+        case 6: { const float t3 = t2 * d; return make_float2(fabsf(t3) * s, t3); }
+        case 7: return make_float2(t2 * d * s, t2 * t2);
+        default: { const float t3 = t2 * d; return make_float2(fabsf(t3) * s, t3 * t2); }
+    }
+}
+
+template <int IP>
+__device__ __forceinline__ float ratio_power(float sr) {
+    const float t = sr * sr;
+    switch (IP) {
+        case 0: return sr >= 0.f ? 1.f : -1.f;
+        case 1: return sr;
+        case 2: return fabsf(sr) * sr;
+        case 3: return sr * t;
+        case 4: return fabsf(sr) * sr * t;
+        case 5: return sr * t * t;
+        case 6: return fabsf(sr) * sr * t * t;
+        case 7: return sr * t * t * t;
+        default: return fabsf(sr) * sr * t * (t * t);
+    }
+}
+
+// ---- batch side ---------------------------------------------------------------------------------------------------
+// A workgroup lays out 32 rows x 64 channels; workgroups behind those clear grad_weight and, where slices add to it, grad_x.
+template <int IP>
+__global__ void __launch_bounds__(256) lp_grad_batch_kernel(Args k, float* __restrict__ zero0, size_t zero0_n,
+                                                            float* __restrict__ zero1, size_t zero1_n, unsigned fill_from) {
+    const LpGradArgs& a = k.a;
+    const int tid = threadIdx.x;
+    if (blockIdx.x >= fill_from) {
+        const size_t step = (size_t)(gridDim.x - fill_from) * 256, i0 = (size_t)(blockIdx.x - fill_from) * 256 + tid;
+        for (size_t i = i0; i < zero0_n / 4; i += step) reinterpret_cast<float4*>(zero0)[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (size_t i = i0 + zero0_n / 4 * 4; i < zero0_n; i += step) zero0[i] = 0.f;
+        for (size_t i = i0; i < zero1_n / 4; i += step) reinterpret_cast<float4*>(zero1)[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (size_t i = i0 + zero1_n / 4 * 4; i < zero1_n; i += step) zero1[i] = 0.f;
+        return;
+    }
+    __shared__ float gs[RB][65], ys[RB][65];
+    const unsigned cols = (unsigned)(k.COp + 63) / 64;
+    const int c = blockIdx.x % cols, g = (blockIdx.x / cols) % a.G, t = blockIdx.x / cols / a.G;
+    const int r0 = (k.tile0 + t) * RB, m0 = c * 64;
+    // neighbouring work-items read neighbouring channels (one position per image) or rows
+    #pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const int f = tid + 256 * e, i = a.HW == 1 ? f / 64 : f % RB, j = a.HW == 1 ? f % 64 : f / RB;
+        const int r = r0 + i, m = m0 + j;
+        float gv = 0.f, yv = 1.f;
+        if (r < a.R && m < a.COg) {
+            const int b = a.HW == 1 ? r : r / a.HW, hw = r - b * a.HW;
+            const size_t o = ((size_t)(b * a.G + g) * a.COg + m) * a.HW + hw;
+            gv = a.gy[o];
+            yv = a.y[o];
+        }
+        gs[i][j] = gv;
+        ys[i][j] = yv;
+    }
+    __syncthreads();
+    // a work-item owns four rows of two channels; eight of them make a channel, 32 a chunk
+    const size_t base = ((size_t)t * a.G + g) * k.COp;
+    const int i0 = (tid & 7) * 4;
+    #pragma unroll
+    for (int e = 0; e < 2; e++) {
+        const int j = (tid >> 3) + 32 * e, m = m0 + j;
+        float s[4], yv[4], gv[4];
+        bool bad = false;
+        #pragma unroll
+        for (int i = 0; i < 4; i++) {
+            gv[i] = gs[i0 + i][j]; yv[i] = ys[i0 + i][j];
+            if (IP > 0) {
+                const double v = 1.0 / (double)yv[i], v2 = v * v, v4 = v2 * v2;
+                double pw = IP & 1 ? v : 1.0;
+                if (IP & 2) pw *= v2;
+                if (IP & 4) pw *= v4;
+                if (IP & 8) pw *= v4 * v4;
+                s[i] = (float)((double)gv[i] * pw);
+                const float size = fabsf(s[i]);
+                bad |= !(yv[i] >= kYLow && yv[i] <= kYHigh) || !(gv[i] == 0.f || (size >= kGLow && size <= kGHigh));
+            } else s[i] = gv[i];
+        }
+        const bool ratio = ((__builtin_amdgcn_ballot_w64(bad) >> (threadIdx.x & 32)) & 0xffffffffull) != 0ull;
+        if (m < k.COp) {
+            float* dst = k.s.scale + (base + m) * RB + i0;
+            *reinterpret_cast<float4*>(dst) = ratio ? make_float4(gv[0], gv[1], gv[2], gv[3]) : make_float4(s[0], s[1], s[2], s[3]);
+            if (ratio) *reinterpret_cast<float4*>(k.s.recip + (base + m) * RB + i0) =
+                make_float4(1.f / yv[0], 1.f / yv[1], 1.f / yv[2], 1.f / yv[3]);
+            if ((threadIdx.x & 31) == 0) k.s.ratio[(base + m) / MC] = ratio ? 1u : 0u;
+        }
+    }
+}
+
+// ---- terms --------------------------------------------------------------------------------------------------------
+// rows i0 .. i0 + 15 of one channel; `rest` is called behind the first row, when the loads before have arrived
+template <int IP, bool GW, class Rest>
+__device__ __forceinline__ void product_rows(const float* xr, float* acc, float (&ws)[2], f16v s, float wk, Rest rest) {
+    #pragma unroll
+    for (int i = 0; i < 16; i++) {
+        const float2 f = power_pair<IP>(xr[i] - wk, s[i]);
+        acc[i] = fmaf(f.x, f.y, acc[i]);
+        asm volatile("" : "+v"(acc[i]));   // added here: put off behind the chunk, the factors of 128 rows would spill
+        if (GW) ws[i & 1] = fmaf(f.x, f.y, ws[i & 1]);
+        if (i == 0) { __builtin_amdgcn_sched_barrier(0); rest(); }
+        if (i % 4 == 0) __builtin_amdgcn_sched_barrier(0);   // more rows at once would take the registers of a fourth wavefront
+    }
+}
+// WAVES = kTiles: the wavefronts of a workgroup take neighbouring batch tiles of the same inputs and their sums of grad_weight
+// meet in LDS, so that memory sees one addition per 128 rows.  WAVES = 1: a workgroup is one wavefront.  STRIDED: several positions per
+// image, whose inputs are not side by side in a row.  LISTS: index lists on either side.
+template <int IP, bool GW, int WAVES, bool STRIDED, bool LISTS>
+__global__ void __launch_bounds__(64 * WAVES, 4) lp_grad_kernel(Args k) {
+    const LpGradArgs& a = k.a;
+    // the tile on its way between memory and registers where a row's inputs are strided; then sums of grad_weight
+    constexpr int TS = 65;
+    __shared__ float lds[WAVES][STRIDED ? RB * TS : 2 * MC * 64];
+    static_assert(2 * MC * 64 <= RB * TS, "both halves of the sums fit");
+    const int lane = threadIdx.x & 63, wave = WAVES > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+    // all batch tiles of a (block of inputs, slice) run on one die one after the other: they share its weights there
+    const unsigned pair = k.by_die ? blockIdx.x % 8 + 8 * (blockIdx.x / 8 / k.groups) : blockIdx.x % k.pairs;
+    const unsigned group = k.by_die ? blockIdx.x / 8 % k.groups : blockIdx.x / k.pairs;
+    if (pair >= k.pairs) return;
+    const int nblock = pair % k.nblocks, g = pair / k.nblocks % a.G, slice = pair / k.nblocks / a.G;
+    const int m_lo = slice * k.per, m_hi = m_lo + k.per < a.COg ? m_lo + k.per : a.COg;
+    if (m_lo >= m_hi) return;
+    const int tile = (int)group * WAVES + wave, r0 = (k.tile0 + tile) * RB;
+    const int n = nblock * 64 + lane;
+    const bool n_ok = n < a.CIg;
+    const int nc = n_ok ? n : a.CIg - 1;
+    int rows = a.R - r0;
+    rows = rows < 0 ? 0 : rows > RB ? RB : rows;
+    const int last = rows > 0 ? rows - 1 : 0, rx = rows > 0 ? r0 : 0;   // rows past the batch repeat one, with g = 0
+    const int sub = (rx / a.HW) / kSubBatch;   // (one tile to a sub-batch where there are index lists)
+
+    const int wcol = a.ci_idx ? a.ci_idx[(sub * a.G + g) * a.CIg + nc] : nc;
+    const float* __restrict__ wbase = a.w + (size_t)g * a.W_COg * a.W_CIg + wcol;
+    float* __restrict__ gwbase = GW ? a.gw + (size_t)g * a.W_COg * a.W_CIg + wcol : nullptr;
+    // weight rows of the channels from m on, inside the slice; LISTS: fetched ahead, one per lane
+    const int* __restrict__ co = LISTS && a.co_idx ? a.co_idx + (size_t)(sub * a.G + g) * a.COg : nullptr;
+    auto rows_of = [&](int m) {
+        m += lane & (MC - 1);
+        m = m < m_hi ? m : m_hi - 1;
+        return LISTS && co ? co[m] : m;
+    };
+    auto row_of = [&](int m0, int j, int rows) {
+        if (LISTS) return __builtin_amdgcn_readlane(rows, j);
+        return m0 + j < m_hi ? m0 + j : m_hi - 1;
+    };
+
+    // where row i of the tile begins, in lane i (the tensors hold fewer than 2^31 values)
+    const int rl = rx + ((lane & (RB - 1)) < last ? (lane & (RB - 1)) : last);
+    const int begin = ((rl / a.HW) * a.G + g) * a.CIg * a.HW + rl % a.HW;
+
+    // step t of a walk over the tile as memory holds it where a row's inputs are strided: `span` rows side by side, then the
+    // next inputs; the row and the input of this lane
+    auto strided = [&](int t) {
+        const int per = RB / k.span;
+        return make_int2((lane & (k.span - 1)) + k.span * (t % per), lane / k.span + 64 / k.span * (t / per));
+    };
+
+    const size_t base = ((size_t)tile * a.G + g) * k.COp;
+    const Const<float> scale = as_const<float>(k.s.scale + base * RB), recip = as_const<float>(k.s.recip + base * RB);
+    const Const<uint32_t> ratio = as_const<uint32_t>(k.s.ratio + base / MC);
+    const uint32_t* modes = k.s.ratio + base / MC;
+    const int c_hi = (m_hi + MC - 1) / MC;
+    uint32_t mode = m_lo / MC + lane < c_hi ? modes[m_lo / MC + lane] : 0u;
+
+    float xr[RB], acc[RB];
+    if constexpr (STRIDED) {
+        #pragma unroll
+        for (int t = 0; t < RB; t++) {
+            const int2 at = strided(t);
+            const int c = nblock * 64 + at.y < a.CIg ? nblock * 64 + at.y : a.CIg - 1;
+            xr[t] = (a.x + __shfl(begin, at.x))[(unsigned)c * (unsigned)a.HW];
+        }
+        #pragma unroll
+        for (int t = 0; t < RB; t++) { const int2 at = strided(t); lds[wave][at.x * TS + at.y] = xr[t]; }
+        #pragma unroll
+        for (int i = 0; i < RB; i++) { xr[i] = lds[wave][i * TS + lane]; acc[i] = 0.f; }
+        if (WAVES > 1) __syncthreads();
+    } else {
+        #pragma unroll
+        for (int i = 0; i < RB; i++) {
+            xr[i] = (a.x + __builtin_amdgcn_readlane(begin, i))[(unsigned)nc];
+            acc[i] = 0.f;
+            if (i % 8 == 7) __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+
+    const int m_end = k.COp;   // channels that the tables hold
+    auto block = [&](int m, int i0) { return *(Const<f16v>)(scale + (size_t)m * RB + i0); };
+
+    int rowv = LISTS ? rows_of(m_lo) : 0, rown = LISTS ? rows_of(m_lo + MC) : 0;
+    float wv[MC];
+    #pragma unroll
+    for (int j = 0; j < MC; j++) wv[j] = wbase[(size_t)row_of(m_lo, j, rowv) * a.W_CIg];
+    // a slice without a chunk that forms ratios runs the loop without that path, which would cost it copies of its sums
+    for (int c = m_lo / MC + 64 + lane; c < c_hi; c += 64) mode |= modes[c];
+    const bool ratios = __builtin_amdgcn_ballot_w64(mode != 0u) != 0ull;
+
+    auto add_weight = [&](int row, float v) {
+        float* dst = gwbase + (size_t)row * a.W_CIg;
+        if (k.gw_store) *dst = v;
+        else unsafeAtomicAdd(dst, v);
+    };
+
+    auto walk = [&](auto mixed) {
+        constexpr bool MIXED = decltype(mixed)::value;
+        int buf = 0;
+        for (int m0 = m_lo; m0 < m_hi; m0 += MC, buf ^= 1) {
+            float wn[MC];
+            #pragma unroll
+            for (int j = 0; j < MC; j++) wn[j] = wbase[(size_t)row_of(m0 + MC, j, rown) * a.W_CIg];
+            float sum[MC] = {};
+            if constexpr (!MIXED) {
+                f16v s0 = block(m0, 0);
+                float next = 0.f;   // brings the next chunk's first block as far as the scalar cache
+                #pragma unroll
+                for (int j = 0; j < MC; j++) {
+                    float ws[2] = {0.f, 0.f};
+                    f16v s1;
+                    product_rows<IP, GW>(xr, acc, ws, s0, wv[j], [&] { s1 = block(m0 + j, 16); });
+                    product_rows<IP, GW>(xr + 16, acc + 16, ws, s1, wv[j], [&] {
+                        if (j + 1 < MC) s0 = block(m0 + j + 1, 0);
+                        else next = scale[(size_t)(m0 + MC < m_end ? m0 + MC : m0) * RB];
+                    });
+                    sum[j] = ws[0] + ws[1];
+                    asm volatile("" : "+v"(sum[j]));
+                }
+                asm volatile("" :: "s"(next));
+            } else {
+                // rare: row by row, with few registers; elsewhere d^(p-1) is the power of a "ratio" d * 1
+                const bool form = ratio[m0 / MC] != 0u;
+                float w0 = wv[0], w1 = wv[1], w2 = wv[2], w3 = wv[3];
+                static_assert(MC == 4, "the weights and sums of a chunk are passed round by hand");
+                #pragma unroll 1
+                for (int j = 0; j < MC; j++) {
+                    const float wk = w0;
+                    float ws = 0.f;
+                    #pragma unroll
+                    for (int i = 0; i < RB; i++) {
+                        if (i < rows && m0 + j < m_hi) {   // rows past the batch count nothing, whatever the operands
+                            const float gv = scale[(size_t)(m0 + j) * RB + i], ry = form ? recip[(size_t)(m0 + j) * RB + i] : 1.f;
+                            const float pw = ratio_power<IP>((xr[i] - wk) * ry);
+                            acc[i] = fmaf(gv, pw, acc[i]);
+                            ws = fmaf(gv, pw, ws);
+                        }
+                        asm volatile("" : "+v"(acc[i]), "+v"(ws));
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    w0 = w1; w1 = w2; w2 = w3; w3 = wk;
+                    sum[0] = sum[1]; sum[1] = sum[2]; sum[2] = sum[3]; sum[3] = ws;
+                }
+            }
+            if (GW && WAVES > 1) {
+                #pragma unroll
+                for (int j = 0; j < MC; j++) lds[wave][(buf * MC + j) * 64 + lane] = sum[j];
+                __syncthreads();   // the other half is written behind the next barrier but one
+            }
+            // the next weights have arrived before the additions below are queued: waiting for them later would wait for these
+            #pragma unroll
+            for (int j = 0; j < MC; j++) { asm volatile("" : "+v"(wn[j])); wv[j] = wn[j]; }
+            if (GW && WAVES > 1) {
+                static_assert(WAVES == 1 || WAVES == MC, "a wavefront adds up one channel of the chunk");
+                float v = 0.f;
+                #pragma unroll
+                for (int j = 0; j < WAVES; j++) v += lds[j][(buf * MC + wave) * 64 + lane];
+                if (n_ok && m0 + wave < m_hi) add_weight(m0 + wave, -v);
+            } else if (GW) {
+                #pragma unroll
+                for (int j = 0; j < MC; j++)
+                    if (n_ok && m0 + j < m_hi) add_weight(row_of(m0, j, rowv), -sum[j]);
+            }
+            if (LISTS) { rowv = rown; rown = rows_of(m0 + 2 * MC); }
+        }
+    };
+    if (ratios) walk(std::true_type{});
+    else walk(std::false_type{});
+    // what only the end needs is read again here: it would take scalar registers all the way
+    Const<Args> late = (Const<Args>)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(late));
+    float* gx = late->a.gx + (size_t)slice * late->gx_plane;
+    const bool add = late->zsplit > 1 && late->gx_plane == 0;
+    if constexpr (STRIDED) {
+        if (WAVES > 1) __syncthreads();
+        #pragma unroll
+        for (int i = 0; i < RB; i++) lds[wave][i * TS + lane] = acc[i];
+        #pragma unroll 8
+        for (int t = 0; t < RB; t++) {
+            const int2 at = strided(t);
+            float* dst = gx + __shfl(begin, at.x) + (unsigned)(nblock * 64 + at.y) * (unsigned)a.HW;
+            const float v = lds[wave][at.x * TS + at.y];
+            if (at.x >= rows || nblock * 64 + at.y >= a.CIg) continue;
+            if (add) unsafeAtomicAdd(dst, v);
+            else *dst = v;
+        }
+    } else if (n_ok) {
+        #pragma unroll
+        for (int i = 0; i < RB; i++) {
+            if (i < rows) {
+                float* dst = gx + __builtin_amdgcn_readlane(begin, i) + (unsigned)n;
+                if (add) unsafeAtomicAdd(dst, acc[i]);
+                else *dst = acc[i];
+            }
+            if (i % 8 == 7) __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+}
+
+struct Plan {
+    int waves, zsplit, per;
+    int tiles, launch_tiles;   // batch tiles, whole workgroups of them; of one launch
+    size_t words, plane;       // floats of a launch's table (each of the two); of a plane of grad_x, 0: no planes
+    size_t bytes;
+};
+
+size_t align256(size_t b) { return (b + 255) / 256 * 256; }
+
+Plan make_plan(const LpGradArgs& a) {
+    Plan p{};
+    const int real = (a.R + RB - 1) / RB, nb = (a.CIg + 63) / 64, COp = (a.COg + MC - 1) / MC * MC;
+    const int whole = (real + kTiles - 1) / kTiles * kTiles;
+    const bool lists = a.ci_idx || a.co_idx;
+    const long long waves = (long long)nb * real * a.G;   // before the output channels are cut
+    p.waves = !lists && a.gw && whole * 8 <= real * 9 && waves >= 4ll * num_cus() ? kTiles : 1;
+    p.tiles = p.waves > 1 ? whole : real;
+    // the device holds four wavefronts per SIMD: the slice count whose last round of them is fullest, a smaller one unless a
+    // larger gains 3 %, slices of at least 64 channels
+    const double slots = 16.0 * num_cus();
+    double best = 0.0;
+    p.zsplit = 1;
+    for (int z = 1; z <= 16 && (z == 1 || a.COg / z >= 64); z++) {
+        const double rounds = (double)nb * p.tiles * a.G * z / slots, eff = rounds / std::ceil(rounds);
+        if (eff > best * 1.03) { best = eff; p.zsplit = z; }
+    }
+    // small layers: slices down to one chunk until every SIMD has two wavefronts; their sums are merged in slice order
+    const long long fill = 8ll * num_cus();
+    bool planes = false;
+    if (waves * p.zsplit < fill && aligned16(a.gx)) {
+        const long long more = (fill + waves - 1) / waves, most = COp / MC;
+        p.zsplit = (int)(more < most ? more : most);
+        planes = p.zsplit > 2;
+    }
+    p.per = ((a.COg + p.zsplit - 1) / p.zsplit + MC - 1) / MC * MC;
+    p.zsplit = (a.COg + p.per - 1) / p.per;
+    if (planes && p.zsplit > 2) p.plane = ((size_t)a.R * a.G * a.CIg + 3) / 4 * 4;
+    // tables of at most 128 MB each: a larger batch is taken in several launches
+    const size_t tile_words = (size_t)a.G * COp * RB;
+    size_t most = ((size_t)1 << 25) / tile_words / kTiles * kTiles;
+    if (most < (size_t)kTiles) most = kTiles;
+    p.launch_tiles = (size_t)p.tiles > most ? (int)most : p.tiles;
+    p.words = tile_words * p.launch_tiles;
+    p.bytes = align256(p.words * 4) * 2 + align256(p.words / RB / MC * 4) + p.plane * p.zsplit * 4;
+    return p;
+}
+
+template <int IP, bool STRIDED>
+void launch_tiles(const Args& k, int waves, dim3 grid, hipStream_t st) {
+    if (k.a.ci_idx || k.a.co_idx) {
+        if (k.a.gw) hipLaunchKernelGGL((lp_grad_kernel<IP, true, 1, STRIDED, true>), grid, dim3(64), 0, st, k);
+        else hipLaunchKernelGGL((lp_grad_kernel<IP, false, 1, STRIDED, true>), grid, dim3(64), 0, st, k);
+    } else if (waves > 1) hipLaunchKernelGGL((lp_grad_kernel<IP, true, kTiles, STRIDED, false>), grid, dim3(64 * kTiles), 0, st, k);
+    else if (k.a.gw) hipLaunchKernelGGL((lp_grad_kernel<IP, true, 1, STRIDED, false>), grid, dim3(64), 0, st, k);
+    else hipLaunchKernelGGL((lp_grad_kernel<IP, false, 1, STRIDED, false>), grid, dim3(64), 0, st, k);
+}
+
+template <int IP>
+int launch(Args& k, const Plan& p, float* part, hipStream_t st) {
+    LpGradArgs& a = k.a;
+    float* const gx = a.gx;
+    const size_t nx = (size_t)a.R * a.G * a.CIg, nw = a.gw ? (size_t)a.G * a.W_COg * a.W_CIg : 0;
+    int rc;
+    if (part) { a.gx = part; k.gx_plane = p.plane; }
+    for (k.tile0 = 0; k.tile0 < p.tiles; k.tile0 += p.launch_tiles) {
+        const int tiles = p.tiles - k.tile0 < p.launch_tiles ? p.tiles - k.tile0 : p.launch_tiles;
+        const unsigned lay = (unsigned)((k.COp + 63) / 64) * a.G * tiles;
+        k.groups = (unsigned)(tiles / p.waves);
+        k.gw_store = !a.ci_idx && !a.co_idx && tiles == p.tiles && k.groups == 1;
+        const size_t z0 = k.tile0 == 0 && k.zsplit > 1 && !part ? nx : 0, z1 = k.tile0 == 0 && !k.gw_store ? nw : 0;
+        size_t fill = ((z0 > z1 ? z0 : z1) / 4 + 255) / 256;
+        if (z0 + z1 && fill == 0) fill = 1;
+        if (fill > 16u * num_cus()) fill = 16u * num_cus();
+        hipLaunchKernelGGL((lp_grad_batch_kernel<IP>), dim3(lay + (unsigned)fill), dim3(256), 0, st, k, a.gx, z0, a.gw, z1, lay);
+        if ((rc = check_launch("lp_grad_batch_kernel"))) return rc;
+        const dim3 grid((k.by_die ? (k.pairs + 7) / 8 * 8 : k.pairs) * k.groups);
+        if (a.HW > 1) launch_tiles<IP, true>(k, p.waves, grid, st);
+        else launch_tiles<IP, false>(k, p.waves, grid, st);
+        if ((rc = check_launch("lp_grad_kernel"))) return rc;
+    }
+    return part ? lp_merge_planes(part, gx, nx, p.plane, k.zsplit, st) : SD_OK;
+}
+
+}  // namespace
+
+size_t lp_grad_workspace(const LpGradArgs& a) { return make_plan(a).bytes; }
+
+int lp_grad(int ip, const LpGradArgs& a, void* ws, hipStream_t st) {
+    const Plan p = make_plan(a);
+    Args k{};
+    k.a = a;
+    k.COp = (a.COg + MC - 1) / MC * MC;
+    k.zsplit = p.zsplit; k.per = p.per;
+    k.nblocks = (unsigned)(a.CIg + 63) / 64;
+    k.pairs = k.nblocks * a.G * k.zsplit;
+    k.by_die = (k.pairs + 7) / 8 * 8 * 32 <= k.pairs * 33;
+    for (k.span = 1; k.span < RB && k.span * 2 <= a.HW; ) k.span *= 2;
+    char* at = static_cast<char*>(ws);
+    k.s.scale = reinterpret_cast<float*>(at); at += align256(p.words * 4);
+    k.s.recip = reinterpret_cast<float*>(at); at += align256(p.words * 4);
+    k.s.ratio = reinterpret_cast<uint32_t*>(at); at += align256(p.words / RB / MC * 4);
+    float* part = p.plane ? reinterpret_cast<float*>(at) : nullptr;
+    switch (ip) {
+        case 0: return launch<0>(k, p, part, st);
+        case 1: return launch<1>(k, p, part, st);
+        case 2: return launch<2>(k, p, part, st);
+        case 3: return launch<3>(k, p, part, st);
+        case 4: return launch<4>(k, p, part, st);
+        case 5: return launch<5>(k, p, part, st);
+        case 6: return launch<6>(k, p, part, st);
+        case 7: return launch<7>(k, p, part, st);
+        default: return launch<8>(k, p, part, st);
+    }
+}
+
+}  // namespace sd

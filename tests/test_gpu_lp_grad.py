@@ -1,0 +1,67 @@
+"""Gradients of the l-p distance at whole p up to 9 (sd_norm_dist_backward_input[_weight]) where their kernel can go wrong:
+tiles of 32 rows and 64 inputs and chunks of 4 channels that are not whole, positions side by side in runs of every length,
+slices merged from planes, batches of several workgroups' tiles, and outputs too small or too large to be raised to the power
+p - 1 by themselves, next to ordinary ones.  Sums of fp32 products in any order: relative error 1e-5 of the largest entry."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(got, want):
+    np.testing.assert_allclose(got.cpu().numpy(), want, rtol=1e-5, atol=1e-5 * np.abs(want).max())
+
+
+def _both(oracle, x, w, gy, p, G=1, ci=None, co=None):
+    from sortnet_amd import ext
+    lists = ci is not None
+    n = lambda t: None if t is None else t.numpy()   # noqa: E731
+    ry = oracle.norm_dist_forward(x.numpy(), w.numpy(), p, G, n(ci), n(co))
+    rgx, rgw = oracle.norm_dist_backward(gy.numpy(), x.numpy(), w.numpy(), ry, p, G, True, n(ci), n(co))
+    dev = torch.device("cuda:0")
+    xd, wd, gd, yd = x.to(dev), w.to(dev), gy.to(dev), torch.from_numpy(ry).to(dev)
+    lists = (ci.to(dev), co.to(dev)) if lists else (None, None)
+    gx, gw, gi = torch.full_like(xd, 7), torch.full_like(wd, 7), torch.full_like(xd, 7)
+    ext.norm_dist_backward_input_weight(gd, xd, wd, yd, gx, gw, G, p, *lists)
+    ext.norm_dist_backward_input(gd, xd, wd, yd, gi, G, p, *lists)
+    _check(gx, rgx)
+    _check(gw, rgw)
+    _check(gi, rgx)
+
+
+@pytest.mark.parametrize("p", [2.0, 7.0, 8.0, 9.0])
+@pytest.mark.parametrize("B,N,M,G,HW", [
+    (1, 1, 1, 1, 1), (33, 65, 5, 1, 1), (130, 700, 67, 1, 1), (31, 64, 1021, 1, 1), (160, 512, 130, 2, 1), (3, 27, 17, 1, 49),
+    (20, 75, 33, 1, 3), (9, 144, 20, 1, 40), (40, 130, 12, 2, 2), (2, 27, 48, 1, 1024), (129, 2048, 260, 1, 1)])
+def test_edges_of_tiles(oracle, p, B, N, M, G, HW):
+    g = torch.Generator().manual_seed(B * 7 + N)
+    x, gy = torch.randn(B, N * G, HW, generator=g), torch.randn(B, M * G, HW, generator=g)
+    _both(oracle, x, torch.randn(M * G, N, generator=g) * 0.4, gy, p, G)
+
+
+@pytest.mark.parametrize("p", [2.0, 8.0, 9.0])
+@pytest.mark.parametrize("HW", [1, 5])
+def test_outputs_of_any_scale(oracle, p, HW):
+    """Rows and channels from 1e-4 to 1e4 times the ordinary scale: chunks that form ratios beside chunks that form products."""
+    g = torch.Generator().manual_seed(3)
+    B, N, M = 70, 130, 44
+    scale = torch.ones(B, 1, 1)
+    scale[5], scale[40:43], scale[69] = 1e-4, 1e4, 1e-3
+    x, gy = torch.randn(B, N, HW, generator=g) * scale, torch.randn(B, M, HW, generator=g)
+    w = torch.randn(M, N, generator=g) * 1e-5
+    w[9], w[20:22] = 1e4, 300.0
+    gy[:, 13] = 0
+    _both(oracle, x, w, gy, p)
+    gy[:, 30] *= 1e-30
+    _both(oracle, x[:33].contiguous(), w, gy[:33].contiguous(), p)
+
+
+@pytest.mark.parametrize("B,N,M,kn,km,G,HW", [(70, 96, 64, 67, 21, 1, 1), (33, 130, 44, 100, 33, 2, 1), (64, 40, 24, 27, 9, 1, 3)])
+def test_index_lists(oracle, B, N, M, kn, km, G, HW):
+    g = torch.Generator().manual_seed(B)
+    keep = lambda c, k: torch.rand(-(-B // 32), G, c, generator=g).argsort(-1)[..., :k].sort(-1)[0].to(torch.int32).contiguous()   # noqa: E731
+    ci, co = keep(N, kn), keep(M, km)
+    x, gy = torch.randn(B, kn * G, HW, generator=g), torch.randn(B, km * G, HW, generator=g)
+    for p in (3.0, 8.0):
+        _both(oracle, x, torch.randn(M * G, N, generator=g), gy, p, G, ci, co)
