@@ -12,6 +12,12 @@
 //   many) go to LDS, one term per lane, are ranked against each other and added up in the order of the other kernels
 //   (largest first, every product rounded on its own), so the result has the same bits.
 // More than 16 such groups, or more than 64 such terms (many equal terms): slower exact paths of the same kernel.
+//
+// The selection bounds it from about three batch rows on, the weights below.  It starts at the bits that all lane maxima share, ranks up
+// to 16 terms in one step of 64 lanes and weighs every term in its own lane; a pass reads at most four groups of a staged row ahead, so
+// that rows of 5120 inputs leave room for four wavefronts per SIMD (three, an odd number, issue at three quarters of the rate) and rows of
+// 3072 for six.  K = 10, us, before -> now: 1 x 5120 x 5120 28.8 -> 23.4 (4.5 TB/s), 8 x 5120 x 5120 103 -> 81, 33 x 1658 x 1658 83 -> 61,
+// 64 x 640 x 640 38 -> 28, 256 x 10240 x 10 31 -> 19; intervals 8 x 5120 x 5120 225 -> 162.
 #include "fwd_tile.h"
 #include "row_stream.h"
 
@@ -24,9 +30,13 @@ enum StreamOp { kStreamMax, kStreamPos, kStreamSort };
 constexpr int stream_waves(StreamOp op) { return op == kStreamSort ? 4 : 8; }
 
 // wavefronts per SIMD that the registers are to leave room for, and how many to count on (rows of up to 1024 inputs leave room for
-// twice as many)
-constexpr int stream_occupancy(int NE, StreamOp op) { return NE <= 48 ? 4 : NE <= 80 ? (op == kStreamSort ? 3 : 4) : (op == kStreamSort ? 1 : 2); }
-constexpr int stream_resident(int NE, int NX, StreamOp op) { return NE <= 16 ? (NX == 2 && op == kStreamPos ? 7 : 8) : stream_occupancy(NE, op); }
+// twice as many; the staged ends of intervals leave room for fewer)
+constexpr int stream_occupancy(int NE, int NX, StreamOp op) { return NE == 48 && NX == 1 && op == kStreamSort ? 6 : NE <= 80 ? 4 : 2; }
+constexpr int stream_resident(int NE, int NX, StreamOp op) {
+    if (NE <= 16) return NX == 2 && op == kStreamPos ? 7 : 8;
+    if (NX == 2 && op == kStreamSort && NE > 48) return NE <= 80 ? 3 : 1;
+    return stream_occupancy(NE, NX, op);
+}
 
 // maximum over the wavefront, in every lane (row-wise shifts, then the two row broadcasts; v >= 0)
 __device__ __forceinline__ float wave_max(float v) {
@@ -41,6 +51,14 @@ __device__ __forceinline__ float wave_max(float v) {
 #undef SD_DPP_MAX
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
+// the minimum of values that are not negative: the maximum of their complements
+__device__ __forceinline__ float wave_min(float v) {
+    uint32_t u = ~__float_as_uint(v);
+#define SD_DPP_MAX(ctrl, rows) { const uint32_t t = __builtin_amdgcn_update_dpp(u, u, ctrl, rows, 0xf, false); u = t > u ? t : u; }
+    SD_DPP_MAX(0x111, 0xf) SD_DPP_MAX(0x112, 0xf) SD_DPP_MAX(0x114, 0xf) SD_DPP_MAX(0x118, 0xf) SD_DPP_MAX(0x142, 0xa) SD_DPP_MAX(0x143, 0xc)
+#undef SD_DPP_MAX
+    return __uint_as_float(~(uint32_t)__builtin_amdgcn_readlane(u, 63));
+}
 
 __device__ __forceinline__ int lanes_below(unsigned long long mask) {
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
@@ -54,7 +72,7 @@ __device__ __forceinline__ void wave_fence() { __builtin_amdgcn_wave_barrier(); 
 // NX = 1: terms |x - w|.  NX = 2: interval bounds, terms -min(w - l, u - w) for the lower (side 0) and
 // max(w - l, u - w) for the upper result (side 1), inverted intervals repaired as everywhere.
 template <int NE, bool VEC, int NX, StreamOp OP>
-__global__ void __launch_bounds__(64 * stream_waves(OP), stream_occupancy(NE, OP))
+__global__ void __launch_bounds__(64 * stream_waves(OP), stream_occupancy(NE, NX, OP))
 row_stream_kernel(FwdArgs a, int K) {
     constexpr int NG = NE / 4, kWaves = stream_waves(OP);
     constexpr bool MASKABLE = NX == 1 && OP != kStreamSort;
@@ -106,7 +124,9 @@ row_stream_kernel(FwdArgs a, int K) {
     // The staged rows stay in LDS between the passes: keeps the compiler from holding what one pass read in registers for
     // the next, and (every few groups) from starting a whole pass's reads at once
     auto pass_fence = []() { asm volatile("" ::: "memory"); };
-    auto group_fence = [](int e) { if (NX == 2 && e % 2 == 1) { asm volatile("" ::: "memory"); __builtin_amdgcn_sched_barrier(0); } };
+    auto group_fence = [](int e) {
+        if (NX == 2 ? e % 2 == 1 : OP == kStreamSort && NE >= 48 && e % 4 == 3) { asm volatile("" ::: "memory"); __builtin_amdgcn_sched_barrier(0); }
+    };
     auto load4 = [&](const float* row, int e, float (&x)[4]) {
         if (VEC) {
             const float4 t = *reinterpret_cast<const float4*>(&row[4 * (64 * e + lane)]);
@@ -131,6 +151,11 @@ row_stream_kernel(FwdArgs a, int K) {
             }
         }
     };
+
+    float coef = 1.f, rest = 1.f;                      // weight of the lane's term, what is left behind the K-th
+    if (OP == kStreamSort) {
+        for (int k = 0; k < K; k++) { coef = lane == k ? rest : coef; rest *= 1.f - a.q; }
+    }
 
     const int r_lo = (int)((long long)blockIdx.y * a.R / gridDim.y), r_hi = (int)((long long)(blockIdx.y + 1) * a.R / gridDim.y);
     for (int r = r_lo; r < r_hi; r++) {
@@ -238,7 +263,14 @@ row_stream_kernel(FwdArgs a, int K) {
             // lower bound of the K-th largest term: the largest bit pattern that K lane maxima reach (their order as
             // numbers is their order as integers), or a smaller one that exactly K reach
             uint32_t bits = 0u;
-            for (int bit = 30; bit >= 0; bit--) {
+            int bit = 30;
+            if (K <= 64) {                             // the bits that all lane maxima share
+                const uint32_t hi = __float_as_uint(wave_max(top)), diff = hi ^ __float_as_uint(wave_min(top));
+                bit = 31 - __builtin_clz(diff | 1u);
+                bits = hi >> (bit + 1) << (bit + 1);
+                if (diff == 0u) { bits = hi; bit = -1; }
+            }
+            for (; bit >= 0; bit--) {
                 const uint32_t t = bits | (1u << bit);
                 const int reach = __builtin_popcountll(__builtin_amdgcn_ballot_w64(__float_as_uint(top) >= t));
                 if (reach < K) continue;
@@ -246,24 +278,21 @@ row_stream_kernel(FwdArgs a, int K) {
                 if (reach == K) break;
             }
             const float T = __uint_as_float(bits > 0u ? bits : 1u);   // fewer than K positive lane maxima: every positive term
-            int groups = 0;
+            int groups = 0, count = 0;                 // groups that reach T, more than 16 of them: not all of them kept
             #pragma unroll
-            for (int e = 0; e < NG; e++) groups += __builtin_popcountll(__builtin_amdgcn_ballot_w64(gm[e] >= T));
-            int count = 0;
-            if (groups <= 16) {
-                int at = 0;
-                #pragma unroll
-                for (int e = 0; e < NG; e++) {
-                    const unsigned long long any = __builtin_amdgcn_ballot_w64(gm[e] >= T);
-                    if (any == 0ull) continue;
-                    if (gm[e] >= T) {
-                        float v[4];
-                        bool flag[4];
-                        terms(side, e, v, flag);
-                        *reinterpret_cast<float4*>(&cand[wave][4 * (at + lanes_below(any))]) = make_float4(v[0], v[1], v[2], v[3]);
-                    }
-                    at += __builtin_popcountll(any);
+            for (int e = 0; e < NG; e++) {
+                const unsigned long long any = __builtin_amdgcn_ballot_w64(gm[e] >= T);
+                if (any == 0ull) continue;
+                const int at = groups;
+                groups += __builtin_popcountll(any);
+                if (groups <= 16 && gm[e] >= T) {
+                    float v[4];
+                    bool flag[4];
+                    terms(side, e, v, flag);
+                    *reinterpret_cast<float4*>(&cand[wave][4 * (at + lanes_below(any))]) = make_float4(v[0], v[1], v[2], v[3]);
                 }
+            }
+            if (groups <= 16) {
                 wave_fence();
                 // the terms that reach T move to the front
                 const float v = lane < 4 * groups ? cand[wave][lane] : 0.f;
@@ -285,11 +314,28 @@ row_stream_kernel(FwdArgs a, int K) {
                         if (v[j] >= T && at < 64) cand[wave][at] = v[j];
                         count += __builtin_popcountll(hit);
                     }
+                    group_fence(e);
                 }
             }
             wave_fence();
             float sorted = 0.f;                        // lane k: the k-th largest term (0 when there are fewer)
-            if (count <= 64) {
+            if (count <= 16) {
+                // lane 16 q + i counts how many of the terms 4 q .. 4 q + 3 come before term i (as numbers, then as listed)
+                if (lane >= count && lane < 16) cand[wave][lane] = 0.f;
+                wave_fence();
+                const uint32_t own = __float_as_uint(cand[wave][lane & 15]);
+                const float4 four = *reinterpret_cast<const float4*>(&cand[wave][lane >> 4 << 2]);
+                const int ahead = (lane & 15) - (lane >> 4 << 2);
+                int rank = (__float_as_uint(four.x) + (ahead > 0 ? 1u : 0u) > own ? 1 : 0) + (__float_as_uint(four.y) + (ahead > 1 ? 1u : 0u) > own ? 1 : 0) +
+                           (__float_as_uint(four.z) + (ahead > 2 ? 1u : 0u) > own ? 1 : 0) + (__float_as_uint(four.w) + (ahead > 3 ? 1u : 0u) > own ? 1 : 0);
+                rank += __shfl_xor(rank, 16);
+                rank += __shfl_xor(rank, 32);
+                wave_fence();
+                if (lane < count) cand[wave][rank] = __uint_as_float(own);
+                wave_fence();
+                sorted = lane < count ? cand[wave][lane] : 0.f;
+                wave_fence();
+            } else if (count <= 64) {
                 const float own = lane < count ? cand[wave][lane] : 0.f;
                 int rank = 0;
                 for (int j = 0; j < count; j++) {
@@ -313,6 +359,7 @@ row_stream_kernel(FwdArgs a, int K) {
                         terms(side, e, v, flag);
                         #pragma unroll
                         for (int j = 0; j < 4; j++) best = (v[j] < below || (first && v[j] == below)) && v[j] > best ? v[j] : best;
+                        group_fence(e);
                     }
                     best = wave_max(best);
                     if (best == 0.f) break;
@@ -324,6 +371,7 @@ row_stream_kernel(FwdArgs a, int K) {
                         terms(side, e, v, flag);
                         #pragma unroll
                         for (int j = 0; j < 4; j++) same += __builtin_popcountll(__builtin_amdgcn_ballot_w64(v[j] == best));
+                        group_fence(e);
                     }
                     if (lane >= k && lane < k + same) sorted = best;
                     k += same;
@@ -331,12 +379,11 @@ row_stream_kernel(FwdArgs a, int K) {
                     first = false;
                 }
             }
-            float ans = kEps, coef = 1.f;
-            for (int k = 0; k < K; k++) {
-                ans += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sorted), k)) * coef * a.q;
-                coef *= 1.f - a.q;
-            }
-            if (mine && lane == 0) (side ? a.y1 : a.y0)[o] = ans / (1.f - coef);
+            // every lane weighs its own term; they are added up from the largest on
+            const int weighed = __float_as_int(sorted * coef * a.q);
+            float ans = kEps;
+            for (int k = 0; k < K; k++) ans += __int_as_float(__builtin_amdgcn_readlane(weighed, k));
+            if (mine && lane == 0) (side ? a.y1 : a.y0)[o] = ans / (1.f - rest);
         }
     }
 }
@@ -344,8 +391,8 @@ row_stream_kernel(FwdArgs a, int K) {
 template <int NE, int NX, StreamOp OP>
 int launch(const FwdArgs& a, int K, hipStream_t stream) {
     // few weight rows: the batch rows are dealt to several workgroups, each of which loads the weight rows again; as many as
-    // the device holds at once, so that none waits for another's end (512 x 5120 x 10, K = 10: 19 us; in 1.3 times as many 26
-    // and, interval bounds, 42 and 55).  Rows of up to 1024 inputs, with twice as many workgroups as for longer ones: 54 x 730 x 730
+    // the device holds at once, so that none waits for another's end (512 x 5120 x 10, K = 10, with three wavefronts per SIMD:
+    // 19 us; in 1.3 times as many 26 and, interval bounds, 42 and 55).  Rows of up to 1024 inputs, with twice as many workgroups as for longer ones: 54 x 730 x 730
     // 40 us instead of 50, intervals 75 and 99, l-inf with positions 11 and 14; 32 x 1024 x 1536 52 and 63.  (Three for two against rows
     // of 1025 to 3072 inputs, values of the l-inf distance: 54 x 1500 x 730 12.5 and 13.9, but 7 x 3072 x 2000 15.1 and 13.2.)
     constexpr int kWaves = stream_waves(OP), kPerCu = 4 * stream_resident(NE, NX, OP) / kWaves;
@@ -390,6 +437,13 @@ bool row_stream_ok(const FwdArgs& a, long long limit) {
 
 bool row_stream_sort_ok(const FwdArgs& a) {
     const long long outputs = (long long)a.R * a.G * a.COg, most = a.x1 ? 3ll << 14 : 1ll << 16, per_input = a.x1 ? 56 : 80;
+    return outputs <= most && outputs <= per_input * a.CIg && row_stream_ok(a, 1ll << 62);
+}
+
+bool row_stream_sort_before_terms(const FwdArgs& a) {
+    const bool longer = a.CIg > 48 * 64;   // (fewer wavefronts at a time)
+    const long long outputs = (long long)a.R * a.G * a.COg, per_input = a.x1 ? 100 : 150;
+    const long long most = a.x1 ? (longer ? 3ll << 14 : 1ll << 17) : (longer ? 1ll << 17 : 1ll << 18);
     return outputs <= most && outputs <= per_input * a.CIg && row_stream_ok(a, 1ll << 62);
 }
 

@@ -246,9 +246,10 @@ extern "C" int sd_sort_neuron_forward_nograd(const float* input, const float* we
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (g_sort_density.load(std::memory_order_relaxed) <= 0.f && row_stream_sort_ok(a))
         return row_stream_sort(a, K, st);
-    const bool small = few_tiles(a, 32, 64);
+    const bool small = few_tiles(a, 32, 64), streamed = g_sort_density.load(std::memory_order_relaxed) <= 0.f && row_stream_sort_before_terms(a);
     const bool two = K <= 12 && two_level_ok(a, K), elig = sort_cols_eligible(a, B, CO, CI, G, HW);
     const bool cols = elig && sort_cols_ok(a, kHintSiteSort, B, CO, CI, st);
+    if (streamed && !elig) return row_stream_sort(a, K, st);
     // one request for both users of the workspace: the tables (with the counter the gates read) first, the key
     // lists of the two-level path behind them
     const size_t tbytes = elig ? sort_tables_bytes(kRowsSortValues, B, CO, CI, K) : 0;
@@ -257,6 +258,7 @@ extern "C" int sd_sort_neuron_forward_nograd(const float* input, const float* we
         base = static_cast<char*>(workspace(tbytes + (two ? two_level_bytes(a, K) : 0), st));
         if (!base) return SD_ERR_HIP;
     }
+    if (streamed && !cols) return row_stream_sort(a, K, st);
     int* keys = reinterpret_cast<int*>(base + tbytes);
     if (cols && (rc = queue_sort_cols(a, kRowsSortValues, input, nullptr, weight, B, CO, CI, q, K, nullptr, output, nullptr, base, st))) return rc;
     if (cols) sort_cols_expect(a, kHintSiteSort, B, CO, CI, st);
@@ -332,6 +334,7 @@ extern "C" int sd_bound_sort_neuron_forward(const float* inputL, const float* in
         if (!ws) return SD_ERR_HIP;
         if (cols && (rc = queue_sort_cols(a, kRowsSortInterval, inputL, inputU, weight, B, CO, CI, q, K, outputL, outputU, nullptr, ws, st))) return rc;
     }
+    if (!cols && g_sort_density.load(std::memory_order_relaxed) <= 0.f && row_stream_sort_before_terms(a)) return row_stream_sort(a, K, st);
     if (cols) sort_cols_expect(a, kHintSiteBoundSort, B, CO, CI, st);
     rc = SD_ERR_ARG;
     switch (K) {

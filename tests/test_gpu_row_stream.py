@@ -111,3 +111,24 @@ def test_batch_rows_dealt_to_workgroups(oracle, B, n, m):
     ext.bound_sort_neuron_forward((x - 0.1).cuda(), (x + 0.1).cuda(), wd, y, y2, 1, 0.6, 10)
     np.testing.assert_allclose(y.cpu().numpy(), rl.reshape(B, m, 1), rtol=1e-5, atol=1e-6)
     np.testing.assert_allclose(y2.cpu().numpy(), ru.reshape(B, m, 1), rtol=1e-5, atol=1e-6)
+
+
+# layers of more outputs than the limit against tables, in shapes that have none: the kernel that streams still comes before the one
+# that forms every term, up to its own limit and not beyond
+@pytest.mark.parametrize("B,n,m,streams,bounds", [(100, 639, 630, True, True), (150, 500, 500, True, False), (40, 1657, 1659, True, True),
+                                                  (20, 3333, 3334, True, False), (151, 500, 500, False, False)])
+def test_layers_without_tables(oracle, B, n, m, streams, bounds):
+    from sortnet_amd import _lib, ext
+    x, w = _data((B, n, m, 1), "ties" if B == 100 else "normal")
+    xd, wd = x.cuda(), w.cuda()
+    y, y2 = (torch.full((B, m, 1), float("nan"), device="cuda") for _ in range(2))
+    ext.sort_neuron_forward_nograd(xd, wd, y, 1, 0.6, 10)
+    assert _lib.last_forward_kernel().startswith("row_stream_kernel") == streams
+    rows = slice(0, B, 7)   # (an output depends on its own row alone)
+    ref = oracle.sort_neuron_forward(x[rows].contiguous().numpy(), w.numpy(), 0.6, 10, need_pos=False)
+    np.testing.assert_allclose(y[rows].cpu().numpy(), ref.reshape(-1, m, 1), rtol=1e-5, atol=1e-6)   # ten products, summed in fp32
+    ext.bound_sort_neuron_forward((x - 0.1).cuda(), (x + 0.1).cuda(), wd, y, y2, 1, 0.6, 10)
+    assert _lib.last_forward_kernel().startswith("row_stream_kernel") == bounds
+    rl, ru = oracle.bound_sort_neuron_forward((x[rows] - 0.1).contiguous().numpy(), (x[rows] + 0.1).contiguous().numpy(), w.numpy(), 0.6, 10)
+    np.testing.assert_allclose(y[rows].cpu().numpy(), rl.reshape(-1, m, 1), rtol=1e-5, atol=1e-6)
+    np.testing.assert_allclose(y2[rows].cpu().numpy(), ru.reshape(-1, m, 1), rtol=1e-5, atol=1e-6)
