@@ -779,17 +779,18 @@ static int lp_backward(const char* who, const float* grad_output, const float* i
     a.skip_thr = int_power(p - 1.f) < 0 ? lp_skip_threshold(1e-16f, p - 1.f, kLpSkipFrom) : 0.f;
     hipStream_t st = static_cast<hipStream_t>(stream);
     int ip = int_power(p - 1.f);
-    // whole p up to 9: from scalar registers; the general kernel below takes them only where the stream is under capture and
-    // its scratch too small for that, and gradients that are not aligned to 16 bytes
-    if (ip >= 0 && aligned16(grad_input) && aligned16(grad_weight)) {
+    // from scalar registers where the scratch for it is at hand (a stream under capture may lack it) and the gradients are aligned
+    // to 16 bytes; else, and for what is left, the general kernel below
+    auto from_scalars = [&](int power) -> int {
+        if (!aligned16(grad_input) || !aligned16(grad_weight)) return -1;
         const LpGradArgs b{grad_output, input, weight, output, grad_input, grad_weight, ci_idx, co_idx,
                            f.R, HW, G, f.COg, f.CIg, f.W_COg, f.W_CIg};
         const size_t bytes = lp_grad_workspace(b);
-        if (workspace_ready(bytes, st)) {
-            void* ws = workspace(bytes, st);
-            return ws ? lp_grad(ip, b, ws, st) : SD_ERR_HIP;
-        }
-    }
+        if (!workspace_ready(bytes, st)) return -1;
+        void* ws = workspace(bytes, st);
+        return ws ? lp_grad(power, a.pm1, b, ws, st) : SD_ERR_HIP;
+    };
+    if (ip >= 0 && (rc = from_scalars(ip)) >= 0) return rc;
     // large p with both gradients in the dense single-group case: the kernel that forms every term once for both
     // sums and owns its grad_weight block tests significance more cheaply than the general kernel, whose
     // test only pays from a higher threshold; everything else goes through the general kernel
@@ -814,6 +815,12 @@ static int lp_backward(const char* who, const float* grad_output, const float* i
     // (both gradients, in us, by atomic additions -> from planes: 250 x 3072 x 1021 at p = 24 297 -> 312, 512 x 600 x 600
     // at p = 100 94 -> 101, 2048 x 1024 x 1024 at p = 120 in eight launches 639 -> 717, the fused kernel 3215).
     const bool same_bits = !fused && (fused_p || (rows_p && !rows));
+    // Other powers without significance tests, as far as none of the above takes them: several positions per image, dense batches that
+    // are no whole tiles, small layers with index lists.  (Both gradients, in us, general kernel / from scalar registers, p = 17.3:
+    // 64 x 288 x 256 on 16 x 16 positions 1040 / 410, 300 x 801 x 333 61 / 52, 250 x 3072 x 1021 298 / 256, lists 64 x 768 x 768 of 1024
+    // 41 / 36; but 512 x 5120 x 2560 1730 / 1800, 128 x 3072 x 1024 128 / 144, lists 512 x 3840 x 3840 of 5120 1880 / 2060.)
+    const bool scalars = HW > 1 || (!ci_idx && !co_idx ? f.R % RB != 0 : (long long)f.R * G * f.COg * f.CIg < (1ll << 26));
+    if (ip < 0 && scalars && a.pm1 > 0.f && a.skip_thr == 0.f && !rows && !fused && !same_bits && (rc = from_scalars(-1)) >= 0) return rc;
     // one request for every user of the workspace: the tables and 1 / y, then the planes of partial sums
     const size_t table_bytes = rows ? (lp_rows_workspace(f.R, f.COg, f.CIg) + (size_t)f.R * f.COg * sizeof(float) + 255) / 256 * 256 : 0;
     LpBwdPlan plan{};

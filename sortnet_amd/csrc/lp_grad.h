@@ -14,8 +14,8 @@ struct LpGradArgs {
 // bytes of workspace (what the kernel reads the batch side from, and planes of partial sums) that lp_grad needs
 size_t lp_grad_workspace(const LpGradArgs& a);
 
-// both gradients (or that of the inputs) for p - 1 = ip, a whole number in 0..8
-int lp_grad(int ip, const LpGradArgs& a, void* ws, hipStream_t st);
+// both gradients (or that of the inputs) for p - 1 = ip, a whole number in 0..8, or any pm1 = p - 1 > 0 (ip < 0)
+int lp_grad(int ip, float pm1, const LpGradArgs& a, void* ws, hipStream_t st);
 
 // out[o] = the sum of `planes` partial sums, `plane` floats apart, in plane order (lp.hip)
 int lp_merge_planes(const float* part, float* out, size_t total, size_t plane, int planes, hipStream_t st);

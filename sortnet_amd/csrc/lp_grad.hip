@@ -9,7 +9,8 @@
 // instructions on registers alone: 60; with the pairs (g, 1/y) read from LDS, 8 instructions and 3 wavefronts per SIMD it was 43).
 // Both gradients in us, that kernel -> this, p = 8: 512 x 5120 x 5120 2300 -> 1630, 250 x 3072 x 1021 251 -> 145, 90 x 1600 x 230
 // 36 -> 26, 32 x 192 x 192 19.4 -> 15.8; convolutions of 80 x 27 x 576 on 32 x 32 positions 1700 -> 590, of 64 x 288 x 256 on
-// 16 x 16 1000 -> 225; index lists, 512 x 3840 x 3840 of 5120 the same 1400 (16 additions per weight go to memory, 0.4 ms).
+// 16 x 16 1000 -> 225; index lists, 512 x 3840 x 3840 of 5120 1390 -> 1320 (16 additions per weight go to memory, 0.4 ms),
+// the inputs' gradient alone 1050 -> 800.
 #include <cmath>
 #include <type_traits>
 #include "fwd_args.h"
@@ -34,7 +35,8 @@ template <class T> __device__ __forceinline__ Const<T> as_const(const void* p) {
 constexpr float kYLow = 1.f / 256.f, kYHigh = 256.f, kGLow = 0x1p-96f, kGHigh = 0x1p+96f;
 
 struct Batch {          // the batch side as the kernel reads it
-    float* scale;       // [tile][group][channel][row]: g y^(1-p), or g in a chunk that forms ratios; 0 for rows past the batch
+    float* scale;       // [tile][group][channel][row]: g y^(1-p), or g in a chunk that forms ratios; 0 for rows past the batch.
+                        // Any other power (IP < 0): pairs (g, 1 / y), and nothing in the two below
     float* recip;       // the same layout: 1 / y in chunks that form ratios
     uint32_t* ratio;    // [tile][group][chunk]: the chunk forms ratios
 };
@@ -49,8 +51,12 @@ struct Args {
     unsigned nblocks, pairs, groups;   // blocks of 64 inputs; (block, group, slice) triples; groups of WAVES batch tiles
     int span;          // the largest power of two up to 32 and the positions per image: rows that lie side by side
     bool by_die;       // the triples fill the eight dies evenly
+    float pm1;         // p - 1 where it is no whole number up to 8
     bool gw_store;     // a workgroup holds the whole batch: its sums are grad_weight
 };
+
+constexpr int TS = 65;   // row stride of a tile in LDS
+constexpr int lds_words(int waves, bool strided) { return strided ? RB * TS : waves > 1 ? 2 * MC * 64 : 0; }
 
 // u = (first of the pair times the second) from the difference and g y^(1-p)
 template <int IP>
@@ -109,7 +115,7 @@ __global__ void __launch_bounds__(256) lp_grad_batch_kernel(Args k, float* __res
     for (int e = 0; e < 8; e++) {
         const int f = tid + 256 * e, i = a.HW == 1 ? f / 64 : f % RB, j = a.HW == 1 ? f % 64 : f / RB;
         const int r = r0 + i, m = m0 + j;
-        float gv = 0.f, yv = 1.f;
+        float gv = 0.f, yv = IP < 0 ? __builtin_inff() : 1.f;
         if (r < a.R && m < a.COg) {
             const int b = a.HW == 1 ? r : r / a.HW, hw = r - b * a.HW;
             const size_t o = ((size_t)(b * a.G + g) * a.COg + m) * a.HW + hw;
@@ -127,6 +133,14 @@ __global__ void __launch_bounds__(256) lp_grad_batch_kernel(Args k, float* __res
     for (int e = 0; e < 2; e++) {
         const int j = (tid >> 3) + 32 * e, m = m0 + j;
         float s[4], yv[4], gv[4];
+        if (IP < 0) {
+            if (m < k.COp) {
+                float4* dst = reinterpret_cast<float4*>(k.s.scale + ((base + m) * RB + i0) * 2);
+                #pragma unroll
+                for (int i = 0; i < 4; i += 2) dst[i / 2] = make_float4(gs[i0 + i][j], 1.f / ys[i0 + i][j], gs[i0 + i + 1][j], 1.f / ys[i0 + i + 1][j]);
+            }
+            continue;
+        }
         bool bad = false;
         #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -167,25 +181,45 @@ __device__ __forceinline__ void product_rows(const float* xr, float* acc, float 
         if (i % 4 == 0) __builtin_amdgcn_sched_barrier(0);   // more rows at once would take the registers of a fourth wavefront
     }
 }
+// eight rows of one channel at any power; rows past the batch have g = 1 / y = 0.  (The transcendentals bound it, at any number of
+// wavefronts: four rows side by side took 4 % longer.)
+template <bool GW, class Rest>
+__device__ __forceinline__ void any_power_rows(const float* xr, float* acc, float (&ws)[2], f16v pairs, float wk, float pm1, Rest rest) {
+    #pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const float sr = (xr[i] - wk) * pairs[2 * i + 1];
+        const float pw = __builtin_copysignf(__builtin_amdgcn_exp2f(pm1 * __builtin_amdgcn_logf(fabsf(sr))), sr);   // 1 / y > 0: the sign of d
+        acc[i] = fmaf(pairs[2 * i], pw, acc[i]);
+        asm volatile("" : "+v"(acc[i]));
+        if (GW) ws[i & 1] = fmaf(pairs[2 * i], pw, ws[i & 1]);
+        if (i == 0) { __builtin_amdgcn_sched_barrier(0); rest(); }
+        if (i % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
 // WAVES = kTiles: the wavefronts of a workgroup take neighbouring batch tiles of the same inputs and their sums of grad_weight
-// meet in LDS, so that memory sees one addition per 128 rows.  WAVES = 1: a workgroup is one wavefront.  STRIDED: several positions per
-// image, whose inputs are not side by side in a row.  LISTS: index lists on either side.
+// meet in LDS, so that memory sees one addition per 128 rows.  WAVES = 1: they have nothing to do with each
+// other, and four of them make a workgroup where there are many, so that every SIMD holds as many (index lists, 512 x 3840 x 3840 of
+// 5120, p = 24: 2.7 ms in workgroups of one wavefront).  STRIDED: several positions per image, whose inputs are not side by side in a row.  LISTS: index lists on either side.
 template <int IP, bool GW, int WAVES, bool STRIDED, bool LISTS>
-__global__ void __launch_bounds__(64 * WAVES, 4) lp_grad_kernel(Args k) {
+__global__ void __launch_bounds__(256, 4) lp_grad_kernel(Args k) {
     const LpGradArgs& a = k.a;
     // the tile on its way between memory and registers where a row's inputs are strided; then sums of grad_weight
-    constexpr int TS = 65;
-    __shared__ float lds[WAVES][STRIDED ? RB * TS : 2 * MC * 64];
+    extern __shared__ float shared[];
+    constexpr int kLds = lds_words(WAVES, STRIDED);   // of a wavefront
     static_assert(2 * MC * 64 <= RB * TS, "both halves of the sums fit");
-    const int lane = threadIdx.x & 63, wave = WAVES > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    float* const lds = shared + wave * kLds;
     // all batch tiles of a (block of inputs, slice) run on one die one after the other: they share its weights there
-    const unsigned pair = k.by_die ? blockIdx.x % 8 + 8 * (blockIdx.x / 8 / k.groups) : blockIdx.x % k.pairs;
-    const unsigned group = k.by_die ? blockIdx.x / 8 % k.groups : blockIdx.x / k.pairs;
-    if (pair >= k.pairs) return;
+    const unsigned die = blockIdx.x % 8, waves = WAVES > 1 ? 1 : blockDim.x / 64, own = WAVES > 1 ? 0 : wave;
+    const unsigned unit = (k.by_die ? blockIdx.x / 8 : blockIdx.x) * waves + own;
+    const unsigned pair = k.by_die ? die + 8 * (unit / k.groups) : unit % k.pairs;
+    const unsigned group = k.by_die ? unit % k.groups : unit / k.pairs;
+    if (pair >= k.pairs || group >= k.groups) return;
     const int nblock = pair % k.nblocks, g = pair / k.nblocks % a.G, slice = pair / k.nblocks / a.G;
     const int m_lo = slice * k.per, m_hi = m_lo + k.per < a.COg ? m_lo + k.per : a.COg;
     if (m_lo >= m_hi) return;
-    const int tile = (int)group * WAVES + wave, r0 = (k.tile0 + tile) * RB;
+    const int tile = (int)group * WAVES + (WAVES > 1 ? wave : 0), r0 = (k.tile0 + tile) * RB;
     const int n = nblock * 64 + lane;
     const bool n_ok = n < a.CIg;
     const int nc = n_ok ? n : a.CIg - 1;
@@ -221,11 +255,11 @@ __global__ void __launch_bounds__(64 * WAVES, 4) lp_grad_kernel(Args k) {
     };
 
     const size_t base = ((size_t)tile * a.G + g) * k.COp;
-    const Const<float> scale = as_const<float>(k.s.scale + base * RB), recip = as_const<float>(k.s.recip + base * RB);
+    const Const<float> scale = as_const<float>(k.s.scale + base * RB * (IP < 0 ? 2 : 1)), recip = as_const<float>(k.s.recip + base * RB);
     const Const<uint32_t> ratio = as_const<uint32_t>(k.s.ratio + base / MC);
     const uint32_t* modes = k.s.ratio + base / MC;
     const int c_hi = (m_hi + MC - 1) / MC;
-    uint32_t mode = m_lo / MC + lane < c_hi ? modes[m_lo / MC + lane] : 0u;
+    uint32_t mode = IP >= 0 && m_lo / MC + lane < c_hi ? modes[m_lo / MC + lane] : 0u;
 
     float xr[RB], acc[RB];
     if constexpr (STRIDED) {
@@ -236,9 +270,9 @@ __global__ void __launch_bounds__(64 * WAVES, 4) lp_grad_kernel(Args k) {
             xr[t] = (a.x + __shfl(begin, at.x))[(unsigned)c * (unsigned)a.HW];
         }
         #pragma unroll
-        for (int t = 0; t < RB; t++) { const int2 at = strided(t); lds[wave][at.x * TS + at.y] = xr[t]; }
+        for (int t = 0; t < RB; t++) { const int2 at = strided(t); lds[at.x * TS + at.y] = xr[t]; }
         #pragma unroll
-        for (int i = 0; i < RB; i++) { xr[i] = lds[wave][i * TS + lane]; acc[i] = 0.f; }
+        for (int i = 0; i < RB; i++) { xr[i] = lds[i * TS + lane]; acc[i] = 0.f; }
         if (WAVES > 1) __syncthreads();
     } else {
         #pragma unroll
@@ -257,7 +291,7 @@ __global__ void __launch_bounds__(64 * WAVES, 4) lp_grad_kernel(Args k) {
     #pragma unroll
     for (int j = 0; j < MC; j++) wv[j] = wbase[(size_t)row_of(m_lo, j, rowv) * a.W_CIg];
     // a slice without a chunk that forms ratios runs the loop without that path, which would cost it copies of its sums
-    for (int c = m_lo / MC + 64 + lane; c < c_hi; c += 64) mode |= modes[c];
+    for (int c = m_lo / MC + 64 + lane; IP >= 0 && c < c_hi; c += 64) mode |= modes[c];
     const bool ratios = __builtin_amdgcn_ballot_w64(mode != 0u) != 0ull;
 
     auto add_weight = [&](int row, float v) {
@@ -274,7 +308,26 @@ __global__ void __launch_bounds__(64 * WAVES, 4) lp_grad_kernel(Args k) {
             #pragma unroll
             for (int j = 0; j < MC; j++) wn[j] = wbase[(size_t)row_of(m0 + MC, j, rown) * a.W_CIg];
             float sum[MC] = {};
-            if constexpr (!MIXED) {
+            if constexpr (IP < 0) {
+                f16v s0 = block(2 * m0, 0);
+                float next = 0.f;
+                #pragma unroll
+                for (int j = 0; j < MC; j++) {
+                    float ws[2] = {0.f, 0.f};
+                    #pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        f16v s1 = s0;
+                        any_power_rows<GW>(xr + 8 * q, acc + 8 * q, ws, s0, wv[j], k.pm1, [&] {
+                            if (j * 4 + q + 1 < 4 * MC) s1 = block(2 * (m0 + j), 16 * (q + 1));
+                            else next = scale[(size_t)(m0 + MC < m_end ? m0 + MC : m0) * RB * 2];
+                        });
+                        s0 = s1;
+                    }
+                    sum[j] = ws[0] + ws[1];
+                    asm volatile("" : "+v"(sum[j]));
+                }
+                asm volatile("" :: "s"(next));
+            } else if constexpr (!MIXED) {
                 f16v s0 = block(m0, 0);
                 float next = 0.f;   // brings the next chunk's first block as far as the scalar cache
                 #pragma unroll
@@ -316,7 +369,7 @@ __global__ void __launch_bounds__(64 * WAVES, 4) lp_grad_kernel(Args k) {
             }
             if (GW && WAVES > 1) {
                 #pragma unroll
-                for (int j = 0; j < MC; j++) lds[wave][(buf * MC + j) * 64 + lane] = sum[j];
+                for (int j = 0; j < MC; j++) lds[(buf * MC + j) * 64 + lane] = sum[j];
                 __syncthreads();   // the other half is written behind the next barrier but one
             }
             // the next weights have arrived before the additions below are queued: waiting for them later would wait for these
@@ -326,7 +379,7 @@ __global__ void __launch_bounds__(64 * WAVES, 4) lp_grad_kernel(Args k) {
                 static_assert(WAVES == 1 || WAVES == MC, "a wavefront adds up one channel of the chunk");
                 float v = 0.f;
                 #pragma unroll
-                for (int j = 0; j < WAVES; j++) v += lds[j][(buf * MC + wave) * 64 + lane];
+                for (int j = 0; j < WAVES; j++) v += shared[j * kLds + (buf * MC + wave) * 64 + lane];
                 if (n_ok && m0 + wave < m_hi) add_weight(m0 + wave, -v);
             } else if (GW) {
                 #pragma unroll
@@ -336,7 +389,8 @@ __global__ void __launch_bounds__(64 * WAVES, 4) lp_grad_kernel(Args k) {
             if (LISTS) { rowv = rown; rown = rows_of(m0 + 2 * MC); }
         }
     };
-    if (ratios) walk(std::true_type{});
+    if constexpr (IP < 0) walk(std::false_type{});
+    else if (ratios) walk(std::true_type{});
     else walk(std::false_type{});
     // what only the end needs is read again here: it would take scalar registers all the way
     Const<Args> late = (Const<Args>)__builtin_amdgcn_kernarg_segment_ptr();
@@ -346,12 +400,12 @@ __global__ void __launch_bounds__(64 * WAVES, 4) lp_grad_kernel(Args k) {
     if constexpr (STRIDED) {
         if (WAVES > 1) __syncthreads();
         #pragma unroll
-        for (int i = 0; i < RB; i++) lds[wave][i * TS + lane] = acc[i];
+        for (int i = 0; i < RB; i++) lds[i * TS + lane] = acc[i];
         #pragma unroll 8
         for (int t = 0; t < RB; t++) {
             const int2 at = strided(t);
             float* dst = gx + __shfl(begin, at.x) + (unsigned)(nblock * 64 + at.y) * (unsigned)a.HW;
-            const float v = lds[wave][at.x * TS + at.y];
+            const float v = lds[at.x * TS + at.y];
             if (at.x >= rows || nblock * 64 + at.y >= a.CIg) continue;
             if (add) unsafeAtomicAdd(dst, v);
             else *dst = v;
@@ -386,15 +440,11 @@ Plan make_plan(const LpGradArgs& a) {
     const long long waves = (long long)nb * real * a.G;   // before the output channels are cut
     p.waves = !lists && a.gw && whole * 8 <= real * 9 && waves >= 4ll * num_cus() ? kTiles : 1;
     p.tiles = p.waves > 1 ? whole : real;
-    // the device holds four wavefronts per SIMD: the slice count whose last round of them is fullest, a smaller one unless a
-    // larger gains 3 %, slices of at least 64 channels
-    const double slots = 16.0 * num_cus();
-    double best = 0.0;
-    p.zsplit = 1;
-    for (int z = 1; z <= 16 && (z == 1 || a.COg / z >= 64); z++) {
-        const double rounds = (double)nb * p.tiles * a.G * z / slots, eff = rounds / std::ceil(rounds);
-        if (eff > best * 1.03) { best = eff; p.zsplit = z; }
-    }
+    // four rounds of the wavefronts that the device holds at once (four per SIMD; the first round is not dealt evenly, and the last
+    // one not filled), slices of at least 64 channels
+    const long long units = (long long)nb * p.tiles * a.G, rounds = (64ll * num_cus() + units - 1) / units, longest = a.COg / 64;
+    p.zsplit = (int)(rounds > 16 ? 16 : rounds);
+    if (p.zsplit > longest) p.zsplit = longest > 1 ? (int)longest : 1;
     // small layers: slices down to one chunk until every SIMD has two wavefronts; their sums are merged in slice order
     const long long fill = 8ll * num_cus();
     bool planes = false;
@@ -417,13 +467,17 @@ Plan make_plan(const LpGradArgs& a) {
 }
 
 template <int IP, bool STRIDED>
-void launch_tiles(const Args& k, int waves, dim3 grid, hipStream_t st) {
-    if (k.a.ci_idx || k.a.co_idx) {
-        if (k.a.gw) hipLaunchKernelGGL((lp_grad_kernel<IP, true, 1, STRIDED, true>), grid, dim3(64), 0, st, k);
-        else hipLaunchKernelGGL((lp_grad_kernel<IP, false, 1, STRIDED, true>), grid, dim3(64), 0, st, k);
-    } else if (waves > 1) hipLaunchKernelGGL((lp_grad_kernel<IP, true, kTiles, STRIDED, false>), grid, dim3(64 * kTiles), 0, st, k);
-    else if (k.a.gw) hipLaunchKernelGGL((lp_grad_kernel<IP, true, 1, STRIDED, false>), grid, dim3(64), 0, st, k);
-    else hipLaunchKernelGGL((lp_grad_kernel<IP, false, 1, STRIDED, false>), grid, dim3(64), 0, st, k);
+void launch_tiles(const Args& k, int waves, hipStream_t st) {
+    const bool lists = k.a.ci_idx || k.a.co_idx;
+    const unsigned units = k.pairs * k.groups, pack = waves > 1 ? 1 : units >= 8u * num_cus() ? 4 : 1;   // units of a workgroup
+    const unsigned per_die = (k.pairs + 7) / 8 * k.groups;
+    const dim3 grid(k.by_die ? 8 * ((per_die + pack - 1) / pack) : (units + pack - 1) / pack), block(64 * waves * pack);
+    const size_t lds = (size_t)lds_words(waves, STRIDED) * waves * pack * sizeof(float);
+    if (lists && k.a.gw) hipLaunchKernelGGL((lp_grad_kernel<IP, true, 1, STRIDED, true>), grid, block, lds, st, k);
+    else if (lists) hipLaunchKernelGGL((lp_grad_kernel<IP, false, 1, STRIDED, true>), grid, block, lds, st, k);
+    else if (waves > 1) hipLaunchKernelGGL((lp_grad_kernel<IP, true, kTiles, STRIDED, false>), grid, block, lds, st, k);
+    else if (k.a.gw) hipLaunchKernelGGL((lp_grad_kernel<IP, true, 1, STRIDED, false>), grid, block, lds, st, k);
+    else hipLaunchKernelGGL((lp_grad_kernel<IP, false, 1, STRIDED, false>), grid, block, lds, st, k);
 }
 
 template <int IP>
@@ -444,9 +498,8 @@ int launch(Args& k, const Plan& p, float* part, hipStream_t st) {
         if (fill > 16u * num_cus()) fill = 16u * num_cus();
         hipLaunchKernelGGL((lp_grad_batch_kernel<IP>), dim3(lay + (unsigned)fill), dim3(256), 0, st, k, a.gx, z0, a.gw, z1, lay);
         if ((rc = check_launch("lp_grad_batch_kernel"))) return rc;
-        const dim3 grid((k.by_die ? (k.pairs + 7) / 8 * 8 : k.pairs) * k.groups);
-        if (a.HW > 1) launch_tiles<IP, true>(k, p.waves, grid, st);
-        else launch_tiles<IP, false>(k, p.waves, grid, st);
+        if (a.HW > 1) launch_tiles<IP, true>(k, p.waves, st);
+        else launch_tiles<IP, false>(k, p.waves, st);
         if ((rc = check_launch("lp_grad_kernel"))) return rc;
     }
     return part ? lp_merge_planes(part, gx, nx, p.plane, k.zsplit, st) : SD_OK;
@@ -456,10 +509,11 @@ int launch(Args& k, const Plan& p, float* part, hipStream_t st) {
 
 size_t lp_grad_workspace(const LpGradArgs& a) { return make_plan(a).bytes; }
 
-int lp_grad(int ip, const LpGradArgs& a, void* ws, hipStream_t st) {
+int lp_grad(int ip, float pm1, const LpGradArgs& a, void* ws, hipStream_t st) {
     const Plan p = make_plan(a);
     Args k{};
     k.a = a;
+    k.pm1 = pm1;
     k.COp = (a.COg + MC - 1) / MC * MC;
     k.zsplit = p.zsplit; k.per = p.per;
     k.nblocks = (unsigned)(a.CIg + 63) / 64;
@@ -480,7 +534,8 @@ int lp_grad(int ip, const LpGradArgs& a, void* ws, hipStream_t st) {
         case 5: return launch<5>(k, p, part, st);
         case 6: return launch<6>(k, p, part, st);
         case 7: return launch<7>(k, p, part, st);
-        default: return launch<8>(k, p, part, st);
+        case 8: return launch<8>(k, p, part, st);
+        default: return launch<-1>(k, p, part, st);   // (scale and recip together: the pairs)
     }
 }
 
