@@ -84,10 +84,22 @@ constexpr int kMaxRowLds = 12288;   // floats of LDS one row histogram may take
 // those adds are the time (128 rows of 5120 outputs, K = 10: 67 us with a workgroup to a row, 37 with four): every
 // part's workgroup reads the positions of its row and adds what falls into its own inputs.
 constexpr int kSlotsAtOnce = 5;     // positions of an output in flight
+// a run of floats of LDS cleared, and written out to memory that lies side by side, 16 bytes at a time where both allow it
+__device__ __forceinline__ void clear_run(float* hist, int n) {
+    for (int i = threadIdx.x; i < n / 4; i += blockDim.x) reinterpret_cast<float4*>(hist)[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int i = n / 4 * 4 + threadIdx.x; i < n; i += blockDim.x) hist[i] = 0.f;
+}
+__device__ __forceinline__ void write_run(float* __restrict__ out, const float* hist, int n) {
+    int from = 0;
+    if (reinterpret_cast<uintptr_t>(out) % 16 == 0 && reinterpret_cast<uintptr_t>(hist) % 16 == 0) {
+        for (int i = threadIdx.x; i < n / 4; i += blockDim.x) reinterpret_cast<float4*>(out)[i] = reinterpret_cast<const float4*>(hist)[i];
+        from = n / 4 * 4;
+    }
+    for (int i = from + threadIdx.x; i < n; i += blockDim.x) out[i] = hist[i];
+}
+
 template <bool SORT, bool HAS_W>
-__global__ void __launch_bounds__(1024) scatter_bwd_rows_kernel(BwdArgs a) {
-    extern __shared__ float hist[];
-    const int row = blockIdx.x;                 // ((b * G) + g) * HW + hw
+__device__ __forceinline__ void input_row(const BwdArgs& a, int row, float* hist) {   // row: ((b * G) + g) * HW + hw
     const int hw = row % a.HW;
     const int bg = row / a.HW;
     const int g = bg % a.G, b = bg / a.G;
@@ -100,7 +112,7 @@ __global__ void __launch_bounds__(1024) scatter_bwd_rows_kernel(BwdArgs a) {
         n0 = a.CIg * (int)blockIdx.y >> parts;
         len = (a.CIg * (int)(blockIdx.y + 1) >> parts) - n0;
     }
-    for (int n = threadIdx.x; n < len; n += blockDim.x) hist[n] = 0.f;
+    clear_run(hist, len);
     __syncthreads();
     const size_t obase = ((size_t)(b * a.G + g) * a.COg) * a.HW + hw;
     const int K = SORT ? a.K : 1;
@@ -133,20 +145,25 @@ __global__ void __launch_bounds__(1024) scatter_bwd_rows_kernel(BwdArgs a) {
     }
     __syncthreads();
     const size_t xbase = ((size_t)(b * a.G + g) * a.CIg + n0) * a.HW + hw;
-    for (int n = threadIdx.x; n < len; n += blockDim.x) a.gx0[xbase + (size_t)n * a.HW] = hist[n];
+    if (a.HW == 1) write_run(a.gx0 + xbase, hist, len);
+    else for (int n = threadIdx.x; n < len; n += blockDim.x) a.gx0[xbase + (size_t)n * a.HW] = hist[n];
+}
+
+template <bool SORT, bool HAS_W>
+__global__ void __launch_bounds__(1024) scatter_bwd_rows_kernel(BwdArgs a) {
+    extern __shared__ __attribute__((aligned(16))) float hist[];
+    input_row<SORT, HAS_W>(a, blockIdx.x, hist);
 }
 
 template <bool HAS_W>
-__global__ void __launch_bounds__(256) bound_bwd_rows_kernel(BwdArgs a) {
-    extern __shared__ float hist[];             // [0, CIg) lower, [CIg, 2 CIg) upper
-    const int row = blockIdx.x;
+__device__ __forceinline__ void bound_row(const BwdArgs& a, int row, float* hist) {   // hist: [0, CIg) lower, [CIg, 2 CIg) upper
     const int hw = row % a.HW;
     const int bg = row / a.HW;
     const int g = bg % a.G, b = bg / a.G;
-    for (int n = threadIdx.x; n < 2 * a.CIg; n += 256) hist[n] = 0.f;
+    clear_run(hist, 2 * a.CIg);
     __syncthreads();
     const size_t obase = ((size_t)(b * a.G + g) * a.COg) * a.HW + hw;
-    for (int m = threadIdx.x; m < a.COg; m += 256) {
+    for (int m = threadIdx.x; m < a.COg; m += blockDim.x) {
         size_t o = obase + (size_t)m * a.HW;
         size_t wrow = (size_t)(g * a.COg + m) * a.CIg;
         int pl = a.p0[o], pu = a.p1[o];
@@ -162,10 +179,69 @@ __global__ void __launch_bounds__(256) bound_bwd_rows_kernel(BwdArgs a) {
     }
     __syncthreads();
     const size_t xbase = ((size_t)(b * a.G + g) * a.CIg) * a.HW + hw;
-    for (int n = threadIdx.x; n < a.CIg; n += 256) {
-        a.gx0[xbase + (size_t)n * a.HW] = hist[n];
-        a.gx1[xbase + (size_t)n * a.HW] = hist[a.CIg + n];
+    if (a.HW == 1) {
+        write_run(a.gx0 + xbase, hist, a.CIg);
+        write_run(a.gx1 + xbase, hist + a.CIg, a.CIg);
+    } else {
+        for (int n = threadIdx.x; n < a.CIg; n += blockDim.x) {
+            a.gx0[xbase + (size_t)n * a.HW] = hist[n];
+            a.gx1[xbase + (size_t)n * a.HW] = hist[a.CIg + n];
+        }
     }
+}
+
+// Several positions per image: a workgroup takes P neighbouring ones (a power of two) of a (sample, group), so that what it reads and
+// writes lies side by side in runs of P (a row to a workgroup touched a cache line per output: both gradients of 128 x 288 x 128 on 8 x 8
+// positions 135 -> 20 us, of 64 x 27 x 576 on 32 x 32 1610 -> 480).  BOUND: interval bounds, the upper bound's rows behind the lower one's.
+template <bool BOUND>
+__device__ __forceinline__ void input_positions(const BwdArgs& a, unsigned block, int P, float* hist) {
+    const int runs = (a.HW + P - 1) / P, bg = (int)(block / (unsigned)runs), hw0 = (int)(block - (unsigned)bg * runs) * P;
+    const int shift = __builtin_ctz(P), p = threadIdx.x & (P - 1), size = a.CIg * P;   // (a workgroup is a multiple of P wide)
+    clear_run(hist, BOUND ? 2 * size : size);
+    __syncthreads();
+    const size_t obase = (size_t)bg * a.COg * a.HW + hw0 + p;
+    if (hw0 + p < a.HW) {
+        for (int m = threadIdx.x >> shift; m < a.COg; m += blockDim.x >> shift) {
+            const size_t o = obase + (size_t)m * a.HW;
+            if (BOUND) {
+                const int pl = a.p0[o], pu = a.p1[o];
+                const float gl = a.g0[o], gu = a.g1[o];
+                if ((uint32_t)pl != kNanId) atomicAdd(&hist[(pl >= 0 ? 0 : size) + ((pl & 0x7fffffff) << shift) + p], pl >= 0 ? gl : -gl);
+                atomicAdd(&hist[(pu >= 0 ? size : 0) + ((pu & 0x7fffffff) << shift) + p], pu >= 0 ? gu : -gu);
+            } else {
+                const int pr = a.p0[o];
+                const float grad = a.g0[o];
+                atomicAdd(&hist[((pr & 0x7fffffff) << shift) + p], pr >= 0 ? grad : -grad);
+            }
+        }
+    }
+    __syncthreads();
+    if (hw0 + p < a.HW) {
+        const size_t xbase = (size_t)bg * a.CIg * a.HW + hw0 + p;
+        for (int n = threadIdx.x >> shift; n < a.CIg; n += blockDim.x >> shift) {
+            a.gx0[xbase + (size_t)n * a.HW] = hist[(n << shift) + p];
+            if (BOUND) a.gx1[xbase + (size_t)n * a.HW] = hist[size + (n << shift) + p];
+        }
+    }
+}
+
+// positions of a workgroup: as many as LDS holds rows of, up to a run of 128 bytes; 1: a row to a workgroup
+static int positions_at_once(const BwdArgs& a, int rows_of) {
+    int P = 1;
+    while (P < 32 && P * 2 <= a.HW && 2 * P * rows_of * a.CIg <= kMaxRowLds) P *= 2;
+    return P;
+}
+
+template <bool BOUND>
+__global__ void __launch_bounds__(1024) positions_bwd_kernel(BwdArgs a, int P) {
+    extern __shared__ __attribute__((aligned(16))) float hist[];
+    input_positions<BOUND>(a, blockIdx.x, P, hist);
+}
+
+template <bool HAS_W>
+__global__ void __launch_bounds__(256) bound_bwd_rows_kernel(BwdArgs a) {
+    extern __shared__ __attribute__((aligned(16))) float hist[];
+    bound_row<HAS_W>(a, blockIdx.x, hist);
 }
 
 // grad_weight by rows (dense layers, no index lists): one workgroup owns WR consecutive weight rows,
@@ -180,20 +256,21 @@ __global__ void __launch_bounds__(256) bound_bwd_rows_kernel(BwdArgs a) {
 constexpr int kMaxWRowsLds = 15360;   // floats of LDS the weight-row histograms of one workgroup may take
 
 template <int MODE>
-__global__ void __launch_bounds__(256) wrows_bwd_kernel(BwdArgs a, int WR) {
-    extern __shared__ float hist[];             // [WR][CIg]
+__device__ __forceinline__ void weight_rows(const BwdArgs& a, int WR, unsigned block, float* hist) {   // hist: [WR][CIg]
     const int CO = a.G * a.COg;
-    const int die = blockIdx.x & 7, k = blockIdx.x >> 3;
+    const int die = block & 7, k = block >> 3;
     const int c0 = ((((k >> 3) * 8 + die) << 3) + (k & 7)) * WR;
     if (c0 >= CO) return;                       // the grid is rounded up to 64 row blocks
     const int nrows = CO - c0 < WR ? CO - c0 : WR;
-    for (int n = threadIdx.x; n < WR * a.CIg; n += 256) hist[n] = 0.f;
+    clear_run(hist, WR * a.CIg);
     __syncthreads();
-    const int j = threadIdx.x % WR, rstep = 256 / WR;
+    // neighbouring work-items read neighbouring rows of a sample, or positions of an image
+    const int rstep = blockDim.x / WR, j = a.HW >= 8 ? threadIdx.x / rstep : threadIdx.x % WR;
     const int R = a.B * a.HW;
     if (j < nrows) {
         float* h = hist + (size_t)j * a.CIg;
-        for (int r = threadIdx.x / WR; r < R; r += rstep) {
+        #pragma unroll 4
+        for (int r = a.HW >= 8 ? threadIdx.x % rstep : threadIdx.x / WR; r < R; r += rstep) {
             int b = r, hw = 0;
             if (a.HW > 1) { b = r / a.HW; hw = r - b * a.HW; }
             const size_t o = ((size_t)b * CO + c0 + j) * a.HW + hw;
@@ -216,8 +293,13 @@ __global__ void __launch_bounds__(256) wrows_bwd_kernel(BwdArgs a, int WR) {
         }
     }
     __syncthreads();
-    float* out = a.gw + (size_t)c0 * a.CIg;
-    for (int n = threadIdx.x; n < nrows * a.CIg; n += 256) out[n] = hist[n];
+    write_run(a.gw + (size_t)c0 * a.CIg, hist, nrows * a.CIg);
+}
+
+template <int MODE>
+__global__ void __launch_bounds__(256) wrows_bwd_kernel(BwdArgs a, int WR) {
+    extern __shared__ __attribute__((aligned(16))) float hist[];
+    weight_rows<MODE>(a, WR, blockIdx.x, hist);
 }
 
 // The same for the l-inf layer with index lists (core/cuda/inf_dist_cuda.cu:214-275 scatters with global atomics into a
@@ -238,16 +320,16 @@ __global__ void __launch_bounds__(256) row_place_kernel(const int* __restrict__ 
     }
 }
 
-__global__ void __launch_bounds__(256) wrows_lists_bwd_kernel(BwdArgs a, int WR, const int* __restrict__ place) {
-    extern __shared__ float hist[];             // [WR][W_CIg]
+__device__ __forceinline__ void weight_rows_lists(const BwdArgs& a, int WR, const int* __restrict__ place, unsigned block,
+                                                  float* hist) {   // hist: [WR][W_CIg]
     const int rows_total = a.G * a.W_COg;
-    const int die = blockIdx.x & 7, k = blockIdx.x >> 3;
+    const int die = block & 7, k = block >> 3;
     const int c0 = ((((k >> 3) * 8 + die) << 3) + (k & 7)) * WR;      // as in wrows_bwd_kernel
     if (c0 >= rows_total) return;
     const int nrows = rows_total - c0 < WR ? rows_total - c0 : WR;
-    for (int n = threadIdx.x; n < WR * a.W_CIg; n += 256) hist[n] = 0.f;
+    clear_run(hist, WR * a.W_CIg);
     __syncthreads();
-    const int j = threadIdx.x % WR, rstep = 256 / WR;
+    const int j = threadIdx.x % WR, rstep = blockDim.x / WR;
     const int R = a.B * a.HW;
     if (j < nrows) {
         const int g = (c0 + j) / a.W_COg, rr = (c0 + j) - g * a.W_COg;
@@ -268,37 +350,60 @@ __global__ void __launch_bounds__(256) wrows_lists_bwd_kernel(BwdArgs a, int WR,
         }
     }
     __syncthreads();
-    float* out = a.gw + (size_t)c0 * a.W_CIg;
-    for (int n = threadIdx.x; n < nrows * a.W_CIg; n += 256) out[n] = hist[n];
+    write_run(a.gw + (size_t)c0 * a.W_CIg, hist, nrows * a.W_CIg);
 }
 
-// launches wrows_bwd_kernel when the layer is dense and a row fits; returns false when the caller has to
-// take the zero-fill + atomics path for grad_weight
+__global__ void __launch_bounds__(256) wrows_lists_bwd_kernel(BwdArgs a, int WR, const int* __restrict__ place) {
+    extern __shared__ __attribute__((aligned(16))) float hist[];
+    weight_rows_lists(a, WR, place, blockIdx.x, hist);
+}
+
+// Both gradients in one launch, the workgroups of grad_weight (w_blocks of them, the longer ones) first: a launch less, and the
+// rows of grad_input fill the device where those of grad_weight run out.  MODE 0: l-inf, 2: interval bounds, 3: l-inf with index lists.
+// Memory bounds it: 512 x 5120 x 5120 50 -> 42.5 us (3.2 TB/s), intervals 83 -> 71, lists 57 -> 50; 128 x 3072 x 1024 10.9 -> 6.8, with four
+// positions 128 x 2700 x 1024 19.1 -> 13.6, 512 x 256 x 10 9.9 -> 3.7 (two launches -> this).
 template <int MODE>
-static bool launch_wrows(const BwdArgs& a, hipStream_t st) {
-    if ((a.ci_idx || a.co_idx) && MODE == 0 && a.W_CIg <= kMaxWRowsLds) {
-        int* place = nullptr;
-        if (a.co_idx) {
-            const int SG = (a.B + kSubBatch - 1) / kSubBatch * a.G;
-            place = static_cast<int*>(workspace((size_t)SG * a.W_COg * sizeof(int), st));   // the only request of the call
-            if (!place) return false;
-            hipLaunchKernelGGL(row_place_kernel, dim3((unsigned)SG), dim3(256), 0, st, a.co_idx, a.COg, a.W_COg, place);
-        }
-        int WR = 1;
-        while (WR < 8 && 2 * WR * a.W_CIg <= kMaxWRowsLds) WR *= 2;
-        const int blocks = (a.G * a.W_COg + WR - 1) / WR;
-        hipLaunchKernelGGL(wrows_lists_bwd_kernel, dim3((unsigned)((blocks + 63) / 64 * 64)), dim3(256),
-                           (size_t)WR * a.W_CIg * sizeof(float), st, a, WR, place);
-        return true;
+__global__ void __launch_bounds__(1024) both_bwd_kernel(BwdArgs a, int WR, const int* __restrict__ place, unsigned w_blocks, int P) {
+    extern __shared__ __attribute__((aligned(16))) float hist[];
+    if (blockIdx.x < w_blocks) {
+        if constexpr (MODE == 3) weight_rows_lists(a, WR, place, blockIdx.x, hist);
+        else weight_rows<MODE>(a, WR, blockIdx.x, hist);
+    } else if (P > 1) input_positions<MODE == 2>(a, blockIdx.x - w_blocks, P, hist);
+    else if constexpr (MODE == 2) bound_row<false>(a, blockIdx.x - w_blocks, hist);
+    else input_row<false, false>(a, blockIdx.x - w_blocks, hist);
+}
+
+// How grad_weight is summed by rows: weight rows per workgroup, 0 when a row does not fit and the caller has to take the
+// zero-fill + atomics path
+struct WeightRows { int WR; unsigned blocks; size_t lds; const int* place; };
+static int plan_wrows(const BwdArgs& a, bool lists_ok, WeightRows& w, hipStream_t st) {
+    w = WeightRows{};
+    const bool lists = a.ci_idx || a.co_idx;
+    if (a.W_CIg > kMaxWRowsLds || (lists && !lists_ok)) return SD_OK;
+    if (a.co_idx) {
+        const int SG = (a.B + kSubBatch - 1) / kSubBatch * a.G;
+        int* place = static_cast<int*>(workspace((size_t)SG * a.W_COg * sizeof(int), st));   // the only request of the call
+        if (!place) return SD_OK;
+        hipLaunchKernelGGL(row_place_kernel, dim3((unsigned)SG), dim3(256), 0, st, a.co_idx, a.COg, a.W_COg, place);
+        w.place = place;
+        const int rc = check_launch("row_place_kernel");
+        if (rc) return rc;
     }
-    if (a.ci_idx || a.co_idx || a.CIg > kMaxWRowsLds) return false;
-    int WR = 1;
-    while (WR < 8 && 2 * WR * a.CIg <= kMaxWRowsLds) WR *= 2;
-    const int CO = a.G * a.COg;
-    const int blocks = (CO + WR - 1) / WR;
-    hipLaunchKernelGGL((wrows_bwd_kernel<MODE>), dim3((unsigned)((blocks + 63) / 64 * 64)), dim3(256),
-                       (size_t)WR * a.CIg * sizeof(float), st, a, WR);
-    return true;
+    // no more rows than leave a workgroup per compute unit (us, one, two, four rows: 250 x 3072 x 1021 10.6, -, 8.3; intervals 17.6, -, 12.0;
+    // with as many as LDS holds 512 x 256 x 10 7.5 and now 3.6, 512 x 784 x 256 8.7 and 6.0)
+    w.WR = 1;
+    while (w.WR < 8 && 2 * w.WR * a.W_CIg <= kMaxWRowsLds && (a.G * a.W_COg + 2 * w.WR - 1) / (2 * w.WR) >= num_cus()) w.WR *= 2;
+    w.blocks = (unsigned)(((a.G * a.W_COg + w.WR - 1) / w.WR + 63) / 64 * 64);
+    w.lds = (size_t)w.WR * a.W_CIg * sizeof(float);
+    return SD_OK;
+}
+
+// grad_weight alone by rows; MODE as in weight_rows
+template <int MODE>
+static int launch_wrows(const BwdArgs& a, const WeightRows& w, hipStream_t st) {
+    if (a.ci_idx || a.co_idx) hipLaunchKernelGGL(wrows_lists_bwd_kernel, dim3(w.blocks), dim3(256), w.lds, st, a, w.WR, w.place);
+    else hipLaunchKernelGGL((wrows_bwd_kernel<MODE>), dim3(w.blocks), dim3(256), w.lds, st, a, w.WR);
+    return check_launch("wrows_bwd_kernel");
 }
 
 static int make_bwd_args(BwdArgs& a, const char* who, int B, int CO, int CI, int G, int HW,
@@ -323,18 +428,35 @@ template <bool SORT>
 static int run_scatter(BwdArgs& a, hipStream_t st) {
     int rc;
     float* gw_atomic = a.gw;      // grad_weight target of the atomics path, null once the row kernel has taken it
-    if (a.gw && launch_wrows<SORT ? 1 : 0>(a, st)) {
-        if ((rc = check_launch("wrows_bwd_kernel"))) return rc;
+    WeightRows w{};
+    if (a.gw && (rc = plan_wrows(a, !SORT, w, st))) return rc;
+    const int P = SORT ? 1 : positions_at_once(a, 1);
+    const unsigned x_rows = (unsigned)(a.B * a.G * ((a.HW + P - 1) / P));
+    // few rows: more work-items per row, so that enough position / index loads are in flight
+    const unsigned x_block = x_rows < 4u * (unsigned)num_cus() ? 1024 : 256;
+    if (w.WR) {
         gw_atomic = nullptr;
+        if (!SORT && a.CIg <= kMaxRowLds) {
+            const size_t x_lds = (size_t)a.CIg * P * sizeof(float), lds = w.lds > x_lds ? w.lds : x_lds;
+            const dim3 grid(w.blocks + x_rows), block(x_block);
+            if (a.ci_idx || a.co_idx) hipLaunchKernelGGL((both_bwd_kernel<3>), grid, block, lds, st, a, w.WR, w.place, w.blocks, P);
+            else hipLaunchKernelGGL((both_bwd_kernel<0>), grid, block, lds, st, a, w.WR, nullptr, w.blocks, P);
+            return check_launch("both_bwd_kernel");
+        }
+        if ((rc = launch_wrows<SORT ? 1 : 0>(a, w, st))) return rc;
     }
     if (gw_atomic && (rc = fill_zero(gw_atomic, (size_t)a.G * a.W_COg * a.W_CIg, st))) return rc;
     BwdArgs x = a;
     x.gw = gw_atomic;
+    if (P > 1 && !x.gw) {
+        hipLaunchKernelGGL(positions_bwd_kernel<false>, dim3(x_rows), dim3(x_block), (size_t)a.CIg * P * sizeof(float), st, x, P);
+        return check_launch("positions_bwd_kernel");
+    }
     if (a.CIg <= kMaxRowLds) {
         dim3 rows((unsigned)(a.B * a.G * a.HW));
-        // few rows: more work-items per row, so that enough position / index loads are in flight, and, where a row is sent many
-        // values (and grad_weight is not scattered as well), parts of the inputs until every compute unit has two workgroups
-        const dim3 block(rows.x < 4u * (unsigned)num_cus() ? 1024 : 256);
+        const dim3 block(x_block);
+        // where a row is sent many values (and grad_weight is not scattered as well), parts of the inputs until every compute unit
+        // has two workgroups
         if (SORT && !x.gw) {
             while (rows.y < 8u && rows.x * rows.y < 2u * (unsigned)num_cus() && a.CIg / (int)(2 * rows.y) >= 256) rows.y *= 2;
         }
@@ -418,11 +540,26 @@ static int bound_bwd(const char* who, const float* gL, const float* gU, const in
     a.g0 = gL; a.g1 = gU; a.p0 = posL; a.p1 = posU; a.gx0 = gxL; a.gx1 = gxU; a.gw = gw;
     hipStream_t st = static_cast<hipStream_t>(stream);
     size_t nx = (size_t)B * CI * HW;
-    if (gw && launch_wrows<2>(a, st)) {
-        if ((rc = check_launch("wrows_bwd_kernel"))) return rc;
+    WeightRows w{};
+    if (gw && (rc = plan_wrows(a, false, w, st))) return rc;
+    const int P = positions_at_once(a, 2);
+    const unsigned x_rows = (unsigned)(B * G * ((HW + P - 1) / P));
+    if (w.WR) {
+        if (2 * a.CIg <= kMaxRowLds) {
+            const size_t x_lds = (size_t)2 * a.CIg * P * sizeof(float), lds = w.lds > x_lds ? w.lds : x_lds;
+            hipLaunchKernelGGL((both_bwd_kernel<2>), dim3(w.blocks + x_rows), dim3(x_rows < 4u * (unsigned)num_cus() ? 1024 : 256), lds, st, a,
+                               w.WR, nullptr, w.blocks, P);
+            return check_launch("both_bwd_kernel");
+        }
+        if ((rc = launch_wrows<2>(a, w, st))) return rc;
         a.gw = gw = nullptr;
     }
     if (gw && (rc = fill_zero(gw, (size_t)CO * a.CIg, st))) return rc;
+    if (P > 1 && !gw) {
+        hipLaunchKernelGGL(positions_bwd_kernel<true>, dim3(x_rows), dim3(x_rows < 4u * (unsigned)num_cus() ? 1024 : 256),
+                           (size_t)2 * a.CIg * P * sizeof(float), st, a, P);
+        return check_launch("positions_bwd_kernel");
+    }
     if (2 * a.CIg <= kMaxRowLds) {
         dim3 rows((unsigned)(B * G * HW));
         size_t lds = (size_t)2 * a.CIg * sizeof(float);
