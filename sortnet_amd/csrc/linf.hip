@@ -1,6 +1,7 @@
 // l-inf distance, masked order-statistic neuron and interval-bound forward entry points.
 #include "fwd_tile.h"
 #include "fwd_args.h"
+#include "fwd_cols.h"
 #include "bound_cols.h"
 #include "sort_cols.h"
 #include "row_cands.h"
@@ -216,6 +217,13 @@ extern "C" int sd_inf_dist_forward_nograd(const float* input, const float* weigh
     hipStream_t st = static_cast<hipStream_t>(stream);
     const bool streamed = g_linf_density.load(std::memory_order_relaxed) <= 0.f;   // not where tables are forced
     if (streamed && row_stream_ok(a, kStreamMaxTerms)) return row_stream_linf(a, st);
+    if (cols_ok(a, kColsHW, kColsTerms) && workspace_ready(cols_workspace(a), st)) {
+        void* ws = workspace(cols_workspace(a), st);
+        if (!ws) return SD_ERR_HIP;
+        a.nsplit = cols_nsplit(a);
+        if (a.nsplit > 1 && (rc = fill_zero(output, (size_t)B * CO * HW, st))) return rc;
+        return cols_linf(a, ws, st);
+    }
     static const int kTb42[] = {4, 2};   // 8 rows per work-item measured slower (168 registers, three waves per SIMD)
     const bool narrow = narrow_tiles(a);
     const int TB = narrow ? 2 : pick_tb(a, kTb42, 2, 128);
@@ -247,6 +255,17 @@ extern "C" int sd_inf_dist_forward(const float* input, const float* weight,
     a.y0 = output; a.p0 = pos;
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (g_linf_density.load(std::memory_order_relaxed) <= 0.f && row_stream_ok(a, kStreamPosTerms)) return row_stream_linf(a, st);
+    if (cols_ok(a, kColsPosHW, kColsPosTerms)) {
+        a.nsplit = cols_nsplit(a);
+        const size_t weights = (cols_workspace(a) + 255) / 256 * 256, merge = a.nsplit > 1 ? (size_t)a.R * CO * 8 : 0;
+        if (workspace_ready(weights + merge, st)) {
+            char* ws = static_cast<char*>(workspace(weights + merge, st));
+            if (!ws) return SD_ERR_HIP;
+            a.packed0 = reinterpret_cast<unsigned long long*>(ws + weights);
+            if (merge && (rc = fill_zero(a.packed0, merge / 4, st))) return rc;
+            return cols_linf(a, ws, st);
+        }
+    }
     const int KE = max_cols_eligible(a, 1.f, B, CO, CI, G, HW);
     if (!KE) return run_chunk_pos<LinfChunk>(a, w_index_ci || w_index_co, st);
     const int K = max_cols_wanted(a, KE, kHintSiteLinf, B, CO, CI, st);

@@ -3,6 +3,7 @@
 #include <cstdlib>
 #include "fwd_tile.h"
 #include "fwd_args.h"
+#include "fwd_cols.h"
 #include "lp_grad.h"
 #include "lp_rows.h"
 
@@ -878,6 +879,18 @@ extern "C" int sd_norm_dist_forward(const float* input, const float* weight,
     const bool max_first = online && ((a.fast_x && a.fast_w && !w_index_co) || (lists && a.HW == 1));
     a.skip_thr = lp_skip_threshold(1e-6f / (float)a.CIg, p, max_first ? kLpSkipFrom : kLpSkipFromOnline);
     if (max_first) return lp_forward_max_first(a, small, st);
+    if (int_power(p) > 0 && cols_ok(a, kColsHW, kColsLpTerms)) {
+        a.nsplit = cols_nsplit(a);
+        a.part_stride = (size_t)a.R * a.G * a.COg;
+        const size_t weights = (cols_workspace(a) + 255) / 256 * 256, parts = a.nsplit > 1 ? a.part_stride * a.nsplit * 4 : 0;
+        if (workspace_ready(weights + parts, st)) {
+            char* ws = static_cast<char*>(workspace(weights + parts, st));
+            if (!ws) return SD_ERR_HIP;
+            a.part0 = reinterpret_cast<float*>(ws + weights);
+            if ((rc = cols_lp(int_power(p), a, ws, st))) return rc;
+            return lp_split_finish(a, st);
+        }
+    }
     if ((rc = lp_split_setup(a, small ? 32 : 64, narrow ? 32 : 128, online, st))) return rc;
     if (!online) {
         int ip = int_power(p);
