@@ -150,5 +150,7 @@ void hint_forget(unsigned long long* word);
 int fill_zero(void* ptr, size_t n_words, hipStream_t stream);
 // the same for two buffers with one launch
 int fill_zero2(void* a, size_t na_words, void* b, size_t nb_words, hipStream_t stream);
+// copies up to three matrices whose rows hold n values to rows of np, zeros behind the values, with one launch (rows: 0 for none)
+int pad_rows(const float* const (&src)[3], float* const (&dst)[3], const int (&rows)[3], int n, int np, hipStream_t stream);
 
 }  // namespace sd

@@ -436,7 +436,13 @@ bool row_stream_ok(const FwdArgs& a, long long limit) {
 }
 
 bool row_stream_sort_ok(const FwdArgs& a) {
-    const long long outputs = (long long)a.R * a.G * a.COg, most = a.x1 ? 3ll << 14 : 1ll << 16, per_input = a.x1 ? 56 : 80;
+    const long long outputs = (long long)a.R * a.G * a.COg, per_input = a.x1 ? 56 : 80;
+    long long most = a.x1 ? 3ll << 14 : 1ll << 16;
+    // Rows that are loaded value by value meet the tables on their padded copies earlier (in us, streamed -> tables at spreads 0.05 / 0.3
+    // / 3 of the inputs, K = 10): values 24 x 2199 x 2199 71 -> 40 / 56 / 67, 32 x 1067 x 1067 36 -> 28 / 42 / 36, 8 x 4443 x 4443 118 ->
+    // 71 / 90 / 110, 4 x 4443 x 4443 64 -> 70 / 83 / 61; intervals 16 x 1067 x 1067 54 -> 33 / 46 / 49, 4 x 4443 x 4443 109 -> 75 / 93 /
+    // 101, 2 x 4443 x 4443 60 -> 73 / 85 / 121.
+    if (!a.fast_w) most = a.x1 ? 1ll << 14 : a.CIg > 48 * 64 ? 1ll << 15 : 3ll << 14;
     return outputs <= most && outputs <= per_input * a.CIg && row_stream_ok(a, 1ll << 62);
 }
 

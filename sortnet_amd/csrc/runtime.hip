@@ -229,6 +229,39 @@ void hint_forget(unsigned long long* word) {
     if (word) __atomic_store_n(word, kHintVoid, __ATOMIC_RELEASE);
 }
 
+// A copy: bytes bound it (1306 x 1306 and twice 128 x 1306 in 5 us, of which 3 are the launch).
+struct PadArgs { const float* src[3]; float* dst[3]; int until[3]; };   // until: rows of the matrices up to and with this one
+__global__ void __launch_bounds__(256) pad_rows_kernel(PadArgs a, int n, int np) {
+    const int row = blockIdx.y * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (row >= a.until[2]) return;
+    const int k = row < a.until[0] ? 0 : row < a.until[1] ? 1 : 2, r = row - (k ? a.until[k - 1] : 0);
+    const float* src = a.src[k] + (size_t)r * n;
+    float* dst = a.dst[k] + (size_t)r * np;
+    float v[8];
+    #pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const int c = blockIdx.x * 512 + 64 * i + lane;
+        v[i] = c < n ? src[c] : 0.f;
+    }
+    #pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const int c = blockIdx.x * 512 + 64 * i + lane;
+        if (c < np) dst[c] = v[i];
+    }
+}
+
+int pad_rows(const float* const (&src)[3], float* const (&dst)[3], const int (&rows)[3], int n, int np, hipStream_t stream) {
+    PadArgs a;
+    int total = 0;
+    for (int k = 0; k < 3; k++) {
+        a.src[k] = src[k]; a.dst[k] = dst[k];
+        a.until[k] = total += rows[k];
+    }
+    SD_REQUIRE((total + 3) / 4 <= 65535, "pad_rows: %d rows", total);
+    hipLaunchKernelGGL(pad_rows_kernel, dim3((np + 511) / 512, (total + 3) / 4), dim3(256), 0, stream, a, n, np);
+    return check_launch("pad_rows");
+}
+
 __global__ void __launch_bounds__(256) fill_zero_kernel(uint32_t* __restrict__ p, size_t n) {
     size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     size_t stride = (size_t)gridDim.x * 256;

@@ -115,6 +115,7 @@ static bool two_level_ok(const FwdArgs& a, int K) {
 }
 
 // bytes of the two-level path's key lists
+static inline size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 static size_t two_level_bytes(const FwdArgs& a, int K) {
     return (size_t)(K + kKeySlack) * ((size_t)a.R * a.G * a.COg) * sizeof(int);
 }
@@ -165,12 +166,12 @@ static bool sort_cols_eligible(const FwdArgs& a, int B, int CO, int CI, int G, i
     return density > 0.f || (long long)B * CO * CI >= kSortColsMinTerms;
 }
 // eligible, and (with the built-in limit) the layer's tables have paid lately
-static bool sort_cols_ok(const FwdArgs& a, int site, int B, int CO, int CI, hipStream_t st) {
-    return g_sort_density.load(std::memory_order_relaxed) > 0.f || hint_build_tables(site, a.w, B, CO, CI, st);
+static bool sort_cols_ok(const float* weight, int site, int B, int CO, int CI, hipStream_t st) {
+    return g_sort_density.load(std::memory_order_relaxed) > 0.f || hint_build_tables(site, weight, B, CO, CI, st);
 }
 // before the every-term kernels are queued behind the table kernel: where they report
-static void sort_cols_expect(FwdArgs& a, int site, int B, int CO, int CI, hipStream_t st) {
-    if (g_sort_density.load(std::memory_order_relaxed) < 0.f && a.gate) a.told = hint_expect(site, a.w, B, CO, CI, st);
+static void sort_cols_expect(FwdArgs& a, const float* weight, int site, int B, int CO, int CI, hipStream_t st) {
+    if (g_sort_density.load(std::memory_order_relaxed) < 0.f && a.gate) a.told = hint_expect(site, weight, B, CO, CI, st);
 }
 
 // Largest share of marked (tile of 128 weight rows, batch row, input) triples at which the kernel of the tables per
@@ -221,6 +222,38 @@ static int queue_sort_cols(FwdArgs& a, int form, const float* xl, const float* x
     return SD_OK;
 }
 
+// Layers whose rows are no whole number of table words (32 inputs) work on copies of inputs and weights with zeros behind every
+// row: a term of 0 enters no list.  The kernels that form every term then load 16 bytes at a time, too.  Sets the shape of `a` and CI to
+// the copies' and returns their bytes, or 0 (as they were) where there are too few terms for tables: half as many do where rows of
+// whole 16 bytes have such kernels already (positions of 16 x 1300 x 1300 at a spread of 3 100 us, 107 with copies).
+// In us, without copies -> with them, inputs of spread 0.05 / 0.3 / 3 against unit weights, K = 10:
+//   values       128 x 1306 x 1306 160 -> 34 / 56 / 146, 250 x 3071 x 500 160 -> 42 / 70 / 108, 512 x 5001 x 2000 1660 -> 77 / 167 / 288
+//   interval     128 x 1306 x 1306 258 -> 38 / 70 / 190, 14 x 4443 x 4443 668 -> 85 / 123 / 204, 512 x 5001 x 2000 2602 -> 96 / 258 / 450
+//   positions    128 x 1306 x 1306 310 -> 45 / 153 / 179, 8 x 2198 x 2198 372 -> 51 / 65 / 152, 100 x 530 x 400 (21 M terms) 139 -> 34 / 143 / 114
+static size_t sort_pad(FwdArgs& a, int B, int CO, int& CI, int G, int HW) {
+    const int N = (CI + kSortColsChunk - 1) / kSortColsChunk * kSortColsChunk;
+    if (N == CI || G != 1 || HW != 1 || N > 65536 || (long long)(B + CO) * N >= (1ll << 31) || 2ll * B + CO > 4 * 65535) return 0;
+    const float density = g_sort_density.load(std::memory_order_relaxed);
+    if (density == 0.f || (density < 0.f && (long long)B * CO * CI < (CI % 4 == 0 ? 2 : 1) * kSortColsMinTerms)) return 0;
+    CI = a.CIg = a.W_CIg = N;
+    a.fast_x = a.fast_w = 1;
+    const size_t x = ((size_t)B * N * 4 + 255) / 256 * 256;
+    return (a.x1 ? 2 : 1) * x + ((size_t)CO * N * 4 + 255) / 256 * 256;
+}
+// makes the copies; `raw`: the call's own operands
+static int sort_pad_copy(FwdArgs& a, const FwdArgs& raw, void* mem, hipStream_t st) {
+    const size_t x = ((size_t)a.B * a.CIg * 4 + 255) / 256 * 256;
+    char* p = static_cast<char*>(mem);
+    float* x0 = reinterpret_cast<float*>(p);
+    float* x1 = a.x1 ? reinterpret_cast<float*>(p + x) : x0;
+    float* w = reinterpret_cast<float*>(p + (a.x1 ? 2 : 1) * x);
+    const int rc = pad_rows({raw.x0, raw.x1, raw.w}, {x0, x1, w}, {a.B, a.x1 ? a.B : 0, a.COg}, raw.CIg, a.CIg, st);
+    a.x0 = x0;
+    if (a.x1) a.x1 = x1;
+    a.w = w;
+    return rc;
+}
+
 extern "C" int sd_set_sort_candidate_density(float density) {
     SD_REQUIRE(density <= 1.f, "set_sort_candidate_density: %g is above 1", (double)density);
     g_sort_density = density;
@@ -247,21 +280,27 @@ extern "C" int sd_sort_neuron_forward_nograd(const float* input, const float* we
     if (g_sort_density.load(std::memory_order_relaxed) <= 0.f && row_stream_sort_ok(a))
         return row_stream_sort(a, K, st);
     const bool small = few_tiles(a, 32, 64), streamed = g_sort_density.load(std::memory_order_relaxed) <= 0.f && row_stream_sort_before_terms(a);
+    const FwdArgs raw = a;
+    size_t copies = sort_pad(a, B, CO, CI, G, HW);
+    if (copies && !workspace_ready(sort_tables_bytes(kRowsSortValues, B, CO, CI, K) + (two_level_ok(a, K) ? align256(two_level_bytes(a, K)) : 0) + copies, st)) {
+        a = raw; CI = raw.CIg; copies = 0;
+    }
     const bool two = K <= 12 && two_level_ok(a, K), elig = sort_cols_eligible(a, B, CO, CI, G, HW);
-    const bool cols = elig && sort_cols_ok(a, kHintSiteSort, B, CO, CI, st);
+    const bool cols = elig && sort_cols_ok(weight, kHintSiteSort, B, CO, CI, st);
     if (streamed && !elig) return row_stream_sort(a, K, st);
     // one request for both users of the workspace: the tables (with the counter the gates read) first, the key
     // lists of the two-level path behind them
-    const size_t tbytes = elig ? sort_tables_bytes(kRowsSortValues, B, CO, CI, K) : 0;
+    const size_t tbytes = elig ? sort_tables_bytes(kRowsSortValues, B, CO, CI, K) : 0, kbytes = two ? align256(two_level_bytes(a, K)) : 0;
     char* base = nullptr;
     if (elig || two) {
-        base = static_cast<char*>(workspace(tbytes + (two ? two_level_bytes(a, K) : 0), st));
+        base = static_cast<char*>(workspace(tbytes + kbytes + copies, st));
         if (!base) return SD_ERR_HIP;
     }
-    if (streamed && !cols) return row_stream_sort(a, K, st);
+    if (streamed && !cols) return row_stream_sort(raw, K, st);
+    if (copies && (rc = sort_pad_copy(a, raw, base + tbytes + kbytes, st))) return rc;
     int* keys = reinterpret_cast<int*>(base + tbytes);
-    if (cols && (rc = queue_sort_cols(a, kRowsSortValues, input, nullptr, weight, B, CO, CI, q, K, nullptr, output, nullptr, base, st))) return rc;
-    if (cols) sort_cols_expect(a, kHintSiteSort, B, CO, CI, st);
+    if (cols && (rc = queue_sort_cols(a, kRowsSortValues, a.x0, nullptr, a.w, B, CO, CI, q, K, nullptr, output, nullptr, base, st))) return rc;
+    if (cols) sort_cols_expect(a, weight, kHintSiteSort, B, CO, CI, st);
     rc = SD_ERR_ARG;
     switch (K) {
 #define X(k) case k: if (k <= 12 && two) rc = run_two_level<(k <= 12 ? k : 2), true>(a, small, keys, st); \
@@ -287,19 +326,25 @@ extern "C" int sd_sort_neuron_forward(const float* input, const float* weight,
     a.y0 = output; a.p0 = pos; a.q = q;
     hipStream_t st = static_cast<hipStream_t>(stream);
     const bool small = few_tiles(a, 32, 32);
+    const FwdArgs raw = a;
+    size_t copies = sort_pad(a, B, CO, CI, G, HW);
+    if (copies && !workspace_ready(sort_tables_bytes(kRowsSortPos, B, CO, CI, K) + (two_level_ok(a, K) ? align256(two_level_bytes(a, K)) : 0) + copies, st)) {
+        a = raw; CI = raw.CIg; copies = 0;
+    }
     const bool two = K <= 12 && two_level_ok(a, K);
     const bool elig = sort_cols_eligible(a, B, CO, CI, G, HW);
-    const bool cols = elig && sort_cols_ok(a, kHintSiteSortPos, B, CO, CI, st);
+    const bool cols = elig && sort_cols_ok(weight, kHintSiteSortPos, B, CO, CI, st);
     // one request for both users of the workspace, as in sd_sort_neuron_forward_nograd
-    const size_t tbytes = elig ? sort_tables_bytes(kRowsSortPos, B, CO, CI, K) : 0;
+    const size_t tbytes = elig ? sort_tables_bytes(kRowsSortPos, B, CO, CI, K) : 0, kbytes = two ? align256(two_level_bytes(a, K)) : 0;
     char* base = nullptr;
     if (elig || two) {
-        base = static_cast<char*>(workspace(tbytes + (two ? two_level_bytes(a, K) : 0), st));
+        base = static_cast<char*>(workspace(tbytes + kbytes + copies, st));
         if (!base) return SD_ERR_HIP;
     }
+    if (copies && (rc = sort_pad_copy(a, raw, base + tbytes + kbytes, st))) return rc;
     int* keys = reinterpret_cast<int*>(base + tbytes);
-    if (cols && (rc = queue_sort_cols(a, kRowsSortPos, input, nullptr, weight, B, CO, CI, q, K, nullptr, output, pos, base, st))) return rc;
-    if (cols) sort_cols_expect(a, kHintSiteSortPos, B, CO, CI, st);
+    if (cols && (rc = queue_sort_cols(a, kRowsSortPos, a.x0, nullptr, a.w, B, CO, CI, q, K, nullptr, output, pos, base, st))) return rc;
+    if (cols) sort_cols_expect(a, weight, kHintSiteSortPos, B, CO, CI, st);
     rc = SD_ERR_ARG;
     switch (K) {
 #define X(k) case k: if (k <= 12 && two) rc = run_two_level<(k <= 12 ? k : 2), false>(a, few_tiles(a, 32, 64), keys, st); \
@@ -327,15 +372,21 @@ extern "C" int sd_bound_sort_neuron_forward(const float* inputL, const float* in
     if (g_sort_density.load(std::memory_order_relaxed) <= 0.f && row_stream_sort_ok(a))
         return row_stream_sort(a, K, st);
     const bool small = few_tiles(a, 32, 32);
+    const FwdArgs raw = a;
+    size_t copies = sort_pad(a, B, CO, CI, G, HW);
+    if (copies && !workspace_ready(sort_tables_bytes(kRowsSortInterval, B, CO, CI, K) + copies, st)) { a = raw; CI = raw.CIg; copies = 0; }
     const bool elig = sort_cols_eligible(a, B, CO, CI, G, HW);
-    const bool cols = elig && sort_cols_ok(a, kHintSiteBoundSort, B, CO, CI, st);
+    const bool cols = elig && sort_cols_ok(weight, kHintSiteBoundSort, B, CO, CI, st);
+    const bool streamed = !cols && g_sort_density.load(std::memory_order_relaxed) <= 0.f && row_stream_sort_before_terms(raw);
     if (elig) {
-        void* ws = workspace(sort_tables_bytes(kRowsSortInterval, B, CO, CI, K), st);   // the only request of this call
+        const size_t tbytes = sort_tables_bytes(kRowsSortInterval, B, CO, CI, K);
+        char* ws = static_cast<char*>(workspace(tbytes + copies, st));   // the only request of this call
         if (!ws) return SD_ERR_HIP;
-        if (cols && (rc = queue_sort_cols(a, kRowsSortInterval, inputL, inputU, weight, B, CO, CI, q, K, outputL, outputU, nullptr, ws, st))) return rc;
+        if (copies && !streamed && (rc = sort_pad_copy(a, raw, ws + tbytes, st))) return rc;
+        if (cols && (rc = queue_sort_cols(a, kRowsSortInterval, a.x0, a.x1, a.w, B, CO, CI, q, K, outputL, outputU, nullptr, ws, st))) return rc;
     }
-    if (!cols && g_sort_density.load(std::memory_order_relaxed) <= 0.f && row_stream_sort_before_terms(a)) return row_stream_sort(a, K, st);
-    if (cols) sort_cols_expect(a, kHintSiteBoundSort, B, CO, CI, st);
+    if (streamed) return row_stream_sort(raw, K, st);
+    if (cols) sort_cols_expect(a, weight, kHintSiteBoundSort, B, CO, CI, st);
     rc = SD_ERR_ARG;
     switch (K) {
 #define X(k) case k: rc = small ? launch_fwd<BoundSort<k>, 1, 2>(a, st) : launch_fwd<BoundSort<k>, 2, 2>(a, st); break;

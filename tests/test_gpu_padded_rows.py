@@ -1,0 +1,58 @@
+"""Sort neuron of layers whose rows are no multiple of 32 inputs, on padded copies: one to 31 inputs missing, one batch row, batch
+tiles that are not full, tables that serve and tables that do not, ties, undefined inputs; a stream under capture that has not run
+the call.  Values, bounds and positions bit for bit against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+Q, K = 0.75, 10
+
+
+def _data(B, N, M, spread, seed=0):
+    g = torch.Generator().manual_seed(B + N + seed)
+    return torch.randn(B, N, 1, generator=g) * spread, torch.randn(M, N, generator=g)
+
+
+def _run(x, w):
+    from sortnet_amd import ext
+    B, M = x.shape[0], w.shape[0]
+    new = lambda *s: torch.full(s, 7.0, device="cuda")   # noqa: E731
+    y, yp, lo, up, pos = new(B, M, 1), new(B, M, 1), new(B, M, 1), new(B, M, 1), torch.full((K, B, M, 1), 7, device="cuda", dtype=torch.int32)
+    ext.sort_neuron_forward_nograd(x, w, y, 1, Q, K)
+    ext.sort_neuron_forward(x, w, yp, pos, 1, Q, K)
+    ext.bound_sort_neuron_forward(x - 0.03, x + 0.03, w, lo, up, 1, Q, K)
+    return y, yp, pos, lo, up
+
+
+@pytest.mark.parametrize("B,N,M,spread,kind", [
+    (1, 4129, 4100, 0.3, ""), (129, 1055, 140, 0.05, "odd"), (70, 1567, 161, 0.3, "ties"), (300, 335, 300, 3.0, ""), (260, 1030, 130, 0.3, "odd"),
+    (64, 4081, 65, 1.0, "ties"), (33, 2049, 251, 0.05, ""), (130, 12290, 11, 0.3, "")])
+def test_against_the_oracle(oracle, B, N, M, spread, kind):
+    x, w = _data(B, N, M, spread)
+    if kind == "ties":
+        x, w = (x * 4).round() / 4, (w * 4).round() / 4
+    if kind == "odd":
+        x[0, 3], w[1, 2], x[1, N - 1], w[2, N - 1] = float("nan"), float("inf"), float("inf"), float("nan")
+    y, yp, pos, lo, up = _run(x.cuda(), w.cuda())
+    ry, rp = oracle.sort_neuron_forward(x.numpy(), w.numpy(), Q, K)
+    rl, ru = oracle.bound_sort_neuron_forward((x - 0.03).numpy(), (x + 0.03).numpy(), w.numpy(), Q, K)
+    for got, want in ((y, ry), (yp, ry), (lo, rl), (up, ru)):
+        np.testing.assert_array_equal(got.cpu().numpy(), want)
+    np.testing.assert_array_equal(pos.cpu().numpy(), np.asarray(rp).astype(np.int32).reshape(tuple(pos.shape)))
+
+
+def test_tables_serve_and_capture_needs_no_scratch():
+    from sortnet_amd import _lib
+    x, w = (t.cuda() for t in _data(128, 1306, 1306, 0.05))
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        fresh = _run(x, w)                       # a stream without a workspace: every term
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        want = _run(x, w)
+        assert _lib.last_forward_term_share() < 0.5
+        for a, b in zip(fresh, want):
+            assert torch.equal(a, b)
+            a.zero_()

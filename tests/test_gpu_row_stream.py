@@ -113,11 +113,19 @@ def test_batch_rows_dealt_to_workgroups(oracle, B, n, m):
     np.testing.assert_allclose(y2.cpu().numpy(), ru.reshape(B, m, 1), rtol=1e-5, atol=1e-6)
 
 
-# layers of more outputs than the limit against tables, in shapes that have none: the kernel that streams still comes before the one
+@pytest.fixture
+def no_sort_tables():
+    from sortnet_amd import _lib
+    _lib.set_sort_candidate_density(0.0)
+    yield
+    _lib.set_sort_candidate_density(-1.0)
+
+
+# layers of more outputs than the limit against tables, where there are none: the kernel that streams still comes before the one
 # that forms every term, up to its own limit and not beyond
 @pytest.mark.parametrize("B,n,m,streams,bounds", [(100, 639, 630, True, True), (150, 500, 500, True, False), (40, 1657, 1659, True, True),
                                                   (20, 3333, 3334, True, False), (151, 500, 500, False, False)])
-def test_layers_without_tables(oracle, B, n, m, streams, bounds):
+def test_layers_without_tables(oracle, no_sort_tables, B, n, m, streams, bounds):
     from sortnet_amd import _lib, ext
     x, w = _data((B, n, m, 1), "ties" if B == 100 else "normal")
     xd, wd = x.cuda(), w.cuda()
