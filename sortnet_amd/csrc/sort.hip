@@ -153,17 +153,23 @@ static float sort_cols_cap(int form, int CI) {
     return form == kRowsSortPos ? 0.22f : form == kRowsSortValues && CI < 320 ? 0.10f : 0.40f;
 }
 constexpr long long kSortColsMinTerms = 1ll << 24;
+// Positions have no kernel that streams the weights, and every term of a few outputs is formed by few wavefronts: tables from 2^20 terms on
+// where rows are at least 320 inputs long.  Every term -> tables at spreads 0.05 / 0.3 of the inputs, K = 10: 99 x 2304 x 59 107 -> 36, 121 -> 66; 50 x
+// 1000 x 64 238 -> 36, 286 -> 57; 128 x 5120 x 10 180 -> 39, 198 -> 82; 16 x 320 x 250 112 -> 33; where they do not serve (64 x 512 x 64 at
+// 0.3, 185 us) building them takes 18 us, for one call in 32.
+constexpr long long kSortPosMinTerms = 1ll << 20;
+static long long sort_cols_min_terms(bool pos, int CI) { return pos && CI >= 320 ? kSortPosMinTerms : kSortColsMinTerms; }
 
 // `site`: which entry point asks (with the built-in limit, a layer whose tables have not paid lately is not given
 // any for a while, see hint_build_tables)
 constexpr int kHintSiteSort = 2, kHintSiteBoundSort = 3, kHintSiteSortPos = 6;
 // shape and size alone: the workspace is sized by this, so that a call under graph capture (which always builds
 // tables) never needs more than the eager call before it did
-static bool sort_cols_eligible(const FwdArgs& a, int B, int CO, int CI, int G, int HW) {
+static bool sort_cols_eligible(const FwdArgs& a, bool pos, int B, int CO, int CI, int G, int HW) {
     const float density = g_sort_density.load(std::memory_order_relaxed);
     // the mark lists of the table kernels hold 16-bit input numbers
     if (density == 0.f || G != 1 || HW != 1 || CI % kSortColsChunk != 0 || CI > 65536 || !a.fast_x || !a.fast_w) return false;
-    return density > 0.f || (long long)B * CO * CI >= kSortColsMinTerms;
+    return density > 0.f || (long long)B * CO * CI >= sort_cols_min_terms(pos, CI);
 }
 // eligible, and (with the built-in limit) the layer's tables have paid lately
 static bool sort_cols_ok(const float* weight, int site, int B, int CO, int CI, hipStream_t st) {
@@ -223,18 +229,18 @@ static int queue_sort_cols(FwdArgs& a, int form, const float* xl, const float* x
 }
 
 // Layers whose rows are no whole number of table words (32 inputs) work on copies of inputs and weights with zeros behind every
-// row: a term of 0 enters no list.  The kernels that form every term then load 16 bytes at a time, too.  Sets the shape of `a` and CI to
-// the copies' and returns their bytes, or 0 (as they were) where there are too few terms for tables: half as many do where rows of
-// whole 16 bytes have such kernels already (positions of 16 x 1300 x 1300 at a spread of 3 100 us, 107 with copies).
+// row: a term of 0 enters no list.  The kernels that form every term then load 16 bytes at a time, too; rows that did so anyway
+// are only copied for a call that builds tables.  Sets the shape of `a` and CI to the copies' and returns their bytes, or 0 (as they
+// were) where there are too few terms for tables.
 // In us, without copies -> with them, inputs of spread 0.05 / 0.3 / 3 against unit weights, K = 10:
 //   values       128 x 1306 x 1306 160 -> 34 / 56 / 146, 250 x 3071 x 500 160 -> 42 / 70 / 108, 512 x 5001 x 2000 1660 -> 77 / 167 / 288
 //   interval     128 x 1306 x 1306 258 -> 38 / 70 / 190, 14 x 4443 x 4443 668 -> 85 / 123 / 204, 512 x 5001 x 2000 2602 -> 96 / 258 / 450
-//   positions    128 x 1306 x 1306 310 -> 45 / 153 / 179, 8 x 2198 x 2198 372 -> 51 / 65 / 152, 100 x 530 x 400 (21 M terms) 139 -> 34 / 143 / 114
-static size_t sort_pad(FwdArgs& a, int B, int CO, int& CI, int G, int HW) {
+//   positions    128 x 1306 x 1306 310 -> 45 / 153 / 179, 8 x 2198 x 2198 372 -> 51 / 65 / 152, 99 x 2303 x 59 450 -> 41 / 74 / 106
+static size_t sort_pad(FwdArgs& a, bool pos, int B, int CO, int& CI, int G, int HW) {
     const int N = (CI + kSortColsChunk - 1) / kSortColsChunk * kSortColsChunk;
     if (N == CI || G != 1 || HW != 1 || N > 65536 || (long long)(B + CO) * N >= (1ll << 31) || 2ll * B + CO > 4 * 65535) return 0;
     const float density = g_sort_density.load(std::memory_order_relaxed);
-    if (density == 0.f || (density < 0.f && (long long)B * CO * CI < (CI % 4 == 0 ? 2 : 1) * kSortColsMinTerms)) return 0;
+    if (density == 0.f || (density < 0.f && (long long)B * CO * CI < sort_cols_min_terms(pos, N))) return 0;
     CI = a.CIg = a.W_CIg = N;
     a.fast_x = a.fast_w = 1;
     const size_t x = ((size_t)B * N * 4 + 255) / 256 * 256;
@@ -252,6 +258,14 @@ static int sort_pad_copy(FwdArgs& a, const FwdArgs& raw, void* mem, hipStream_t 
     if (a.x1) a.x1 = x1;
     a.w = w;
     return rc;
+}
+
+// what a call does that has copies planned but builds no tables: whether it goes on without them
+static bool sort_unpad(FwdArgs& a, const FwdArgs& raw, int& CI, bool tables) {
+    if (tables || !(raw.fast_x && raw.fast_w)) return false;
+    a = raw;
+    CI = raw.CIg;
+    return true;
 }
 
 extern "C" int sd_set_sort_candidate_density(float density) {
@@ -281,11 +295,11 @@ extern "C" int sd_sort_neuron_forward_nograd(const float* input, const float* we
         return row_stream_sort(a, K, st);
     const bool small = few_tiles(a, 32, 64), streamed = g_sort_density.load(std::memory_order_relaxed) <= 0.f && row_stream_sort_before_terms(a);
     const FwdArgs raw = a;
-    size_t copies = sort_pad(a, B, CO, CI, G, HW);
+    size_t copies = sort_pad(a, false, B, CO, CI, G, HW);
     if (copies && !workspace_ready(sort_tables_bytes(kRowsSortValues, B, CO, CI, K) + (two_level_ok(a, K) ? align256(two_level_bytes(a, K)) : 0) + copies, st)) {
         a = raw; CI = raw.CIg; copies = 0;
     }
-    const bool two = K <= 12 && two_level_ok(a, K), elig = sort_cols_eligible(a, B, CO, CI, G, HW);
+    const bool two = K <= 12 && two_level_ok(a, K), elig = sort_cols_eligible(a, false, B, CO, CI, G, HW);
     const bool cols = elig && sort_cols_ok(weight, kHintSiteSort, B, CO, CI, st);
     if (streamed && !elig) return row_stream_sort(a, K, st);
     // one request for both users of the workspace: the tables (with the counter the gates read) first, the key
@@ -297,7 +311,7 @@ extern "C" int sd_sort_neuron_forward_nograd(const float* input, const float* we
         if (!base) return SD_ERR_HIP;
     }
     if (streamed && !cols) return row_stream_sort(raw, K, st);
-    if (copies && (rc = sort_pad_copy(a, raw, base + tbytes + kbytes, st))) return rc;
+    if (copies && !sort_unpad(a, raw, CI, cols) && (rc = sort_pad_copy(a, raw, base + tbytes + kbytes, st))) return rc;
     int* keys = reinterpret_cast<int*>(base + tbytes);
     if (cols && (rc = queue_sort_cols(a, kRowsSortValues, a.x0, nullptr, a.w, B, CO, CI, q, K, nullptr, output, nullptr, base, st))) return rc;
     if (cols) sort_cols_expect(a, weight, kHintSiteSort, B, CO, CI, st);
@@ -327,12 +341,16 @@ extern "C" int sd_sort_neuron_forward(const float* input, const float* weight,
     hipStream_t st = static_cast<hipStream_t>(stream);
     const bool small = few_tiles(a, 32, 32);
     const FwdArgs raw = a;
-    size_t copies = sort_pad(a, B, CO, CI, G, HW);
-    if (copies && !workspace_ready(sort_tables_bytes(kRowsSortPos, B, CO, CI, K) + (two_level_ok(a, K) ? align256(two_level_bytes(a, K)) : 0) + copies, st)) {
+    size_t copies = sort_pad(a, true, B, CO, CI, G, HW);
+    const bool vectors = K <= 12 && two_level_ok(a, K);
+    bool elig = sort_cols_eligible(a, true, B, CO, CI, G, HW);
+    // (what was formed without scratch, or with the key lists alone, can be captured unprepared)
+    if (elig && (copies || (long long)B * CO * CI < kSortColsMinTerms) &&
+        !workspace_ready(sort_tables_bytes(kRowsSortPos, B, CO, CI, K) + (vectors ? align256(two_level_bytes(a, K)) : 0) + copies, st)) {
+        elig = false;
         a = raw; CI = raw.CIg; copies = 0;
     }
     const bool two = K <= 12 && two_level_ok(a, K);
-    const bool elig = sort_cols_eligible(a, B, CO, CI, G, HW);
     const bool cols = elig && sort_cols_ok(weight, kHintSiteSortPos, B, CO, CI, st);
     // one request for both users of the workspace, as in sd_sort_neuron_forward_nograd
     const size_t tbytes = elig ? sort_tables_bytes(kRowsSortPos, B, CO, CI, K) : 0, kbytes = two ? align256(two_level_bytes(a, K)) : 0;
@@ -341,7 +359,7 @@ extern "C" int sd_sort_neuron_forward(const float* input, const float* weight,
         base = static_cast<char*>(workspace(tbytes + kbytes + copies, st));
         if (!base) return SD_ERR_HIP;
     }
-    if (copies && (rc = sort_pad_copy(a, raw, base + tbytes + kbytes, st))) return rc;
+    if (copies && !sort_unpad(a, raw, CI, cols) && (rc = sort_pad_copy(a, raw, base + tbytes + kbytes, st))) return rc;
     int* keys = reinterpret_cast<int*>(base + tbytes);
     if (cols && (rc = queue_sort_cols(a, kRowsSortPos, a.x0, nullptr, a.w, B, CO, CI, q, K, nullptr, output, pos, base, st))) return rc;
     if (cols) sort_cols_expect(a, weight, kHintSiteSortPos, B, CO, CI, st);
@@ -373,16 +391,16 @@ extern "C" int sd_bound_sort_neuron_forward(const float* inputL, const float* in
         return row_stream_sort(a, K, st);
     const bool small = few_tiles(a, 32, 32);
     const FwdArgs raw = a;
-    size_t copies = sort_pad(a, B, CO, CI, G, HW);
+    size_t copies = sort_pad(a, false, B, CO, CI, G, HW);
     if (copies && !workspace_ready(sort_tables_bytes(kRowsSortInterval, B, CO, CI, K) + copies, st)) { a = raw; CI = raw.CIg; copies = 0; }
-    const bool elig = sort_cols_eligible(a, B, CO, CI, G, HW);
+    const bool elig = sort_cols_eligible(a, false, B, CO, CI, G, HW);
     const bool cols = elig && sort_cols_ok(weight, kHintSiteBoundSort, B, CO, CI, st);
     const bool streamed = !cols && g_sort_density.load(std::memory_order_relaxed) <= 0.f && row_stream_sort_before_terms(raw);
     if (elig) {
         const size_t tbytes = sort_tables_bytes(kRowsSortInterval, B, CO, CI, K);
         char* ws = static_cast<char*>(workspace(tbytes + copies, st));   // the only request of this call
         if (!ws) return SD_ERR_HIP;
-        if (copies && !streamed && (rc = sort_pad_copy(a, raw, ws + tbytes, st))) return rc;
+        if (copies && !streamed && !sort_unpad(a, raw, CI, cols) && (rc = sort_pad_copy(a, raw, ws + tbytes, st))) return rc;
         if (cols && (rc = queue_sort_cols(a, kRowsSortInterval, a.x0, a.x1, a.w, B, CO, CI, q, K, outputL, outputU, nullptr, ws, st))) return rc;
     }
     if (streamed) return row_stream_sort(raw, K, st);
