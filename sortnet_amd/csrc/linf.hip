@@ -451,6 +451,36 @@ static int bound_tables_eligible(const FwdArgs& a, float cap, int B, int CO, int
     return terms >= kBoundRowsMinTerms + kBoundRowsMinOutputs * CI && bound_rows_bytes(B, CO, CI) > 0 ? 1 : 0;
 }
 
+// Interval layers whose rows are no whole number of table words (32 inputs) work on copies of bounds and weights with zeros behind every
+// row, whose terms raise no bound.  Sets the shape of `a` and CI to the copies' and returns their bytes, or 0 (as they were).  Rows that
+// can be loaded 16 bytes at a time are copied for tables that a probe of the operands goes before (without it, images gain 96 -> 74 us at
+// 118 x 2596 x 2596, and rows that are alike pay 94 -> 103, one call in 32 with tables); others also for the kernels that load so.
+// In us, without copies -> with them, inputs in [0, 1] / centred, spread 0.05, weights ~ N(0, 1 / inputs) / the same, weights ~ N(0, 1):
+//   without positions  250 x 3071 x 1021 120 -> 56 / 118 -> 61 / 118 -> 99, 300 x 3001 x 3000 355 -> 134 / 360 -> 137 / 357 -> 70, 53 x 10187 x
+//                      1472 (no tables) 162 -> 136, 100 x 1001 x 1400 34 -> 31
+//   with them          250 x 3071 x 1021 155 -> 70 / 155 -> 75 / 154 -> 126, 300 x 3001 x 3000 621 -> 171 / 622 -> 166 / 620 -> 211, 53 x 10187 x
+//                      1472 211 -> 149, 100 x 1001 x 1400 57 -> 51
+constexpr long long kBoundPadMinTerms = 1ll << 27;
+static size_t bound_pad(FwdArgs& a, float cap, int B, int CO, int& CI, int G, int HW) {
+    const int N = (CI + kColsChunk - 1) / kColsChunk * kColsChunk;
+    if (N == CI || a.G != 1 || a.HW != 1 || N > 65536 || (long long)(B + CO) * N >= (1ll << 31) || 2ll * B + CO > 4 * 65535) return 0;
+    FwdArgs t = a;
+    t.CIg = t.W_CIg = N;
+    t.fast_x = t.fast_w = 1;
+    const bool vectors = a.fast_x && a.fast_w;
+    if (bound_tables_eligible(t, cap, B, CO, N, G, HW) < (vectors ? 2 : 1) && (vectors || (long long)B * CO * CI < kBoundPadMinTerms)) return 0;
+    a = t;
+    CI = N;
+    return 2 * (((size_t)B * N * 4 + 255) / 256 * 256) + ((size_t)CO * N * 4 + 255) / 256 * 256;
+}
+static int bound_pad_copy(FwdArgs& a, const FwdArgs& raw, char* mem, hipStream_t st) {
+    const size_t x = ((size_t)a.R * a.CIg * 4 + 255) / 256 * 256;
+    float *l = reinterpret_cast<float*>(mem), *u = reinterpret_cast<float*>(mem + x), *w = reinterpret_cast<float*>(mem + 2 * x);
+    const int rc = pad_rows({raw.x0, raw.x1, raw.w}, {l, u, w}, {a.R, a.R, a.COg}, raw.CIg, a.CIg, st);
+    a.x0 = l; a.x1 = u; a.w = w;
+    return rc;
+}
+
 extern "C" int sd_bound_inf_dist_forward_nograd(const float* inputL, const float* inputU, const float* weight,
                                                 int B, int CO, int CI, int G, int HW, float* outputL, float* outputU,
                                                 sd_stream_t stream) {
@@ -464,28 +494,38 @@ extern "C" int sd_bound_inf_dist_forward_nograd(const float* inputL, const float
     a.y0 = outputL; a.y1 = outputU;
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (g_bound_density.load(std::memory_order_relaxed) <= 0.f && row_stream_ok(a, kStreamBoundTerms)) return row_stream_bound(a, st);
-    static const int kTb42[] = {4, 2};
-    const bool narrow = narrow_tiles(a);
-    const int TB = narrow ? 2 : pick_tb(a, kTb42, 2, 128);
-    a.nsplit = pick_nsplit(a, 16 * TB, narrow ? 32 : 128);
     // dense single-group layers: a kernel that works from per-weight-row candidate tables is queued in front of the
     // one that evaluates every term, and a count taken on the device decides which of the two runs
     const float bound_density = g_bound_density.load(std::memory_order_relaxed);
     const int bound_form = g_bound_form.load(std::memory_order_relaxed);
     const float cap = bound_density >= 0.f ? bound_density : kBoundColsCap;
+    const FwdArgs raw = a;
+    size_t copies = bound_pad(a, cap, B, CO, CI, G, HW);
     int tables = bound_tables_eligible(a, cap, B, CO, CI, G, HW);
     // The workspace is sized by shape alone (whatever the hints below decide), so that a call under graph capture, for
     // which they may decide otherwise, never needs more than the eager call before it did.
     char* wsbase = nullptr;
-    if (tables) {
-        const size_t both = bound_tables_bytes(tables == 2, B, CO, CI), walk = tables == 2 && CI <= 65536 ? sort_cols_workspace(B, CO, CI) : 0;
+    size_t cbytes = 0;
+    if (tables || copies) {
+        const size_t both = !tables ? 0 : bound_tables_bytes(tables == 2, B, CO, CI), walk = tables == 2 && CI <= 65536 ? sort_cols_workspace(B, CO, CI) : 0;
         const size_t bytes = both > walk ? both : walk;
-        if (bound_density < 0.f && !workspace_ready(bytes, st)) tables = 0;   // a first call under capture forms every term
-        else if (!(wsbase = static_cast<char*>(workspace(bytes, st)))) return SD_ERR_HIP;   // the only request of this call
+        cbytes = (bytes + 255) / 256 * 256;
+        if ((bound_density < 0.f || copies) && !workspace_ready(cbytes + copies, st)) tables = 0;   // a first call under capture forms every term
+        else if (!(wsbase = static_cast<char*>(workspace(cbytes + copies, st)))) return SD_ERR_HIP;   // the only request of this call
     }
     // with the built-in limit, a layer whose tables have not paid lately is not given any for a while
     const bool hinted = tables && bound_density < 0.f;
     if (hinted && !hint_build_tables(kHintSiteBound, weight, B, CO, CI, st, tables == 1)) tables = 0;
+    if (copies) {
+        // without tables the copies serve rows that could not be loaded 16 bytes at a time
+        if (wsbase && (tables || !(raw.fast_x && raw.fast_w))) {
+            if ((rc = bound_pad_copy(a, raw, wsbase + cbytes, st))) return rc;
+        } else { a = raw; CI = raw.CIg; }
+    }
+    static const int kTb42[] = {4, 2};
+    const bool narrow = narrow_tiles(a);
+    const int TB = narrow ? 2 : pick_tb(a, kTb42, 2, 128);
+    a.nsplit = pick_nsplit(a, 16 * TB, narrow ? 32 : 128);
     // Very few marks (weights of unit scale against rows that are alike: below 1 %): the staged kernel would spend its
     // time moving tiles through LDS, and the kernel that walks a weight row's marks over a transposed copy of the
     // inputs serves better.  Chosen by hand (sd_set_bound_candidate_form) or, with the built-in limit, for a layer
@@ -498,7 +538,7 @@ extern "C" int sd_bound_inf_dist_forward_nograd(const float* inputL, const float
         if (a.nsplit > 1) {   // the every-term kernel, should it run, merges its slices into zeros
             if ((rc = fill_zero2(outputL, (size_t)B * CO * HW, outputU, (size_t)B * CO * HW, st))) return rc;
         }
-        if ((rc = sort_cols_forward(inputL, inputU, weight, B, CO, CI, 0.f, 1, outputL, outputU, nullptr, ws,
+        if ((rc = sort_cols_forward(a.x0, a.x1, a.w, B, CO, CI, 0.f, 1, outputL, outputU, nullptr, ws,
                                     bound_density > 0.f ? bound_density : kBoundSparseCap, &a.gate, &a.gate_limit, st)))
             return rc;
         a.gate_above = 1;
@@ -550,26 +590,35 @@ extern "C" int sd_bound_inf_dist_forward(const float* inputL, const float* input
     a.y0 = outputL; a.y1 = outputU; a.p0 = posL; a.p1 = posU;
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (g_bound_density.load(std::memory_order_relaxed) <= 0.f && row_stream_ok(a, kStreamBoundPosTerms)) return row_stream_bound(a, st);
+    // dense single-group layers: the table kernel, tracking the chunk of every result, is queued in front
+    // of the every-term kernel as for the forward without positions; both leave (value, chunk) pairs for the resolve
+    const float bound_density = g_bound_density.load(std::memory_order_relaxed);
+    const float cap = bound_density >= 0.f ? bound_density : kBoundPosColsCap;
+    const FwdArgs raw = a;
+    size_t copies = bound_pad(a, cap, B, CO, CI, G, HW);
+    int tables = bound_tables_eligible(a, cap, B, CO, CI, G, HW);
+    const size_t pairs = ((size_t)a.R * a.G * a.COg * 16 + 255) / 256 * 256;
+    const size_t tbytes = tables ? (bound_tables_bytes(tables == 2, B, CO, CI) + 255) / 256 * 256 : 0;
+    if ((tables || copies) && (bound_density < 0.f || copies) && !workspace_ready(pairs + tbytes + copies, st)) {   // a first call under capture
+        tables = 0;
+        if (copies) { a = raw; CI = raw.CIg; copies = 0; }
+    }
+    const bool elig = tables || copies;   // by shape alone: what the workspace is sized by (a captured call may build tables that an eager one does not)
+    const bool hinted = tables && bound_density < 0.f;
+    if (hinted && !hint_build_tables(kHintSiteBoundPos, weight, B, CO, CI, st, tables == 1)) tables = 0;
+    const bool copied = copies && (tables || !(raw.fast_x && raw.fast_w));   // (as without positions)
+    if (copies && !copied) { a = raw; CI = raw.CIg; }
     static const int kTb42[] = {4, 2};
     const bool narrow = narrow_tiles(a);
     const int TB = narrow ? 2 : pick_tb(a, kTb42, 2, 64);
     a.nsplit = pick_nsplit(a, 16 * TB, narrow ? 32 : 64);
     if (a.nsplit > 1 && !workspace_ready((size_t)a.R * a.G * a.COg * 16, st)) { a.coarse = 1; a.nsplit = pick_nsplit(a, 16 * TB, narrow ? 32 : 64); }
-    // dense single-group layers: the table kernel, tracking the chunk of every result, is queued in front
-    // of the every-term kernel as for the forward without positions; both leave (value, chunk) pairs for the resolve
-    const float bound_density = g_bound_density.load(std::memory_order_relaxed);
-    const float cap = bound_density >= 0.f ? bound_density : kBoundPosColsCap;
-    int tables = bound_tables_eligible(a, cap, B, CO, CI, G, HW);
-    const size_t pairs = ((size_t)a.R * a.G * a.COg * 16 + 255) / 256 * 256;
-    if (tables && bound_density < 0.f && !workspace_ready(pairs + bound_tables_bytes(tables == 2, B, CO, CI), st)) tables = 0;   // a first call under capture
-    const int elig = tables;   // by shape alone: what the workspace is sized by (a captured call may build tables that an eager one does not)
-    const bool hinted = tables && bound_density < 0.f;
-    if (hinted && !hint_build_tables(kHintSiteBoundPos, weight, B, CO, CI, st, tables == 1)) tables = 0;
     if (tables == 2 && a.nsplit < 2) a.nsplit = 2;   // both kernels merge into the packed pairs
     if (a.nsplit > 1 || elig) {
         size_t n = (size_t)a.R * a.G * a.COg;
-        char* ws = static_cast<char*>(workspace(pairs + (elig ? bound_tables_bytes(elig == 2, B, CO, CI) : 0), st));   // the only request
+        char* ws = static_cast<char*>(workspace(pairs + (elig ? tbytes + copies : 0), st));   // the only request
         if (!ws) return SD_ERR_HIP;
+        if (copied && (rc = bound_pad_copy(a, raw, ws + pairs + tbytes, st))) return rc;
         a.packed0 = reinterpret_cast<unsigned long long*>(ws);
         a.packed1 = a.packed0 + n;
         if (a.nsplit > 1 && (rc = fill_zero(a.packed0, n * 4, st))) return rc;

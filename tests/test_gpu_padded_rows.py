@@ -56,3 +56,35 @@ def test_tables_serve_and_capture_needs_no_scratch():
         for a, b in zip(fresh, want):
             assert torch.equal(a, b)
             a.zero_()
+
+
+@pytest.mark.parametrize("B,N,M,kind", [(129, 1057, 1030, ""), (64, 4081, 530, "ties"), (33, 5121, 840, "odd"), (257, 2050, 4130, ""),
+                                        (70, 5829, 5270, "odd"), (131, 9998, 1645, "ties")])
+def test_interval_bounds_against_the_oracle(oracle, B, N, M, kind):
+    from sortnet_amd import ext
+    x, w = _data(B, N, M, 0.5)
+    w *= N ** -0.5
+    if kind == "ties":
+        x, w = (x * 8).round() / 8, (w * 64).round() / 64
+    lo, up = x - 0.03, x + 0.03
+    if kind == "odd":
+        lo[0, 3], w[1, 2], up[1, N - 1], w[2, N - 1], lo[2, 5] = float("nan"), float("inf"), float("inf"), float("nan"), up[2, 5] + 1
+    # an output depends on its own rows alone: some of the largest layers
+    rows, cols = slice(0, B, 1 + B * M * N // 2 ** 28), slice(0, M, 1 + B * M * N // 2 ** 29)
+    rl, ru, rpl, rpu = oracle.bound_inf_dist_forward(lo[rows].contiguous().numpy(), up[rows].contiguous().numpy(), w[cols].contiguous().numpy())
+    new = lambda t: torch.full((B, M, 1), 7, device="cuda", dtype=t)   # noqa: E731
+    l, u, l2, u2, pl, pu = (new(t) for t in (torch.float32,) * 4 + (torch.int32,) * 2)
+    ext.bound_inf_dist_forward_nograd(lo.cuda(), up.cuda(), w.cuda(), l, u, 1)
+    ext.bound_inf_dist_forward(lo.cuda(), up.cuda(), w.cuda(), l2, u2, pl, pu, 1)
+    for got, want in ((l, rl), (u, ru), (l2, rl), (u2, ru), (pl, rpl), (pu, rpu)):
+        got = got[rows][:, cols].cpu().numpy()
+        np.testing.assert_array_equal(got, np.asarray(want).reshape(got.shape).astype(got.dtype))
+
+
+@pytest.mark.parametrize("B,N,M,spread", [(99, 2304, 59, 0.3), (16, 320, 250, 0.05), (64, 511, 65, 3.0), (1, 1200, 900, 0.3), (129, 5120, 3, 0.3)])
+def test_positions_of_few_outputs(oracle, B, N, M, spread):
+    x, w = _data(B, N, M, spread)
+    _, yp, pos, _, _ = _run(x.cuda(), w.cuda())
+    ry, rp = oracle.sort_neuron_forward(x.numpy(), w.numpy(), Q, K)
+    np.testing.assert_array_equal(yp.cpu().numpy(), ry)
+    np.testing.assert_array_equal(pos.cpu().numpy(), np.asarray(rp).astype(np.int32).reshape(tuple(pos.shape)))
