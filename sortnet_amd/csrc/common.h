@@ -143,6 +143,8 @@ public:
 // is known of.  hint_forget: the kernel was not launched after all.
 constexpr int kHintStreak = 3, kHintSkip = 31;
 bool hint_build_tables(int site, const void* weight, int B, int CO, int CI, hipStream_t stream, bool unprobed = false);
+// whether the layer's last call whose outcome is there was served from tables
+bool hint_paid(int site, const void* weight, int B, int CO, int CI);
 unsigned long long* hint_expect(int site, const void* weight, int B, int CO, int CI, hipStream_t stream);
 void hint_forget(unsigned long long* word);
 

@@ -54,4 +54,7 @@ int row_cands_forward(int form, const float* xl, const float* xu, const float* w
                       void* ws, float density, bool forced, const float* col_stat, const unsigned long long* col_count,
                       const unsigned long long** every, hipStream_t st, int* pos_lower = nullptr);
 
+// the word that is 1 after a call whose tables per batch row did not serve, from its `every`
+const unsigned long long* row_cands_idle(const unsigned long long* every);
+
 }  // namespace sd

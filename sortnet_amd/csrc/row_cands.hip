@@ -1,5 +1,6 @@
 // Sort neuron, its interval bounds and the l-inf forward from candidate tables per batch row (see row_cands.h).
 #include "row_cands.h"
+#include <cstddef>
 #include <type_traits>
 #include "cand_tables.h"
 #include "cand_walk.h"
@@ -24,6 +25,7 @@ struct RowCount {
     unsigned long long col_marks;  // marks per weight row (copy)
     unsigned long long fixes;      // outputs to recompute
     unsigned long long sum;        // see add_marks
+    unsigned long long idle;       // 1: it does not
 };
 
 struct Carve {
@@ -149,6 +151,7 @@ rc_tables_kernel(TableArgs a, RowCount* __restrict__ c, const unsigned long long
     c->marks = marks;
     c->every = ((col_count == nullptr || col_count[1] != 0ull) && !run) ? 1ull : 0ull;
     c->run = run ? 1ull : 0ull;
+    c->idle = run ? 0ull : 1ull;
     c->col_marks = col_count == nullptr ? ~0ull : col_count[0];
 }
 
@@ -499,6 +502,10 @@ bool row_cands_supported(int form, int K) {
 #define SD_ROWS_K12(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12)
 #define SD_ROWS_K18(X) SD_ROWS_K12(X) X(13) X(14) X(15) X(16) X(17) X(18)
 #define SD_ROWS_K25(X) SD_ROWS_K18(X) X(19) X(20) X(21) X(22) X(23) X(24) X(25)
+
+const unsigned long long* row_cands_idle(const unsigned long long* every) {
+    return every + (offsetof(RowCount, idle) - offsetof(RowCount, every)) / sizeof(unsigned long long);
+}
 
 int row_cands_forward(int form, const float* xl, const float* xu, const float* w, const uint32_t* xkeep,
                       const uint32_t* wkeep, int B, int CO, int CI, float q, int K, float* outL, float* outU, int* pos,

@@ -214,6 +214,12 @@ bool hint_build_tables(int site, const void* weight, int B, int CO, int CI, hipS
     return true;
 }
 
+bool hint_paid(int site, const void* weight, int B, int CO, int CI) {
+    std::lock_guard<std::mutex> lock(g_hint_mu);
+    const HintSlot* h = hint_slot(site, weight, B, CO, CI, false);
+    return h && h->known && h->streak == 0;
+}
+
 unsigned long long* hint_expect(int site, const void* weight, int B, int CO, int CI, hipStream_t stream) {
     if (capturing(stream)) return nullptr;
     std::lock_guard<std::mutex> lock(g_hint_mu);

@@ -163,6 +163,7 @@ static long long sort_cols_min_terms(bool pos, int CI) { return pos && CI >= 320
 // `site`: which entry point asks (with the built-in limit, a layer whose tables have not paid lately is not given
 // any for a while, see hint_build_tables)
 constexpr int kHintSiteSort = 2, kHintSiteBoundSort = 3, kHintSiteSortPos = 6;
+constexpr int kHintSiteRows = 10;   // and with the form added: whether the tables per batch row served
 // shape and size alone: the workspace is sized by this, so that a call under graph capture (which always builds
 // tables) never needs more than the eager call before it did
 static bool sort_cols_eligible(const FwdArgs& a, bool pos, int B, int CO, int CI, int G, int HW) {
@@ -202,15 +203,18 @@ static size_t sort_tables_bytes(int form, int B, int CO, int CI, int K) {
 // `ws`: sort_tables_bytes() bytes.  The gate it leaves in `a` points into `ws`: the kernels queued behind it must
 // not be given memory that overlaps it, and `ws` must stay allocated until they have run (one workspace request
 // per call, carved by the caller).  Afterwards a.gate[0] is non-zero when the every-term kernels are to run.
-static int queue_sort_cols(FwdArgs& a, int form, const float* xl, const float* xu, const float* w, int B, int CO, int CI,
+// A layer that the tables per weight row serve queues those per batch row in vain, three kernels that return at once (4.6 us each): where
+// they ran in none of three calls they are left out of the next 31, unless the call before formed every term (evaluation pass of 6 x
+// 5120 at batch 512 1636 -> 1575 us, attack on 128 x 5120 x 5120 225 -> 215).  `site`, `layer`: see sort_cols_ok.
+static int queue_sort_cols(FwdArgs& a, int site, const float* layer, int form, const float* xl, const float* xu, const float* w, int B, int CO, int CI,
                            float q, int K, float* outL, float* outU, int* pos, void* ws, hipStream_t st) {
     const float density = g_sort_density.load(std::memory_order_relaxed);
     const float cap = density > 0.f ? density : sort_cols_cap(form, CI);
     int rc = sort_cols_forward(xl, xu, w, B, CO, CI, q, K, outL, outU, pos, ws, cap, &a.gate, &a.gate_limit, st);
     a.gate_above = 1;
     const long long terms = (long long)B * CO * CI;
-    const bool rows = row_cands_supported(form, K) &&
-                      (density > 0.f || terms >= kSortRowsMinTerms);
+    const bool rows = row_cands_supported(form, K) && (density > 0.f || terms >= kSortRowsMinTerms) &&
+                      (density > 0.f || hint_build_tables(kHintSiteRows + form, layer, B, CO, CI, st) || !hint_paid(site, layer, B, CO, CI));
     if (rc || !rows) {
         // the every-term kernels read the flag behind the counter, as with both tables
         if (!rc) { a.gate = a.gate + 1; a.gate_limit = 0ull; }
@@ -224,6 +228,10 @@ static int queue_sort_cols(FwdArgs& a, int form, const float* xl, const float* x
     if (rc) return rc;
     a.gate = every;
     a.gate_limit = 0ull;
+    if (density < 0.f) {
+        a.told2 = hint_expect(kHintSiteRows + form, layer, B, CO, CI, st);
+        a.few = row_cands_idle(every);
+    }
     note_term_counts(every - 1, 3, (double)((CO + 127) / 128) * B * CI, (double)((B + 127) / 128) * CO * CI);
     return SD_OK;
 }
@@ -313,7 +321,7 @@ extern "C" int sd_sort_neuron_forward_nograd(const float* input, const float* we
     if (streamed && !cols) return row_stream_sort(raw, K, st);
     if (copies && !sort_unpad(a, raw, CI, cols) && (rc = sort_pad_copy(a, raw, base + tbytes + kbytes, st))) return rc;
     int* keys = reinterpret_cast<int*>(base + tbytes);
-    if (cols && (rc = queue_sort_cols(a, kRowsSortValues, a.x0, nullptr, a.w, B, CO, CI, q, K, nullptr, output, nullptr, base, st))) return rc;
+    if (cols && (rc = queue_sort_cols(a, kHintSiteSort, weight, kRowsSortValues, a.x0, nullptr, a.w, B, CO, CI, q, K, nullptr, output, nullptr, base, st))) return rc;
     if (cols) sort_cols_expect(a, weight, kHintSiteSort, B, CO, CI, st);
     rc = SD_ERR_ARG;
     switch (K) {
@@ -323,7 +331,7 @@ extern "C" int sd_sort_neuron_forward_nograd(const float* input, const float* we
         SD_FOR_EACH_K(X)
 #undef X
     }
-    if (rc) hint_forget(a.told);
+    if (rc) { hint_forget(a.told); hint_forget(a.told2); }
     return rc;
 }
 
@@ -361,7 +369,7 @@ extern "C" int sd_sort_neuron_forward(const float* input, const float* weight,
     }
     if (copies && !sort_unpad(a, raw, CI, cols) && (rc = sort_pad_copy(a, raw, base + tbytes + kbytes, st))) return rc;
     int* keys = reinterpret_cast<int*>(base + tbytes);
-    if (cols && (rc = queue_sort_cols(a, kRowsSortPos, a.x0, nullptr, a.w, B, CO, CI, q, K, nullptr, output, pos, base, st))) return rc;
+    if (cols && (rc = queue_sort_cols(a, kHintSiteSortPos, weight, kRowsSortPos, a.x0, nullptr, a.w, B, CO, CI, q, K, nullptr, output, pos, base, st))) return rc;
     if (cols) sort_cols_expect(a, weight, kHintSiteSortPos, B, CO, CI, st);
     rc = SD_ERR_ARG;
     switch (K) {
@@ -371,7 +379,7 @@ extern "C" int sd_sort_neuron_forward(const float* input, const float* weight,
         SD_FOR_EACH_K(X)
 #undef X
     }
-    if (rc) hint_forget(a.told);
+    if (rc) { hint_forget(a.told); hint_forget(a.told2); }
     return rc;
 }
 
@@ -401,7 +409,7 @@ extern "C" int sd_bound_sort_neuron_forward(const float* inputL, const float* in
         char* ws = static_cast<char*>(workspace(tbytes + copies, st));   // the only request of this call
         if (!ws) return SD_ERR_HIP;
         if (copies && !streamed && !sort_unpad(a, raw, CI, cols) && (rc = sort_pad_copy(a, raw, ws + tbytes, st))) return rc;
-        if (cols && (rc = queue_sort_cols(a, kRowsSortInterval, a.x0, a.x1, a.w, B, CO, CI, q, K, outputL, outputU, nullptr, ws, st))) return rc;
+        if (cols && (rc = queue_sort_cols(a, kHintSiteBoundSort, weight, kRowsSortInterval, a.x0, a.x1, a.w, B, CO, CI, q, K, outputL, outputU, nullptr, ws, st))) return rc;
     }
     if (streamed) return row_stream_sort(raw, K, st);
     if (cols) sort_cols_expect(a, weight, kHintSiteBoundSort, B, CO, CI, st);
@@ -411,6 +419,6 @@ extern "C" int sd_bound_sort_neuron_forward(const float* inputL, const float* in
         SD_FOR_EACH_K(X)
 #undef X
     }
-    if (rc) hint_forget(a.told);
+    if (rc) { hint_forget(a.told); hint_forget(a.told2); }
     return rc;
 }
