@@ -116,8 +116,8 @@ static int queue_max_cols(FwdArgs& a, int K, int B, int CO, int CI, void* ws, hi
 }
 
 // before the every-term kernel is queued behind the table kernels: where it reports
-static void max_cols_expect(FwdArgs& a, int site, int B, int CO, int CI, hipStream_t st) {
-    if (g_linf_density.load(std::memory_order_relaxed) < 0.f && a.gate) a.told = hint_expect(site, a.w, B, CO, CI, st);
+static void max_cols_expect(FwdArgs& a, const float* weight, int site, int B, int CO, int CI, hipStream_t st) {
+    if (g_linf_density.load(std::memory_order_relaxed) < 0.f && a.gate) a.told = hint_expect(site, weight, B, CO, CI, st);
 }
 
 extern "C" int sd_set_linf_candidate_density(float density) {
@@ -236,7 +236,7 @@ extern "C" int sd_inf_dist_forward_nograd(const float* input, const float* weigh
         if (!ws) return SD_ERR_HIP;
         if (K && (rc = queue_max_cols(a, K, B, CO, CI, ws, st))) return rc;
     }
-    if (K) max_cols_expect(a, kHintSiteLinf, B, CO, CI, st);
+    if (K) max_cols_expect(a, weight, kHintSiteLinf, B, CO, CI, st);
     rc = narrow ? launch_fwd<LinfNograd, 2, 2>(a, st) : TB == 2 ? launch_fwd<LinfNograd, 2, 8>(a, st) : launch_fwd<LinfNograd, 4, 8>(a, st);
     if (rc) hint_forget(a.told);
     return rc;
@@ -275,7 +275,7 @@ extern "C" int sd_inf_dist_forward(const float* input, const float* weight,
     char* base = static_cast<char*>(workspace(merge + max_tables_bytes(B, CO, CI, KE), st));
     if (!base) return SD_ERR_HIP;
     if (K && (rc = queue_max_cols(a, K, B, CO, CI, base + merge, st))) return rc;
-    if (K) max_cols_expect(a, kHintSiteLinf, B, CO, CI, st);
+    if (K) max_cols_expect(a, weight, kHintSiteLinf, B, CO, CI, st);
     rc = run_chunk_pos<LinfChunk>(a, false, st, base, merge);
     if (rc) hint_forget(a.told);
     return rc;
@@ -335,6 +335,21 @@ extern "C" int sd_inf_dist_forward_noalloc(const float* input, const float* weig
     return run_chunk_pos<LinfChunk>(a, w_index_ci || w_index_co, static_cast<hipStream_t>(stream), buf, kScratchBytes);
 }
 
+// Factored mask on rows that cannot be loaded 16 bytes at a time: sets the shape of `a` and CI to that of copies whose rows are whole chunks,
+// and returns their bytes, or 0 (as they were).  The kernel that loads value by value draws the keep bits of a tile as it stages it,
+// again for every tile.  Without copies -> with them, q = 0.3, without / with positions, us: 91 x 799 x 1920 28 -> 25 / 47 -> 38, 250 x 3071 x
+// 1021 92 -> 53 / 118 -> 67, 300 x 5001 x 3000 332 -> 214 / 497 -> 244, 512 x 5121 x 5120 839 -> 298 / 1441 -> 311, 20 x 7001 x 2001 59 -> 54 / 70 -> 61.
+// Below 2^27 terms, where there is little to gain, the kernel stays; the smallest layers are streamed.
+constexpr long long kMaskPadMinTerms = 1ll << 27;
+static size_t masked_pad(FwdArgs& a, int B, int CO, int& CI, int G, int HW) {
+    const int N = (CI + KT - 1) / KT * KT;
+    if ((a.fast_x && a.fast_w) || G != 1 || HW != 1 || (long long)(B + CO) * N >= (1ll << 31) || B + CO > 4 * 65535 ||
+        (long long)B * CO * CI < kMaskPadMinTerms) return 0;
+    CI = a.CIg = a.W_CIg = N;
+    a.fast_x = a.fast_w = 1;
+    return (((size_t)B * N + 63) / 64 * 64 + (size_t)CO * N) * 4;
+}
+
 extern "C" int sd_masked_inf_dist_forward(const float* input, const float* weight,
                                           int B, int CO, int CI, int G, int HW, float* output, int* pos,
                                           float q, uint32_t seed, int mode, sd_stream_t stream) {
@@ -366,28 +381,43 @@ extern "C" int sd_masked_inf_dist_forward(const float* input, const float* weigh
     const long long xrows = (long long)a.R * G, wrows = (long long)CO;
     const size_t packed_bytes = pos ? (((size_t)a.R * CO * 8 + 255) / 256) * 256 : 0;
     const size_t mask_bytes = ((size_t)(xrows + wrows) * nchunks * 4 + 255) / 256 * 256;
-    const bool vector = a.fast_x && a.fast_w;
     // (rows that are not streamed for speed need no scratch without positions, so a stream under capture must not ask for it)
     const bool streamed = g_linf_density.load(std::memory_order_relaxed) <= 0.f && row_stream_sizes_ok(a, kStreamMaskTerms) &&
-                          (vector || workspace_ready(packed_bytes + mask_bytes, st));
+                          ((a.fast_x && a.fast_w) || workspace_ready(packed_bytes + mask_bytes, st));
+    // rows that cannot be loaded 16 bytes at a time: copies with zeros behind every row, which the keep bits drop
+    const FwdArgs raw = a;
+    const size_t copies = streamed ? 0 : masked_pad(a, B, CO, CI, G, HW);
+    if (copies) {
+        const int KE = max_cols_eligible(a, (float)a.t16 / 65536.f, B, CO, CI, G, HW);
+        if (!workspace_ready(packed_bytes + mask_bytes + (KE ? max_tables_bytes(B, CO, CI, KE) : 0) + 256 + copies, st)) { a = raw; CI = raw.CIg; }
+    }
+    const bool vector = a.fast_x && a.fast_w, padded = vector && !(raw.fast_x && raw.fast_w);
     if (vector || streamed) {
         // one request for every user of the workspace: merge buffer, keep bits, candidate tables
         const int KE = max_cols_eligible(a, (float)a.t16 / 65536.f, B, CO, CI, G, HW);
         K = max_cols_wanted(a, KE, kHintSiteMasked, B, CO, CI, st);
-        char* base = static_cast<char*>(workspace(packed_bytes + mask_bytes + (KE ? max_tables_bytes(B, CO, CI, KE) : 0), st));
+        const size_t table_bytes = KE ? (max_tables_bytes(B, CO, CI, KE) + 255) / 256 * 256 : 0;
+        char* base = static_cast<char*>(workspace(packed_bytes + mask_bytes + table_bytes + (padded ? copies : 0), st));
         if (!base) return SD_ERR_HIP;
+        if (padded) {
+            float* x = reinterpret_cast<float*>(base + packed_bytes + mask_bytes + table_bytes);
+            float* w = x + ((size_t)a.R * a.CIg + 63) / 64 * 64;
+            if ((rc = pad_rows({raw.x0, raw.x0, raw.w}, {x, x, w}, {a.R, 0, a.COg}, raw.CIg, a.CIg, st))) return rc;
+            a.x0 = x;
+            a.w = w;
+        }
         tables = base + packed_bytes + mask_bytes;
         uint32_t* xm = reinterpret_cast<uint32_t*>(base + packed_bytes);
         uint32_t* wm = xm + xrows * nchunks;
         hipLaunchKernelGGL(build_masks_kernel, dim3((unsigned)(((xrows + wrows) * nchunks + 255) / 256)), dim3(256), 0, st,
-                           xm, xrows, xrows + wrows, nchunks, a.CIg, seed, a.t16);
+                           xm, xrows, xrows + wrows, nchunks, raw.CIg, seed, a.t16);
         if ((rc = check_launch("build_masks_kernel"))) return rc;
         a.xmask = xm; a.wmask = wm;
         if (streamed) return row_stream_linf(a, st);
     }
     if (pos) {
         if (K && (rc = queue_max_cols(a, K, B, CO, CI, tables, st))) return rc;
-        if (K) max_cols_expect(a, kHintSiteMasked, B, CO, CI, st);
+        if (K) max_cols_expect(a, weight, kHintSiteMasked, B, CO, CI, st);
         rc = run_chunk_pos<LinfChunk>(a, false, st);
         if (rc) hint_forget(a.told);
         return rc;
@@ -398,7 +428,7 @@ extern "C" int sd_masked_inf_dist_forward(const float* input, const float* weigh
     a.nsplit = pick_nsplit(a, 16 * TB, narrow ? 32 : 128);
     if (a.nsplit > 1 && (rc = fill_zero(output, (size_t)B * CO * HW, st))) return rc;
     if (K && (rc = queue_max_cols(a, K, B, CO, CI, tables, st))) return rc;
-    if (K) max_cols_expect(a, kHintSiteMasked, B, CO, CI, st);
+    if (K) max_cols_expect(a, weight, kHintSiteMasked, B, CO, CI, st);
     rc = narrow ? launch_fwd<LinfNograd, 2, 2>(a, st) : TB == 2 ? launch_fwd<LinfNograd, 2, 8>(a, st) : launch_fwd<LinfNograd, 4, 8>(a, st);
     if (rc) hint_forget(a.told);
     return rc;

@@ -88,3 +88,17 @@ def test_positions_of_few_outputs(oracle, B, N, M, spread):
     ry, rp = oracle.sort_neuron_forward(x.numpy(), w.numpy(), Q, K)
     np.testing.assert_array_equal(yp.cpu().numpy(), ry)
     np.testing.assert_array_equal(pos.cpu().numpy(), np.asarray(rp).astype(np.int32).reshape(tuple(pos.shape)))
+
+
+@pytest.mark.parametrize("B,N,M,q", [(91, 799, 1920, 0.3), (250, 1025, 530, 0.7), (33, 2303, 2001, 0.05), (129, 4097, 261, 1.0), (200, 5131, 140, 0.3)])
+def test_factored_mask_against_the_oracle(oracle, B, N, M, q):
+    from sortnet_amd import _lib, ext
+    x, w = _data(B, N, M, 0.3)
+    x[0, N - 1], w[1, 2], w[2, N - 1] = float("nan"), float("inf"), -9.0
+    y, y2, pos = (torch.full((B, M, 1), 7, device="cuda", dtype=t) for t in (torch.float32, torch.float32, torch.int32))
+    ry, rp = oracle.masked_inf_dist_forward(x.numpy(), w.numpy(), q, 11, oracle.MASK_FACTORED)
+    ext.masked_inf_dist_forward(x.cuda(), w.cuda(), y, pos, 1, q, 11, ext.MASK_FACTORED)
+    ext.masked_inf_dist_forward(x.cuda(), w.cuda(), y2, None, 1, q, 11, ext.MASK_FACTORED)
+    assert _lib.last_forward_kernel().startswith("fwd_kernel_pipe")
+    for got, want in ((y, ry), (y2, ry), (pos, rp)):
+        np.testing.assert_array_equal(got.cpu().numpy(), np.asarray(want).reshape(B, M, 1).astype(got.cpu().numpy().dtype))
