@@ -225,7 +225,8 @@ __global__ void __launch_bounds__(256, 4) lp_grad_kernel(Args k) {
     const int nc = n_ok ? n : a.CIg - 1;
     int rows = a.R - r0;
     rows = rows < 0 ? 0 : rows > RB ? RB : rows;
-    const int last = rows > 0 ? rows - 1 : 0, rx = rows > 0 ? r0 : 0;   // rows past the batch repeat one, with g = 0
+    // rows past the batch repeat one of their tile, with g = 0; a tile behind the batch holds row 0, whose terms are left out
+    const int last = rows > 0 ? rows - 1 : 0, rx = rows > 0 ? r0 : 0;
     const int sub = (rx / a.HW) / kSubBatch;   // (one tile to a sub-batch where there are index lists)
 
     const int wcol = a.ci_idx ? a.ci_idx[(sub * a.G + g) * a.CIg + nc] : nc;
@@ -292,7 +293,8 @@ __global__ void __launch_bounds__(256, 4) lp_grad_kernel(Args k) {
     for (int j = 0; j < MC; j++) wv[j] = wbase[(size_t)row_of(m_lo, j, rowv) * a.W_CIg];
     // a slice without a chunk that forms ratios runs the loop without that path, which would cost it copies of its sums
     for (int c = m_lo / MC + 64 + lane; IP >= 0 && c < c_hi; c += 64) mode |= modes[c];
-    const bool ratios = __builtin_amdgcn_ballot_w64(mode != 0u) != 0ull;
+    // (nor would 0 times a power of a difference be 0 in a tile behind the batch, where no output says that the power is finite)
+    const bool ratios = rows == 0 || __builtin_amdgcn_ballot_w64(mode != 0u) != 0ull;
 
     auto add_weight = [&](int row, float v) {
         float* dst = gwbase + (size_t)row * a.W_CIg;

@@ -65,3 +65,14 @@ def test_index_lists(oracle, B, N, M, kn, km, G, HW):
     x, gy = torch.randn(B, kn * G, HW, generator=g), torch.randn(B, km * G, HW, generator=g)
     for p in (3.0, 8.0, 10.5):
         _both(oracle, x, torch.randn(M * G, N, generator=g), gy, p, G, ci, co)
+
+
+# Workgroups of four batch tiles from 1024 (tile, 64 inputs, group) triples on.  A tile behind the batch has inputs of no row: here row 0 is so
+# far from the weights that the products of a factor 0 with powers of its distances would be undefined.
+@pytest.mark.parametrize("p,far", [(2.0, 1e30), (6.0, 1e16), (8.0, 1e10), (9.0, 1e8), (17.3, 1e8)])
+def test_tiles_behind_the_batch(oracle, p, far):
+    g = torch.Generator().manual_seed(6)
+    B, N, M = 336, 6001, 6
+    x, gy = torch.randn(B, N, 1, generator=g), torch.randn(B, M, 1, generator=g)
+    x[0, 7], x[0, 5990] = far, -far
+    _both(oracle, x, torch.randn(M, N, generator=g) * 0.4, gy, p)
