@@ -27,6 +27,10 @@ namespace {
 constexpr int RC = 8;          // output channels of a wavefront
 constexpr int kWaves = 4;      // wavefronts of a workgroup: the same rows, channels next to each other
 constexpr int kStep = 8;       // inputs of a step
+// Inputs whose powers are added up by themselves: a layer is cut into fewer slices here than by the kernel that stages tiles, and one sum
+// over a slice was further off (rms of the relative error of 24 x 800 x 512 x 256 at p = 2 / 8: 4 slices there 6.7e-8 / 4.3e-8, 2 slices
+// here 1.1e-7 / 5.3e-8, with these sums 4.7e-8 / 3.9e-8).  Time from 5 % less (p = 2) to 2 % more (p = 8).
+constexpr int kRun = 64;
 
 typedef float f16s __attribute__((ext_vector_type(16)));
 // memory that no kernel writes while this one runs, read at wave-uniform addresses: scalar loads
@@ -89,7 +93,7 @@ __device__ __forceinline__ int find_input(const float* __restrict__ xp, const fl
 
 template <class P>
 __global__ void __launch_bounds__(64 * kWaves, 4) fwd_cols_kernel(FwdArgs a, const float* __restrict__ wl, int quads) {
-    constexpr bool POS = std::is_same<P, LinfQuad>::value;
+    constexpr bool POS = std::is_same<P, LinfQuad>::value, SUM = !POS && !std::is_same<P, LinfNograd>::value;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = blockIdx.z % a.G, split = blockIdx.z / a.G;
     const int r0 = blockIdx.x * 64, block = blockIdx.y * kWaves + wave, m0 = block * RC;
@@ -138,10 +142,8 @@ __global__ void __launch_bounds__(64 * kWaves, 4) fwd_cols_kernel(FwdArgs a, con
     if (n_begin < n_full) { xload(x, n_begin); wload(w, n_begin / 4); }
     // The first channel's terms wait for the weights of the quad; behind them the next quad's are requested, so that they are on their
     // way while the other channels' terms are formed (scalar loads return in any order: a wait covers all).
-    #pragma unroll 2
-    for (int n = n_begin; n < n_full; n += kStep) {
+    auto step = [&](const Inputs& x, Inputs& xn, int n) __attribute__((always_inline)) {
         const int next = n + kStep < n_full ? n + kStep : n;
-        Inputs xn;
         Quad w1, wn;
         xload(xn, next);
         terms(x, w, 0, 0, n);
@@ -157,9 +159,25 @@ __global__ void __launch_bounds__(64 * kWaves, 4) fwd_cols_kernel(FwdArgs a, con
         __builtin_amdgcn_sched_barrier(0);
         #pragma unroll
         for (int i = 1; i < RC; i++) terms(x, w1, 1, i, n + 4);
-        x = xn;
         w = wn;
-    }
+    };
+    auto steps = [&](int n, int to) __attribute__((always_inline)) {
+        Inputs x1;
+        for (; n + 2 * kStep <= to; n += 2 * kStep) { step(x, x1, n); step(x1, x, n + kStep); }
+        if (n < to) { step(x, x1, n); x = x1; }
+    };
+    float total[RC] = {};   // of the runs that are done
+    if constexpr (SUM) {
+        for (int n0 = n_begin; n0 < n_full; n0 += kRun) {
+            steps(n0, n0 + kRun < n_full ? n0 + kRun : n_full);
+            #pragma unroll
+            for (int i = 0; i < RC; i++) {
+                asm volatile("" : "+v"(acc[i].s));
+                total[i] += acc[i].s;
+                acc[i].s = 0.f;
+            }
+        }
+    } else steps(n_begin, n_full);
     if (n_full < n_end) {   // the end of a row: inputs behind it are 0 on both sides
         xload(x, n_full);
         #pragma unroll
@@ -170,6 +188,10 @@ __global__ void __launch_bounds__(64 * kWaves, 4) fwd_cols_kernel(FwdArgs a, con
             #pragma unroll
             for (int i = 0; i < RC; i++) terms(x, w, half, i, n_full + 4 * half);
         }
+    }
+    if constexpr (SUM) {
+        #pragma unroll
+        for (int i = 0; i < RC; i++) acc[i].s += total[i];
     }
 
     if (r >= a.R) return;

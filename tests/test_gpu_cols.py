@@ -54,3 +54,30 @@ def test_powers(p, B, N, M, G, HW):
             d = (x[b, None, g * N:(g + 1) * N].double() - w[m:min(m + 16, (g + 1) * M), :, None].double()).abs()
             ref = d.pow(p).sum(1).pow(1 / p)
             torch.testing.assert_close(y[b, m:m + ref.shape[0]].double(), ref, rtol=rtol, atol=0)
+
+
+@pytest.mark.parametrize("p", [2.0, 8.0])
+@pytest.mark.parametrize("B,N,M,HW,slices", [(24, 800, 512, 256, 4), (12, 4000, 256, 256, 8), (64, 400, 256, 256, 2)])
+def test_sums_are_no_longer_than_slices(p, B, N, M, HW, slices):
+    """Long rows of many outputs, where a wavefront sums a whole row or half of it: the spread of the error is not above (by more than its
+    sampling, a tenth) that of 32-bit sums over `slices` parts of the row, as many as tiles of 32 x 128 outputs are cut in."""
+    from sortnet_amd import _lib, ext
+    x, w = (t.cuda() for t in _data(B, N, M, 1, HW, ""))
+    y = torch.full((B, M, HW), 7.0, device="cuda")
+    ext.norm_dist_forward(x, w, y, 1, p)
+    assert _lib.last_forward_kernel().startswith("fwd_cols_kernel")
+    rows, cols, chunks = x[:: B // 6], w[:: M // 32], -(-N // 32)
+    exact = torch.zeros(rows.shape[0], cols.shape[0], HW, device="cuda", dtype=torch.float64)
+    parts = []
+    for k in range(slices):
+        s = torch.zeros_like(exact, dtype=torch.float32)
+        for n in range(k * chunks // slices * 32, min((k + 1) * chunks // slices * 32, N)):
+            t = (rows[:, None, n] - cols[None, :, n, None]).abs()
+            exact += (rows[:, None, n].double() - cols[None, :, n, None].double()).abs() ** p
+            if p == 8.0:
+                t = t * t
+                t = t * t
+            s = (s.double() + t.double() * t.double()).float()   # one fused multiply-add
+        parts.append(s)
+    spread = lambda got: float(((got.double() - exact ** (1 / p)) / exact ** (1 / p)).pow(2).mean().sqrt())   # noqa: E731
+    assert spread(y[:: B // 6][:, :: M // 32]) <= 1.1 * spread(sum(parts) ** (1 / p))
