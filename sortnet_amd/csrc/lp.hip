@@ -661,6 +661,18 @@ struct LpBwdPlan {
     size_t words() const { return gx_words + gw_words; }
 };
 
+// workgroups run in rounds of (resident workgroups per CU) x CUs: the slice count whose last round is fullest, a smaller count
+// unless a larger one gains 3 %, slices of at least 64 channels
+int lp_even_slices(long long blocks, int slots, int channels) {
+    int slices = 1;
+    double best = 0.0;
+    for (int z = 1; z <= 16 && (z == 1 || channels / z >= 64); z++) {
+        const double rounds = (double)blocks * z / slots, eff = rounds / std::ceil(rounds);
+        if (eff > best * 1.03) { best = eff; slices = z; }
+    }
+    return slices;
+}
+
 // same_bits: the planes that make the gradients of a dense layer the same bits in every call
 static LpBwdPlan plan_lp_bwd(const LpBwdArgs& a, bool same_bits, bool planes) {
     LpBwdPlan plan{1, a.R, 0, 0, 0, 0};
@@ -676,14 +688,7 @@ static LpBwdPlan plan_lp_bwd(const LpBwdArgs& a, bool same_bits, bool planes) {
     // device mostly idle (index lists: a few hundred kept inputs per sub-batch) the output-channel range is
     // cut in slices
     const long long blocks = (long long)((a.CIg + 255) / 256) * tiles * a.G;
-    // workgroups run in rounds of (resident workgroups per CU) x CUs: take the slice count whose last round
-    // is fullest, a smaller count unless a larger one gains 3 %, slices of at least 64 channels
-    const double slots = (double)((a.skip_thr > 0.f ? 4 : 3) * num_cus());
-    double best = 0.0;
-    for (int z = 1; z <= 16 && (z == 1 || a.COg / z >= 64); z++) {
-        const double rounds = (double)blocks * z / slots, eff = rounds / std::ceil(rounds);
-        if (eff > best * 1.03) { best = eff; plan.zsplit = z; }
-    }
+    plan.zsplit = lp_even_slices(blocks, (a.skip_thr > 0.f ? 4 : 3) * num_cus(), a.COg);
     if (!planes || !aligned16(a.gx)) return plan;
     // small layers: slices down to one chunk of MC channels until every compute unit has two workgroups, merged in slice order
     // (p = 8, both gradients, in us, slices of 64 channels -> this, in brackets with atomic additions in any order:

@@ -17,6 +17,9 @@ size_t lp_grad_workspace(const LpGradArgs& a);
 // both gradients (or that of the inputs) for p - 1 = ip, a whole number in 0..8, or any pm1 = p - 1 > 0 (ip < 0)
 int lp_grad(int ip, float pm1, const LpGradArgs& a, void* ws, hipStream_t st);
 
+// slices of the output channels that the general kernel (lp.hip) cuts `blocks` workgroups of 256 inputs and 32 rows into
+int lp_even_slices(long long blocks, int slots, int channels);
+
 // out[o] = the sum of `planes` partial sums, `plane` floats apart, in plane order (lp.hip)
 int lp_merge_planes(const float* part, float* out, size_t total, size_t plane, int planes, hipStream_t st);
 

@@ -76,3 +76,30 @@ def test_tiles_behind_the_batch(oracle, p, far):
     x, gy = torch.randn(B, N, 1, generator=g), torch.randn(B, M, 1, generator=g)
     x[0, 7], x[0, 5990] = far, -far
     _both(oracle, x, torch.randn(M, N, generator=g) * 0.4, gy, p)
+
+
+@pytest.mark.parametrize("p", [2.0, 3.0])
+def test_input_gradients_of_large_batches(p):
+    """Sums over the output channels are cut into as many slices as by the general kernel (three here): the error of grad_input is not above
+    (by more than its sampling, a tenth) that of 32-bit sums over slices of 344 channels."""
+    from sortnet_amd import ext
+    g = torch.Generator(device="cuda").manual_seed(8)
+    B, N, M = 8192, 2048, 1024
+    x, w, gy = (torch.randn(*s, generator=g, device="cuda") for s in ((B, N, 1), (M, N), (B, M, 1)))
+    y, gx, gw = torch.empty_like(gy), torch.empty_like(x), torch.empty_like(w)
+    ext.norm_dist_forward(x, w, y, 1, p)
+    ext.norm_dist_backward_input_weight(gy, x, w, y, gx, gw, 1, p)
+    rows = slice(None, None, 512)
+    xs, gs, ys = x[rows, :, 0], gy[rows, :, 0], y[rows, :, 0].double()
+    exact, parts = torch.zeros_like(xs, dtype=torch.float64), []
+    for m in range(M):
+        if m % 344 == 0:
+            parts.append(torch.zeros_like(xs))
+        d = xs - w[m]
+        k = gs[:, m, None].double() * ys[:, m, None] ** (1 - p)
+        e = xs.double() - w[m].double()
+        exact += k * e * e.abs() ** (p - 2)
+        t = d.abs() * k.float() if p == 3.0 else k.float()
+        parts[-1] = (parts[-1].double() + t.double() * d.double()).float()   # one fused multiply-add
+    error = lambda got: float((got.double() - exact).norm() / exact.norm())   # noqa: E731
+    assert error(gx[rows, :, 0]) <= 1.1 * error(sum(parts))
