@@ -117,8 +117,8 @@ int num_cus();
 // sums.  Work queued on different streams never shares one; calls on ONE stream use it in queue order.
 // Growing waits for that stream and re-allocates (bytes == 0 returns the current buffer).
 void* workspace(size_t bytes, hipStream_t stream);
-// whether a request of that size would be met: false while `stream` records a graph and its buffer is smaller.  Asked by
-// paths that use scratch for speed where another needs none.
+// the same for paths that use scratch for speed where another needs none: whether the buffer holds so many bytes, grown if it has to be.
+// False while `stream` records a graph and its buffer is smaller, and where the memory is not to be had.
 bool workspace_ready(size_t bytes, hipStream_t stream);
 
 // Held by an entry point while it queues its kernels.  The calls of several host threads then reach their streams

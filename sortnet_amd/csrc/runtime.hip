@@ -89,11 +89,19 @@ bool capturing(hipStream_t stream) {
 bool workspace_ready(size_t bytes, hipStream_t stream) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0) { (void)hipGetLastError(); return false; }
-    {
-        std::lock_guard<std::mutex> lock(g_slot_mu);
-        for (const Slot& c : g_slots) if (c.dev == dev && c.stream == stream && c.cap >= bytes) return true;
-    }
-    return !capturing(stream);
+    std::lock_guard<std::mutex> lock(g_slot_mu);
+    Slot* slot = nullptr;
+    for (Slot& c : g_slots) if (c.dev == dev && c.stream == stream) { slot = &c; break; }
+    if (slot && slot->cap >= bytes) return true;
+    if (capturing(stream)) return false;
+    // the old buffer stays until there is a new one: the caller's other path may do with it, now and in every later call
+    const size_t want = bytes + bytes / 4;
+    void* p = nullptr;
+    if (hipMalloc(&p, want) != hipSuccess) { (void)hipGetLastError(); return false; }
+    if (!slot) { g_slots.push_back(Slot{dev, stream, nullptr, 0}); slot = &g_slots.back(); }
+    if (slot->buf) { (void)hipStreamSynchronize(stream); (void)hipFree(slot->buf); }
+    slot->buf = p; slot->cap = want;
+    return true;
 }
 
 void* workspace(size_t bytes, hipStream_t stream) {
