@@ -143,6 +143,12 @@ public:
 // is known of.  hint_forget: the kernel was not launched after all.
 constexpr int kHintStreak = 3, kHintSkip = 31;
 bool hint_build_tables(int site, const void* weight, int B, int CO, int CI, hipStream_t stream, bool unprobed = false);
+// The same for tables that the layer's other tables make spare (`served`: these served the last call that is known of): built wherever
+// those did not serve.  A call that formed every term without the spare ones may have wanted them (operands of one layer that alternate:
+// 512 x 2048 x 2048, sort neuron, 150 us from them, 490 for every term), so four times as many calls in a row must not have needed them before
+// they are left out again, up to kHintSpareMost: a call in vain costs 14 us.
+constexpr int kHintSpareMost = 192;
+bool hint_build_spare(int site, const void* weight, int B, int CO, int CI, hipStream_t stream, bool served);
 // whether the layer's last call whose outcome is there was served from tables
 bool hint_paid(int site, const void* weight, int B, int CO, int CI);
 unsigned long long* hint_expect(int site, const void* weight, int B, int CO, int CI, hipStream_t stream);

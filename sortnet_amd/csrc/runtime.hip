@@ -139,6 +139,8 @@ struct HintSlot {
     int head, queued;           // oldest outcome not yet looked at, and how many are queued
     int stale;                  // of the queued outcomes, how many belong to the layer the slot stood for before
     int streak, skip_left;
+    int need;                   // outcomes without tables in a row before they are left out
+    bool left_out;              // spare tables (hint_build_spare): not built in the last call that could have had them
     bool known;                 // an outcome of this layer has arrived
     unsigned long long used;    // g_hint_clock at the slot's last use: the least recently used slot is given away
 };
@@ -151,7 +153,8 @@ void hint_rekey(HintSlot& h, int dev, int site, const void* weight, int B, int C
     h.dev = dev; h.site = site; h.weight = weight; h.B = B; h.CO = CO; h.CI = CI;
     h.stale = h.queued;
     h.streak = h.skip_left = 0;
-    h.known = false;
+    h.need = kHintStreak;
+    h.left_out = h.known = false;
 }
 
 HintSlot* hint_slot(int site, const void* weight, int B, int CO, int CI, bool create) {
@@ -198,7 +201,7 @@ void hint_drain(HintSlot& h) {
             h.streak = ran != 0ull ? h.streak + 1 : 0;
             // the streak is long enough (or the probe after a stretch without tables came out the same): no tables
             // for the next kHintSkip calls, then one call probes again; tables at once where they served
-            h.skip_left = h.streak >= kHintStreak ? kHintSkip : 0;
+            h.skip_left = h.streak >= h.need ? kHintSkip : 0;
         }
         h.head = (h.head + 1) % kHintRing;
         h.queued--;
@@ -219,6 +222,23 @@ bool hint_build_tables(int site, const void* weight, int B, int CO, int CI, hipS
     // (When they all built tables meanwhile, 25 us each: interval pass of 784 - 6 x 1600 - 10 at batch 300, 448 us without any
     // tables, 513; 332 x 784 - 3 x 1984 - 10 228 and 244.)
     if (h->streak >= kHintStreak) h->skip_left = kHintSkip;
+    return true;
+}
+
+bool hint_build_spare(int site, const void* weight, int B, int CO, int CI, hipStream_t stream, bool served) {
+    if (capturing(stream)) return true;
+    std::lock_guard<std::mutex> lock(g_hint_mu);
+    HintSlot* h = hint_slot(site, weight, B, CO, CI, false);
+    if (!h) return true;
+    hint_drain(*h);
+    if (!served) {
+        if (h->left_out) { h->streak = h->skip_left = 0; h->need = h->need < kHintSpareMost / 4 ? h->need * 4 : kHintSpareMost; }
+        h->left_out = false;
+        return true;
+    }
+    h->left_out = h->skip_left > 0;
+    if (h->left_out) { h->skip_left--; return false; }
+    if (h->streak >= h->need) h->skip_left = kHintSkip;
     return true;
 }
 

@@ -204,8 +204,8 @@ static size_t sort_tables_bytes(int form, int B, int CO, int CI, int K) {
 // not be given memory that overlaps it, and `ws` must stay allocated until they have run (one workspace request
 // per call, carved by the caller).  Afterwards a.gate[0] is non-zero when the every-term kernels are to run.
 // A layer that the tables per weight row serve queues those per batch row in vain, three kernels that return at once (4.6 us each): where
-// they ran in none of three calls they are left out of the next 31, unless the call before formed every term (evaluation pass of 6 x
-// 5120 at batch 512 1636 -> 1575 us, attack on 128 x 5120 x 5120 225 -> 215).  `site`, `layer`: see sort_cols_ok.
+// they ran in none of three calls they are left out of the next 31, unless the call before formed every term (hint_build_spare;
+// evaluation pass of 6 x 5120 at batch 512 1636 -> 1575 us, attack on 128 x 5120 x 5120 225 -> 215).  `site`, `layer`: see sort_cols_ok.
 static int queue_sort_cols(FwdArgs& a, int site, const float* layer, int form, const float* xl, const float* xu, const float* w, int B, int CO, int CI,
                            float q, int K, float* outL, float* outU, int* pos, void* ws, hipStream_t st) {
     const float density = g_sort_density.load(std::memory_order_relaxed);
@@ -214,7 +214,7 @@ static int queue_sort_cols(FwdArgs& a, int site, const float* layer, int form, c
     a.gate_above = 1;
     const long long terms = (long long)B * CO * CI;
     const bool rows = row_cands_supported(form, K) && (density > 0.f || terms >= kSortRowsMinTerms) &&
-                      (density > 0.f || hint_build_tables(kHintSiteRows + form, layer, B, CO, CI, st) || !hint_paid(site, layer, B, CO, CI));
+                      (density > 0.f || hint_build_spare(kHintSiteRows + form, layer, B, CO, CI, st, hint_paid(site, layer, B, CO, CI)));
     if (rc || !rows) {
         // the every-term kernels read the flag behind the counter, as with both tables
         if (!rc) { a.gate = a.gate + 1; a.gate_limit = 0ull; }

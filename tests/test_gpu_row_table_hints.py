@@ -60,3 +60,30 @@ def test_tables_per_batch_row_come_and_go(form):
     assert _row_tables(call, 8) >= 7
     same(images)
     assert _lib.last_forward_term_share() < 1.0
+
+
+@pytest.mark.parametrize("form", ["values", "interval", "positions"])
+@pytest.mark.parametrize("every", [2, 7])
+def test_operands_that_alternate(form, every):
+    """One layer whose operands are served by the tables per weight row in all calls but each `every`-th, which those per batch row serve: after
+    a few rounds no call forms every term any more."""
+    from sortnet_amd import _lib, ext
+    B, N, M = 512, 1056, 1030
+    g = torch.Generator().manual_seed(5)
+    w = torch.randn(M, N, generator=g).cuda() * N ** -0.5
+    alike, images = (torch.randn(B, N, 1, generator=g) * 0.05 * N ** -0.5).cuda(), torch.rand(B, N, 1, generator=g).cuda()
+    o, pos = [torch.empty(B, M, 1, device="cuda") for _ in range(2)], torch.empty(K, B, M, 1, device="cuda", dtype=torch.int32)
+
+    def share(x):
+        if form == "values":
+            ext.sort_neuron_forward_nograd(x, w, o[0], 1, Q, K)
+        elif form == "positions":
+            ext.sort_neuron_forward(x, w, o[0], pos, 1, Q, K)
+        else:
+            ext.bound_sort_neuron_forward(x - 1e-4, x + 1e-4, w, o[0], o[1], 1, Q, K)
+        return _lib.last_forward_term_share()   # (waits for the stream)
+
+    for _ in range(6):
+        assert share(alike) < 1.0
+    shares = [share(images if k % every == 0 else alike) for k in range(6 * every)]
+    assert max(shares[4 * every:]) < 1.0, shares
