@@ -25,19 +25,32 @@ constexpr int MC = 4;    // output channels of a chunk: their weights are loaded
 constexpr int kTiles = 4;   // batch tiles of a workgroup of four wavefronts
 
 typedef float f16v __attribute__((ext_vector_type(16)));
+typedef float f8v __attribute__((ext_vector_type(8)));
+typedef uint32_t u8v __attribute__((ext_vector_type(8)));
 // memory that no kernel writes while this one runs, read at wave-uniform addresses: scalar loads
 template <class T> using Const = const __attribute__((address_space(4))) T*;
 template <class T> __device__ __forceinline__ Const<T> as_const(const void* p) { return (Const<T>)(uintptr_t)p; }
 
-// Scales of y between which d^(p-1) g y^(1-p) is formed as the product of d^(p-1) and g y^(1-p), one multiplication less per
-// term than the power of the ratio: for p - 1 <= 8 neither overflows, and a d^(p-1) that is no normal number has
-// (|d| / y)^(p-1) below 2^-56.  Chunks with an output outside form the ratio.
-constexpr float kYLow = 1.f / 256.f, kYHigh = 256.f, kGLow = 0x1p-96f, kGHigh = 0x1p+96f;
+// d^(p-1) g y^(1-p) is formed as the product of two factors, d^I g y^(1-p) and d^J with I + J = p - 1 (power_pair), one multiplication less
+// per term than the power of the ratio.  That holds where |d| <= y, as in every output, keeps both factors and d^(p-1) itself below 2^120 and
+// makes them normal numbers wherever (|d| / y)^(p-1) is above 2^-56.  Chunks with an output (or its gradient) outside form the ratio.
+constexpr int second_factor(int ip) { return ip <= 2 ? 1 : ip == 3 ? 2 : ip == 4 || ip == 6 ? 3 : ip == 8 ? 5 : 4; }
+constexpr double two_to(int e) { double v = 1.0; for (; e > 0; e--) v *= 2.0; for (; e < 0; e++) v *= 0.5; return v; }
+template <int IP> struct Limits {
+    static constexpr int J = second_factor(IP), I = IP - J;
+    static constexpr double kYLow = two_to(-70 / IP), kYHigh = two_to(120 / IP);
+    static constexpr double kFirstLow = two_to(-126 + (56 * I + IP - 1) / IP), kFirstHigh = two_to(120);   // |g| y^-J, the first factor at |d| = y
+    static constexpr double kScaleLow = two_to(-125), kScaleHigh = two_to(120);                        // |g| y^(1-p)
+};
+template <int N> __device__ __forceinline__ double power(double v) {
+    if constexpr (N <= 1) return N ? v : 1.0;
+    else { const double h = power<N / 2>(v); return N % 2 ? h * h * v : h * h; }
+}
 
 struct Batch {          // the batch side as the kernel reads it
     float* scale;       // [tile][group][channel][row]: g y^(1-p), or g in a chunk that forms ratios; 0 for rows past the batch.
                         // Any other power (IP < 0): pairs (g, 1 / y), and nothing in the two below
-    float* recip;       // the same layout: 1 / y in chunks that form ratios
+    float* recip;       // the same layout: 1 / y in chunks that form ratios, 0 for rows past the batch
     uint32_t* ratio;    // [tile][group][chunk]: the chunk forms ratios
 };
 
@@ -133,6 +146,7 @@ __global__ void __launch_bounds__(256) lp_grad_batch_kernel(Args k, float* __res
     for (int e = 0; e < 2; e++) {
         const int j = (tid >> 3) + 32 * e, m = m0 + j;
         float s[4], yv[4], gv[4];
+        bool real[4];
         if (IP < 0) {
             if (m < k.COp) {
                 float4* dst = reinterpret_cast<float4*>(k.s.scale + ((base + m) * RB + i0) * 2);
@@ -145,15 +159,14 @@ __global__ void __launch_bounds__(256) lp_grad_batch_kernel(Args k, float* __res
         #pragma unroll
         for (int i = 0; i < 4; i++) {
             gv[i] = gs[i0 + i][j]; yv[i] = ys[i0 + i][j];
-            if (IP > 0) {
-                const double v = 1.0 / (double)yv[i], v2 = v * v, v4 = v2 * v2;
-                double pw = IP & 1 ? v : 1.0;
-                if (IP & 2) pw *= v2;
-                if (IP & 4) pw *= v4;
-                if (IP & 8) pw *= v4 * v4;
-                s[i] = (float)((double)gv[i] * pw);
-                const float size = fabsf(s[i]);
-                bad |= !(yv[i] >= kYLow && yv[i] <= kYHigh) || !(gv[i] == 0.f || (size >= kGLow && size <= kGHigh));
+            real[i] = r0 + i0 + i < a.R && m < a.COg;
+            if constexpr (IP > 0) {
+                using L = Limits<IP>;
+                const double y = (double)yv[i], v = 1.0 / y, scale = (double)gv[i] * power<IP>(v), size = fabs(scale);
+                const double first = fabs((double)gv[i]) * power<L::J>(v);
+                s[i] = (float)scale;
+                bad |= real[i] && (!(y >= L::kYLow && y <= L::kYHigh) ||
+                                   !(gv[i] == 0.f || (size >= L::kScaleLow && size <= L::kScaleHigh && first >= L::kFirstLow && first <= L::kFirstHigh)));
             } else s[i] = gv[i];
         }
         const bool ratio = ((__builtin_amdgcn_ballot_w64(bad) >> (threadIdx.x & 32)) & 0xffffffffull) != 0ull;
@@ -161,7 +174,7 @@ __global__ void __launch_bounds__(256) lp_grad_batch_kernel(Args k, float* __res
             float* dst = k.s.scale + (base + m) * RB + i0;
             *reinterpret_cast<float4*>(dst) = ratio ? make_float4(gv[0], gv[1], gv[2], gv[3]) : make_float4(s[0], s[1], s[2], s[3]);
             if (ratio) *reinterpret_cast<float4*>(k.s.recip + (base + m) * RB + i0) =
-                make_float4(1.f / yv[0], 1.f / yv[1], 1.f / yv[2], 1.f / yv[3]);
+                make_float4(real[0] ? 1.f / yv[0] : 0.f, real[1] ? 1.f / yv[1] : 0.f, real[2] ? 1.f / yv[2] : 0.f, real[3] ? 1.f / yv[3] : 0.f);
             if ((threadIdx.x & 31) == 0) k.s.ratio[(base + m) / MC] = ratio ? 1u : 0u;
         }
     }
@@ -181,6 +194,19 @@ __device__ __forceinline__ void product_rows(const float* xr, float* acc, float 
         if (i % 4 == 0) __builtin_amdgcn_sched_barrier(0);   // more rows at once would take the registers of a fourth wavefront
     }
 }
+// eight rows of one channel from the ratio
+template <int IP, bool GW, class Rest>
+__device__ __forceinline__ void ratio_rows(const float* xr, float* acc, float (&ws)[2], f8v g, f8v recip, float wk, Rest rest) {
+    #pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const float pw = ratio_power<IP>((xr[i] - wk) * recip[i]);
+        acc[i] = fmaf(g[i], pw, acc[i]);
+        asm volatile("" : "+v"(acc[i]));
+        if (GW) ws[i & 1] = fmaf(g[i], pw, ws[i & 1]);
+        if (i == 0) { __builtin_amdgcn_sched_barrier(0); rest(); }
+        if (i % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+    }
+}
 // eight rows of one channel at any power; rows past the batch have g = 1 / y = 0.  (The transcendentals bound it, at any number of
 // wavefronts: four rows side by side took 4 % longer.)
 template <bool GW, class Rest>
@@ -196,6 +222,8 @@ __device__ __forceinline__ void any_power_rows(const float* xr, float* acc, floa
         if (i % 4 == 0) __builtin_amdgcn_sched_barrier(0);
     }
 }
+
+enum Form { kProduct, kRatio, kNothing };
 
 // WAVES = kTiles: the wavefronts of a workgroup take neighbouring batch tiles of the same inputs and their sums of grad_weight
 // meet in LDS, so that memory sees one addition per 128 rows.  WAVES = 1: they have nothing to do with each
@@ -213,8 +241,9 @@ __global__ void __launch_bounds__(256, 4) lp_grad_kernel(Args k) {
     // all batch tiles of a (block of inputs, slice) run on one die one after the other: they share its weights there
     const unsigned die = blockIdx.x % 8, waves = WAVES > 1 ? 1 : blockDim.x / 64, own = WAVES > 1 ? 0 : wave;
     const unsigned unit = (k.by_die ? blockIdx.x / 8 : blockIdx.x) * waves + own;
-    const unsigned pair = k.by_die ? die + 8 * (unit / k.groups) : unit % k.pairs;
-    const unsigned group = k.by_die ? unit % k.groups : unit / k.pairs;
+    // (in scalar registers, with all that follows from them: the compiler kept some of it in vector registers)
+    const unsigned pair = __builtin_amdgcn_readfirstlane(k.by_die ? die + 8 * (unit / k.groups) : unit % k.pairs);
+    const unsigned group = __builtin_amdgcn_readfirstlane(k.by_die ? unit % k.groups : unit / k.pairs);
     if (pair >= k.pairs || group >= k.groups) return;
     const int nblock = pair % k.nblocks, g = pair / k.nblocks % a.G, slice = pair / k.nblocks / a.G;
     const int m_lo = slice * k.per, m_hi = m_lo + k.per < a.COg ? m_lo + k.per : a.COg;
@@ -260,7 +289,7 @@ __global__ void __launch_bounds__(256, 4) lp_grad_kernel(Args k) {
     const Const<uint32_t> ratio = as_const<uint32_t>(k.s.ratio + base / MC);
     const uint32_t* modes = k.s.ratio + base / MC;
     const int c_hi = (m_hi + MC - 1) / MC;
-    uint32_t mode = IP >= 0 && m_lo / MC + lane < c_hi ? modes[m_lo / MC + lane] : 0u;
+    uint32_t mode = IP > 0 && m_lo / MC + lane < c_hi ? modes[m_lo / MC + lane] : 0u;
 
     float xr[RB], acc[RB];
     if constexpr (STRIDED) {
@@ -291,10 +320,10 @@ __global__ void __launch_bounds__(256, 4) lp_grad_kernel(Args k) {
     float wv[MC];
     #pragma unroll
     for (int j = 0; j < MC; j++) wv[j] = wbase[(size_t)row_of(m_lo, j, rowv) * a.W_CIg];
-    // a slice without a chunk that forms ratios runs the loop without that path, which would cost it copies of its sums
-    for (int c = m_lo / MC + 64 + lane; IP >= 0 && c < c_hi; c += 64) mode |= modes[c];
-    // (nor would 0 times a power of a difference be 0 in a tile behind the batch, where no output says that the power is finite)
-    const bool ratios = rows == 0 || __builtin_amdgcn_ballot_w64(mode != 0u) != 0ull;
+    for (int c = m_lo / MC + 64 + lane; IP > 0 && c < c_hi; c += 64) mode |= modes[c];
+    // A slice without a chunk that forms ratios runs a loop without them, one instruction less per term (both gradients of 512 x 5120 x
+    // 512 with such chunks / without, us: p = 3 198 / 148, p = 8 231 / 190; row by row, with loads of one value, 507 and 519).
+    const bool ratios = __builtin_amdgcn_ballot_w64(mode != 0u) != 0ull;
 
     auto add_weight = [&](int row, float v) {
         float* dst = gwbase + (size_t)row * a.W_CIg;
@@ -302,8 +331,8 @@ __global__ void __launch_bounds__(256, 4) lp_grad_kernel(Args k) {
         else unsafeAtomicAdd(dst, v);
     };
 
-    auto walk = [&](auto mixed) {
-        constexpr bool MIXED = decltype(mixed)::value;
+    auto walk = [&](auto tag) {
+        constexpr Form FORM = decltype(tag)::value;
         int buf = 0;
         for (int m0 = m_lo; m0 < m_hi; m0 += MC, buf ^= 1) {
             float wn[MC];
@@ -329,7 +358,7 @@ __global__ void __launch_bounds__(256, 4) lp_grad_kernel(Args k) {
                     asm volatile("" : "+v"(sum[j]));
                 }
                 asm volatile("" :: "s"(next));
-            } else if constexpr (!MIXED) {
+            } else if constexpr (FORM == kProduct) {
                 f16v s0 = block(m0, 0);
                 float next = 0.f;   // brings the next chunk's first block as far as the scalar cache
                 #pragma unroll
@@ -345,28 +374,33 @@ __global__ void __launch_bounds__(256, 4) lp_grad_kernel(Args k) {
                     asm volatile("" : "+v"(sum[j]));
                 }
                 asm volatile("" :: "s"(next));
-            } else {
-                // rare: row by row, with few registers; elsewhere d^(p-1) is the power of a "ratio" d * 1
+            } else if constexpr (FORM == kRatio) {
+                // (a chunk of products: d^(p-1) is the power of the "ratio" d * 1)
                 const bool form = ratio[m0 / MC] != 0u;
-                float w0 = wv[0], w1 = wv[1], w2 = wv[2], w3 = wv[3];
-                static_assert(MC == 4, "the weights and sums of a chunk are passed round by hand");
-                #pragma unroll 1
-                for (int j = 0; j < MC; j++) {
-                    const float wk = w0;
-                    float ws = 0.f;
+                const Const<float> g = scale + (size_t)m0 * RB, r = recip + (size_t)m0 * RB;
+                auto recips = [&](int at) {
+                    u8v v = *(Const<u8v>)(r + at);   // (whole numbers: a choice between floats would take vector instructions)
                     #pragma unroll
-                    for (int i = 0; i < RB; i++) {
-                        if (i < rows && m0 + j < m_hi) {   // rows past the batch count nothing, whatever the operands
-                            const float gv = scale[(size_t)(m0 + j) * RB + i], ry = form ? recip[(size_t)(m0 + j) * RB + i] : 1.f;
-                            const float pw = ratio_power<IP>((xr[i] - wk) * ry);
-                            acc[i] = fmaf(gv, pw, acc[i]);
-                            ws = fmaf(gv, pw, ws);
-                        }
-                        asm volatile("" : "+v"(acc[i]), "+v"(ws));
-                        __builtin_amdgcn_sched_barrier(0);
+                    for (int i = 0; i < 8; i++) v[i] = form ? v[i] : 0x3f800000u;
+                    return __builtin_bit_cast(f8v, v);
+                };
+                f8v g0 = *(Const<f8v>)g, r0 = recips(0);
+                #pragma unroll
+                for (int j = 0; j < MC; j++) {
+                    float ws[2] = {0.f, 0.f};
+                    #pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        f8v g1 = g0, r1 = r0;
+                        ratio_rows<IP, GW>(xr + 8 * q, acc + 8 * q, ws, g0, r0, wv[j], [&] {
+                            if (j * 4 + q + 1 < 4 * MC) {
+                                g1 = *(Const<f8v>)(g + (j * 4 + q + 1) * 8);
+                                r1 = recips((j * 4 + q + 1) * 8);
+                            }
+                        });
+                        g0 = g1; r0 = r1;
                     }
-                    w0 = w1; w1 = w2; w2 = w3; w3 = wk;
-                    sum[0] = sum[1]; sum[1] = sum[2]; sum[2] = sum[3]; sum[3] = ws;
+                    sum[j] = ws[0] + ws[1];
+                    asm volatile("" : "+v"(sum[j]));
                 }
             }
             if (GW && WAVES > 1) {
@@ -391,9 +425,10 @@ __global__ void __launch_bounds__(256, 4) lp_grad_kernel(Args k) {
             if (LISTS) { rowv = rown; rown = rows_of(m0 + 2 * MC); }
         }
     };
-    if constexpr (IP < 0) walk(std::false_type{});
-    else if (ratios) walk(std::true_type{});
-    else walk(std::false_type{});
+    // (0 times the power of a difference is not 0 where the power overflows, and no output says that it does not in a tile behind the batch)
+    if (WAVES > 1 && IP >= 0 && rows == 0) walk(std::integral_constant<Form, kNothing>{});
+    else if (IP <= 0 || !ratios) walk(std::integral_constant<Form, kProduct>{});
+    else walk(std::integral_constant<Form, IP <= 0 ? kProduct : kRatio>{});
     // what only the end needs is read again here: it would take scalar registers all the way
     Const<Args> late = (Const<Args>)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(late));

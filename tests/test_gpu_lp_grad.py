@@ -103,3 +103,45 @@ def test_input_gradients_of_large_batches(p):
         parts[-1] = (parts[-1].double() + t.double() * d.double()).float()   # one fused multiply-add
     error = lambda got: float((got.double() - exact).norm() / exact.norm())   # noqa: E731
     assert error(gx[rows, :, 0]) <= 1.1 * error(sum(parts))
+
+
+@pytest.mark.parametrize("p", [2.0, 3.0, 4.0, 5.0, 6.0, 7.0, 8.0, 9.0])
+@pytest.mark.parametrize("gscale", [1e-30, 1.0, 1e30])
+def test_edges_of_the_ranges(oracle, p, gscale):
+    """Every row at a scale of its own, from far below to far above the limits of the product form (2^(-70 / (p-1)) to 2^(120 / (p-1)) for an
+    output); gradients are so of ratios, whatever the scale."""
+    g = torch.Generator().manual_seed(int(p))
+    B, N, M = 64, 70, 40
+    reach = 124 / (p - 1)
+    scale = 2.0 ** torch.linspace(-max(80 / (p - 1), 8), min(reach, 110), 32).repeat_interleave(2).view(B, 1, 1)
+    x, gy = torch.randn(B, N, 1, generator=g) * scale, torch.randn(B, M, 1, generator=g) * gscale
+    _both(oracle, x, torch.randn(M, N, generator=g) * 1e-4, gy, p)
+    tile = x[30:31] * torch.randn(33, N, 1, generator=g)   # a whole tile and a row at one scale, and with zeros among the gradients
+    gy[:33, ::3] = 0
+    _both(oracle, tile.contiguous(), torch.randn(M, N, generator=g) * 1e-4, gy[:33].contiguous(), p)
+
+
+@pytest.mark.parametrize("p,xscale,gscale", [(2.0, 1000.0, 1.0), (8.0, 1000.0, 1.0), (8.0, 1.0, 1e-30)])
+def test_time_follows_the_sizes(p, xscale, gscale):
+    """Large outputs, and gradients that are almost nothing in one channel of four, take at most 1.6 times as long as ordinary ones (the
+    loop that forms ratios: 1.25; row by row it took 2.7)."""
+    from sortnet_amd import ext
+    g = torch.Generator(device="cuda").manual_seed(9)
+    x, w, gy = (torch.randn(*s, generator=g, device="cuda") for s in ((512, 5120, 1), (512, 5120), (512, 512, 1)))
+    y, gx, gw = torch.empty_like(gy), torch.empty_like(x), torch.empty_like(w)
+
+    def least(x, w, gy):
+        ext.norm_dist_forward(x, w, y, 1, p)
+        times = []
+        for _ in range(12):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            ext.norm_dist_backward_input_weight(gy, x, w, y, gx, gw, 1, p)
+            end.record()
+            end.synchronize()
+            times.append(start.elapsed_time(end))
+        return min(times)
+
+    ordinary = least(x, w, gy)
+    gy[:, ::4] *= gscale
+    assert least(x * xscale, w * xscale, gy) <= 1.6 * ordinary
