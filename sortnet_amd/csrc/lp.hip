@@ -765,6 +765,28 @@ static int run_lp_bwd(int ip, LpBwdArgs& a, const LpBwdPlan& plan, float* part, 
     return SD_OK;
 }
 
+// Whether the gradients are formed from scalar registers (lp_grad.hip) or by the general kernel.  That one leaves out groups of eight rows
+// without work where a tile of 32 is not full, and takes a launch less; it loads strided inputs one value per cache line.  Both
+// gradients / the inputs' alone, us, general kernel -> from scalar registers, rows x inputs x outputs (x positions):
+//   whole p (p = 8)  1 x 2001 x 2000 31 -> 37 / 20 -> 33, 8 x 1024 x 1024 18 -> 21 / 14 -> 20, 17 x 640 x 640 22 -> 21 / 18 -> 20, 1 x 5120 x 5120 157 -> 147
+//                    / 104 -> 128, 10 x 5120 x 5120 208 -> 151 / 153 -> 130; lists 8 x 2048 x 2048 28 -> 38 / 20 -> 28, 32 x 512 x 512 22 -> 20 / 19 -> 19
+//                    positions: 6 x 2700 x 256 x 2 +51 % / +99 %, 144 x 64 x 64 with 512 rows +21 % / +35 %, 288 x 512 with 2048 rows -62 % / -66 %
+//   p = 17.3         1 x 5120 x 2560 76 -> 171 / 56 -> 139, 17 x 3072 x 1024 57 -> 52 / 45 -> 48, 33 x 3072 x 1024 80 -> 84 / 69 -> 75, 33 x 800 x 800 40 -> 32 / 35 ->
+//                    30, 65 x 2001 x 2000 141 -> 167 / 121 -> 148, 250 x 3072 x 1021 301 -> 245 / 233 -> 218, 500 x 5120 x 2560 1941 -> 1810 / 1586 -> 1608; whole
+//                    tiles 512 x 5120 x 2560 1730 -> 1800, 128 x 3072 x 1024 128 -> 144; lists 8 x 1024 x 1024 19 -> 26, 100 x 512 x 512 31 -> 28, 512 x 1024 x 1024
+//                    129 -> 153; positions 4: 128 x 800 x 256 (105 M terms) +38 %, 512 x 2700 x 256 (354 M) -9 %, 16 and more: 64 x 64 x 27 x 1024 -55 %
+// (Both gradients of layers with positions stay with scalar registers at whole p from 17 rows on, also where they take longer, 8 x 2700 x 256 x 4
+// 32 -> 36 us, 32 x 288 x 512 x 2 23 -> 29: their error against 64 bits is smaller, 32 x 2700 x 256 x 4 3.7e-7 -> 2.5e-7.)
+static bool lp_grad_pays(const FwdArgs& f, bool both, bool whole) {
+    const long long weights = (long long)f.G * f.COg * f.CIg, terms = weights * f.R;
+    if (f.HW > 1) return f.R > 16 && ((whole && both) || terms >= (f.HW >= 16 ? 1ll << 23 : f.HW >= 9 ? 1ll << 26 : 1ll << 28));
+    if (f.ci_idx || f.co_idx) return whole ? f.R > (both ? 8 : 16) : f.R > 16 && terms < (1ll << 26);
+    if (whole) return both ? f.R > 8 || weights >= (1ll << 23) : f.R > 8 && terms >= (1ll << 24) && (f.R > 16 || weights >= (1ll << 24));
+    // rows that the two kernels go through
+    const int tiles = (f.R + RB - 1) / RB * RB, eights = (f.R + 7) / 8 * 8;
+    return f.R % RB != 0 && f.R > 16 && (7ll * tiles <= 8ll * eights || terms < (1ll << 26));
+}
+
 static int lp_backward(const char* who, const float* grad_output, const float* input, const float* weight,
                        const float* output, int B, int CO, int CI, int G, int HW, float* grad_input,
                        float* grad_weight, float p, const int* ci_idx, const int* co_idx, int W_CO, int W_CI,
@@ -785,8 +807,9 @@ static int lp_backward(const char* who, const float* grad_output, const float* i
     a.skip_thr = int_power(p - 1.f) < 0 ? lp_skip_threshold(1e-16f, p - 1.f, kLpSkipFrom) : 0.f;
     hipStream_t st = static_cast<hipStream_t>(stream);
     int ip = int_power(p - 1.f);
-    // from scalar registers where the scratch for it is at hand (a stream under capture may lack it) and the gradients are aligned
-    // to 16 bytes; else, and for what is left, the general kernel below
+    // from scalar registers where that pays, the scratch for it is at hand (a stream under capture may lack it) and the gradients are
+    // aligned to 16 bytes; else, and for what is left, the general kernel below
+    const bool pays = lp_grad_pays(f, grad_weight != nullptr, ip >= 0);
     auto from_scalars = [&](int power) -> int {
         if (!aligned16(grad_input) || !aligned16(grad_weight)) return -1;
         const LpGradArgs b{grad_output, input, weight, output, grad_input, grad_weight, ci_idx, co_idx,
@@ -796,7 +819,7 @@ static int lp_backward(const char* who, const float* grad_output, const float* i
         void* ws = workspace(bytes, st);
         return ws ? lp_grad(power, a.pm1, b, ws, st) : SD_ERR_HIP;
     };
-    if (ip >= 0 && (rc = from_scalars(ip)) >= 0) return rc;
+    if (ip >= 0 && pays && (rc = from_scalars(ip)) >= 0) return rc;
     // large p with both gradients in the dense single-group case: the kernel that forms every term once for both
     // sums and owns its grad_weight block tests significance more cheaply than the general kernel, whose
     // test only pays from a higher threshold; everything else goes through the general kernel
@@ -821,12 +844,8 @@ static int lp_backward(const char* who, const float* grad_output, const float* i
     // (both gradients, in us, by atomic additions -> from planes: 250 x 3072 x 1021 at p = 24 297 -> 312, 512 x 600 x 600
     // at p = 100 94 -> 101, 2048 x 1024 x 1024 at p = 120 in eight launches 639 -> 717, the fused kernel 3215).
     const bool same_bits = !fused && (fused_p || (rows_p && !rows));
-    // Other powers without significance tests, as far as none of the above takes them: several positions per image, dense batches that
-    // are no whole tiles, small layers with index lists.  (Both gradients, in us, general kernel / from scalar registers, p = 17.3:
-    // 64 x 288 x 256 on 16 x 16 positions 1040 / 410, 300 x 801 x 333 61 / 52, 250 x 3072 x 1021 298 / 256, lists 64 x 768 x 768 of 1024
-    // 41 / 36; but 512 x 5120 x 2560 1730 / 1800, 128 x 3072 x 1024 128 / 144, lists 512 x 3840 x 3840 of 5120 1880 / 2060.)
-    const bool scalars = HW > 1 || (!ci_idx && !co_idx ? f.R % RB != 0 : (long long)f.R * G * f.COg * f.CIg < (1ll << 26));
-    if (ip < 0 && scalars && a.pm1 > 0.f && a.skip_thr == 0.f && !rows && !fused && !same_bits && (rc = from_scalars(-1)) >= 0) return rc;
+    // other powers without significance tests, as far as none of the above takes them
+    if (ip < 0 && pays && a.pm1 > 0.f && a.skip_thr == 0.f && !rows && !fused && !same_bits && (rc = from_scalars(-1)) >= 0) return rc;
     // one request for every user of the workspace: the tables and 1 / y, then the planes of partial sums
     const size_t table_bytes = rows ? (lp_rows_workspace(f.R, f.COg, f.CIg) + (size_t)f.R * f.COg * sizeof(float) + 255) / 256 * 256 : 0;
     LpBwdPlan plan{};

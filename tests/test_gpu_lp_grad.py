@@ -145,3 +145,33 @@ def test_time_follows_the_sizes(p, xscale, gscale):
     ordinary = least(x, w, gy)
     gy[:, ::4] *= gscale
     assert least(x * xscale, w * xscale, gy) <= 1.6 * ordinary
+
+
+@pytest.mark.parametrize("p,B,N,M,HW,both,scalars", [
+    (8.0, 8, 1024, 1024, 1, True, False), (8.0, 9, 1024, 1024, 1, True, True), (8.0, 3, 3072, 2800, 1, True, True), (8.0, 8, 5120, 5120, 1, False, False),
+    (8.0, 17, 640, 640, 1, False, False), (8.0, 33, 1024, 1024, 1, False, True), (2.0, 8, 27, 64, 2, True, False), (8.0, 9, 27, 64, 2, True, True),
+    (8.0, 64, 288, 256, 4, False, False), (8.0, 32, 288, 128, 16, False, True), (17.3, 4, 1024, 1024, 1, True, False), (17.3, 33, 2001, 2000, 1, True, False),
+    (17.3, 33, 800, 800, 1, True, True), (17.3, 250, 1024, 1024, 1, True, True), (17.3, 64, 800, 800, 1, True, False), (17.3, 128, 800, 256, 4, True, False)])
+def test_which_kernel(oracle, p, B, N, M, HW, both, scalars):
+    """Few rows, and small layers where only the gradient of the inputs is asked for, go through the general kernel."""
+    from torch.profiler import ProfilerActivity, profile
+    from sortnet_amd import ext
+    g = torch.Generator().manual_seed(B)
+    x, w, gy = (torch.randn(*s, generator=g) for s in ((B, N, HW), (M, N), (B, M, HW)))
+    y = torch.empty(B, M, HW, device="cuda")
+    xd, wd, gd = x.cuda(), w.cuda(), gy.cuda()
+    ext.norm_dist_forward(xd, wd, y, 1, p)
+    gx, gw = torch.empty_like(xd), torch.empty_like(wd)
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        if both:
+            ext.norm_dist_backward_input_weight(gd, xd, wd, y, gx, gw, 1, p)
+        else:
+            ext.norm_dist_backward_input(gd, xd, wd, y, gx, 1, p)
+        torch.cuda.synchronize()
+    names = [e.name for e in prof.events()]
+    assert any("lp_grad_kernel" in n for n in names) == scalars and any("lp_bwd_kernel" in n for n in names) != scalars, names
+    if B * N * M * HW < 1 << 25:
+        rgx, rgw = oracle.norm_dist_backward(gy.numpy(), x.numpy(), w.numpy(), y.cpu().numpy(), p)
+        _check(gx, rgx)
+        if both:
+            _check(gw, rgw)
