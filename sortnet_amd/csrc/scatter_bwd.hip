@@ -155,7 +155,6 @@ __global__ void __launch_bounds__(1024) scatter_bwd_rows_kernel(BwdArgs a) {
     input_row<SORT, HAS_W>(a, blockIdx.x, hist);
 }
 
-template <bool HAS_W>
 __device__ __forceinline__ void bound_row(const BwdArgs& a, int row, float* hist) {   // hist: [0, CIg) lower, [CIg, 2 CIg) upper
     const int hw = row % a.HW;
     const int bg = row / a.HW;
@@ -165,17 +164,12 @@ __device__ __forceinline__ void bound_row(const BwdArgs& a, int row, float* hist
     const size_t obase = ((size_t)(b * a.G + g) * a.COg) * a.HW + hw;
     for (int m = threadIdx.x; m < a.COg; m += blockDim.x) {
         size_t o = obase + (size_t)m * a.HW;
-        size_t wrow = (size_t)(g * a.COg + m) * a.CIg;
         int pl = a.p0[o], pu = a.p1[o];
         float gl = a.g0[o], gu = a.g1[o];
         int nl = pl & 0x7fffffff, nu = pu & 0x7fffffff;
         float vl = pl >= 0 ? gl : -gl, vu = pu >= 0 ? gu : -gu;
-        if ((uint32_t)pl != kNanId) {
-            atomicAdd(&hist[(pl >= 0 ? 0 : a.CIg) + nl], vl);
-            if (HAS_W) unsafeAtomicAdd(a.gw + wrow + nl, -vl);
-        }
+        if ((uint32_t)pl != kNanId) atomicAdd(&hist[(pl >= 0 ? 0 : a.CIg) + nl], vl);
         atomicAdd(&hist[(pu >= 0 ? a.CIg : 0) + nu], vu);
-        if (HAS_W) unsafeAtomicAdd(a.gw + wrow + nu, -vu);
     }
     __syncthreads();
     const size_t xbase = ((size_t)(b * a.G + g) * a.CIg) * a.HW + hw;
@@ -238,10 +232,9 @@ __global__ void __launch_bounds__(1024) positions_bwd_kernel(BwdArgs a, int P) {
     input_positions<BOUND>(a, blockIdx.x, P, hist);
 }
 
-template <bool HAS_W>
 __global__ void __launch_bounds__(256) bound_bwd_rows_kernel(BwdArgs a) {
     extern __shared__ __attribute__((aligned(16))) float hist[];
-    bound_row<HAS_W>(a, blockIdx.x, hist);
+    bound_row(a, blockIdx.x, hist);
 }
 
 // grad_weight by rows (dense layers, no index lists): one workgroup owns WR consecutive weight rows,
@@ -369,7 +362,7 @@ __global__ void __launch_bounds__(1024) both_bwd_kernel(BwdArgs a, int WR, const
         if constexpr (MODE == 3) weight_rows_lists(a, WR, place, blockIdx.x, hist);
         else weight_rows<MODE>(a, WR, blockIdx.x, hist);
     } else if (P > 1) input_positions<MODE == 2>(a, blockIdx.x - w_blocks, P, hist);
-    else if constexpr (MODE == 2) bound_row<false>(a, blockIdx.x - w_blocks, hist);
+    else if constexpr (MODE == 2) bound_row(a, blockIdx.x - w_blocks, hist);
     else input_row<false, false>(a, blockIdx.x - w_blocks, hist);
 }
 
@@ -461,7 +454,8 @@ static int run_scatter(BwdArgs& a, hipStream_t st) {
             while (rows.y < 8u && rows.x * rows.y < 2u * (unsigned)num_cus() && a.CIg / (int)(2 * rows.y) >= 256) rows.y *= 2;
         }
         const size_t lds = (size_t)((a.CIg + (int)rows.y - 1) / (int)rows.y) * sizeof(float);
-        if (x.gw) hipLaunchKernelGGL((scatter_bwd_rows_kernel<SORT, true>), rows, block, lds, st, x);
+        // (weight rows of so many inputs have been taken by rows, but for index lists)
+        if (!SORT && x.gw) hipLaunchKernelGGL((scatter_bwd_rows_kernel<false, true>), rows, block, lds, st, x);
         else hipLaunchKernelGGL((scatter_bwd_rows_kernel<SORT, false>), rows, block, lds, st, x);
         return check_launch("scatter_bwd_rows_kernel");
     }
@@ -560,11 +554,8 @@ static int bound_bwd(const char* who, const float* gL, const float* gU, const in
                            (size_t)2 * a.CIg * P * sizeof(float), st, a, P);
         return check_launch("positions_bwd_kernel");
     }
-    if (2 * a.CIg <= kMaxRowLds) {
-        dim3 rows((unsigned)(B * G * HW));
-        size_t lds = (size_t)2 * a.CIg * sizeof(float);
-        if (gw) hipLaunchKernelGGL((bound_bwd_rows_kernel<true>), rows, dim3(256), lds, st, a);
-        else hipLaunchKernelGGL((bound_bwd_rows_kernel<false>), rows, dim3(256), lds, st, a);
+    if (2 * a.CIg <= kMaxRowLds) {   // (weight rows of such inputs have been taken by rows above)
+        hipLaunchKernelGGL(bound_bwd_rows_kernel, dim3((unsigned)(B * G * HW)), dim3(256), (size_t)2 * a.CIg * sizeof(float), st, a);
         return check_launch("bound_bwd_rows_kernel");
     }
     if ((rc = fill_zero(gxL, nx, st))) return rc;
