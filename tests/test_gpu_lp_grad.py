@@ -175,3 +175,48 @@ def test_which_kernel(oracle, p, B, N, M, HW, both, scalars):
         _check(gx, rgx)
         if both:
             _check(gw, rgw)
+
+
+def _against_64(x, w, gy, p):
+    """Both gradients on the GPU against 64-bit sums there, channel by channel; y as a forward in 64 bits gives it."""
+    from sortnet_amd import ext
+    x, w, gy = x.cuda(), w.cuda(), gy.cuda()
+    y = torch.empty_like(gy)
+    gx, gw = torch.full_like(x, 7), torch.full_like(w, 7)
+    rx, rw = torch.zeros_like(x, dtype=torch.float64), torch.zeros_like(w, dtype=torch.float64)
+    for m in range(w.shape[0]):
+        d = x.double() - w[m, None, :, None].double()
+        y[:, m] = (d.abs() ** p).sum(1) ** (1 / p)
+        u = gy[:, m, None].double() * d.sign() * (d.abs() / y[:, m, None].double()) ** (p - 1)
+        rx += u
+        rw[m] = -u.sum((0, 2))
+    ext.norm_dist_backward_input_weight(gy, x, w, y, gx, gw, 1, p)
+    _check(gx, rx.cpu().numpy())
+    _check(gw, rw.cpu().numpy())
+
+
+@pytest.mark.parametrize("p", [2.0, 8.0, 9.0])
+@pytest.mark.parametrize("B,N,M,HW,odd", [
+    (337, 6016, 10, 1, False), (337, 6016, 10, 1, True),      # 11 tiles of three workgroups, the last one's with one row; chunks that form ratios in it
+    (43, 27, 17, 784, False), (43, 27, 17, 784, True),        # positions, 1054 tiles
+    (128, 16500, 9, 1, True), (101, 16500, 9, 1, False),      # the whole batch in a workgroup
+    (79, 3, 577, 1009, True)])                                # more tiles than the tables of one launch hold
+def test_workgroups_of_four_tiles(p, B, N, M, HW, odd):
+    assert -(-N // 64) * -(-B * HW // 32) >= 1024   # (batch tile, 64 inputs) pairs from which on four tiles make a workgroup
+    g = torch.Generator().manual_seed(B + N)
+    x, w, gy = torch.randn(B, N, HW, generator=g), torch.randn(M, N, generator=g), torch.randn(B, M, HW, generator=g)
+    if odd:   # outputs outside the product form's range in one tile of a workgroup, and in the chunks of one channel
+        x[B // 2] *= 1e9 if p > 2 else 1e36
+        w[M // 2] *= 1e-9
+        x[B // 3] *= 1e-9
+    _against_64(x, w, gy, p)
+
+
+@pytest.mark.parametrize("p", [3.0, 17.3])
+def test_other_shapes_with_many_tiles(oracle, p):
+    """Groups and four tiles to a workgroup at other powers; index lists over more than one round of wavefronts."""
+    g = torch.Generator().manual_seed(2)
+    _both(oracle, torch.randn(333, 2 * 3010, 1, generator=g), torch.randn(10, 3010, generator=g), torch.randn(333, 10, 1, generator=g), p, 2)
+    keep = lambda c, k: torch.rand(18, 1, c, generator=g).argsort(-1)[..., :k].sort(-1)[0].to(torch.int32).contiguous()   # noqa: E731
+    x, gy = torch.randn(570, 3900, 1, generator=g), torch.randn(570, 9, 1, generator=g)
+    _both(oracle, x, torch.randn(14, 5000, generator=g), gy, p, 1, keep(5000, 3900), keep(14, 9))

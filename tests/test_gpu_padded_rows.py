@@ -102,3 +102,38 @@ def test_factored_mask_against_the_oracle(oracle, B, N, M, q):
     assert _lib.last_forward_kernel().startswith("fwd_kernel_pipe")
     for got, want in ((y, ry), (y2, ry), (pos, rp)):
         np.testing.assert_array_equal(got.cpu().numpy(), np.asarray(want).reshape(B, M, 1).astype(got.cpu().numpy().dtype))
+
+
+@pytest.mark.parametrize("B,N,M,q,density", [(200, 5131, 140, 0.3, 1.0), (129, 2049, 517, 0.6, 1.0), (257, 4097, 2100, 0.3, None)])
+def test_factored_mask_from_tables(oracle, B, N, M, q, density):
+    """Padded copies, keep bits of the raw length and candidate tables together: at a forced density, and at the built-in limit (2^31 terms)."""
+    from sortnet_amd import _lib, ext
+    g = torch.Generator().manual_seed(B)
+    x, w = torch.randn(B, N, 1, generator=g) * 0.02, torch.randn(M, N, generator=g)   # (batch rows alike: tables per weight row)
+    x[0, N - 1], w[1, 2], w[2, N - 1], w[3] = float("nan"), float("inf"), -9.0, 0.0
+    rows, cols = min(B, 40), min(M, 300)   # (a row's keep bits come from its number)
+    ry, rp = oracle.masked_inf_dist_forward(x[:rows].numpy(), w[:cols].numpy(), q, 11, oracle.MASK_FACTORED)
+    xd, wd = x.cuda(), w.cuda()
+    new = lambda t: torch.full((B, M, 1), 7, device="cuda", dtype=t)   # noqa: E731
+
+    def run():
+        y, y2, pos = new(torch.float32), new(torch.float32), new(torch.int32)
+        ext.masked_inf_dist_forward(xd, wd, y, pos, 1, q, 11, ext.MASK_FACTORED)
+        share = _lib.last_forward_term_share()
+        ext.masked_inf_dist_forward(xd, wd, y2, None, 1, q, 11, ext.MASK_FACTORED)
+        return y, y2, pos, max(share, _lib.last_forward_term_share())
+
+    try:
+        _lib.set_linf_candidate_density(0.0)
+        *every, share = run()
+        assert share == 1.0
+        _lib.set_linf_candidate_density(-1.0 if density is None else density)
+        *got, share = run()
+    finally:
+        _lib.set_linf_candidate_density(-1.0)
+    assert share < 1.0
+    for a, b in zip(got, every):
+        assert torch.equal(a, b)
+    for a, want in zip(got, (ry, ry, rp)):
+        a = a[:rows, :cols].cpu().numpy()
+        np.testing.assert_array_equal(a, np.asarray(want).reshape(a.shape).astype(a.dtype))
