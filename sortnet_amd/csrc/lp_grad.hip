@@ -38,9 +38,9 @@ constexpr int second_factor(int ip) { return ip <= 2 ? 1 : ip == 3 ? 2 : ip == 4
 constexpr double two_to(int e) { double v = 1.0; for (; e > 0; e--) v *= 2.0; for (; e < 0; e++) v *= 0.5; return v; }
 template <int IP> struct Limits {
     static constexpr int J = second_factor(IP), I = IP - J;
-    static constexpr double kYLow = two_to(-70 / IP), kYHigh = two_to(120 / IP);
-    static constexpr double kFirstLow = two_to(-126 + (56 * I + IP - 1) / IP), kFirstHigh = two_to(120);   // |g| y^-J, the first factor at |d| = y
-    static constexpr double kScaleLow = two_to(-125), kScaleHigh = two_to(120);                        // |g| y^(1-p)
+    static constexpr float kYLow = (float)two_to(-70 / IP), kYHigh = (float)two_to(120 / IP);
+    static constexpr float kFirstLow = (float)two_to(-126 + (56 * I + IP - 1) / IP), kFirstHigh = 0x1p+120f;   // |g| y^-J, the first factor at |d| = y
+    static constexpr float kScaleLow = 0x1p-125f, kScaleHigh = 0x1p+120f;                                  // |g| y^(1-p)
 };
 template <int N> __device__ __forceinline__ double power(double v) {
     if constexpr (N <= 1) return N ? v : 1.0;
@@ -146,7 +146,6 @@ __global__ void __launch_bounds__(256) lp_grad_batch_kernel(Args k, float* __res
     for (int e = 0; e < 2; e++) {
         const int j = (tid >> 3) + 32 * e, m = m0 + j;
         float s[4], yv[4], gv[4];
-        bool real[4];
         if (IP < 0) {
             if (m < k.COp) {
                 float4* dst = reinterpret_cast<float4*>(k.s.scale + ((base + m) * RB + i0) * 2);
@@ -159,22 +158,25 @@ __global__ void __launch_bounds__(256) lp_grad_batch_kernel(Args k, float* __res
         #pragma unroll
         for (int i = 0; i < 4; i++) {
             gv[i] = gs[i0 + i][j]; yv[i] = ys[i0 + i][j];
-            real[i] = r0 + i0 + i < a.R && m < a.COg;
             if constexpr (IP > 0) {
                 using L = Limits<IP>;
-                const double y = (double)yv[i], v = 1.0 / y, scale = (double)gv[i] * power<IP>(v), size = fabs(scale);
-                const double first = fabs((double)gv[i]) * power<L::J>(v);
-                s[i] = (float)scale;
-                bad |= real[i] && (!(y >= L::kYLow && y <= L::kYHigh) ||
-                                   !(gv[i] == 0.f || (size >= L::kScaleLow && size <= L::kScaleHigh && first >= L::kFirstLow && first <= L::kFirstHigh)));
+                // (few operations on 64 bits, and the limits tested on 32: they are this kernel's time)
+                const double v = 1.0 / (double)yv[i], first = (double)gv[i] * power<L::J>(v);
+                s[i] = (float)(first * power<L::I>(v));
+                const float size = fabsf(s[i]), part = fabsf((float)first);
+                const bool fits = (size >= L::kScaleLow) & (size <= L::kScaleHigh) & (part >= L::kFirstLow) & (part <= L::kFirstHigh);
+                bad |= !((yv[i] >= L::kYLow) & (yv[i] <= L::kYHigh) & (fits | (gv[i] == 0.f)));   // (never a row past the batch: 0 and 1)
             } else s[i] = gv[i];
         }
         const bool ratio = ((__builtin_amdgcn_ballot_w64(bad) >> (threadIdx.x & 32)) & 0xffffffffull) != 0ull;
         if (m < k.COp) {
             float* dst = k.s.scale + (base + m) * RB + i0;
             *reinterpret_cast<float4*>(dst) = ratio ? make_float4(gv[0], gv[1], gv[2], gv[3]) : make_float4(s[0], s[1], s[2], s[3]);
-            if (ratio) *reinterpret_cast<float4*>(k.s.recip + (base + m) * RB + i0) =
-                make_float4(real[0] ? 1.f / yv[0] : 0.f, real[1] ? 1.f / yv[1] : 0.f, real[2] ? 1.f / yv[2] : 0.f, real[3] ? 1.f / yv[3] : 0.f);
+            if (ratio) {
+                const int real = m < a.COg ? a.R - r0 - i0 : 0;
+                *reinterpret_cast<float4*>(k.s.recip + (base + m) * RB + i0) =
+                    make_float4(real > 0 ? 1.f / yv[0] : 0.f, real > 1 ? 1.f / yv[1] : 0.f, real > 2 ? 1.f / yv[2] : 0.f, real > 3 ? 1.f / yv[3] : 0.f);
+            }
             if ((threadIdx.x & 31) == 0) k.s.ratio[(base + m) / MC] = ratio ? 1u : 0u;
         }
     }
