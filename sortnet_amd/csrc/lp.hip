@@ -624,11 +624,22 @@ __global__ void __launch_bounds__(256) lp_merge_kernel(LpMerge gx, LpMerge gw, c
     const int per = (m.planes + 3) / 4, lo = quarter * per, hi = lo + per < m.planes ? lo + per : m.planes;
     float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
     if (o < m.total) {      // (a plane is a whole number of 16-byte words)
-        #pragma unroll 8
-        for (int k = lo; k < hi; k++) {
+        // Every fourth plane to a sum of its own: a small layer is cut into slices of four channels, and one sum over a quarter of them was
+        // further off than with fewer planes (relative error of grad_input, 16 x 164 x 1417 at p = 1: 178 planes 1.4e-7, 355 planes 1.7e-7, with
+        // these sums 1.1e-7; 4.1 us either way).
+        auto add = [&](float4& t, int k) __attribute__((always_inline)) {
             const float4 v = *reinterpret_cast<const float4*>(m.part + k * m.plane + o);
-            s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
-        }
+            t.x += v.x; t.y += v.y; t.z += v.z; t.w += v.w;
+        };
+        float4 t[3] = {s, s, s};
+        int k = lo;
+        #pragma unroll 2
+        for (; k + 4 <= hi; k += 4) { add(s, k); add(t[0], k + 1); add(t[1], k + 2); add(t[2], k + 3); }
+        for (; k < hi; k++) add(s, k);
+        s.x = (s.x + t[0].x) + (t[1].x + t[2].x);
+        s.y = (s.y + t[0].y) + (t[1].y + t[2].y);
+        s.z = (s.z + t[0].z) + (t[1].z + t[2].z);
+        s.w = (s.w + t[0].w) + (t[1].w + t[2].w);
     }
     sums[quarter][lane] = s;
     __syncthreads();

@@ -105,6 +105,32 @@ def test_input_gradients_of_large_batches(p):
     assert error(gx[rows, :, 0]) <= 1.1 * error(sum(parts))
 
 
+@pytest.mark.parametrize("p,B,N,M,channels", [(2.0, 167, 62, 883, 16), (1.0, 16, 164, 1417, 8)])
+def test_input_gradients_of_fine_slices(p, B, N, M, channels):
+    """Small layers, cut into slices of four output channels: the error of grad_input is not above (by more than its sampling, a tenth) that of
+    32-bit sums over slices of `channels`, as the general kernel cuts them, merged a quarter of the slices at a time."""
+    from sortnet_amd import ext
+    g = torch.Generator(device="cuda").manual_seed(8)
+    x, w, gy = (torch.randn(*s, generator=g, device="cuda") for s in ((B, N, 1), (M, N), (B, M, 1)))
+    y, gx, gw = torch.empty_like(gy), torch.empty_like(x), torch.empty_like(w)
+    ext.norm_dist_forward(x, w, y, 1, p)
+    ext.norm_dist_backward_input_weight(gy, x, w, y, gx, gw, 1, p)
+    exact, parts = torch.zeros(B, N, device="cuda", dtype=torch.float64), []
+    for m in range(M):
+        if m % channels == 0:
+            parts.append(torch.zeros(B, N, device="cuda"))
+        d = x[:, :, 0] - w[m]
+        e = x[:, :, 0].double() - w[m].double()
+        u = gy[:, m].double() * (e / y[:, m].double() if p == 2.0 else e.sign())
+        exact += u
+        t = gy[:, m] / y[:, m] if p == 2.0 else gy[:, m]
+        parts[-1] = (parts[-1].double() + t.double() * (d if p == 2.0 else d.sign()).double()).float()   # one fused multiply-add
+    per = -(-len(parts) // 4)
+    quarters = [sum(parts[q * per:(q + 1) * per]) for q in range(4)]
+    error = lambda got: float((got.double() - exact).norm() / exact.norm())   # noqa: E731
+    assert error(gx[:, :, 0]) <= 1.1 * error(quarters[0] + quarters[1] + quarters[2] + quarters[3])
+
+
 @pytest.mark.parametrize("p", [2.0, 3.0, 4.0, 5.0, 6.0, 7.0, 8.0, 9.0])
 @pytest.mark.parametrize("gscale", [1e-30, 1.0, 1e30])
 def test_edges_of_the_ranges(oracle, p, gscale):
