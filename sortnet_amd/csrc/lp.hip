@@ -728,7 +728,7 @@ static int launch_lp_bwd(int ip, const LpBwdArgs& a, hipStream_t st) {
         if (ragged) hipLaunchKernelGGL((lp_bwd_kernel<k, GW, skip, true>), grid, dim3(256), 0, st, a);   \
         else hipLaunchKernelGGL((lp_bwd_kernel<k, GW, skip, false>), grid, dim3(256), 0, st, a);         \
     } while (0)
-#define SD_CASE(k) case k: SD_LAUNCH(k, false); break;
+#define SD_CASE(k) case k: if constexpr (GW != kGwStore) SD_LAUNCH(k, false); break;   // (planes of grad_weight: p from about 20)
     switch (ip) {
         SD_CASE(0) SD_CASE(1) SD_CASE(2) SD_CASE(3) SD_CASE(4) SD_CASE(5) SD_CASE(6) SD_CASE(7) SD_CASE(8)
         default:
