@@ -85,13 +85,15 @@ float sd_last_forward_term_share(sd_stream_t stream);
  * are the default: 0.05 to 0.2 depending on the call).  Process-wide; no reference counterpart
  * (core/cuda/norm_dist_cuda.cu evaluates every term). */
 int sd_set_lp_candidate_density(float density);
-/* The same for sd_bound_inf_dist_forward_nograd and sd_bound_inf_dist_forward on dense single-group layers (CI a multiple of 32): a kernel that works
- * from a table of the inputs that can hold the maximum of a weight row over a tile of 128 batch rows, and the kernel
- * that evaluates every term; both give the same bits.  Built-in limits, layers of at least 2^31 terms: 0.30, with positions
- * 0.15; 0.40 where the table is built per batch row and tile of 128 weight rows instead, which the call decides from its
- * operands.  Smaller layers, of at least 2^27 + 3 * 2^16 * CI terms, get tables per batch row alone, at 0.18.  A `density` of 0 or
- * more applies at any size.  Values and positions are the every-term kernel's.  No reference counterpart
- * (core/cuda/bound_inf_dist_cuda.cu evaluates every term). */
+/* The same for sd_bound_inf_dist_forward_nograd and sd_bound_inf_dist_forward on dense single-group layers (where CI is
+ * no multiple of 32, and at most 65536, on copies with zeros behind every row, in the workspace; of rows that can be
+ * loaded 16 bytes at a time only from 2^31 terms): a kernel that works from a table of the inputs that can hold the
+ * maximum of a weight row over a tile of 128 batch rows, and the kernel that evaluates every term; both give the same
+ * bits.  Built-in limits, layers of at least 2^31 terms: 0.30, with positions 0.15; 0.40 where the table is built per
+ * batch row and tile of 128 weight rows instead, which the call decides from its operands.  Smaller layers, of at least
+ * 2^27 + 3 * 2^16 * CI terms, get tables per batch row alone, at 0.18.  A `density` of 0 or more applies at any size.
+ * Values and positions are the every-term kernel's.  No reference counterpart (core/cuda/bound_inf_dist_cuda.cu
+ * evaluates every term). */
 int sd_set_bound_candidate_density(float density);
 /* Which table kernel serves sd_bound_inf_dist_forward_nograd: 1 = the one that stages tiles of inputs and weights
  * through LDS (marked shares of a few per cent and more), 2 = the one that walks a weight row's marks over a
@@ -99,21 +101,24 @@ int sd_set_bound_candidate_density(float density);
  * alike), 0 (default) = 1 until a layer has reported that few marks three calls in a row, then 2 for 31 calls.  Same
  * bits whichever runs. */
 int sd_set_bound_candidate_form(int form);
-/* The same for sd_sort_neuron_forward[_nograd] and sd_bound_sort_neuron_forward on dense single-group layers (CI a
- * multiple of 32): a kernel that works from a table of the inputs that can be among the K largest terms of a weight
- * row over a tile of 128 batch rows, and the kernels that evaluate every term; both give the same bits (positions
- * included).  Built-in limits 0.40 (values of rows of fewer than 320 inputs 0.10) and, with positions, 0.22, layers of
- * at least 2^24 terms; per batch row and tile of 128 weight rows 0.27, interval bounds 0.45, positions 0.22, from 2^28 terms.  A positive
- * `density` applies at any size.  No reference counterpart (core/cuda/sort_neuron.cu evaluates every term). */
+/* The same for sd_sort_neuron_forward[_nograd] and sd_bound_sort_neuron_forward on dense single-group layers of at most
+ * 65536 inputs (where CI is no multiple of 32 on copies with zeros behind every row): a kernel that works from a table
+ * of the inputs that can be among the K largest terms of a weight row over a tile of 128 batch rows, and the kernels
+ * that evaluate every term; both give the same bits (positions included).  Built-in limits 0.40 (values of rows of
+ * fewer than 320 inputs 0.10) and, with positions, 0.22, layers of at least 2^24 terms (with positions and rows of at
+ * least 320 inputs 2^20); per batch row and tile of 128 weight rows 0.27, interval bounds 0.45, positions 0.22, from
+ * 2^28 terms.  A positive `density` applies at any size.  No reference counterpart (core/cuda/sort_neuron.cu evaluates
+ * every term). */
 int sd_set_sort_candidate_density(float density);
 /* The same for sd_inf_dist_forward[_nograd] (no index lists) and sd_masked_inf_dist_forward (factored mask) on dense
- * single-group layers (CI a multiple of 32, at most 65536): a kernel that works from a table of the inputs that can hold
- * the maximum of a weight row over a tile of 128 batch rows, and the kernels that evaluate every term; same values and
- * positions either way.  Built-in limit 0.10, layers of at least 2^31 terms; where the table is built per batch row and tile of
- * 128 weight rows instead 0.20, from 2^33 terms.  Under the mask the table's bound rests on
- * `depth` inputs per weight row, chosen so that a batch row keeps none of them less than once in 10^4 outputs (such an
- * output is recomputed from every input); sd_set_linf_candidate_depth overrides the choice (0 = automatic; 8, 12, 16,
- * 20 or 24).  No reference counterpart (core/cuda/inf_dist_cuda.cu evaluates every term). */
+ * single-group layers (CI a multiple of 32, at most 65536; under the mask also rows that cannot be loaded 16 bytes at a
+ * time, on copies with zeros behind every row): a kernel that works from a table of the inputs that can hold the
+ * maximum of a weight row over a tile of 128 batch rows, and the kernels that evaluate every term; same values and
+ * positions either way.  Built-in limit 0.10, layers of at least 2^31 terms; where the table is built per batch row and
+ * tile of 128 weight rows instead 0.20, from 2^33 terms.  Under the mask the table's bound rests on `depth` inputs per
+ * weight row, chosen so that a batch row keeps none of them less than once in 10^4 outputs (such an output is
+ * recomputed from every input); sd_set_linf_candidate_depth overrides the choice (0 = automatic; 8, 12, 16, 20 or 24).
+ * No reference counterpart (core/cuda/inf_dist_cuda.cu evaluates every term). */
 int sd_set_linf_candidate_density(float density);
 int sd_set_linf_candidate_depth(int depth);
 

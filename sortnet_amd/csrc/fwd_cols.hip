@@ -4,17 +4,17 @@
 // step ahead, without a tile in LDS; results leave in the order of memory.  The kernel that stages tiles read one input of a
 // row per cache line and stored one result per line, and the pass that finds positions behind it read 32 lines per output.
 //
-// Scalar loads and vector issue bound it: l-p at p = 8 runs at 56 T lane instructions/s, the maximum at 40.  Finding the
+// Scalar loads and vector issue bound it: l-p at p = 8 runs at 51 to 56 T lane instructions/s, the maximum at 37 to 40.  Finding the
 // positions is a gather of four inputs per output, a third of the time at 400 inputs, half at 800.  In us, tiles -> this:
 //   samples x inputs x outputs x positions   l-inf with positions   without        p = 8
-//   64 x 288 x 256 x 64                      124 -> 51              35 -> 26       40 -> 40
-//   64 x 288 x 256 x 256                     537 -> 90              86 -> 62       121 -> 101
-//   100 x 144 x 100 x 1024                   1106 -> 152            139 -> 76      210 -> 141
-//   80 x 27 x 576 x 1024                     3103 -> 244            157 -> 93      282 -> 230
-//   32 x 400 x 512 x 1024                    2297 -> 498            303 -> 271     573 -> 487
-//   128 x 800 x 1024 x 256                   5390 -> 2036           1046 -> 1027   2060 -> 1831
-// Two rows per lane (half the scalar loads per term, four wavefronts per SIMD) were slower, 62 -> 70 us at 64 x 288 x 256 x 256
-// without positions; a maximum per eight inputs, with positions, 90 -> 109 there and 2036 -> 2562 on the last.
+//   64 x 288 x 256 x 64                      135 -> 57              39 -> 31       50 -> 47
+//   64 x 288 x 256 x 256                     548 -> 102             91 -> 69       128 -> 113
+//   100 x 144 x 100 x 1024                   1101 -> 160            150 -> 81      226 -> 152
+//   80 x 27 x 576 x 1024                     3131 -> 252            173 -> 98      297 -> 242
+//   32 x 400 x 512 x 1024                    2304 -> 505            321 -> 277     592 -> 522
+//   128 x 800 x 1024 x 256                   5397 -> 1809           1071 -> 1036   2153 -> 1938
+// Two rows per lane (half the scalar loads per term, four wavefronts per SIMD) were slower, by 13 % at 64 x 288 x 256 x 256
+// without positions; a maximum per eight inputs, with positions, by 21 % there and 26 % on the last.
 #include "fwd_cols.h"
 #include "fwd_args.h"
 #include "fwd_tile.h"

@@ -5,12 +5,12 @@
 // is the same for the 64 lanes; it is laid out by tile, channel and row beforehand and read with scalar loads, 16 rows at a
 // time and one block ahead, straight into an operand of the vector instructions.
 //
-// Vector issue bounds it: 7 instructions per term at p = 8 and no LDS read, at 59 T lane instructions/s (a loop of the same
-// instructions on registers alone: 60; with the pairs (g, 1/y) read from LDS, 8 instructions and 3 wavefronts per SIMD it was 43).
-// Both gradients in us, that kernel -> this, p = 8: 512 x 5120 x 5120 2300 -> 1630, 250 x 3072 x 1021 251 -> 145, 90 x 1600 x 230
-// 36 -> 26, 32 x 192 x 192 19.4 -> 15.8; convolutions of 80 x 27 x 576 on 32 x 32 positions 1700 -> 590, of 64 x 288 x 256 on
-// 16 x 16 1000 -> 225; index lists, 512 x 3840 x 3840 of 5120 1390 -> 1320 (16 additions per weight go to memory, 0.4 ms),
-// the inputs' gradient alone 1050 -> 800.
+// Vector issue bounds it: 7 instructions per term at p = 8 and no LDS read, at 54 to 59 T lane instructions/s from one card to
+// another (a loop of the same instructions on registers alone: 60; with the pairs (g, 1/y) read from LDS, 8 instructions and 3
+// wavefronts per SIMD it was 43).  Both gradients in us, that kernel -> this, p = 8: 512 x 5120 x 5120 2460 -> 1720, 250 x 3072 x 1021 258
+// -> 151, 90 x 1600 x 230 40 -> 31, 32 x 192 x 192 24 -> 20; convolutions of 80 x 27 x 576 on 32 x 32 positions 1735 -> 610, of
+// 64 x 288 x 256 on 16 x 16 1000 -> 224; index lists, 512 x 3840 x 3840 of 5120 1436 -> 1310 (16 additions per weight go to memory,
+// 0.4 ms), the inputs' gradient alone 1049 -> 802.
 #include <cmath>
 #include <type_traits>
 #include "fwd_args.h"
