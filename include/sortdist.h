@@ -272,6 +272,20 @@ int sd_mean_shift_forward(const float* input, int B, int C, int HW, float* mean,
 int sd_channel_shift(const float* input, const float* shift, int B, int C, int HW, float sign,
                      float* output, sd_stream_t stream);
 
+/* The forwards of an evaluation pass with sd_channel_shift behind them, in one call: the same bits as the two calls
+ * (shift (CO), sign 1 or -1; outputs are those of sd_inf_dist_forward_nograd, sd_bound_inf_dist_forward_nograd,
+ * sd_sort_neuron_forward_nograd and sd_bound_sort_neuron_forward plus sign * shift[c]). */
+int sd_inf_dist_forward_shifted(const float* input, const float* weight, int B, int CO, int CI, int G, int HW,
+                                float* output, const float* shift, float sign, sd_stream_t stream);
+int sd_bound_inf_dist_forward_shifted(const float* inputL, const float* inputU, const float* weight,
+                                      int B, int CO, int CI, int G, int HW, float* outputL, float* outputU,
+                                      const float* shift, float sign, sd_stream_t stream);
+int sd_sort_neuron_forward_shifted(const float* input, const float* weight, int B, int CO, int CI, int G, int HW,
+                                   float* output, float q, int K, const float* shift, float sign, sd_stream_t stream);
+int sd_bound_sort_neuron_forward_shifted(const float* inputL, const float* inputU, const float* weight,
+                                         int B, int CO, int CI, int G, int HW, float* outputL, float* outputU,
+                                         float q, int K, const float* shift, float sign, sd_stream_t stream);
+
 /* Training-mode mean shift when every 32-sample sub-batch keeps its own channel subset
  * (core/models/bound_basic_module.py:125-137,146-153, done there with torch ops).  input / output are
  * (B, G * cnt, HW), already compacted; index is (S, G, cnt), S = ceil(B / 32), ascending channel numbers below

@@ -19,19 +19,23 @@ _u = ctypes.c_uint32
 # name -> argument types, in the order of include/sortdist.h
 SIGNATURES = {
     "sd_inf_dist_forward_nograd": [_F, _F, _i, _i, _i, _i, _i, _F, _S],
+    "sd_inf_dist_forward_shifted": [_F, _F, _i, _i, _i, _i, _i, _F, _F, _f, _S],
     "sd_inf_dist_forward": [_F, _F, _i, _i, _i, _i, _i, _F, _I, _I, _I, _i, _i, _S],
     "sd_inf_dist_forward_noalloc": [_F, _F, _i, _i, _i, _i, _i, _F, _I, _I, _I, _i, _i, _S],
     "sd_inf_dist_backward_input": [_F, _I, _i, _i, _i, _i, _i, _F, _S],
     "sd_inf_dist_backward_input_weight": [_F, _I, _i, _i, _i, _i, _i, _F, _F, _I, _I, _i, _i, _S],
     "sd_bound_inf_dist_forward_nograd": [_F, _F, _F, _i, _i, _i, _i, _i, _F, _F, _S],
+    "sd_bound_inf_dist_forward_shifted": [_F, _F, _F, _i, _i, _i, _i, _i, _F, _F, _F, _f, _S],
     "sd_bound_inf_dist_forward": [_F, _F, _F, _i, _i, _i, _i, _i, _F, _F, _I, _I, _S],
     "sd_bound_inf_dist_backward_input": [_F, _F, _I, _I, _i, _i, _i, _i, _i, _F, _F, _S],
     "sd_bound_inf_dist_backward_input_weight": [_F, _F, _I, _I, _i, _i, _i, _i, _i, _F, _F, _F, _S],
     "sd_sort_neuron_forward_nograd": [_F, _F, _i, _i, _i, _i, _i, _F, _f, _i, _S],
+    "sd_sort_neuron_forward_shifted": [_F, _F, _i, _i, _i, _i, _i, _F, _f, _i, _F, _f, _S],
     "sd_sort_neuron_forward": [_F, _F, _i, _i, _i, _i, _i, _F, _I, _f, _i, _S],
     "sd_sort_neuron_backward_input": [_F, _I, _i, _i, _i, _i, _i, _F, _f, _i, _S],
     "sd_sort_neuron_backward_input_weight": [_F, _I, _i, _i, _i, _i, _i, _F, _F, _f, _i, _S],
     "sd_bound_sort_neuron_forward": [_F, _F, _F, _i, _i, _i, _i, _i, _F, _F, _f, _i, _S],
+    "sd_bound_sort_neuron_forward_shifted": [_F, _F, _F, _i, _i, _i, _i, _i, _F, _F, _f, _i, _F, _f, _S],
     "sd_norm_dist_forward": [_F, _F, _i, _i, _i, _i, _i, _F, _f, _I, _I, _i, _i, _S],
     "sd_norm_dist_forward_with_max": [_F, _F, _F, _i, _i, _i, _i, _i, _F, _f, _I, _I, _i, _i, _S],
     "sd_norm_dist_backward_input": [_F, _F, _F, _F, _i, _i, _i, _i, _i, _F, _f, _I, _I, _i, _i, _S],

@@ -884,6 +884,11 @@ __device__ __forceinline__ float geo_sum(const float (&res)[K], float q) {
     return ans / (1.f - c);
 }
 
+// what is added to the value at output index o
+__device__ __forceinline__ float shift_at(const FwdArgs& a, size_t o) {
+    return output_shift(a.shift, a.shift_sign, (int)(o / a.HW % (uint32_t)(a.G * a.COg)));
+}
+
 template <int K>
 struct SortNograd : PolicyBase {
     static constexpr bool GATED = true;   // one of two queued for a result when FwdArgs::gate is set
@@ -901,7 +906,7 @@ struct SortNograd : PolicyBase {
                                                  const float4& w, int, int) {
         term(A, x.x, w.x); term(A, x.y, w.y); term(A, x.z, w.z); term(A, x.w, w.w);
     }
-    static __device__ __forceinline__ void store(Acc& A, const FwdArgs& a, size_t o, int split = 0) { a.y0[o] = geo_sum<K>(A.res, a.q); }
+    static __device__ __forceinline__ void store(Acc& A, const FwdArgs& a, size_t o, int split = 0) { a.y0[o] = geo_sum<K>(A.res, a.q) + shift_at(a, o); }
 };
 
 template <int K>
@@ -1013,8 +1018,9 @@ struct BoundSort : PolicyBase {
         term(A, l.x, u.x, w.x); term(A, l.y, u.y, w.y); term(A, l.z, u.z, w.z); term(A, l.w, u.w, w.w);
     }
     static __device__ __forceinline__ void store(Acc& A, const FwdArgs& a, size_t o, int split = 0) {
-        a.y0[o] = geo_sum<K>(A.lo, a.q);
-        a.y1[o] = geo_sum<K>(A.hi, a.q);
+        const float sh = shift_at(a, o);
+        a.y0[o] = geo_sum<K>(A.lo, a.q) + sh;
+        a.y1[o] = geo_sum<K>(A.hi, a.q) + sh;
     }
 };
 

@@ -436,6 +436,59 @@ Tensor channel_shift(const Tensor& z_in, const Tensor& vec_in, double sign) {
     return out;
 }
 
+// ---- evaluation pass: a layer's values or bounds with sign * shift[channel] added, outside any graph ------------------
+Tensor norm_dist_shifted(const Tensor& x, const Tensor& w, int64_t groups, const Tensor& shift_in, double sign) {
+    reverse_mode_only("norm_dist", x, w, shift_in);
+    at::AutoDispatchBelowADInplaceOrView below;
+    const c10::DeviceGuard guard(x.device());
+    Tensor y = new_out(x, w.size(0));
+    const Tensor shift = shift_in.contiguous();
+    const Dims d(x, groups, w.size(0));
+    require(sd_inf_dist_forward_shifted(floats(x, "input"), floats(w, "weight"), d.B, d.CO, d.CI, d.G, d.HW, floats(y, "output"),
+                                        floats(shift, "shift"), (float)sign, stream_of(x)), "sd_inf_dist_forward_shifted");
+    return y;
+}
+
+Tensor sort_neuron_shifted(const Tensor& x, const Tensor& w, int64_t groups, double q, int truncate, const Tensor& shift_in, double sign) {
+    reverse_mode_only("sort_neuron", x, w, shift_in);
+    at::AutoDispatchBelowADInplaceOrView below;
+    const c10::DeviceGuard guard(x.device());
+    Tensor y = new_out(x, w.size(0));
+    const Tensor shift = shift_in.contiguous();
+    const Dims d(x, groups, w.size(0));
+    require(sd_sort_neuron_forward_shifted(floats(x, "input"), floats(w, "weight"), d.B, d.CO, d.CI, d.G, d.HW, floats(y, "output"), (float)q,
+                                           truncate, floats(shift, "shift"), (float)sign, stream_of(x)), "sd_sort_neuron_forward_shifted");
+    return y;
+}
+
+std::pair<Tensor, Tensor> bound_inf_dist_shifted(const Tensor& xl, const Tensor& xu, const Tensor& w, int64_t groups, const Tensor& shift_in,
+                                                 double sign) {
+    reverse_mode_only("bound_inf_dist", xl, xu, w, shift_in);
+    at::AutoDispatchBelowADInplaceOrView below;
+    const c10::DeviceGuard guard(xl.device());
+    Tensor lo = new_out(xl, w.size(0)), up = new_out(xl, w.size(0));
+    const Tensor shift = shift_in.contiguous();
+    const Dims d(xl, groups, w.size(0));
+    require(sd_bound_inf_dist_forward_shifted(floats(xl, "inputL"), floats(xu, "inputU"), floats(w, "weight"), d.B, d.CO, d.CI, d.G, d.HW,
+                                              floats(lo, "outputL"), floats(up, "outputU"), floats(shift, "shift"), (float)sign, stream_of(xl)),
+            "sd_bound_inf_dist_forward_shifted");
+    return {lo, up};
+}
+
+std::pair<Tensor, Tensor> bound_sort_neuron_shifted(const Tensor& xl, const Tensor& xu, const Tensor& w, int64_t groups, double q, int truncate,
+                                                    const Tensor& shift_in, double sign) {
+    reverse_mode_only("bound_sort_neuron", xl, xu, w, shift_in);
+    at::AutoDispatchBelowADInplaceOrView below;
+    const c10::DeviceGuard guard(xl.device());
+    Tensor lo = new_out(xl, w.size(0)), up = new_out(xl, w.size(0));
+    const Tensor shift = shift_in.contiguous();
+    const Dims d(xl, groups, w.size(0));
+    require(sd_bound_sort_neuron_forward_shifted(floats(xl, "inputL"), floats(xu, "inputU"), floats(w, "weight"), d.B, d.CO, d.CI, d.G, d.HW,
+                                                 floats(lo, "outputL"), floats(up, "outputU"), (float)q, truncate, floats(shift, "shift"),
+                                                 (float)sign, stream_of(xl)), "sd_bound_sort_neuron_forward_shifted");
+    return {lo, up};
+}
+
 // ---- windows of a convolutional layer as columns; the gradient is the sum back into the image --------------------------
 struct UnfoldNode : Node {   // saves sizes only, which nothing changes or frees
     int B, C, H, W, KH, KW, stride, pad, dil;
@@ -493,5 +546,9 @@ PYBIND11_MODULE(_host, m) {
     m.def("mean_shift_index", &mean_shift_index, released());
     m.def("channel_shift", &channel_shift, released());
     m.def("sample_index_lists", &sample_index_lists, released());
+    m.def("norm_dist_shifted", &norm_dist_shifted, released());
+    m.def("sort_neuron_shifted", &sort_neuron_shifted, released());
+    m.def("bound_inf_dist_shifted", &bound_inf_dist_shifted, released());
+    m.def("bound_sort_neuron_shifted", &bound_sort_neuron_shifted, released());
     m.def("unfold", &unfold, released());
 }

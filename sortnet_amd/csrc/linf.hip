@@ -206,17 +206,23 @@ static int run_chunk_pos(FwdArgs& a, bool index_lists, hipStream_t st, void* mer
     return launch_resolve(a, st);
 }
 
-extern "C" int sd_inf_dist_forward_nograd(const float* input, const float* weight,
-                                          int B, int CO, int CI, int G, int HW, float* output, sd_stream_t stream) {
-    sd::CallGuard call_guard;   // calls of several host threads reach a stream one after the other, whole
+// shift: see FwdArgs.  Only the kernels that stream the weights add it to what they store; the others' slices meet in the output (by atomic
+// maxima, or by either of two kernels, as the device decides), so there it is added behind them, by the caller: *shifted tells which.
+static int linf_values(const float* input, const float* weight, int B, int CO, int CI, int G, int HW, float* output, const float* shift,
+                       float sign, bool* shifted, sd_stream_t stream) {
     FwdArgs a;
+    *shifted = false;
     int rc = make_fwd_args(a, "inf_dist_forward_nograd", input, nullptr, weight, B, CO, CI, G, HW, nullptr, nullptr, 0, 0);
     if (rc) return rc;
     SD_REQUIRE(output, "inf_dist_forward_nograd: null output");
     a.y0 = output;
     hipStream_t st = static_cast<hipStream_t>(stream);
     const bool streamed = g_linf_density.load(std::memory_order_relaxed) <= 0.f;   // not where tables are forced
-    if (streamed && row_stream_ok(a, kStreamMaxTerms)) return row_stream_linf(a, st);
+    if (streamed && row_stream_ok(a, kStreamMaxTerms)) {
+        a.shift = shift; a.shift_sign = sign;
+        *shifted = true;
+        return row_stream_linf(a, st);
+    }
     if (cols_ok(a, kColsHW, kColsTerms) && workspace_ready(cols_workspace(a), st)) {
         void* ws = workspace(cols_workspace(a), st);
         if (!ws) return SD_ERR_HIP;
@@ -240,6 +246,23 @@ extern "C" int sd_inf_dist_forward_nograd(const float* input, const float* weigh
     rc = narrow ? launch_fwd<LinfNograd, 2, 2>(a, st) : TB == 2 ? launch_fwd<LinfNograd, 2, 8>(a, st) : launch_fwd<LinfNograd, 4, 8>(a, st);
     if (rc) hint_forget(a.told);
     return rc;
+}
+
+extern "C" int sd_inf_dist_forward_nograd(const float* input, const float* weight,
+                                          int B, int CO, int CI, int G, int HW, float* output, sd_stream_t stream) {
+    sd::CallGuard call_guard;   // calls of several host threads reach a stream one after the other, whole
+    bool shifted;
+    return linf_values(input, weight, B, CO, CI, G, HW, output, nullptr, 0.f, &shifted, stream);
+}
+
+extern "C" int sd_inf_dist_forward_shifted(const float* input, const float* weight, int B, int CO, int CI, int G, int HW, float* output,
+                                           const float* shift, float sign, sd_stream_t stream) {
+    sd::CallGuard call_guard;   // calls of several host threads reach a stream one after the other, whole
+    SD_REQUIRE(shift && (sign == 1.f || sign == -1.f), "inf_dist_forward_shifted: null shift, or a sign (%g) other than 1 and -1", (double)sign);
+    SD_REQUIRE(aligned16(shift) && aligned16(output), "inf_dist_forward_shifted: shift and output must be 16-byte aligned");
+    bool shifted;
+    const int rc = linf_values(input, weight, B, CO, CI, G, HW, output, shift, sign, &shifted, stream);
+    return rc || shifted ? rc : channel_shift(output, shift, B, CO, HW, sign, output, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int sd_inf_dist_forward(const float* input, const float* weight,
@@ -511,11 +534,11 @@ static int bound_pad_copy(FwdArgs& a, const FwdArgs& raw, char* mem, hipStream_t
     return rc;
 }
 
-extern "C" int sd_bound_inf_dist_forward_nograd(const float* inputL, const float* inputU, const float* weight,
-                                                int B, int CO, int CI, int G, int HW, float* outputL, float* outputU,
-                                                sd_stream_t stream) {
-    sd::CallGuard call_guard;   // calls of several host threads reach a stream one after the other, whole
+// shift, *shifted: see linf_values
+static int bound_values(const float* inputL, const float* inputU, const float* weight, int B, int CO, int CI, int G, int HW, float* outputL,
+                        float* outputU, const float* shift, float sign, bool* shifted, sd_stream_t stream) {
     FwdArgs a;
+    *shifted = false;
     SD_REQUIRE(inputU, "bound_inf_dist_forward_nograd: null upper input");
     int rc = make_fwd_args(a, "bound_inf_dist_forward_nograd", inputL, inputU, weight, B, CO, CI, G, HW,
                            nullptr, nullptr, 0, 0);
@@ -523,7 +546,11 @@ extern "C" int sd_bound_inf_dist_forward_nograd(const float* inputL, const float
     SD_REQUIRE(outputL && outputU, "bound_inf_dist_forward_nograd: null output");
     a.y0 = outputL; a.y1 = outputU;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (g_bound_density.load(std::memory_order_relaxed) <= 0.f && row_stream_ok(a, kStreamBoundTerms)) return row_stream_bound(a, st);
+    if (g_bound_density.load(std::memory_order_relaxed) <= 0.f && row_stream_ok(a, kStreamBoundTerms)) {
+        a.shift = shift; a.shift_sign = sign;
+        *shifted = true;
+        return row_stream_bound(a, st);
+    }
     // dense single-group layers: a kernel that works from per-weight-row candidate tables is queued in front of the
     // one that evaluates every term, and a count taken on the device decides which of the two runs
     const float bound_density = g_bound_density.load(std::memory_order_relaxed);
@@ -593,6 +620,26 @@ extern "C" int sd_bound_inf_dist_forward_nograd(const float* inputL, const float
     if (narrow) return launch_fwd<BoundNograd, 2, 2>(a, st);
     if (TB == 2) return launch_fwd<BoundNograd, 2, 8>(a, st);
     return launch_fwd<BoundNograd, 4, 8>(a, st);
+}
+
+extern "C" int sd_bound_inf_dist_forward_nograd(const float* inputL, const float* inputU, const float* weight,
+                                                int B, int CO, int CI, int G, int HW, float* outputL, float* outputU,
+                                                sd_stream_t stream) {
+    sd::CallGuard call_guard;   // calls of several host threads reach a stream one after the other, whole
+    bool shifted;
+    return bound_values(inputL, inputU, weight, B, CO, CI, G, HW, outputL, outputU, nullptr, 0.f, &shifted, stream);
+}
+
+extern "C" int sd_bound_inf_dist_forward_shifted(const float* inputL, const float* inputU, const float* weight,
+                                                 int B, int CO, int CI, int G, int HW, float* outputL, float* outputU,
+                                                 const float* shift, float sign, sd_stream_t stream) {
+    sd::CallGuard call_guard;   // calls of several host threads reach a stream one after the other, whole
+    SD_REQUIRE(shift && (sign == 1.f || sign == -1.f), "bound_inf_dist_forward_shifted: null shift, or a sign (%g) other than 1 and -1",
+               (double)sign);
+    SD_REQUIRE(aligned16(shift) && aligned16(outputL) && aligned16(outputU), "bound_inf_dist_forward_shifted: shift and outputs must be 16-byte aligned");
+    bool shifted;
+    const int rc = bound_values(inputL, inputU, weight, B, CO, CI, G, HW, outputL, outputU, shift, sign, &shifted, stream);
+    return rc || shifted ? rc : channel_shift_both(outputL, outputU, shift, B, CO, HW, sign, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int sd_set_bound_candidate_density(float density) {

@@ -57,9 +57,10 @@ __global__ void __launch_bounds__(1024) channel_mean_kernel(const float* __restr
     }
 }
 
-__global__ void __launch_bounds__(256) channel_shift_kernel(const float* __restrict__ x, const float* __restrict__ shift,
+__global__ void __launch_bounds__(256) channel_shift_kernel(const float* x, const float* __restrict__ shift,
                                                             long long total, int C, int HW, float sign,
-                                                            float* __restrict__ y) {
+                                                            float* y, float* both) {   // (y may be x; grid.y = 2: `both` in place, too)
+    if (blockIdx.y) x = y = both;
     long long i = ((long long)blockIdx.x * 256 + threadIdx.x) * 4;
     if (i >= total) return;
     if (HW == 1 && C % 4 == 0 && i + 3 < total) {
@@ -223,6 +224,18 @@ __global__ void __launch_bounds__(64 * kFuseWaves) index_mean_shift_kernel(
     }
 }
 
+int channel_shift(const float* x, const float* shift, int B, int C, int HW, float sign, float* y, hipStream_t stream) {
+    const long long total = (long long)B * C * HW;
+    hipLaunchKernelGGL(channel_shift_kernel, dim3((unsigned)((total / 4 + 255) / 256 + 1)), dim3(256), 0, stream, x, shift, total, C, HW, sign, y, nullptr);
+    return check_launch("channel_shift_kernel");
+}
+
+int channel_shift_both(float* a, float* b, const float* shift, int B, int C, int HW, float sign, hipStream_t stream) {
+    const long long total = (long long)B * C * HW;
+    hipLaunchKernelGGL(channel_shift_kernel, dim3((unsigned)((total / 4 + 255) / 256 + 1), 2), dim3(256), 0, stream, a, shift, total, C, HW, sign, a, b);
+    return check_launch("channel_shift_kernel");
+}
+
 static int check_dims(const char* who, int B, int C, int HW) {
     SD_REQUIRE(B > 0 && C > 0 && HW > 0, "%s: sizes must be positive", who);
     SD_REQUIRE((long long)B * C * HW < (1ll << 31), "%s: tensor too large for 32-bit indexing", who);
@@ -245,10 +258,7 @@ extern "C" int sd_mean_shift_forward(const float* input, int B, int C, int HW, f
     dim3 grid(HW == 1 ? (C + 63) / 64 : C);
     hipLaunchKernelGGL(channel_mean_kernel, grid, dim3(1024), 0, st, input, B, C, HW, mean, running_mean, momentum);
     if ((rc = check_launch("channel_mean_kernel"))) return rc;
-    long long total = (long long)B * C * HW;
-    hipLaunchKernelGGL(channel_shift_kernel, dim3((unsigned)((total / 4 + 255) / 256 + 1)), dim3(256), 0, st,
-                       input, mean, total, C, HW, -1.f, output);
-    return check_launch("channel_shift_kernel");
+    return channel_shift(input, mean, B, C, HW, -1.f, output, st);
 }
 
 extern "C" int sd_channel_shift(const float* input, const float* shift, int B, int C, int HW, float sign,
@@ -259,10 +269,7 @@ extern "C" int sd_channel_shift(const float* input, const float* shift, int B, i
     SD_REQUIRE(input && shift && output, "channel_shift: null pointer");
     SD_REQUIRE(reinterpret_cast<uintptr_t>(input) % 16 == 0 && reinterpret_cast<uintptr_t>(output) % 16 == 0 &&
                reinterpret_cast<uintptr_t>(shift) % 16 == 0, "channel_shift: buffers must be 16-byte aligned");
-    long long total = (long long)B * C * HW;
-    hipLaunchKernelGGL(channel_shift_kernel, dim3((unsigned)((total / 4 + 255) / 256 + 1)), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), input, shift, total, C, HW, sign, output);
-    return check_launch("channel_shift_kernel");
+    return channel_shift(input, shift, B, C, HW, sign, output, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int sd_mean_shift_index_forward(const float* input, const int* index, int B, int G, int cnt, int Cg, int HW,

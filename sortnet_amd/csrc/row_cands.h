@@ -49,10 +49,12 @@ bool row_cands_supported(int form, int K);
 //   xkeep / wkeep (kRowsMax only, both or neither): keep bits of the factored mask, one word per (row, 32 inputs).
 //   outL / outU / pos as in sort_cols_forward / max_cols_forward (values go to outU; kRowsBound: pos of the upper, pos_lower
 //     of the lower bound, both or neither: core/cuda/bound_inf_dist_cuda.cu:176-212).
+//   shift, shift_sign: see FwdArgs (kRowsSortValues and kRowsSortInterval).
 int row_cands_forward(int form, const float* xl, const float* xu, const float* w, const uint32_t* xkeep,
                       const uint32_t* wkeep, int B, int CO, int CI, float q, int K, float* outL, float* outU, int* pos,
                       void* ws, float density, bool forced, const float* col_stat, const unsigned long long* col_count,
-                      const unsigned long long** every, hipStream_t st, int* pos_lower = nullptr);
+                      const unsigned long long** every, hipStream_t st, int* pos_lower = nullptr,
+                      const float* shift = nullptr, float shift_sign = 0.f);
 
 // the word that is 1 after a call whose tables per batch row did not serve, from its `every`
 const unsigned long long* row_cands_idle(const unsigned long long* every);

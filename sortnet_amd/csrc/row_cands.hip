@@ -177,6 +177,8 @@ struct RtArgs {
     int B, Bp, M, N;
     float q;
     float* outL; float* outU; int* pos; int* posL;
+    const float* shift;   // kRowsSortValues, kRowsSortInterval: see FwdArgs
+    float shift_sign;
 };
 
 template <int FORM, int K, bool POS, bool MASKED>
@@ -336,8 +338,11 @@ __global__ void __launch_bounds__(64 * kRtWaves) rt_main_kernel(RtArgs a) {
             const size_t o = (size_t)b * M + col;
             if constexpr (LISTS) {
                 if constexpr (FORM == kRowsSortPos) a.outU[o] = geo_sum<K>(hi[j], a.q);
-                else a.outU[o] = geo_sum_bits<K>(hi[j], a.q);
-                if constexpr (IV) a.outL[o] = geo_sum_bits<K>(lo[j], a.q);
+                else {
+                    const float add = output_shift(a.shift, a.shift_sign, col);
+                    a.outU[o] = geo_sum_bits<K>(hi[j], a.q) + add;
+                    if constexpr (IV) a.outL[o] = geo_sum_bits<K>(lo[j], a.q) + add;
+                }
                 if constexpr (FORM == kRowsSortPos) {
                     #pragma unroll
                     for (int k = 0; k < K; k++) a.pos[(size_t)(K - 1 - k) * plane + o] = idx[j][k];   // plane 0 = largest
@@ -449,11 +454,12 @@ int run_tables(const float* xl, const float* xu, const float* w, const uint32_t*
 
 template <int FORM, int K>
 int run(const float* xl, const float* xu, const float* w, int B, int M, int N, float q, float* outL, float* outU, int* pos,
-        const Carve& c, unsigned long long limit, const float* col_stat, const unsigned long long* col_count, hipStream_t st) {
+        const Carve& c, unsigned long long limit, const float* col_stat, const unsigned long long* col_count, const float* shift,
+        float shift_sign, hipStream_t st) {
     constexpr bool IV = FORM == kRowsSortInterval;
     const int rc = run_tables<IV, false, false>(xl, xu, w, nullptr, nullptr, B, M, N, K, c, limit, col_stat, col_count, kProbeRatio, st);
     if (rc) return rc;
-    RtArgs a{xl, xu, c.wt, c.wr, c.bits, c.low, c.count, c.fix, B, bpad_of(B), M, N, q, outL, outU, pos, nullptr};
+    RtArgs a{xl, xu, c.wt, c.wr, c.bits, c.low, c.count, c.fix, B, bpad_of(B), M, N, q, outL, outU, pos, nullptr, shift, shift_sign};
     return launch_rt<FORM, K, false, false>(a, st);
 }
 
@@ -463,7 +469,7 @@ int run_max(const float* x, const float* w, const uint32_t* xkeep, const uint32_
             float ratio, hipStream_t st) {
     int rc = run_tables<false, false, MASKED>(x, nullptr, w, xkeep, wkeep, B, M, N, K, c, limit, col_stat, col_count, ratio, st);
     if (rc) return rc;
-    RtArgs a{x, nullptr, c.wt, c.wr, c.bits, c.low, c.count, c.fix, B, bpad_of(B), M, N, 0.f, nullptr, y, pos, nullptr};
+    RtArgs a{x, nullptr, c.wt, c.wr, c.bits, c.low, c.count, c.fix, B, bpad_of(B), M, N, 0.f, nullptr, y, pos, nullptr, nullptr, 0.f};
     if (pos) rc = launch_rt<kRowsMax, 1, true, MASKED>(a, st);
     else rc = launch_rt<kRowsMax, 1, false, MASKED>(a, st);
     if (rc || !MASKED) return rc;
@@ -477,7 +483,7 @@ int run_bound(const float* xl, const float* xu, const float* w, int B, int M, in
               const Carve& c, unsigned long long limit, const float* col_stat, const unsigned long long* col_count, hipStream_t st) {
     const int rc = run_tables<true, true, false>(xl, xu, w, nullptr, nullptr, B, M, N, 1, c, limit, col_stat, col_count, kProbeRatio, st);
     if (rc) return rc;
-    RtArgs a{xl, xu, c.wt, c.wr, c.bits, c.low, c.count, c.fix, B, bpad_of(B), M, N, 0.f, outL, outU, posU, posL};
+    RtArgs a{xl, xu, c.wt, c.wr, c.bits, c.low, c.count, c.fix, B, bpad_of(B), M, N, 0.f, outL, outU, posU, posL, nullptr, 0.f};
     return posU ? launch_rt<kRowsBound, 1, true, false>(a, st) : launch_rt<kRowsBound, 1, false, false>(a, st);
 }
 
@@ -510,7 +516,7 @@ const unsigned long long* row_cands_idle(const unsigned long long* every) {
 int row_cands_forward(int form, const float* xl, const float* xu, const float* w, const uint32_t* xkeep,
                       const uint32_t* wkeep, int B, int CO, int CI, float q, int K, float* outL, float* outU, int* pos,
                       void* ws, float density, bool forced, const float* col_stat, const unsigned long long* col_count,
-                      const unsigned long long** every, hipStream_t st, int* pos_lower) {
+                      const unsigned long long** every, hipStream_t st, int* pos_lower, const float* shift, float shift_sign) {
     const float ratio_max = forced ? kProbeRatio : kProbeRatioMax;
     if (CI % kChunk != 0 || B < 1 || CO < 1 || !row_cands_supported(form, K) || (xkeep == nullptr) != (wkeep == nullptr) ||
         (long long)B * CO >= (1ll << 32)) {
@@ -528,21 +534,21 @@ int row_cands_forward(int form, const float* xl, const float* xu, const float* w
     switch (form) {
         case kRowsSortValues:
             switch (K) {
-#define X(k) case k: return run<kRowsSortValues, k>(xl, nullptr, w, B, CO, CI, q, outL, outU, nullptr, c, limit, col_stat, col_count, st);
+#define X(k) case k: return run<kRowsSortValues, k>(xl, nullptr, w, B, CO, CI, q, outL, outU, nullptr, c, limit, col_stat, col_count, shift, shift_sign, st);
                 SD_ROWS_K25(X)
 #undef X
             }
             break;
         case kRowsSortInterval:
             switch (K) {
-#define X(k) case k: return run<kRowsSortInterval, k>(xl, xu, w, B, CO, CI, q, outL, outU, nullptr, c, limit, col_stat, col_count, st);
+#define X(k) case k: return run<kRowsSortInterval, k>(xl, xu, w, B, CO, CI, q, outL, outU, nullptr, c, limit, col_stat, col_count, shift, shift_sign, st);
                 SD_ROWS_K25(X)
 #undef X
             }
             break;
         case kRowsSortPos:
             switch (K) {
-#define X(k) case k: return run<kRowsSortPos, k>(xl, nullptr, w, B, CO, CI, q, outL, outU, pos, c, limit, col_stat, col_count, st);
+#define X(k) case k: return run<kRowsSortPos, k>(xl, nullptr, w, B, CO, CI, q, outL, outU, pos, c, limit, col_stat, col_count, shift, shift_sign, st);
                 SD_ROWS_K25(X)
 #undef X
             }

@@ -152,6 +152,7 @@ row_stream_kernel(FwdArgs a, int K) {
         }
     };
 
+    const float sh = output_shift(a.shift, a.shift_sign, c);
     float coef = 1.f, rest = 1.f;                      // weight of the lane's term, what is left behind the K-th
     if (OP == kStreamSort) {
         for (int k = 0; k < K; k++) { coef = lane == k ? rest : coef; rest *= 1.f - a.q; }
@@ -206,7 +207,7 @@ row_stream_kernel(FwdArgs a, int K) {
             #pragma unroll
             for (int k = 0; k < NX; k++) {
                 top[k] = wave_max(top[k]);
-                if (mine && lane == 0) (k ? a.y1 : a.y0)[o] = fmaxf(top[k], kEps);
+                if (mine && lane == 0) (k ? a.y1 : a.y0)[o] = fmaxf(top[k], kEps) + sh;
             }
             continue;
         }
@@ -383,7 +384,7 @@ row_stream_kernel(FwdArgs a, int K) {
             const int weighed = __float_as_int(sorted * coef * a.q);
             float ans = kEps;
             for (int k = 0; k < K; k++) ans += __int_as_float(__builtin_amdgcn_readlane(weighed, k));
-            if (mine && lane == 0) (side ? a.y1 : a.y0)[o] = ans / (1.f - rest);
+            if (mine && lane == 0) (side ? a.y1 : a.y0)[o] = ans / (1.f - rest) + sh;
         }
     }
 }

@@ -43,6 +43,7 @@ __global__ void __launch_bounds__(256) sort_rows_kernel(FwdArgs a, const int* __
     __syncthreads();
     const size_t size = (size_t)a.B * a.G * a.COg;
     const int nchunks = (a.CIg + KT - 1) / KT;
+    const float sh = VALUES ? output_shift(a.shift, a.shift_sign, c) : 0.f;
     for (int b = threadIdx.x; b < a.B; b += 256) {
         const size_t o = (size_t)b * a.G * a.COg + c;
         const float* xr = a.x0 + (size_t)(b * a.G + g) * a.CIg;
@@ -99,7 +100,7 @@ __global__ void __launch_bounds__(256) sort_rows_kernel(FwdArgs a, const int* __
                 if (ids[k] < nchunks) chunk(ids[k]);
             }
         }
-        a.y0[o] = geo_sum<K>(res, a.q);
+        a.y0[o] = geo_sum<K>(res, a.q) + sh;
         if (!VALUES) {
             #pragma unroll
             for (int k = K - 1; k >= 0; k--) a.p0[(size_t)(K - 1 - k) * size + o] = idx[k];
@@ -210,7 +211,7 @@ static int queue_sort_cols(FwdArgs& a, int site, const float* layer, int form, c
                            float q, int K, float* outL, float* outU, int* pos, void* ws, hipStream_t st) {
     const float density = g_sort_density.load(std::memory_order_relaxed);
     const float cap = density > 0.f ? density : sort_cols_cap(form, CI);
-    int rc = sort_cols_forward(xl, xu, w, B, CO, CI, q, K, outL, outU, pos, ws, cap, &a.gate, &a.gate_limit, st);
+    int rc = sort_cols_forward(xl, xu, w, B, CO, CI, q, K, outL, outU, pos, ws, cap, &a.gate, &a.gate_limit, st, a.shift, a.shift_sign);
     a.gate_above = 1;
     const long long terms = (long long)B * CO * CI;
     const bool rows = row_cands_supported(form, K) && (density > 0.f || terms >= kSortRowsMinTerms) &&
@@ -224,7 +225,7 @@ static int queue_sort_cols(FwdArgs& a, int site, const float* layer, int form, c
     char* rows_ws = static_cast<char*>(ws) + (sort_cols_workspace(B, CO, CI) + 255) / 256 * 256;
     const unsigned long long* every = nullptr;
     rc = row_cands_forward(form, xl, xu, w, nullptr, nullptr, B, CO, CI, q, K, outL, outU, pos, rows_ws,
-                           density > 0.f ? density : sort_rows_cap(form), density > 0.f, sort_cols_probe_sums(col_count), col_count, &every, st);
+                           density > 0.f ? density : sort_rows_cap(form), density > 0.f, sort_cols_probe_sums(col_count), col_count, &every, st, nullptr, a.shift, a.shift_sign);
     if (rc) return rc;
     a.gate = every;
     a.gate_limit = 0ull;
@@ -288,16 +289,14 @@ static bool few_tiles(const FwdArgs& a, int BB, int BM) {
     return tiles < 2ll * num_cus();
 }
 
-extern "C" int sd_sort_neuron_forward_nograd(const float* input, const float* weight,
-                                             int B, int CO, int CI, int G, int HW, float* output, float q, int K,
-                                             sd_stream_t stream) {
-    sd::CallGuard call_guard;   // calls of several host threads reach a stream one after the other, whole
+static int sort_values(const float* input, const float* weight, int B, int CO, int CI, int G, int HW, float* output, float q, int K,
+                       const float* shift, float sign, sd_stream_t stream) {
     FwdArgs a;
     int rc = make_fwd_args(a, "sort_neuron_forward_nograd", input, nullptr, weight, B, CO, CI, G, HW, nullptr, nullptr, 0, 0);
     if (rc) return rc;
     if ((rc = check_qk("sort_neuron_forward_nograd", q, K, a.CIg))) return rc;
     SD_REQUIRE(output, "sort_neuron_forward_nograd: null output");
-    a.y0 = output; a.q = q;
+    a.y0 = output; a.q = q; a.shift = shift; a.shift_sign = sign;
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (g_sort_density.load(std::memory_order_relaxed) <= 0.f && row_stream_sort_ok(a))
         return row_stream_sort(a, K, st);
@@ -333,6 +332,21 @@ extern "C" int sd_sort_neuron_forward_nograd(const float* input, const float* we
     }
     if (rc) { hint_forget(a.told); hint_forget(a.told2); }
     return rc;
+}
+
+extern "C" int sd_sort_neuron_forward_nograd(const float* input, const float* weight,
+                                             int B, int CO, int CI, int G, int HW, float* output, float q, int K,
+                                             sd_stream_t stream) {
+    sd::CallGuard call_guard;   // calls of several host threads reach a stream one after the other, whole
+    return sort_values(input, weight, B, CO, CI, G, HW, output, q, K, nullptr, 0.f, stream);
+}
+
+extern "C" int sd_sort_neuron_forward_shifted(const float* input, const float* weight,
+                                              int B, int CO, int CI, int G, int HW, float* output, float q, int K,
+                                              const float* shift, float sign, sd_stream_t stream) {
+    sd::CallGuard call_guard;   // calls of several host threads reach a stream one after the other, whole
+    SD_REQUIRE(shift && (sign == 1.f || sign == -1.f), "sort_neuron_forward_shifted: null shift, or a sign (%g) other than 1 and -1", (double)sign);
+    return sort_values(input, weight, B, CO, CI, G, HW, output, q, K, shift, sign, stream);
 }
 
 extern "C" int sd_sort_neuron_forward(const float* input, const float* weight,
@@ -383,17 +397,15 @@ extern "C" int sd_sort_neuron_forward(const float* input, const float* weight,
     return rc;
 }
 
-extern "C" int sd_bound_sort_neuron_forward(const float* inputL, const float* inputU, const float* weight,
-                                            int B, int CO, int CI, int G, int HW, float* outputL, float* outputU,
-                                            float q, int K, sd_stream_t stream) {
-    sd::CallGuard call_guard;   // calls of several host threads reach a stream one after the other, whole
+static int sort_bounds(const float* inputL, const float* inputU, const float* weight, int B, int CO, int CI, int G, int HW, float* outputL,
+                       float* outputU, float q, int K, const float* shift, float sign, sd_stream_t stream) {
     FwdArgs a;
     SD_REQUIRE(inputU, "bound_sort_neuron_forward: null upper input");
     int rc = make_fwd_args(a, "bound_sort_neuron_forward", inputL, inputU, weight, B, CO, CI, G, HW, nullptr, nullptr, 0, 0);
     if (rc) return rc;
     if ((rc = check_qk("bound_sort_neuron_forward", q, K, a.CIg))) return rc;
     SD_REQUIRE(outputL && outputU, "bound_sort_neuron_forward: null output");
-    a.y0 = outputL; a.y1 = outputU; a.q = q;
+    a.y0 = outputL; a.y1 = outputU; a.q = q; a.shift = shift; a.shift_sign = sign;
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (g_sort_density.load(std::memory_order_relaxed) <= 0.f && row_stream_sort_ok(a))
         return row_stream_sort(a, K, st);
@@ -421,4 +433,20 @@ extern "C" int sd_bound_sort_neuron_forward(const float* inputL, const float* in
     }
     if (rc) { hint_forget(a.told); hint_forget(a.told2); }
     return rc;
+}
+
+extern "C" int sd_bound_sort_neuron_forward(const float* inputL, const float* inputU, const float* weight,
+                                            int B, int CO, int CI, int G, int HW, float* outputL, float* outputU,
+                                            float q, int K, sd_stream_t stream) {
+    sd::CallGuard call_guard;   // calls of several host threads reach a stream one after the other, whole
+    return sort_bounds(inputL, inputU, weight, B, CO, CI, G, HW, outputL, outputU, q, K, nullptr, 0.f, stream);
+}
+
+extern "C" int sd_bound_sort_neuron_forward_shifted(const float* inputL, const float* inputU, const float* weight,
+                                                    int B, int CO, int CI, int G, int HW, float* outputL, float* outputU,
+                                                    float q, int K, const float* shift, float sign, sd_stream_t stream) {
+    sd::CallGuard call_guard;   // calls of several host threads reach a stream one after the other, whole
+    SD_REQUIRE(shift && (sign == 1.f || sign == -1.f), "bound_sort_neuron_forward_shifted: null shift, or a sign (%g) other than 1 and -1",
+               (double)sign);
+    return sort_bounds(inputL, inputU, weight, B, CO, CI, G, HW, outputL, outputU, q, K, shift, sign, stream);
 }

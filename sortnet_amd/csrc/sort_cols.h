@@ -26,9 +26,10 @@ size_t sort_cols_workspace(int B, int CO, int CI);
 //   l-inf distance (maxima with the 1e-10 floor, q unused), for layers whose marks are too few to stage tiles for;
 //   xu == nullptr: value form on xl, outU receives the values (outL is not used) and pos, if not null, the K planes
 //   of positions (K, B, CO), largest first.
+//   shift, shift_sign: see FwdArgs (forms without positions).
 int sort_cols_forward(const float* xl, const float* xu, const float* w, int B, int CO, int CI, float q, int K,
                       float* outL, float* outU, int* pos, void* ws, float density, const unsigned long long** gate,
-                      unsigned long long* gate_limit, hipStream_t st);
+                      unsigned long long* gate_limit, hipStream_t st, const float* shift = nullptr, float shift_sign = 0.f);
 
 // The two sums of the probe that sort_cols_forward / max_cols_forward leave behind the counter words *gate points at
 // (widths of the input columns over all batch tiles; widths of the same columns over 16 weight rows), for the tables

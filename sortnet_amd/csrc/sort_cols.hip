@@ -266,7 +266,7 @@ __global__ void __launch_bounds__(64 * kMainWaves)
 sc_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const uint32_t* __restrict__ bits,
                const float* __restrict__ xr, const float* __restrict__ low, const unsigned long long* __restrict__ count,
                unsigned long long limit, int B, int Bp, int M, int Mp, int N, float q, float* __restrict__ yL,
-               float* __restrict__ yU) {
+               float* __restrict__ yU, const float* __restrict__ shift, float shift_sign) {
     if (gate_closed(count, limit, 0)) return;
     static_assert(!MAXFORM || (K == 1 && IV), "the maximum form is the interval form with one entry");
     union Shared {
@@ -358,8 +358,9 @@ sc_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const 
         const int bl = e / kMainTile, mloc = e % kMainTile;
         const int b = s * kTileB + bl, mm = mb * kMainTile + mloc;
         if (b < B && mm < M) {
-            yU[(size_t)b * M + mm] = sh.stage[0][bl][mloc];
-            if constexpr (IV) yL[(size_t)b * M + mm] = sh.stage[1][bl][mloc];
+            const float add = output_shift(shift, shift_sign, mm);
+            yU[(size_t)b * M + mm] = sh.stage[0][bl][mloc] + add;
+            if constexpr (IV) yL[(size_t)b * M + mm] = sh.stage[1][bl][mloc] + add;
         }
     }
 }
@@ -619,7 +620,7 @@ sp_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const 
 
 template <int K, bool IV, bool MAXFORM = false>
 int run(const float* xl, const float* xu, const float* w, int B, int M, int N, float q, float* outL, float* outU,
-        int* pos, const Carve& c, unsigned long long limit, hipStream_t st) {
+        int* pos, const Carve& c, unsigned long long limit, const float* shift, float shift_sign, hipStream_t st) {
     const int S = tiles_b(B), Bp = S * kTileB, Mp = mpad_of(M);
     int rc;
     hipLaunchKernelGGL((sc_range_kernel<IV, MAXFORM, false>), dim3(N / kChunk, S), dim3(256), 0, st, xl, xu, w, nullptr, B, M, N, Bp, c.xr, c.xT, c.widths, c.count);
@@ -633,7 +634,7 @@ int run(const float* xl, const float* xu, const float* w, int B, int M, int N, f
         }
     }
     hipLaunchKernelGGL((sc_main_kernel<K, IV, MAXFORM>), dim3((unsigned)(S * (Mp / kMainTile))), dim3(64 * kMainWaves), 0, st,
-                       c.xT, w, c.bits, c.xr, c.low, &c.count->marks, limit, B, Bp, M, Mp, N, q, outL, outU);
+                       c.xT, w, c.bits, c.xr, c.low, &c.count->marks, limit, B, Bp, M, Mp, N, q, outL, outU, shift, shift_sign);
     return check_launch("sc_main_kernel");
 }
 
@@ -650,7 +651,7 @@ size_t sort_cols_workspace(int B, int CO, int CI) {
 
 int sort_cols_forward(const float* xl, const float* xu, const float* w, int B, int CO, int CI, float q, int K,
                       float* outL, float* outU, int* pos, void* ws, float density, const unsigned long long** gate,
-                      unsigned long long* gate_limit, hipStream_t st) {
+                      unsigned long long* gate_limit, hipStream_t st, const float* shift, float shift_sign) {
     if (CI % kChunk != 0 || CI > 65536 || B < 1 || CO < 1) {
         set_error("sort_cols_forward: shape not supported");
         return SD_ERR_ARG;
@@ -661,10 +662,10 @@ int sort_cols_forward(const float* xl, const float* xu, const float* w, int B, i
     *gate = &c.count->marks;
     *gate_limit = limit;
     note_term_counts(&c.count->marks, 1, (double)tiles_b(B) * CO * CI, 1.0);
-    if (K == 1 && xu) return run<1, true, true>(xl, xu, w, B, CO, CI, q, outL, outU, nullptr, c, limit, st);
+    if (K == 1 && xu) return run<1, true, true>(xl, xu, w, B, CO, CI, q, outL, outU, nullptr, c, limit, shift, shift_sign, st);
     switch (K) {
-#define X(k) case k: return xu ? run<k, true>(xl, xu, w, B, CO, CI, q, outL, outU, nullptr, c, limit, st) \
-                               : run<k, false>(xl, nullptr, w, B, CO, CI, q, outL, outU, pos, c, limit, st);
+#define X(k) case k: return xu ? run<k, true>(xl, xu, w, B, CO, CI, q, outL, outU, nullptr, c, limit, shift, shift_sign, st) \
+                               : run<k, false>(xl, nullptr, w, B, CO, CI, q, outL, outU, pos, c, limit, shift, shift_sign, st);
         SD_SORT_COLS_K(X)
 #undef X
     }

@@ -241,6 +241,31 @@ def bound_inf_dist(x_lower, x_upper, weight, groups=1, use_custom_cuda_func=True
     return BoundInfDistF.apply(x_lower, x_upper, weight, groups)
 
 
+# ---- evaluation pass: the values or bounds of a layer with sign * shift[channel] added, in one native call -----------------
+# The same bits as the op above with the shift behind it; outside any graph.
+def _kernels_can_add(vec, weight):
+    """Whether the kernels take `vec` as it is (a call that torch would convert, broadcast or refuse is left to torch)."""
+    return (vec.dtype == torch.float32 and vec.dim() == 1 and vec.size(0) == weight.size(0) and vec.device == weight.device
+            and vec.is_contiguous() and vec.data_ptr() % 16 == 0)
+
+
+def _shifted_values(x, weight, groups, q, shift, sign, truncate=10):
+    truncate = min(weight.size(-1), truncate)
+    host = _checked(x, weight, groups)
+    if q is None or q == 1.0 or truncate == 1:
+        return host.norm_dist_shifted(x, weight, groups, shift, sign)
+    return host.sort_neuron_shifted(x, weight, groups, q, truncate, shift, sign)
+
+
+def _shifted_bounds(x_lower, x_upper, weight, groups, q, shift, sign, truncate=10):
+    truncate = min(weight.size(-1), truncate)
+    assert x_lower.size() == x_upper.size()
+    host = _checked(x_lower, weight, groups)
+    if q is None or q == 1.0 or truncate == 1:
+        return host.bound_inf_dist_shifted(x_lower, x_upper, weight, groups, shift, sign)
+    return host.bound_sort_neuron_shifted(x_lower, x_upper, weight, groups, q, truncate, shift, sign)
+
+
 def masked_inf_dist(input, weight, q, seed, groups=1, mode=_C.MASK_TERM, tag=None):
     """Masked order-statistic neuron (see MaskedInfDistF).  `mode` is ext.MASK_TERM (independent
     draw per term) or ext.MASK_FACTORED (keep = keep_x(b, n) & keep_w(m, n))."""

@@ -21,6 +21,7 @@ from collections.abc import Iterable
 
 import torch
 import torch.nn as nn
+from torch.nn.modules.module import _has_any_global_hook
 
 from . import ext
 from . import functional as F
@@ -171,7 +172,7 @@ class NormDistBase(nn.Module):
 
     def forward(self, x=None, lower=None, upper=None):
         reg = self.registry
-        index_out, bias = None, self.bias
+        index_out, bias, shifted = None, self.bias, None
         if reg.entries:
             assert x is not None
             grad = torch.is_grad_enabled() and (x.requires_grad or self.weight.requires_grad)
@@ -179,20 +180,51 @@ class NormDistBase(nn.Module):
             if grad and self.training:
                 x, index_out, bias = self._forward_index_lists(x)
             else:
-                x = F.sort_neuron(x, self.weight, self.groups, q=self.dropout, tag=self.tag)
-                if lower is not None and upper is not None:
-                    lower, upper = F.bound_sort_neuron(lower, upper, self.weight, self.groups, q=self.dropout,
-                                                       tag=self.tag)
+                shifted = self._evaluation_shift(x, lower, upper)
+                if shifted is None:
+                    x = F.sort_neuron(x, self.weight, self.groups, q=self.dropout, tag=self.tag)
+                    if lower is not None and upper is not None:
+                        lower, upper = F.bound_sort_neuron(lower, upper, self.weight, self.groups, q=self.dropout,
+                                                           tag=self.tag)
+                else:
+                    x, lower, upper = self._forward_shifted(x, lower, upper, self.dropout, *shifted)
         else:
-            if x is not None:
+            shifted = self._evaluation_shift(x, lower, upper) if math.isinf(self.p) else None
+            if shifted is not None:
+                x, lower, upper = self._forward_shifted(x, lower, upper, None, *shifted)
+            elif x is not None:
                 x = F.norm_dist(x, self.weight, self.p, self.groups, tag=self.tag)
-            if lower is not None and upper is not None:
+            if shifted is None and lower is not None and upper is not None:
                 assert math.isinf(self.p)
                 lower, upper = F.bound_inf_dist(lower, upper, self.weight, self.groups, tag=self.tag)
-        if self.mean_shift is not None:
+        if self.mean_shift is not None and shifted is None:
             x, lower, upper = self.mean_shift(x, lower, upper, index=index_out)
-        if bias is not None:
+        if bias is not None and (shifted is None or self.mean_shift is not None):
             x, lower, upper = apply_if_not_none((x, lower, upper), lambda z: z + bias.unsqueeze(-1))
+        return x, lower, upper
+
+    def _evaluation_shift(self, x, lower, upper):
+        """(vector, sign) of the step that follows the distances outside a graph - the mean shift, or the bias of a layer without
+        one - where the kernels may add it to what they store: the sums are the same, and at 1 x 5120 outputs the launch that only
+        adds them is 3.7 us behind a layer of 23.  None where that step has to be seen to run: by a hook, a subclass or, for
+        operands that the kernels would refuse, an error."""
+        if torch.is_grad_enabled() or (lower is None) != (upper is None):
+            return None
+        step = self.mean_shift
+        if step is None:
+            vec, sign = self.bias, 1.0
+        elif (type(step) is MeanShiftDropout and not step.training and step.bias is None and "forward" not in step.__dict__
+              and not step._forward_hooks and not step._forward_pre_hooks and not _has_any_global_hook()):
+            vec, sign = step.running_mean, -1.0
+        else:
+            return None
+        return (vec, sign) if vec is not None and F._kernels_can_add(vec, self.weight) else None
+
+    def _forward_shifted(self, x, lower, upper, q, shift, sign):
+        if x is not None:
+            x = F._shifted_values(x, self.weight, self.groups, q, shift, sign)
+        if lower is not None:
+            lower, upper = F._shifted_bounds(lower, upper, self.weight, self.groups, q, shift, sign)
         return x, lower, upper
 
     def _forward_index_lists(self, x):

@@ -68,9 +68,11 @@ class DistanceMLP:
         the running means -- the value that `bounds()` brackets."""
         h = x.unsqueeze(-1).contiguous()
         for i, w in enumerate(self.weights):
-            h = F.norm_dist(h, w, float("inf"))
-            shift = self.running_mean[i].view(1, -1, 1) if i < self.num_layers - 1 else -self.bias.view(1, -1, 1)
-            h = h - shift
+            shift, sign = (self.running_mean[i], -1.0) if i < self.num_layers - 1 else (self.bias, 1.0)
+            if F._kernels_can_add(shift, w):
+                h = F._shifted_values(h, w, 1, None, shift, sign)
+            else:
+                h = F.norm_dist(h, w, float("inf")) + sign * shift.view(1, -1, 1)
         return h.squeeze(-1)
 
     @torch.no_grad()
@@ -83,9 +85,13 @@ class DistanceMLP:
         for i, w in enumerate(self.weights):
             if before_layer is not None:
                 before_layer(i)
-            lo, up = F.bound_inf_dist(lo, up, w)
-            shift = means[i].view(1, -1, 1) if i < self.num_layers - 1 else -self.bias.view(1, -1, 1)
-            lo, up = lo - shift, up - shift
+            shift, sign = (means[i], -1.0) if i < self.num_layers - 1 else (self.bias, 1.0)
+            if F._kernels_can_add(shift, w):
+                lo, up = F._shifted_bounds(lo, up, w, 1, None, shift, sign)
+            else:
+                lo, up = F.bound_inf_dist(lo, up, w)
+                shift = sign * shift.view(1, -1, 1)
+                lo, up = lo + shift, up + shift
         return lo.squeeze(-1), up.squeeze(-1)
 
 
