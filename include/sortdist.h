@@ -286,6 +286,13 @@ int sd_bound_sort_neuron_forward_shifted(const float* inputL, const float* input
                                          int B, int CO, int CI, int G, int HW, float* outputL, float* outputU,
                                          float q, int K, const float* shift, float sign, sd_stream_t stream);
 
+/* Values and interval bounds of one layer of an evaluation pass: sd_sort_neuron_forward_shifted on (input, output) and
+ * sd_bound_sort_neuron_forward_shifted on the others, the same bits (shift may be NULL: without it); where both work from
+ * candidate tables, from one. */
+int sd_sort_neuron_box_forward(const float* input, const float* inputL, const float* inputU, const float* weight,
+                               int B, int CO, int CI, int G, int HW, float* output, float* outputL, float* outputU,
+                               float q, int K, const float* shift, float sign, sd_stream_t stream);
+
 /* Training-mode mean shift when every 32-sample sub-batch keeps its own channel subset
  * (core/models/bound_basic_module.py:125-137,146-153, done there with torch ops).  input / output are
  * (B, G * cnt, HW), already compacted; index is (S, G, cnt), S = ceil(B / 32), ascending channel numbers below

@@ -36,6 +36,7 @@ SIGNATURES = {
     "sd_sort_neuron_backward_input_weight": [_F, _I, _i, _i, _i, _i, _i, _F, _F, _f, _i, _S],
     "sd_bound_sort_neuron_forward": [_F, _F, _F, _i, _i, _i, _i, _i, _F, _F, _f, _i, _S],
     "sd_bound_sort_neuron_forward_shifted": [_F, _F, _F, _i, _i, _i, _i, _i, _F, _F, _f, _i, _F, _f, _S],
+    "sd_sort_neuron_box_forward": [_F, _F, _F, _F, _i, _i, _i, _i, _i, _F, _F, _F, _f, _i, _F, _f, _S],
     "sd_norm_dist_forward": [_F, _F, _i, _i, _i, _i, _i, _F, _f, _I, _I, _i, _i, _S],
     "sd_norm_dist_forward_with_max": [_F, _F, _F, _i, _i, _i, _i, _i, _F, _f, _I, _I, _i, _i, _S],
     "sd_norm_dist_backward_input": [_F, _F, _F, _F, _i, _i, _i, _i, _i, _F, _f, _I, _I, _i, _i, _S],

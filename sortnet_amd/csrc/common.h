@@ -70,6 +70,8 @@ struct FwdArgs {
     unsigned long long* told;
     unsigned long long* told2;
     const unsigned long long* few;
+    unsigned long long* told3;   // the same for another word of the device
+    const unsigned long long* few3;
     // interval forward with positions: non-null and non-zero on the device when a table kernel has already stored the
     // final values and positions, so that resolve_bound_kernel has nothing to do
     const unsigned long long* resolved;
@@ -88,9 +90,10 @@ __device__ __forceinline__ bool gate_closed(const unsigned long long* gate, unsi
 __device__ __forceinline__ bool gate_closed(const FwdArgs& a) {
     if (a.gate == nullptr) return false;
     const bool closed = gate_closed(a.gate, a.gate_limit, a.gate_above);
-    if ((a.told || a.told2) && threadIdx.x == 0 && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) {
+    if ((a.told || a.told2 || a.told3) && threadIdx.x == 0 && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) {
         if (a.told) __hip_atomic_store(a.told, closed ? 0ull : 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         if (a.told2) __hip_atomic_store(a.told2, *a.few != 0ull ? 1ull : 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (a.told3) __hip_atomic_store(a.told3, *a.few3 != 0ull ? 1ull : 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
     return closed;
 }
@@ -127,6 +130,9 @@ void* workspace(size_t bytes, hipStream_t stream);
 // the same for paths that use scratch for speed where another needs none: whether the buffer holds so many bytes, grown if it has to be.
 // False while `stream` records a graph and its buffer is smaller, and where the memory is not to be had.
 bool workspace_ready(size_t bytes, hipStream_t stream);
+
+// whether `stream` records a graph
+bool stream_captures(hipStream_t stream);
 
 // Held by an entry point while it queues its kernels.  The calls of several host threads then reach their streams
 // one after the other, whole, so that a stream's workspace is used in call order even when threads share the stream

@@ -489,6 +489,21 @@ std::pair<Tensor, Tensor> bound_sort_neuron_shifted(const Tensor& xl, const Tens
     return {lo, up};
 }
 
+// values and bounds of a layer together
+std::tuple<Tensor, Tensor, Tensor> sort_neuron_box_shifted(const Tensor& x, const Tensor& xl, const Tensor& xu, const Tensor& w, int64_t groups,
+                                                           double q, int truncate, const Tensor& shift_in, double sign) {
+    reverse_mode_only("sort_neuron", x, xl, xu, w, shift_in);
+    at::AutoDispatchBelowADInplaceOrView below;
+    const c10::DeviceGuard guard(x.device());
+    Tensor y = new_out(x, w.size(0)), lo = new_out(xl, w.size(0)), up = new_out(xl, w.size(0));
+    const Tensor shift = shift_in.contiguous();
+    const Dims d(x, groups, w.size(0));
+    require(sd_sort_neuron_box_forward(floats(x, "input"), floats(xl, "inputL"), floats(xu, "inputU"), floats(w, "weight"), d.B, d.CO, d.CI, d.G,
+                                       d.HW, floats(y, "output"), floats(lo, "outputL"), floats(up, "outputU"), (float)q, truncate,
+                                       floats(shift, "shift"), (float)sign, stream_of(x)), "sd_sort_neuron_box_forward");
+    return {y, lo, up};
+}
+
 // ---- windows of a convolutional layer as columns; the gradient is the sum back into the image --------------------------
 struct UnfoldNode : Node {   // saves sizes only, which nothing changes or frees
     int B, C, H, W, KH, KW, stride, pad, dil;
@@ -550,5 +565,6 @@ PYBIND11_MODULE(_host, m) {
     m.def("sort_neuron_shifted", &sort_neuron_shifted, released());
     m.def("bound_inf_dist_shifted", &bound_inf_dist_shifted, released());
     m.def("bound_sort_neuron_shifted", &bound_sort_neuron_shifted, released());
+    m.def("sort_neuron_box_shifted", &sort_neuron_box_shifted, released());
     m.def("unfold", &unfold, released());
 }

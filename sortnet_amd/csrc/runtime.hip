@@ -86,6 +86,8 @@ bool capturing(hipStream_t stream) {
 }
 }  // namespace
 
+bool stream_captures(hipStream_t stream) { return capturing(stream); }
+
 bool workspace_ready(size_t bytes, hipStream_t stream) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0) { (void)hipGetLastError(); return false; }

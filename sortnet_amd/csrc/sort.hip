@@ -164,6 +164,7 @@ static long long sort_cols_min_terms(bool pos, int CI) { return pos && CI >= 320
 // `site`: which entry point asks (with the built-in limit, a layer whose tables have not paid lately is not given
 // any for a while, see hint_build_tables)
 constexpr int kHintSiteSort = 2, kHintSiteBoundSort = 3, kHintSiteSortPos = 6;
+constexpr int kHintSiteBox = 16;    // tables for values and bounds together
 constexpr int kHintSiteRows = 10;   // and with the form added: whether the tables per batch row served
 // shape and size alone: the workspace is sized by this, so that a call under graph capture (which always builds
 // tables) never needs more than the eager call before it did
@@ -201,6 +202,17 @@ static size_t sort_tables_bytes(int form, int B, int CO, int CI, int K) {
     return cols + (row_cands_supported(form, K) ? (row_cands_workspace(form, B, CO, CI) + 255) / 256 * 256 : 0);
 }
 
+// One table for the values and the bounds of a layer, and its kernel (sort_cols_box_tables, sort_cols_box_main), queued for both before either.
+// own: the values' own tables behind it, for a layer that it does not serve.
+struct SortBox {
+    const unsigned long long* count;
+    unsigned long long limit;
+    void* ws;
+    char* rest;             // workspace of the two forms, one after the other
+    const float* layer;     // the weights as the caller has them, which the hints know the layer by
+    bool own;
+};
+
 // `ws`: sort_tables_bytes() bytes.  The gate it leaves in `a` points into `ws`: the kernels queued behind it must
 // not be given memory that overlaps it, and `ws` must stay allocated until they have run (one workspace request
 // per call, carved by the caller).  Afterwards a.gate[0] is non-zero when the every-term kernels are to run.
@@ -208,10 +220,16 @@ static size_t sort_tables_bytes(int form, int B, int CO, int CI, int K) {
 // they ran in none of three calls they are left out of the next 31, unless the call before formed every term (hint_build_spare;
 // evaluation pass of 6 x 5120 at batch 512 1636 -> 1575 us, attack on 128 x 5120 x 5120 225 -> 215).  `site`, `layer`: see sort_cols_ok.
 static int queue_sort_cols(FwdArgs& a, int site, const float* layer, int form, const float* xl, const float* xu, const float* w, int B, int CO, int CI,
-                           float q, int K, float* outL, float* outU, int* pos, void* ws, hipStream_t st) {
+                           float q, int K, float* outL, float* outU, int* pos, void* ws, const SortBox* box, hipStream_t st) {
     const float density = g_sort_density.load(std::memory_order_relaxed);
     const float cap = density > 0.f ? density : sort_cols_cap(form, CI);
-    int rc = sort_cols_forward(xl, xu, w, B, CO, CI, q, K, outL, outU, pos, ws, cap, &a.gate, &a.gate_limit, st, a.shift, a.shift_sign);
+    int rc = SD_OK;
+    if (box) {
+        a.gate = box->count;
+        a.gate_limit = box->limit;
+    }
+    if (!rc && (!box || (box->own && form == kRowsSortValues)))
+        rc = sort_cols_forward(xl, xu, w, B, CO, CI, q, K, outL, outU, pos, ws, cap, &a.gate, &a.gate_limit, st, a.shift, a.shift_sign, box ? box->count : nullptr);
     a.gate_above = 1;
     const long long terms = (long long)B * CO * CI;
     const bool rows = row_cands_supported(form, K) && (density > 0.f || terms >= kSortRowsMinTerms) &&
@@ -290,7 +308,7 @@ static bool few_tiles(const FwdArgs& a, int BB, int BM) {
 }
 
 static int sort_values(const float* input, const float* weight, int B, int CO, int CI, int G, int HW, float* output, float q, int K,
-                       const float* shift, float sign, sd_stream_t stream) {
+                       const float* shift, float sign, const SortBox* box, sd_stream_t stream) {
     FwdArgs a;
     int rc = make_fwd_args(a, "sort_neuron_forward_nograd", input, nullptr, weight, B, CO, CI, G, HW, nullptr, nullptr, 0, 0);
     if (rc) return rc;
@@ -298,30 +316,36 @@ static int sort_values(const float* input, const float* weight, int B, int CO, i
     SD_REQUIRE(output, "sort_neuron_forward_nograd: null output");
     a.y0 = output; a.q = q; a.shift = shift; a.shift_sign = sign;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (g_sort_density.load(std::memory_order_relaxed) <= 0.f && row_stream_sort_ok(a))
+    if (!box && g_sort_density.load(std::memory_order_relaxed) <= 0.f && row_stream_sort_ok(a))
         return row_stream_sort(a, K, st);
-    const bool small = few_tiles(a, 32, 64), streamed = g_sort_density.load(std::memory_order_relaxed) <= 0.f && row_stream_sort_before_terms(a);
+    const bool small = few_tiles(a, 32, 64), streamed = !box && g_sort_density.load(std::memory_order_relaxed) <= 0.f && row_stream_sort_before_terms(a);
     const FwdArgs raw = a;
     size_t copies = sort_pad(a, false, B, CO, CI, G, HW);
     if (copies && !workspace_ready(sort_tables_bytes(kRowsSortValues, B, CO, CI, K) + (two_level_ok(a, K) ? align256(two_level_bytes(a, K)) : 0) + copies, st)) {
         a = raw; CI = raw.CIg; copies = 0;
     }
-    const bool two = K <= 12 && two_level_ok(a, K), elig = sort_cols_eligible(a, false, B, CO, CI, G, HW);
-    const bool cols = elig && sort_cols_ok(weight, kHintSiteSort, B, CO, CI, st);
+    const bool two = K <= 12 && two_level_ok(a, K), elig = box || sort_cols_eligible(a, false, B, CO, CI, G, HW);
+    const float* layer = box ? box->layer : weight;
+    const bool cols = box || (elig && sort_cols_ok(layer, kHintSiteSort, B, CO, CI, st));
     if (streamed && !elig) return row_stream_sort(a, K, st);
     // one request for both users of the workspace: the tables (with the counter the gates read) first, the key
     // lists of the two-level path behind them
     const size_t tbytes = elig ? sort_tables_bytes(kRowsSortValues, B, CO, CI, K) : 0, kbytes = two ? align256(two_level_bytes(a, K)) : 0;
     char* base = nullptr;
-    if (elig || two) {
+    if (box) base = box->rest;
+    else if (elig || two) {
         base = static_cast<char*>(workspace(tbytes + kbytes + copies, st));
         if (!base) return SD_ERR_HIP;
     }
     if (streamed && !cols) return row_stream_sort(raw, K, st);
     if (copies && !sort_unpad(a, raw, CI, cols) && (rc = sort_pad_copy(a, raw, base + tbytes + kbytes, st))) return rc;
     int* keys = reinterpret_cast<int*>(base + tbytes);
-    if (cols && (rc = queue_sort_cols(a, kHintSiteSort, weight, kRowsSortValues, a.x0, nullptr, a.w, B, CO, CI, q, K, nullptr, output, nullptr, base, st))) return rc;
-    if (cols) sort_cols_expect(a, weight, kHintSiteSort, B, CO, CI, st);
+    if (cols && (rc = queue_sort_cols(a, kHintSiteSort, layer, kRowsSortValues, a.x0, nullptr, a.w, B, CO, CI, q, K, nullptr, output, nullptr, base, box, st))) return rc;
+    if (cols) sort_cols_expect(a, layer, kHintSiteSort, B, CO, CI, st);
+    if (box && g_sort_density.load(std::memory_order_relaxed) < 0.f) {
+        a.told3 = hint_expect(kHintSiteBox, layer, B, CO, CI, st);
+        a.few3 = box->count + 1;
+    }
     rc = SD_ERR_ARG;
     switch (K) {
 #define X(k) case k: if (k <= 12 && two) rc = run_two_level<(k <= 12 ? k : 2), true>(a, small, keys, st); \
@@ -330,7 +354,7 @@ static int sort_values(const float* input, const float* weight, int B, int CO, i
         SD_FOR_EACH_K(X)
 #undef X
     }
-    if (rc) { hint_forget(a.told); hint_forget(a.told2); }
+    if (rc) { hint_forget(a.told); hint_forget(a.told2); hint_forget(a.told3); }
     return rc;
 }
 
@@ -338,7 +362,7 @@ extern "C" int sd_sort_neuron_forward_nograd(const float* input, const float* we
                                              int B, int CO, int CI, int G, int HW, float* output, float q, int K,
                                              sd_stream_t stream) {
     sd::CallGuard call_guard;   // calls of several host threads reach a stream one after the other, whole
-    return sort_values(input, weight, B, CO, CI, G, HW, output, q, K, nullptr, 0.f, stream);
+    return sort_values(input, weight, B, CO, CI, G, HW, output, q, K, nullptr, 0.f, nullptr, stream);
 }
 
 extern "C" int sd_sort_neuron_forward_shifted(const float* input, const float* weight,
@@ -346,7 +370,7 @@ extern "C" int sd_sort_neuron_forward_shifted(const float* input, const float* w
                                               const float* shift, float sign, sd_stream_t stream) {
     sd::CallGuard call_guard;   // calls of several host threads reach a stream one after the other, whole
     SD_REQUIRE(shift && (sign == 1.f || sign == -1.f), "sort_neuron_forward_shifted: null shift, or a sign (%g) other than 1 and -1", (double)sign);
-    return sort_values(input, weight, B, CO, CI, G, HW, output, q, K, shift, sign, stream);
+    return sort_values(input, weight, B, CO, CI, G, HW, output, q, K, shift, sign, nullptr, stream);
 }
 
 extern "C" int sd_sort_neuron_forward(const float* input, const float* weight,
@@ -383,7 +407,7 @@ extern "C" int sd_sort_neuron_forward(const float* input, const float* weight,
     }
     if (copies && !sort_unpad(a, raw, CI, cols) && (rc = sort_pad_copy(a, raw, base + tbytes + kbytes, st))) return rc;
     int* keys = reinterpret_cast<int*>(base + tbytes);
-    if (cols && (rc = queue_sort_cols(a, kHintSiteSortPos, weight, kRowsSortPos, a.x0, nullptr, a.w, B, CO, CI, q, K, nullptr, output, pos, base, st))) return rc;
+    if (cols && (rc = queue_sort_cols(a, kHintSiteSortPos, weight, kRowsSortPos, a.x0, nullptr, a.w, B, CO, CI, q, K, nullptr, output, pos, base, nullptr, st))) return rc;
     if (cols) sort_cols_expect(a, weight, kHintSiteSortPos, B, CO, CI, st);
     rc = SD_ERR_ARG;
     switch (K) {
@@ -398,7 +422,7 @@ extern "C" int sd_sort_neuron_forward(const float* input, const float* weight,
 }
 
 static int sort_bounds(const float* inputL, const float* inputU, const float* weight, int B, int CO, int CI, int G, int HW, float* outputL,
-                       float* outputU, float q, int K, const float* shift, float sign, sd_stream_t stream) {
+                       float* outputU, float q, int K, const float* shift, float sign, const SortBox* box, sd_stream_t stream) {
     FwdArgs a;
     SD_REQUIRE(inputU, "bound_sort_neuron_forward: null upper input");
     int rc = make_fwd_args(a, "bound_sort_neuron_forward", inputL, inputU, weight, B, CO, CI, G, HW, nullptr, nullptr, 0, 0);
@@ -407,24 +431,25 @@ static int sort_bounds(const float* inputL, const float* inputU, const float* we
     SD_REQUIRE(outputL && outputU, "bound_sort_neuron_forward: null output");
     a.y0 = outputL; a.y1 = outputU; a.q = q; a.shift = shift; a.shift_sign = sign;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (g_sort_density.load(std::memory_order_relaxed) <= 0.f && row_stream_sort_ok(a))
+    if (!box && g_sort_density.load(std::memory_order_relaxed) <= 0.f && row_stream_sort_ok(a))
         return row_stream_sort(a, K, st);
     const bool small = few_tiles(a, 32, 32);
     const FwdArgs raw = a;
     size_t copies = sort_pad(a, false, B, CO, CI, G, HW);
     if (copies && !workspace_ready(sort_tables_bytes(kRowsSortInterval, B, CO, CI, K) + copies, st)) { a = raw; CI = raw.CIg; copies = 0; }
-    const bool elig = sort_cols_eligible(a, false, B, CO, CI, G, HW);
-    const bool cols = elig && sort_cols_ok(weight, kHintSiteBoundSort, B, CO, CI, st);
+    const bool elig = box || sort_cols_eligible(a, false, B, CO, CI, G, HW);
+    const float* layer = box ? box->layer : weight;
+    const bool cols = box || (elig && sort_cols_ok(layer, kHintSiteBoundSort, B, CO, CI, st));
     const bool streamed = !cols && g_sort_density.load(std::memory_order_relaxed) <= 0.f && row_stream_sort_before_terms(raw);
     if (elig) {
         const size_t tbytes = sort_tables_bytes(kRowsSortInterval, B, CO, CI, K);
-        char* ws = static_cast<char*>(workspace(tbytes + copies, st));   // the only request of this call
+        char* ws = box ? box->rest : static_cast<char*>(workspace(tbytes + copies, st));   // the only request of this call
         if (!ws) return SD_ERR_HIP;
         if (copies && !streamed && !sort_unpad(a, raw, CI, cols) && (rc = sort_pad_copy(a, raw, ws + tbytes, st))) return rc;
-        if (cols && (rc = queue_sort_cols(a, kHintSiteBoundSort, weight, kRowsSortInterval, a.x0, a.x1, a.w, B, CO, CI, q, K, outputL, outputU, nullptr, ws, st))) return rc;
+        if (cols && (rc = queue_sort_cols(a, kHintSiteBoundSort, layer, kRowsSortInterval, a.x0, a.x1, a.w, B, CO, CI, q, K, outputL, outputU, nullptr, ws, box, st))) return rc;
     }
     if (streamed) return row_stream_sort(raw, K, st);
-    if (cols) sort_cols_expect(a, weight, kHintSiteBoundSort, B, CO, CI, st);
+    if (cols) sort_cols_expect(a, layer, kHintSiteBoundSort, B, CO, CI, st);
     rc = SD_ERR_ARG;
     switch (K) {
 #define X(k) case k: rc = small ? launch_fwd<BoundSort<k>, 1, 2>(a, st) : launch_fwd<BoundSort<k>, 2, 2>(a, st); break;
@@ -439,7 +464,7 @@ extern "C" int sd_bound_sort_neuron_forward(const float* inputL, const float* in
                                             int B, int CO, int CI, int G, int HW, float* outputL, float* outputU,
                                             float q, int K, sd_stream_t stream) {
     sd::CallGuard call_guard;   // calls of several host threads reach a stream one after the other, whole
-    return sort_bounds(inputL, inputU, weight, B, CO, CI, G, HW, outputL, outputU, q, K, nullptr, 0.f, stream);
+    return sort_bounds(inputL, inputU, weight, B, CO, CI, G, HW, outputL, outputU, q, K, nullptr, 0.f, nullptr, stream);
 }
 
 extern "C" int sd_bound_sort_neuron_forward_shifted(const float* inputL, const float* inputU, const float* weight,
@@ -448,5 +473,63 @@ extern "C" int sd_bound_sort_neuron_forward_shifted(const float* inputL, const f
     sd::CallGuard call_guard;   // calls of several host threads reach a stream one after the other, whole
     SD_REQUIRE(shift && (sign == 1.f || sign == -1.f), "bound_sort_neuron_forward_shifted: null shift, or a sign (%g) other than 1 and -1",
                (double)sign);
-    return sort_bounds(inputL, inputU, weight, B, CO, CI, G, HW, outputL, outputU, q, K, shift, sign, stream);
+    return sort_bounds(inputL, inputU, weight, B, CO, CI, G, HW, outputL, outputU, q, K, shift, sign, nullptr, stream);
+}
+
+// Values and bounds of one layer.  Where both would be given tables per weight row they share one, and one walk: at 512 x 5120 x 5120, K = 10,
+// ranges and table take 59 us where those of the two forms took 102, the walk 192 where theirs took 203 (certification of 6 x 5120 at batch 512
+// 1503 -> 1406 us with the table, 1347 with the walk).  A layer whose shared table does not serve (intervals so wide that they
+// mark nearly everything) goes on as the two calls by themselves: the values' own tables are queued behind the shared one, and return at
+// once where that serves, until it is known to; where it did not in three calls it is left out of the next 31.
+static int sort_box(const float* input, const float* inputL, const float* inputU, const float* weight, int B, int CO, int CI, int G, int HW,
+                    float* output, float* outputL, float* outputU, float q, int K, const float* shift, float sign, sd_stream_t stream) {
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    auto apart = [&]() {
+        const int rc = sort_values(input, weight, B, CO, CI, G, HW, output, q, K, shift, sign, nullptr, stream);
+        return rc ? rc : sort_bounds(inputL, inputU, weight, B, CO, CI, G, HW, outputL, outputU, q, K, shift, sign, nullptr, stream);
+    };
+    FwdArgs v, b;
+    int rc = make_fwd_args(v, "sort_neuron_box_forward", input, nullptr, weight, B, CO, CI, G, HW, nullptr, nullptr, 0, 0);
+    if (rc) return rc;
+    if ((rc = make_fwd_args(b, "sort_neuron_box_forward", inputL, inputU, weight, B, CO, CI, G, HW, nullptr, nullptr, 0, 0))) return rc;
+    if ((rc = check_qk("sort_neuron_box_forward", q, K, v.CIg))) return rc;
+    SD_REQUIRE(inputU && output && outputL && outputU, "sort_neuron_box_forward: null upper input or output");
+    const float density = g_sort_density.load(std::memory_order_relaxed);
+    const FwdArgs raw = v;
+    int N = CI, NB = CI;
+    const size_t copies = sort_pad(v, false, B, CO, N, G, HW), copies_b = sort_pad(b, false, B, CO, NB, G, HW);
+    if ((density <= 0.f && (row_stream_sort_ok(raw) || row_stream_sort_ok(b))) || (copies == 0) != (copies_b == 0) ||
+        !sort_cols_eligible(v, false, B, CO, N, G, HW) || !sort_cols_eligible(b, false, B, CO, NB, G, HW) ||
+        sort_cols_cap(kRowsSortValues, N) != sort_cols_cap(kRowsSortInterval, N))
+        return apart();
+    auto al = [](size_t n) { return (n + 255) / 256 * 256; };
+    const size_t shared = al(sort_cols_box_workspace(B, CO, N)), x = al((size_t)B * N * 4);
+    const size_t values = sort_tables_bytes(kRowsSortValues, B, CO, N, K) + (two_level_ok(v, K) ? al(two_level_bytes(v, K)) : 0);
+    const size_t bounds = sort_tables_bytes(kRowsSortInterval, B, CO, N, K), rest = al(values > bounds ? values : bounds);
+    const size_t bytes = shared + rest + (copies ? 3 * x + al((size_t)CO * N * 4) : 0);
+    if ((density < 0.f && !hint_build_tables(kHintSiteBox, weight, B, CO, N, st)) || !workspace_ready(bytes, st)) return apart();
+    char* ws = static_cast<char*>(workspace(bytes, st));
+    if (!ws) return SD_ERR_HIP;
+    const float *xv = input, *xl = inputL, *xu = inputU, *w = weight;
+    if (copies) {
+        float* p = reinterpret_cast<float*>(ws + shared + rest);
+        float *pv = p, *pl = p + x / 4, *pu = p + x / 2, *pw = p + 3 * (x / 4);
+        if ((rc = pad_rows({input, weight, inputL}, {pv, pw, pl}, {B, CO, B}, CI, N, st))) return rc;
+        if ((rc = pad_rows({inputU, inputU, inputU}, {pu, pu, pu}, {B, 0, 0}, CI, N, st))) return rc;
+        xv = pv; xl = pl; xu = pu; w = pw;
+    }
+    SortBox box{nullptr, 0ull, ws, ws + shared, weight, density < 0.f ? !hint_paid(kHintSiteBox, weight, B, CO, N) || stream_captures(st) : true};
+    if ((rc = sort_cols_box_tables(xv, xl, xu, w, B, CO, N, K, ws, density > 0.f ? density : sort_cols_cap(kRowsSortValues, N), &box.count, &box.limit, st)))
+        return rc;
+    if ((rc = sort_cols_box_main(w, B, CO, N, q, K, output, outputL, outputU, ws, box.limit, shift, sign, st))) return rc;
+    if ((rc = sort_values(xv, w, B, CO, N, G, HW, output, q, K, shift, sign, &box, stream))) return rc;
+    return sort_bounds(xl, xu, w, B, CO, N, G, HW, outputL, outputU, q, K, shift, sign, &box, stream);
+}
+
+extern "C" int sd_sort_neuron_box_forward(const float* input, const float* inputL, const float* inputU, const float* weight,
+                                          int B, int CO, int CI, int G, int HW, float* output, float* outputL, float* outputU,
+                                          float q, int K, const float* shift, float sign, sd_stream_t stream) {
+    sd::CallGuard call_guard;   // calls of several host threads reach a stream one after the other, whole
+    SD_REQUIRE(!shift || sign == 1.f || sign == -1.f, "sort_neuron_box_forward: a sign (%g) other than 1 and -1", (double)sign);
+    return sort_box(input, inputL, inputU, weight, B, CO, CI, G, HW, output, outputL, outputU, q, K, shift, sign, stream);
 }

@@ -27,9 +27,21 @@ size_t sort_cols_workspace(int B, int CO, int CI);
 //   xu == nullptr: value form on xl, outU receives the values (outL is not used) and pos, if not null, the K planes
 //   of positions (K, B, CO), largest first.
 //   shift, shift_sign: see FwdArgs (forms without positions).
+//   unless: counter words of a table queued before; nothing is built, and no kernel of the call runs, where that one served.
 int sort_cols_forward(const float* xl, const float* xu, const float* w, int B, int CO, int CI, float q, int K,
                       float* outL, float* outU, int* pos, void* ws, float density, const unsigned long long** gate,
-                      unsigned long long* gate_limit, hipStream_t st, const float* shift = nullptr, float shift_sign = 0.f);
+                      unsigned long long* gate_limit, hipStream_t st, const float* shift = nullptr, float shift_sign = 0.f,
+                      const unsigned long long* unless = nullptr);
+
+// Values and interval bounds of one layer from one table: the ranges are those of inputs and both ends together, so one table
+// holds a superset of each form's marks, and the walks drop what is not needed (cand_walk.h).  sort_cols_box_tables builds it,
+// sort_cols_box_main walks it for the values (out) and the bounds.  `ws`: sort_cols_box_workspace bytes, kept until both have run;
+// gate, gate_limit and density as in sort_cols_forward.
+size_t sort_cols_box_workspace(int B, int CO, int CI);
+int sort_cols_box_tables(const float* x, const float* xl, const float* xu, const float* w, int B, int CO, int CI, int K, void* ws,
+                         float density, const unsigned long long** gate, unsigned long long* gate_limit, hipStream_t st);
+int sort_cols_box_main(const float* w, int B, int CO, int CI, float q, int K, float* out, float* outL, float* outU, void* ws,
+                       unsigned long long gate_limit, const float* shift, float shift_sign, hipStream_t st);
 
 // The two sums of the probe that sort_cols_forward / max_cols_forward leave behind the counter words *gate points at
 // (widths of the input columns over all batch tiles; widths of the same columns over 16 weight rows), for the tables

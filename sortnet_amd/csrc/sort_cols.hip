@@ -16,6 +16,7 @@ constexpr int kRowPad = 128;         // weight rows are padded to a multiple of 
 constexpr int kMainWaves = 4;        // wavefronts of a workgroup of the main kernels
 constexpr int kMainTile = kMainWaves;   // weight rows of a workgroup, one per wavefront
 constexpr int kSample = 640;         // see walk_marks
+constexpr int kBoxK = 10;            // see sort_cols_box_main
 
 inline size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 inline int tiles_b(int B) { return (B + kTileB - 1) / kTileB; }
@@ -72,29 +73,35 @@ __device__ __forceinline__ void repair(float& l, float& u) {
 // MASKED (value form only): xkeep holds one word per (batch row, 32 inputs); an input a row does not keep takes no
 // part in the ranges and is undefined in the transposed copy, so that its term never wins a comparison.  A column no
 // row of the tile keeps has neither a lower bound nor a candidate.
-// TWO: the ranges of l and of u apart.
-template <bool IV, bool TWO, bool MASKED>
+// TWO: the ranges of l and of u apart.  BOX: intervals with the inputs x beside them, one range over all three; xT2: x transposed.
+// unless: see sort_cols.h.
+template <bool IV, bool TWO, bool MASKED, bool BOX = false>
 __global__ void __launch_bounds__(256) sc_range_kernel(const float* __restrict__ xl, const float* __restrict__ xu,
                                                        const float* __restrict__ w, const uint32_t* __restrict__ xkeep,
                                                        int B, int M, int N, int Bp, float* __restrict__ xr,
                                                        float* __restrict__ xT, float2* __restrict__ widths,
-                                                       TableCount* __restrict__ count) {
+                                                       TableCount* __restrict__ count, const unsigned long long* __restrict__ unless,
+                                                       const float* __restrict__ x, float* __restrict__ xT2) {
     if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) count->sum = 0ull;
+    if (unless != nullptr && unless[1] == 0ull) return;
+    static_assert(!BOX || (IV && !TWO), "");
     static_assert(!(IV && MASKED) && (IV || !TWO), "the factored mask belongs to the value form, two ranges to the interval form");
     constexpr int kCols = kChunk, kGroups = 256 / kCols, kRows = kTileB / kGroups;
     __shared__ float part[kGroups][5][kCols];
     __shared__ float wpart[kGroups][2][kCols];
     __shared__ float tl[kCols][kTileB + 1];
     __shared__ float tu[IV ? kCols : 1][kTileB + 1];
+    __shared__ float tx[BOX ? kCols : 1][kTileB + 1];
     const int tid = threadIdx.x, nl = tid % kCols, grp = tid / kCols;
     const int n0 = blockIdx.x * kCols, n = n0 + nl, s = blockIdx.y;   // (N is a multiple of 32)
-    float l[kRows], u[IV ? kRows : 1];
+    float l[kRows], u[IV ? kRows : 1], v[BOX ? kRows : 1];
     uint32_t kept = ~0u;
     #pragma unroll
     for (int r = 0; r < kRows; r++) {
         const int row = s * kTileB + grp * kRows + r, rr = row < B ? row : B - 1;
         l[r] = xl[(size_t)rr * N + n];
         if constexpr (IV) u[r] = xu[(size_t)rr * N + n];
+        if constexpr (BOX) v[r] = x[(size_t)rr * N + n];
         if constexpr (MASKED) { if (!((xkeep[(size_t)rr * (N / kChunk) + blockIdx.x] >> nl) & 1u)) kept &= ~(1u << r); }
     }
     // the probe: ranges of the same columns over the first 16 weight rows (tile 0 only)
@@ -111,16 +118,18 @@ __global__ void __launch_bounds__(256) sc_range_kernel(const float* __restrict__
     #pragma unroll
     for (int r = 0; r < kRows; r++) {
         const int col = grp * kRows + r;
-        float a = l[r], b = IV ? u[IV ? r : 0] : a;
-        if (s * kTileB + col >= B) a = b = 0.f;
+        float a = l[r], b = IV ? u[IV ? r : 0] : a, m = BOX ? v[BOX ? r : 0] : a;
+        if (s * kTileB + col >= B) a = b = m = 0.f;
         else if ((kept >> r) & 1u) {
             odd += (a - a) + (b - b);
             if (IV) repair(a, b);
             lmin = fminf(lmin, a); lmax = fmaxf(lmax, a);
             umin = fminf(umin, b); umax = fmaxf(umax, b);
+            if (BOX) { odd += m - m; lmin = fminf(lmin, m); umax = fmaxf(umax, m); }
         } else a = b = __builtin_nanf("");
         tl[nl][col] = a;
         if (IV) tu[nl][col] = b;
+        if (BOX) tx[nl][col] = m;
     }
     part[grp][0][nl] = lmin; part[grp][1][nl] = lmax; part[grp][2][nl] = umin; part[grp][3][nl] = umax;
     part[grp][4][nl] = odd;
@@ -155,6 +164,7 @@ __global__ void __launch_bounds__(256) sc_range_kernel(const float* __restrict__
         const size_t o = (size_t)(n0 + nn) * Bp + s * kTileB + col;
         if (IV) reinterpret_cast<float2*>(xT)[o] = make_float2(tl[nn][col], tu[nn][col]);
         else xT[o] = tl[nn][col];
+        if (BOX) xT2[o] = tx[nn][col];
     }
 }
 
@@ -181,8 +191,13 @@ __device__ __forceinline__ bool table_pointless(const float2* __restrict__ width
 // Bounds and marks (cand_tables.h); J = 0: rows of any length
 template <int J, int R, int NT, bool TWO, bool MASK>
 __global__ void __launch_bounds__(64 * (J ? kStreamWaves : kTableWaves))
-sc_tables_kernel(TableArgs a, const float2* __restrict__ widths, TableCount* __restrict__ c, unsigned long long limit) {
+sc_tables_kernel(TableArgs a, const float2* __restrict__ widths, TableCount* __restrict__ c, unsigned long long limit,
+                 const unsigned long long* __restrict__ unless) {
     extern __shared__ __attribute__((aligned(16))) float smem[];
+    if (unless != nullptr && unless[1] == 0ull) {   // not needed: no kernel of this table, none that forms every term, and none of the other orientation
+        if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) { c->marks = ~0ull; c->above = 0ull; c->stat[0] = c->stat[1] = 0.f; }
+        return;
+    }
     if (table_pointless(widths, a.tiles * (a.N / kChunk), a.tiles, c->stat)) {
         if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) { c->marks = ~0ull; c->above = 1ull; }
         return;
@@ -195,7 +210,7 @@ sc_tables_kernel(TableArgs a, const float2* __restrict__ widths, TableCount* __r
 }
 
 template <int J, int R, int NT, bool TWO, bool MASK>
-int launch_tables(const TableArgs& t, const Carve& c, unsigned long long limit, hipStream_t st) {
+int launch_tables(const TableArgs& t, const Carve& c, unsigned long long limit, const unsigned long long* unless, hipStream_t st) {
     const int groups = (t.tiles + NT - 1) / NT;
     dim3 grid((t.R + R * kTableWaves - 1) / (R * kTableWaves), groups), block(64 * kTableWaves);
     size_t lds = (size_t)NT * (TWO ? 4 : 2) * kTableSlice * 4;
@@ -205,28 +220,28 @@ int launch_tables(const TableArgs& t, const Carve& c, unsigned long long limit, 
         block.x = 64 * s.waves;
         lds = stream_lds(s.waves, R * NT * (TWO ? 2 : 1));
     }
-    hipLaunchKernelGGL((sc_tables_kernel<J, R, NT, TWO, MASK>), grid, block, lds, st, t, c.widths, c.count, limit);
+    hipLaunchKernelGGL((sc_tables_kernel<J, R, NT, TWO, MASK>), grid, block, lds, st, t, c.widths, c.count, limit, unless);
     return check_launch("sc_tables_kernel");
 }
 // As many batch tiles at a time as there are, up to four, and as the registers hold ranges of (64 per lane).
 template <bool TWO, bool MASK>
 int run_tables(const float* w, const uint32_t* wkeep, int S, int M, int Mp, int N, int K, const Carve& c,
-               unsigned long long limit, hipStream_t st) {
+               unsigned long long limit, const unsigned long long* unless, hipStream_t st) {
     const TableArgs t{w, w, wkeep, c.xr, M, Mp, N, S, K, c.low, c.bits};
     switch (stream_blocks(N)) {
         case 1:
-            if (S == 1) return launch_tables<1, 4, 1, TWO, MASK>(t, c, limit, st);
-            if (S == 2) return launch_tables<1, 2, 2, TWO, MASK>(t, c, limit, st);
-            return launch_tables<1, 2, 4, TWO, MASK>(t, c, limit, st);
+            if (S == 1) return launch_tables<1, 4, 1, TWO, MASK>(t, c, limit, unless, st);
+            if (S == 2) return launch_tables<1, 2, 2, TWO, MASK>(t, c, limit, unless, st);
+            return launch_tables<1, 2, 4, TWO, MASK>(t, c, limit, unless, st);
         case 2:
-            if (S == 1) return launch_tables<2, 2, 1, TWO, MASK>(t, c, limit, st);
-            if (TWO || S == 2) return launch_tables<2, TWO ? 1 : 2, 2, TWO, MASK>(t, c, limit, st);
-            return launch_tables<2, MASK ? 1 : 2, TWO ? 2 : 4, TWO, MASK>(t, c, limit, st);
+            if (S == 1) return launch_tables<2, 2, 1, TWO, MASK>(t, c, limit, unless, st);
+            if (TWO || S == 2) return launch_tables<2, TWO ? 1 : 2, 2, TWO, MASK>(t, c, limit, unless, st);
+            return launch_tables<2, MASK ? 1 : 2, TWO ? 2 : 4, TWO, MASK>(t, c, limit, unless, st);
         case 3:
-            if (TWO || S == 1) return launch_tables<3, 2, 1, TWO, MASK>(t, c, limit, st);
-            return launch_tables<3, 1, TWO ? 1 : 2, TWO, MASK>(t, c, limit, st);
+            if (TWO || S == 1) return launch_tables<3, 2, 1, TWO, MASK>(t, c, limit, unless, st);
+            return launch_tables<3, 1, TWO ? 1 : 2, TWO, MASK>(t, c, limit, unless, st);
     }
-    return launch_tables<0, 1, 4, TWO, MASK>(t, c, limit, st);
+    return launch_tables<0, 1, 4, TWO, MASK>(t, c, limit, unless, st);
 }
 
 // ---- main kernels ------------------------------------------------------------------------------
@@ -261,17 +276,21 @@ struct Caps {
 // (branch-free medians; same terms, same lists).
 // MAXFORM (K = 1, interval form): the lists are the running maxima of the interval bounds of the l-inf distance
 // (core/cuda/bound_inf_dist_cuda.cu:15-118), which leave as max(1e-10, .) instead of through the geometric sum.
-template <int K, bool IV, bool MAXFORM = false>
-__global__ void __launch_bounds__(64 * kMainWaves)
+// BOX (with IV): values and bounds in one walk, which meets no more marks than the bounds' alone (an input in its interval has the K-th
+// largest term between theirs): 512 x 5120 x 5120, K = 10,
+// 192 us, 133 and 78 for the two by themselves.  Four wavefronts per SIMD of 128 registers (five of 96 for the bounds alone).
+template <int K, bool IV, bool MAXFORM = false, bool BOX = false>
+__global__ void __launch_bounds__(64 * kMainWaves, BOX ? 4 : 1)
 sc_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const uint32_t* __restrict__ bits,
                const float* __restrict__ xr, const float* __restrict__ low, const unsigned long long* __restrict__ count,
                unsigned long long limit, int B, int Bp, int M, int Mp, int N, float q, float* __restrict__ yL,
-               float* __restrict__ yU, const float* __restrict__ shift, float shift_sign) {
+               float* __restrict__ yU, const float* __restrict__ shift, float shift_sign, const float* __restrict__ xT2,
+               float* __restrict__ y) {
     if (gate_closed(count, limit, 0)) return;
     static_assert(!MAXFORM || (K == 1 && IV), "the maximum form is the interval form with one entry");
     union Shared {
         uint16_t list[kMainWaves][kWalkListCap];
-        float stage[IV ? 2 : 1][kTileB][kMainTile + 1];
+        float stage[BOX ? 3 : IV ? 2 : 1][kTileB][kMainTile + 1];
     };
     __shared__ Shared sh;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -280,10 +299,12 @@ sc_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const 
     const int mb = item % MB, s = item / MB, m = mb * kMainTile + wave;
     using X = typename std::conditional<IV, float2, float>::type;
     const X* __restrict__ xcol = reinterpret_cast<const X*>(xT) + (size_t)s * kTileB + lane;
-    int hi[2][K], lo[IV ? 2 : 1][IV ? K : 1];
+    const float* __restrict__ vcol = BOX ? xT2 + (size_t)s * kTileB + lane : nullptr;
+    int hi[2][K], lo[IV ? 2 : 1][IV ? K : 1], val[BOX ? 2 : 1][BOX ? K : 1];
     #pragma unroll
     for (int k = 0; k < K; k++) {
         hi[0][k] = hi[1][k] = 0;
+        if constexpr (BOX) val[0][k] = val[1][k] = 0;
         if constexpr (IV) lo[0][k] = lo[1][k] = 0;
     }
     if (m < M) {   // wave-uniform
@@ -293,12 +314,15 @@ sc_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const 
         const float LU = low[(size_t)s * (MAXFORM ? 2 : 1) * Mp + m], LL = MAXFORM ? low[(size_t)(s * 2 + 1) * Mp + m] : LU;
         const bool in0 = s * kTileB + lane < B, in1 = s * kTileB + lane + 64 < B;   // the lane's batch rows exist
         X xa[2][4], xb[2][4];
+        float va[BOX ? 2 : 1][BOX ? 4 : 1], vb[BOX ? 2 : 1][BOX ? 4 : 1];
         auto load = [&](int buf, int i, int n) __attribute__((always_inline)) {
             xa[buf][i] = xcol[(size_t)n * Bp];
             xb[buf][i] = xcol[(size_t)n * Bp + 64];
+            if constexpr (BOX) { va[buf][i] = vcol[(size_t)n * Bp]; vb[buf][i] = vcol[(size_t)n * Bp + 64]; }
         };
         auto use = [&](int buf, int i, int k, int, const Own& o) __attribute__((always_inline)) {
             const float wi = lane_value(o.a, k);
+            if constexpr (BOX) insert_pair<K>(val[0], fmaxf(fabsf(va[buf][i] - wi), -1.f), val[1], fmaxf(fabsf(vb[buf][i] - wi), -1.f));
             if constexpr (IV && MAXFORM) {
                 // a term with an undefined operand is dropped (min / max keep the defined one, as the reference's do;
                 // the final max with 0 drops a term that is undefined altogether)
@@ -334,9 +358,14 @@ sc_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const 
                 [&](int n, const Own& o) __attribute__((always_inline)) { const float2 v = caps(n, o.a); return fmaxf(v.x - LU, v.y - LL); },
                 load, use, use,
                 [&](bool) __attribute__((always_inline)) {
-                    thU = smallest(hi[0][0], hi[1][0]);
-                    if constexpr (IV) thL = smallest(lo[0][0], lo[1][0]);
-                    else thL = thU;
+                    // (one cap stands for every result of the forms without ranges of l and u apart)
+                    if constexpr (BOX) thU = thL = smallest(min(min(hi[0][0], lo[0][0]), val[0][0]), min(min(hi[1][0], lo[1][0]), val[1][0]));
+                    else if constexpr (IV && !MAXFORM) thU = thL = smallest(min(hi[0][0], lo[0][0]), min(hi[1][0], lo[1][0]));
+                    else {
+                        thU = smallest(hi[0][0], hi[1][0]);
+                        if constexpr (IV) thL = smallest(lo[0][0], lo[1][0]);
+                        else thL = thU;
+                    }
                 },
                 [&](int n, const Own& o) __attribute__((always_inline)) { const float2 v = caps(n, o.a); return !(v.x < thU) || !(v.y < thL); },
                 [] {});
@@ -351,6 +380,7 @@ sc_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const 
         } else {
             sh.stage[0][lane + 64 * j][wave] = geo_sum_bits<K>(hi[j], q);
             if constexpr (IV) sh.stage[1][lane + 64 * j][wave] = geo_sum_bits<K>(lo[j], q);
+            if constexpr (BOX) sh.stage[2][lane + 64 * j][wave] = geo_sum_bits<K>(val[j], q);
         }
     }
     __syncthreads();
@@ -361,6 +391,7 @@ sc_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const 
             const float add = output_shift(shift, shift_sign, mm);
             yU[(size_t)b * M + mm] = sh.stage[0][bl][mloc] + add;
             if constexpr (IV) yL[(size_t)b * M + mm] = sh.stage[1][bl][mloc] + add;
+            if constexpr (BOX) y[(size_t)b * M + mm] = sh.stage[2][bl][mloc] + add;
         }
     }
 }
@@ -465,9 +496,9 @@ int run_max(const float* x, const float* w, const uint32_t* xkeep, const uint32_
             int* pos, const Carve& c, unsigned long long limit, hipStream_t st) {
     const int S = tiles_b(B), Bp = S * kTileB, Mp = mpad_of(M);
     int rc;
-    hipLaunchKernelGGL((sc_range_kernel<false, false, MASK>), dim3(N / kChunk, S), dim3(256), 0, st, x, nullptr, w, xkeep, B, M, N, Bp, c.xr, c.xT, c.widths, c.count);
+    hipLaunchKernelGGL((sc_range_kernel<false, false, MASK>), dim3(N / kChunk, S), dim3(256), 0, st, x, nullptr, w, xkeep, B, M, N, Bp, c.xr, c.xT, c.widths, c.count, nullptr, nullptr, nullptr);
     if ((rc = check_launch("sc_range_kernel"))) return rc;
-    if ((rc = run_tables<false, MASK>(w, wkeep, S, M, Mp, N, K, c, limit, st))) return rc;
+    if ((rc = run_tables<false, MASK>(w, wkeep, S, M, Mp, N, K, c, limit, nullptr, st))) return rc;
     const dim3 grid((unsigned)(S * (Mp / kMainTile)));
     if (pos) hipLaunchKernelGGL((mc_main_kernel<true>), grid, dim3(64 * kMainWaves), 0, st, c.xT, w, c.bits, wkeep, c.xr, c.low, &c.count->marks, limit, B, Bp, M, Mp, N, y, pos);
     else hipLaunchKernelGGL((mc_main_kernel<false>), grid, dim3(64 * kMainWaves), 0, st, c.xT, w, c.bits, wkeep, c.xr, c.low, &c.count->marks, limit, B, Bp, M, Mp, N, y, pos);
@@ -620,12 +651,12 @@ sp_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const 
 
 template <int K, bool IV, bool MAXFORM = false>
 int run(const float* xl, const float* xu, const float* w, int B, int M, int N, float q, float* outL, float* outU,
-        int* pos, const Carve& c, unsigned long long limit, const float* shift, float shift_sign, hipStream_t st) {
+        int* pos, const Carve& c, unsigned long long limit, const float* shift, float shift_sign, const unsigned long long* unless, hipStream_t st) {
     const int S = tiles_b(B), Bp = S * kTileB, Mp = mpad_of(M);
     int rc;
-    hipLaunchKernelGGL((sc_range_kernel<IV, MAXFORM, false>), dim3(N / kChunk, S), dim3(256), 0, st, xl, xu, w, nullptr, B, M, N, Bp, c.xr, c.xT, c.widths, c.count);
+    hipLaunchKernelGGL((sc_range_kernel<IV, MAXFORM, false>), dim3(N / kChunk, S), dim3(256), 0, st, xl, xu, w, nullptr, B, M, N, Bp, c.xr, c.xT, c.widths, c.count, unless, nullptr, nullptr);
     if ((rc = check_launch("sc_range_kernel"))) return rc;
-    if ((rc = run_tables<MAXFORM, false>(w, nullptr, S, M, Mp, N, K, c, limit, st))) return rc;
+    if ((rc = run_tables<MAXFORM, false>(w, nullptr, S, M, Mp, N, K, c, limit, unless, st))) return rc;
     if constexpr (!IV) {
         if (pos) {
             hipLaunchKernelGGL((sp_main_kernel<K>), dim3((unsigned)(S * (Mp / kMainTile))), dim3(64 * kMainWaves), 0, st,
@@ -634,7 +665,7 @@ int run(const float* xl, const float* xu, const float* w, int B, int M, int N, f
         }
     }
     hipLaunchKernelGGL((sc_main_kernel<K, IV, MAXFORM>), dim3((unsigned)(S * (Mp / kMainTile))), dim3(64 * kMainWaves), 0, st,
-                       c.xT, w, c.bits, c.xr, c.low, &c.count->marks, limit, B, Bp, M, Mp, N, q, outL, outU, shift, shift_sign);
+                       c.xT, w, c.bits, c.xr, c.low, &c.count->marks, limit, B, Bp, M, Mp, N, q, outL, outU, shift, shift_sign, nullptr, nullptr);
     return check_launch("sc_main_kernel");
 }
 
@@ -651,7 +682,7 @@ size_t sort_cols_workspace(int B, int CO, int CI) {
 
 int sort_cols_forward(const float* xl, const float* xu, const float* w, int B, int CO, int CI, float q, int K,
                       float* outL, float* outU, int* pos, void* ws, float density, const unsigned long long** gate,
-                      unsigned long long* gate_limit, hipStream_t st, const float* shift, float shift_sign) {
+                      unsigned long long* gate_limit, hipStream_t st, const float* shift, float shift_sign, const unsigned long long* unless) {
     if (CI % kChunk != 0 || CI > 65536 || B < 1 || CO < 1) {
         set_error("sort_cols_forward: shape not supported");
         return SD_ERR_ARG;
@@ -662,10 +693,10 @@ int sort_cols_forward(const float* xl, const float* xu, const float* w, int B, i
     *gate = &c.count->marks;
     *gate_limit = limit;
     note_term_counts(&c.count->marks, 1, (double)tiles_b(B) * CO * CI, 1.0);
-    if (K == 1 && xu) return run<1, true, true>(xl, xu, w, B, CO, CI, q, outL, outU, nullptr, c, limit, shift, shift_sign, st);
+    if (K == 1 && xu) return run<1, true, true>(xl, xu, w, B, CO, CI, q, outL, outU, nullptr, c, limit, shift, shift_sign, unless, st);
     switch (K) {
-#define X(k) case k: return xu ? run<k, true>(xl, xu, w, B, CO, CI, q, outL, outU, nullptr, c, limit, shift, shift_sign, st) \
-                               : run<k, false>(xl, nullptr, w, B, CO, CI, q, outL, outU, pos, c, limit, shift, shift_sign, st);
+#define X(k) case k: return xu ? run<k, true>(xl, xu, w, B, CO, CI, q, outL, outU, nullptr, c, limit, shift, shift_sign, unless, st) \
+                               : run<k, false>(xl, nullptr, w, B, CO, CI, q, outL, outU, pos, c, limit, shift, shift_sign, unless, st);
         SD_SORT_COLS_K(X)
 #undef X
     }
@@ -673,6 +704,56 @@ int sort_cols_forward(const float* xl, const float* xu, const float* w, int B, i
     return SD_ERR_ARG;
 }
 
+
+namespace {
+float* box_inputs(void* ws, int B, int M, int N) { return reinterpret_cast<float*>(static_cast<char*>(ws) + align256(sort_cols_workspace(B, M, N))); }
+}
+
+size_t sort_cols_box_workspace(int B, int CO, int CI) {
+    return align256(sort_cols_workspace(B, CO, CI)) + align256((size_t)CI * tiles_b(B) * kTileB * 4);
+}
+
+int sort_cols_box_tables(const float* x, const float* xl, const float* xu, const float* w, int B, int CO, int CI, int K, void* ws,
+                         float density, const unsigned long long** gate, unsigned long long* gate_limit, hipStream_t st) {
+    if (CI % kChunk != 0 || CI > 65536 || B < 1 || CO < 1 || K < 2 || K > 25) {
+        set_error("sort_cols_box_tables: shape not supported");
+        return SD_ERR_ARG;
+    }
+    const Carve c = carve(ws, B, CO, CI);
+    const float d = density < 0.f ? 0.f : density > 1.f ? 1.f : density;
+    const int S = tiles_b(B), Bp = S * kTileB;
+    *gate = &c.count->marks;
+    *gate_limit = (unsigned long long)((double)S * CO * CI * d);
+    note_term_counts(&c.count->marks, 1, (double)S * CO * CI, 1.0);
+    hipLaunchKernelGGL((sc_range_kernel<true, false, false, true>), dim3(CI / kChunk, S), dim3(256), 0, st, xl, xu, w, nullptr, B, CO, CI, Bp, c.xr, c.xT,
+                       c.widths, c.count, nullptr, x, box_inputs(ws, B, CO, CI));
+    const int rc = check_launch("sc_range_kernel");
+    return rc ? rc : run_tables<false, false>(w, nullptr, S, CO, mpad_of(CO), CI, K, c, *gate_limit, nullptr, st);
+}
+
+int sort_cols_box_main(const float* w, int B, int CO, int CI, float q, int K, float* out, float* outL, float* outU, void* ws,
+                       unsigned long long gate_limit, const float* shift, float shift_sign, hipStream_t st) {
+    const Carve c = carve(ws, B, CO, CI);
+    const int S = tiles_b(B), Bp = S * kTileB, Mp = mpad_of(CO);
+    const dim3 grid((unsigned)(S * (Mp / kMainTile))), block(64 * kMainWaves);
+    const float* xT2 = box_inputs(ws, B, CO, CI);
+    if (K == kBoxK) {   // the depth of the layers' neuron (its default)
+        hipLaunchKernelGGL((sc_main_kernel<kBoxK, true, false, true>), grid, block, 0, st, c.xT, w, c.bits, c.xr, c.low, &c.count->marks, gate_limit, B, Bp,
+                           CO, Mp, CI, q, outL, outU, shift, shift_sign, xT2, out);
+        return check_launch("sc_main_kernel");
+    }
+    switch (K) {
+#define X(k) case k: \
+        hipLaunchKernelGGL((sc_main_kernel<k, true>), grid, block, 0, st, c.xT, w, c.bits, c.xr, c.low, &c.count->marks, gate_limit, B, Bp, \
+                           CO, Mp, CI, q, outL, outU, shift, shift_sign, nullptr, nullptr); \
+        hipLaunchKernelGGL((sc_main_kernel<k, false>), grid, block, 0, st, xT2, w, c.bits, c.xr, c.low, &c.count->marks, gate_limit, B, Bp, \
+                           CO, Mp, CI, q, nullptr, out, shift, shift_sign, nullptr, nullptr); \
+        break;
+        SD_SORT_COLS_K(X)
+#undef X
+    }
+    return check_launch("sc_main_kernel");
+}
 
 int max_cols_depth(float keep_x) {
     if (keep_x >= 1.f) return 1;

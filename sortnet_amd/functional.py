@@ -266,6 +266,16 @@ def _shifted_bounds(x_lower, x_upper, weight, groups, q, shift, sign, truncate=1
     return host.bound_sort_neuron_shifted(x_lower, x_upper, weight, groups, q, truncate, shift, sign)
 
 
+def _shifted_box(x, x_lower, x_upper, weight, groups, q, shift, sign, truncate=10):
+    """Values and bounds of one layer."""
+    truncate = min(weight.size(-1), truncate)
+    if q is None or q == 1.0 or truncate == 1 or x.size() != x_lower.size():
+        return (_shifted_values(x, weight, groups, q, shift, sign, truncate),
+                *_shifted_bounds(x_lower, x_upper, weight, groups, q, shift, sign, truncate))
+    assert x_lower.size() == x_upper.size()
+    return _checked(x, weight, groups).sort_neuron_box_shifted(x, x_lower, x_upper, weight, groups, q, truncate, shift, sign)
+
+
 def masked_inf_dist(input, weight, q, seed, groups=1, mode=_C.MASK_TERM, tag=None):
     """Masked order-statistic neuron (see MaskedInfDistF).  `mode` is ext.MASK_TERM (independent
     draw per term) or ext.MASK_FACTORED (keep = keep_x(b, n) & keep_w(m, n))."""

@@ -221,6 +221,8 @@ class NormDistBase(nn.Module):
         return (vec, sign) if vec is not None and F._kernels_can_add(vec, self.weight) else None
 
     def _forward_shifted(self, x, lower, upper, q, shift, sign):
+        if x is not None and lower is not None:
+            return F._shifted_box(x, lower, upper, self.weight, self.groups, q, shift, sign)
         if x is not None:
             x = F._shifted_values(x, self.weight, self.groups, q, shift, sign)
         if lower is not None:

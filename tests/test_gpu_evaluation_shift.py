@@ -149,3 +149,55 @@ def test_arguments_are_checked():
         ext.host().sort_neuron_shifted(x, w, 1, 0.5, 10, shift, 0.5)
     with pytest.raises(RuntimeError, match="must be a CUDA tensor"):
         ext.host().norm_dist_shifted(x, w, 1, shift.cpu(), 1.0)
+
+
+# one table for values and bounds: served (whole and padded rows, tiles that are not full), too many marks for the bounds alone (wide
+# intervals), undefined and infinite entries, inputs outside their intervals, intervals turned round
+@pytest.mark.parametrize("density", [-1.0, 0.03, 1.0])
+@pytest.mark.parametrize("width", [0.02, 3.0])
+@pytest.mark.parametrize("B,N,M", [(128, 320, 450), (257, 1024, 300), (200, 1306, 700), (130, 4443, 515), (384, 5120, 129), (150, 12320, 64)])
+def test_box_has_the_bits_of_both_calls(B, N, M, width, density):
+    g = torch.Generator(device="cuda").manual_seed(B + N)
+    x = torch.randn(B, N, 1, device="cuda", generator=g).mul_(0.1)
+    w = torch.randn(M, N, device="cuda", generator=g)
+    lo, up = x - width, x + width
+    lo[3, 5], up[3, 5] = up[3, 5].clone(), lo[3, 5].clone()
+    x[1, 7] = 9.0
+    x[2, 3], lo[4, 1], up[5, 2], w[6, 4], w[7, 8] = float("nan"), float("-inf"), float("inf"), float("inf"), float("nan")
+    shift = torch.randn(M, device="cuda", generator=g)
+    _lib.set_sort_candidate_density(density)
+    try:
+        want = [F._shifted_values(x, w, 1, 0.75, shift, -1.0), *F._shifted_bounds(lo, up, w, 1, 0.75, shift, -1.0)]
+        for _ in range(6):                                    # as the hints learn
+            for got, ref in zip(F._shifted_box(x, lo, up, w, 1, 0.75, shift, -1.0), want):
+                assert torch.equal(got.nan_to_num(nan=-1.0), ref.nan_to_num(nan=-1.0))
+            torch.cuda.synchronize()
+    finally:
+        _lib.set_sort_candidate_density(-1.0)
+
+
+def test_box_under_capture():
+    """Recorded before and after a call has sized the workspace, replayed on narrow and wide intervals."""
+    g = torch.Generator(device="cuda").manual_seed(11)
+    B, N, M = 256, 1024, 512
+    w = torch.randn(M, N, device="cuda", generator=g)
+    shift = torch.randn(M, device="cuda", generator=g)
+    x = torch.randn(B, N, 1, device="cuda", generator=g).mul_(0.1)
+    lo, up = x - 0.02, x + 0.02
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        for _ in range(3):
+            F._shifted_box(x, lo, up, w, 1, 0.75, shift, -1.0)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = F._shifted_box(x, lo, up, w, 1, 0.75, shift, -1.0)
+    for width in (0.02, 2.0, 0.0, 5.0, 0.02):
+        x.copy_(torch.randn(B, N, 1, device="cuda", generator=g).mul_(0.1))
+        lo.copy_(x - width)
+        up.copy_(x + width)
+        graph.replay()
+        torch.cuda.synchronize()
+        want = [F._shifted_values(x, w, 1, 0.75, shift, -1.0), *F._shifted_bounds(lo, up, w, 1, 0.75, shift, -1.0)]
+        for got, ref in zip(out, want):
+            assert torch.equal(got, ref)
