@@ -305,7 +305,7 @@ __global__ void __launch_bounds__(64 * kRtWaves) rt_main_kernel(RtArgs a) {
     // order may leave the others out.
     for_marks(list, NCH, lane, [&](int c) __attribute__((always_inline)) { return rowbits[c]; },
               [&](int total, bool first) __attribute__((always_inline)) {
-        walk_marks<ORDERED, IV, 128>(list, total, first, lane,
+        walk_marks<ORDERED, IV, 128, LISTS && !ORDERED ? walk_short(K) : 0>(list, total, first, lane,
             [&](int n) __attribute__((always_inline)) {
                 Own o{xlrow[n], 0.f};
                 if constexpr (IV) { o.b = xurow[n]; repair(o.a, o.b); }

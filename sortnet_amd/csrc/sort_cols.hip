@@ -353,7 +353,7 @@ sc_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const 
         };
         for_marks(list, NCH, lane, [&](int c) __attribute__((always_inline)) { return rowbits[c]; },
                   [&](int total, bool first) __attribute__((always_inline)) {
-            walk_marks<false, false, kSample>(list, total, first, lane,
+            walk_marks<false, false, kSample, walk_short(K)>(list, total, first, lane,
                 [&](int n) __attribute__((always_inline)) { return Own{wrow[n], 0.f}; },
                 [&](int n, const Own& o) __attribute__((always_inline)) { const float2 v = caps(n, o.a); return fmaxf(v.x - LU, v.y - LL); },
                 load, use, use,
@@ -456,7 +456,7 @@ mc_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const 
                           return pass == 0 ? rowbits[c] : wkeep ? wkeep[(size_t)m * NCH + c] : ~0u;
                       },
                       [&](int total, bool first) __attribute__((always_inline)) {
-                walk_marks<POS, false, kSample>(list, total, first, lane,
+                walk_marks<POS, false, kSample, 0>(list, total, first, lane,
                     [&](int n) __attribute__((always_inline)) { return Own{wrow[n], 0.f}; },
                     [&](int n, const Own& o) __attribute__((always_inline)) { return caps(n, o.a).x; },
                     load, use, use,
@@ -573,7 +573,7 @@ sp_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const 
                 th = wave_min_nonneg(__builtin_bit_cast(float, min(in0 ? top[0][0] : none, in1 ? top[1][0] : none)));
             };
             listed = for_marks(list, NCH, lane, word, [&](int total, bool first) __attribute__((always_inline)) {
-                walk_marks<false, false, kSample>(list, total, first, lane, own, cap, load, value, value,
+                walk_marks<false, false, kSample, walk_short(K)>(list, total, first, lane, own, cap, load, value, value,
                                          [&](bool) __attribute__((always_inline)) { smallest(); }, keep, [] {});
             });
             smallest();
@@ -588,7 +588,7 @@ sp_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const 
             if (fabsf(xb[buf][i] - wi) >= least[1]) { noted[wave][min(cnt[1], kSlots - 1)][lane + 64] = (uint16_t)n; cnt[1]++; }
         };
         for_marks(list, NCH, lane, word, [&](int total, bool) __attribute__((always_inline)) {
-            walk_marks<true, false, kSample>(list, total, false, lane, own, cap, load, note, note, [](bool) {}, keep, [] {});
+            walk_marks<true, false, kSample, 0>(list, total, false, lane, own, cap, load, note, note, [](bool) {}, keep, [] {});
         }, listed);
         auto enter = [&](int j, float d, int n) __attribute__((always_inline)) {
             if (fabsf(d) > res[j][0] && fabsf(d) >= least[j]) topk_insert<K>(res[j], idx[j], fabsf(d), n | (d >= 0.f ? 0 : (int)kSign));
@@ -618,7 +618,7 @@ sp_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const 
                 enter(1, xb[buf][i] - wi, n);
             };
             for_marks(list, NCH, lane, word, [&](int total, bool) __attribute__((always_inline)) {
-                walk_marks<true, false, kSample>(list, total, false, lane, own, cap, load, ordered, ordered, [](bool) {}, keep, [] {});
+                walk_marks<true, false, kSample, 0>(list, total, false, lane, own, cap, load, ordered, ordered, [](bool) {}, keep, [] {});
             }, listed);
         }
     }
