@@ -31,7 +31,10 @@ constexpr int stream_waves(StreamOp op) { return op == kStreamSort ? 4 : 8; }
 
 // wavefronts per SIMD that the registers are to leave room for, and how many to count on (rows of up to 1024 inputs leave room for
 // twice as many; the staged ends of intervals leave room for fewer)
-constexpr int stream_occupancy(int NE, int NX, StreamOp op) { return NE == 48 && NX == 1 && op == kStreamSort ? 6 : NE <= 80 ? 4 : 2; }
+constexpr int stream_occupancy(int NE, int NX, StreamOp op, bool one = false, bool vec = true) {
+    if (one) return NE <= 16 ? 8 : NE == 48 ? (vec ? 8 : 6) : NE == 80 ? (vec ? 5 : 4) : 2;
+    return NE == 48 && NX == 1 && op == kStreamSort ? 6 : NE <= 80 ? 4 : 2;
+}
 constexpr int stream_resident(int NE, int NX, StreamOp op) {
     if (NE <= 16) return NX == 2 && op == kStreamPos ? 7 : 8;
     if (NX == 2 && op == kStreamSort && NE > 48) return NE <= 80 ? 3 : 1;
@@ -71,10 +74,13 @@ __device__ __forceinline__ void wave_fence() { __builtin_amdgcn_wave_barrier(); 
 // aligned), otherwise inputs 64 apart, so that loads coalesce either way.  grid.y: slices of the batch rows.
 // NX = 1: terms |x - w|.  NX = 2: interval bounds, terms -min(w - l, u - w) for the lower (side 0) and
 // max(w - l, u - w) for the upper result (side 1), inverted intervals repaired as everywhere.
-template <int NE, bool VEC, int NX, StreamOp OP>
-__global__ void __launch_bounds__(64 * stream_waves(OP), stream_occupancy(NE, NX, OP))
+// ONE: every workgroup meets one batch row (sort neuron, values): the terms take the place of the weights as these arrive, behind an
+// input row that is asked for before them.
+template <int NE, bool VEC, int NX, StreamOp OP, bool ONE>
+__global__ void __launch_bounds__(64 * stream_waves(OP), (stream_occupancy(NE, NX, OP, ONE, VEC)))
 row_stream_kernel(FwdArgs a, int K) {
     constexpr int NG = NE / 4, kWaves = stream_waves(OP);
+    static_assert(!ONE || (NX == 1 && OP == kStreamSort), "one set of terms per weight row");
     constexpr bool MASKABLE = NX == 1 && OP != kStreamSort;
     __shared__ __attribute__((aligned(16))) float xs[NX][NE * 64];
     __shared__ __attribute__((aligned(16))) float cand[OP == kStreamSort ? kWaves : 1][64];
@@ -96,11 +102,32 @@ row_stream_kernel(FwdArgs a, int K) {
                                          (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)wbits));
     const auto wrsrc = __builtin_amdgcn_make_buffer_rsrc(wuni, 0, 4 * CI, 0x00020000);
 
+    const int r_lo = (int)((long long)blockIdx.y * a.R / gridDim.y), r_hi = (int)((long long)(blockIdx.y + 1) * a.R / gridDim.y);
+    // ONE: the batch row is on its way before the weights, so that none of them has to have arrived when it is staged
+    constexpr int XV = ONE ? (NE + 4 * kWaves - 1) / (4 * kWaves) : 1;
+    float4 xfirst[XV];
+    if constexpr (ONE) {
+        #pragma unroll
+        for (int i = 0; i < XV; i++) {
+            const int n = 4 * (tid + 64 * kWaves * i);
+            const float* src = a.x0 + (size_t)(r_lo * a.G + g) * CI;
+            if (VEC) {
+                xfirst[i] = *reinterpret_cast<const float4*>(src + (n < CI ? n : 0));
+                if (n >= CI) xfirst[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+            } else
+                xfirst[i] = make_float4(n < CI ? src[n] : 0.f, n + 1 < CI ? src[n + 1] : 0.f, n + 2 < CI ? src[n + 2] : 0.f, n + 3 < CI ? src[n + 3] : 0.f);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+
     // inputs of group e of this lane: VEC: 4 (64 e + lane) + j, else 256 e + 64 j + lane; beyond the row x = w = 0
     float w[NG][4];
-    #pragma unroll
-    for (int e = 0; e < NG; e++) {
-        if (VEC) {
+    auto load_weights = [&](int e) {
+        if (VEC && ONE) {   // (one address for all groups)
+            const auto v = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, 16 * lane, 1024 * e, 0);
+            #pragma unroll
+            for (int j = 0; j < 4; j++) w[e][j] = __uint_as_float(v[j]);
+        } else if (VEC) {
             const int n = 4 * (64 * e + lane);
             const bool in = n < CI;
             const int nn = in ? n : 0;
@@ -116,14 +143,31 @@ row_stream_kernel(FwdArgs a, int K) {
                 if (wkeep && n < CI) w[e][j] = masked(w[e][j], wkeep, n);
             }
         }
-    }
+    };
     #pragma unroll
-    for (int k = 0; k < NX; k++)
-        for (int n = CI + tid; n < NE * 64; n += 64 * kWaves) xs[k][n] = 0.f;
+    for (int e = 0; e < NG - (ONE ? XV : 0); e++) load_weights(e);
+    if constexpr (ONE) {   // the last groups' weights take the registers that the input row came in
+        __builtin_amdgcn_sched_barrier(0);
+        #pragma unroll
+        for (int i = 0; i < XV; i++) {
+            const int n = 4 * (tid + 64 * kWaves * i);
+            if (NE % (4 * kWaves) == 0 || n < NE * 64) *reinterpret_cast<float4*>(&xs[0][n]) = xfirst[i];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        #pragma unroll
+        for (int e = NG - XV; e < NG; e++) load_weights(e);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (!ONE) {
+        #pragma unroll
+        for (int k = 0; k < NX; k++)
+            for (int n = CI + tid; n < NE * 64; n += 64 * kWaves) xs[k][n] = 0.f;
+    }
 
     // The staged rows stay in LDS between the passes: keeps the compiler from holding what one pass read in registers for
     // the next, and (every few groups) from starting a whole pass's reads at once
-    auto pass_fence = []() { asm volatile("" ::: "memory"); };
+    float zero = 0.f;   // (ONE: a value the compiler does not know, another one in every pass, so that no pass holds the maxima of the one before)
+    auto pass_fence = [&]() { asm volatile("" : "+v"(zero) : : "memory"); };
     auto group_fence = [](int e) {
         if (NX == 2 ? e % 2 == 1 : OP == kStreamSort && NE >= 48 && e % 4 == 3) { asm volatile("" ::: "memory"); __builtin_amdgcn_sched_barrier(0); }
     };
@@ -138,6 +182,11 @@ row_stream_kernel(FwdArgs a, int K) {
     };
     // terms of group e, and what bit 31 of a position says about each (only evaluated where it is used)
     auto terms = [&](int side, int e, float (&v)[4], bool (&flag)[4]) {
+        if constexpr (ONE) {
+            #pragma unroll
+            for (int j = 0; j < 4; j++) { v[j] = w[e][j]; flag[j] = false; }
+            return;
+        }
         float x[4], u[4];
         load4(xs[0], e, x);
         if (NX == 2) load4(xs[NX - 1], e, u);
@@ -158,12 +207,11 @@ row_stream_kernel(FwdArgs a, int K) {
         for (int k = 0; k < K; k++) { coef = lane == k ? rest : coef; rest *= 1.f - a.q; }
     }
 
-    const int r_lo = (int)((long long)blockIdx.y * a.R / gridDim.y), r_hi = (int)((long long)(blockIdx.y + 1) * a.R / gridDim.y);
-    for (int r = r_lo; r < r_hi; r++) {
+    for (int r = r_lo; r < (ONE ? r_lo + 1 : r_hi); r++) {
         const size_t xoff = (size_t)(r * a.G + g) * CI;
         const uint32_t* xkeep = MASKABLE && a.xmask ? a.xmask + (size_t)(r * a.G + g) * nchunks : nullptr;
         if (r > r_lo) __syncthreads();                 // every wavefront is done with the row before
-        for (int n = VEC ? 4 * tid : tid; n < CI; n += (VEC ? 4 : 1) * 64 * kWaves) {
+        for (int n = VEC ? 4 * tid : tid; !ONE && n < CI; n += (VEC ? 4 : 1) * 64 * kWaves) {
             constexpr int W = VEC ? 4 : 1;
             float x[W], u[W];
             if (VEC) {
@@ -185,6 +233,19 @@ row_stream_kernel(FwdArgs a, int K) {
             }
         }
         __syncthreads();
+        if constexpr (ONE) {
+            #pragma unroll
+            for (int e = 0; e < NG; e++) {
+                float x[4];
+                load4(xs[0], e, x);
+                #pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    w[e][j] = fabsf(x[j] - w[e][j]);
+                    asm volatile("" : "+v"(w[e][j]));   // the magnitude itself, not the difference and a modifier at each use
+                }
+                if (e % 2 == 1) { asm volatile("" ::: "memory"); __builtin_amdgcn_sched_barrier(0); }
+            }
+        }
 
         const size_t o = (size_t)(r * a.G + g) * a.COg + m;
         if (OP == kStreamMax) {
@@ -213,14 +274,20 @@ row_stream_kernel(FwdArgs a, int K) {
         }
         #pragma unroll
         for (int side = 0; side < NX; side++) {
-            float gm[NG], top = 0.f;                   // maxima per group and per lane (undefined terms never win)
+            float gm[ONE ? 1 : NG], top = 0.f;         // maxima per group and per lane (undefined terms never win)
+            // (ONE forms the maximum of a group from its terms again: 20 registers less, of which a fifth wavefront is made)
+            auto group_max = [&](int e) {
+                if constexpr (ONE) return fmaxf(fmaxf(fmaxf(fmaxf(zero, w[e][0]), w[e][1]), w[e][2]), w[e][3]);
+                else return gm[e];
+            };
             #pragma unroll
             for (int e = 0; e < NG; e++) {
                 float v[4];
                 bool flag[4];
                 terms(side, e, v, flag);
-                gm[e] = fmaxf(fmaxf(fmaxf(v[0], v[1]), v[2]), v[3]);
-                top = fmaxf(top, gm[e]);
+                const float most = fmaxf(fmaxf(fmaxf(v[0], v[1]), v[2]), v[3]);
+                if constexpr (!ONE) gm[e] = most;
+                top = fmaxf(top, most);
                 group_fence(e);
             }
             pass_fence();
@@ -232,7 +299,7 @@ row_stream_kernel(FwdArgs a, int K) {
                 // else the element before the lane
                 #pragma unroll
                 for (int e = 0; e < NG; e++) {
-                    if (found || __builtin_amdgcn_ballot_w64(gm[e] == top) == 0ull) continue;
+                    if (found || __builtin_amdgcn_ballot_w64(group_max(e) == top) == 0ull) continue;
                     found = true;
                     float v[4];
                     bool flag[4];
@@ -282,11 +349,11 @@ row_stream_kernel(FwdArgs a, int K) {
             int groups = 0, count = 0;                 // groups that reach T, more than 16 of them: not all of them kept
             #pragma unroll
             for (int e = 0; e < NG; e++) {
-                const unsigned long long any = __builtin_amdgcn_ballot_w64(gm[e] >= T);
+                const unsigned long long any = __builtin_amdgcn_ballot_w64(group_max(e) >= T);
                 if (any == 0ull) continue;
                 const int at = groups;
                 groups += __builtin_popcountll(any);
-                if (groups <= 16 && gm[e] >= T) {
+                if (groups <= 16 && group_max(e) >= T) {
                     float v[4];
                     bool flag[4];
                     terms(side, e, v, flag);
@@ -302,9 +369,10 @@ row_stream_kernel(FwdArgs a, int K) {
                 wave_fence();
                 if (v >= T) cand[wave][lanes_below(hit)] = v;
             } else {
+                if constexpr (ONE) pass_fence();
                 #pragma unroll
                 for (int e = 0; e < NG; e++) {
-                    if (__builtin_amdgcn_ballot_w64(gm[e] >= T) == 0ull) continue;
+                    if (__builtin_amdgcn_ballot_w64(group_max(e) >= T) == 0ull) continue;
                     float v[4];
                     bool flag[4];
                     terms(side, e, v, flag);
@@ -411,8 +479,19 @@ int launch(const FwdArgs& a, int K, hipStream_t stream) {
     const dim3 grid(tiles, (a.R + rows - 1) / rows), block(64 * kWaves);
     note_forward_kernel("row_stream_kernel", kWaves, NE);
     forward_kernel_timer(stream, false);
-    if (a.fast_x && a.fast_w) hipLaunchKernelGGL((row_stream_kernel<NE, true, NX, OP>), grid, block, 0, stream, a, K);
-    else hipLaunchKernelGGL((row_stream_kernel<NE, false, NX, OP>), grid, block, 0, stream, a, K);
+    const bool vec = a.fast_x && a.fast_w;
+    if constexpr (NX == 1 && OP == kStreamSort) {
+        // (up to four rounds of workgroups: in many more the selection, which forms the maxima again, weighs more than the loads. 1 x 640 x
+        // 20000 17.7 -> 15.4 us, x 200000 325 -> 333)
+        if (rows == 1 && tiles <= 4 * most) {
+            if (vec) hipLaunchKernelGGL((row_stream_kernel<NE, true, NX, OP, true>), grid, block, 0, stream, a, K);
+            else hipLaunchKernelGGL((row_stream_kernel<NE, false, NX, OP, true>), grid, block, 0, stream, a, K);
+            forward_kernel_timer(stream, true);
+            return check_launch("row_stream_kernel");
+        }
+    }
+    if (vec) hipLaunchKernelGGL((row_stream_kernel<NE, true, NX, OP, false>), grid, block, 0, stream, a, K);
+    else hipLaunchKernelGGL((row_stream_kernel<NE, false, NX, OP, false>), grid, block, 0, stream, a, K);
     forward_kernel_timer(stream, true);
     return check_launch("row_stream_kernel");
 }

@@ -113,6 +113,25 @@ def test_batch_rows_dealt_to_workgroups(oracle, B, n, m):
     np.testing.assert_allclose(y2.cpu().numpy(), ru.reshape(B, m, 1), rtol=1e-5, atol=1e-6)
 
 
+# one batch row per workgroup: the terms take the weights' registers.  Same products and sums as the kernels with positions, largest
+# first: the same bits.  (Few weight rows: several batch rows, each in a workgroup of its own; 16384 and more: more than one round.)
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("B,n,m", [(1, 255, 4), (1, 1023, 9), (1, 1024, 33), (1, 1025, 6), (1, 3071, 5), (1, 3072, 5), (1, 3076, 7), (1, 5119, 6),
+                                   (1, 5120, 1030), (1, 5121, 3), (1, 10239, 3), (1, 10240, 5), (9, 4100, 10), (33, 641, 3), (1, 60, 20001),
+                                   (1, 64, 33000)])
+def test_one_batch_row_has_the_same_bits(B, n, m, kind):
+    from sortnet_amd import _lib, ext
+    x, w = (t.cuda() for t in _data((B, n, m, 1), kind))
+    y, y2 = (torch.full((B, m, 1), float("nan"), device="cuda") for _ in range(2))
+    for K in (2, 10, 25):
+        pos = torch.empty(K, B, m, 1, device="cuda", dtype=torch.int32)
+        ext.sort_neuron_forward_nograd(x, w, y, 1, 0.6, K)
+        if m < 20000:
+            assert _lib.last_forward_kernel().startswith("row_stream_kernel")
+        ext.sort_neuron_forward(x, w, y2, pos, 1, 0.6, K)
+        assert np.array_equal(y.cpu().numpy(), y2.cpu().numpy(), equal_nan=True)
+
+
 @pytest.fixture
 def no_sort_tables():
     from sortnet_amd import _lib
