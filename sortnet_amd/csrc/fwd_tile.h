@@ -218,14 +218,22 @@ __global__ void __launch_bounds__(256, P::MIN_WAVES) fwd_kernel(FwdArgs a) {
 // least two wavefronts per SIMD have VALU work ready.
 // In the factored mask mode the keep bits come from bit-mask words built by build_masks_kernel
 // (one 32-bit word per row and chunk).
+// With narrow tiles the LDS reads bound it, beside them the vector instructions: 1.76 per term of the l-inf distance with positions at
+// 128 x 3072 x 1024 (1.5 in the step itself), 2.29 with 64-bit addresses, selects for rows and masks that are not there, and a loop over
+// the steps.  Before -> now, us: with positions 39.8 -> 37.4 in all there, without 27.7 -> 25.7, p = 8 48.9 -> 43.2, interval 78.9 -> 75.7;
+// class layer 256 x 10240 x 200 49.3 -> 47.0, p = 8 70.0 -> 62.2; lists (fwd_kernel_lists) 512 x 2048 x 2048 at p = 8 133 -> 122, at p = 24
+// 304 -> 294; convolution 128 x 2700 x 1024 x 4 102 -> 98.
 // -------------------------------------------------------------------------------------------
 // waves per SIMD the pipelined kernels are compiled for and the unroll factor of their inner loop: a policy may
 // name other values for register tiles of at most four channels per work-item (PIPE_WAVES_TM4, UNROLL4_TM4;
-// 0 = same)
+// 0 = same).  With NARROW_WAVES a tile of 2 x 2 outputs has the loop over a chunk unrolled whole (every LDS address a constant offset), two
+// steps at a time in the registers that so many wavefronts per SIMD leave.
 template <class P, int TB, int TM>
-constexpr int pipe_waves() { return (TM <= 4 && P::PIPE_WAVES_TM4) ? P::PIPE_WAVES_TM4 : P::PIPE_WAVES; }
+constexpr int pipe_waves() { return TB * TM <= 4 && P::NARROW_WAVES ? P::NARROW_WAVES : (TM <= 4 && P::PIPE_WAVES_TM4) ? P::PIPE_WAVES_TM4 : P::PIPE_WAVES; }
 template <class P, int TB, int TM>
-constexpr int pipe_unroll() { return (TM <= 4 && P::UNROLL4_TM4) ? P::UNROLL4_TM4 : P::UNROLL4; }
+constexpr bool lists_whole() { return TB * TM <= 4 && P::NARROW_WAVES && P::LISTS_WHOLE; }
+template <class P, int TB, int TM>
+constexpr int pipe_unroll() { return TB * TM <= 4 && P::NARROW_WAVES ? KT / 4 : (TM <= 4 && P::UNROLL4_TM4) ? P::UNROLL4_TM4 : P::UNROLL4; }
 
 template <class P, int TB, int TM>
 __global__ void __launch_bounds__(256, (pipe_waves<P, TB, TM>())) fwd_kernel_pipe(FwdArgs a) {
@@ -247,89 +255,93 @@ __global__ void __launch_bounds__(256, (pipe_waves<P, TB, TM>())) fwd_kernel_pip
     if (n_end > a.CIg) n_end = a.CIg;
 
     // staging slot v of a work-item: float4 number v * 256 + tid of a tile = row (tid >> 3) + 32 v,
-    // columns (tid & 7) * 4 .. +3.  Rows outside the tensor read row 0 of the tile's first valid
-    // row instead (always a legal address) and are zeroed afterwards.
+    // columns (tid & 7) * 4 .. +3.  Rows outside the tensor hold the tile's first row, whose results nothing stores.
+    // Byte offsets from uniform bases that move on with the chunks: a load costs no vector instruction (pipe_ok: they fit 32 bits).
     const int lrow = tid >> 3, lc4 = (tid & 7) * 4;
-    // 32-bit element offsets of the rows this work-item stages (pointers would cost twice the registers)
-    int xoff[NXV], woff[NWV], xmoff[NXV], wmoff[NWV];
-    uint32_t okbits = 0;   // bit v: x row v valid, bit 8 + v: w row v valid
+    const char* xbase0 = reinterpret_cast<const char*>(a.x0 + (size_t)(r0 * a.G + g) * a.CIg);
+    const char* xbase1 = NX == 2 ? reinterpret_cast<const char*>(a.x1 + (size_t)(r0 * a.G + g) * a.CIg) : xbase0;
+    const char* wbase = reinterpret_cast<const char*>(a.w + (size_t)(g * a.W_COg + (a.co_idx ? 0 : m0)) * a.W_CIg);
+    uint32_t xoff[NXV], woff[NWV];
+    int xmoff[NXV], wmoff[NWV];
     #pragma unroll
     for (int v = 0; v < NXV; v++) {
-        int row = lrow + 32 * v, r = r0 + row;
-        bool ok = row < BB && r < a.R;
-        int rr = ok ? r : r0;
-        okbits |= ok ? 1u << v : 0u;
-        xoff[v] = (rr * a.G + g) * a.CIg;
-        xmoff[v] = masked ? (rr * a.G + g) * nchunks : 0;
+        const int row = lrow + 32 * v, rr = row < BB && r0 + row < a.R ? row : 0;
+        xoff[v] = ((uint32_t)(rr * a.G) * (uint32_t)a.CIg + (uint32_t)lc4) * 4u;
+        xmoff[v] = masked ? ((r0 + rr) * a.G + g) * nchunks : 0;
     }
     #pragma unroll
     for (int v = 0; v < NWV; v++) {
-        int row = lrow + 32 * v, m = m0 + row;
-        bool ok = row < BM && m < a.COg;
-        int mm = ok ? m : m0;
-        okbits |= ok ? 1u << (8 + v) : 0u;
-        int wrow = a.co_idx ? a.co_idx[(s * a.G + g) * a.COg + mm] : mm;
-        woff[v] = (g * a.W_COg + wrow) * a.W_CIg;
-        wmoff[v] = masked ? (g * a.COg + mm) * nchunks : 0;
+        const int row = lrow + 32 * v, mm = row < BM && m0 + row < a.COg ? row : 0;
+        const int wrow = a.co_idx ? a.co_idx[(s * a.G + g) * a.COg + m0 + mm] : mm;
+        woff[v] = ((uint32_t)wrow * (uint32_t)a.W_CIg + (uint32_t)lc4) * 4u;
+        wmoff[v] = masked ? (g * a.COg + m0 + mm) * nchunks : 0;
     }
-    // unmasked: the mask pointers alias x and word 0 is read and ignored
-    const uint32_t* xmbase = masked ? a.xmask : reinterpret_cast<const uint32_t*>(a.x0);
-    const uint32_t* wmbase = masked ? a.wmask : reinterpret_cast<const uint32_t*>(a.x0);
-    const int mstep = masked ? 1 : 0;
 
     float4 px0[NXV], px1[NXV], pw[NWV];
     uint32_t mx[NXV], mw[NWV];
 
     auto gload = [&](int k0) {
-        int n = k0 + lc4;
-        if (n > a.CIg - 4) n = a.CIg - 4;     // keeps the address inside the row; zeroed in sstore()
-        #pragma unroll
-        for (int v = 0; v < NXV; v++) {
-            px0[v] = *reinterpret_cast<const float4*>(a.x0 + xoff[v] + n);
-            if (NX == 2) px1[v] = *reinterpret_cast<const float4*>(a.x1 + xoff[v] + n);
-            if (NX == 1) mx[v] = xmbase[xmoff[v] + (k0 / KT) * mstep];
+        const size_t at = (size_t)k0 * 4;
+        auto loads = [&](uint32_t back) {
+            #pragma unroll
+            for (int v = 0; v < NXV; v++) {
+                px0[v] = *reinterpret_cast<const float4*>(xbase0 + at + (xoff[v] - back));
+                if (NX == 2) px1[v] = *reinterpret_cast<const float4*>(xbase1 + at + (xoff[v] - back));
+            }
+            #pragma unroll
+            for (int v = 0; v < NWV; v++) pw[v] = *reinterpret_cast<const float4*>(wbase + at + (woff[v] - back));
+        };
+        if (NX == 1 && masked) {
+            #pragma unroll
+            for (int v = 0; v < NXV; v++) mx[v] = a.xmask[xmoff[v] + k0 / KT];
+            #pragma unroll
+            for (int v = 0; v < NWV; v++) mw[v] = a.wmask[wmoff[v] + k0 / KT];
         }
-        #pragma unroll
-        for (int v = 0; v < NWV; v++) {
-            pw[v] = *reinterpret_cast<const float4*>(a.w + woff[v] + n);
-            if (NX == 1) mw[v] = wmbase[wmoff[v] + (k0 / KT) * mstep];
-        }
+        if (k0 + KT <= n_end) loads(0u);
+        else loads(k0 + lc4 < n_end ? 0u : (uint32_t)lc4 * 4u);   // the chunk's first inputs instead of what lies behind the row; zeroed in sstore()
     };
-    auto fix = [&](float4& v, bool ok, uint32_t bits) {
-        const float qnan = __builtin_nanf("");
-        if (NX == 1) {
-            bits = masked ? bits >> lc4 : 0xfu;
-            v.x = (bits & 1u) ? v.x : qnan; v.y = (bits & 2u) ? v.y : qnan;
-            v.z = (bits & 4u) ? v.z : qnan; v.w = (bits & 8u) ? v.w : qnan;
-        }
-        v.x = ok ? v.x : 0.f; v.y = ok ? v.y : 0.f; v.z = ok ? v.z : 0.f; v.w = ok ? v.w : 0.f;
+    auto drop = [&](float4& v, uint32_t bits) {   // all bits of a dropped value are set: undefined
+        const uint32_t gone = ~(bits >> lc4);
+        auto one = [&](float& f, int k) { f = __uint_as_float(__float_as_uint(f) | (uint32_t)((int)(gone << (31 - k)) >> 31)); };
+        one(v.x, 0); one(v.y, 1); one(v.z, 2); one(v.w, 3);
     };
-    // writes the staged chunk k0 to LDS (zeroing what lies outside the tensor / the slice)
+    // writes the staged chunk k0 to LDS (zeroing what lies behind the row)
     auto sstore = [&](int k0) {
-        const bool in = k0 + lc4 < n_end;
-        #pragma unroll
-        for (int v = 0; v < NXV; v++) {
-            int row = lrow + 32 * v;
-            float4 l = px0[v], u = px1[v];
-            if (NX == 2) {
+        if (NX == 2) {
+            #pragma unroll
+            for (int v = 0; v < NXV; v++) {
+                float4 &l = px0[v], &u = px1[v];
                 if (l.x > u.x) l.x = u.x = (l.x + u.x) * 0.5f;
                 if (l.y > u.y) l.y = u.y = (l.y + u.y) * 0.5f;
                 if (l.z > u.z) l.z = u.z = (l.z + u.z) * 0.5f;
                 if (l.w > u.w) l.w = u.w = (l.w + u.w) * 0.5f;
-                fix(u, ((okbits >> v) & 1u) && in, 0u);
             }
-            fix(l, ((okbits >> v) & 1u) && in, NX == 1 ? mx[v] : 0u);
+        }
+        if (NX == 1 && masked) {
+            #pragma unroll
+            for (int v = 0; v < NXV; v++) drop(px0[v], mx[v]);
+            #pragma unroll
+            for (int v = 0; v < NWV; v++) drop(pw[v], mw[v]);
+        }
+        if (k0 + KT > n_end && k0 + lc4 >= n_end) {
+            const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+            #pragma unroll
+            for (int v = 0; v < NXV; v++) { px0[v] = zero; if (NX == 2) px1[v] = zero; }
+            #pragma unroll
+            for (int v = 0; v < NWV; v++) pw[v] = zero;
+        }
+        #pragma unroll
+        for (int v = 0; v < NXV; v++) {
+            const int row = lrow + 32 * v;
             if (NXV * 32 == BB || row < BB) {
-                *reinterpret_cast<float4*>(&xs[0][row][lc4]) = l;
-                if (NX == 2) *reinterpret_cast<float4*>(&xs[NX - 1][row][lc4]) = u;
+                *reinterpret_cast<float4*>(&xs[0][row][lc4]) = px0[v];
+                if (NX == 2) *reinterpret_cast<float4*>(&xs[NX - 1][row][lc4]) = px1[v];
             }
         }
         #pragma unroll
         for (int v = 0; v < NWV; v++) {
-            int row = lrow + 32 * v;
-            float4 t = pw[v];
-            fix(t, ((okbits >> (8 + v)) & 1u) && in, NX == 1 ? mw[v] : 0u);
-            if (NWV * 32 == BM || row < BM) *reinterpret_cast<float4*>(&ws[row][lc4]) = t;
+            const int row = lrow + 32 * v;
+            if (NWV * 32 == BM || row < BM) *reinterpret_cast<float4*>(&ws[row][lc4]) = pw[v];
         }
     };
 
@@ -363,6 +375,7 @@ __global__ void __launch_bounds__(256, (pipe_waves<P, TB, TM>())) fwd_kernel_pip
                     #pragma unroll
                     for (int j = 0; j < TM; j++) P::step4(acc[i][j], a, xl, xu, wv[j], k0 + n4, pass);
                 }
+                if (TB * TM <= 4 && P::NARROW_WAVES && n4 % (8 / NX) == 8 / NX - 4) __builtin_amdgcn_sched_barrier(0);
             }
             #pragma unroll
             for (int i = 0; i < TB; i++) {
@@ -391,7 +404,7 @@ __global__ void __launch_bounds__(256, (pipe_waves<P, TB, TM>())) fwd_kernel_pip
 // chunk k+1 (index, then the gathered weights) are in flight while chunk k is consumed.
 // -------------------------------------------------------------------------------------------
 template <class P, int TB, int TM>
-__global__ void __launch_bounds__(256, (pipe_waves<P, TB, TM>())) fwd_kernel_lists(FwdArgs a) {
+__global__ void __launch_bounds__(256, (lists_whole<P, TB, TM>() ? P::NARROW_WAVES : TM <= 4 && P::PIPE_WAVES_TM4 ? P::PIPE_WAVES_TM4 : P::PIPE_WAVES)) fwd_kernel_lists(FwdArgs a) {
     if constexpr (P::GATED) { if (gate_closed(a)) return; }
     static_assert(P::NX == 1 && KT == 32, "one input tile, 32 columns per chunk");
     constexpr int BB = 16 * TB, BM = 16 * TM;
@@ -409,44 +422,50 @@ __global__ void __launch_bounds__(256, (pipe_waves<P, TB, TM>())) fwd_kernel_lis
     int n_end = (int)((long long)(split + 1) * nchunks / a.nsplit) * KT;
     if (n_end > a.CIg) n_end = a.CIg;
 
+    // Rows outside the tensor hold the tile's first row, whose results nothing stores.  Byte offsets from uniform bases, which move on with
+    // the chunks where there is no index list (pipe_ok: they fit 32 bits)
     const int col = tid & 31, lrow = tid >> 5;
-    int xoff[NXR], woff[NWR];
-    uint32_t okx = 0u, okw = 0u;
+    const int b0 = r0 / a.HW;
+    const char* xbase = reinterpret_cast<const char*>(a.x0 + (size_t)(b0 * a.G + g) * a.CIg * a.HW);
+    const char* wbase = reinterpret_cast<const char*>(a.w + (size_t)(g * a.W_COg + (a.co_idx ? 0 : m0)) * a.W_CIg);
+    uint32_t xoff[NXR], woff[NWR];
     #pragma unroll
     for (int k = 0; k < NXR; k++) {
-        const int r = r0 + lrow + 8 * k;
-        const bool ok = r < a.R;
-        okx |= ok ? 1u << k : 0u;
-        const int rr = ok ? r : r0, b = rr / a.HW, hw = rr - b * a.HW;
-        xoff[k] = (b * a.G + g) * a.CIg * a.HW + hw;
-    }
-    #pragma unroll
-    for (int k = 0; k < NWR; k++) {
-        const int m = m0 + lrow + 8 * k;
-        const bool ok = m < a.COg;
-        okw |= ok ? 1u << k : 0u;
-        const int mm = ok ? m : m0;
-        const int wrow = a.co_idx ? a.co_idx[(s * a.G + g) * a.COg + mm] : mm;
-        woff[k] = (g * a.W_COg + wrow) * a.W_CIg;
+        const int r = r0 + lrow + 8 * k, rr = r < a.R ? r : r0, b = rr / a.HW, hw = rr - b * a.HW;
+        xoff[k] = (((uint32_t)((b - b0) * a.G) * (uint32_t)a.CIg + (uint32_t)col) * (uint32_t)a.HW + (uint32_t)hw) * 4u;
     }
     const int* cidx = a.ci_idx ? a.ci_idx + (size_t)(s * a.G + g) * a.CIg : nullptr;
+    #pragma unroll
+    for (int k = 0; k < NWR; k++) {
+        const int m = lrow + 8 * k, mm = m0 + m < a.COg ? m : 0;
+        const int wrow = a.co_idx ? a.co_idx[(s * a.G + g) * a.COg + m0 + mm] : mm;
+        woff[k] = ((uint32_t)wrow * (uint32_t)a.W_CIg + (cidx ? 0u : (uint32_t)col)) * 4u;
+    }
 
     float px[NXR], pw[NWR];
     auto gload = [&](int k0) {
-        int n = k0 + col;
-        if (n >= n_end) n = n_begin;                  // a legal column; zeroed in sstore()
-        const int wcol = cidx ? cidx[n] : n;
-        #pragma unroll
-        for (int k = 0; k < NXR; k++) px[k] = a.x0[xoff[k] + n * a.HW];
-        #pragma unroll
-        for (int k = 0; k < NWR; k++) pw[k] = a.w[woff[k] + wcol];
+        const size_t atx = (size_t)k0 * a.HW * 4, atw = cidx ? 0 : (size_t)k0 * 4;
+        auto loads = [&](uint32_t back) {   // columns from this one to the chunk's first, which is there
+            const uint32_t wcol = cidx ? (uint32_t)cidx[k0 + col - (int)back] : 0u - back, xback = back * (uint32_t)a.HW * 4u;
+            #pragma unroll
+            for (int k = 0; k < NXR; k++) px[k] = *reinterpret_cast<const float*>(xbase + atx + (xoff[k] - xback));
+            #pragma unroll
+            for (int k = 0; k < NWR; k++) pw[k] = *reinterpret_cast<const float*>(wbase + atw + (woff[k] + wcol * 4u));
+        };
+        if (k0 + KT <= n_end) loads(0u);
+        else loads(k0 + col < n_end ? 0u : (uint32_t)col);   // zeroed in sstore()
     };
     auto sstore = [&](int k0) {
-        const bool in = k0 + col < n_end;
+        if (k0 + KT > n_end && k0 + col >= n_end) {
+            #pragma unroll
+            for (int k = 0; k < NXR; k++) px[k] = 0.f;
+            #pragma unroll
+            for (int k = 0; k < NWR; k++) pw[k] = 0.f;
+        }
         #pragma unroll
-        for (int k = 0; k < NXR; k++) xs[lrow + 8 * k][col] = (in && ((okx >> k) & 1u)) ? px[k] : 0.f;
+        for (int k = 0; k < NXR; k++) xs[lrow + 8 * k][col] = px[k];
         #pragma unroll
-        for (int k = 0; k < NWR; k++) ws[lrow + 8 * k][col] = (in && ((okw >> k) & 1u)) ? pw[k] : 0.f;
+        for (int k = 0; k < NWR; k++) ws[lrow + 8 * k][col] = pw[k];
     };
 
     typename P::Acc acc[TB][TM];
@@ -468,7 +487,7 @@ __global__ void __launch_bounds__(256, (pipe_waves<P, TB, TM>())) fwd_kernel_lis
         if (k0 + KT < n_end) gload(k0 + KT);
         #pragma unroll
         for (int pass = 0; pass < P::PASSES; pass++) {
-            #pragma unroll (pipe_unroll<P, TB, TM>())
+            #pragma unroll (lists_whole<P, TB, TM>() ? KT / 4 : TM <= 4 && P::UNROLL4_TM4 ? P::UNROLL4_TM4 : P::UNROLL4)
             for (int n4 = 0; n4 < KT; n4 += 4) {
                 float4 wv[TM];
                 #pragma unroll
@@ -479,6 +498,7 @@ __global__ void __launch_bounds__(256, (pipe_waves<P, TB, TM>())) fwd_kernel_lis
                     #pragma unroll
                     for (int j = 0; j < TM; j++) P::step4(acc[i][j], a, xl, xl, wv[j], k0 + n4, pass);
                 }
+                if (lists_whole<P, TB, TM>() && n4 % 8 == 4) __builtin_amdgcn_sched_barrier(0);
             }
             #pragma unroll
             for (int i = 0; i < TB; i++) {
@@ -506,6 +526,14 @@ __global__ void __launch_bounds__(256, (pipe_waves<P, TB, TM>())) fwd_kernel_lis
 #include "fwd_direct.h"
 namespace sd {
 
+// whether the byte offsets of a tile's rows from its bases fit 32 bits (rows of the weights anywhere with an index list of outputs): rows of
+// up to 31 million inputs on narrow tiles.  Longer ones take the kernel that forms whole addresses and loads a chunk when the one before it is done.
+template <int BB, int BM>
+bool pipe_ok(const FwdArgs& a) {
+    const long long most = (1ll << 32) / 4 - KT, samples = BB / a.HW + 2;
+    return samples * a.G * a.CIg * a.HW <= most && (long long)(a.co_idx ? a.W_COg : BM) * a.W_CIg <= most;
+}
+
 // host-side launcher; the caller has validated shapes
 template <class P, int TB, int TM>
 int launch_fwd_kernel(const FwdArgs& a, hipStream_t stream) {
@@ -514,13 +542,14 @@ int launch_fwd_kernel(const FwdArgs& a, hipStream_t stream) {
         if (direct_ok<TB, TM, P::MASKABLE>(a)) return launch_fwd_direct<P, TB, TM>(a, stream);
     }
     dim3 grid((a.COg + 16 * TM - 1) / (16 * TM), (a.R + 16 * TB - 1) / (16 * TB), a.G * a.nsplit);
-    if (a.fast_x && a.fast_w && (a.mask_mode != SD_MASK_FACTORED || a.xmask)) {
+    const bool offsets = pipe_ok<16 * TB, 16 * TM>(a);
+    if (offsets && a.fast_x && a.fast_w && (a.mask_mode != SD_MASK_FACTORED || a.xmask)) {
         note_forward_kernel("fwd_kernel_pipe", TB, TM);
         hipLaunchKernelGGL((fwd_kernel_pipe<P, TB, TM>), grid, dim3(256), 0, stream, a);
         return check_launch("fwd_kernel");
     }
     if constexpr (P::LISTS && TB == 2) {
-        if (a.mask_mode != SD_MASK_FACTORED) {
+        if (offsets && a.mask_mode != SD_MASK_FACTORED) {
             note_forward_kernel("fwd_kernel_lists", TB, TM);
             hipLaunchKernelGGL((fwd_kernel_lists<P, TB, TM>), grid, dim3(256), 0, stream, a);
             return check_launch("fwd_kernel");
@@ -549,6 +578,8 @@ struct PolicyBase {
     static constexpr int PIPE_WAVES = 2;  // same for the pipelined kernel
     static constexpr int UNROLL4 = 2;     // unroll factor of the loop over groups of four inputs
     static constexpr int PIPE_WAVES_TM4 = 0, UNROLL4_TM4 = 0;   // overrides for tiles of <= 4 channels (0: none)
+    static constexpr int NARROW_WAVES = 0;   // see pipe_unroll
+    static constexpr bool LISTS_WHOLE = true;   // the same in fwd_kernel_lists
     static constexpr int WIDE_TB = 4, WIDE_TM = 8;   // register tile of the large-batch launch of position kernels
     static constexpr bool LISTS = false;  // also built as fwd_kernel_lists (ops that accept kept-channel index lists)
     static constexpr bool DIRECT = false; // also built as fwd_kernel_direct (global -> LDS loads, exact dense tiles)
@@ -565,6 +596,7 @@ struct PolicyBase {
 
 // l-inf forward without indices (core/cuda/inf_dist_cuda.cu:17-107)
 struct LinfNograd : PolicyBase {
+    static constexpr int NARROW_WAVES = 6;
     static constexpr bool GATED = true;   // one of two queued for a result when FwdArgs::gate is set
     static constexpr bool LISTS = true;
     static constexpr bool DIRECT = true;
@@ -613,6 +645,8 @@ __device__ __forceinline__ void store_chunk_winner(const FwdArgs& a, size_t o, f
 }
 
 struct LinfChunk : PolicyBase {
+    static constexpr int NARROW_WAVES = 8;
+    static constexpr bool LISTS_WHOLE = false;   // (lists, 64 x 300 x 300: 11.7 us, whole 12.3; convolutions of 128 x 2700 x 1024 x 4 the same)
     static constexpr bool GATED = true;   // one of two queued for a result when FwdArgs::gate is set
     static constexpr bool LISTS = true;
     static constexpr int PIPE_WAVES = 2;   // three accumulator registers per output: 2 x 8 outputs leave no room for more
@@ -738,6 +772,7 @@ struct MaskedTermMax : PolicyBase {
 
 // interval bounds, values only (core/cuda/bound_inf_dist_cuda.cu:15-118)
 struct BoundNograd : PolicyBase {
+    static constexpr int NARROW_WAVES = 6;
     static constexpr bool DIRECT = true;
     static constexpr int PIPE_WAVES = 3;
     static constexpr int NX = 2;
@@ -771,6 +806,7 @@ struct BoundNogradGated : BoundNograd {
 // -min(t1,t2) (a positive number once it passes 1e-10), the upper side the largest max(t1,t2);
 // resolve_bound_kernel recovers the exact positions and branch bits
 struct BoundChunk : PolicyBase {
+    static constexpr int NARROW_WAVES = 6;
     static constexpr bool GATED = true;   // one of two queued for a result when FwdArgs::gate is set
     static constexpr int NX = 2;
     static constexpr int PIPE_WAVES = 2;
@@ -1065,6 +1101,7 @@ __device__ __forceinline__ float add_pow(float s, float a, float p) {
 // p <= 10: y = max(sum |d|^p, FLT_MIN)^(1/p)   (core/cuda/norm_dist_cuda.cu:163-259, no max)
 template <int IP>
 struct LpPlain : PolicyBase {
+    static constexpr int NARROW_WAVES = 8;
     static constexpr bool LISTS = true;
     static constexpr bool DIRECT = true;
     static constexpr int PIPE_WAVES = 3;
@@ -1146,6 +1183,7 @@ struct LpOnline : PolicyBase {
 // general-p forward, whose first step is the l-inf kernel
 template <int IP, bool FOLD = (IP < 0)>
 struct LpWithMax : PolicyBase {
+    static constexpr int NARROW_WAVES = 6;
     static constexpr bool LISTS = true;
     static constexpr bool DIRECT = true;
     static constexpr bool GATED = true;
