@@ -57,6 +57,10 @@ struct FwdArgs {
     float p, inv_p, q;
     const float* shift;   // vector added to the finished values, one entry per output channel, times shift_sign (+1 or -1); or null
     float shift_sign;
+    int sample;           // above 1: of every slice of the reduction range only this part (l-inf as a scale, see lp_forward_max_first)
+    uint32_t* redo;       // l-p relative to a scale: one word per tile of outputs, set to 1 where a sum is not finite (null: not asked for)
+    const uint32_t* only; // not null: gated policies run on the tiles whose word is set
+    int pow2_scale;       // the scale is aux rounded up to a power of two
     float skip_thr;       // l-p, large p: ratios to the running scale below this cannot change the fp32 result (0 = unused)
     uint32_t seed, t8, t16;
     int mask_mode;        // -1 none, SD_MASK_TERM, SD_MASK_FACTORED
@@ -88,6 +92,7 @@ __device__ __forceinline__ bool gate_closed(const unsigned long long* gate, unsi
 
 // the same for a forward tile kernel, whose first work-item reports the outcome (nothing is reported without a gate)
 __device__ __forceinline__ bool gate_closed(const FwdArgs& a) {
+    if (a.only && a.only[((blockIdx.z % a.G) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] == 0u) return true;
     if (a.gate == nullptr) return false;
     const bool closed = gate_closed(a.gate, a.gate_limit, a.gate_above);
     if ((a.told || a.told2 || a.told3) && threadIdx.x == 0 && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) {
@@ -97,6 +102,9 @@ __device__ __forceinline__ bool gate_closed(const FwdArgs& a) {
     }
     return closed;
 }
+
+// v > 0 rounded up to a power of two (infinite where there is none)
+__device__ __forceinline__ float pow2_above(float v) { return __uint_as_float((__float_as_uint(v) + 0x7fffffu) & 0x7f800000u); }
 
 // ---- error reporting ---------------------------------------------------------------------------
 void set_error(const char* fmt, ...);

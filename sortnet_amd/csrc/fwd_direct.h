@@ -64,7 +64,8 @@ __global__ void __launch_bounds__(256, 4) fwd_kernel_direct(FwdArgs a) {
 
     const int nchunks = a.CIg / KT;
     const int n_begin = (int)((long long)split * nchunks / a.nsplit) * KT;
-    const int n_end = (int)((long long)(split + 1) * nchunks / a.nsplit) * KT;
+    int n_end = (int)((long long)(split + 1) * nchunks / a.nsplit) * KT;
+    if constexpr (P::SAMPLED) n_end = sampled_end(a, n_begin, n_end);
 
     // Loads of this wave (GPW per chunk, the same number for every wave).  One x tile: x groups wave + 4 u, then
     // w groups wave + 4 u.  Interval policies repair inverted intervals in LDS before the chunk is published, which

@@ -137,6 +137,13 @@ __device__ __forceinline__ void load_w_tile(float (*ws)[LDP], const FwdArgs& a,
 // -------------------------------------------------------------------------------------------
 // the kernel
 // -------------------------------------------------------------------------------------------
+// end of the part of a slice that FwdArgs::sample asks for: whole chunks, at least one
+__device__ __forceinline__ int sampled_end(const FwdArgs& a, int n_begin, int n_end) {
+    if (a.sample <= 1) return n_end;
+    const int end = n_begin + ((n_end - n_begin + a.sample * KT - 1) / (a.sample * KT)) * KT;
+    return end < n_end ? end : n_end;
+}
+
 template <class P, int TB, int TM>
 __global__ void __launch_bounds__(256, P::MIN_WAVES) fwd_kernel(FwdArgs a) {
     if constexpr (P::GATED) { if (gate_closed(a)) return; }
@@ -153,6 +160,7 @@ __global__ void __launch_bounds__(256, P::MIN_WAVES) fwd_kernel(FwdArgs a) {
     const int n_begin = (int)((long long)split * nchunks / a.nsplit) * KT;
     int n_end = (int)((long long)(split + 1) * nchunks / a.nsplit) * KT;
     if (n_end > a.CIg) n_end = a.CIg;
+    if constexpr (P::SAMPLED) n_end = sampled_end(a, n_begin, n_end);
 
     typename P::Acc acc[TB][TM];
     #pragma unroll
@@ -253,6 +261,7 @@ __global__ void __launch_bounds__(256, (pipe_waves<P, TB, TM>())) fwd_kernel_pip
     const int n_begin = (int)((long long)split * nchunks / a.nsplit) * KT;
     int n_end = (int)((long long)(split + 1) * nchunks / a.nsplit) * KT;
     if (n_end > a.CIg) n_end = a.CIg;
+    if constexpr (P::SAMPLED) n_end = sampled_end(a, n_begin, n_end);
 
     // staging slot v of a work-item: float4 number v * 256 + tid of a tile = row (tid >> 3) + 32 v,
     // columns (tid & 7) * 4 .. +3.  Rows outside the tensor hold the tile's first row, whose results nothing stores.
@@ -421,6 +430,7 @@ __global__ void __launch_bounds__(256, (lists_whole<P, TB, TM>() ? P::NARROW_WAV
     const int n_begin = (int)((long long)split * nchunks / a.nsplit) * KT;
     int n_end = (int)((long long)(split + 1) * nchunks / a.nsplit) * KT;
     if (n_end > a.CIg) n_end = a.CIg;
+    if constexpr (P::SAMPLED) n_end = sampled_end(a, n_begin, n_end);
 
     // Rows outside the tensor hold the tile's first row, whose results nothing stores.  Byte offsets from uniform bases, which move on with
     // the chunks where there is no index list (pipe_ok: they fit 32 bits)
@@ -581,6 +591,7 @@ struct PolicyBase {
     static constexpr int NARROW_WAVES = 0;   // see pipe_unroll
     static constexpr bool LISTS_WHOLE = true;   // the same in fwd_kernel_lists
     static constexpr int WIDE_TB = 4, WIDE_TM = 8;   // register tile of the large-batch launch of position kernels
+    static constexpr bool SAMPLED = false;   // the kernels honour FwdArgs::sample
     static constexpr bool LISTS = false;  // also built as fwd_kernel_lists (ops that accept kept-channel index lists)
     static constexpr bool DIRECT = false; // also built as fwd_kernel_direct (global -> LDS loads, exact dense tiles)
     static constexpr bool MASKABLE = false;  // fwd_kernel_direct is also built with the factored mask patched into LDS
@@ -596,6 +607,7 @@ struct PolicyBase {
 
 // l-inf forward without indices (core/cuda/inf_dist_cuda.cu:17-107)
 struct LinfNograd : PolicyBase {
+    static constexpr bool SAMPLED = true;
     static constexpr int NARROW_WAVES = 6;
     static constexpr bool GATED = true;   // one of two queued for a result when FwdArgs::gate is set
     static constexpr bool LISTS = true;
@@ -1194,7 +1206,7 @@ struct LpWithMax : PolicyBase {
     // log2|d|, about 2.5e-7 absolute, reaches y divided by p times p, i.e. unchanged: far inside the 1e-5 bar)
     struct Acc { float s, rinv; };
     static __device__ __forceinline__ void init(Acc& A, const FwdArgs& a, size_t o, bool valid, int split = 0) {
-        const float rinv = valid ? 1.f / a.aux[o] : 1.f;
+        const float rinv = valid ? 1.f / (FOLD && a.pow2_scale ? pow2_above(a.aux[o]) : a.aux[o]) : 1.f;
         // the virtual term of size 1e-10 belongs to slice 0 only
         A.s = split == 0 ? __builtin_amdgcn_exp2f(a.p * __builtin_amdgcn_logf(kEps * rinv)) : 0.f;
         A.rinv = FOLD ? a.p * __builtin_amdgcn_logf(rinv) : rinv;
@@ -1212,7 +1224,10 @@ struct LpWithMax : PolicyBase {
     }
     static __device__ __forceinline__ void store(Acc& A, const FwdArgs& a, size_t o, int split = 0) {
         if (a.nsplit > 1) a.part0[(size_t)split * a.part_stride + o] = A.s;   // merged by lp_finalize_kernel
-        else a.y0[o] = powf(A.s, a.inv_p) * a.aux[o];
+        else {
+            a.y0[o] = powf(A.s, a.inv_p) * (FOLD && a.pow2_scale ? pow2_above(a.aux[o]) : a.aux[o]);
+            if (FOLD && a.redo && !(A.s <= FLT_MAX)) a.redo[((blockIdx.z % a.G) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = 1u;
+        }
     }
 };
 
