@@ -57,6 +57,81 @@ __global__ void __launch_bounds__(1024) channel_mean_kernel(const float* __restr
     }
 }
 
+// Both in one launch for up to 512 samples and 1, 4, 8 .. 64 positions: a workgroup owns 64 neighbouring values of a sample (64 / HW channels),
+// its wavefronts keep every 16th sample in registers, and the values leave again with the mean subtracted.  Two launches were bound
+// by the launches and, with positions, by reading one channel at a time (16 bytes of a cache line at HW = 4).  The order of the sums is
+// that of the kernel above, so the bits are: with positions, where its 1024 work-items took every 1024th value of a channel and one added
+// their sums up, the sums of `span` = 1024 / HW samples lie in LDS for one lane per channel to add.  Two launches -> one, us of the device (the
+// host has a launch of 3 us less): 512 x 5120 9.3 -> 6.3, 128 x 1024 8.1 -> 4.7, with 4 positions 10.0 -> 7.7, 512 x 5120 x 4 72.6 -> 31.5.
+constexpr int kShiftRows = 32;   // samples of a wavefront
+template <int ROWS, bool POSITIONS>
+__global__ void __launch_bounds__(1024) channel_mean_shift_kernel(const float* x, int B, int cols, int HW, float* __restrict__ mean,
+                                                                  float* __restrict__ running, float momentum, float* y) {   // (y may be x)
+    extern __shared__ __attribute__((aligned(16))) float part[];   // [16 or min(B, span)][64]
+    __shared__ float shift[64];
+    const int lane = threadIdx.x & 63, grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = blockIdx.x * 64 + lane, span = POSITIONS ? 1024 / HW : 16;
+    const bool ok = col < cols;
+    const float* src = x + (ok ? col : 0);
+    float v[ROWS];
+    #pragma unroll
+    for (int k = 0; k < ROWS; k++) {
+        const int b = grp + 16 * k;
+        v[k] = src[(size_t)(b < B ? b : B - 1) * cols];
+    }
+    if constexpr (POSITIONS) {   // (the samples of a sum are all this wavefront's: span is a multiple of 16)
+        #pragma unroll
+        for (int k = 0; k < ROWS; k++) {
+            const int b = grp + 16 * k;
+            if (b < B) {
+                float* sum = part + (b & (span - 1)) * 64 + lane;
+                *sum = (b < span ? 0.f : *sum) + v[k];
+            }
+        }
+    } else {
+        float s = 0.f;
+        #pragma unroll
+        for (int k = 0; k < ROWS; k++) s += grp + 16 * k < B ? v[k] : 0.f;
+        part[grp * 64 + lane] = s;
+    }
+    __syncthreads();
+    if (grp == 0) {
+        float t = 0.f;
+        const int c = POSITIONS ? (int)(blockIdx.x * 64) / HW + lane : col;
+        const bool mine = POSITIONS ? lane < 64 / HW && c * HW < cols : ok;
+        if constexpr (POSITIONS) {
+            if (mine) {
+                const int rows = B < span ? B : span;
+                const float* own = part + lane * HW;
+                const int steps = __builtin_ctz(HW) - 2;   // of four positions: 2^steps to a sample
+                #pragma unroll 8
+                for (int i = 0; i < rows << steps; i++) {
+                    const float4 e = *reinterpret_cast<const float4*>(own + (i >> steps) * 64 + 4 * (i & ((1 << steps) - 1)));
+                    t += e.x; t += e.y; t += e.z; t += e.w;
+                }
+            }
+        } else {
+            #pragma unroll
+            for (int k = 0; k < 16; k++) t += part[k * 64 + lane];
+        }
+        const float m = t / (float)((uint32_t)B * (uint32_t)HW);
+        if constexpr (POSITIONS) { if (mine) for (int h = 0; h < HW; h++) shift[lane * HW + h] = m; }
+        else shift[lane] = m;
+        if (mine) {
+            mean[c] = m;
+            if (running) running[c] = (1.f - momentum) * running[c] + momentum * m;
+        }
+    }
+    __syncthreads();
+    if (!ok) return;
+    const float m = shift[lane];
+    #pragma unroll
+    for (int k = 0; k < ROWS; k++) {
+        const int b = grp + 16 * k;
+        if (b < B) y[(size_t)b * cols + col] = v[k] - m;
+    }
+}
+
 __global__ void __launch_bounds__(256) channel_shift_kernel(const float* x, const float* __restrict__ shift,
                                                             long long total, int C, int HW, float sign,
                                                             float* y, float* both) {   // (y may be x; grid.y = 2: `both` in place, too)
@@ -255,6 +330,19 @@ extern "C" int sd_mean_shift_forward(const float* input, int B, int C, int HW, f
     SD_REQUIRE(reinterpret_cast<uintptr_t>(input) % 16 == 0 && reinterpret_cast<uintptr_t>(output) % 16 == 0 &&
                reinterpret_cast<uintptr_t>(mean) % 16 == 0, "mean_shift_forward: buffers must be 16-byte aligned");
     hipStream_t st = static_cast<hipStream_t>(stream);
+    // With positions the chain of one lane's additions bounds small layers (256 x 512 x 4 11.6 us in two launches, 12.8 in one; 129 x 64 x 16 10.5,
+    // 12.1): up to 512 values of a channel, or tensors whose second reading costs more (512 x 1000 x 4 21.9 -> 15.3)
+    const bool positions = HW >= 4 && HW <= 64 && (HW & (HW - 1)) == 0 && (B * HW <= 512 || (long long)B * C * HW >= 1ll << 20);
+    if (B <= 16 * kShiftRows && (HW == 1 || positions)) {
+        const int cols = C * HW, span = 1024 / HW;
+        const dim3 blocks((cols + 63) / 64), threads(1024);
+        const size_t lds = (size_t)(HW == 1 ? 16 : B < span ? B : span) * 64 * sizeof(float);
+        if (HW == 1 && B <= 128) hipLaunchKernelGGL((channel_mean_shift_kernel<8, false>), blocks, threads, lds, st, input, B, cols, HW, mean, running_mean, momentum, output);
+        else if (HW == 1) hipLaunchKernelGGL((channel_mean_shift_kernel<kShiftRows, false>), blocks, threads, lds, st, input, B, cols, HW, mean, running_mean, momentum, output);
+        else if (B <= 128) hipLaunchKernelGGL((channel_mean_shift_kernel<8, true>), blocks, threads, lds, st, input, B, cols, HW, mean, running_mean, momentum, output);
+        else hipLaunchKernelGGL((channel_mean_shift_kernel<kShiftRows, true>), blocks, threads, lds, st, input, B, cols, HW, mean, running_mean, momentum, output);
+        return check_launch("channel_mean_shift_kernel");
+    }
     dim3 grid(HW == 1 ? (C + 63) / 64 : C);
     hipLaunchKernelGGL(channel_mean_kernel, grid, dim3(1024), 0, st, input, B, C, HW, mean, running_mean, momentum);
     if ((rc = check_launch("channel_mean_kernel"))) return rc;
