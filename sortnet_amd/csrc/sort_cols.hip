@@ -188,13 +188,14 @@ __device__ __forceinline__ bool table_pointless(const float2* __restrict__ width
     return __builtin_amdgcn_readfirstlane(bw > kProbeRatio * (float)S * ww ? 1 : 0) != 0;
 }
 
-// Bounds and marks (cand_tables.h); J = 0: rows of any length
-template <int J, int R, int NT, bool TWO, bool MASK>
+// Bounds and marks (cand_tables.h); J = 0: rows of any length.  SPARE: tables that may not be needed, see `unless` (a form of its own: the
+// test alone took the others from 28.2 to 29.3 us at 128 x 5120 x 5120)
+template <int J, int R, int NT, bool TWO, bool MASK, bool SPARE>
 __global__ void __launch_bounds__(64 * (J ? kStreamWaves : kTableWaves))
 sc_tables_kernel(TableArgs a, const float2* __restrict__ widths, TableCount* __restrict__ c, unsigned long long limit,
                  const unsigned long long* __restrict__ unless) {
     extern __shared__ __attribute__((aligned(16))) float smem[];
-    if (unless != nullptr && unless[1] == 0ull) {   // not needed: no kernel of this table, none that forms every term, and none of the other orientation
+    if (SPARE && unless[1] == 0ull) {   // not needed: no kernel of this table, none that forms every term, and none of the other orientation
         if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) { c->marks = ~0ull; c->above = 0ull; c->stat[0] = c->stat[1] = 0.f; }
         return;
     }
@@ -220,7 +221,8 @@ int launch_tables(const TableArgs& t, const Carve& c, unsigned long long limit, 
         block.x = 64 * s.waves;
         lds = stream_lds(s.waves, R * NT * (TWO ? 2 : 1));
     }
-    hipLaunchKernelGGL((sc_tables_kernel<J, R, NT, TWO, MASK>), grid, block, lds, st, t, c.widths, c.count, limit, unless);
+    if (!MASK && unless != nullptr) hipLaunchKernelGGL((sc_tables_kernel<J, R, NT, TWO, MASK, !MASK>), grid, block, lds, st, t, c.widths, c.count, limit, unless);
+    else hipLaunchKernelGGL((sc_tables_kernel<J, R, NT, TWO, MASK, false>), grid, block, lds, st, t, c.widths, c.count, limit, nullptr);
     return check_launch("sc_tables_kernel");
 }
 // As many batch tiles at a time as there are, up to four, and as the registers hold ranges of (64 per lane).
