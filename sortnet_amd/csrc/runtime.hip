@@ -246,7 +246,8 @@ bool hint_build_spare(int site, const void* weight, int B, int CO, int CI, hipSt
 
 bool hint_paid(int site, const void* weight, int B, int CO, int CI) {
     std::lock_guard<std::mutex> lock(g_hint_mu);
-    const HintSlot* h = hint_slot(site, weight, B, CO, CI, false);
+    HintSlot* h = hint_slot(site, weight, B, CO, CI, false);
+    if (h) hint_drain(*h);
     return h && h->known && h->streak == 0;
 }
 

@@ -211,6 +211,7 @@ struct SortBox {
     char* rest;             // workspace of the two forms, one after the other
     const float* layer;     // the weights as the caller has them, which the hints know the layer by
     bool own;
+    bool own_tables(int form) const { return own && form == kRowsSortValues; }
 };
 
 // `ws`: sort_tables_bytes() bytes.  The gate it leaves in `a` points into `ws`: the kernels queued behind it must
@@ -218,7 +219,8 @@ struct SortBox {
 // per call, carved by the caller).  Afterwards a.gate[0] is non-zero when the every-term kernels are to run.
 // A layer that the tables per weight row serve queues those per batch row in vain, three kernels that return at once (4.6 us each): where
 // they ran in none of three calls they are left out of the next 31, unless the call before formed every term (hint_build_spare;
-// evaluation pass of 6 x 5120 at batch 512 1636 -> 1575 us, attack on 128 x 5120 x 5120 225 -> 215).  `site`, `layer`: see sort_cols_ok.
+// evaluation pass of 6 x 5120 at batch 512 1636 -> 1575 us, attack on 128 x 5120 x 5120 225 -> 215).  `site`, `layer`: see sort_cols_ok;
+// with a box it is the shared table that serves, or the values' own one beside it, and `site` hears only of tables that the call builds.
 static int queue_sort_cols(FwdArgs& a, int site, const float* layer, int form, const float* xl, const float* xu, const float* w, int B, int CO, int CI,
                            float q, int K, float* outL, float* outU, int* pos, void* ws, const SortBox* box, hipStream_t st) {
     const float density = g_sort_density.load(std::memory_order_relaxed);
@@ -228,12 +230,16 @@ static int queue_sort_cols(FwdArgs& a, int site, const float* layer, int form, c
         a.gate = box->count;
         a.gate_limit = box->limit;
     }
-    if (!rc && (!box || (box->own && form == kRowsSortValues)))
+    if (!rc && (!box || box->own_tables(form)))
         rc = sort_cols_forward(xl, xu, w, B, CO, CI, q, K, outL, outU, pos, ws, cap, &a.gate, &a.gate_limit, st, a.shift, a.shift_sign, box ? box->count : nullptr);
     a.gate_above = 1;
     const long long terms = (long long)B * CO * CI;
+    auto served = [&] {
+        if (box && !box->own_tables(form)) return hint_paid(kHintSiteBox, layer, B, CO, CI);
+        return hint_paid(site, layer, B, CO, CI);
+    };
     const bool rows = row_cands_supported(form, K) && (density > 0.f || terms >= kSortRowsMinTerms) &&
-                      (density > 0.f || hint_build_spare(kHintSiteRows + form, layer, B, CO, CI, st, hint_paid(site, layer, B, CO, CI)));
+                      (density > 0.f || hint_build_spare(kHintSiteRows + form, layer, B, CO, CI, st, served()));
     if (rc || !rows) {
         // the every-term kernels read the flag behind the counter, as with both tables
         if (!rc) { a.gate = a.gate + 1; a.gate_limit = 0ull; }
@@ -341,7 +347,7 @@ static int sort_values(const float* input, const float* weight, int B, int CO, i
     if (copies && !sort_unpad(a, raw, CI, cols) && (rc = sort_pad_copy(a, raw, base + tbytes + kbytes, st))) return rc;
     int* keys = reinterpret_cast<int*>(base + tbytes);
     if (cols && (rc = queue_sort_cols(a, kHintSiteSort, layer, kRowsSortValues, a.x0, nullptr, a.w, B, CO, CI, q, K, nullptr, output, nullptr, base, box, st))) return rc;
-    if (cols) sort_cols_expect(a, layer, kHintSiteSort, B, CO, CI, st);
+    if (cols && (!box || box->own)) sort_cols_expect(a, layer, kHintSiteSort, B, CO, CI, st);
     if (box && g_sort_density.load(std::memory_order_relaxed) < 0.f) {
         a.told3 = hint_expect(kHintSiteBox, layer, B, CO, CI, st);
         a.few3 = box->count + 1;
@@ -449,7 +455,7 @@ static int sort_bounds(const float* inputL, const float* inputU, const float* we
         if (cols && (rc = queue_sort_cols(a, kHintSiteBoundSort, layer, kRowsSortInterval, a.x0, a.x1, a.w, B, CO, CI, q, K, outputL, outputU, nullptr, ws, box, st))) return rc;
     }
     if (streamed) return row_stream_sort(raw, K, st);
-    if (cols) sort_cols_expect(a, layer, kHintSiteBoundSort, B, CO, CI, st);
+    if (cols && !box) sort_cols_expect(a, layer, kHintSiteBoundSort, B, CO, CI, st);
     rc = SD_ERR_ARG;
     switch (K) {
 #define X(k) case k: rc = small ? launch_fwd<BoundSort<k>, 1, 2>(a, st) : launch_fwd<BoundSort<k>, 2, 2>(a, st); break;
