@@ -139,9 +139,6 @@ void* workspace(size_t bytes, hipStream_t stream);
 // False while `stream` records a graph and its buffer is smaller, and where the memory is not to be had.
 bool workspace_ready(size_t bytes, hipStream_t stream);
 
-// whether `stream` records a graph
-bool stream_captures(hipStream_t stream);
-
 // Held by an entry point while it queues its kernels.  The calls of several host threads then reach their streams
 // one after the other, whole, so that a stream's workspace is used in call order even when threads share the stream
 // (as they do by default); only the queueing is serialised, the work of different streams still overlaps.
@@ -170,6 +167,10 @@ bool hint_build_tables(int site, const void* weight, int B, int CO, int CI, hipS
 // they are left out again, up to kHintSpareMost: a call in vain costs 14 us.
 constexpr int kHintSpareMost = 192;
 bool hint_build_spare(int site, const void* weight, int B, int CO, int CI, hipStream_t stream, bool served);
+// Whether to queue tables that stand in for those of `site` where these do not serve: left out once those have served kHintStreak
+// calls in a row, and, each time they then do not, only after four times as many (up to kHintSpareMost); never while a graph is recorded.
+// The slot is that of `site`: nothing is expected for the tables that stand in.
+bool hint_stand_in(int site, const void* weight, int B, int CO, int CI, hipStream_t stream);
 // whether the layer's last call whose outcome is there was served from tables
 bool hint_paid(int site, const void* weight, int B, int CO, int CI);
 unsigned long long* hint_expect(int site, const void* weight, int B, int CO, int CI, hipStream_t stream);

@@ -86,8 +86,6 @@ bool capturing(hipStream_t stream) {
 }
 }  // namespace
 
-bool stream_captures(hipStream_t stream) { return capturing(stream); }
-
 bool workspace_ready(size_t bytes, hipStream_t stream) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0) { (void)hipGetLastError(); return false; }
@@ -142,7 +140,8 @@ struct HintSlot {
     int stale;                  // of the queued outcomes, how many belong to the layer the slot stood for before
     int streak, skip_left;
     int need;                   // outcomes without tables in a row before they are left out
-    bool left_out;              // spare tables (hint_build_spare): not built in the last call that could have had them
+    bool left_out;              // spare tables (hint_build_spare, hint_stand_in): not built in the last call that could have had them
+    int served, enough;         // calls in a row that these tables served, and how many before what stands in for them is left out
     bool known;                 // an outcome of this layer has arrived
     unsigned long long used;    // g_hint_clock at the slot's last use: the least recently used slot is given away
 };
@@ -155,7 +154,8 @@ void hint_rekey(HintSlot& h, int dev, int site, const void* weight, int B, int C
     h.dev = dev; h.site = site; h.weight = weight; h.B = B; h.CO = CO; h.CI = CI;
     h.stale = h.queued;
     h.streak = h.skip_left = 0;
-    h.need = kHintStreak;
+    h.need = h.enough = kHintStreak;
+    h.served = 0;
     h.left_out = h.known = false;
 }
 
@@ -201,6 +201,7 @@ void hint_drain(HintSlot& h) {
         else if (ran != kHintVoid) {
             h.known = true;
             h.streak = ran != 0ull ? h.streak + 1 : 0;
+            h.served = ran != 0ull ? 0 : h.served + 1;
             // the streak is long enough (or the probe after a stretch without tables came out the same): no tables
             // for the next kHintSkip calls, then one call probes again; tables at once where they served
             h.skip_left = h.streak >= h.need ? kHintSkip : 0;
@@ -242,6 +243,17 @@ bool hint_build_spare(int site, const void* weight, int B, int CO, int CI, hipSt
     if (h->left_out) { h->skip_left--; return false; }
     if (h->streak >= h->need) h->skip_left = kHintSkip;
     return true;
+}
+
+bool hint_stand_in(int site, const void* weight, int B, int CO, int CI, hipStream_t stream) {
+    if (capturing(stream)) return true;
+    std::lock_guard<std::mutex> lock(g_hint_mu);
+    HintSlot* h = hint_slot(site, weight, B, CO, CI, false);
+    if (!h) return true;
+    hint_drain(*h);
+    if (h->left_out && h->served == 0) h->enough = h->enough < kHintSpareMost / 4 ? h->enough * 4 : kHintSpareMost;
+    h->left_out = h->served >= h->enough;
+    return !h->left_out;
 }
 
 bool hint_paid(int site, const void* weight, int B, int CO, int CI) {

@@ -486,7 +486,7 @@ extern "C" int sd_bound_sort_neuron_forward_shifted(const float* inputL, const f
 // ranges and table take 59 us where those of the two forms took 102, the walk 192 where theirs took 203 (certification of 6 x 5120 at batch 512
 // 1503 -> 1406 us with the table, 1347 with the walk).  A layer whose shared table does not serve (intervals so wide that they
 // mark nearly everything) goes on as the two calls by themselves: the values' own tables are queued behind the shared one, and return at
-// once where that serves, until it is known to; where it did not in three calls it is left out of the next 31.
+// once where that serves, until it has in several calls; where it did not in three calls it is left out of the next 31.
 static int sort_box(const float* input, const float* inputL, const float* inputU, const float* weight, int B, int CO, int CI, int G, int HW,
                     float* output, float* outputL, float* outputU, float q, int K, const float* shift, float sign, sd_stream_t stream) {
     hipStream_t st = static_cast<hipStream_t>(stream);
@@ -524,7 +524,7 @@ static int sort_box(const float* input, const float* inputL, const float* inputU
         if ((rc = pad_rows({inputU, inputU, inputU}, {pu, pu, pu}, {B, 0, 0}, CI, N, st))) return rc;
         xv = pv; xl = pl; xu = pu; w = pw;
     }
-    SortBox box{nullptr, 0ull, ws, ws + shared, weight, density < 0.f ? !hint_paid(kHintSiteBox, weight, B, CO, N) || stream_captures(st) : true};
+    SortBox box{nullptr, 0ull, ws, ws + shared, weight, density > 0.f || hint_stand_in(kHintSiteBox, weight, B, CO, N, st)};
     if ((rc = sort_cols_box_tables(xv, xl, xu, w, B, CO, N, K, ws, density > 0.f ? density : sort_cols_cap(kRowsSortValues, N), &box.count, &box.limit, st)))
         return rc;
     if ((rc = sort_cols_box_main(w, B, CO, N, q, K, output, outputL, outputU, ws, box.limit, shift, sign, st))) return rc;

@@ -53,3 +53,28 @@ def test_tables_per_batch_row_are_left_out():
     assert _count(names, "sc_main_kernel") >= 12
     assert _count(names, "rc_tables_kernel") == 0, names
     assert all(torch.equal(a, b) for a, b in zip(layer.box(0.02), want))
+
+
+def test_values_beside_intervals_that_alternate():
+    """Narrow and wide intervals in turn, the wide ones beyond the shared table: after a few rounds the values' own tables stand in for it in
+    every wide call, and they are left out again where the intervals stay narrow."""
+    layer = _Layer(300, 1056, 1030)
+    want = {width: layer.apart(width) for width in (0.02, 3.0)}
+
+    def call(width):
+        assert all(torch.equal(a, b) for a, b in zip(layer.box(width), want[width]))
+        torch.cuda.synchronize()
+    own = "sc_main_kernel<10, false"
+    for _ in range(5):
+        call(0.02)
+    assert _count(_names(lambda: call(0.02)), own) == 0
+    for _ in range(2):
+        call(3.0)
+        call(0.02)
+    for _ in range(6):
+        names = _names(lambda: call(3.0))
+        assert _count(names, own) == 1, names
+        call(0.02)
+    for _ in range(14):
+        call(0.02)
+    assert _count(_names(lambda: call(0.02)), own) == 0
