@@ -21,7 +21,11 @@ from collections.abc import Iterable
 
 import torch
 import torch.nn as nn
-from torch.nn.modules.module import _has_any_global_hook
+try:
+    from torch.nn.modules.module import _has_any_global_hook
+except ImportError:      # a private name of torch: without it, hooks of all modules count as there
+    def _has_any_global_hook():
+        return True
 
 from . import ext
 from . import functional as F
