@@ -103,8 +103,11 @@ __device__ __forceinline__ bool gate_closed(const FwdArgs& a) {
     return closed;
 }
 
-// v > 0 rounded up to a power of two (infinite where there is none)
-__device__ __forceinline__ float pow2_above(float v) { return __uint_as_float((__float_as_uint(v) + 0x7fffffu) & 0x7f800000u); }
+// v > 0 rounded up to a power of two, to the largest there is above it
+__device__ __forceinline__ float pow2_above(float v) {
+    const uint32_t up = (__float_as_uint(v) + 0x7fffffu) & 0x7f800000u;
+    return __uint_as_float(up < 0x7f000000u ? up : 0x7f000000u);
+}
 
 // ---- error reporting ---------------------------------------------------------------------------
 void set_error(const char* fmt, ...);

@@ -1201,15 +1201,16 @@ struct LpWithMax : PolicyBase {
     static constexpr bool GATED = true;
     static constexpr int PIPE_WAVES = 3;
     static constexpr int MIN_WAVES = 3;
-    // rinv = 1 / maximum; FOLD (general p) keeps c = p log2(1 / maximum) instead, so that a term is
+    // rinv = 1 / maximum; FOLD (general p) keeps c = -p log2(maximum) instead, so that a term is
     // exp2(p log2|d| + c): one fused multiply-add in place of the scaling and the product (the rounding of
-    // log2|d|, about 2.5e-7 absolute, reaches y divided by p times p, i.e. unchanged: far inside the 1e-5 bar)
+    // log2|d|, about 2.5e-7 absolute, reaches y divided by p times p, i.e. unchanged: far inside the 1e-5 bar).
+    // Not the logarithm of the reciprocal: that of a maximum above 2^126 is subnormal, which the unit takes for 0.
     struct Acc { float s, rinv; };
     static __device__ __forceinline__ void init(Acc& A, const FwdArgs& a, size_t o, bool valid, int split = 0) {
-        const float rinv = valid ? 1.f / (FOLD && a.pow2_scale ? pow2_above(a.aux[o]) : a.aux[o]) : 1.f;
+        const float scale = !valid ? 1.f : FOLD && a.pow2_scale ? pow2_above(a.aux[o]) : a.aux[o], rinv = 1.f / scale;
         // the virtual term of size 1e-10 belongs to slice 0 only
         A.s = split == 0 ? __builtin_amdgcn_exp2f(a.p * __builtin_amdgcn_logf(kEps * rinv)) : 0.f;
-        A.rinv = FOLD ? a.p * __builtin_amdgcn_logf(rinv) : rinv;
+        A.rinv = FOLD ? -a.p * __builtin_amdgcn_logf(scale) : rinv;
     }
     static __device__ __forceinline__ float term(const Acc& A, const FwdArgs& a, float d) {
         if (FOLD) return __builtin_amdgcn_exp2f(fmaf(a.p, __builtin_amdgcn_logf(fabsf(d)), A.rinv));
