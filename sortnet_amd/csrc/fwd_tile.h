@@ -1191,6 +1191,9 @@ struct LpOnline : PolicyBase {
     }
 };
 
+// whether an output is formed again in its tile, see FwdArgs::redo: those whose sum was not finite are left undefined, the others keep their bits
+__device__ __forceinline__ bool lp_redo(float y) { return y != y; }
+
 // caller-supplied maximum (core/cuda/norm_dist_cuda.cu:163-259 with has_max); also the second step of the
 // general-p forward, whose first step is the l-inf kernel
 template <int IP, bool FOLD = (IP < 0)>
@@ -1225,9 +1228,12 @@ struct LpWithMax : PolicyBase {
     }
     static __device__ __forceinline__ void store(Acc& A, const FwdArgs& a, size_t o, int split = 0) {
         if (a.nsplit > 1) a.part0[(size_t)split * a.part_stride + o] = A.s;   // merged by lp_finalize_kernel
-        else {
+        else if (!FOLD || !a.only || lp_redo(a.y0[o])) {
             a.y0[o] = powf(A.s, a.inv_p) * (FOLD && a.pow2_scale ? pow2_above(a.aux[o]) : a.aux[o]);
-            if (FOLD && a.redo && !(A.s <= FLT_MAX)) a.redo[((blockIdx.z % a.G) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = 1u;
+            if (FOLD && a.redo && !(A.s <= FLT_MAX)) {
+                a.y0[o] = __builtin_nanf("");
+                a.redo[((blockIdx.z % a.G) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = 1u;
+            }
         }
     }
 };

@@ -98,13 +98,16 @@ __global__ void __launch_bounds__(256) lp_finalize_kernel(const float* __restric
                                                           unsigned long long gate_limit, int gate_above, LpRedo redo) {
     size_t o = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (o >= total || gate_closed(gate, gate_limit, gate_above)) return;
-    if (redo.only && redo.only[redo.tile(o)] == 0u) return;
+    if (redo.only && (redo.only[redo.tile(o)] == 0u || !lp_redo(y[o]))) return;
     if (part1 == nullptr) {
         float s = 0.f;
         #pragma unroll 16   // (loads in flight: 64 slices of 32 x 256 outputs 9.4 us one after the other)
         for (int k = 0; k < nsplit; k++) s += part0[(size_t)k * total + o];
         y[o] = scale ? powf(s, inv_p) * (redo.pow2 ? pow2_above(scale[o]) : scale[o]) : powf(fmaxf(s, FLT_MIN), inv_p);
-        if (redo.flags && !(s <= FLT_MAX)) redo.flags[redo.tile(o)] = 1u;
+        if (redo.flags && !(s <= FLT_MAX)) {
+            y[o] = __builtin_nanf("");
+            redo.flags[redo.tile(o)] = 1u;
+        }
     } else {
         float M = kEps;
         #pragma unroll 8
@@ -150,7 +153,7 @@ static int lp_split_finish(const FwdArgs& a, hipStream_t st, const LpRedo& redo 
 // finite, by a factor of 2^(127 / p), less what the number of terms takes (28 at p = 24 and 5120 inputs).  Layers of at least kSampledTerms terms take the
 // maximum over a part of the inputs, whole chunks from all over the row, up to the next power of two, which spares the result a
 // rounding.  The tiles of outputs that have a sum that is not finite (undefined or infinite operands among them) then run both steps
-// on all inputs, which is what all of them did before.  Index lists, 512 x 3840 x 3840 of 5120 at p = 24: 1741 -> 1467 us (maxima 312 -> 45,
+// on all inputs, which is what all of them did before, and store the outputs that had one: those beside them keep their bits.  Index lists, 512 x 3840 x 3840 of 5120 at p = 24: 1741 -> 1467 us (maxima 312 -> 45,
 // launches that return at once 10), with one weight 1e4 times the others 1713 -> 1750; lists 96 x 2250 x 3840, 8.3e8 terms, 229 -> 202; 250 x
 // 3072 x 1021 203 -> 182, 64 x 10240 x 1024 179 -> 151.  Where most tiles have such sums the layer takes twice as long.  Error against 64 bits, rms,
 // p = 24: lists 1.3e-7 -> 7.0e-8, images against small weights 4.6e-8 -> 3.7e-8, inputs whose spread grows along the row 1.9e-7 -> 1.0e-7.
