@@ -504,7 +504,9 @@ static int sort_box(const float* input, const float* inputL, const float* inputU
     const FwdArgs raw = v;
     int N = CI, NB = CI;
     const size_t copies = sort_pad(v, false, B, CO, N, G, HW), copies_b = sort_pad(b, false, B, CO, NB, G, HW);
-    if ((density <= 0.f && (row_stream_sort_ok(raw) || row_stream_sort_ok(b))) || (copies == 0) != (copies_b == 0) ||
+    // (where the values do not stream the weights the bounds do not: their limits are lower. Asked of the operands as they come: copies count
+    // as whole rows, whose limits are higher)
+    if ((density <= 0.f && row_stream_sort_ok(raw)) || (copies == 0) != (copies_b == 0) ||
         !sort_cols_eligible(v, false, B, CO, N, G, HW) || !sort_cols_eligible(b, false, B, CO, NB, G, HW) ||
         sort_cols_cap(kRowsSortValues, N) != sort_cols_cap(kRowsSortInterval, N))
         return apart();
