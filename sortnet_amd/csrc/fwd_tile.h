@@ -1191,7 +1191,11 @@ struct LpOnline : PolicyBase {
     }
 };
 
-// whether an output is formed again in its tile, see FwdArgs::redo: those whose sum was not finite are left undefined, the others keep their bits
+// Largest result, relative to a scale from a part of the inputs, that keeps that scale (an infinite sum's is none).  The exponents of the
+// terms reach p log2 of it and their rounding reaches y divided by p: up to 8, at powers from 10 to 31, it is at most what a power of
+// two as the scale spares in reciprocal and product, 5e-8 rms (any finite sum, at p = 10.5: 1.5e-7).
+constexpr float kSampledRoot = 8.f;
+// whether an output is formed again in its tile, see FwdArgs::redo: those beyond kSampledRoot are left undefined, the others keep their bits
 __device__ __forceinline__ bool lp_redo(float y) { return y != y; }
 
 // caller-supplied maximum (core/cuda/norm_dist_cuda.cu:163-259 with has_max); also the second step of the
@@ -1229,8 +1233,9 @@ struct LpWithMax : PolicyBase {
     static __device__ __forceinline__ void store(Acc& A, const FwdArgs& a, size_t o, int split = 0) {
         if (a.nsplit > 1) a.part0[(size_t)split * a.part_stride + o] = A.s;   // merged by lp_finalize_kernel
         else if (!FOLD || !a.only || lp_redo(a.y0[o])) {
-            a.y0[o] = powf(A.s, a.inv_p) * (FOLD && a.pow2_scale ? pow2_above(a.aux[o]) : a.aux[o]);
-            if (FOLD && a.redo && !(A.s <= FLT_MAX)) {
+            const float root = powf(A.s, a.inv_p);
+            a.y0[o] = root * (FOLD && a.pow2_scale ? pow2_above(a.aux[o]) : a.aux[o]);
+            if (FOLD && a.redo && !(root <= kSampledRoot)) {
                 a.y0[o] = __builtin_nanf("");
                 a.redo[((blockIdx.z % a.G) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = 1u;
             }

@@ -103,8 +103,9 @@ __global__ void __launch_bounds__(256) lp_finalize_kernel(const float* __restric
         float s = 0.f;
         #pragma unroll 16   // (loads in flight: 64 slices of 32 x 256 outputs 9.4 us one after the other)
         for (int k = 0; k < nsplit; k++) s += part0[(size_t)k * total + o];
-        y[o] = scale ? powf(s, inv_p) * (redo.pow2 ? pow2_above(scale[o]) : scale[o]) : powf(fmaxf(s, FLT_MIN), inv_p);
-        if (redo.flags && !(s <= FLT_MAX)) {
+        const float root = powf(scale ? s : fmaxf(s, FLT_MIN), inv_p);
+        y[o] = scale ? root * (redo.pow2 ? pow2_above(scale[o]) : scale[o]) : root;
+        if (redo.flags && !(root <= kSampledRoot)) {
             y[o] = __builtin_nanf("");
             redo.flags[redo.tile(o)] = 1u;
         }
@@ -149,13 +150,13 @@ static int lp_split_finish(const FwdArgs& a, hipStream_t st, const LpRedo& redo 
 // instructions per term), then one pass of sums relative to it, instead of the online form's two passes over
 // every LDS chunk.  Workspace: the maxima, then the partial sums of the split reduction.
 //
-// Where every term is formed whatever its size, the scale need not be the maximum: any M0 <= max |x - w| will do as long as (max / M0)^p stays
-// finite, by a factor of 2^(127 / p), less what the number of terms takes (28 at p = 24 and 5120 inputs).  Layers of at least kSampledTerms terms take the
-// maximum over a part of the inputs, whole chunks from all over the row, up to the next power of two, which spares the result a
-// rounding.  The tiles of outputs that have a sum that is not finite (undefined or infinite operands among them) then run both steps
-// on all inputs, which is what all of them did before, and store the outputs that had one: those beside them keep their bits.  Index lists, 512 x 3840 x 3840 of 5120 at p = 24: 1741 -> 1467 us (maxima 312 -> 45,
+// Where every term is formed whatever its size, the scale need not be the maximum: any M0 <= max |x - w| will do that leaves the result within
+// kSampledRoot times it.  Layers of at least kSampledTerms terms take the maximum over a part of the inputs, whole chunks from all over the row,
+// up to the next power of two, which spares the result a rounding.  The tiles of outputs beyond that (undefined or infinite operands
+// among them) then run both steps on all inputs, which is what all of them did before, and store these outputs: those beside them keep
+// their bits.  Index lists, 512 x 3840 x 3840 of 5120 at p = 24: 1741 -> 1467 us (maxima 312 -> 45,
 // launches that return at once 10), with one weight 1e4 times the others 1713 -> 1750; lists 96 x 2250 x 3840, 8.3e8 terms, 229 -> 202; 250 x
-// 3072 x 1021 203 -> 182, 64 x 10240 x 1024 179 -> 151.  Where most tiles have such sums the layer takes twice as long.  Error against 64 bits, rms,
+// 3072 x 1021 203 -> 182, 64 x 10240 x 1024 179 -> 151.  Where most tiles have such outputs the layer takes twice as long.  Error against 64 bits, rms,
 // p = 24: lists 1.3e-7 -> 7.0e-8, images against small weights 4.6e-8 -> 3.7e-8, inputs whose spread grows along the row 1.9e-7 -> 1.0e-7.
 constexpr int kSampledPart = 8;
 constexpr long long kSampledTerms = 1ll << 29;
