@@ -57,7 +57,7 @@ struct FwdArgs {
     float p, inv_p, q;
     const float* shift;   // vector added to the finished values, one entry per output channel, times shift_sign (+1 or -1); or null
     float shift_sign;
-    int sample;           // above 1: of every slice of the reduction range only this part (l-inf as a scale, see lp_forward_max_first)
+    int sample;           // above 1: of the row only every so many'th chunk (l-inf as a scale, see lp_forward_max_first)
     uint32_t* redo;       // l-p relative to a scale: one word per tile of outputs, set to 1 where a result is too far above its scale (kSampledRoot), and left undefined (null: not asked for)
     const uint32_t* only; // not null: gated policies run on the tiles whose word is set, l-p sums for the undefined outputs
     int pow2_scale;       // the scale is aux rounded up to a power of two

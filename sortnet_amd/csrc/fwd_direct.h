@@ -63,9 +63,8 @@ __global__ void __launch_bounds__(256, 4) fwd_kernel_direct(FwdArgs a) {
     const int r0 = blockIdx.y * BB, m0 = blockIdx.x * BM;
 
     const int nchunks = a.CIg / KT;
-    const int n_begin = (int)((long long)split * nchunks / a.nsplit) * KT;
-    int n_end = (int)((long long)(split + 1) * nchunks / a.nsplit) * KT;
-    if constexpr (P::SAMPLED) n_end = sampled_end(a, n_begin, n_end);
+    const int n_begin = first_chunk<P>(a, (int)((long long)split * nchunks / a.nsplit) * KT), step = chunk_step<P>(a);
+    const int n_end = (int)((long long)(split + 1) * nchunks / a.nsplit) * KT;
 
     // Loads of this wave (GPW per chunk, the same number for every wave).  One x tile: x groups wave + 4 u, then
     // w groups wave + 4 u.  Interval policies repair inverted intervals in LDS before the chunk is published, which
@@ -197,7 +196,7 @@ __global__ void __launch_bounds__(256, 4) fwd_kernel_direct(FwdArgs a) {
 
     // one iteration = one chunk of KT = 32 inputs = two LDS-direct sub-chunks (buffers 0 and 1)
     if (n_begin < n_end) { fetch_masks(n_begin); issue(n_begin, 0); }
-    for (int k0 = n_begin; k0 < n_end; k0 += KT) {
+    for (int k0 = n_begin; k0 < n_end; k0 += step) {
         landed();
         repair(0);
         apply_masks(0, k0);
@@ -208,7 +207,7 @@ __global__ void __launch_bounds__(256, 4) fwd_kernel_direct(FwdArgs a) {
         repair(1);
         apply_masks(1, k0 + KD);
         __syncthreads();                          // buffer 1 complete; everyone is done reading buffer 0
-        if (k0 + KT < n_end) { fetch_masks(k0 + KT); issue(k0 + KT, 0); }
+        if (k0 + step < n_end) { fetch_masks(k0 + step); issue(k0 + step, 0); }
         compute(1, k0 + KD);
         #pragma unroll
         for (int i = 0; i < TB; i++) {

@@ -137,11 +137,12 @@ __device__ __forceinline__ void load_w_tile(float (*ws)[LDP], const FwdArgs& a,
 // -------------------------------------------------------------------------------------------
 // the kernel
 // -------------------------------------------------------------------------------------------
-// end of the part of a slice that FwdArgs::sample asks for: whole chunks, at least one
-__device__ __forceinline__ int sampled_end(const FwdArgs& a, int n_begin, int n_end) {
-    if (a.sample <= 1) return n_end;
-    const int end = n_begin + ((n_end - n_begin + a.sample * KT - 1) / (a.sample * KT)) * KT;
-    return end < n_end ? end : n_end;
+// from one chunk of a slice to the next, and its first one: FwdArgs::sample takes every so many'th chunk of the row, wherever the slices end
+template <class P>
+__device__ __forceinline__ int chunk_step(const FwdArgs& a) { return P::SAMPLED && a.sample > 1 ? a.sample * KT : KT; }
+template <class P>
+__device__ __forceinline__ int first_chunk(const FwdArgs& a, int n) {
+    return P::SAMPLED && a.sample > 1 ? (n + a.sample * KT - 1) / (a.sample * KT) * (a.sample * KT) : n;
 }
 
 template <class P, int TB, int TM>
@@ -157,10 +158,9 @@ __global__ void __launch_bounds__(256, P::MIN_WAVES) fwd_kernel(FwdArgs a) {
     const int s = (r0 / a.HW) / kSubBatch;
 
     const int nchunks = (a.CIg + KT - 1) / KT;
-    const int n_begin = (int)((long long)split * nchunks / a.nsplit) * KT;
+    const int n_begin = first_chunk<P>(a, (int)((long long)split * nchunks / a.nsplit) * KT), step = chunk_step<P>(a);
     int n_end = (int)((long long)(split + 1) * nchunks / a.nsplit) * KT;
     if (n_end > a.CIg) n_end = a.CIg;
-    if constexpr (P::SAMPLED) n_end = sampled_end(a, n_begin, n_end);
 
     typename P::Acc acc[TB][TM];
     #pragma unroll
@@ -174,7 +174,7 @@ __global__ void __launch_bounds__(256, P::MIN_WAVES) fwd_kernel(FwdArgs a) {
         }
     }
 
-    for (int k0 = n_begin; k0 < n_end; k0 += KT) {
+    for (int k0 = n_begin; k0 < n_end; k0 += step) {
         load_x_tiles<NX, BB>(xs[0], xs[NX - 1], a, g, r0, k0, n_end);
         load_w_tile<BM>(ws, a, g, s, m0, k0, n_end);
         __syncthreads();
@@ -258,10 +258,9 @@ __global__ void __launch_bounds__(256, (pipe_waves<P, TB, TM>())) fwd_kernel_pip
     const bool masked = (NX == 1) && a.mask_mode == SD_MASK_FACTORED;
 
     const int nchunks = (a.CIg + KT - 1) / KT;
-    const int n_begin = (int)((long long)split * nchunks / a.nsplit) * KT;
+    const int n_begin = first_chunk<P>(a, (int)((long long)split * nchunks / a.nsplit) * KT), step = chunk_step<P>(a);
     int n_end = (int)((long long)(split + 1) * nchunks / a.nsplit) * KT;
     if (n_end > a.CIg) n_end = a.CIg;
-    if constexpr (P::SAMPLED) n_end = sampled_end(a, n_begin, n_end);
 
     // staging slot v of a work-item: float4 number v * 256 + tid of a tile = row (tid >> 3) + 32 v,
     // columns (tid & 7) * 4 .. +3.  Rows outside the tensor hold the tile's first row, whose results nothing stores.
@@ -366,10 +365,10 @@ __global__ void __launch_bounds__(256, (pipe_waves<P, TB, TM>())) fwd_kernel_pip
     }
 
     if (n_begin < n_end) gload(n_begin);
-    for (int k0 = n_begin; k0 < n_end; k0 += KT) {
+    for (int k0 = n_begin; k0 < n_end; k0 += step) {
         sstore(k0);
         __syncthreads();
-        if (k0 + KT < n_end) gload(k0 + KT);
+        if (k0 + step < n_end) gload(k0 + step);
         #pragma unroll
         for (int pass = 0; pass < P::PASSES; pass++) {
             #pragma unroll (pipe_unroll<P, TB, TM>())
@@ -427,10 +426,9 @@ __global__ void __launch_bounds__(256, (lists_whole<P, TB, TM>() ? P::NARROW_WAV
     const int s = (r0 / a.HW) / kSubBatch;
 
     const int nchunks = (a.CIg + KT - 1) / KT;
-    const int n_begin = (int)((long long)split * nchunks / a.nsplit) * KT;
+    const int n_begin = first_chunk<P>(a, (int)((long long)split * nchunks / a.nsplit) * KT), step = chunk_step<P>(a);
     int n_end = (int)((long long)(split + 1) * nchunks / a.nsplit) * KT;
     if (n_end > a.CIg) n_end = a.CIg;
-    if constexpr (P::SAMPLED) n_end = sampled_end(a, n_begin, n_end);
 
     // Rows outside the tensor hold the tile's first row, whose results nothing stores.  Byte offsets from uniform bases, which move on with
     // the chunks where there is no index list (pipe_ok: they fit 32 bits)
@@ -491,10 +489,10 @@ __global__ void __launch_bounds__(256, (lists_whole<P, TB, TM>() ? P::NARROW_WAV
     }
 
     if (n_begin < n_end) gload(n_begin);
-    for (int k0 = n_begin; k0 < n_end; k0 += KT) {
+    for (int k0 = n_begin; k0 < n_end; k0 += step) {
         sstore(k0);
         __syncthreads();
-        if (k0 + KT < n_end) gload(k0 + KT);
+        if (k0 + step < n_end) gload(k0 + step);
         #pragma unroll
         for (int pass = 0; pass < P::PASSES; pass++) {
             #pragma unroll (lists_whole<P, TB, TM>() ? KT / 4 : TM <= 4 && P::UNROLL4_TM4 ? P::UNROLL4_TM4 : P::UNROLL4)

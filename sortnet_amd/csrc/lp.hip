@@ -151,13 +151,15 @@ static int lp_split_finish(const FwdArgs& a, hipStream_t st, const LpRedo& redo 
 // every LDS chunk.  Workspace: the maxima, then the partial sums of the split reduction.
 //
 // Where every term is formed whatever its size, the scale need not be the maximum: any M0 <= max |x - w| will do that leaves the result within
-// kSampledRoot times it.  Layers of at least kSampledTerms terms take the maximum over a part of the inputs, whole chunks from all over the row,
+// kSampledRoot times it.  Layers of at least kSampledTerms terms take the maximum over a part of the inputs, one chunk of eight from all over the row,
 // up to the next power of two, which spares the result a rounding.  The tiles of outputs beyond that (undefined or infinite operands
 // among them) then run both steps on all inputs, which is what all of them did before, and store these outputs: those beside them keep
 // their bits.  Index lists, 512 x 3840 x 3840 of 5120 at p = 24: 1741 -> 1467 us (maxima 312 -> 45,
 // launches that return at once 10), with one weight 1e4 times the others 1713 -> 1750; lists 96 x 2250 x 3840, 8.3e8 terms, 229 -> 202; 250 x
 // 3072 x 1021 203 -> 182, 64 x 10240 x 1024 179 -> 151.  Where most tiles have such outputs the layer takes twice as long.  Error against 64 bits, rms,
-// p = 24: lists 1.3e-7 -> 7.0e-8, images against small weights 4.6e-8 -> 3.7e-8, inputs whose spread grows along the row 1.9e-7 -> 1.0e-7.
+// lists of all 3840 inputs, with the maximum of all inputs -> now: p = 24 6.3e-8 -> 3.8e-8, images against small weights 4.6e-8 -> 3.8e-8, one input
+// 6 / 300 times the others 3.2e-7 / 6.8e-7 -> 8.0e-8 / 1.7e-7; p = 10.5 6.9e-8 -> 4.3e-8, 3.0e-7 / 6.8e-7 -> 8.1e-8 / 1.6e-7; p = 31 6.2e-8 -> 3.4e-8,
+// 3.1e-7 / 7.0e-7 -> 1.2e-7 / 2.0e-7.  Which outputs keep the scale is decided by the call's own operands alone, so equal calls have equal bits.
 constexpr int kSampledPart = 8;
 constexpr long long kSampledTerms = 1ll << 29;
 static int lp_forward_max_first(FwdArgs& a, bool small, hipStream_t st) {
@@ -194,7 +196,12 @@ static int lp_forward_max_first(FwdArgs& a, bool small, hipStream_t st) {
     int rc;
     uint32_t* const flags = reinterpret_cast<uint32_t*>(base);
     base += flag_words;
-    if (sampled) m.sample = kSampledPart;
+    const int slices = m.nsplit;
+    if (sampled) {   // (slices that hold a chunk of the part each)
+        const int most = (a.CIg + KT - 1) / KT / kSampledPart;
+        m.sample = kSampledPart;
+        m.nsplit = slices < most ? slices : most > 1 ? most : 1;
+    }
     if (rows) {
         FwdArgs r = a;
         r.nsplit = ns_rows;
@@ -234,6 +241,7 @@ static int lp_forward_max_first(FwdArgs& a, bool small, hipStream_t st) {
     if ((rc = sums())) return rc;
     // (the maxima of all inputs meet those of the part in the same buffer)
     m.sample = 0;
+    m.nsplit = slices;
     m.only = a.only = redo.only = flags;
     a.redo = redo.flags = nullptr;
     a.pow2_scale = redo.pow2 = 0;

@@ -66,3 +66,31 @@ def test_error_where_the_part_misses_the_largest_differences():
     ref = torch.cat([_ref(x[b:b + 4, :, 0], w, 10.5) for b in range(0, B, 16)])
     err = torch.cat([y[b:b + 4] for b in range(0, B, 16)]).double() / ref - 1
     assert float(err.pow(2).mean().sqrt()) < 1.1e-7
+
+
+def _us(fn, n=10):
+    fn()
+    times = []
+    for _ in range(5):
+        e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        e0.record()
+        for _ in range(n):
+            fn()
+        e1.record()
+        torch.cuda.synchronize()
+        times.append(e0.elapsed_time(e1) * 1e3 / n)
+    return min(times)
+
+
+@pytest.mark.parametrize("B,N,M", [(1024, 1024, 8192), (2048, 1701, 4099)])
+def test_part_is_taken_from_all_over_the_row(B, N, M):
+    """Layers whose tiles fill the device without a split of the rows, three quarters of the inputs 100 times the others: a part from all over the row holds some of them, one from its start does not, and the
+    layer runs both steps twice (1.8 times as long). A quarter more is the limit."""
+    from sortnet_amd import functional as F
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x, w = torch.randn(B, N, 1, generator=g, device="cuda") * 0.3, torch.randn(M, N, generator=g, device="cuda")
+    ci = torch.arange(0, N, dtype=torch.int32, device="cuda").expand(B // 32, 1, N).contiguous()
+    even = _us(lambda: F.norm_dist_dropout(x, w, ci, None, 24.0))
+    w[:, N // 4:] *= 100
+    x[:, N // 4:] *= 100
+    assert _us(lambda: F.norm_dist_dropout(x, w, ci, None, 24.0)) < 1.25 * even
