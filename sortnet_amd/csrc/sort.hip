@@ -506,7 +506,7 @@ static int sort_box(const float* input, const float* inputL, const float* inputU
     const size_t copies = sort_pad(v, false, B, CO, N, G, HW), copies_b = sort_pad(b, false, B, CO, NB, G, HW);
     // (where the values do not stream the weights the bounds do not: their limits are lower. Asked of the operands as they come: copies count
     // as whole rows, whose limits are higher)
-    if ((density <= 0.f && row_stream_sort_ok(raw)) || (copies == 0) != (copies_b == 0) ||
+    if (K != kBoxK || (density <= 0.f && row_stream_sort_ok(raw)) || (copies == 0) != (copies_b == 0) ||
         !sort_cols_eligible(v, false, B, CO, N, G, HW) || !sort_cols_eligible(b, false, B, CO, NB, G, HW) ||
         sort_cols_cap(kRowsSortValues, N) != sort_cols_cap(kRowsSortInterval, N))
         return apart();
@@ -527,9 +527,9 @@ static int sort_box(const float* input, const float* inputL, const float* inputU
         xv = pv; xl = pl; xu = pu; w = pw;
     }
     SortBox box{nullptr, 0ull, ws, ws + shared, weight, density > 0.f || hint_stand_in(kHintSiteBox, weight, B, CO, N, st)};
-    if ((rc = sort_cols_box_tables(xv, xl, xu, w, B, CO, N, K, ws, density > 0.f ? density : sort_cols_cap(kRowsSortValues, N), &box.count, &box.limit, st)))
+    if ((rc = sort_cols_box_tables(xv, xl, xu, w, B, CO, N, ws, density > 0.f ? density : sort_cols_cap(kRowsSortValues, N), &box.count, &box.limit, st)))
         return rc;
-    if ((rc = sort_cols_box_main(w, B, CO, N, q, K, output, outputL, outputU, ws, box.limit, shift, sign, st))) return rc;
+    if ((rc = sort_cols_box_main(w, B, CO, N, q, output, outputL, outputU, ws, box.limit, shift, sign, st))) return rc;
     if ((rc = sort_values(xv, w, B, CO, N, G, HW, output, q, K, shift, sign, &box, stream))) return rc;
     return sort_bounds(xl, xu, w, B, CO, N, G, HW, outputL, outputU, q, K, shift, sign, &box, stream);
 }

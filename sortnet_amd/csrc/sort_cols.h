@@ -36,11 +36,12 @@ int sort_cols_forward(const float* xl, const float* xu, const float* w, int B, i
 // Values and interval bounds of one layer from one table: the ranges are those of inputs and both ends together, so one table
 // holds a superset of each form's marks, and the walks drop what is not needed (cand_walk.h).  sort_cols_box_tables builds it,
 // sort_cols_box_main walks it for the values (out) and the bounds.  `ws`: sort_cols_box_workspace bytes, kept until both have run;
-// gate, gate_limit and density as in sort_cols_forward.
+// gate, gate_limit and density as in sort_cols_forward.  Built for the depth of the layers' neuron, its default; other depths have two tables.
+constexpr int kBoxK = 10;
 size_t sort_cols_box_workspace(int B, int CO, int CI);
-int sort_cols_box_tables(const float* x, const float* xl, const float* xu, const float* w, int B, int CO, int CI, int K, void* ws,
+int sort_cols_box_tables(const float* x, const float* xl, const float* xu, const float* w, int B, int CO, int CI, void* ws,
                          float density, const unsigned long long** gate, unsigned long long* gate_limit, hipStream_t st);
-int sort_cols_box_main(const float* w, int B, int CO, int CI, float q, int K, float* out, float* outL, float* outU, void* ws,
+int sort_cols_box_main(const float* w, int B, int CO, int CI, float q, float* out, float* outL, float* outU, void* ws,
                        unsigned long long gate_limit, const float* shift, float shift_sign, hipStream_t st);
 
 // The two sums of the probe that sort_cols_forward / max_cols_forward leave behind the counter words *gate points at

@@ -16,7 +16,6 @@ constexpr int kRowPad = 128;         // weight rows are padded to a multiple of 
 constexpr int kMainWaves = 4;        // wavefronts of a workgroup of the main kernels
 constexpr int kMainTile = kMainWaves;   // weight rows of a workgroup, one per wavefront
 constexpr int kSample = 640;         // see walk_marks
-constexpr int kBoxK = 10;            // see sort_cols_box_main
 
 inline size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 inline int tiles_b(int B) { return (B + kTileB - 1) / kTileB; }
@@ -715,9 +714,9 @@ size_t sort_cols_box_workspace(int B, int CO, int CI) {
     return align256(sort_cols_workspace(B, CO, CI)) + align256((size_t)CI * tiles_b(B) * kTileB * 4);
 }
 
-int sort_cols_box_tables(const float* x, const float* xl, const float* xu, const float* w, int B, int CO, int CI, int K, void* ws,
+int sort_cols_box_tables(const float* x, const float* xl, const float* xu, const float* w, int B, int CO, int CI, void* ws,
                          float density, const unsigned long long** gate, unsigned long long* gate_limit, hipStream_t st) {
-    if (CI % kChunk != 0 || CI > 65536 || B < 1 || CO < 1 || K < 2 || K > 25) {
+    if (CI % kChunk != 0 || CI > 65536 || B < 1 || CO < 1) {
         set_error("sort_cols_box_tables: shape not supported");
         return SD_ERR_ARG;
     }
@@ -730,30 +729,17 @@ int sort_cols_box_tables(const float* x, const float* xl, const float* xu, const
     hipLaunchKernelGGL((sc_range_kernel<true, false, false, true>), dim3(CI / kChunk, S), dim3(256), 0, st, xl, xu, w, nullptr, B, CO, CI, Bp, c.xr, c.xT,
                        c.widths, c.count, nullptr, x, box_inputs(ws, B, CO, CI));
     const int rc = check_launch("sc_range_kernel");
-    return rc ? rc : run_tables<false, false>(w, nullptr, S, CO, mpad_of(CO), CI, K, c, *gate_limit, nullptr, st);
+    return rc ? rc : run_tables<false, false>(w, nullptr, S, CO, mpad_of(CO), CI, kBoxK, c, *gate_limit, nullptr, st);
 }
 
-int sort_cols_box_main(const float* w, int B, int CO, int CI, float q, int K, float* out, float* outL, float* outU, void* ws,
+int sort_cols_box_main(const float* w, int B, int CO, int CI, float q, float* out, float* outL, float* outU, void* ws,
                        unsigned long long gate_limit, const float* shift, float shift_sign, hipStream_t st) {
     const Carve c = carve(ws, B, CO, CI);
     const int S = tiles_b(B), Bp = S * kTileB, Mp = mpad_of(CO);
     const dim3 grid((unsigned)(S * (Mp / kMainTile))), block(64 * kMainWaves);
     const float* xT2 = box_inputs(ws, B, CO, CI);
-    if (K == kBoxK) {   // the depth of the layers' neuron (its default)
-        hipLaunchKernelGGL((sc_main_kernel<kBoxK, true, false, true>), grid, block, 0, st, c.xT, w, c.bits, c.xr, c.low, &c.count->marks, gate_limit, B, Bp,
-                           CO, Mp, CI, q, outL, outU, shift, shift_sign, xT2, out);
-        return check_launch("sc_main_kernel");
-    }
-    switch (K) {
-#define X(k) case k: \
-        hipLaunchKernelGGL((sc_main_kernel<k, true>), grid, block, 0, st, c.xT, w, c.bits, c.xr, c.low, &c.count->marks, gate_limit, B, Bp, \
-                           CO, Mp, CI, q, outL, outU, shift, shift_sign, nullptr, nullptr); \
-        hipLaunchKernelGGL((sc_main_kernel<k, false>), grid, block, 0, st, xT2, w, c.bits, c.xr, c.low, &c.count->marks, gate_limit, B, Bp, \
-                           CO, Mp, CI, q, nullptr, out, shift, shift_sign, nullptr, nullptr); \
-        break;
-        SD_SORT_COLS_K(X)
-#undef X
-    }
+    hipLaunchKernelGGL((sc_main_kernel<kBoxK, true, false, true>), grid, block, 0, st, c.xT, w, c.bits, c.xr, c.low, &c.count->marks, gate_limit, B, Bp,
+                       CO, Mp, CI, q, outL, outU, shift, shift_sign, xT2, out);
     return check_launch("sc_main_kernel");
 }
 
