@@ -146,7 +146,7 @@ __device__ __forceinline__ int first_chunk(const FwdArgs& a, int n) {
 }
 
 template <class P, int TB, int TM>
-__global__ void __launch_bounds__(256, P::MIN_WAVES) fwd_kernel(FwdArgs a) {
+__global__ void __launch_bounds__(256, TB * TM <= 4 && P::MIN_WAVES_NARROW ? P::MIN_WAVES_NARROW : P::MIN_WAVES) fwd_kernel(FwdArgs a) {
     if constexpr (P::GATED) { if (gate_closed(a)) return; }
     constexpr int BB = 16 * TB, BM = 16 * TM, NX = P::NX;
     __shared__ __attribute__((aligned(16))) float xs[NX][BB][LDP];
@@ -586,6 +586,10 @@ struct PolicyBase {
     static constexpr int NX = 1;
     static constexpr int PASSES = 1;
     static constexpr int MIN_WAVES = 1;   // waves per SIMD the register budget must allow
+    // same for tiles of 2 x 2 outputs (0: no other): left alone the compiler takes 79 registers for the interval bounds and 108 for the masked
+    // neuron, of which 61 and 84 serve as well (bounds of convolutions 128 x 75 x 100 x 196 52 -> 48 us, 64 x 27 x 64 x 256 11.6 -> 11.1, masked
+    // 100 x 3071 x 515 72 -> 64; bounds of 64 x 2049 x 1000 29 -> 32)
+    static constexpr int MIN_WAVES_NARROW = 0;
     static constexpr int PIPE_WAVES = 2;  // same for the pipelined kernel
     static constexpr int UNROLL4 = 2;     // unroll factor of the loop over groups of four inputs
     static constexpr int PIPE_WAVES_TM4 = 0, UNROLL4_TM4 = 0;   // overrides for tiles of <= 4 channels (0: none)
@@ -741,6 +745,7 @@ __device__ __forceinline__ float masked_abs(float d, uint32_t byte, uint32_t t8)
 struct MaskedTermChunk : PolicyBase {
     static constexpr int PIPE_WAVES = 2;   // hash-bound: timings were flat over 2..4 waves and 4x8 / 4x4 / 2x8 tiles
     static constexpr int MIN_WAVES = 2;
+    static constexpr int MIN_WAVES_NARROW = 5;
     struct Acc { float best, cm; int cid; uint32_t key; };
     static __device__ __forceinline__ void init(Acc& A, const FwdArgs& a, size_t o, bool, int split = 0) {
         A.best = kEps; A.cm = 0.f; A.cid = -1; A.key = rng_row_key(a.seed, 0u, (uint32_t)o);
@@ -790,6 +795,7 @@ struct BoundNograd : PolicyBase {
     static constexpr int PIPE_WAVES = 3;
     static constexpr int NX = 2;
     static constexpr int MIN_WAVES = 3;
+    static constexpr int MIN_WAVES_NARROW = 7;
     static constexpr int UNROLL4 = 1;
     struct Acc { float lo, hi; };
     static __device__ __forceinline__ void init(Acc& A, const FwdArgs&, size_t, bool, int split = 0) { A.lo = -kEps; A.hi = kEps; }
