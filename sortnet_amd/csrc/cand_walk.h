@@ -121,7 +121,8 @@ __device__ __forceinline__ void walk_block(int n, const Own& o, int cnt, Load&& 
 //   SHORT: of a list of up to 64 marks, a mark per lane, about so many of the strongest go first and the others by keep(), as in a long
 //   list (0: such lists are walked as they are).  Most rows of an evaluated network's later layers have such lists: certification of
 //   6 x 5120 at batch 512 1347 -> 1312 us (13 strongest 1324, lists of up to 40 as they are 1318); 16 instead of 32 of the long
-//   lists' strongest marks first: 1347 -> 1360.
+//   lists' strongest marks first: 1347 -> 1360.  Not in the values' walk of the sort neuron with positions, which another walk follows: 512 x 5120 x
+//   5120 at spreads 0.05 and 0.3 168.3 and 520.2 us without, 170.4 and 521.9 with, 64 x 2048 x 2048 at 0.3 73.3 and 74.2.
 //   own(input) -> Own: a gather;  load / use: see walk_block;
 //   threshold(strong): brings what keep() compares with up to date, after the strong marks and after every 64;
 //   ORDERED: forms for which the order of the inputs counts.  The strong marks are then walked for their values alone, by

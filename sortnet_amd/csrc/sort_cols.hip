@@ -574,7 +574,7 @@ sp_main_kernel(const float* __restrict__ xT, const float* __restrict__ w, const 
                 th = wave_min_nonneg(__builtin_bit_cast(float, min(in0 ? top[0][0] : none, in1 ? top[1][0] : none)));
             };
             listed = for_marks(list, NCH, lane, word, [&](int total, bool first) __attribute__((always_inline)) {
-                walk_marks<false, false, kSample, walk_short(K)>(list, total, first, lane, own, cap, load, value, value,
+                walk_marks<false, false, kSample, 0>(list, total, first, lane, own, cap, load, value, value,
                                          [&](bool) __attribute__((always_inline)) { smallest(); }, keep, [] {});
             });
             smallest();
