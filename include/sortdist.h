@@ -288,7 +288,7 @@ int sd_bound_sort_neuron_forward_shifted(const float* inputL, const float* input
 
 /* Values and interval bounds of one layer of an evaluation pass: sd_sort_neuron_forward_shifted on (input, output) and
  * sd_bound_sort_neuron_forward_shifted on the others, the same bits (shift may be NULL: without it); where both work from
- * candidate tables, from one. */
+ * candidate tables, from one where K is 10, the depth of the layers. */
 int sd_sort_neuron_box_forward(const float* input, const float* inputL, const float* inputU, const float* weight,
                                int B, int CO, int CI, int G, int HW, float* output, float* outputL, float* outputU,
                                float q, int K, const float* shift, float sign, sd_stream_t stream);
