@@ -19,14 +19,14 @@ def _us(fn, n=40):
     return min(times)
 
 
-@pytest.mark.parametrize("B,N,M", [(64, 512, 512), (64, 3072, 200)])
+@pytest.mark.parametrize("B,N,M", [(64, 512, 512), (48, 480, 512)])
 def test_stores_do_not_wait_for_each_other(B, N, M):
-    """Values alone, on wide tiles, against the same with positions, on narrow ones: 18.6 and 14.5 us, 32.5 and 20.5; with stores that wait for the
-    one before them 26.9 and 39.9. The line is between the two, at 1.7 times."""
+    """Values alone, on wide tiles, against the same with positions, on narrow ones: 18.6 and 14.5 us at the first size; with stores that wait for the
+    one before them 26.9. The line is between the two, at 1.65 times."""
     from sortnet_amd import ext
     g = torch.Generator(device="cuda").manual_seed(1)
     x, w = torch.randn(B, N, 1, generator=g, device="cuda"), torch.randn(M, N, generator=g, device="cuda")
     y, pos = torch.empty(B, M, 1, device="cuda"), torch.empty(B, M, 1, device="cuda", dtype=torch.int32)
     alone = _us(lambda: ext.masked_inf_dist_forward(x, w, y, None, 1, 0.3, 7, ext.MASK_TERM))
     both = _us(lambda: ext.masked_inf_dist_forward(x, w, y, pos, 1, 0.3, 7, ext.MASK_TERM))
-    assert alone < 1.7 * both
+    assert alone < 1.65 * both
